@@ -19,6 +19,7 @@
 #include "common.h"
 #include "gemm_q6k.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -58,6 +59,16 @@ __device__ __forceinline__ void store_tile_scaled(const float16_t& acc, float* _
             float* dst = c + (size_t)row * ldc + col;
             *dst = accumulate ? *dst + acc[r] * sc[r] : acc[r] * sc[r];
         }
+    }
+}
+
+// a partial tile of a workgroup that holds a part of k: no scale, rows of ldc
+__device__ __forceinline__ void store_tile_part(const float16_t& acc, float* __restrict__ part, int ldc, int row0, int col0, int m, int n, int lane) {
+    const int col = col0 + (lane & 31);
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        if (row < m && col < n) part[(size_t)row * ldc + col] = acc[r];
     }
 }
 
@@ -374,6 +385,10 @@ struct Q4kFragSegs {
     // pair != 0: w[0], w[1] are the gate and up matrices of a SwiGLU; a tile holds the same 32 columns of both
     // (its two 32-column halves) and stores silu(gate) * up into c[0]
     int pair;
+    // gemm_q4k_frag_kernel with k split over workgroups (gridDim.y of them per tile): the unscaled partial products go to
+    // part[blockIdx.y][m][part_cols], matrix i at column part_col0[i] (a pair: gate, then up); null: no split
+    float* part;
+    int part_cols, part_col0[3];
 };
 
 // the kernel's LDS (weight buffers, then the tile exchange) exceeds the static limit (the scales of the tile's rows follow it): dynamic, opted in per
@@ -401,7 +416,10 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kq = wave & 3, mh = wave >> 2;
     const int h = lane >> 5, r = lane & 31;
-    const int nb = k >> 8, nch = k >> 6, groups = (nb + 3) >> 2;
+    const int nb = k >> 8, nch = k >> 6;
+    // (this workgroup's superblocks: all of them, or a part of k)
+    const int sb0 = nb * (int)blockIdx.y / (int)gridDim.y, sb1 = nb * ((int)blockIdx.y + 1) / (int)gridDim.y;
+    const int groups = (sb1 - sb0 + 3) >> 2;
     // tile -> (row tile, weight matrix, column tile): the column tiles of up to three matrices sharing the
     // activations are laid side by side
     const int mt = blockIdx.x / segs.n_tiles, tn = blockIdx.x - mt * segs.n_tiles;
@@ -422,7 +440,7 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
             const int i = wave + 4 * MH * x;
             if (i < kWPieces) {
                 const int p = i * 64 + lane, row = p / kWPieces, col = min(p - kWPieces * row, 35);
-                const int off = min(g * 576 + col * 16, nb * 144 - 16);  // (a short last group repeats the row's last piece)
+                const int off = min(sb0 * 144 + g * 576 + col * 16, nb * 144 - 16);  // (a short last group repeats the row's last piece)
                 const uint8_t* wsrc = pair && row >= 32 ? segs.w[1] : w;  // (pair: tile rows 32.. are the up matrix)
                 const uint8_t* src = wsrc + (size_t)min(n0 + (pair ? row & 31 : row), n - 1) * nb * 144 + off;
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
@@ -458,10 +476,10 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
     float* isc_lds = reinterpret_cast<float*>(lds + frag_lds_bytes<MT, MH>());
     wfetch(0, 0);
     if (tid < 32 * MT * MH) isc_lds[tid] = inv_scale[MH * mt * MT * 32 + tid];
-    if (kq < nb) {
+    if (sb0 + kq < sb1) {
         // (the first eight fragment steps are requested behind the weights and stay in flight past the barrier)
 #pragma unroll
-        for (int s = 0; s < 8; s++) afetch(16 * kq + s, s);
+        for (int s = 0; s < 8; s++) afetch(16 * (sb0 + kq) + s, s);
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * MT) : "memory");
     } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -469,9 +487,9 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
     for (int g = 0; g < groups; g++) {
-        const int sb = 4 * g + kq;
+        const int sb = sb0 + 4 * g + kq;
         if (g + 1 < groups) wfetch(g + 1, (g + 1) & 1);
-        if (sb < nb) {
+        if (sb < sb1) {
             // this lane's weight rows (one per 32-column tile): the 144 bytes of superblock sb
             const uint8_t* wl = lds + (g & 1) * kWBuf + r * kWPitch + kq * 144;
             constexpr int kTile = 32 * kWPitch;  // the lane's row of the second 32-column tile
@@ -606,7 +624,7 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
         // a bare barrier: a full __syncthreads() would also wait for the fragment loads in flight
         // The next group's weights were requested before this superblock's 16 MT fragment loads, and loads
         // complete in order: once all but the newest 8 MT have landed, so have they.
-        if (sb < nb) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * MT) : "memory");
+        if (sb < sb1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * MT) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
@@ -656,6 +674,11 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                         // register x of lane l: row 8 (x / 4) + 4 (l / 32) + x % 4 of the 32 x 32 tile
                         const int row = (mb0 + i) * 32 + 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3);
                         if (row < m && col < n) {
+                            if (segs.part) {
+                                float* dst = segs.part + ((size_t)blockIdx.y * m + row) * segs.part_cols + col;
+                                dst[0] = g, dst[segs.part_col0[1]] = u;
+                                continue;
+                            }
                             const float sc = isc_lds[row - MH * mt * MT * 32];
                             const float a = g * sc;
                             c[(size_t)row * n + col] = a / (1.0f + expf(-a)) * (u * sc);  // silu(gate) * up
@@ -676,19 +699,91 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                 float sc[16];
 #pragma unroll
                 for (int x = 0; x < 16; x++) sc[x] = isc_lds[(mh * MT + i) * 32 + 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3)];
-                store_tile_scaled(sum, c, n, (mb0 + i) * 32, n0 + 32 * j, m, n, sc, lane, segs.accumulate[seg] != 0);
+                if (segs.part)
+                    store_tile_part(sum, segs.part + (size_t)blockIdx.y * m * segs.part_cols + segs.part_col0[seg], segs.part_cols, (mb0 + i) * 32,
+                                    n0 + 32 * j, m, n, lane);
+                else
+                    store_tile_scaled(sum, c, n, (mb0 + i) * 32, n0 + 32 * j, m, n, sc, lane, segs.accumulate[seg] != 0);
             }
         }
     }
 }
 
 
+// ---- k split over workgroups ------------------------------------------------------------------------------------
+// A product of few rows has few tiles (64 of them for 41 x 4096), each a serial walk along all of k by one workgroup.
+// Where the tiles leave compute units idle, k is divided over `splits` workgroups per tile as well; each leaves its
+// unscaled partial products in the workspace and this kernel adds them in a fixed order, applies the row scale and does
+// what the store would have done (add into c, or silu(gate) * up of a pair).
+struct PartSegs {
+    float* c[3];
+    int n[3], col0[3], accumulate[3];
+    int count, pair;
+};
+
+template <int W>  // columns per thread: 4, or 1 where a matrix has a number of columns that is no multiple of 4
+__global__ __launch_bounds__(256) void gemm_add_parts_kernel(const float* __restrict__ part, int splits, int cols, const PartSegs segs,
+                                                            const float* __restrict__ inv_scale, int m) {
+    const int row = blockIdx.y, col = (blockIdx.x * 256 + threadIdx.x) * W;
+    if (col >= (segs.pair ? segs.n[0] : cols)) return;
+    typedef float vec __attribute__((ext_vector_type(W)));
+    const float* src = part + (size_t)row * cols + col;
+    const size_t stride = (size_t)m * cols;
+    auto total = [&](const float* p) __attribute__((always_inline)) {
+        vec sum = *reinterpret_cast<const vec*>(p);
+        int z = 1;
+        for (; z + 4 <= splits; z += 4) {  // four parts requested together, added one after the other
+            vec v[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = *reinterpret_cast<const vec*>(p + (z + i) * stride);
+#pragma unroll
+            for (int i = 0; i < 4; i++) sum += v[i];
+        }
+        for (; z < splits; z++) sum += *reinterpret_cast<const vec*>(p + z * stride);
+        return sum;
+    };
+    const float sc = inv_scale[row];
+    vec v = total(src) * sc;
+    if (segs.pair) {
+        const vec u = total(src + segs.col0[1]) * sc;
+#pragma unroll
+        for (int i = 0; i < W; i++) v[i] = v[i] / (1.0f + expf(-v[i])) * u[i];
+        *reinterpret_cast<vec*>(segs.c[0] + (size_t)row * segs.n[0] + col) = v;
+        return;
+    }
+    const int i = segs.count > 2 && col >= segs.col0[2] ? 2 : (segs.count > 1 && col >= segs.col0[1] ? 1 : 0);
+    vec* dst = reinterpret_cast<vec*>(segs.c[i] + (size_t)row * segs.n[i] + (col - segs.col0[i]));
+    *dst = segs.accumulate[i] ? *dst + v : v;
+}
+
+int launch_add_parts(skn_ctx* ctx, const float* part, int splits, int cols, const PartSegs& segs, const float* isc, int m) {
+    bool wide = true;
+    for (int i = 0; i < segs.count; i++) wide = wide && segs.n[i] % 4 == 0 && ((uintptr_t)segs.c[i] & 15) == 0;
+    const int n = segs.pair ? segs.n[0] : cols;
+    if (wide) skn_launch(ctx, gemm_add_parts_kernel<4>, dim3((n / 4 + 255) / 256, m), dim3(256), 0, part, splits, cols, segs, isc, m);
+    else skn_launch(ctx, gemm_add_parts_kernel<1>, dim3((n + 255) / 256, m), dim3(256), 0, part, splits, cols, segs, isc, m);
+    SKN_LAUNCH_CHECK(ctx);
+    return SKN_OK;
+}
+
+// How many workgroups share a tile's k: as many as there are compute units for, at least one superblock for each of a
+// workgroup's four k-parts.  us per call, unsplit -> chosen: Q6_K 41 x 4096 x 11008 (64 tiles) 81 -> 34.5, 120 x 4096 x 11008
+// 106 -> 45, 200 x 4096 x 11008 (128 tiles) 108 -> 71; Q4_K 41 x 4096 x 11008 35.7 -> 24.6, 41 x 4096 x 4096 17.8 -> 15.1,
+// 200 x 4096 x 4096 25.9 -> 24.8.  Filling every compute unit twice is no gain (Q4_K 41 x 4096 x 11008 27.2, 120 x 4096 x 4096
+// 21.5 against 18.7), nor is a second part for tiles that fill two thirds of the device (Q4_K 41 x 11008 x 4096 22.2 against
+// 19.6, Q6_K 333 x 4096 x 4096 59 against 54): the addition costs 3 us and the parts their way through memory.
+int k_splits(const skn_ctx* ctx, int m, int tiles, int nb) {
+    if (m > 65535) return 1;  // (a grid dimension of the addition)
+    if (ctx->opt_gemm_split > 0) return std::min(ctx->opt_gemm_split, nb);
+    return std::max(1, std::min({ctx->compute_units / tiles, (nb + 3) / 4, 16}));
+}
+
 template <int MT, int MH>
 int launch_frag(skn_ctx* ctx, int m_tiles, const u32x4* afrag, const u32x4* sfrag, const Q4kFragSegs& segs, const float* isc,
-                int m, int k) {
+                int m, int k, int splits) {
     constexpr int kLds = frag_lds_bytes<MT, MH>() + 32 * MT * MH * 4;
     const uint32_t a_bytes = (uint32_t)((size_t)m_tiles * 32 * MT * MH * k * 2);  // (checked by the caller to fit)
-    skn_launch(ctx, gemm_q4k_frag_kernel<MT, MH>, dim3(m_tiles * segs.n_tiles), dim3(256 * MH), kLds, afrag, sfrag, segs, isc, m, k, a_bytes);
+    skn_launch(ctx, gemm_q4k_frag_kernel<MT, MH>, dim3(m_tiles * segs.n_tiles, splits), dim3(256 * MH), kLds, afrag, sfrag, segs, isc, m, k, a_bytes);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
@@ -1191,7 +1286,7 @@ template <int MT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_q6k_frag_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restrict__ w, const float* __restrict__ inv_scale,
                           float* __restrict__ c, int m, int n, int k, int m_tiles, int n_tiles, int accumulate,
-                          uint32_t a_bytes, uint32_t w_bytes, int xcd_rows) {
+                          uint32_t a_bytes, uint32_t w_bytes, int xcd_rows, float* __restrict__ part) {
     extern __shared__ __align__(16) float red[];  // 2 MT tiles x 3 copies x 1024 floats
     const int lane = threadIdx.x & 63;
     const int kq = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -1211,6 +1306,8 @@ void gemm_q6k_frag_kernel(const u32x4* __restrict__ afrag, const uint8_t* __rest
     }
     if (tn >= n_tiles) return;
     const int nb = k >> 8, nch = k >> 6;
+    // (this workgroup's superblocks: all of them, or a part of k whose products go unscaled to part[blockIdx.y][m][n])
+    const int sb0 = nb * (int)blockIdx.y / (int)gridDim.y, sb1 = nb * ((int)blockIdx.y + 1) / (int)gridDim.y;
     // The weights are read with buffer loads too: the lane's byte offset (its weight row, its sixteen-byte half) plus
     // a scalar one (superblock, piece).  A piece of an odd superblock starts at an address that is only a multiple
     // of two.
@@ -1262,13 +1359,13 @@ void gemm_q6k_frag_kernel(const u32x4* __restrict__ afrag, const uint8_t* __rest
             for (int x = 0; x < 16; x++) total[i][j][x] = 0.f;
 
     Q6kHalf H0, H1;
-    if (kq < nb) {
-        load_head(kq, scl_n, dh_n);
-        load_half(kq, 0, H0);
+    if (sb0 + kq < sb1) {
+        load_head(sb0 + kq, scl_n, dh_n);
+        load_half(sb0 + kq, 0, H0);
 #pragma unroll
-        for (int s = 0; s < RING - 1; s++) afetch(16 * kq + s, s);
+        for (int s = 0; s < RING - 1; s++) afetch(16 * (sb0 + kq) + s, s);
     }
-    for (int sb = kq; sb < nb; sb += 4) {
+    for (int sb = sb0 + kq; sb < sb1; sb += 4) {
         const int sb_next = min(sb + 4, nb - 1);  // (past the end: a repeat of the last superblock, unused)
         float dsc[2];
 #pragma unroll
@@ -1382,7 +1479,8 @@ void gemm_q6k_frag_kernel(const u32x4* __restrict__ afrag, const uint8_t* __rest
                 for (int o = 0; o < 3; o++)
 #pragma unroll
                     for (int x = 0; x < 16; x++) sum[x] += red[(t * 3 + o) * 1024 + 64 * x + lane];
-                store_tile(sum, c, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, inv_scale, lane, accumulate != 0);
+                if (part) store_tile_part(sum, part + (size_t)blockIdx.y * m * n, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, lane);
+                else store_tile(sum, c, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, inv_scale, lane, accumulate != 0);
             }
         }
 }
@@ -1402,7 +1500,7 @@ constexpr int kQ6PcLds = 4 * 2 * kQ6Stage + 4 * kQ6Aux;
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restrict__ w, const float* __restrict__ inv_scale,
                         float* __restrict__ c, int m, int n, int k, int m_tiles, int n_tiles, int accumulate,
-                        uint32_t a_bytes, uint32_t w_bytes) {
+                        uint32_t a_bytes, uint32_t w_bytes, float* __restrict__ part) {
     constexpr int MT = 4;
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1413,7 +1511,9 @@ void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restri
     const int xcd = blockIdx.x & 7, per = 8 / m_tiles;  // (an XCD keeps to one row tile, as above; m_tiles divides 8)
     const int mt = xcd % m_tiles, tn = (blockIdx.x >> 3) * per + xcd / m_tiles;
     if (tn >= n_tiles) return;
-    const int nb = k >> 8, nch = k >> 6, nsb = (nb + 3) >> 2;  // nsb: superblocks of the busiest pair
+    const int nb = k >> 8, nch = k >> 6;
+    const int sb0 = nb * (int)blockIdx.y / (int)gridDim.y, sb1 = nb * ((int)blockIdx.y + 1) / (int)gridDim.y;  // (as above)
+    const int nsb = (sb1 - sb0 + 3) >> 2;  // superblocks of the busiest pair
     uint8_t* stage = lds + kq * 2 * kQ6Stage;
     uint8_t* aux = lds + 4 * 2 * kQ6Stage + kq * kQ6Aux;
     auto barrier = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
@@ -1512,8 +1612,8 @@ void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restri
         // before their use: head and first half of the next superblock with chunk 2, its second half with its chunk 0.
         auto phase = [&](int i, auto cc_const) __attribute__((always_inline)) {
             constexpr int cc = decltype(cc_const)::value;
-            const int sb = 4 * i + kq;
-            if (sb < nb) {
+            const int sb = sb0 + 4 * i + kq;
+            if (sb < sb1) {
                 const int sbn = min(sb + 4, nb - 1);  // (past the end: a repeat, unused)
                 if (cc == 0) unpack(C1{}, H0, 1);
                 if (cc == 1) {
@@ -1522,7 +1622,7 @@ void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restri
                     unpack(C2{}, H1, 0);
                 }
                 if (cc == 2) unpack(C3{}, H1, 1);
-                if (cc == 3 && sb + 4 < nb) {
+                if (cc == 3 && sb + 4 < sb1) {
                     enter(i + 1);
                     load_half(sb + 4, 1, H1);
                     unpack(C0{}, H0, 0);
@@ -1530,10 +1630,10 @@ void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restri
             }
             barrier();
         };
-        if (kq < nb) {
-            load_head(kq, scl_n, dh_n);
-            load_half(kq, 0, H0);
-            load_half(kq, 1, H1);
+        if (sb0 + kq < sb1) {
+            load_head(sb0 + kq, scl_n, dh_n);
+            load_half(sb0 + kq, 0, H0);
+            load_half(sb0 + kq, 1, H1);
             enter(0);
             unpack(C0{}, H0, 0);
         }
@@ -1570,8 +1670,8 @@ void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restri
                 for (int x = 0; x < 16; x++) acc[i][j][x] = 0.f;
         auto phase = [&](int i, auto cc_const) __attribute__((always_inline)) {
             constexpr int cc = decltype(cc_const)::value;
-            const int sb = 4 * i + kq;
-            if (sb < nb) {
+            const int sb = sb0 + 4 * i + kq;
+            if (sb < sb1) {
                 if (cc == 0) {
 #pragma unroll
                     for (int j = 0; j < 2; j++) {
@@ -1617,9 +1717,9 @@ void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restri
             }
             barrier();
         };
-        if (kq < nb) {
+        if (sb0 + kq < sb1) {
 #pragma unroll
-            for (int s = 0; s < 3; s++) afetch(16 * kq + s, s);
+            for (int s = 0; s < 3; s++) afetch(16 * (sb0 + kq) + s, s);
         }
         barrier();
         for (int i = 0; i < nsb; i++) {
@@ -1656,7 +1756,8 @@ void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restri
                     for (int o = 0; o < 3; o++)
 #pragma unroll
                         for (int x = 0; x < 16; x++) sum[x] += red[(t * 3 + o) * 1024 + 64 * x + lane];
-                    store_tile(sum, c, n, (mt * MT + ii) * 32, tn * kBN + 32 * j, m, n, inv_scale, lane, accumulate != 0);
+                    if (part) store_tile_part(sum, part + (size_t)blockIdx.y * m * n, n, (mt * MT + ii) * 32, tn * kBN + 32 * j, m, n, lane);
+                    else store_tile(sum, c, n, (mt * MT + ii) * 32, tn * kBN + 32 * j, m, n, inv_scale, lane, accumulate != 0);
                 }
             }
     }
@@ -1928,7 +2029,7 @@ void gemm_q6k_tall_kernel(const u32x4* __restrict__ afrag, const uint8_t* __rest
 
 template <int MT>
 int launch_q6k_gemm(skn_ctx* ctx, const u32x4* afrag, const uint8_t* w, const float* isc, float* c, int m, int n, int k,
-                    int accumulate) {
+                    int accumulate, int splits, float* part) {
     constexpr int kLds = 2 * MT * 3 * 4096;
     const int m_tiles = (m + 32 * MT - 1) / (32 * MT), n_tiles = (n + kBN - 1) / kBN;
     const int xcd_rows = 8 % m_tiles == 0 ? 1 : 0;
@@ -1938,22 +2039,26 @@ int launch_q6k_gemm(skn_ctx* ctx, const u32x4* afrag, const uint8_t* w, const fl
     // 128-row tiles: the kernel with specialised wavefronts (measured 6 - 11 % faster); option value 2 keeps to the other
     // (up to 16384 elements per row: a rescale per superblock rounds the accumulators once more, the other form does not)
     if (MT == 4 && xcd_rows && k <= 16384 && ctx->opt_gemm_q6k_fused != 2) {
-        skn_launch(ctx, gemm_q6k_pc_kernel, dim3(grid), dim3(512), kQ6PcLds, afrag, w, isc, c, m, n, k, m_tiles, n_tiles, accumulate,
-                   a_bytes, w_bytes);
+        skn_launch(ctx, gemm_q6k_pc_kernel, dim3(grid, splits), dim3(512), kQ6PcLds, afrag, w, isc, c, m, n, k, m_tiles, n_tiles, accumulate,
+                   a_bytes, w_bytes, part);
         SKN_LAUNCH_CHECK(ctx);
         return SKN_OK;
     }
-    skn_launch(ctx, gemm_q6k_frag_kernel<MT>, dim3(grid), dim3(256), kLds, afrag, w, isc, c, m, n, k, m_tiles, n_tiles, accumulate,
-               a_bytes, w_bytes, xcd_rows);
+    skn_launch(ctx, gemm_q6k_frag_kernel<MT>, dim3(grid, splits), dim3(256), kLds, afrag, w, isc, c, m, n, k, m_tiles, n_tiles, accumulate,
+               a_bytes, w_bytes, xcd_rows, part);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
 
 int launch_q6k_gemm_mt(skn_ctx* ctx, int mt, const u32x4* afrag, const uint8_t* w, const float* isc, float* c, int m, int n,
-                       int k, int accumulate) {
-    if (mt == 1) return launch_q6k_gemm<1>(ctx, afrag, w, isc, c, m, n, k, accumulate);
-    if (mt == 2) return launch_q6k_gemm<2>(ctx, afrag, w, isc, c, m, n, k, accumulate);
-    return launch_q6k_gemm<4>(ctx, afrag, w, isc, c, m, n, k, accumulate);
+                       int k, int accumulate, int splits, float* part) {
+    if (splits < 2) part = nullptr;
+    if (mt == 1) SKN_TRY(launch_q6k_gemm<1>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part));
+    else if (mt == 2) SKN_TRY(launch_q6k_gemm<2>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part));
+    else SKN_TRY(launch_q6k_gemm<4>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part));
+    if (!part) return SKN_OK;
+    const PartSegs ps = {{c, nullptr, nullptr}, {n, 0, 0}, {0, 0, 0}, {accumulate, 0, 0}, 1, 0};
+    return launch_add_parts(ctx, part, splits, n, ps, isc, m);
 }
 
 // grows the context's GEMM workspace; the pointer stays valid until the next growth
@@ -2002,7 +2107,7 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
                 "Q4_K GEMM: bad segment count or shape");
     SKN_REQUIRE(ctx, !swiglu_pair || (nseg == 2 && segs[0].n == segs[1].n && !segs[0].accumulate), SKN_ERR_ARG,
                 "Q4_K GEMM: a SwiGLU pair is two matrices of the same shape");
-    Q4kFragSegs fs;
+    Q4kFragSegs fs = {};
     int tiles = 0;
     for (int i = 0; i < 3; i++) {
         const skn_gemm_seg& s = segs[i < nseg ? i : nseg - 1];
@@ -2047,9 +2152,20 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     SKN_REQUIRE(ctx, af_bytes < ((size_t)1 << 31), SKN_ERR_SHAPE,
                 "Q4_K GEMM: %d rows of %d activations exceed the 2^30 elements one call takes", m, k);
     const size_t is_bytes = align_up((size_t)m_pad * 4);
+    const int splits = tall ? 1 : k_splits(ctx, m, m_tiles * fs.n_tiles, k / 256);
+    PartSegs ps = {};
+    ps.count = nseg, ps.pair = fs.pair;
+    for (int i = 0; i < nseg; i++) {
+        ps.c[i] = segs[i].c, ps.n[i] = segs[i].n, ps.accumulate[i] = segs[i].accumulate;
+        ps.col0[i] = fs.part_cols;
+        fs.part_cols += segs[i].n;
+    }
+    for (int i = 0; i < 3; i++) fs.part_col0[i] = ps.col0[i];
+    const size_t part_bytes = splits > 1 ? (size_t)splits * m * fs.part_cols * 4 : 0;
     uint8_t* ws;
-    int rc = gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes, &ws);
+    int rc = gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes + part_bytes, &ws);
     if (rc != SKN_OK) return rc;
+    if (splits > 1) fs.part = (float*)(ws + af_bytes + sf_bytes + is_bytes);
     _Float16* afrag = (_Float16*)ws;
     _Float16* sfrag = (_Float16*)(ws + af_bytes);
     float* isc = (float*)(ws + af_bytes + sf_bytes);
@@ -2068,8 +2184,9 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
         SKN_LAUNCH_CHECK(ctx);
         return SKN_OK;
     }
-    if (mt_rows == 128) return launch_frag<2, 2>(ctx, m_tiles, (const u32x4*)afrag, (const u32x4*)sfrag, fs, isc, m, k);
-    return launch_frag<2, 1>(ctx, m_tiles, (const u32x4*)afrag, (const u32x4*)sfrag, fs, isc, m, k);
+    if (mt_rows == 128) SKN_TRY((launch_frag<2, 2>(ctx, m_tiles, (const u32x4*)afrag, (const u32x4*)sfrag, fs, isc, m, k, splits)));
+    else SKN_TRY((launch_frag<2, 1>(ctx, m_tiles, (const u32x4*)afrag, (const u32x4*)sfrag, fs, isc, m, k, splits)));
+    return splits > 1 ? launch_add_parts(ctx, fs.part, splits, fs.part_cols, ps, isc, m) : SKN_OK;
 }
 
 extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n, int k, const uint16_t* a_bf16_dev,
@@ -2154,11 +2271,19 @@ int skn_gemm_q6k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     const int m_rows = any_wide ? 256 : 32 * mt;
     const int m_pad = (m + m_rows - 1) / m_rows * m_rows;
     const size_t af_bytes = align_up((size_t)m_pad * k * 2), is_bytes = align_up((size_t)m_pad * 4);
+    int splits[3] = {1, 1, 1};
+    size_t part_bytes = 0;  // (the matrices' products run one after the other: they share the room for their parts)
+    for (int i = 0; i < nseg; i++) {
+        if (q6k_wide_tiles(ctx, segs[i].n, k, m)) continue;
+        splits[i] = k_splits(ctx, m, ((m + 32 * mt - 1) / (32 * mt)) * ((segs[i].n + kBN - 1) / kBN), k / 256);
+        if (splits[i] > 1) part_bytes = std::max(part_bytes, (size_t)splits[i] * m * segs[i].n * 4);
+    }
     uint8_t* ws;
-    int rc = gemm_workspace(ctx, af_bytes + is_bytes, &ws);
+    int rc = gemm_workspace(ctx, af_bytes + is_bytes + part_bytes, &ws);
     if (rc != SKN_OK) return rc;
     _Float16* afrag = (_Float16*)ws;
     float* isc = (float*)(ws + af_bytes);
+    float* part = (float*)(ws + af_bytes + is_bytes);
     _Float16* no_sums = nullptr;
     switch (src.kind) {
         case SKN_SRC_BF16: launch_prep<SKN_SRC_BF16, false>(ctx, src, afrag, isc, no_sums, m, m_pad, k); break;
@@ -2176,7 +2301,7 @@ int skn_gemm_q6k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
                        (uint32_t)((size_t)n * (k / 256) * 210));
             SKN_LAUNCH_CHECK(ctx);
         } else {
-            rc = launch_q6k_gemm_mt(ctx, mt, (const u32x4*)afrag, (const uint8_t*)segs[i].w, isc, segs[i].c, m, n, k, segs[i].accumulate);
+            rc = launch_q6k_gemm_mt(ctx, mt, (const u32x4*)afrag, (const uint8_t*)segs[i].w, isc, segs[i].c, m, n, k, segs[i].accumulate, splits[i], part);
             if (rc != SKN_OK) return rc;
         }
     }

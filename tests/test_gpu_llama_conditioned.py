@@ -108,6 +108,23 @@ def test_prompt_with_the_wide_tile_gemm_forced(hip, case):
         hip.set_option("gemm.tile", 0)
 
 
+@pytest.mark.parametrize("case", ["q4_k", "q4_k_kv2", "mixed", "q6_k"])
+def test_prompt_with_k_split_over_workgroups(hip, case):
+    """The prompt's products with the k of a tile divided over two workgroups (the library does it by itself from five
+    superblocks on): the addition of the parts stores q, k, v into three buffers, adds a residual, multiplies silu(gate) by up."""
+    cfg = CASES[case]
+    prompt, first, _, _ = _oracle_prompt(case, 41, 12)
+    hip.set_option("gemm.split", 2)
+    try:
+        model = llama.LlamaModel(hip, cfg, weights=llama.conditioned_weights(cfg, SEED))
+        model.prefill(prompt)
+        err = logit_err(model.logits(), first)
+        assert err <= PROMPT_TOL, (case, err)
+        model.free()
+    finally:
+        hip.set_option("gemm.split", 0)
+
+
 @pytest.mark.parametrize("fused,graph", [(1, 1), (0, 0)])
 @pytest.mark.parametrize("case", list(CASES))
 def test_41_token_prompt_then_decode_steps(hip, case, fused, graph):
