@@ -15,8 +15,12 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kThreads = 1024, kWaves = kThreads / 64;
-constexpr int kR = 1;  // rows per wavefront and turn (measured with two as well: slower at 1024 threads)
+// Eight wavefronts per workgroup: a matrix of 2048 rows then reaches 256 compute units (sixteen: half of them), and up to three
+// workgroups share a compute unit.  A decode step of eight layers of width 2048 (945 MB of weights, 27 launches): 313 us; one
+// workgroup of sixteen wavefronts per compute unit 330, two of them 341; eight wavefronts, one / two / four workgroups per compute
+// unit 327 / 319 / 338; four wavefronts, two / four / six / eight workgroups 342 / 335 / 331 / 351.
+constexpr int kThreads = 512, kWaves = kThreads / 64, kPerCu = 3;
+constexpr int kR = 1;  // rows per wavefront and turn (measured with two as well: slower)
 constexpr int kU = 4;  // 16-byte pieces per row and lane in flight, twice
 constexpr int kMaxGroups = 256, kMaxMerge = 4096, kMaxSplits = 16;  // norm groups; heads x splits and splits of a merge
 
@@ -323,8 +327,9 @@ int launch(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, cons
     const size_t scratch = MODE == SKN_XSRC_GROUP_NORM || MODE == SKN_XSRC_ADD_NORM ? (kMaxGroups + 16 * kWaves) * 4 : MODE == SKN_XSRC_MERGE ? (size_t)src.heads * src.splits * 4 : 0;
     const size_t lds = (size_t)plane * 32 + scratch;
     SKN_REQUIRE(ctx, lds <= kMaxLds, SKN_ERR_SHAPE, "dense matvec: %d columns need %zu bytes of LDS (at most %d)", w.k_pad, lds, kMaxLds);
-    // one workgroup per compute unit at most: its staging serves all the rows its wavefronts walk through
-    const int groups = (w.rows + kR - 1) / kR, blocks = std::min((groups + kWaves - 1) / kWaves, ctx->compute_units);
+    // no more workgroups than fit on the device at once: a staging serves all the rows its wavefronts walk through
+    const int groups = (w.rows + kR - 1) / kR, per_cu = std::min(kPerCu, (int)(kMaxLds / lds));
+    const int blocks = std::min((groups + kWaves - 1) / kWaves, per_cu * ctx->compute_units);
     skn_launch(ctx, dense_matvec_kernel<W, MODE>, dim3((unsigned)blocks), dim3(kThreads), lds, (const W*)w.w, w.rows, w.k_pad, plane, w.bias, src, out);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
