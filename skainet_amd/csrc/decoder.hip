@@ -3,6 +3,7 @@
 // x += Wdown . (silu(Wgate xn) * (Wup xn)).  Logits = Whead . rmsnorm(x).
 // The decode loop around a step (device scalars, greedy choice, captured graph) is csrc/stepper.h.
 #include "kv.h"
+#include "gemm_blocks.h"
 #include "gemm_q6k.h"
 #include "stepper.h"
 
@@ -499,32 +500,33 @@ static int expanded_copy(skn_ctx* ctx, skn_llama* m, int l, int which, int type,
 }
 
 // Prompt rows times up to three matrices of any formats, one activation source (fp32 rows, with RMSNorm when norm_w
-// is given).  Q4_K and Q6_K matrices go behind the fused activation pass of their GEMMs -- the row-wise work inside
-// the pass, one pass per format, a residual (`accumulate`) in the store --, the others through a norm, a bf16
-// conversion, skn_gemm_q per matrix and an add.
+// is given).  Matrices whose GEMM unpacks the blocks itself (Q4_K, Q6_K, the formats in blocks of 32) go behind its fused
+// activation pass -- the row-wise work inside the pass, one pass per kind of GEMM, a residual (`accumulate`) in the store --,
+// the others through a norm, a bf16 conversion, skn_gemm_q per matrix and an add.
 int project_rows(skn_ctx* ctx, skn_llama* m, const int* types, const void* const* blocks, const int* rows, float* const* outs,
                  int count, int k, const float* x, const float* norm_w, int T, int accumulate) {
     const skn_llama_config& c = m->cfg;
     const skn_gemm_src src = {norm_w ? SKN_SRC_RMSNORM : SKN_SRC_F32, x, norm_w, norm_w ? c.rms_eps : 0.f};
-    skn_gemm_seg q4[3], q6[3];
-    int n4 = 0, n6 = 0;
-    bool plain = false;
+    skn_gemm_seg q4[3], q6[3], bl[3];
+    int n4 = 0, n6 = 0, nbl = 0, np = 0, bl_types[3], plain[3];
     for (int i = 0; i < count; i++) {
-        if (types[i] == SKN_TYPE_Q4_K && k <= 16384) q4[n4++] = {blocks[i], rows[i], outs[i], accumulate};
-        else if (types[i] == SKN_TYPE_Q6_K && skn_gemm_q6k_direct_ok(ctx, rows[i], k, T)) q6[n6++] = {blocks[i], rows[i], outs[i], accumulate};
-        else plain = true;
+        const skn_gemm_seg seg = {blocks[i], rows[i], outs[i], accumulate};
+        if (types[i] == SKN_TYPE_Q4_K && k <= 16384) q4[n4++] = seg;
+        else if (types[i] == SKN_TYPE_Q6_K && skn_gemm_q6k_direct_ok(ctx, rows[i], k, T)) q6[n6++] = seg;
+        else if (skn_gemm_blocks_ok(ctx, types[i], blocks[i], rows[i], k, T)) bl_types[nbl] = types[i], bl[nbl++] = seg;
+        else plain[np++] = i;
     }
     if (n4) SKN_TRY(skn_gemm_q4k_multi(ctx, q4, n4, k, src, T));
     if (n6) SKN_TRY(skn_gemm_q6k_multi(ctx, q6, n6, k, src, T));
-    if (!plain) return SKN_OK;
+    if (nbl) SKN_TRY(skn_gemm_blocks_multi(ctx, bl_types, bl, nbl, k, src, T));
+    if (!np) return SKN_OK;
     if (norm_w) {
         skn_launch(ctx, rmsnorm_rows_kernel, dim3(T), dim3(256), 0, x, norm_w, m->pxn, k, c.rms_eps);
         SKN_LAUNCH_CHECK(ctx);
     }
     SKN_TRY(to_bf16(ctx, norm_w ? m->pxn : x, m->pb16, (int64_t)T * k));
-    for (int i = 0; i < count; i++) {
-        const bool fused = (types[i] == SKN_TYPE_Q4_K && k <= 16384) || (types[i] == SKN_TYPE_Q6_K && skn_gemm_q6k_direct_ok(ctx, rows[i], k, T));
-        if (fused) continue;
+    for (int j = 0; j < np; j++) {
+        const int i = plain[j];
         if (accumulate) {
             SKN_TRY(skn_gemm_q(ctx, types[i], blocks[i], rows[i], k, m->pb16, T, m->pproj));
             skn_launch(ctx, add_rows_kernel, dim3(nblk((int64_t)T * rows[i])), dim3(256), 0, outs[i], (const float*)m->pproj,
@@ -534,6 +536,35 @@ int project_rows(skn_ctx* ctx, skn_llama* m, const int* types, const void* const
             SKN_TRY(skn_gemm_q(ctx, types[i], blocks[i], rows[i], k, m->pb16, T, outs[i]));
         }
     }
+    return SKN_OK;
+}
+
+// The same with the option llama.expand_weights: Q4_K matrices on their own kernel, the others through their kept copies
+// (`which`: the first matrix's place among a layer's seven), except that up to 256 rows the formats in blocks of 32 are faster from
+// their blocks (us per call, Q8_0, blocks | copy: 120 x 4096 x 4096 21.7 | 32, 333 x 4096 x 4096 38.7 | 34).
+static int project_expanded(skn_ctx* ctx, skn_llama* m, int l, int which, const int* types, const void* const* blocks, const int* rows, float* const* outs,
+                            int count, int k, const float* x, const float* norm_w, int T, int accumulate) {
+    const skn_gemm_src src = {norm_w ? SKN_SRC_RMSNORM : SKN_SRC_F32, x, norm_w, norm_w ? m->cfg.rms_eps : 0.f};
+    skn_gemm_seg q4[3], ex[3], bl[3];
+    int n4 = 0, nx = 0, nbl = 0, bl_types[3];
+    for (int i = 0; i < count; i++) {
+        skn_gemm_seg seg = {blocks[i], rows[i], outs[i], accumulate};
+        if (types[i] == SKN_TYPE_Q4_K && k <= 16384) {
+            q4[n4++] = seg;
+            continue;
+        }
+        const void* copy;
+        SKN_TRY(expanded_copy(ctx, m, l, which + i, types[i], blocks[i], rows[i], k, &copy));
+        if (T <= 256 && skn_gemm_blocks_ok(ctx, types[i], blocks[i], rows[i], k, T)) {
+            bl_types[nbl] = types[i], bl[nbl++] = seg;
+        } else {
+            seg.w = copy;
+            ex[nx++] = seg;
+        }
+    }
+    if (n4) SKN_TRY(skn_gemm_q4k_multi(ctx, q4, n4, k, src, T));
+    if (nx) SKN_TRY(skn_gemm_expanded_multi(ctx, ex, nx, k, src, T));
+    if (nbl) SKN_TRY(skn_gemm_blocks_multi(ctx, bl_types, bl, nbl, k, src, T));
     return SKN_OK;
 }
 
@@ -578,29 +609,12 @@ int skn_llama_prefill(skn_ctx* ctx, skn_llama* m, const int32_t* tokens_host, in
             const skn_gemm_seg qkv[3] = {{L.wq, H, m->pq, 0}, {L.wk, KVD, m->pk, 0}, {L.wv, KVD, m->pv, 0}};
             const skn_gemm_src src = {SKN_SRC_RMSNORM, m->px, L.attn_norm, c.rms_eps};
             SKN_TRY(skn_gemm_q4k_multi(ctx, qkv, 3, H, src, T));
-        } else if (expand) {  // Q4_K matrices of the group on their own kernel, the others through their kept copies
-            const int types[3] = {L.type_q, L.type_k, L.type_v}, rows[3] = {H, KVD, KVD};
-            const void* blocks[3] = {L.wq, L.wk, L.wv};
-            float* outs[3] = {m->pq, m->pk, m->pv};
-            skn_gemm_seg q4[3], ex[3];
-            int n4 = 0, nx = 0;
-            for (int i = 0; i < 3; i++) {
-                if (types[i] == SKN_TYPE_Q4_K && H <= 16384) {
-                    q4[n4++] = {blocks[i], rows[i], outs[i], 0};
-                } else {
-                    ex[nx] = {nullptr, rows[i], outs[i], 0};
-                    SKN_TRY(expanded_copy(ctx, m, l, i, types[i], blocks[i], rows[i], H, &ex[nx].w));
-                    nx++;
-                }
-            }
-            const skn_gemm_src src = {SKN_SRC_RMSNORM, m->px, L.attn_norm, c.rms_eps};
-            if (n4) SKN_TRY(skn_gemm_q4k_multi(ctx, q4, n4, H, src, T));
-            if (nx) SKN_TRY(skn_gemm_expanded_multi(ctx, ex, nx, H, src, T));
         } else {
             const int types[3] = {L.type_q, L.type_k, L.type_v}, rows[3] = {H, KVD, KVD};
             const void* blocks[3] = {L.wq, L.wk, L.wv};
             float* outs[3] = {m->pq, m->pk, m->pv};
-            SKN_TRY(project_rows(ctx, m, types, blocks, rows, outs, 3, H, m->px, L.attn_norm, T, 0));
+            if (expand) SKN_TRY(project_expanded(ctx, m, l, 0, types, blocks, rows, outs, 3, H, m->px, L.attn_norm, T, 0));
+            else SKN_TRY(project_rows(ctx, m, types, blocks, rows, outs, 3, H, m->px, L.attn_norm, T, 0));
         }
         skn_launch(ctx, rope_store_kernel, dim3(T, NH), dim3(D / 2), 0, m->pq, (const float*)m->pk, (const float*)m->pv,
                    kv->k_pool, kv->v_pool, (const int32_t*)kv->page_table_dev, (const int32_t*)(m->step.state + 1), NH, KVH, D,
@@ -615,42 +629,22 @@ int skn_llama_prefill(skn_ctx* ctx, skn_llama* m, const int32_t* tokens_host, in
             const skn_gemm_seg wo = {L.wo, H, m->px, 1};
             const skn_gemm_src src = {SKN_SRC_F32, m->patt, nullptr, 0.f};
             SKN_TRY(skn_gemm_q4k_multi(ctx, &wo, 1, H, src, T));
-        } else if (expand) {
-            skn_gemm_seg wo = {nullptr, H, m->px, 1};
-            SKN_TRY(expanded_copy(ctx, m, l, 3, L.type_o, L.wo, H, H, &wo.w));
-            const skn_gemm_src src = {SKN_SRC_F32, m->patt, nullptr, 0.f};
-            SKN_TRY(skn_gemm_expanded_multi(ctx, &wo, 1, H, src, T));
         } else {
             const void* blocks[1] = {L.wo};
             float* outs[1] = {m->px};
-            SKN_TRY(project_rows(ctx, m, &L.type_o, blocks, &H, outs, 1, H, m->patt, nullptr, T, 1));
+            if (expand) SKN_TRY(project_expanded(ctx, m, l, 3, &L.type_o, blocks, &H, outs, 1, H, m->patt, nullptr, T, 1));
+            else SKN_TRY(project_rows(ctx, m, &L.type_o, blocks, &H, outs, 1, H, m->patt, nullptr, T, 1));
         }
         if (q4k_gu) {  // RMSNorm inside the activation pass, SwiGLU inside the store: gate and up never reach memory
             const skn_gemm_seg gu[2] = {{L.w_gate, F, m->pmid, 0}, {L.w_up, F, m->pmid, 0}};
             const skn_gemm_src src = {SKN_SRC_RMSNORM, m->px, L.ffn_norm, c.rms_eps};
             SKN_TRY(skn_gemm_q4k_multi(ctx, gu, 2, H, src, T, true));
-        } else if (expand) {
-            const int types[2] = {L.type_gate, L.type_up};
-            const void* blocks[2] = {L.w_gate, L.w_up};
-            float* outs[2] = {m->pgate, m->pup};
-            const skn_gemm_src src = {SKN_SRC_RMSNORM, m->px, L.ffn_norm, c.rms_eps};
-            for (int i = 0; i < 2; i++) {
-                skn_gemm_seg seg = {blocks[i], F, outs[i], 0};
-                if (types[i] == SKN_TYPE_Q4_K && H <= 16384) {
-                    SKN_TRY(skn_gemm_q4k_multi(ctx, &seg, 1, H, src, T));
-                } else {
-                    SKN_TRY(expanded_copy(ctx, m, l, 4 + i, types[i], blocks[i], F, H, &seg.w));
-                    SKN_TRY(skn_gemm_expanded_multi(ctx, &seg, 1, H, src, T));
-                }
-            }
-            skn_launch(ctx, swiglu_rows_kernel, dim3(nblk((int64_t)T * F)), dim3(256), 0, (const float*)m->pgate,
-                       (const float*)m->pup, m->pmid, (int64_t)T * F);
-            SKN_LAUNCH_CHECK(ctx);
         } else {
             const int types[2] = {L.type_gate, L.type_up}, rows[2] = {F, F};
             const void* blocks[2] = {L.w_gate, L.w_up};
             float* outs[2] = {m->pgate, m->pup};
-            SKN_TRY(project_rows(ctx, m, types, blocks, rows, outs, 2, H, m->px, L.ffn_norm, T, 0));
+            if (expand) SKN_TRY(project_expanded(ctx, m, l, 4, types, blocks, rows, outs, 2, H, m->px, L.ffn_norm, T, 0));
+            else SKN_TRY(project_rows(ctx, m, types, blocks, rows, outs, 2, H, m->px, L.ffn_norm, T, 0));
             skn_launch(ctx, swiglu_rows_kernel, dim3(nblk((int64_t)T * F)), dim3(256), 0, (const float*)m->pgate,
                        (const float*)m->pup, m->pmid, (int64_t)T * F);
             SKN_LAUNCH_CHECK(ctx);
@@ -659,15 +653,11 @@ int skn_llama_prefill(skn_ctx* ctx, skn_llama* m, const int32_t* tokens_host, in
             const skn_gemm_seg down = {L.w_down, H, m->px, 1};  // residual added by the store
             const skn_gemm_src mid = {SKN_SRC_F32, m->pmid, nullptr, 0.f};
             SKN_TRY(skn_gemm_q4k_multi(ctx, &down, 1, F, mid, T));
-        } else if (expand) {
-            skn_gemm_seg down = {nullptr, H, m->px, 1};
-            SKN_TRY(expanded_copy(ctx, m, l, 6, L.type_down, L.w_down, H, F, &down.w));
-            const skn_gemm_src mid = {SKN_SRC_F32, m->pmid, nullptr, 0.f};
-            SKN_TRY(skn_gemm_expanded_multi(ctx, &down, 1, F, mid, T));
         } else {
             const void* blocks[1] = {L.w_down};
             float* outs[1] = {m->px};
-            SKN_TRY(project_rows(ctx, m, &L.type_down, blocks, &H, outs, 1, F, m->pmid, nullptr, T, 1));
+            if (expand) SKN_TRY(project_expanded(ctx, m, l, 6, &L.type_down, blocks, &H, outs, 1, F, m->pmid, nullptr, T, 1));
+            else SKN_TRY(project_rows(ctx, m, &L.type_down, blocks, &H, outs, 1, F, m->pmid, nullptr, T, 1));
         }
         // the cache of this layer now holds pos0 + T tokens
         kv->len[0] = pos0 + T;

@@ -17,60 +17,14 @@
 //     integers below 2^10, exact in fp16, so one MFMA per k-step suffices; the f16 superblock scale d is the
 //     unit in which a column's accumulators are kept.
 #include "common.h"
+#include "gemm_blocks.h"
 #include "gemm_q6k.h"
+#include "gemm_tiles.h"
 
 #include <algorithm>
 #include <type_traits>
 
 namespace {
-
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
-
-constexpr int kBN = 64;   // workgroup tile columns (weight rows)
-
-// C tile store: acc register r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32 of the 32x32 tile
-__device__ __forceinline__ void store_tile(const float16_t& acc, float* __restrict__ c, int ldc, int row0, int col0,
-                                           int m, int n, const float* __restrict__ inv_scale, int lane,
-                                           bool accumulate = false) {
-    const int col = col0 + (lane & 31);
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row < m && col < n) {
-            float* dst = c + (size_t)row * ldc + col;
-            *dst = accumulate ? *dst + acc[r] * inv_scale[row] : acc[r] * inv_scale[row];
-        }
-    }
-}
-
-// the same with the sixteen row scales in hand (sc[r]: the scale of the row that register r holds)
-__device__ __forceinline__ void store_tile_scaled(const float16_t& acc, float* __restrict__ c, int ldc, int row0, int col0,
-                                                  int m, int n, const float (&sc)[16], int lane, bool accumulate) {
-    const int col = col0 + (lane & 31);
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row < m && col < n) {
-            float* dst = c + (size_t)row * ldc + col;
-            *dst = accumulate ? *dst + acc[r] * sc[r] : acc[r] * sc[r];
-        }
-    }
-}
-
-// a partial tile of a workgroup that holds a part of k: no scale, rows of ldc
-__device__ __forceinline__ void store_tile_part(const float16_t& acc, float* __restrict__ part, int ldc, int row0, int col0, int m, int n, int lane) {
-    const int col = col0 + (lane & 31);
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row < m && col < n) part[(size_t)row * ldc + col] = acc[r];
-    }
-}
 
 // ---- Q4_K path: weights unpacked in the kernel, one MFMA per k-step, operands loaded by the wavefronts ------
 // Workgroup of eight wavefronts, tile (64 MT) x 64.  The tile is divided in two along m; along k it is not
@@ -107,11 +61,6 @@ struct PrepRow {
     const void* b;   // SKN_SRC_RMSNORM: the norm weights
     float r;         // SKN_SRC_RMSNORM: 1 / sqrt(mean(x^2) + eps)
 };
-
-__device__ __forceinline__ uint32_t bf16_rne(float f) {
-    const uint32_t u = __float_as_uint(f);
-    return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
-}
 
 // elements [i, i + 4) of the row as four bf16 bit patterns in two words
 template <int SRC>
@@ -715,14 +664,8 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
 // Where the tiles leave compute units idle, k is divided over `splits` workgroups per tile as well; each leaves its
 // unscaled partial products in the workspace and this kernel adds them in a fixed order, applies the row scale and does
 // what the store would have done (add into c, or silu(gate) * up of a pair).
-struct PartSegs {
-    float* c[3];
-    int n[3], col0[3], accumulate[3];
-    int count, pair;
-};
-
 template <int W>  // columns per thread: 4, or 1 where a matrix has a number of columns that is no multiple of 4
-__global__ __launch_bounds__(256) void gemm_add_parts_kernel(const float* __restrict__ part, int splits, int cols, const PartSegs segs,
+__global__ __launch_bounds__(256) void gemm_add_parts_kernel(const float* __restrict__ part, int splits, int cols, const skn_gemm_parts segs,
                                                             const float* __restrict__ inv_scale, int m) {
     const int row = blockIdx.y, col = (blockIdx.x * 256 + threadIdx.x) * W;
     if (col >= (segs.pair ? segs.n[0] : cols)) return;
@@ -754,28 +697,6 @@ __global__ __launch_bounds__(256) void gemm_add_parts_kernel(const float* __rest
     const int i = segs.count > 2 && col >= segs.col0[2] ? 2 : (segs.count > 1 && col >= segs.col0[1] ? 1 : 0);
     vec* dst = reinterpret_cast<vec*>(segs.c[i] + (size_t)row * segs.n[i] + (col - segs.col0[i]));
     *dst = segs.accumulate[i] ? *dst + v : v;
-}
-
-int launch_add_parts(skn_ctx* ctx, const float* part, int splits, int cols, const PartSegs& segs, const float* isc, int m) {
-    bool wide = true;
-    for (int i = 0; i < segs.count; i++) wide = wide && segs.n[i] % 4 == 0 && ((uintptr_t)segs.c[i] & 15) == 0;
-    const int n = segs.pair ? segs.n[0] : cols;
-    if (wide) skn_launch(ctx, gemm_add_parts_kernel<4>, dim3((n / 4 + 255) / 256, m), dim3(256), 0, part, splits, cols, segs, isc, m);
-    else skn_launch(ctx, gemm_add_parts_kernel<1>, dim3((n + 255) / 256, m), dim3(256), 0, part, splits, cols, segs, isc, m);
-    SKN_LAUNCH_CHECK(ctx);
-    return SKN_OK;
-}
-
-// How many workgroups share a tile's k: as many as there are compute units for, at least one superblock for each of a
-// workgroup's four k-parts.  us per call, unsplit -> chosen: Q6_K 41 x 4096 x 11008 (64 tiles) 81 -> 34.5, 120 x 4096 x 11008
-// 106 -> 45, 200 x 4096 x 11008 (128 tiles) 108 -> 71; Q4_K 41 x 4096 x 11008 35.7 -> 24.6, 41 x 4096 x 4096 17.8 -> 15.1,
-// 200 x 4096 x 4096 25.9 -> 24.8.  Filling every compute unit twice is no gain (Q4_K 41 x 4096 x 11008 27.2, 120 x 4096 x 4096
-// 21.5 against 18.7), nor is a second part for tiles that fill two thirds of the device (Q4_K 41 x 11008 x 4096 22.2 against
-// 19.6, Q6_K 333 x 4096 x 4096 59 against 54): the addition costs 3 us and the parts their way through memory.
-int k_splits(const skn_ctx* ctx, int m, int tiles, int nb) {
-    if (m > 65535) return 1;  // (a grid dimension of the addition)
-    if (ctx->opt_gemm_split > 0) return std::min(ctx->opt_gemm_split, nb);
-    return std::max(1, std::min({ctx->compute_units / tiles, (nb + 3) / 4, 16}));
 }
 
 template <int MT, int MH>
@@ -1247,9 +1168,6 @@ int launch_hilo_gemm(skn_ctx* ctx, const u32x4* afrag, const u32x4* bfrag, const
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
-
-// row blocks per tile of the general path: 32 MT rows
-inline int hilo_mt(int m) { return m <= 32 ? 1 : (m <= 64 ? 2 : 4); }
 
 int launch_hilo_gemm_mt(skn_ctx* ctx, int mt, const u32x4* afrag, const u32x4* bfrag, const float* isc, float* c, int m, int n,
                         int k, int accumulate) {
@@ -2057,12 +1975,35 @@ int launch_q6k_gemm_mt(skn_ctx* ctx, int mt, const u32x4* afrag, const uint8_t* 
     else if (mt == 2) SKN_TRY(launch_q6k_gemm<2>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part));
     else SKN_TRY(launch_q6k_gemm<4>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part));
     if (!part) return SKN_OK;
-    const PartSegs ps = {{c, nullptr, nullptr}, {n, 0, 0}, {0, 0, 0}, {accumulate, 0, 0}, 1, 0};
-    return launch_add_parts(ctx, part, splits, n, ps, isc, m);
+    const skn_gemm_parts ps = {{c, nullptr, nullptr}, {n, 0, 0}, {0, 0, 0}, {accumulate, 0, 0}, 1, 0};
+    return skn_gemm_add_parts(ctx, part, splits, n, ps, isc, m);
 }
 
-// grows the context's GEMM workspace; the pointer stays valid until the next growth
-int gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out) {
+}  // namespace
+
+int skn_gemm_add_parts(skn_ctx* ctx, const float* part, int splits, int cols, const skn_gemm_parts& segs, const float* isc, int m) {
+    bool wide = true;
+    for (int i = 0; i < segs.count; i++) wide = wide && segs.n[i] % 4 == 0 && ((uintptr_t)segs.c[i] & 15) == 0;
+    const int n = segs.pair ? segs.n[0] : cols;
+    if (wide) skn_launch(ctx, gemm_add_parts_kernel<4>, dim3((n / 4 + 255) / 256, m), dim3(256), 0, part, splits, cols, segs, isc, m);
+    else skn_launch(ctx, gemm_add_parts_kernel<1>, dim3((n + 255) / 256, m), dim3(256), 0, part, splits, cols, segs, isc, m);
+    SKN_LAUNCH_CHECK(ctx);
+    return SKN_OK;
+}
+
+// How many workgroups share a tile's k: as many as there are compute units for, at least one superblock for each of a
+// workgroup's four k-parts.  us per call, unsplit -> chosen: Q6_K 41 x 4096 x 11008 (64 tiles) 81 -> 34.5, 120 x 4096 x 11008
+// 106 -> 45, 200 x 4096 x 11008 (128 tiles) 108 -> 71; Q4_K 41 x 4096 x 11008 35.7 -> 24.6, 41 x 4096 x 4096 17.8 -> 15.1,
+// 200 x 4096 x 4096 25.9 -> 24.8.  Filling every compute unit twice is no gain (Q4_K 41 x 4096 x 11008 27.2, 120 x 4096 x 4096
+// 21.5 against 18.7), nor is a second part for tiles that fill two thirds of the device (Q4_K 41 x 11008 x 4096 22.2 against
+// 19.6, Q6_K 333 x 4096 x 4096 59 against 54): the addition costs 3 us and the parts their way through memory.
+int skn_gemm_k_splits(const skn_ctx* ctx, int m, int tiles, int nb) {
+    if (m > 65535) return 1;  // (a grid dimension of the addition)
+    if (ctx->opt_gemm_split > 0) return std::min(ctx->opt_gemm_split, nb);
+    return std::max(1, std::min({ctx->compute_units / tiles, (nb + 3) / 4, 16}));
+}
+
+int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out) {
     if (bytes > ctx->gemm_ws_bytes) {
         SKN_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (ctx->gemm_ws) SKN_HIP(ctx, hipFree(ctx->gemm_ws));
@@ -2078,10 +2019,6 @@ int gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out) {
     *out = (uint8_t*)ctx->gemm_ws;
     return SKN_OK;
 }
-
-inline size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
-
-}  // namespace
 
 // Dynamic LDS above 48 KiB must be allowed per kernel and device; done once per context here so that no launch
 // path has to.
@@ -2148,12 +2085,12 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
                              (ctx->opt_gemm_tile == 0 && (m <= 128 || ((m + 127) / 128) * n_tiles_all > ctx->compute_units)));
     const int mt_rows = tall ? 256 : small_tiles ? 64 : 128;
     const int m_tiles = (m + mt_rows - 1) / mt_rows, m_pad = m_tiles * mt_rows;
-    const size_t af_bytes = align_up((size_t)m_pad * k * 2), sf_bytes = align_up((size_t)m_pad * (k / 256) * 16 * 2);
+    const size_t af_bytes = skn_align_up((size_t)m_pad * k * 2), sf_bytes = skn_align_up((size_t)m_pad * (k / 256) * 16 * 2);
     SKN_REQUIRE(ctx, af_bytes < ((size_t)1 << 31), SKN_ERR_SHAPE,
                 "Q4_K GEMM: %d rows of %d activations exceed the 2^30 elements one call takes", m, k);
-    const size_t is_bytes = align_up((size_t)m_pad * 4);
-    const int splits = tall ? 1 : k_splits(ctx, m, m_tiles * fs.n_tiles, k / 256);
-    PartSegs ps = {};
+    const size_t is_bytes = skn_align_up((size_t)m_pad * 4);
+    const int splits = tall ? 1 : skn_gemm_k_splits(ctx, m, m_tiles * fs.n_tiles, k / 256);
+    skn_gemm_parts ps = {};
     ps.count = nseg, ps.pair = fs.pair;
     for (int i = 0; i < nseg; i++) {
         ps.c[i] = segs[i].c, ps.n[i] = segs[i].n, ps.accumulate[i] = segs[i].accumulate;
@@ -2163,7 +2100,7 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     for (int i = 0; i < 3; i++) fs.part_col0[i] = ps.col0[i];
     const size_t part_bytes = splits > 1 ? (size_t)splits * m * fs.part_cols * 4 : 0;
     uint8_t* ws;
-    int rc = gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes + part_bytes, &ws);
+    int rc = skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes + part_bytes, &ws);
     if (rc != SKN_OK) return rc;
     if (splits > 1) fs.part = (float*)(ws + af_bytes + sf_bytes + is_bytes);
     _Float16* afrag = (_Float16*)ws;
@@ -2186,7 +2123,7 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     }
     if (mt_rows == 128) SKN_TRY((launch_frag<2, 2>(ctx, m_tiles, (const u32x4*)afrag, (const u32x4*)sfrag, fs, isc, m, k, splits)));
     else SKN_TRY((launch_frag<2, 1>(ctx, m_tiles, (const u32x4*)afrag, (const u32x4*)sfrag, fs, isc, m, k, splits)));
-    return splits > 1 ? launch_add_parts(ctx, fs.part, splits, fs.part_cols, ps, isc, m) : SKN_OK;
+    return splits > 1 ? skn_gemm_add_parts(ctx, fs.part, splits, fs.part_cols, ps, isc, m) : SKN_OK;
 }
 
 extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n, int k, const uint16_t* a_bf16_dev,
@@ -2209,6 +2146,10 @@ extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n,
                     "skn_gemm_q: Q4_K weights must be 16-byte aligned, activations 8-byte aligned");
         const skn_gemm_seg seg = {w_dev, n, c_dev, 0};
         const skn_gemm_src src = {SKN_SRC_BF16, a_bf16_dev, nullptr, 0.f};
+        // up to 32 rows: the kernel for blocks of 32, whose tile has as many (us per call, this | that: 2 x 4096 x 4096 14.2 | 12.8, 16 x
+        // 4096 x 4096 14.3 | 12.3, 8 x 1000 x 2048 12.5 | 10.7; on two row blocks 41 x 4096 x 4096 15.2 | 14.9, 64 x 11008 x 4096 20.1 | 23.8)
+        if (ctx->opt_gemm_tile == 0 && m <= 32 && skn_gemm_blocks_ok(ctx, ggml_type, w_dev, n, k, m))
+            return skn_gemm_blocks_multi(ctx, &ggml_type, &seg, 1, k, src, m);
         return skn_gemm_q4k_multi(ctx, &seg, 1, k, src, m);
     }
 
@@ -2221,11 +2162,16 @@ extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n,
         const skn_gemm_seg seg = {w_dev, n, c_dev, 0};
         return skn_gemm_q6k_multi(ctx, &seg, 1, k, src, m);
     }
-    const int mt = hilo_mt(m);
+    // formats in blocks of 32: likewise
+    if (skn_gemm_blocks_ok(ctx, ggml_type, w_dev, n, k, m)) {
+        const skn_gemm_seg seg = {w_dev, n, c_dev, 0};
+        return skn_gemm_blocks_multi(ctx, &ggml_type, &seg, 1, k, src, m);
+    }
+    const int mt = skn_gemm_mt(m);
     const int m_pad = (m + 32 * mt - 1) / (32 * mt) * (32 * mt), n_pad = (n + kBN - 1) / kBN * kBN;
-    const size_t af_bytes = align_up((size_t)m_pad * k * 2), is_bytes = align_up((size_t)m_pad * 4);
+    const size_t af_bytes = skn_align_up((size_t)m_pad * k * 2), is_bytes = skn_align_up((size_t)m_pad * 4);
     uint8_t* ws;
-    int rc = gemm_workspace(ctx, af_bytes + is_bytes + (size_t)n_pad * k * 4, &ws);
+    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes + (size_t)n_pad * k * 4, &ws);
     if (rc != SKN_OK) return rc;
     _Float16* afrag = (_Float16*)ws;
     float* isc = (float*)(ws + af_bytes);
@@ -2267,19 +2213,19 @@ int skn_gemm_q6k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
         any_wide = any_wide || q6k_wide_tiles(ctx, segs[i].n, k, m);
     }
     // (rows padded to the tallest tile in use: the kernels with shorter tiles address their own row blocks inside it)
-    const int mt = hilo_mt(m);
+    const int mt = skn_gemm_mt(m);
     const int m_rows = any_wide ? 256 : 32 * mt;
     const int m_pad = (m + m_rows - 1) / m_rows * m_rows;
-    const size_t af_bytes = align_up((size_t)m_pad * k * 2), is_bytes = align_up((size_t)m_pad * 4);
+    const size_t af_bytes = skn_align_up((size_t)m_pad * k * 2), is_bytes = skn_align_up((size_t)m_pad * 4);
     int splits[3] = {1, 1, 1};
     size_t part_bytes = 0;  // (the matrices' products run one after the other: they share the room for their parts)
     for (int i = 0; i < nseg; i++) {
         if (q6k_wide_tiles(ctx, segs[i].n, k, m)) continue;
-        splits[i] = k_splits(ctx, m, ((m + 32 * mt - 1) / (32 * mt)) * ((segs[i].n + kBN - 1) / kBN), k / 256);
+        splits[i] = skn_gemm_k_splits(ctx, m, ((m + 32 * mt - 1) / (32 * mt)) * ((segs[i].n + kBN - 1) / kBN), k / 256);
         if (splits[i] > 1) part_bytes = std::max(part_bytes, (size_t)splits[i] * m * segs[i].n * 4);
     }
     uint8_t* ws;
-    int rc = gemm_workspace(ctx, af_bytes + is_bytes + part_bytes, &ws);
+    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes + part_bytes, &ws);
     if (rc != SKN_OK) return rc;
     _Float16* afrag = (_Float16*)ws;
     float* isc = (float*)(ws + af_bytes);
@@ -2323,13 +2269,13 @@ int skn_gemm_expanded_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, in
     for (int i = 0; i < nseg; i++)
         SKN_REQUIRE(ctx, segs[i].w && segs[i].c && segs[i].n > 0 && ((uintptr_t)segs[i].w & 15) == 0, SKN_ERR_ARG,
                     "expanded GEMM: weights must be non-null and 16-byte aligned");
-    const int mt = hilo_mt(m);
+    const int mt = skn_gemm_mt(m);
     const int m_pad = (m + 32 * mt - 1) / (32 * mt) * (32 * mt);
-    const size_t af_bytes = align_up((size_t)m_pad * k * 2), is_bytes = align_up((size_t)m_pad * 4);
+    const size_t af_bytes = skn_align_up((size_t)m_pad * k * 2), is_bytes = skn_align_up((size_t)m_pad * 4);
     SKN_REQUIRE(ctx, af_bytes < ((size_t)1 << 31), SKN_ERR_SHAPE,
                 "expanded GEMM: %d rows of %d activations exceed the 2^30 elements one call takes", m, k);
     uint8_t* ws;
-    int rc = gemm_workspace(ctx, af_bytes + is_bytes, &ws);
+    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes, &ws);
     if (rc != SKN_OK) return rc;
     _Float16* afrag = (_Float16*)ws;
     float* isc = (float*)(ws + af_bytes);

@@ -1,0 +1,74 @@
+// What the quantized GEMMs (csrc/gemm.hip, csrc/gemm_blocks.hip) share: operand types, the store of a tile, the division of k
+// over workgroups, the workspace.
+#pragma once
+#include "common.h"
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
+
+constexpr int kBN = 64;   // workgroup tile columns (weight rows)
+
+static inline size_t skn_align_up(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// row blocks per tile where the tile follows the rows: 32 MT rows
+static inline int skn_gemm_mt(int m) { return m <= 32 ? 1 : (m <= 64 ? 2 : 4); }
+
+// C tile store: acc register r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32 of the 32x32 tile
+__device__ __forceinline__ void store_tile(const float16_t& acc, float* __restrict__ c, int ldc, int row0, int col0,
+                                           int m, int n, const float* __restrict__ inv_scale, int lane,
+                                           bool accumulate = false) {
+    const int col = col0 + (lane & 31);
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        if (row < m && col < n) {
+            float* dst = c + (size_t)row * ldc + col;
+            *dst = accumulate ? *dst + acc[r] * inv_scale[row] : acc[r] * inv_scale[row];
+        }
+    }
+}
+
+// the same with the sixteen row scales in hand (sc[r]: the scale of the row that register r holds)
+__device__ __forceinline__ void store_tile_scaled(const float16_t& acc, float* __restrict__ c, int ldc, int row0, int col0,
+                                                  int m, int n, const float (&sc)[16], int lane, bool accumulate) {
+    const int col = col0 + (lane & 31);
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        if (row < m && col < n) {
+            float* dst = c + (size_t)row * ldc + col;
+            *dst = accumulate ? *dst + acc[r] * sc[r] : acc[r] * sc[r];
+        }
+    }
+}
+
+// a partial tile of a workgroup that holds a part of k: no scale, rows of ldc
+__device__ __forceinline__ void store_tile_part(const float16_t& acc, float* __restrict__ part, int ldc, int row0, int col0, int m, int n, int lane) {
+    const int col = col0 + (lane & 31);
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        if (row < m && col < n) part[(size_t)row * ldc + col] = acc[r];
+    }
+}
+
+__device__ __forceinline__ uint32_t bf16_rne(float f) {
+    const uint32_t u = __float_as_uint(f);
+    return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
+}
+
+// Matrices that share a division of k: the parts of their products lie side by side, col0 the first column of each.
+struct skn_gemm_parts {
+    float* c[3];
+    int n[3], col0[3], accumulate[3];
+    int count, pair;
+};
+
+int skn_gemm_add_parts(skn_ctx* ctx, const float* part, int splits, int cols, const skn_gemm_parts& segs, const float* inv_scale, int m);
+int skn_gemm_k_splits(const skn_ctx* ctx, int m, int tiles, int nb);
+// grows the context's GEMM workspace; the pointer stays valid until the next growth
+int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out);

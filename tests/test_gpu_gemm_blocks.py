@@ -1,0 +1,69 @@
+"""GPU parity of the prompt GEMM that unpacks formats in blocks of 32 itself, against the oracle."""
+import numpy as np
+import pytest
+
+from oracle import oracle_c, oracle_np
+from skainet_amd import synth
+
+pytestmark = pytest.mark.gpu
+FORMATS = {"q8_0": synth.Q8_0, "q4_0": synth.Q4_0, "q4_1": synth.Q4_1, "q5_0": synth.Q5_0, "q5_1": synth.Q5_1, "q5_k": synth.Q5_K}
+# fp32 sums of exact products: 2^-24 per addition, of which a chain has k / 4 / 32 blocks of two; 1e-5 of the largest output holds
+# for k = 16384, and the floor of the metric is a thousandth of that output
+TOL = 1e-3
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("m,n,k", [(1, 1, 256), (32, 64, 256), (33, 65, 512), (64, 63, 1280), (65, 100, 768), (128, 130, 2816), (129, 64, 1024), (3, 600, 16384)])
+def test_every_tile_height_and_remainder(hip, name, m, n, k):
+    """One row and column to ragged tiles of 32, 64 and 128 rows; fewer superblocks than a workgroup has k-parts, unequal
+    parts, and the longest row the path takes; with k divided over workgroups as the library chooses, not at all, in unequal
+    parts and superblock by superblock."""
+    t = FORMATS[name]
+    raw = synth.weight(t, n, k, seed=n + k + t)
+    a = synth.activation_bf16((m, k), seed=m + 1)
+    want = oracle_c.gemm_q(t, raw, n, k, a, m)
+    for splits in (0, 1, 3, 64):
+        hip.set_option("gemm.split", splits)
+        try:
+            got = hip.gemm_q_host(t, raw, n, k, a, m)
+        finally:
+            hip.set_option("gemm.split", 0)
+        err = oracle_np.rel_err(got, want)
+        assert err <= TOL, f"{splits} parts: rel err {err}"
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+def test_whole_range_of_fields_and_rows_far_apart(hip, name):
+    """Random bytes in every field but the scales (zero, subnormal and of both signs among them), rows of 1e6 beside rows of
+    1e-6 and a row of zeros."""
+    t = FORMATS[name]
+    m, n, k = 70, 96, 1024
+    be, bb = synth.BLOCK[t]
+    rng = np.random.default_rng(t)
+    raw = rng.integers(0, 256, (n * k // be, bb), dtype=np.uint8)
+    d = (rng.standard_normal(len(raw)) * 0.01).astype(np.float16)
+    d[::5], d[3::11] = 0.0, np.float16(6e-8)
+    raw[:, 0:2] = d.view(np.uint8).reshape(-1, 2)
+    if name in ("q4_1", "q5_1", "q5_k"):
+        raw[:, 2:4] = (rng.standard_normal(len(raw)) * 0.02).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[0] *= 1e6
+    x[1] *= 1e-6
+    x[2] = 0.0
+    a = synth.f32_to_bf16_bits(x)
+    got = hip.gemm_q_host(t, raw.reshape(-1), n, k, a, m)
+    want = oracle_c.gemm_q(t, raw.reshape(-1), n, k, a, m)
+    for r in range(m):
+        assert oracle_np.rel_err(got[r], want[r]) <= TOL if np.any(want[r]) else not np.any(got[r]), r
+
+
+def test_weights_off_the_16_byte_grid_take_the_general_path(hip):
+    m, n, k = 5, 70, 512
+    raw = synth.weight(synth.Q8_0, n, k, seed=4)
+    buf = hip.alloc(raw.nbytes + 16)
+    buf.upload(raw, offset=2)
+    a = synth.activation_bf16((m, k), seed=5)
+    c = hip.alloc(4 * m * n)
+    hip.gemm_q(synth.Q8_0, buf.ptr + 2, n, k, hip.to_device(a), m, c)
+    got = c.download(np.float32, m * n).reshape(m, n)
+    assert oracle_np.rel_err(got, oracle_c.gemm_q(synth.Q8_0, raw, n, k, a, m)) <= TOL
