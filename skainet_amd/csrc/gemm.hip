@@ -726,6 +726,12 @@ int launch_frag(skn_ctx* ctx, int m_tiles, const u32x4* afrag, const u32x4* sfra
 // 1.8 - 1.9 GHz with all compute units at this work.)
 constexpr int kTlStage = 4 * 4 * 1024;           // a phase: four k-steps x four column blocks x 1 KiB
 constexpr int kTlAux = 128 * 32 + 128 * 4;       // a superblock's min operands (128 columns x (hi, lo) x 16 B) and ratios
+// The last `tiles` tiles of a launch, from tile0 on, with their k divided over `splits` workgroups: part[split][tile][consumer]
+// [row block][column block][register group][lane] x 4.
+struct TallTail {
+    int tile0, tiles, splits;
+    float* part;
+};
 constexpr int kTlLds = 3 * kTlStage + 2 * kTlAux + 128 * 4 + 256 * 4;
 
 // One to three matrices per launch as in gemm_q4k_frag_kernel (tile0 counts 128-column tiles here); pair: a tile holds
@@ -733,7 +739,7 @@ constexpr int kTlLds = 3 * kTlStage + 2 * kTlAux + 128 * 4 + 256 * 4;
 // consumer's column blocks 0, 1 and 2, 3 meet lane by lane in the store -- and stores silu(gate) * up into c[0].
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restrict__ sfrag, const Q4kFragSegs segs,
-                          const float* __restrict__ inv_scale, int m, int k, int m_tiles, uint32_t a_bytes) {
+                          const float* __restrict__ inv_scale, int m, int k, int m_tiles, uint32_t a_bytes, const TallTail tail) {
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -741,7 +747,11 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
     const bool producer = wave >= 4;
     const int h = lane >> 5, r = lane & 31;
     const int nb = k >> 8, nch = k >> 6;
-    const int mt = blockIdx.x % m_tiles, tn = blockIdx.x / m_tiles;  // (the row tiles of a column tile run side by side)
+    // the last tiles are shared by tail.splits workgroups each, neighbours in the grid, with a part of k each
+    const int over = (int)blockIdx.x - tail.tile0, z = over < 0 ? 0 : over % tail.splits;
+    const int tile = over < 0 ? (int)blockIdx.x : tail.tile0 + over / tail.splits, parts = over < 0 ? 1 : tail.splits;
+    const int sb0 = nb * z / parts, sb1 = nb * (z + 1) / parts;
+    const int mt = tile % m_tiles, tn = tile / m_tiles;  // (the row tiles of a column tile run side by side)
     const bool pair = segs.pair != 0;
     const int seg = pair ? 0 : (tn >= segs.tile0[2] ? 2 : (tn >= segs.tile0[1] ? 1 : 0));
     const int n = segs.n[seg];
@@ -859,7 +869,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
             if (cc == 2) {
                 const float keep = cs;
                 enter(sb + 1);
-                if (sb + 1 >= nb) cs = keep;
+                if (sb + 1 >= sb1) cs = keep;
                 unpack(C0{}, b_nx2);
                 load_header(sb + 2);
                 load_piece(sb + 2, 0);
@@ -871,17 +881,17 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
             barrier();
             turn();
         };
-        load_header(0);
+        load_header(sb0);
 #pragma unroll
-        for (int x = 0; x < 4; x++) load_piece(0, x);
-        enter(0);
+        for (int x = 0; x < 4; x++) load_piece(sb0, x);
+        enter(sb0);
         unpack(C0{}, b_cur);
         unpack(C1{}, b_nxt);
-        load_header(1);
-        load_piece(1, 0);
-        load_piece(1, 1);
+        load_header(sb0 + 1);
+        load_piece(sb0 + 1, 0);
+        load_piece(sb0 + 1, 1);
         barrier();
-        for (int sb = 0; sb < nb; sb++) {
+        for (int sb = sb0; sb < sb1; sb++) {
             phase(sb, C0{});
             phase(sb, C1{});
             phase(sb, C2{});
@@ -988,7 +998,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
 #pragma unroll
                 for (int j = 0; j < 4; j++) fb[0][j] = *reinterpret_cast<const half8_t*>(srcn + j * 1024);
 #pragma unroll
-                for (int j = 0; j < 4; j++) ratio[j] = sb + 1 < nb ? rnext[j] : 1.0f;  // (none after the last superblock)
+                for (int j = 0; j < 4; j++) ratio[j] = sb + 1 < sb1 ? rnext[j] : 1.0f;  // (none after the last superblock)
                 fence();
                 // tiles 0 .. 2 change their unit between the last of these instructions
 #pragma unroll
@@ -1003,17 +1013,31 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
             turn();
         };
 #pragma unroll
-        for (int s = 0; s < 7; s++) afetch(s, s);
+        for (int s = 0; s < 7; s++) afetch(16 * sb0 + s, s);
         barrier();
 #pragma unroll
         for (int j = 0; j < 4; j++) fb[0][j] = *reinterpret_cast<const half8_t*>(stage + b_cur + lane * 16 + j * 1024);
-        for (int sb = 0; sb < nb; sb++) {
+        for (int sb = sb0; sb < sb1; sb++) {
             phase(sb, C0{});
             phase(sb, C1{});
             phase(sb, C2{});
             phase(sb, C3{});
         }
         barrier();
+        if (parts > 1) {  // (unscaled, every element of the tile, in the order of the matrix core's registers: see gemm_add_tall_kernel)
+            float* dst = tail.part + ((size_t)(z * tail.tiles + tile - tail.tile0) * 4 + me) * (MT * 4 * 1024) + lane * 4;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float unit = *reinterpret_cast<const float*>(fin + (j * 32 + r) * 4);
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int x = 0; x < 4; x++)
+                        *reinterpret_cast<float4*>(dst + ((i * 4 + j) * 4 + x) * 256) =
+                            make_float4(acc[i][j][4 * x] * unit, acc[i][j][4 * x + 1] * unit, acc[i][j][4 * x + 2] * unit, acc[i][j][4 * x + 3] * unit);
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < MT; i++) {
             float sc[16];
@@ -1045,6 +1069,44 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                 store_tile_scaled(acc[i][j], c, n, (mb0 + i) * 32, n0 + 32 * j, m, n, sc, lane, segs.accumulate[seg] != 0);
             }
         }
+    }
+}
+
+// The tiles that workgroups shared: grid (tiles, 8), a wavefront per row block and column block of 32 (wavefront w of block y: row
+// block y of the tile, column block w; a pair: wavefronts 0 and 1, both halves).  Lane l of register group x holds rows
+// 8 x + 4 (l / 32) .. + 3 of column l % 32, as the matrix core does.
+__global__ __launch_bounds__(256) void gemm_add_tall_kernel(const TallTail tail, const Q4kFragSegs segs, const float* __restrict__ inv_scale, int m, int m_tiles) {
+    const int tile = tail.tile0 + (int)blockIdx.x, mt = tile % m_tiles, tn = tile / m_tiles, lane = threadIdx.x & 63, j = threadIdx.x >> 6;
+    const int i = blockIdx.y, row0 = mt * 256 + 32 * i;  // (consumer i / 2, its row block i % 2)
+    const bool pair = segs.pair != 0;
+    if (row0 >= m || (pair && j > 1)) return;
+    const int seg = pair ? 0 : (tn >= segs.tile0[2] ? 2 : (tn >= segs.tile0[1] ? 1 : 0));
+    const int n = segs.n[seg], col = (pair ? tn * 64 : (tn - segs.tile0[seg]) * 128) + 32 * j + (lane & 31);
+    float* __restrict__ c = segs.c[seg];
+    auto total = [&](int jj, float (&v)[16]) __attribute__((always_inline)) {
+        const float4* src = reinterpret_cast<const float4*>(tail.part) + (((size_t)blockIdx.x * 4 + (i >> 1)) * 8 + (i & 1) * 4 + jj) * 256 + lane;
+        const size_t stride = (size_t)tail.tiles * 8192;
+#pragma unroll
+        for (int x = 0; x < 16; x++) v[x] = 0.f;
+        for (int z = 0; z < tail.splits; z++)
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                const float4 p = src[z * stride + 64 * x];
+                v[4 * x] += p.x, v[4 * x + 1] += p.y, v[4 * x + 2] += p.z, v[4 * x + 3] += p.w;
+            }
+    };
+    float v[16], u[16];
+    total(j, v);
+    if (pair) total(j + 2, u);
+    if (col >= n) return;
+#pragma unroll
+    for (int x = 0; x < 16; x++) {
+        const int row = row0 + 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3);
+        if (row >= m) continue;
+        const float sc = inv_scale[row], g = v[x] * sc;
+        float* dst = c + (size_t)row * n + col;
+        if (pair) *dst = g / (1.0f + expf(-g)) * (u[x] * sc);  // silu(gate) * up
+        else *dst = segs.accumulate[seg] != 0 ? *dst + g : g;
     }
 }
 
@@ -2038,6 +2100,16 @@ static int skn_gemm_init(skn_ctx* ctx) {
 }
 static skn_family register_family(skn_gemm_init);
 
+// The tiles past the last whole round of compute units: shared where at least two workgroups each find room in that round.
+static TallTail tall_tail(const skn_ctx* ctx, int tiles, int m_tiles, int nb) {
+    const int cus = ctx->compute_units, rest = tiles % cus;
+    TallTail t = {tiles, 0, 1, nullptr};
+    int splits = rest ? std::min(cus / rest, nb / 4) : 1;
+    if (ctx->opt_gemm_split > 0) splits = std::min(ctx->opt_gemm_split, nb);
+    if (rest == 0 || splits < 2) return t;
+    return TallTail{tiles - rest, rest, splits, nullptr};
+}
+
 int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, const skn_gemm_src& src, int m,
                        bool swiglu_pair) {
     SKN_REQUIRE(ctx, nseg >= 1 && nseg <= 3 && m > 0 && k > 0 && k % 256 == 0 && k <= 16384, SKN_ERR_ARG,
@@ -2081,6 +2153,8 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     const int tall_rounds = (tall_tiles + ctx->compute_units - 1) / ctx->compute_units;
     const bool tall = tall_fits && (ctx->opt_gemm_tile == 3 ||
                                     (ctx->opt_gemm_tile == 0 && m > 128 && 3 * tall_tiles >= 2 * tall_rounds * ctx->compute_units));
+    TallTail tail = {tall_tiles, 0, 1, nullptr};
+    if (tall) tail = tall_tail(ctx, tall_tiles, (m + 255) / 256, k / 256);
     const bool small_tiles = !tall && (ctx->opt_gemm_tile == 1 ||
                              (ctx->opt_gemm_tile == 0 && (m <= 128 || ((m + 127) / 128) * n_tiles_all > ctx->compute_units)));
     const int mt_rows = tall ? 256 : small_tiles ? 64 : 128;
@@ -2098,7 +2172,7 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
         fs.part_cols += segs[i].n;
     }
     for (int i = 0; i < 3; i++) fs.part_col0[i] = ps.col0[i];
-    const size_t part_bytes = splits > 1 ? (size_t)splits * m * fs.part_cols * 4 : 0;
+    const size_t part_bytes = tall ? (size_t)tail.tiles * tail.splits * 131072 : splits > 1 ? (size_t)splits * m * fs.part_cols * 4 : 0;
     uint8_t* ws;
     int rc = skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes + part_bytes, &ws);
     if (rc != SKN_OK) return rc;
@@ -2116,9 +2190,14 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     if (tall) {
         for (int i = 0; i < 3; i++) fs.tile0[i] = tall_tile0[i];
         fs.n_tiles = tall_cols;
-        skn_launch(ctx, gemm_q4k_tall_kernel, dim3(m_tiles * tall_cols), dim3(512), kTlLds, (const u32x4*)afrag, (const u32x4*)sfrag, fs, isc, m,
-                   k, m_tiles, (uint32_t)((size_t)m_pad * k * 2));
+        tail.part = (float*)(ws + af_bytes + sf_bytes + is_bytes);
+        skn_launch(ctx, gemm_q4k_tall_kernel, dim3(tail.tile0 + tail.tiles * tail.splits), dim3(512), kTlLds, (const u32x4*)afrag, (const u32x4*)sfrag, fs,
+                   (const float*)isc, m, k, m_tiles, (uint32_t)((size_t)m_pad * k * 2), tail);
         SKN_LAUNCH_CHECK(ctx);
+        if (tail.tiles) {
+            skn_launch(ctx, gemm_add_tall_kernel, dim3(tail.tiles, 8), dim3(256), 0, tail, fs, (const float*)isc, m, m_tiles);
+            SKN_LAUNCH_CHECK(ctx);
+        }
         return SKN_OK;
     }
     if (mt_rows == 128) SKN_TRY((launch_frag<2, 2>(ctx, m_tiles, (const u32x4*)afrag, (const u32x4*)sfrag, fs, isc, m, k, splits)));

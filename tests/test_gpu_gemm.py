@@ -219,25 +219,28 @@ def test_gemm_q6k_full_range_of_the_block_fields(hip, m, n, k):
 
 
 @pytest.mark.parametrize("qtype", [Q4_K, Q6_K])
-@pytest.mark.parametrize("m,n,k", [(1, 64, 512), (33, 100, 1280), (65, 65, 768), (130, 65, 2816), (130, 192, 2816)])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 512), (33, 100, 1280), (65, 65, 768), (130, 65, 2816), (130, 192, 2816), (300, 130, 768)])
 def test_gemm_with_k_split_over_workgroups(hip, qtype, m, n, k):
     """k divided over 2, 3, 5 and as many workgroups per tile as there are superblocks: parts with fewer superblocks than a
     workgroup has k-parts, with unequal ones and with one, ragged tiles, columns that are and are not a multiple of four (the
-    width of the addition), all tile heights of both formats (Q6_K at 130 rows with and without specialised wavefronts)."""
+    width of the addition), all tile heights of both formats (Q6_K at 130 rows with and without specialised wavefronts; Q4_K on
+    256 x 128 tiles too)."""
     raw = synth.weight(qtype, n, k, seed=n + k + qtype)
     a = synth.activation_bf16((m, k), seed=m + 3)
     want = oracle_c.gemm_q(qtype, raw, n, k, a, m)
     for splits in (2, 3, 5, 64):
-        for form in ((1, 2) if qtype == Q6_K else (1,)):
+        for form, tile in (((1, 0), (2, 0)) if qtype == Q6_K else ((1, 0), (1, 3))):  # (tile 3: the 256 x 128 tiles)
             hip.set_option("gemm.split", splits)
             hip.set_option("gemm.q6k_fused", form)
+            hip.set_option("gemm.tile", tile)
             try:
                 got = hip.gemm_q_host(qtype, raw, n, k, a, m)
             finally:
                 hip.set_option("gemm.split", 0)
                 hip.set_option("gemm.q6k_fused", 1)
+                hip.set_option("gemm.tile", 0)
             err = oracle_np.rel_err(got, want)
-            assert err <= TOL, f"{splits} parts, form {form}: rel err {err}"
+            assert err <= TOL, f"{splits} parts, form {form}, tile {tile}: rel err {err}"
 
 
 @pytest.mark.parametrize("n", [4096, 14336])

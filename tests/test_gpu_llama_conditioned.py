@@ -108,13 +108,16 @@ def test_prompt_with_the_wide_tile_gemm_forced(hip, case):
         hip.set_option("gemm.tile", 0)
 
 
+@pytest.mark.parametrize("tile", [0, 3])
 @pytest.mark.parametrize("case", ["q4_k", "q4_k_kv2", "mixed", "q6_k"])
-def test_prompt_with_k_split_over_workgroups(hip, case):
+def test_prompt_with_k_split_over_workgroups(hip, case, tile):
     """The prompt's products with the k of a tile divided over two workgroups (the library does it by itself from five
-    superblocks on): the addition of the parts stores q, k, v into three buffers, adds a residual, multiplies silu(gate) by up."""
+    superblocks on; tile 3: on 256 x 128 tiles): the addition of the parts stores q, k, v into three buffers, adds a residual,
+    multiplies silu(gate) by up."""
     cfg = CASES[case]
     prompt, first, _, _ = _oracle_prompt(case, 41, 12)
     hip.set_option("gemm.split", 2)
+    hip.set_option("gemm.tile", tile)
     try:
         model = llama.LlamaModel(hip, cfg, weights=llama.conditioned_weights(cfg, SEED))
         model.prefill(prompt)
@@ -123,6 +126,7 @@ def test_prompt_with_k_split_over_workgroups(hip, case):
         model.free()
     finally:
         hip.set_option("gemm.split", 0)
+        hip.set_option("gemm.tile", 0)
 
 
 @pytest.mark.parametrize("fused,graph", [(1, 1), (0, 0)])
