@@ -90,6 +90,8 @@ int skn_attn_launch_unmerged(skn_ctx* ctx, skn_kv* kv, const float* q_dev, const
                              int seq_fixed, int n_splits, float* opart, float* ml, float scale, float* out_dev, int n_q_head);
 int skn_matvec_q4k_fused(skn_ctx* ctx, const skn_q4k_segments& seg, int n_out, int k, const float* x, const float* norm_w,
                          float eps, float* y, int epi, const skn_rope_epilogue* rope = nullptr, int ggml_type = SKN_TYPE_Q4_K);
+int skn_matvec_fused_two(skn_ctx* ctx, const skn_q4k_segments& q6, int n_q6, const skn_q4k_segments& other, int n_other, int other_type, int k,
+                         const float* x, const float* norm_w, float eps, float* y, const skn_rope_epilogue& rope);
 // the formats the fused kernels take (every matrix of a launch in the same one; k a multiple of 256)
 bool skn_matvec_fusable(int ggml_type);
 

@@ -210,9 +210,10 @@ int dev_alloc(skn_ctx* ctx, skn_llama* m, T** p, size_t count) {
 
 unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
 
-// the launches of one decode step (eagerly or under stream capture)
-int decode_step(skn_ctx* ctx, skn_llama* m, int n_splits) {
+// The launches of one decode step (eagerly or under stream capture) at contexts of up to 128 * units tokens.
+int decode_step(skn_ctx* ctx, skn_llama* m, int units) {
     const skn_llama_config& c = m->cfg;
+    const int n_splits = std::min(units, skn_attn_splits(ctx, c.n_head, c.max_tokens));
     const int H = c.hidden, F = c.ffn, NH = c.n_head, D = c.head_dim, KVH = c.n_kv_head, KVD = KVH * D;
     const float scale = 1.0f / sqrtf((float)D);
     skn_launch(ctx, embed_rows_kernel, dim3(1), dim3(1024), 0, (const uint8_t*)m->w.tok_embd, m->w.type_embd, H,
@@ -244,14 +245,35 @@ int decode_step(skn_ctx* ctx, skn_llama* m, int n_splits) {
             rope.inv_freq = m->inv_freq;
             const int types[3] = {L.type_q, L.type_k, L.type_v}, rows[3] = {H, KVD, KVD};
             const uint8_t* mats[3] = {(const uint8_t*)L.wq, (const uint8_t*)L.wk, (const uint8_t*)L.wv};
+            auto part = [&](bool (&in)[3], skn_q4k_segments& seg) {
+                int n_out = 0;
+                for (int j = 0; j < 3; j++)
+                    if (in[j]) seg.w[j] = mats[j], seg.rows[j] = rows[j], n_out += rows[j];
+                return n_out;
+            };
             bool done[3] = {false, false, false};
+            // Q6_K beside one other format: one launch for both (a decode step of a mixed 7B file: 1447 us, 1475 in two launches)
+            bool in6[3], rest[3];
+            int other = -1;
+            bool two = true;
+            for (int j = 0; j < 3; j++) {
+                in6[j] = types[j] == SKN_TYPE_Q6_K, rest[j] = !in6[j];
+                if (rest[j]) two = two && (other < 0 || types[j] == other), other = types[j];
+            }
+            if (two && other >= 0 && (in6[0] || in6[1] || in6[2])) {
+                skn_q4k_segments s6 = {{nullptr, nullptr, nullptr}, {0, 0, 0}}, so = s6;
+                const int n6 = part(in6, s6), no = part(rest, so);
+                const int rc = skn_matvec_fused_two(ctx, s6, n6, so, no, other, H, m->x, L.attn_norm, c.rms_eps, m->q, rope);
+                if (rc == SKN_OK) done[0] = done[1] = done[2] = true;
+                else if (rc != SKN_ERR_TYPE) return rc;
+            }
             for (int i = 0; i < 3; i++) {
                 if (done[i]) continue;
-                skn_q4k_segments part = {{nullptr, nullptr, nullptr}, {0, 0, 0}};
-                int n_out = 0;
-                for (int j = i; j < 3; j++)
-                    if (types[j] == types[i]) part.w[j] = mats[j], part.rows[j] = rows[j], n_out += rows[j], done[j] = true;
-                SKN_TRY(skn_matvec_q4k_fused(ctx, part, n_out, H, m->x, L.attn_norm, c.rms_eps, m->q, SKN_EPI_ROPE, &rope, types[i]));
+                bool in[3];
+                for (int j = 0; j < 3; j++) in[j] = types[j] == types[i], done[j] = done[j] || in[j];
+                skn_q4k_segments seg = {{nullptr, nullptr, nullptr}, {0, 0, 0}};
+                const int n_out = part(in, seg);
+                SKN_TRY(skn_matvec_q4k_fused(ctx, seg, n_out, H, m->x, L.attn_norm, c.rms_eps, m->q, SKN_EPI_ROPE, &rope, types[i]));
             }
         } else {
             skn_launch(ctx, rmsnorm_rows_kernel, dim3(1), dim3(256), 0, (const float*)m->x, L.attn_norm, m->xn, H, c.rms_eps);
@@ -264,13 +286,12 @@ int decode_step(skn_ctx* ctx, skn_llama* m, int n_splits) {
                        kv->page_tokens, log2((double)c.rope_base));
             SKN_LAUNCH_CHECK(ctx);
         }
-        if (f_o && ctx->opt_llama_attn_wide && n_splits * 128 > 32768 / D) {
+        const int per_round = 32768 / D;  // tokens that a workgroup of sixteen wavefronts takes per round of requests
+        if (f_o && ctx->opt_llama_attn_wide && units * 128 > per_round) {
             // The attention leaves the partials of its splits unmerged and the output projection's staging merges them:
-            // no device-wide counter, no store-then-reload chain inside the attention launch.  A workgroup of sixteen
-            // wavefronts takes 32768 / head_dim tokens per round of requests, so the splits are counted in those units.
-            const int per_round = 32768 / D;
+            // no device-wide counter, no store-then-reload chain inside the attention launch.
             int wide = 2;  // 2, 4 or 8 (what the merge in the projection's staging is built for)
-            while (wide < 8 && wide * per_round < n_splits * 128) wide *= 2;
+            while (wide < 8 && wide * per_round < units * 128) wide *= 2;
             if (ctx->opt_llama_attn_wide > 1) wide = std::min(wide, ctx->opt_llama_attn_wide);  // (tuning: 2, 4 or 8 caps the count)
             float* opart = m->attn_partial;
             float* ml = m->attn_partial + (size_t)wide * NH * D;
@@ -283,7 +304,12 @@ int decode_step(skn_ctx* ctx, skn_llama* m, int n_splits) {
             mg.merge_head_f4 = D / 4;
             SKN_TRY(skn_matvec_q4k_fused(ctx, wo, H, H, opart, nullptr, 0.f, m->x, SKN_EPI_ADD, &mg, L.type_o));
         } else if (f_o) {
-            SKN_TRY(skn_attn_launch_ex(ctx, kv, m->q, m->step.state + 2, 1, 0, n_splits, m->attn_partial, m->attn_counters, scale, m->att, NH));
+            // up to one round: a workgroup per head, nothing to merge (contexts of 120 - 184 tokens, 32 heads of 128: 5.1 us against
+            // 6.9 us for two splits behind a counter)
+            if (ctx->opt_llama_attn_wide)
+                SKN_TRY(skn_attn_launch_unmerged(ctx, kv, m->q, m->step.state + 2, 1, 0, 1, nullptr, nullptr, scale, m->att, NH));
+            else
+                SKN_TRY(skn_attn_launch_ex(ctx, kv, m->q, m->step.state + 2, 1, 0, n_splits, m->attn_partial, m->attn_counters, scale, m->att, NH));
             skn_q4k_segments wo = {{(const uint8_t*)L.wo, nullptr, nullptr}, {H, 0, 0}};
             SKN_TRY(skn_matvec_q4k_fused(ctx, wo, H, H, m->att, nullptr, 0.f, m->x, SKN_EPI_ADD, nullptr, L.type_o));
         } else {
@@ -691,14 +717,13 @@ int skn_llama_decode(skn_ctx* ctx, skn_llama* m, int32_t first_token, int n_step
                 "skn_llama_decode: not available while per-launch timing is on (except with llama.graph = 0)");
     // every page the run will touch is mapped now; the step itself never talks to the host
     for (skn_kv* kv : m->kv) SKN_TRY(skn_kv_reserve(ctx, kv, 0, m->pos + n_steps));
-    // A split count for the longest context of this run, rounded up to a power of two of 128-token units (the kernel
-    // derives its ranges from the actual length, so one captured step serves every position up to there): the step is
+    // The longest context of this run, rounded up to a power of two of 128-token units, decides the attention's splits (the
+    // kernels derive their ranges from the actual length, so one captured step serves every position up to there): the step is
     // captured again only when a sequence grows past 128, 256, 512, ... tokens, and a short context is not cut into
     // more pieces than it has work for (sixteen splits of 600 tokens cost 2 % of the step against eight).
-    int n_splits = 1;
-    while (n_splits * 128 < m->pos + n_steps) n_splits *= 2;
-    n_splits = std::min(n_splits, skn_attn_splits(ctx, c.n_head, c.max_tokens));
-    SKN_TRY(skn_stepper_run(ctx, &m->step, first_token, m->pos, n_steps, n_splits, [&]() { return decode_step(ctx, m, n_splits); },
+    int units = 1;
+    while (units * 128 < m->pos + n_steps) units *= 2;
+    SKN_TRY(skn_stepper_run(ctx, &m->step, first_token, m->pos, n_steps, units, [&]() { return decode_step(ctx, m, units); },
                             tokens_out_host));
     m->pos += n_steps;
     for (skn_kv* kv : m->kv) kv->len[0] = m->pos;

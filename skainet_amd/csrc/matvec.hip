@@ -1468,14 +1468,13 @@ __device__ __forceinline__ float4 q4k_merge_splits(const float4* __restrict__ pa
 // Up to three weight matrices with the same k stacked along the output axis (q, k, v projections in one launch;
 // gate and up paired row by row), optional RMSNorm of x folded into the staging (every workgroup needs all of
 // x anyway, so it also forms sum(x^2) and stores x * r * norm_w), and an epilogue that stores, adds into the
-// residual stream, or applies SwiGLU to a (gate, up) row pair.  Two rows per wavefront.
-// F: the format of all the matrices of the launch, as in matvec_q4k_kernel.
-template <int STEPS, int EPI, bool NORM, int F = kFmtQ4K>
-__global__ __launch_bounds__(512) void matvec_q4k_fused_kernel(skn_q4k_segments seg, const float* __restrict__ x,
-                                                               const float* __restrict__ norm_w, float eps,
-                                                               float* __restrict__ y, int n_out, int nb,
-                                                               skn_rope_epilogue rope) {
-    constexpr int R = 2;
+// residual stream, or applies SwiGLU to a (gate, up) row pair.  Two rows per wavefront, or one where rows are added into few
+// outputs (see dispatch_q4k_fused).  F: the format of all the matrices, as in matvec_q4k_kernel; block: the workgroup's place
+// among those that share the matrices.
+template <int STEPS, int EPI, bool NORM, int F, int R>
+__device__ __forceinline__ void q4k_fused_block(const skn_q4k_segments& seg, const float* __restrict__ x, const float* __restrict__ norm_w, float eps,
+                                                float* __restrict__ y, int n_out, int nb, const skn_rope_epilogue& rope, int block) {
+    static_assert(R == 2 || EPI == SKN_EPI_ADD, "row pairs");
     constexpr bool Q5 = F == kFmtQ5K, Q6 = F == kFmtQ6K, Q8 = F == kFmtQ80, Q2 = F == kFmtQ2K, Q3 = F == kFmtQ3K, Q8K = F == kFmtQ8K;
     constexpr bool T2 = F == kFmtTQ2, T1 = F == kFmtTQ1;
     constexpr bool kRuns = Q6 || Q2 || Q3 || T2;  // the Q6_K lane map: four runs of sixteen per lane, a float4 of run sums
@@ -1503,7 +1502,7 @@ __global__ __launch_bounds__(512) void matvec_q4k_fused_kernel(skn_q4k_segments 
     if (EPI == SKN_EPI_ROPE) {
         rope_pos = rope.pos_dev[0];
         if (rope.inv_freq)
-            rope_freq = rope.inv_freq[q4k_rope_elem(seg, rope, min((int)(blockIdx.x * 8 + (threadIdx.x >> 6)), (n_out + 1) / 2 - 1)) >> 1];
+            rope_freq = rope.inv_freq[q4k_rope_elem(seg, rope, min(block * 8 + (int)(threadIdx.x >> 6), (n_out + 1) / 2 - 1)) >> 1];
     }
     Q4kStage<J> st, nw;
     bool merged = false;
@@ -1531,7 +1530,7 @@ __global__ __launch_bounds__(512) void matvec_q4k_fused_kernel(skn_q4k_segments 
     if (NORM) q4k_stage_load<J>(norm_w, n4, tid, 512, nw);
 
     // the two rows of this wavefront: consecutive rows of the stacked matrices, or row i of gate and of up
-    const int unit = blockIdx.x * 8 + wave;
+    const int unit = block * 8 + wave;
     const uint8_t* rowp[R];
     bool row_ok[R];
     const size_t row_bytes = (size_t)nb * (Q8 ? 272 : Q6 ? 210 : Q2 ? 84 : Q3 ? 110 : T2 ? 66 : T1 ? 54 : Q8K ? 292 : kXS ? 136 : kSmall ? 8 * kSmallBytes : 16 * kChunks);
@@ -1668,7 +1667,7 @@ __global__ __launch_bounds__(512) void matvec_q4k_fused_kernel(skn_q4k_segments 
         rinv = 1.0f / sqrtf(total / (float)(nb * 256) + eps);
     }
 
-    float acc[R] = {0.f, 0.f};
+    float acc[R] = {};
     int tie = 0;
     asm volatile("" : "+v"(tie));
 #pragma unroll
@@ -1688,17 +1687,53 @@ __global__ __launch_bounds__(512) void matvec_q4k_fused_kernel(skn_q4k_segments 
     }
     const float back = (Q8 || Q8K || T1 || kPlainX) ? rinv : 16777216.0f * rinv;  // (the nibble formats work in units of 2^-24)
     const float t0 = wave_sum(acc[0]) * back;
-    const float t1 = wave_sum(acc[1]) * back;
-    if (lane == 0) q4k_epilogue<EPI>(rope, rc, y, n_out, unit, t0, t1);
+    if constexpr (R == 1) {
+        if (lane == 0 && unit < n_out) y[unit] += t0;
+    } else {
+        const float t1 = wave_sum(acc[1]) * back;
+        if (lane == 0) q4k_epilogue<EPI>(rope, rc, y, n_out, unit, t0, t1);
+    }
 }
 
-template <int STEPS, int EPI, bool NORM, int F>
+template <int STEPS, int EPI, bool NORM, int F = kFmtQ4K, int R = 2>
+__global__ __launch_bounds__(512) void matvec_q4k_fused_kernel(skn_q4k_segments seg, const float* __restrict__ x,
+                                                               const float* __restrict__ norm_w, float eps,
+                                                               float* __restrict__ y, int n_out, int nb,
+                                                               skn_rope_epilogue rope) {
+    q4k_fused_block<STEPS, EPI, NORM, F, R>(seg, x, norm_w, eps, y, n_out, nb, rope, (int)blockIdx.x);
+}
+
+// q, k and v in two formats (mixed files give the values more bits): the workgroups of both in one launch, the larger blocks first.
+template <int STEPS, int FA, int FB>
+__global__ __launch_bounds__(512) void matvec_fused_two_formats_kernel(skn_q4k_segments sa, skn_q4k_segments sb, const float* __restrict__ x,
+                                                                      const float* __restrict__ norm_w, float eps, float* __restrict__ y,
+                                                                      int n_a, int n_b, int blocks_a, int nb, skn_rope_epilogue rope) {
+    if ((int)blockIdx.x < blocks_a) q4k_fused_block<STEPS, SKN_EPI_ROPE, true, FA, 2>(sa, x, norm_w, eps, y, n_a, nb, rope, (int)blockIdx.x);
+    else q4k_fused_block<STEPS, SKN_EPI_ROPE, true, FB, 2>(sb, x, norm_w, eps, y, n_b, nb, rope, (int)blockIdx.x - blocks_a);
+}
+
+template <int F>
+constexpr size_t fused_lds_bytes(int steps) {
+    return (size_t)steps * (16 * kXPitch * sizeof(float4) + 64 * ((F == kFmtQ6K || F == kFmtQ2K || F == kFmtQ3K || F == kFmtTQ2) ? sizeof(float4) : sizeof(float2))) + 8 * sizeof(float);
+}
+
+template <int STEPS, int F>
+int launch_fused_beside_q6k(skn_ctx* ctx, const skn_q4k_segments& q6, int n_q6, const skn_q4k_segments& other, int n_other, int nb, const float* x,
+                            const float* norm_w, float eps, float* y, const skn_rope_epilogue& rope) {
+    const int blocks_q6 = (n_q6 + 15) / 16, blocks = blocks_q6 + (n_other + 15) / 16;
+    skn_launch(ctx, matvec_fused_two_formats_kernel<STEPS, kFmtQ6K, F>, dim3((unsigned)blocks), dim3(512), fused_lds_bytes<kFmtQ6K>(STEPS), q6, other, x, norm_w,
+               eps, y, n_q6, n_other, blocks_q6, nb, rope);
+    SKN_LAUNCH_CHECK(ctx);
+    return SKN_OK;
+}
+
+template <int STEPS, int EPI, bool NORM, int F, int R = 2>
 int launch_q4k_fused(skn_ctx* ctx, const skn_q4k_segments& seg, int n_out, int nb, const float* x, const float* norm_w,
                      float eps, float* y, const skn_rope_epilogue& rope) {
-    const size_t lds = (size_t)STEPS * (16 * kXPitch * sizeof(float4) + 64 * ((F == kFmtQ6K || F == kFmtQ2K || F == kFmtQ3K || F == kFmtTQ2) ? sizeof(float4) : sizeof(float2))) + 8 * sizeof(float);
-    const int units = EPI == SKN_EPI_SWIGLU ? n_out : (n_out + 1) / 2;
+    const size_t lds = fused_lds_bytes<F>(STEPS);
+    const int units = EPI == SKN_EPI_SWIGLU ? n_out : (n_out + R - 1) / R;
     dim3 grid((unsigned)((units + 7) / 8)), block(512);
-    skn_launch(ctx, matvec_q4k_fused_kernel<STEPS, EPI, NORM, F>, grid, block, lds, seg, x, norm_w, eps, y, n_out, nb, rope);
+    skn_launch(ctx, matvec_q4k_fused_kernel<STEPS, EPI, NORM, F, R>, grid, block, lds, seg, x, norm_w, eps, y, n_out, nb, rope);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
@@ -1713,6 +1748,11 @@ int dispatch_q4k_fused(skn_ctx* ctx, const skn_q4k_segments& seg, int n_out, int
     if (epi == SKN_EPI_SWIGLU)
         return norm ? launch_q4k_fused<STEPS, SKN_EPI_SWIGLU, true, F>(ctx, seg, n_out, nb, x, norm_w, eps, y, rope)
                     : launch_q4k_fused<STEPS, SKN_EPI_SWIGLU, false, F>(ctx, seg, n_out, nb, x, norm_w, eps, y, rope);
+    // One row per wavefront where pairs would give fewer than two workgroups per compute unit (the output and down projections of
+    // widths up to 8192): a decode step of the 7B shape at 150 tokens 1481 -> 1449 us, of 8 layers of width 2048 at 2000 tokens 299 ->
+    // 279.  Before, the plain matvec alone divided its rows so.
+    if (epi == SKN_EPI_ADD && !norm && n_out < 32 * ctx->compute_units)
+        return launch_q4k_fused<STEPS, SKN_EPI_ADD, false, F, 1>(ctx, seg, n_out, nb, x, norm_w, eps, y, rope);
     if (epi == SKN_EPI_ADD)
         return norm ? launch_q4k_fused<STEPS, SKN_EPI_ADD, true, F>(ctx, seg, n_out, nb, x, norm_w, eps, y, rope)
                     : launch_q4k_fused<STEPS, SKN_EPI_ADD, false, F>(ctx, seg, n_out, nb, x, norm_w, eps, y, rope);
@@ -1720,9 +1760,9 @@ int dispatch_q4k_fused(skn_ctx* ctx, const skn_q4k_segments& seg, int n_out, int
                 : launch_q4k_fused<STEPS, SKN_EPI_STORE, false, F>(ctx, seg, n_out, nb, x, norm_w, eps, y, rope);
 }
 
-template <int STEPS, int EPI, bool NORM, int F>
+template <int STEPS, int EPI, bool NORM, int F, int R = 2>
 hipError_t allow_big_lds_fused() {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(matvec_q4k_fused_kernel<STEPS, EPI, NORM, F>),
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(matvec_q4k_fused_kernel<STEPS, EPI, NORM, F, R>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
 }
 
@@ -1731,11 +1771,25 @@ hipError_t allow_big_lds_fused_all() {
     hipError_t e = allow_big_lds_fused<STEPS, SKN_EPI_STORE, false, F>();
     if (e == hipSuccess) e = allow_big_lds_fused<STEPS, SKN_EPI_STORE, true, F>();
     if (e == hipSuccess) e = allow_big_lds_fused<STEPS, SKN_EPI_ADD, false, F>();
+    if (e == hipSuccess) e = allow_big_lds_fused<STEPS, SKN_EPI_ADD, false, F, 1>();
     if (e == hipSuccess) e = allow_big_lds_fused<STEPS, SKN_EPI_ADD, true, F>();
     if (e == hipSuccess) e = allow_big_lds_fused<STEPS, SKN_EPI_SWIGLU, false, F>();
     if (e == hipSuccess) e = allow_big_lds_fused<STEPS, SKN_EPI_SWIGLU, true, F>();
     if (e == hipSuccess) e = allow_big_lds_fused<STEPS, SKN_EPI_ROPE, false, F>();
     if (e == hipSuccess) e = allow_big_lds_fused<STEPS, SKN_EPI_ROPE, true, F>();
+    return e;
+}
+
+template <int F>
+hipError_t allow_big_lds_two() {
+    hipError_t e = hipSuccess;
+    auto allow = [&](const void* f) {
+        if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    };
+    allow(reinterpret_cast<const void*>(matvec_fused_two_formats_kernel<1, kFmtQ6K, F>));
+    allow(reinterpret_cast<const void*>(matvec_fused_two_formats_kernel<2, kFmtQ6K, F>));
+    allow(reinterpret_cast<const void*>(matvec_fused_two_formats_kernel<3, kFmtQ6K, F>));
+    allow(reinterpret_cast<const void*>(matvec_fused_two_formats_kernel<4, kFmtQ6K, F>));
     return e;
 }
 
@@ -1929,6 +1983,9 @@ static int skn_matvec_init(skn_ctx* ctx) {
     SKN_ALLOW_FUSED(kFmtTQ2);
     SKN_ALLOW_FUSED(kFmtTQ1);
 #undef SKN_ALLOW_FUSED
+    SKN_HIP(ctx, allow_big_lds_two<kFmtQ4K>());
+    SKN_HIP(ctx, allow_big_lds_two<kFmtQ5K>());
+    SKN_HIP(ctx, allow_big_lds_two<kFmtQ80>());
     return SKN_OK;
 }
 static skn_family register_family(skn_matvec_init);
@@ -2004,6 +2061,30 @@ int skn_matvec_q4k_fused(skn_ctx* ctx, const skn_q4k_segments& seg, int n_out, i
         default: SKN_FUSED(kFmtQ4K)
     }
 #undef SKN_FUSED
+}
+
+// q, k, v of two formats in one launch where one is Q6_K and the other Q4_K, Q5_K or Q8_0 (each segment list holds the rows of its
+// format, the rest empty); SKN_ERR_TYPE without a message for other pairs.
+int skn_matvec_fused_two(skn_ctx* ctx, const skn_q4k_segments& q6, int n_q6, const skn_q4k_segments& other, int n_other, int other_type, int k,
+                         const float* x, const float* norm_w, float eps, float* y, const skn_rope_epilogue& rope) {
+    if (other_type != SKN_TYPE_Q4_K && other_type != SKN_TYPE_Q5_K && other_type != SKN_TYPE_Q8_0) return SKN_ERR_TYPE;
+    SKN_REQUIRE(ctx, k > 0 && k % 256 == 0 && k <= 16384 && n_q6 > 0 && n_other > 0, SKN_ERR_SHAPE, "fused matvec of two formats: unsupported shape");
+    const uintptr_t mask = other_type == SKN_TYPE_Q8_0 ? 3 : 15;
+    for (int i = 0; i < 3; i++)
+        SKN_REQUIRE(ctx, (q6.rows[i] == 0 || (q6.w[i] && ((uintptr_t)q6.w[i] & 1) == 0)) && (other.rows[i] == 0 || (other.w[i] && ((uintptr_t)other.w[i] & mask) == 0)),
+                    SKN_ERR_ARG, "fused matvec of two formats: null or misaligned weights");
+    const int nb = k / 256;
+#define SKN_TWO(F)                                                                                                              \
+    switch ((nb + 15) / 16) {                                                                                                   \
+        case 1: return launch_fused_beside_q6k<1, F>(ctx, q6, n_q6, other, n_other, nb, x, norm_w, eps, y, rope);               \
+        case 2: return launch_fused_beside_q6k<2, F>(ctx, q6, n_q6, other, n_other, nb, x, norm_w, eps, y, rope);               \
+        case 3: return launch_fused_beside_q6k<3, F>(ctx, q6, n_q6, other, n_other, nb, x, norm_w, eps, y, rope);               \
+        default: return launch_fused_beside_q6k<4, F>(ctx, q6, n_q6, other, n_other, nb, x, norm_w, eps, y, rope);              \
+    }
+    if (other_type == SKN_TYPE_Q4_K) SKN_TWO(kFmtQ4K)
+    if (other_type == SKN_TYPE_Q5_K) SKN_TWO(kFmtQ5K)
+    SKN_TWO(kFmtQ80)
+#undef SKN_TWO
 }
 
 // Test hook: one launch of the decoder's fused matvec, so that each fused form can be held against the oracle as an

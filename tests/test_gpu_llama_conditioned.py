@@ -152,6 +152,51 @@ def test_41_token_prompt_then_decode_steps(hip, case, fused, graph):
         model.free()
 
 
+@pytest.mark.parametrize("other", [12, 13, 8])
+@pytest.mark.parametrize("six", [("wv",), ("wq",), ("wk", "wv")])
+@pytest.mark.parametrize("hidden,n_kv", [(512, 2), (256, 1)])
+def test_q6k_beside_another_format_in_one_launch(hip, other, six, hidden, n_kv):
+    """Decode steps of layers whose q, k and v are Q6_K and one other format: one launch for both, a workgroup boundary between
+    them, each with the rows of its own matrices (four and two query heads of 128 and 64: segments that end inside a workgroup's
+    sixteen rows do not exist, 256 and 512 rows of values do)."""
+    types = {f"l{l}.{w}": 14 if w in six else other for l in range(2) for w in ("wq", "wk", "wv")}
+    cfg = llama.Config(n_layer=2, hidden=hidden, ffn=768, n_head=4, n_kv_head=n_kv, head_dim=hidden // 4, vocab=512, max_tokens=96, page_tokens=16,
+                       matrix_types=types)
+    w = llama.conditioned_weights(cfg, SEED)
+    ora, model = OracleLlama(cfg, w), llama.LlamaModel(hip, cfg, weights=w)
+    before = hip.stat("launches")
+    hip.set_option("llama.graph", 0)
+    try:
+        for i, t in enumerate(tokens(20, cfg.vocab)):
+            ora.step(t)
+            model.decode(t, 1)
+            err = logit_err(model.logits(), ora.logits)
+            assert err <= DECODE_TOL, (other, six, i, err)
+    finally:
+        hip.set_option("llama.graph", 1)
+    # (state, embedding, five launches a layer, norm, head, choice)
+    assert hip.stat("launches") - before == 20 * (2 + 2 * 5 + 3), "q, k and v took more than one launch"
+    model.free()
+
+
+@pytest.mark.parametrize("head_dim,context", [(64, 500), (128, 250), (256, 120)])
+def test_contexts_of_one_round_take_one_workgroup_per_head(hip, head_dim, context):
+    """Decode steps up to, at and past the tokens that a workgroup takes in one round (512, 256, 128): one workgroup per head with
+    nothing to merge below, split partials merged by the projection above."""
+    cfg = llama.Config(n_layer=2, hidden=512, ffn=768, n_head=512 // head_dim, head_dim=head_dim, vocab=512, max_tokens=640, page_tokens=16)
+    w = llama.conditioned_weights(cfg, SEED)
+    ora, model = OracleLlama(cfg, w), llama.LlamaModel(hip, cfg, weights=w)
+    prompt = tokens(context, cfg.vocab, seed=2)
+    ora.prefill(prompt, bf16_gemm=True)
+    model.prefill(prompt)
+    for i, t in enumerate(tokens(24, cfg.vocab, seed=4)):
+        ora.step(t)
+        model.decode(t, 1)
+        err = logit_err(model.logits(), ora.logits)
+        assert err <= 8e-3, (head_dim, context + i, err)  # (the bound of the long-prompt test)
+    model.free()
+
+
 def test_several_steps_per_call_equal_one_step_per_call(hip):
     """skn_llama_decode with n steps feeds its own greedy tokens back: the same tokens and final logits as n calls."""
     cfg = CASES["q4_k_kv2"]
