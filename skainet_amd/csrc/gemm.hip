@@ -338,6 +338,7 @@ struct Q4kFragSegs {
     // part[blockIdx.y][m][part_cols], matrix i at column part_col0[i] (a pair: gate, then up); null: no split
     float* part;
     int part_cols, part_col0[3];
+    int part_blocks;  // superblocks of a workgroup (all of a row's: no split)
 };
 
 // the kernel's LDS (weight buffers, then the tile exchange) exceeds the static limit (the scales of the tile's rows follow it): dynamic, opted in per
@@ -352,7 +353,7 @@ constexpr int frag_lds_bytes() {
 // superblock, against the 1e-3 asked of the op); the superblock's integer products then add to it as they come
 // out of the matrix core, and so does the "- dmin * m_j" term: one more sixteen-deep product per tile between
 // the activation sub-block sums (fp16 hi | lo) and -(dmin / cs) * m_j * 2^12, itself split into an fp16 pair.
-template <int MT, int MH>
+template <int MT, int MH, bool SPLIT>
 __global__ __launch_bounds__(256 * MH) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restrict__ sfrag, const Q4kFragSegs segs,
                           const float* __restrict__ inv_scale, int m, int k, uint32_t a_bytes) {
@@ -367,7 +368,7 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
     const int h = lane >> 5, r = lane & 31;
     const int nb = k >> 8, nch = k >> 6;
     // (this workgroup's superblocks: all of them, or a part of k)
-    const int sb0 = nb * (int)blockIdx.y / (int)gridDim.y, sb1 = nb * ((int)blockIdx.y + 1) / (int)gridDim.y;
+    const int sb0 = SPLIT ? (int)blockIdx.y * segs.part_blocks : 0, sb1 = SPLIT ? min(sb0 + segs.part_blocks, nb) : nb;
     const int groups = (sb1 - sb0 + 3) >> 2;
     // tile -> (row tile, weight matrix, column tile): the column tiles of up to three matrices sharing the
     // activations are laid side by side
@@ -623,7 +624,7 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                         // register x of lane l: row 8 (x / 4) + 4 (l / 32) + x % 4 of the 32 x 32 tile
                         const int row = (mb0 + i) * 32 + 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3);
                         if (row < m && col < n) {
-                            if (segs.part) {
+                            if constexpr (SPLIT) {
                                 float* dst = segs.part + ((size_t)blockIdx.y * m + row) * segs.part_cols + col;
                                 dst[0] = g, dst[segs.part_col0[1]] = u;
                                 continue;
@@ -648,7 +649,7 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                 float sc[16];
 #pragma unroll
                 for (int x = 0; x < 16; x++) sc[x] = isc_lds[(mh * MT + i) * 32 + 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3)];
-                if (segs.part)
+                if constexpr (SPLIT)
                     store_tile_part(sum, segs.part + (size_t)blockIdx.y * m * segs.part_cols + segs.part_col0[seg], segs.part_cols, (mb0 + i) * 32,
                                     n0 + 32 * j, m, n, lane);
                 else
@@ -704,7 +705,7 @@ int launch_frag(skn_ctx* ctx, int m_tiles, const u32x4* afrag, const u32x4* sfra
                 int m, int k, int splits) {
     constexpr int kLds = frag_lds_bytes<MT, MH>() + 32 * MT * MH * 4;
     const uint32_t a_bytes = (uint32_t)((size_t)m_tiles * 32 * MT * MH * k * 2);  // (checked by the caller to fit)
-    skn_launch(ctx, gemm_q4k_frag_kernel<MT, MH>, dim3(m_tiles * segs.n_tiles, splits), dim3(256 * MH), kLds, afrag, sfrag, segs, isc, m, k, a_bytes);
+    skn_launch(ctx, splits > 1 ? gemm_q4k_frag_kernel<MT, MH, true> : gemm_q4k_frag_kernel<MT, MH, false>, dim3(m_tiles * segs.n_tiles, splits), dim3(256 * MH), kLds, afrag, sfrag, segs, isc, m, k, a_bytes);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
@@ -748,9 +749,12 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
     const int h = lane >> 5, r = lane & 31;
     const int nb = k >> 8, nch = k >> 6;
     // the last tiles are shared by tail.splits workgroups each, neighbours in the grid, with a part of k each
-    const int over = (int)blockIdx.x - tail.tile0, z = over < 0 ? 0 : over % tail.splits;
-    const int tile = over < 0 ? (int)blockIdx.x : tail.tile0 + over / tail.splits, parts = over < 0 ? 1 : tail.splits;
-    const int sb0 = nb * z / parts, sb1 = nb * (z + 1) / parts;
+    int tile = (int)blockIdx.x, z = 0, parts = 1, sb0 = 0, sb1 = nb;
+    if (tile >= tail.tile0) {
+        const int over = tile - tail.tile0;
+        parts = tail.splits, z = over % parts, tile = tail.tile0 + over / parts;
+        sb0 = nb * z / parts, sb1 = nb * (z + 1) / parts;
+    }
     const int mt = tile % m_tiles, tn = tile / m_tiles;  // (the row tiles of a column tile run side by side)
     const bool pair = segs.pair != 0;
     const int seg = pair ? 0 : (tn >= segs.tile0[2] ? 2 : (tn >= segs.tile0[1] ? 1 : 0));
@@ -1262,11 +1266,11 @@ struct Q6kHalf {
     u32x4 qa[2], qb[2], qh[2];  // per 32-column block: ql + 16 h, ql + 32 + 16 h, qh + 16 h of the half
 };
 
-template <int MT>
+template <int MT, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_q6k_frag_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restrict__ w, const float* __restrict__ inv_scale,
                           float* __restrict__ c, int m, int n, int k, int m_tiles, int n_tiles, int accumulate,
-                          uint32_t a_bytes, uint32_t w_bytes, int xcd_rows, float* __restrict__ part) {
+                          uint32_t a_bytes, uint32_t w_bytes, int xcd_rows, float* __restrict__ part, int part_blocks) {
     extern __shared__ __align__(16) float red[];  // 2 MT tiles x 3 copies x 1024 floats
     const int lane = threadIdx.x & 63;
     const int kq = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -1287,7 +1291,7 @@ void gemm_q6k_frag_kernel(const u32x4* __restrict__ afrag, const uint8_t* __rest
     if (tn >= n_tiles) return;
     const int nb = k >> 8, nch = k >> 6;
     // (this workgroup's superblocks: all of them, or a part of k whose products go unscaled to part[blockIdx.y][m][n])
-    const int sb0 = nb * (int)blockIdx.y / (int)gridDim.y, sb1 = nb * ((int)blockIdx.y + 1) / (int)gridDim.y;
+    const int sb0 = SPLIT ? (int)blockIdx.y * part_blocks : 0, sb1 = SPLIT ? min(sb0 + part_blocks, nb) : nb;
     // The weights are read with buffer loads too: the lane's byte offset (its weight row, its sixteen-byte half) plus
     // a scalar one (superblock, piece).  A piece of an odd superblock starts at an address that is only a multiple
     // of two.
@@ -1459,7 +1463,7 @@ void gemm_q6k_frag_kernel(const u32x4* __restrict__ afrag, const uint8_t* __rest
                 for (int o = 0; o < 3; o++)
 #pragma unroll
                     for (int x = 0; x < 16; x++) sum[x] += red[(t * 3 + o) * 1024 + 64 * x + lane];
-                if (part) store_tile_part(sum, part + (size_t)blockIdx.y * m * n, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, lane);
+                if constexpr (SPLIT) store_tile_part(sum, part + (size_t)blockIdx.y * m * n, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, lane);
                 else store_tile(sum, c, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, inv_scale, lane, accumulate != 0);
             }
         }
@@ -1477,10 +1481,11 @@ constexpr int kQ6Stage = 4 * 4 * 1024;         // a phase of one pair: four k-st
 constexpr int kQ6Aux = 2 * 256 + 256;          // per pair: the ratios of two superblocks in turn, then the last unit
 constexpr int kQ6PcLds = 4 * 2 * kQ6Stage + 4 * kQ6Aux;
 
+template <bool SPLIT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restrict__ w, const float* __restrict__ inv_scale,
                         float* __restrict__ c, int m, int n, int k, int m_tiles, int n_tiles, int accumulate,
-                        uint32_t a_bytes, uint32_t w_bytes, float* __restrict__ part) {
+                        uint32_t a_bytes, uint32_t w_bytes, float* __restrict__ part, int part_blocks) {
     constexpr int MT = 4;
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1492,7 +1497,7 @@ void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restri
     const int mt = xcd % m_tiles, tn = (blockIdx.x >> 3) * per + xcd / m_tiles;
     if (tn >= n_tiles) return;
     const int nb = k >> 8, nch = k >> 6;
-    const int sb0 = nb * (int)blockIdx.y / (int)gridDim.y, sb1 = nb * ((int)blockIdx.y + 1) / (int)gridDim.y;  // (as above)
+    const int sb0 = SPLIT ? (int)blockIdx.y * part_blocks : 0, sb1 = SPLIT ? min(sb0 + part_blocks, nb) : nb;  // (as above)
     const int nsb = (sb1 - sb0 + 3) >> 2;  // superblocks of the busiest pair
     uint8_t* stage = lds + kq * 2 * kQ6Stage;
     uint8_t* aux = lds + 4 * 2 * kQ6Stage + kq * kQ6Aux;
@@ -1736,7 +1741,7 @@ void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restri
                     for (int o = 0; o < 3; o++)
 #pragma unroll
                         for (int x = 0; x < 16; x++) sum[x] += red[(t * 3 + o) * 1024 + 64 * x + lane];
-                    if (part) store_tile_part(sum, part + (size_t)blockIdx.y * m * n, n, (mt * MT + ii) * 32, tn * kBN + 32 * j, m, n, lane);
+                    if constexpr (SPLIT) store_tile_part(sum, part + (size_t)blockIdx.y * m * n, n, (mt * MT + ii) * 32, tn * kBN + 32 * j, m, n, lane);
                     else store_tile(sum, c, n, (mt * MT + ii) * 32, tn * kBN + 32 * j, m, n, inv_scale, lane, accumulate != 0);
                 }
             }
@@ -2007,25 +2012,25 @@ void gemm_q6k_tall_kernel(const u32x4* __restrict__ afrag, const uint8_t* __rest
     }
 }
 
-template <int MT>
+template <int MT, bool SPLIT>
 int launch_q6k_gemm(skn_ctx* ctx, const u32x4* afrag, const uint8_t* w, const float* isc, float* c, int m, int n, int k,
                     int accumulate, int splits, float* part) {
     constexpr int kLds = 2 * MT * 3 * 4096;
     const int m_tiles = (m + 32 * MT - 1) / (32 * MT), n_tiles = (n + kBN - 1) / kBN;
-    const int xcd_rows = 8 % m_tiles == 0 ? 1 : 0;
+    const int xcd_rows = 8 % m_tiles == 0 ? 1 : 0, part_blocks = (k / 256 + splits - 1) / splits;
     const unsigned grid = xcd_rows ? (unsigned)(8 * ((n_tiles + 8 / m_tiles - 1) / (8 / m_tiles))) : (unsigned)(((n_tiles + 7) / 8) * 8 * m_tiles);
     const uint32_t a_bytes = (uint32_t)((size_t)m_tiles * 32 * MT * k * 2);  // (checked by the caller to fit)
     const uint32_t w_bytes = (uint32_t)((size_t)n * (k / 256) * 210);  // (checked by the caller to fit)
     // 128-row tiles: the kernel with specialised wavefronts (measured 6 - 11 % faster); option value 2 keeps to the other
     // (up to 16384 elements per row: a rescale per superblock rounds the accumulators once more, the other form does not)
     if (MT == 4 && xcd_rows && k <= 16384 && ctx->opt_gemm_q6k_fused != 2) {
-        skn_launch(ctx, gemm_q6k_pc_kernel, dim3(grid, splits), dim3(512), kQ6PcLds, afrag, w, isc, c, m, n, k, m_tiles, n_tiles, accumulate,
-                   a_bytes, w_bytes, part);
+        skn_launch(ctx, gemm_q6k_pc_kernel<SPLIT>, dim3(grid, splits), dim3(512), kQ6PcLds, afrag, w, isc, c, m, n, k, m_tiles, n_tiles, accumulate,
+                   a_bytes, w_bytes, part, part_blocks);
         SKN_LAUNCH_CHECK(ctx);
         return SKN_OK;
     }
-    skn_launch(ctx, gemm_q6k_frag_kernel<MT>, dim3(grid, splits), dim3(256), kLds, afrag, w, isc, c, m, n, k, m_tiles, n_tiles, accumulate,
-               a_bytes, w_bytes, xcd_rows, part);
+    skn_launch(ctx, gemm_q6k_frag_kernel<MT, SPLIT>, dim3(grid, splits), dim3(256), kLds, afrag, w, isc, c, m, n, k, m_tiles, n_tiles, accumulate,
+               a_bytes, w_bytes, xcd_rows, part, part_blocks);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
@@ -2033,10 +2038,14 @@ int launch_q6k_gemm(skn_ctx* ctx, const u32x4* afrag, const uint8_t* w, const fl
 int launch_q6k_gemm_mt(skn_ctx* ctx, int mt, const u32x4* afrag, const uint8_t* w, const float* isc, float* c, int m, int n,
                        int k, int accumulate, int splits, float* part) {
     if (splits < 2) part = nullptr;
-    if (mt == 1) SKN_TRY(launch_q6k_gemm<1>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part));
-    else if (mt == 2) SKN_TRY(launch_q6k_gemm<2>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part));
-    else SKN_TRY(launch_q6k_gemm<4>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part));
-    if (!part) return SKN_OK;
+    if (!part) {
+        if (mt == 1) return launch_q6k_gemm<1, false>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part);
+        if (mt == 2) return launch_q6k_gemm<2, false>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part);
+        return launch_q6k_gemm<4, false>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part);
+    }
+    if (mt == 1) SKN_TRY((launch_q6k_gemm<1, true>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part)));
+    else if (mt == 2) SKN_TRY((launch_q6k_gemm<2, true>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part)));
+    else SKN_TRY((launch_q6k_gemm<4, true>(ctx, afrag, w, isc, c, m, n, k, accumulate, splits, part)));
     const skn_gemm_parts ps = {{c, nullptr, nullptr}, {n, 0, 0}, {0, 0, 0}, {accumulate, 0, 0}, 1, 0};
     return skn_gemm_add_parts(ctx, part, splits, n, ps, isc, m);
 }
@@ -2061,8 +2070,9 @@ int skn_gemm_add_parts(skn_ctx* ctx, const float* part, int splits, int cols, co
 // 19.6, Q6_K 333 x 4096 x 4096 59 against 54): the addition costs 3 us and the parts their way through memory.
 int skn_gemm_k_splits(const skn_ctx* ctx, int m, int tiles, int nb) {
     if (m > 65535) return 1;  // (a grid dimension of the addition)
-    if (ctx->opt_gemm_split > 0) return std::min(ctx->opt_gemm_split, nb);
-    return std::max(1, std::min({ctx->compute_units / tiles, (nb + 3) / 4, 16}));
+    const int want = ctx->opt_gemm_split > 0 ? std::min(ctx->opt_gemm_split, nb) : std::max(1, std::min({ctx->compute_units / tiles, (nb + 3) / 4, 16}));
+    const int each = (nb + want - 1) / want;
+    return (nb + each - 1) / each;  // (no workgroup without a superblock)
 }
 
 int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out) {
@@ -2085,17 +2095,23 @@ int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out) {
 // Dynamic LDS above 48 KiB must be allowed per kernel and device; done once per context here so that no launch
 // path has to.
 static int skn_gemm_init(skn_ctx* ctx) {
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 2>() + 32 * 2 * 2 * 4));
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 1>() + 32 * 2 * 1 * 4));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 2, false>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 2>() + 32 * 2 * 2 * 4));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 2, true>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 2>() + 32 * 2 * 2 * 4));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 1, false>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 1>() + 32 * 2 * 1 * 4));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 1, true>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 1>() + 32 * 2 * 1 * 4));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_tall_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kTlLds));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_hilo_frag_kernel<1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 1 * 3 * 4096));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_hilo_frag_kernel<2, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 2 * 3 * 4096));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_hilo_frag_kernel<4, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 4 * 3 * 4096));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_tall_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kQ6TlLds));
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_pc_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kQ6PcLds));
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_frag_kernel<1>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 1 * 3 * 4096));
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_frag_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 2 * 3 * 4096));
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_frag_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 4 * 3 * 4096));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_pc_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, kQ6PcLds));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_pc_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, kQ6PcLds));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_frag_kernel<1, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 1 * 3 * 4096));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_frag_kernel<1, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 1 * 3 * 4096));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_frag_kernel<2, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 2 * 3 * 4096));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_frag_kernel<2, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 2 * 3 * 4096));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_frag_kernel<4, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 4 * 3 * 4096));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q6k_frag_kernel<4, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 4 * 3 * 4096));
     return SKN_OK;
 }
 static skn_family register_family(skn_gemm_init);
@@ -2172,6 +2188,7 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
         fs.part_cols += segs[i].n;
     }
     for (int i = 0; i < 3; i++) fs.part_col0[i] = ps.col0[i];
+    fs.part_blocks = (k / 256 + splits - 1) / splits;
     const size_t part_bytes = tall ? (size_t)tail.tiles * tail.splits * 131072 : splits > 1 ? (size_t)splits * m * fs.part_cols * 4 : 0;
     uint8_t* ws;
     int rc = skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes + part_bytes, &ws);

@@ -333,7 +333,7 @@ template <typename F, int MT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_blocks_kernel(const u32x4* __restrict__ afrag, const u32x4* __restrict__ sfrag, const uint8_t* __restrict__ w,
                         const float* __restrict__ inv_scale, float* __restrict__ c, int m, int n, int k, int m_tiles, int n_tiles, int accumulate,
-                        uint32_t a_bytes, uint32_t w_bytes, float* __restrict__ part) {
+                        uint32_t a_bytes, uint32_t w_bytes, float* __restrict__ part, int part_blocks) {
     extern __shared__ __align__(16) uint8_t lds[];  // a superblock of 64 rows per wavefront, then the exchange of the tiles
     constexpr int P = F::kBytes / 16;               // sixteen-byte pieces of a row's superblock
     const int lane = threadIdx.x & 63;
@@ -343,7 +343,7 @@ void gemm_blocks_kernel(const u32x4* __restrict__ afrag, const u32x4* __restrict
     const int mt = slot_in_xcd % m_tiles, tn = (slot_in_xcd / m_tiles) * 8 + (blockIdx.x & 7);
     if (tn >= n_tiles) return;
     const int nb = k >> 8;
-    const int sb0 = nb * (int)blockIdx.y / (int)gridDim.y, sb1 = nb * ((int)blockIdx.y + 1) / (int)gridDim.y;
+    const int sb0 = (int)blockIdx.y * part_blocks, sb1 = min(sb0 + part_blocks, nb);  // (all, or a part of k)
 
     const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, (int)w_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc((void*)afrag, 0, (int)a_bytes, 0x00020000);
@@ -489,7 +489,7 @@ int launch_blocks(skn_ctx* ctx, const u32x4* afrag, const u32x4* sfrag, const fl
     const unsigned grid = (unsigned)(((n_tiles + 7) / 8) * 8 * m_tiles);
     const uint32_t a_bytes = (uint32_t)((size_t)m_tiles * 32 * MT * k * 2), w_bytes = (uint32_t)((size_t)seg.n * (k / 256) * F::kBytes);
     skn_launch(ctx, gemm_blocks_kernel<F, MT>, dim3(grid, splits), dim3(256), blocks_lds_bytes<F, MT>(), afrag, sfrag, (const uint8_t*)seg.w, isc, seg.c, m,
-               seg.n, k, m_tiles, n_tiles, seg.accumulate, a_bytes, w_bytes, splits > 1 ? part : (float*)nullptr);
+               seg.n, k, m_tiles, n_tiles, seg.accumulate, a_bytes, w_bytes, splits > 1 ? part : (float*)nullptr, (k / 256 + splits - 1) / splits);
     SKN_LAUNCH_CHECK(ctx);
     if (splits < 2) return SKN_OK;
     const skn_gemm_parts ps = {{seg.c, nullptr, nullptr}, {seg.n, 0, 0}, {0, 0, 0}, {seg.accumulate, 0, 0}, 1, 0};
