@@ -252,6 +252,37 @@ def test_prefill_attention_vs_oracle(hip, n_head, dim, page, cached, n_queries):
     kv.free()
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("cached,n_queries", [(1, 1), (31, 31), (32, 32), (33, 33), (64, 32), (65, 32), (63, 32), (96, 33), (97, 31), (160, 5)])
+def test_prefill_attention_tiles_with_and_without_a_mask(hip, dim, cached, n_queries):
+    """Tiles that every query of a block sees take no causal mask: the first and the last query of a block at, before and after
+    an edge of 32 keys, with fewer tiles than wavefronts, and with scores so far apart that most weights are zero.  In both cases
+    a key let in too many (or left out) would be the one with the largest score: keys grow along the sequence."""
+    n_head = 2
+    rng = np.random.default_rng(cached * 100 + n_queries)
+    q = np.abs(rng.standard_normal((n_queries, n_head, dim))).astype(np.float32)
+    k = (np.abs(rng.standard_normal((1, cached, n_head, dim))) * (1 + np.arange(cached) / 16.0)[None, :, None, None]).astype(np.float16).view(np.uint16)
+    v = rng.standard_normal((1, cached, n_head, dim)).astype(np.float16).view(np.uint16)
+    kv = hip.kv_cache(1, n_head, dim, 16, cached + 16)
+    kv.append_run(0, hip.to_device(k[0]), hip.to_device(v[0]), cached)
+    for scale in (1.0 / np.sqrt(dim) / 16, 4.0):
+        out = hip.alloc(q.nbytes)
+        kv.attn_prefill(0, hip.to_device(q), n_queries, out, scale)
+        got = out.download(np.float32, q.size).reshape(q.shape)
+        ctx_len = [cached - n_queries + t + 1 for t in range(n_queries)]
+        kk = np.ascontiguousarray(np.broadcast_to(k, (n_queries,) + k.shape[1:]))
+        vv = np.ascontiguousarray(np.broadcast_to(v, (n_queries,) + v.shape[1:]))
+        want = oracle_c.attn_decode(q, kk, vv, ctx_len, scale)
+        # q enters as an fp16 pair (22 bits) and the scores are fp32 sums of `dim` products: a score of size s is off by no more
+        # than s (2^-21 + dim 2^-24), a weight by that much of itself, a row by twice that
+        qa, ka = np.abs(q).astype(np.float64), np.abs(k[0].view(np.float16)).astype(np.float64)
+        s_max = scale * np.einsum("thd,khd->thk", qa, ka).max()
+        bound = TOL + 2 * s_max * (2.0**-21 + dim * 2.0**-24)
+        for t in range(n_queries):
+            assert oracle_np.rel_err(got[t], want[t]) <= bound, (scale, t)
+    kv.free()
+
+
 def test_prefill_attention_arguments_and_closed_form(hip):
     n_head, dim, tok = 2, 128, 96
     kv = hip.kv_cache(1, n_head, dim, 32, 128)
