@@ -12,7 +12,7 @@
 // stream per query head, nothing is staged and no barrier is met while tokens stream.  A step's launch computes the two
 // norms of its own token in its prologue (every workgroup for itself, from L2) while its first rows are on their way.
 #include "attention_stream.h"
-#include "dense.h"
+#include "dense_beside.h"
 #include "kv.h"
 
 #include <algorithm>
@@ -79,17 +79,15 @@ __device__ __forceinline__ void block_sum2(float& a, float& b, float* red) {
     for (int i = 0; i < nw; i++) a += red[i], b += red[nw + i];
 }
 
-// grid (splits, kv heads x head groups, query rows)
 template <typename E, int D, int QG, bool STEP>
-__global__ __launch_bounds__(kThreads) void shared_attn_kernel(const AttnArgs p) {
+__device__ __forceinline__ void shared_attn_block(const AttnArgs& p, const int split, const int hg, const int row) {
     constexpr int LPT = D / 8, G = 64 / LPT, NS = kWaves * G, U = kU;
     __shared__ float so[kWaves][QG][D];
     __shared__ float sm[kWaves][QG], sl[kWaves][QG];
     __shared__ float red[2 * kWaves];
     __shared__ __align__(16) float qs[STEP ? QG * D : 4];
-    const int split = blockIdx.x, row = blockIdx.z;
     const int per_kv = p.n_head / p.kv_heads, n_groups = (per_kv + QG - 1) / QG;
-    const int kvh = blockIdx.y / n_groups, h0 = kvh * per_kv + (blockIdx.y % n_groups) * QG, h_end = (kvh + 1) * per_kv;
+    const int kvh = hg / n_groups, h0 = kvh * per_kv + (hg % n_groups) * QG, h_end = (kvh + 1) * per_kv;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = lane % LPT, g = lane / LPT, stream = wave * G + g;
     // what does not wait for the position is requested first: the token's projections, whose norms are computed while the
@@ -132,7 +130,7 @@ __global__ __launch_bounds__(kThreads) void shared_attn_kernel(const AttnArgs p)
         block_sum2(sq, sk, red);
         newest_scale = 1.0f / sqrtf(sk / (float)(p.kv_heads * p.dim) + p.eps);
         fq *= query_temperature(n - 1, p.temp_coef, p.temp_every) / sqrtf(sq / (float)(p.n_head * p.dim) + p.eps);
-        if (split == 0 && blockIdx.y == 0 && tid == 0) {  // for the steps to come (this one uses its own)
+        if (split == 0 && hg == 0 && tid == 0) {  // for the steps to come (this one uses its own)
             const int pi = (n - 1) / p.page_tokens;
             p.key_scale[(int64_t)p.table[pi] * p.page_tokens + (n - 1) - pi * p.page_tokens] = newest_scale;
         }
@@ -251,6 +249,21 @@ __global__ __launch_bounds__(kThreads) void shared_attn_kernel(const AttnArgs p)
     }
 }
 
+// grid (splits, kv heads x head groups, query rows)
+template <typename E, int D, int QG, bool STEP>
+__global__ __launch_bounds__(kThreads) void shared_attn_kernel(const AttnArgs p) {
+    shared_attn_block<E, D, QG, STEP>(p, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// a step's attention and a product beside it: grid (workgroups of the attention, then s.blocks)
+template <typename E, int D, int QG, typename W>
+__global__ __launch_bounds__(kThreads) void shared_attn_beside_kernel(const AttnArgs p, int attn_blocks, const skn_beside s, int plane) {
+    extern __shared__ __align__(16) float4 lds4[];
+    const int b = blockIdx.x;
+    if (b < attn_blocks) shared_attn_block<E, D, QG, true>(p, b % p.n_splits, b / p.n_splits, 0);
+    else beside_block<W, kThreads>(s, b - attn_blocks, plane, lds4);
+}
+
 // one workgroup per row: norms, temperature, the query in its padded layout with the key's norm weights, the key to the cache
 template <typename E>
 __global__ __launch_bounds__(256) void shared_prep_kernel(const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk,
@@ -289,28 +302,41 @@ int heads_per_group(const skn_ctx* ctx, int per_kv, int kv_heads, int splits) {
 }
 
 template <typename E, int D, int QG, bool STEP>
-int launch_as(skn_ctx* ctx, const AttnArgs& a, int rows) {
-    const int per_kv = a.n_head / a.kv_heads;
-    skn_launch(ctx, shared_attn_kernel<E, D, QG, STEP>, dim3(a.n_splits, a.kv_heads * ((per_kv + QG - 1) / QG), rows), dim3(kThreads), 0, a);
+int launch_as(skn_ctx* ctx, const AttnArgs& a, int rows, const skn_beside& beside) {
+    const int per_kv = a.n_head / a.kv_heads, hgs = a.kv_heads * ((per_kv + QG - 1) / QG);
+    if constexpr (STEP) {
+        if (beside.w) {
+            const int attn_blocks = a.n_splits * hgs, plane = skn_beside_plane(beside);
+            const dim3 grid((unsigned)(attn_blocks + beside.blocks));
+            const size_t lds = skn_beside_lds(beside);
+            if (beside.type == SKN_TYPE_F32)
+                skn_launch(ctx, shared_attn_beside_kernel<E, D, QG, float>, grid, dim3(kThreads), lds, a, attn_blocks, beside, plane);
+            else
+                skn_launch(ctx, shared_attn_beside_kernel<E, D, QG, uint16_t>, grid, dim3(kThreads), lds, a, attn_blocks, beside, plane);
+            SKN_LAUNCH_CHECK(ctx);
+            return SKN_OK;
+        }
+    }
+    skn_launch(ctx, shared_attn_kernel<E, D, QG, STEP>, dim3(a.n_splits, hgs, rows), dim3(kThreads), 0, a);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
 
 template <int D, bool STEP>
-int launch_dim(skn_ctx* ctx, const skn_kv* kv, const AttnArgs& a, int rows) {
-    if (kv->elem_type == SKN_TYPE_F32) return launch_as<float, D, 1, STEP>(ctx, a, rows);
+int launch_dim(skn_ctx* ctx, const skn_kv* kv, const AttnArgs& a, int rows, const skn_beside& beside) {
+    if (kv->elem_type == SKN_TYPE_F32) return launch_as<float, D, 1, STEP>(ctx, a, rows, beside);
     if constexpr (STEP) {
         const int qg = heads_per_group(ctx, a.n_head / a.kv_heads, a.kv_heads, a.n_splits);
-        if (qg == 2) return launch_as<uint16_t, D, 2, true>(ctx, a, rows);
+        if (qg == 2) return launch_as<uint16_t, D, 2, true>(ctx, a, rows, beside);
     }
-    return launch_as<uint16_t, D, 1, STEP>(ctx, a, rows);
+    return launch_as<uint16_t, D, 1, STEP>(ctx, a, rows, beside);
 }
 
 template <bool STEP>
-int launch_attn(skn_ctx* ctx, const skn_kv* kv, const AttnArgs& a, int rows) {
-    if (kv->head_dim == 64) return launch_dim<64, STEP>(ctx, kv, a, rows);
-    if (kv->head_dim == 128) return launch_dim<128, STEP>(ctx, kv, a, rows);
-    return launch_dim<256, STEP>(ctx, kv, a, rows);
+int launch_attn(skn_ctx* ctx, const skn_kv* kv, const AttnArgs& a, int rows, const skn_beside& beside = {}) {
+    if (kv->head_dim == 64) return launch_dim<64, STEP>(ctx, kv, a, rows, beside);
+    if (kv->head_dim == 128) return launch_dim<128, STEP>(ctx, kv, a, rows, beside);
+    return launch_dim<256, STEP>(ctx, kv, a, rows, beside);
 }
 
 AttnArgs base_args(const skn_kv* kv, int seq, const skn_shared_attn& p) {
@@ -376,7 +402,7 @@ int skn_shared_attn_rows(skn_ctx* ctx, skn_kv* kv, int seq, const skn_shared_att
 }
 
 int skn_shared_attn_step(skn_ctx* ctx, skn_kv* kv, int seq, const skn_shared_attn& p, const float* q, const float* k, const int32_t* state_dev,
-                         int n_splits, float* opart, float* ml, float* out) {
+                         int n_splits, float* opart, float* ml, float* out, const skn_beside* beside) {
     SKN_TRY(check(ctx, kv, p));
     SKN_REQUIRE(ctx, n_splits >= 1 && n_splits <= kMaxSplits && (n_splits == 1 ? out != nullptr : opart && ml), SKN_ERR_ARG,
                 "shared attention: %d splits without their buffers", n_splits);
@@ -389,8 +415,13 @@ int skn_shared_attn_step(skn_ctx* ctx, skn_kv* kv, int seq, const skn_shared_att
     a.ml = ml;
     a.out = out;
     a.out_type = SKN_TYPE_F32;
-    return launch_attn<true>(ctx, kv, a, 1);
+    if (!beside) return launch_attn<true>(ctx, kv, a, 1);
+    skn_beside s = *beside;
+    skn_beside_plan(ctx, s, kThreads);
+    return launch_attn<true>(ctx, kv, a, 1, s);
 }
+
+size_t skn_shared_attn_step_lds(const skn_kv* kv) { return (size_t)2 * kv->head_dim * (kWaves + 1) * sizeof(float) + 1024; }
 
 // Splits for contexts up to max_ctx: a power of two, at most eight (sixteen where few heads would read a long context: the
 // merge reads every split in every workgroup that follows), so that a workgroup has at least a round of requests.

@@ -18,7 +18,7 @@
 // (Decays enter the triangles as ratios of products over at most sixteen tokens: any decay from 0.01 to 1 is safe in fp32.)
 // A decode step is one launch, one workgroup per head: the decay's low-rank product, the step, the head's norm and the gate.
 #include "delta.h"
-#include "dense.h"
+#include "dense_beside.h"
 #include "rstate.h"
 
 #include <algorithm>
@@ -306,11 +306,12 @@ __global__ __launch_bounds__(256) void delta_gate_kernel(const float* __restrict
 
 // one workgroup of NW wavefronts per head
 template <int L, int NW, typename W>
-__global__ __launch_bounds__(64 * NW) void delta_step_kernel(const skn_delta_step p, int dim, float* __restrict__ state) {
+__device__ __forceinline__ void delta_step_block(const skn_delta_step& p, int dim, float* __restrict__ state) {
     constexpr int DP = 8 * L, CW = 64 / L, kThreads = 64 * NW;  // columns per wavefront
     constexpr int kPasses = (DP + NW * CW - 1) / (NW * CW);
     __shared__ __align__(16) float vec[5][DP];  // k, w, b, r, v
     __shared__ float so[DP], red[NW];
+    static_assert((6 * DP + NW) * sizeof(float) <= kDeltaStepLds, "what a product beside a step counts on");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = blockIdx.x, rl = lane & (L - 1);
     const int off = h * dim;
     // the state first: it does not wait for anything
@@ -382,6 +383,19 @@ __global__ __launch_bounds__(64 * NW) void delta_step_kernel(const skn_delta_ste
     for (int d = tid; d < dim; d += kThreads) p.y[off + d] = so[d] * inv * p.norm[off + d] * p.g[off + d];
 }
 
+template <int L, int NW, typename W>
+__global__ __launch_bounds__(64 * NW) void delta_step_kernel(const skn_delta_step p, int dim, float* __restrict__ state) {
+    delta_step_block<L, NW, W>(p, dim, state);
+}
+
+// a step and a product (of weights of the same type) beside it: grid (heads, then s.blocks)
+template <int L, int NW, typename W>
+__global__ __launch_bounds__(64 * NW) void delta_step_beside_kernel(const skn_delta_step p, int dim, float* __restrict__ state, int heads, const skn_beside s, int plane) {
+    extern __shared__ __align__(16) float4 lds4[];
+    if ((int)blockIdx.x < heads) delta_step_block<L, NW, W>(p, dim, state);
+    else beside_block<W, 64 * NW>(s, (int)blockIdx.x - heads, plane, lds4);
+}
+
 template <int DP>
 int launch_rows(skn_ctx* ctx, const skn_rstate* st, const float* r, const float* k, const float* v, const float* w, const float* a, int ld, int n, float* ops,
                 float* state, float* o) {
@@ -396,7 +410,19 @@ int launch_rows(skn_ctx* ctx, const skn_rstate* st, const float* r, const float*
 }
 
 template <int L, int NW>
-int launch_step(skn_ctx* ctx, const skn_rstate* st, const skn_delta_step& p, float* state) {
+int launch_step(skn_ctx* ctx, const skn_rstate* st, const skn_delta_step& p, float* state, const skn_beside* beside) {
+    if (beside) {
+        SKN_REQUIRE(ctx, beside->type == p.w2_type, SKN_ERR_TYPE, "delta rule: a product of another type beside a step");
+        skn_beside s = *beside;
+        skn_beside_plan(ctx, s, 64 * NW);
+        const dim3 grid((unsigned)(st->heads + s.blocks));
+        const int plane = skn_beside_plane(s);
+        const size_t lds = skn_beside_lds(s);
+        if (s.type == SKN_TYPE_F32) skn_launch(ctx, delta_step_beside_kernel<L, NW, float>, grid, dim3(64 * NW), lds, p, st->dim, state, st->heads, s, plane);
+        else skn_launch(ctx, delta_step_beside_kernel<L, NW, uint16_t>, grid, dim3(64 * NW), lds, p, st->dim, state, st->heads, s, plane);
+        SKN_LAUNCH_CHECK(ctx);
+        return SKN_OK;
+    }
     if (p.w2_type == SKN_TYPE_F32) skn_launch(ctx, delta_step_kernel<L, NW, float>, dim3(st->heads), dim3(64 * NW), 0, p, st->dim, state);
     else skn_launch(ctx, delta_step_kernel<L, NW, uint16_t>, dim3(st->heads), dim3(64 * NW), 0, p, st->dim, state);
     SKN_LAUNCH_CHECK(ctx);
@@ -433,13 +459,13 @@ int skn_delta_gate_rows(skn_ctx* ctx, const float* o, const float* g, int ldg, c
     return SKN_OK;
 }
 
-int skn_delta_step_launch(skn_ctx* ctx, skn_rstate* st, int seq, const skn_delta_step& p) {
+int skn_delta_step_launch(skn_ctx* ctx, skn_rstate* st, int seq, const skn_delta_step& p, const skn_beside* beside) {
     float* s = st->seq_state(seq);
     switch (st->dim_pad) {
-        case 32: return launch_step<4, 2>(ctx, st, p, s);
-        case 64: return launch_step<8, 8>(ctx, st, p, s);
-        case 128: return launch_step<16, 16>(ctx, st, p, s);
-        default: return launch_step<32, 16>(ctx, st, p, s);
+        case 32: return launch_step<4, 2>(ctx, st, p, s, beside);
+        case 64: return launch_step<8, 8>(ctx, st, p, s, beside);
+        case 128: return launch_step<16, 16>(ctx, st, p, s, beside);
+        default: return launch_step<32, 16>(ctx, st, p, s, beside);
     }
 }
 

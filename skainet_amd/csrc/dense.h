@@ -16,6 +16,7 @@ struct skn_dense_mat {
     int rows = 0;                 // stacked rows, a multiple of 32
     int k_pad = 0;                // a multiple of 64
     const float* bias = nullptr;  // [rows] or null
+    int ld = 0;                   // matvec only: elements from row to row, a multiple of 64 (0: k_pad)
 };
 
 // what a segment does to z = W x (+ bias)

@@ -177,7 +177,7 @@ __device__ __forceinline__ void stage_merge(const skn_matvec_src& s, const XPlan
 
 // W: uint16_t (bf16) or float.  LDS: two planes of `plane` float4, then the scratch of the staging.
 template <typename W, int MODE>
-__global__ __launch_bounds__(kThreads) void dense_matvec_kernel(const W* __restrict__ w, int rows, int k_pad, int plane,
+__global__ __launch_bounds__(kThreads) void dense_matvec_kernel(const W* __restrict__ w, int rows, int k_pad, int ld, int plane,
                                                                 const float* __restrict__ bias, const skn_matvec_src src,
                                                                 const skn_dense_out out) {
     extern __shared__ __align__(16) float4 lds4[];
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(kThreads) void dense_matvec_kernel(const W* __restr
     auto fetch = [&](u32x4(&buf)[kR][kU], int g, int t) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < kR; r++) {
-            const u32x4* row = reinterpret_cast<const u32x4*>(w + (int64_t)min(kR * g + r, rows - 1) * k_pad);
+            const u32x4* row = reinterpret_cast<const u32x4*>(w + (int64_t)min(kR * g + r, rows - 1) * ld);
 #pragma unroll
             for (int u = 0; u < kU; u++) buf[r][u] = row[min((t * kU + u) * 64 + lane, pieces - 1)];  // (past the end: times a zero of x)
         }
@@ -330,7 +330,7 @@ int launch(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, cons
     // no more workgroups than fit on the device at once: a staging serves all the rows its wavefronts walk through
     const int groups = (w.rows + kR - 1) / kR, per_cu = std::min(kPerCu, (int)(kMaxLds / lds));
     const int blocks = std::min((groups + kWaves - 1) / kWaves, per_cu * ctx->compute_units);
-    skn_launch(ctx, dense_matvec_kernel<W, MODE>, dim3((unsigned)blocks), dim3(kThreads), lds, (const W*)w.w, w.rows, w.k_pad, plane, w.bias, src, out);
+    skn_launch(ctx, dense_matvec_kernel<W, MODE>, dim3((unsigned)blocks), dim3(kThreads), lds, (const W*)w.w, w.rows, w.k_pad, w.ld ? w.ld : w.k_pad, plane, w.bias, src, out);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
@@ -364,7 +364,7 @@ skn_family register_family(dense_matvec_init);
 }  // namespace
 
 int skn_dense_matvec(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, const skn_dense_out& out) {
-    SKN_REQUIRE(ctx, w.w && w.rows > 0 && w.k_pad > 0 && w.k_pad % kDenseColPad == 0 && ((uintptr_t)w.w & 15) == 0, SKN_ERR_ARG,
+    SKN_REQUIRE(ctx, w.w && w.rows > 0 && w.k_pad > 0 && w.k_pad % kDenseColPad == 0 && w.ld % kDenseColPad == 0 && (w.ld == 0 || w.ld >= w.k_pad) && ((uintptr_t)w.w & 15) == 0, SKN_ERR_ARG,
                 "dense matvec: bad matrix (%d x %d)", w.rows, w.k_pad);
     SKN_REQUIRE(ctx, src.x0 && ((uintptr_t)src.x0 & 15) == 0 && src.k0 > 0 && src.k0 <= w.k_pad, SKN_ERR_ARG, "dense matvec: bad input");
     SKN_REQUIRE(ctx, !src.x1 || (src.off1 >= src.k0 && src.off1 % 4 == 0 && src.off1 + src.k1 <= w.k_pad && ((uintptr_t)src.x1 & 15) == 0), SKN_ERR_ARG,

@@ -13,7 +13,7 @@
 // same products as GEMMs with the same epilogues, and the row-wise parts between them.
 // Weights are bf16 or fp32; with fp32 weights every operand, the cached rows included, is fp32.
 // The decode loop around a step is csrc/stepper.h; pages come from csrc/kv.h and states from csrc/rstate.h.
-#include "dense.h"
+#include "dense_beside.h"
 #include "kv.h"
 #include "rstate.h"
 #include "stepper.h"
@@ -199,8 +199,30 @@ skn_dense_out side_segment(const skn_hybrid* m, int l, const int32_t* tokens, vo
 
 // ---- decode -----------------------------------------------------------------------------------------------------------
 
+// The feed-forward's part of the output product, to run beside the mixer (no w: it stays in the output product).  Wherever the mixer
+// can take it: the two together read what they read apart, in a launch that is at least as full; the limit is the LDS that a launch
+// has without asking for more (feed-forwards of 14336 columns beside the delta rule, 12288, 10240 and 6144
+// beside attention heads of 64, 128 and 256).
+skn_beside ff_beside(const skn_hybrid* m, const Layer& L, float* x) {
+    skn_beside s;
+    const bool general_delta = L.p.mixer == SKN_MIX_GENERAL_DELTA;
+    if (L.p.mixer != SKN_MIX_SHARED_ATTN && !general_delta) return s;
+    s.type = L.out.type;
+    s.rows = m->cfg.width;
+    s.k_pad = L.out.k_pad - L.off_ff;
+    s.ld = L.out.k_pad;
+    s.x = m->mid;
+    s.k = L.p.ff;
+    s.resid = x;
+    s.mult = m->cfg.residual_mult;
+    const size_t mixer_lds = general_delta ? kDeltaStepLds : skn_shared_attn_step_lds(L.kv);
+    if (skn_beside_lds(s) + mixer_lds > kBesideMaxLds || (general_delta && L.decay.type != s.type)) return s;
+    s.w = (const uint8_t*)L.out.w + (size_t)L.off_ff * (s.type == SKN_TYPE_F32 ? 4 : 2);
+    return s;
+}
+
 // the mixer of a decode step, from m->cols to m->mix, or to the split partials that `src` then names
-int mixer_step(skn_ctx* ctx, skn_hybrid* m, Layer& L, int max_ctx, skn_matvec_src& src) {
+int mixer_step(skn_ctx* ctx, skn_hybrid* m, Layer& L, int max_ctx, skn_matvec_src& src, const skn_beside* beside) {
     const float* col[kStepCols];
     for (int i = 0; i < kStepCols; i++) col[i] = m->cols + (int64_t)i * m->max_cols;
     const int32_t* state = m->step.state;
@@ -217,7 +239,7 @@ int mixer_step(skn_ctx* ctx, skn_hybrid* m, Layer& L, int max_ctx, skn_matvec_sr
     switch (L.p.mixer) {
         case SKN_MIX_SHARED_ATTN: {
             const int splits = skn_shared_attn_splits(ctx, L.kv, L.shared.n_head, max_ctx);
-            SKN_TRY(skn_shared_attn_step(ctx, L.kv, 0, L.shared, col[0], col[1], state, splits, m->opart, m->ml, m->mix));
+            SKN_TRY(skn_shared_attn_step(ctx, L.kv, 0, L.shared, col[0], col[1], state, splits, m->opart, m->ml, m->mix, beside));
             merge(splits, L.shared.n_head, L.kv->dim);
             return SKN_OK;
         }
@@ -263,7 +285,7 @@ int mixer_step(skn_ctx* ctx, skn_hybrid* m, Layer& L, int max_ctx, skn_matvec_sr
             d.norm = L.p.o_norm;
             d.eps = m->cfg.norm_eps;
             d.y = m->mix;
-            return skn_delta_step_launch(ctx, L.state, 0, d);
+            return skn_delta_step_launch(ctx, L.state, 0, d, beside);
         }
     }
 }
@@ -309,13 +331,21 @@ int decode_step(skn_ctx* ctx, skn_hybrid* m, int max_ctx) {
         skn_matvec_src src;
         src.x0 = m->mix;
         src.k0 = L.hd;
+        skn_dense_mat out = L.out;
+        skn_beside ff;
         if (L.p.ff && !L.p.norm2) {
-            src.x1 = m->mid;
-            src.off1 = L.off_ff;
-            src.k1 = L.p.ff;
+            ff = ff_beside(m, L, x);
+            if (ff.w) {
+                out.k_pad = L.off_ff;
+                out.ld = L.out.k_pad;
+            } else {
+                src.x1 = m->mid;
+                src.off1 = L.off_ff;
+                src.k1 = L.p.ff;
+            }
         }
-        SKN_TRY(mixer_step(ctx, m, L, max_ctx, src));
-        SKN_TRY(skn_dense_matvec(ctx, L.out, src, residual(m, x)));
+        SKN_TRY(mixer_step(ctx, m, L, max_ctx, src, ff.w ? &ff : nullptr));
+        SKN_TRY(skn_dense_matvec(ctx, out, src, residual(m, x)));
         if (L.p.ff && L.p.norm2) {
             normed(L.p.norm2);
             skn_dense_out up;

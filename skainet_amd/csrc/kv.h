@@ -67,7 +67,8 @@ int skn_shared_attn_rows(skn_ctx* ctx, skn_kv* kv, int seq, const skn_shared_att
 // state_dev: device {token, position, context length, ...}.  n_splits == 1: out [n_head * dim] fp32; otherwise the
 // unmerged partials opart[split][head][head_dim] and ml[split][head] (maximum in units of log2 e, sum).
 int skn_shared_attn_step(skn_ctx* ctx, skn_kv* kv, int seq, const skn_shared_attn& p, const float* q, const float* k, const int32_t* state_dev,
-                         int n_splits, float* opart, float* ml, float* out);
+                         int n_splits, float* opart, float* ml, float* out, const struct skn_beside* beside = nullptr);
+size_t skn_shared_attn_step_lds(const skn_kv* kv);  // at most, of a workgroup without a product beside it
 int skn_shared_attn_splits(skn_ctx* ctx, const skn_kv* kv, int n_head, int max_ctx);
 // the matrix-core form for prompts (csrc/attention_prefill.hip): fp16 caches, head_dim 64 or 128
 int skn_shared_attn_prefill_launch(skn_ctx* ctx, skn_kv* kv, int seq, const float* q_prep, int n_queries, int first_ctx, int n_head, float scale,

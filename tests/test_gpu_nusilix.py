@@ -46,6 +46,20 @@ def test_prompts_portions_and_single_tokens_match_the_oracle(hip, name, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,ff", [(48, 1023), (48, 1025), (48, 2048), (48, 2049), (33, 5000), (48, 13000), (40, 17000), (4200, 70)])
+def test_feed_forward_beside_the_mixer_of_a_step(hip, width, ff, dtype):
+    """A step's output product over the feed-forward's columns runs in the mixer's launch: rows of one, of two (the first past a
+    multiple of 1024 or 2048 columns) and of many turns, more rows than wavefronts in flight, and columns whose input does not fit
+    beside the mixer's LDS, which stay with the mixer's columns."""
+    cfg = cases.model([cases.attention(2, 1, 16, ff=ff), cases.delta(2, 24, ff=ff), cases.delta(1, 48, ff=ff)], width=width, vocab=40, groups=1)
+    w = cases.weights(cfg, 4, seed=ff)
+    toks = cases.tokens(cfg, 8, seed=2)
+    m = cases.device_model(hip, cfg, w, dtype)
+    cases.check(run(m, toks, [1] * 8), orc.forward(cfg, w, toks), dtype, (width, ff))
+    m.free()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_logits_do_not_depend_on_the_cut(hip, dtype):
     cfg, rank = cases.MODELS["mixed"]
     w = cases.weights(cfg, rank)
