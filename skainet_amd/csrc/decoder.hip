@@ -97,31 +97,43 @@ __global__ __launch_bounds__(1024) void embed_rows_kernel(const uint8_t* __restr
 }
 
 // Rotary embedding of q and k rows at positions pos0 + row (pos0 from device), then k and v rows go to the
-// cache as fp16 at those positions.  grid = (rows, n_head), block = head_dim / 2 threads (one pair each); q has
-// n_head heads per row, k and v kv_heads (the first kv_heads blocks of a row handle them).
-__global__ void rope_store_kernel(float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+// cache as fp16 at those positions.  grid = (rows, parts of the heads); q has n_head heads per row, k and v kv_heads.
+// LDS: a sine and a cosine per pair of a head.  They are computed in double precision, which bound the kernel when every
+// head, in a workgroup of half a wavefront at 64 elements, computed its own: 2000 rows of 32 + 8 heads of 64 19.3 -> 9.6 us
+// (45 MB: what a copy takes), 512 rows of 32 + 32 heads of 128 8.7 -> 8.6 us.
+__global__ __launch_bounds__(256) void rope_store_kernel(float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
                                   uint16_t* __restrict__ k_pool, uint16_t* __restrict__ v_pool,
                                   const int32_t* __restrict__ table, const int32_t* __restrict__ pos0_dev, int n_head,
                                   int kv_heads, int head_dim, int page_tokens, double log2_base) {
-    const int row = blockIdx.x, h = blockIdx.y, i = threadIdx.x;
+    extern __shared__ float2 turn[];  // cosine, sine
+    const int row = blockIdx.x, half = head_dim >> 1, tid = threadIdx.x;
     const int pos = pos0_dev[0] + row;
-    float sn, cs;
-    skn_rope_sincos(pos, 2 * i, head_dim, log2_base, &sn, &cs);
-    const size_t qbase = ((size_t)row * n_head + h) * head_dim + 2 * i;
-    const float qa = q[qbase], qb = q[qbase + 1];
-    q[qbase] = qa * cs - qb * sn;
-    q[qbase + 1] = qa * sn + qb * cs;
-    if (h >= kv_heads) return;
-    const size_t base = ((size_t)row * kv_heads + h) * head_dim + 2 * i;
-    const float ka = k[base], kb = k[base + 1];
-    const float k0 = ka * cs - kb * sn, k1 = ka * sn + kb * cs;
+    for (int i = tid; i < half; i += 256) skn_rope_sincos(pos, 2 * i, head_dim, log2_base, &turn[i].y, &turn[i].x);
     const int page = table[pos / page_tokens];
-    const size_t dst = (((size_t)page * kv_heads + h) * page_tokens + (pos % page_tokens)) * head_dim + 2 * i;
-    const uint32_t kk = (uint32_t)__half_as_ushort(__float2half_rn(k0)) | ((uint32_t)__half_as_ushort(__float2half_rn(k1)) << 16);
-    const uint32_t vv = (uint32_t)__half_as_ushort(__float2half_rn(v[base])) |
-                        ((uint32_t)__half_as_ushort(__float2half_rn(v[base + 1])) << 16);
-    *reinterpret_cast<uint32_t*>(k_pool + dst) = kk;
-    *reinterpret_cast<uint32_t*>(v_pool + dst) = vv;
+    const size_t page_row = (size_t)page * kv_heads * page_tokens + pos % page_tokens;
+    __syncthreads();
+    float2* qr = reinterpret_cast<float2*>(q) + (size_t)row * n_head * half;
+    const float2* kr = reinterpret_cast<const float2*>(k) + (size_t)row * kv_heads * half;
+    const float2* vr = reinterpret_cast<const float2*>(v) + (size_t)row * kv_heads * half;
+    auto rotate = [&](float2 x, int i) {
+        const float2 t = turn[i];
+        return make_float2(x.x * t.x - x.y * t.y, x.x * t.y + x.y * t.x);
+    };
+    auto pack = [](float2 x) { return (uint32_t)__half_as_ushort(__float2half_rn(x.x)) | ((uint32_t)__half_as_ushort(__float2half_rn(x.y)) << 16); };
+    const int first = blockIdx.y * 256 + tid, step = gridDim.y * 256;
+    for (int e = first; e < n_head * half; e += step) qr[e] = rotate(qr[e], e % half);
+    for (int e = first; e < kv_heads * half; e += step) {
+        const int h = e / half, i = e - h * half;
+        const size_t dst = (page_row + (size_t)h * page_tokens) * half + i;
+        reinterpret_cast<uint32_t*>(k_pool)[dst] = pack(rotate(kr[e], i));
+        reinterpret_cast<uint32_t*>(v_pool)[dst] = pack(vr[e]);
+    }
+}
+
+// workgroups for the heads of a row, eight on a compute unit where there is work for them (512 rows: four take 8.9 us, eight 8.6)
+dim3 rope_grid(const skn_ctx* ctx, int rows, int n_head, int head_dim) {
+    const int most = (n_head * (head_dim / 2) + 255) / 256, want = (8 * ctx->compute_units + rows - 1) / rows;
+    return dim3((unsigned)rows, (unsigned)std::min(most, want));
 }
 
 // grid = rows, block = 256.  Rows of up to 8192 elements (multiple of 4) stay in registers between the two
@@ -281,7 +293,7 @@ int decode_step(skn_ctx* ctx, skn_llama* m, int units) {
             SKN_TRY(skn_matvec_q(ctx, L.type_q, L.wq, H, H, m->xn, m->q));
             SKN_TRY(skn_matvec_q(ctx, L.type_k, L.wk, KVD, H, m->xn, m->k));
             SKN_TRY(skn_matvec_q(ctx, L.type_v, L.wv, KVD, H, m->xn, m->v));
-            skn_launch(ctx, rope_store_kernel, dim3(1, NH), dim3(D / 2), 0, m->q, (const float*)m->k, (const float*)m->v,
+            skn_launch(ctx, rope_store_kernel, rope_grid(ctx, 1, NH, D), dim3(256), (size_t)D / 2 * sizeof(float2), m->q, (const float*)m->k, (const float*)m->v,
                        kv->k_pool, kv->v_pool, (const int32_t*)kv->page_table_dev, (const int32_t*)(m->step.state + 1), NH, KVH, D,
                        kv->page_tokens, log2((double)c.rope_base));
             SKN_LAUNCH_CHECK(ctx);
@@ -642,7 +654,7 @@ int skn_llama_prefill(skn_ctx* ctx, skn_llama* m, const int32_t* tokens_host, in
             if (expand) SKN_TRY(project_expanded(ctx, m, l, 0, types, blocks, rows, outs, 3, H, m->px, L.attn_norm, T, 0));
             else SKN_TRY(project_rows(ctx, m, types, blocks, rows, outs, 3, H, m->px, L.attn_norm, T, 0));
         }
-        skn_launch(ctx, rope_store_kernel, dim3(T, NH), dim3(D / 2), 0, m->pq, (const float*)m->pk, (const float*)m->pv,
+        skn_launch(ctx, rope_store_kernel, rope_grid(ctx, T, NH, D), dim3(256), (size_t)D / 2 * sizeof(float2), m->pq, (const float*)m->pk, (const float*)m->pv,
                    kv->k_pool, kv->v_pool, (const int32_t*)kv->page_table_dev, (const int32_t*)(m->step.state + 1), NH, KVH, D,
                    kv->page_tokens, log2((double)c.rope_base));
         SKN_LAUNCH_CHECK(ctx);
