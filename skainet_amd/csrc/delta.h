@@ -32,5 +32,26 @@ __device__ __forceinline__ float dot_over_lanes(const Vec8& a, const Vec8& s) {
 
 __device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ f32x4 load4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+// of a lane's byte offset from an address that all lanes share
+__device__ __forceinline__ f32x4 load4(const float* p, uint32_t bytes) { return *reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(p) + bytes); }
+__device__ __forceinline__ float load1(const float* p, uint32_t bytes) { return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + bytes); }
+
+// The wavefronts that share a tile of sixteen state columns on a prompt.  Each has kOwn of the DP / 16 tiles of channels: its part
+// of S, and of every product with S, whose sum over the wavefronts passes through LDS; of the products over the chunk's tokens and
+// of the output rows it takes kRows in four.
+template <int DP>
+struct ScanSplit {
+    static constexpr int kTiles = DP / 16, kWaves = kTiles < 4 ? kTiles : 4, kOwn = kTiles / kWaves, kRows = 4 / kWaves;
+};
+__device__ __forceinline__ float element(const f32x4& v, int e) { return e == 0 ? v[0] : e == 1 ? v[1] : e == 2 ? v[2] : v[3]; }
+// what the wavefronts wrote to LDS is there (their requests to memory go on)
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+template <int NW>
+__device__ __forceinline__ f32x4 sum_parts(const f32x4 (*part)[64], int lane) {
+    f32x4 v = part[0][lane];
+#pragma unroll
+    for (int w = 1; w < NW; w++) v += part[w][lane];
+    return v;
+}
 
 }  // namespace

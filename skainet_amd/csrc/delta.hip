@@ -13,8 +13,9 @@
 // four triangles on the matrix cores, solves with I + beta, and leaves
 //   Y = K1 S + A1 V,  O = R1 S + G1 V     (K1 = (I + beta)^-1 K0, A1 = (I + beta)^-1 alpha, R1 = R0 - delta K1, G1 = gamma - delta A1)
 // as operands in the order in which the matrix instructions take them.  delta_scan_kernel then walks the chunks with one
-// wavefront per head and sixteen columns, its part of S in accumulator layout -- which is also the layout of a column operand,
-// so S and Y are multiplied as they stand -- and no LDS, no barrier: a chunk's operands are coalesced loads one chunk ahead.
+// workgroup per head and sixteen columns, its wavefronts' parts of S in accumulator layout -- which is also the layout of a column
+// operand, so S and Y are multiplied as they stand.  The wavefronts have a part of the channels each; their parts of Y meet in LDS
+// behind one barrier per chunk, those of O a chunk later.  A chunk's operands are coalesced loads one to three chunks ahead.
 // (Decays enter the triangles as ratios of products over at most sixteen tokens: any decay from 0.01 to 1 is safe in fp32.)
 // A decode step is one launch, one workgroup per head: the decay's low-rank product, the step, the head's norm and the gate.
 #include "delta.h"
@@ -189,92 +190,119 @@ __global__ __launch_bounds__(64) void delta_chunk_kernel(const float* __restrict
 
 template <int DP>
 struct ChunkOps {
-    static constexpr int kTiles = DP / 16;
-    f32x4 k1[kTiles], r1[kTiles], kt[kTiles], bt[kTiles], w[kTiles], v, a1, g1;
-    __device__ __forceinline__ void load(const float* p, int lane, int tile) {
+    using Split = ScanSplit<DP>;
+    static constexpr int kOwn = Split::kOwn, kRows = Split::kRows;
+    f32x4 k1[kOwn], r1[kOwn], kt[kOwn], bt[kOwn], w[kOwn], v;
+    float a1[kRows], g1[kRows];
+    __device__ __forceinline__ void load(const float* p, uint32_t lane, uint32_t wave, uint32_t tile) {
+        const uint32_t own = (wave * kOwn * 64 + lane) * 16, row = (16 * wave * kOwn + 4 * (lane >> 4)) * 4, some = lane * 16 + wave * kRows * 4;
 #pragma unroll
-        for (int j = 0; j < kTiles; j++) {
-            k1[j] = load4(p + off_k1(DP) + (j * 64 + lane) * 4);
-            r1[j] = load4(p + off_r1(DP) + (j * 64 + lane) * 4);
+        for (int i = 0; i < kOwn; i++) {
+            k1[i] = load4(p + off_k1(DP) + 256 * i, own);
+            r1[i] = load4(p + off_r1(DP) + 256 * i, own);
         }
-        v = load4(p + off_v(DP) + (tile * 64 + lane) * 4);
-        a1 = load4(p + off_a1(DP) + lane * 4);
-        g1 = load4(p + off_g1(DP) + lane * 4);
+        v = load4(p + off_v(DP), (tile * 64 + lane) * 16);
 #pragma unroll
-        for (int j = 0; j < kTiles; j++) {
-            kt[j] = load4(p + off_kt(DP) + (j * 64 + lane) * 4);
-            bt[j] = load4(p + off_bt(DP) + (j * 64 + lane) * 4);
-            w[j] = load4(p + off_w(DP) + 16 * j + 4 * (lane >> 4));
+        for (int i = 0; i < kRows; i++) {
+            a1[i] = load1(p + off_a1(DP) + i, some);
+            g1[i] = load1(p + off_g1(DP) + i, some);
+        }
+#pragma unroll
+        for (int i = 0; i < kOwn; i++) {
+            w[i] = load4(p + off_w(DP) + 16 * i, row);
+            kt[i] = load4(p + off_kt(DP) + 256 * i, own);
+            bt[i] = load4(p + off_bt(DP) + 256 * i, own);
         }
     }
 };
 
-// One wavefront per head and tile of sixteen columns.  The wavefronts of a head are on one XCD (blockIdx % 8): they read the
-// same operands, which then come from memory once.
+// One workgroup per head and tile of sixteen columns.  The workgroups of a head are on one XCD (blockIdx % 8): they read the
+// same operands, which then come from memory once.  A chunk's matrix instructions are a chain on one SIMD otherwise (72 of 32
+// clocks at 64 channels): 1000 tokens of 32 heads of 64, one wavefront 90 us, four 48.
 template <int DP>
-__global__ __launch_bounds__(64) void delta_scan_kernel(const float* __restrict__ ops, int n, int chunks, int heads, int dim, float* __restrict__ state,
+__global__ __launch_bounds__(64 * ScanSplit<DP>::kWaves) __attribute__((amdgpu_waves_per_eu(DP <= 128 ? 2 : 1, 2))) void delta_scan_kernel(const float* __restrict__ ops, int n, int chunks, int heads, int dim, float* __restrict__ state,
                                                         float* __restrict__ o, float* __restrict__ trash) {
-    constexpr int kTiles = DP / 16;
-    const int lane = threadIdx.x, tiles = (dim + 15) / 16, turn = (int)(blockIdx.x >> 3), h = (int)(blockIdx.x & 7) + 8 * (turn / tiles), tile = turn % tiles;
+    using Split = ScanSplit<DP>;
+    constexpr int NW = Split::kWaves, kOwn = Split::kOwn, kRows = Split::kRows, R = DP <= 64 ? 4 : 2;  // chunks in registers (what they hold without spilling)
+    __shared__ f32x4 part_y[2][NW][64], part_z[2][NW][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int tiles = (dim + 15) / 16, turn = (int)(blockIdx.x >> 3), h = (int)(blockIdx.x & 7) + 8 * (turn / tiles), tile = turn % tiles;
     if (h >= heads) return;
     // (lanes beyond the last column compute along on zeros of V and store nothing)
     const int col = 16 * tile + (lane & 15);
     const bool live = col < dim;
-    float* sp = state + ((int64_t)h * dim + min(col, dim - 1)) * DP + 4 * (lane >> 4);
-    f32x4 s[kTiles];
+    float* sp = state + ((int64_t)h * dim + min(col, dim - 1)) * DP + 16 * wave * kOwn + 4 * (lane >> 4);
+    f32x4 s[kOwn];
 #pragma unroll
-    for (int j = 0; j < kTiles; j++) s[j] = load4(sp + 16 * j);
+    for (int j = 0; j < kOwn; j++) s[j] = load4(sp + 16 * j);
     const float* src = ops + (int64_t)h * chunks * chunk_floats(DP);
 
-    auto step = [&](const ChunkOps<DP>& x, int chunk) __attribute__((always_inline)) {
-        f32x4 y = {0.f, 0.f, 0.f, 0.f}, z = y;
-#pragma unroll
-        for (int e = 0; e < 4; e++) y = mma(x.a1[e], x.v[e], y), z = mma(x.g1[e], x.v[e], z);
-#pragma unroll
-        for (int j = 0; j < kTiles; j++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) y = mma(x.k1[j][e], s[j][e], y), z = mma(x.r1[j][e], s[j][e], z);
-#pragma unroll
-        for (int j = 0; j < kTiles; j++) s[j] *= x.w[j];
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-#pragma unroll
-            for (int j = 0; j < kTiles; j++) s[j] = mma(x.kt[j][e], x.v[e], s[j]);
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-#pragma unroll
-            for (int j = 0; j < kTiles; j++) s[j] = mma(x.bt[j][e], y[e], s[j]);
-        // (one store per token whatever the lane: a skipped one would leave the number of requests outstanding unknown, and
+    const int t_own = 4 * (lane >> 4) + wave * kRows;
+    float* o_own = o + ((int64_t)t_own * heads + h) * dim + col;
+    // this wavefront's rows of the outputs of a chunk
+    auto store = [&](int chunk) __attribute__((always_inline)) {
+        const f32x4 z = sum_parts<NW>(part_z[chunk & 1], lane);
+        // (one store per row whatever the lane: a skipped one would leave the number of requests outstanding unknown, and
         // the wait for the next chunk's operands would wait for the stores)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int t = chunk * kChunk + 4 * (lane >> 4) + e;
-            float* dst = live && t < n ? o + ((int64_t)t * heads + h) * dim + col : trash + lane;
-            *dst = z[e];
+        for (int i = 0; i < kRows; i++) {
+            const int t = chunk * kChunk + t_own + i;
+            float* dst = live && t >= 0 && t < n ? o_own + (int64_t)(chunk * kChunk + i) * heads * dim : trash + lane;
+            *dst = element(z, wave * kRows + i);
         }
     };
-    ChunkOps<DP> even;
-    if constexpr (DP <= 128) {
-        ChunkOps<DP> odd;
-        even.load(src, lane, tile);
-        for (int c = 0; c < chunks; c += 2) {
-            odd.load(src + (int64_t)min(c + 1, chunks - 1) * chunk_floats(DP), lane, tile);
+    auto step = [&](const ChunkOps<DP>& x, int chunk) __attribute__((always_inline)) {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        f32x4 y[2] = {zero, zero}, z[2] = {zero, zero};
+#pragma unroll
+        for (int i = 0; i < kRows; i++) y[i & 1] = mma(x.a1[i], element(x.v, wave * kRows + i), y[i & 1]);
+#pragma unroll
+        for (int j = 0; j < kOwn; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) y[e & 1] = mma(x.k1[j][e], s[j][e], y[e & 1]);
+        part_y[chunk & 1][wave][lane] = y[0] + y[1];
+#pragma unroll
+        for (int i = 0; i < kRows; i++) z[i & 1] = mma(x.g1[i], element(x.v, wave * kRows + i), z[i & 1]);
+#pragma unroll
+        for (int j = 0; j < kOwn; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) z[e & 1] = mma(x.r1[j][e], s[j][e], z[e & 1]);
+#pragma unroll
+        for (int j = 0; j < kOwn; j++) s[j] *= x.w[j];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int j = 0; j < kOwn; j++) s[j] = mma(x.kt[j][e], x.v[e], s[j]);
+        lds_barrier();  // (a buffer is written again two barriers after the reads of the chunk that had it)
+        const f32x4 all = sum_parts<NW>(part_y[chunk & 1], lane);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int j = 0; j < kOwn; j++) s[j] = mma(x.bt[j][e], all[e], s[j]);
+        store(chunk - 1);
+        part_z[chunk & 1][wave][lane] = z[0] + z[1];
+    };
+    ChunkOps<DP> x[R];
+#pragma unroll
+    for (int r = 0; r < R - 1; r++) x[r].load(src + (int64_t)min(r, chunks - 1) * chunk_floats(DP), lane, wave, tile);
+    int c = 0;
+    for (; c + R <= chunks; c += R) {  // (no condition inside: the number of requests outstanding is known)
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            x[(r + R - 1) % R].load(src + (int64_t)min(c + r + R - 1, chunks - 1) * chunk_floats(DP), lane, wave, tile);
             __builtin_amdgcn_sched_barrier(0);
-            step(even, c);
-            if (c + 1 == chunks) break;
-            even.load(src + (int64_t)min(c + 2, chunks - 1) * chunk_floats(DP), lane, tile);
+            step(x[r], c + r);
             __builtin_amdgcn_sched_barrier(0);
-            step(odd, c + 1);
-        }
-    } else {
-        for (int c = 0; c < chunks; c++) {
-            even.load(src + (int64_t)c * chunk_floats(DP), lane, tile);
-            step(even, c);
         }
     }
+#pragma unroll
+    for (int r = 0; r < R - 1; r++)
+        if (c + r < chunks) step(x[r], c + r);
+    lds_barrier();
+    store(chunks - 1);
     if (live) {
 #pragma unroll
-        for (int j = 0; j < kTiles; j++) *reinterpret_cast<f32x4*>(sp + 16 * j) = s[j];
+        for (int j = 0; j < kOwn; j++) *reinterpret_cast<f32x4*>(sp + 16 * j) = s[j];
     }
 }
 
@@ -403,7 +431,7 @@ int launch_rows(skn_ctx* ctx, const skn_rstate* st, const float* r, const float*
     skn_launch(ctx, delta_chunk_kernel<DP>, dim3(chunks, st->heads), dim3(64), 0, r, k, v, w, a, ld, n, st->heads, st->dim, ops);
     SKN_LAUNCH_CHECK(ctx);
     float* trash = ops + (size_t)chunks * st->heads * chunk_floats(DP);
-    skn_launch(ctx, delta_scan_kernel<DP>, dim3((unsigned)((st->heads + 7) / 8 * 8 * tiles)), dim3(64), 0, (const float*)ops, n, chunks, st->heads, st->dim, state, o,
+    skn_launch(ctx, delta_scan_kernel<DP>, dim3((unsigned)((st->heads + 7) / 8 * 8 * tiles)), dim3(64 * ScanSplit<DP>::kWaves), 0, (const float*)ops, n, chunks, st->heads, st->dim, state, o,
                trash);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;

@@ -284,90 +284,109 @@ __global__ __launch_bounds__(64) void gated_chunk_kernel(const ChunkArgs p) {
 
 template <int DP>
 struct GatedOps {
-    static constexpr int kTiles = DP / 16;
-    f32x4 k1[kTiles], r0[kTiles], kt[kTiles], w[kTiles], v, g;
-    __device__ __forceinline__ void load(const float* p, int lane, int tile) {
-        v = load4(p + off_v(DP) + (tile * 64 + lane) * 4);
+    using Split = ScanSplit<DP>;
+    static constexpr int kOwn = Split::kOwn, kRows = Split::kRows;
+    f32x4 k1[kOwn], r0[kOwn], kt[kOwn], w[kOwn], v;
+    float g[kRows];
+    __device__ __forceinline__ void load(const float* p, uint32_t lane, uint32_t wave, uint32_t tile) {
+        const uint32_t own = (wave * kOwn * 64 + lane) * 16, row = (16 * wave * kOwn + 4 * (lane >> 4)) * 4, some = lane * 16 + wave * kRows * 4;
 #pragma unroll
-        for (int j = 0; j < kTiles; j++) {
-            k1[j] = load4(p + off_k1(DP) + (j * 64 + lane) * 4);
-            r0[j] = load4(p + off_r0(DP) + (j * 64 + lane) * 4);
+        for (int i = 0; i < kOwn; i++) {
+            k1[i] = load4(p + off_k1(DP) + 256 * i, own);
+            r0[i] = load4(p + off_r0(DP) + 256 * i, own);
         }
-        g = load4(p + off_g(DP) + lane * 4);
+        v = load4(p + off_v(DP), (tile * 64 + lane) * 16);
 #pragma unroll
-        for (int j = 0; j < kTiles; j++) {
-            kt[j] = load4(p + off_kt(DP) + (j * 64 + lane) * 4);
-            w[j] = load4(p + off_w(DP) + 16 * j + 4 * (lane >> 4));
+        for (int i = 0; i < kRows; i++) {
+            g[i] = load1(p + off_g(DP) + i, some);
+        }
+#pragma unroll
+        for (int i = 0; i < kOwn; i++) {
+            w[i] = load4(p + off_w(DP) + 16 * i, row);
+            kt[i] = load4(p + off_kt(DP) + 256 * i, own);
         }
     }
 };
 
-// One wavefront per head and tile of sixteen value columns, its part of S in accumulator layout (also the layout of a column operand);
-// the wavefronts of a head are on one XCD (blockIdx % 8), as in delta_scan_kernel.
+// One workgroup per head and tile of sixteen value columns, its parts of S in accumulator layout (also the layout of a column
+// operand); the workgroups of a head are on one XCD (blockIdx % 8), as in delta_scan_kernel.  A chunk's matrix instructions are a
+// chain on one SIMD otherwise (100 of 32 clocks at 128 channels): 2048 tokens of 16 heads of 128, one wavefront 261 us, four 121.
 template <int DP>
-__global__ __launch_bounds__(64) void gated_scan_kernel(const float* __restrict__ ops, int n, int chunks, int heads, int vdim, float* __restrict__ state,
+__global__ __launch_bounds__(64 * ScanSplit<DP>::kWaves) __attribute__((amdgpu_waves_per_eu(DP <= 128 ? 2 : 1, 2))) void gated_scan_kernel(const float* __restrict__ ops, int n, int chunks, int heads, int vdim, float* __restrict__ state,
                                                         float* __restrict__ o, float* __restrict__ trash) {
-    constexpr int kTiles = DP / 16;
-    const int lane = threadIdx.x, tiles = (vdim + 15) / 16, turn = (int)(blockIdx.x >> 3), h = (int)(blockIdx.x & 7) + 8 * (turn / tiles), tile = turn % tiles;
+    using Split = ScanSplit<DP>;
+    constexpr int NW = Split::kWaves, kOwn = Split::kOwn, kRows = Split::kRows, R = DP <= 64 ? 4 : DP <= 128 ? 3 : 2;  // chunks in registers (what they hold without spilling)
+    __shared__ f32x4 part_u[2][NW][64], part_z[2][NW][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int tiles = (vdim + 15) / 16, turn = (int)(blockIdx.x >> 3), h = (int)(blockIdx.x & 7) + 8 * (turn / tiles), tile = turn % tiles;
     if (h >= heads) return;
     const int col = 16 * tile + (lane & 15), size = chunk_floats(DP, vdim);
     const bool live = col < vdim;  // (lanes beyond the last column compute along and store nothing)
-    float* sp = state + ((int64_t)h * vdim + min(col, vdim - 1)) * DP + 4 * (lane >> 4);
-    f32x4 s[kTiles];
+    float* sp = state + ((int64_t)h * vdim + min(col, vdim - 1)) * DP + 16 * wave * kOwn + 4 * (lane >> 4);
+    f32x4 s[kOwn];
 #pragma unroll
-    for (int j = 0; j < kTiles; j++) s[j] = load4(sp + 16 * j);
+    for (int j = 0; j < kOwn; j++) s[j] = load4(sp + 16 * j);
     const float* src = ops + (int64_t)h * chunks * size;
 
-    auto step = [&](const GatedOps<DP>& x, int chunk) __attribute__((always_inline)) {
-        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-        f32x4 u[2] = {x.v, zero}, z[2] = {zero, zero};
+    const int t_own = 4 * (lane >> 4) + wave * kRows;
+    float* o_own = o + ((int64_t)t_own * heads + h) * vdim + col;
+    // this wavefront's rows of the outputs of a chunk
+    auto store = [&](int chunk) __attribute__((always_inline)) {
+        const f32x4 z = sum_parts<NW>(part_z[chunk & 1], lane);
+        // (one store per row whatever the lane, so that the number of requests outstanding is known)
 #pragma unroll
-        for (int j = 0; j < kTiles; j++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                u[e & 1] = mma(x.k1[j][e], s[j][e], u[e & 1]);
-                z[e & 1] = mma(x.r0[j][e], s[j][e], z[e & 1]);
-            }
-        u[0] += u[1];
-#pragma unroll
-        for (int j = 0; j < kTiles; j++) s[j] *= x.w[j];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-#pragma unroll
-            for (int j = 0; j < kTiles; j++) s[j] = mma(x.kt[j][e], u[0][e], s[j]);
-            z[e & 1] = mma(x.g[e], u[0][e], z[e & 1]);
-        }
-        z[0] += z[1];
-        // (one store per token whatever the lane, so that the number of requests outstanding is known)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int t = chunk * kChunk + 4 * (lane >> 4) + e;
-            float* dst = live && t < n ? o + ((int64_t)t * heads + h) * vdim + col : trash + lane;
-            *dst = z[0][e];
+        for (int i = 0; i < kRows; i++) {
+            const int t = chunk * kChunk + t_own + i;
+            float* dst = live && t >= 0 && t < n ? o_own + (int64_t)(chunk * kChunk + i) * heads * vdim : trash + lane;
+            *dst = element(z, wave * kRows + i);
         }
     };
-    GatedOps<DP> even;
-    if constexpr (DP <= 128) {
-        GatedOps<DP> odd;
-        even.load(src, lane, tile);
-        for (int c = 0; c < chunks; c += 2) {
-            odd.load(src + (int64_t)min(c + 1, chunks - 1) * size, lane, tile);
+    auto step = [&](const GatedOps<DP>& x, int chunk) __attribute__((always_inline)) {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        f32x4 u[2] = {zero, zero}, z[2] = {zero, zero};
+#pragma unroll
+        for (int j = 0; j < kOwn; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) u[e & 1] = mma(x.k1[j][e], s[j][e], u[e & 1]);
+        part_u[chunk & 1][wave][lane] = u[0] + u[1];
+#pragma unroll
+        for (int j = 0; j < kOwn; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) z[e & 1] = mma(x.r0[j][e], s[j][e], z[e & 1]);
+#pragma unroll
+        for (int j = 0; j < kOwn; j++) s[j] *= x.w[j];
+        lds_barrier();  // (a buffer is written again two barriers after the reads of the chunk that had it)
+        const f32x4 all = x.v + sum_parts<NW>(part_u[chunk & 1], lane);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int j = 0; j < kOwn; j++) s[j] = mma(x.kt[j][e], all[e], s[j]);
+#pragma unroll
+        for (int i = 0; i < kRows; i++) z[i & 1] = mma(x.g[i], element(all, wave * kRows + i), z[i & 1]);
+        store(chunk - 1);
+        part_z[chunk & 1][wave][lane] = z[0] + z[1];
+    };
+    GatedOps<DP> x[R];
+#pragma unroll
+    for (int r = 0; r < R - 1; r++) x[r].load(src + (int64_t)min(r, chunks - 1) * size, lane, wave, tile);
+    int c = 0;
+    for (; c + R <= chunks; c += R) {  // (no condition inside: the number of requests outstanding is known)
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            x[(r + R - 1) % R].load(src + (int64_t)min(c + r + R - 1, chunks - 1) * size, lane, wave, tile);
             __builtin_amdgcn_sched_barrier(0);
-            step(even, c);
-            if (c + 1 == chunks) break;
-            even.load(src + (int64_t)min(c + 2, chunks - 1) * size, lane, tile);
+            step(x[r], c + r);
             __builtin_amdgcn_sched_barrier(0);
-            step(odd, c + 1);
-        }
-    } else {
-        for (int c = 0; c < chunks; c++) {
-            even.load(src + (int64_t)c * size, lane, tile);
-            step(even, c);
         }
     }
+#pragma unroll
+    for (int r = 0; r < R - 1; r++)
+        if (c + r < chunks) step(x[r], c + r);
+    lds_barrier();
+    store(chunks - 1);
     if (live) {
 #pragma unroll
-        for (int j = 0; j < kTiles; j++) *reinterpret_cast<f32x4*>(sp + 16 * j) = s[j];
+        for (int j = 0; j < kOwn; j++) *reinterpret_cast<f32x4*>(sp + 16 * j) = s[j];
     }
 }
 
@@ -496,7 +515,7 @@ int launch_rows(skn_ctx* ctx, const skn_rstate* st, const ChunkArgs& a, float* s
     skn_launch(ctx, gated_chunk_kernel<DP>, dim3(chunks, a.heads), dim3(64), 0, a);
     SKN_LAUNCH_CHECK(ctx);
     float* trash = a.ops + (size_t)chunks * a.heads * chunk_floats(DP, a.vdim);
-    skn_launch(ctx, gated_scan_kernel<DP>, dim3((unsigned)((a.heads + 7) / 8 * 8 * tiles)), dim3(64), 0, (const float*)a.ops, a.n, chunks, a.heads, a.vdim, state, o,
+    skn_launch(ctx, gated_scan_kernel<DP>, dim3((unsigned)((a.heads + 7) / 8 * 8 * tiles)), dim3(64 * ScanSplit<DP>::kWaves), 0, (const float*)a.ops, a.n, chunks, a.heads, a.vdim, state, o,
                trash);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;

@@ -293,6 +293,20 @@ def test_gated_delta_in_one_go_in_portions_and_token_by_token(hip, heads, kv_hea
     st.free()
 
 
+@pytest.mark.parametrize("dim,vdim", [(32, 48), (64, 20), (128, 128), (256, 16)])
+def test_gated_delta_over_every_number_of_chunks(hip, dim, vdim):
+    """Prompts of one to nine chunks of sixteen tokens (two to four are in registers at once) and of a ragged end, for every split of
+    a chunk over wavefronts; the state after them is read by one more token."""
+    heads, kv_heads, taps = 2, 1, 4
+    c = delta_case(heads, kv_heads, dim, vdim, taps, 9 * 16 + 1, seed=dim + 1)
+    want = delta_oracle(c, heads, kv_heads, dim, vdim)
+    st = runtime.ConvRecurrentState(hip, 1, heads, kv_heads, dim, vdim, taps)
+    for n in [16 * k for k in range(1, 10)] + [47, 65, 130]:
+        st.reset()
+        assert rel(in_portions(n + 1, [n, 1], lambda a, b: advance(st, c, a, b)), want[:n + 1]) < 1e-5, n
+    st.free()
+
+
 def test_decays_from_nothing_to_everything(hip):
     """Some channels forget everything in one token, others nothing over hundreds; both change from token to token."""
     heads, kv_heads, dim, vdim, taps, n = 2, 1, 48, 32, 4, 400

@@ -185,6 +185,22 @@ def test_delta_rule_in_one_go_in_portions_and_token_by_token(hip, heads, dim):
     st.free()
 
 
+@pytest.mark.parametrize("dim", [32, 64, 128, 256])
+def test_delta_rule_over_every_number_of_chunks(hip, dim):
+    """Prompts of one to nine chunks of sixteen tokens: the operands of two to four chunks are in registers at once, the rest of a
+    round is walked by itself, and each size of a head has its own split of a chunk over wavefronts.  The state after them is read
+    by one more token.  (Bound as above: fp32 products and sums in another order.)"""
+    heads = 3
+    c = delta_case(heads, dim, 9 * 16 + 1, seed=dim + 1)
+    st = runtime.RecurrentState(hip, 1, heads, dim)
+    for n in [16 * k for k in range(1, 10)] + [47, 65, 130]:
+        part = tuple(a[:n + 1] for a in c)
+        st.reset()
+        out = [st.advance(0, *(a[:n] for a in part)), st.advance(0, *(a[n:] for a in part))]
+        assert rel(np.concatenate(out), delta_oracle(part, heads, dim)) < 1e-5, n
+    st.free()
+
+
 def test_delta_rule_remembers_over_a_long_sequence(hip):
     """Decays near one: the first token's value is still in the state a thousand tokens later."""
     heads, dim, n = 2, 24, 1000
