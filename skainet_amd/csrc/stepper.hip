@@ -18,6 +18,9 @@ __global__ __launch_bounds__(1024) void finish_step_kernel(const float* __restri
                                                            int32_t* __restrict__ tokens_out, int advance) {
     __shared__ float bv[16];
     __shared__ int bi[16];
+    // (asked for with the logits: behind the choice they were one more trip to memory)
+    int32_t position = 0, context = 0, index = 0;
+    if (threadIdx.x == 0 && advance) position = state[1], context = state[2], index = state[3];
     float best = -INFINITY;
     int besti = 0x7FFFFFFF;
     auto take = [&](float v, int i) {
@@ -44,32 +47,24 @@ __global__ __launch_bounds__(1024) void finish_step_kernel(const float* __restri
         }
     }
     for (int i = 4 * n4 + threadIdx.x; i < n; i += 1024) take(x[i], i);
-    for (int off = 32; off >= 1; off >>= 1) {
-        const float ov = __shfl_xor(best, off, 64);
-        const int oi = __shfl_xor(besti, off, 64);
-        if (ov > best || (ov == best && oi < besti)) {
-            best = ov;
-            besti = oi;
-        }
-    }
+    for (int off = 32; off >= 1; off >>= 1) take(__shfl_xor(best, off, 64), __shfl_xor(besti, off, 64));
     if ((threadIdx.x & 63) == 0) {
         bv[threadIdx.x >> 6] = best;
         bi[threadIdx.x >> 6] = besti;
     }
     __syncthreads();
+    if (threadIdx.x >= 64) return;
+    best = bv[threadIdx.x & 15];
+    besti = bi[threadIdx.x & 15];
+    for (int off = 8; off >= 1; off >>= 1) take(__shfl_xor(best, off, 64), __shfl_xor(besti, off, 64));
     if (threadIdx.x == 0) {
-        for (int w = 1; w < 16; w++)
-            if (bv[w] > best || (bv[w] == best && bi[w] < besti)) {
-                best = bv[w];
-                besti = bi[w];
-            }
         const int tok = besti == 0x7FFFFFFF ? 0 : besti;
         if (advance) {
-            tokens_out[state[3]] = tok;
+            tokens_out[index] = tok;
             state[0] = tok;
-            state[1] += 1;
-            state[2] += 1;
-            state[3] += 1;
+            state[1] = position + 1;
+            state[2] = context + 1;
+            state[3] = index + 1;
         } else {
             tokens_out[0] = tok;
         }
