@@ -1471,10 +1471,12 @@ __device__ __forceinline__ float4 q4k_merge_splits(const float4* __restrict__ pa
 // residual stream, or applies SwiGLU to a (gate, up) row pair.  Two rows per wavefront, or one where rows are added into few
 // outputs (see dispatch_q4k_fused).  F: the format of all the matrices, as in matvec_q4k_kernel; block: the workgroup's place
 // among those that share the matrices.
-template <int STEPS, int EPI, bool NORM, int F, int R>
+template <int STEPS, int EPI, bool NORM, int F, int R, bool HALF = false>
 __device__ __forceinline__ void q4k_fused_block(const skn_q4k_segments& seg, const float* __restrict__ x, const float* __restrict__ norm_w, float eps,
                                                 float* __restrict__ y, int n_out, int nb, const skn_rope_epilogue& rope, int block) {
     static_assert(R == 2 || EPI == SKN_EPI_ADD, "row pairs");
+    static_assert(!HALF || (STEPS == 1 && R == 2), "rows of half a step");
+    constexpr int RL = HALF ? 1 : R;  // rows of a lane
     constexpr bool Q5 = F == kFmtQ5K, Q6 = F == kFmtQ6K, Q8 = F == kFmtQ80, Q2 = F == kFmtQ2K, Q3 = F == kFmtQ3K, Q8K = F == kFmtQ8K;
     constexpr bool T2 = F == kFmtTQ2, T1 = F == kFmtTQ1;
     constexpr bool kRuns = Q6 || Q2 || Q3 || T2;  // the Q6_K lane map: four runs of sixteen per lane, a float4 of run sums
@@ -1491,7 +1493,7 @@ __device__ __forceinline__ void q4k_fused_block(const skn_q4k_segments& seg, con
     float* ss = reinterpret_cast<float*>(lds4 + STEPS * 16 * kXPitch);
     float* red = ss + STEPS * (kRuns ? 256 : 128);  // eight partial sums of x^2 (all LDS here is dynamic)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int sub = lane >> 2, p = lane & 3;
+    const int lx = HALF ? lane & 31 : lane, sub = lx >> 2, p = lane & 3;
     const int n4 = nb * 64;
     constexpr int J = 2 * STEPS;  // 512 threads x J float4 cover k <= STEPS * 4096
 
@@ -1557,13 +1559,17 @@ __device__ __forceinline__ void q4k_fused_block(const skn_q4k_segments& seg, con
             rowp[r] = base + (size_t)row * row_bytes;
         }
     }
-    Loads L[STEPS][R];
+    if constexpr (HALF) {
+        rowp[0] = lane < 32 ? rowp[0] : rowp[1];
+        row_ok[0] = lane < 32 ? row_ok[0] : row_ok[1];
+    }
+    Loads L[STEPS][RL];
     auto issue = [&](int s, int tie) __attribute__((always_inline)) {
         const int blk = s * 16 + sub;
 #pragma unroll
-        for (int r = 0; r < R; r++) {
+        for (int r = 0; r < RL; r++) {
             if constexpr (Q8) {  // lane = pair of blocks, 64 pairs per step
-                const int pr = s * 64 + lane, npairs = 4 * nb;
+                const int pr = s * 64 + lx, npairs = 4 * nb;
                 const uint8_t* bp = rowp[r] + (size_t)(min(pr, npairs - 1) + tie) * 68;
 #pragma unroll
                 for (int i = 0; i < 4; i++) L[s][r].w[i] = reinterpret_cast<const u32x4_a4*>(bp)[i];
@@ -1667,49 +1673,49 @@ __device__ __forceinline__ void q4k_fused_block(const skn_q4k_segments& seg, con
         rinv = 1.0f / sqrtf(total / (float)(nb * 256) + eps);
     }
 
-    float acc[R] = {};
+    float acc[RL] = {};
     int tie = 0;
     asm volatile("" : "+v"(tie));
 #pragma unroll
     for (int s = 0; s < STEPS; s++) {
         if (s + 1 < STEPS) issue(s + 1, tie);
         asm volatile("" ::: "memory");
-        if constexpr (Q8) q80_step<R>(L[s], xs, ss, s, lane + tie, acc);
-        else if constexpr (Q8K) q8k_step<R>(L[s], xs, ss, s, lane + tie, acc);
-        else if constexpr (Q6) q6k_step<R>(L[s], xs, ss, s, lane + tie, p & 1, acc);
-        else if constexpr (Q2) q2k_step<R>(L[s], xs, ss, s, lane + tie, p & 1, acc);
-        else if constexpr (Q3) q3k_step<R>(L[s], xs, ss, s, lane + tie, p >> 1, p & 1, acc);
-        else if constexpr (T2) tq2_step<R>(L[s], xs, ss, s, lane + tie, acc);
-        else if constexpr (T1) tq1_step<R>(L[s], xs, s, lane + tie, acc);
-        else if constexpr (kSmall) q4x_step<R, F>(L[s], xs, ss, s, lane + tie, acc);
-        else q4k_step<R>(L[s], xs, ss, s, lane + tie, p, acc);
-        asm volatile("" : "+v"(tie), "+v"(acc[R - 1]));
+        if constexpr (Q8) q80_step<RL>(L[s], xs, ss, s, lx + tie, acc);
+        else if constexpr (Q8K) q8k_step<RL>(L[s], xs, ss, s, lx + tie, acc);
+        else if constexpr (Q6) q6k_step<RL>(L[s], xs, ss, s, lx + tie, p & 1, acc);
+        else if constexpr (Q2) q2k_step<RL>(L[s], xs, ss, s, lx + tie, p & 1, acc);
+        else if constexpr (Q3) q3k_step<RL>(L[s], xs, ss, s, lx + tie, p >> 1, p & 1, acc);
+        else if constexpr (T2) tq2_step<RL>(L[s], xs, ss, s, lx + tie, acc);
+        else if constexpr (T1) tq1_step<RL>(L[s], xs, s, lx + tie, acc);
+        else if constexpr (kSmall) q4x_step<RL, F>(L[s], xs, ss, s, lx + tie, acc);
+        else q4k_step<RL>(L[s], xs, ss, s, lx + tie, p, acc);
+        asm volatile("" : "+v"(tie), "+v"(acc[RL - 1]));
     }
     const float back = (Q8 || Q8K || T1 || kPlainX) ? rinv : 16777216.0f * rinv;  // (the nibble formats work in units of 2^-24)
-    const float t0 = wave_sum(acc[0]) * back;
+    const float t0 = wave_sum(HALF && lane >= 32 ? 0.f : acc[0]) * back;
     if constexpr (R == 1) {
         if (lane == 0 && unit < n_out) y[unit] += t0;
     } else {
-        const float t1 = wave_sum(acc[1]) * back;
+        const float t1 = wave_sum(!HALF ? acc[RL - 1] : lane >= 32 ? acc[0] : 0.f) * back;
         if (lane == 0) q4k_epilogue<EPI>(rope, rc, y, n_out, unit, t0, t1);
     }
 }
 
-template <int STEPS, int EPI, bool NORM, int F = kFmtQ4K, int R = 2>
+template <int STEPS, int EPI, bool NORM, int F = kFmtQ4K, int R = 2, bool HALF = false>
 __global__ __launch_bounds__(512) void matvec_q4k_fused_kernel(skn_q4k_segments seg, const float* __restrict__ x,
                                                                const float* __restrict__ norm_w, float eps,
                                                                float* __restrict__ y, int n_out, int nb,
                                                                skn_rope_epilogue rope) {
-    q4k_fused_block<STEPS, EPI, NORM, F, R>(seg, x, norm_w, eps, y, n_out, nb, rope, (int)blockIdx.x);
+    q4k_fused_block<STEPS, EPI, NORM, F, R, HALF>(seg, x, norm_w, eps, y, n_out, nb, rope, (int)blockIdx.x);
 }
 
 // q, k and v in two formats (mixed files give the values more bits): the workgroups of both in one launch, the larger blocks first.
-template <int STEPS, int FA, int FB>
+template <int STEPS, int FA, int FB, bool HALF = false>
 __global__ __launch_bounds__(512) void matvec_fused_two_formats_kernel(skn_q4k_segments sa, skn_q4k_segments sb, const float* __restrict__ x,
                                                                       const float* __restrict__ norm_w, float eps, float* __restrict__ y,
                                                                       int n_a, int n_b, int blocks_a, int nb, skn_rope_epilogue rope) {
-    if ((int)blockIdx.x < blocks_a) q4k_fused_block<STEPS, SKN_EPI_ROPE, true, FA, 2>(sa, x, norm_w, eps, y, n_a, nb, rope, (int)blockIdx.x);
-    else q4k_fused_block<STEPS, SKN_EPI_ROPE, true, FB, 2>(sb, x, norm_w, eps, y, n_b, nb, rope, (int)blockIdx.x - blocks_a);
+    if ((int)blockIdx.x < blocks_a) q4k_fused_block<STEPS, SKN_EPI_ROPE, true, FA, 2, HALF>(sa, x, norm_w, eps, y, n_a, nb, rope, (int)blockIdx.x);
+    else q4k_fused_block<STEPS, SKN_EPI_ROPE, true, FB, 2, HALF>(sb, x, norm_w, eps, y, n_b, nb, rope, (int)blockIdx.x - blocks_a);
 }
 
 template <int F>
@@ -1717,12 +1723,20 @@ constexpr size_t fused_lds_bytes(int steps) {
     return (size_t)steps * (16 * kXPitch * sizeof(float4) + 64 * ((F == kFmtQ6K || F == kFmtQ2K || F == kFmtQ3K || F == kFmtTQ2) ? sizeof(float4) : sizeof(float2))) + 8 * sizeof(float);
 }
 
+// Rows of up to half a step (2048 columns): the two rows of a wavefront side by side in its lanes instead of one after the other
+// with half of the lanes idle.  Gate and up of 8192 rows of 2048 in Q4_K: 10.6 -> 8.4 us, q, k, v of 3072
+// rows 5.5 -> 5.1; a decode step of eight layers of width 2048 at 2000 tokens 284 -> 268.
+constexpr int kHalfStep = 8;
+
 template <int STEPS, int F>
 int launch_fused_beside_q6k(skn_ctx* ctx, const skn_q4k_segments& q6, int n_q6, const skn_q4k_segments& other, int n_other, int nb, const float* x,
                             const float* norm_w, float eps, float* y, const skn_rope_epilogue& rope) {
     const int blocks_q6 = (n_q6 + 15) / 16, blocks = blocks_q6 + (n_other + 15) / 16;
-    skn_launch(ctx, matvec_fused_two_formats_kernel<STEPS, kFmtQ6K, F>, dim3((unsigned)blocks), dim3(512), fused_lds_bytes<kFmtQ6K>(STEPS), q6, other, x, norm_w,
-               eps, y, n_q6, n_other, blocks_q6, nb, rope);
+    auto kernel = matvec_fused_two_formats_kernel<STEPS, kFmtQ6K, F>;
+    if constexpr (STEPS == 1)
+        if (nb <= kHalfStep) kernel = matvec_fused_two_formats_kernel<1, kFmtQ6K, F, true>;
+    skn_launch(ctx, kernel, dim3((unsigned)blocks), dim3(512), fused_lds_bytes<kFmtQ6K>(STEPS), q6, other, x, norm_w, eps, y, n_q6, n_other, blocks_q6, nb,
+               rope);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
@@ -1733,7 +1747,10 @@ int launch_q4k_fused(skn_ctx* ctx, const skn_q4k_segments& seg, int n_out, int n
     const size_t lds = fused_lds_bytes<F>(STEPS);
     const int units = EPI == SKN_EPI_SWIGLU ? n_out : (n_out + R - 1) / R;
     dim3 grid((unsigned)((units + 7) / 8)), block(512);
-    skn_launch(ctx, matvec_q4k_fused_kernel<STEPS, EPI, NORM, F, R>, grid, block, lds, seg, x, norm_w, eps, y, n_out, nb, rope);
+    auto kernel = matvec_q4k_fused_kernel<STEPS, EPI, NORM, F, R>;
+    if constexpr (STEPS == 1 && R == 2 && NORM && (EPI == SKN_EPI_ROPE || EPI == SKN_EPI_SWIGLU))
+        if (nb <= kHalfStep) kernel = matvec_q4k_fused_kernel<1, EPI, true, F, 2, true>;
+    skn_launch(ctx, kernel, grid, block, lds, seg, x, norm_w, eps, y, n_out, nb, rope);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }

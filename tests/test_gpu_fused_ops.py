@@ -64,6 +64,22 @@ def test_norm_gate_up_swiglu(hip, qtype):
 
 
 @pytest.mark.parametrize("qtype", FUSED_TYPES)
+@pytest.mark.parametrize("k", [256, 1792, 2048, 2304, 4096])
+def test_rows_of_up_to_half_a_step_and_beyond(hip, qtype, k):
+    """Up to 2048 columns a wavefront has its two rows side by side in its lanes, from 2304 on one after the other; outputs that do
+    not fill a workgroup, the last rows of both forms."""
+    f = 61
+    wg, wu = synth.weight(qtype, f, k, seed=64), synth.weight(qtype, f, k, seed=65)
+    x = synth.activation_f32(k, seed=66)
+    g = (1.0 + 0.1 * np.random.default_rng(67).standard_normal(k)).astype(np.float32)
+    y = hip.alloc(4 * f)
+    hip.test_fused_matvec(qtype, SWIGLU, [(hip.to_device(wg), f), (hip.to_device(wu), f)], k, hip.to_device(x), hip.to_device(g), 1e-5, y)
+    xn = _norm(x, g, 1e-5)
+    want = oracle_c.swiglu(oracle_c.matvec_q(qtype, wg, f, k, xn), oracle_c.matvec_q(qtype, wu, f, k, xn))
+    assert oracle_np.rel_err(y.download(np.float32, f), want) <= TOL
+
+
+@pytest.mark.parametrize("qtype", FUSED_TYPES)
 def test_residual_add_and_plain_store(hip, qtype):
     n, k = 256, 2048
     w = synth.weight(qtype, n, k, seed=70)
