@@ -738,6 +738,9 @@ constexpr int kTlLds = 3 * kTlStage + 2 * kTlAux + 128 * 4 + 256 * 4;
 // One to three matrices per launch as in gemm_q4k_frag_kernel (tile0 counts 128-column tiles here); pair: a tile holds
 // the same 64 columns of the gate and the up matrix -- producers 0 and 1 unpack the gate's, 2 and 3 the up's, so a
 // consumer's column blocks 0, 1 and 2, 3 meet lane by lane in the store -- and stores silu(gate) * up into c[0].
+// TAIL: the last tiles are shared by tail.splits workgroups each, neighbours in the grid, with a part of k each (a template
+// parameter: grids without such tiles were 0.5 us slower at 512 x 14336 x 4096 for the division).
+template <bool TAIL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restrict__ sfrag, const Q4kFragSegs segs,
                           const float* __restrict__ inv_scale, int m, int k, int m_tiles, uint32_t a_bytes, const TallTail tail) {
@@ -748,9 +751,8 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
     const bool producer = wave >= 4;
     const int h = lane >> 5, r = lane & 31;
     const int nb = k >> 8, nch = k >> 6;
-    // the last tiles are shared by tail.splits workgroups each, neighbours in the grid, with a part of k each
     int tile = (int)blockIdx.x, z = 0, parts = 1, sb0 = 0, sb1 = nb;
-    if (tile >= tail.tile0) {
+    if (TAIL && tile >= tail.tile0) {
         const int over = tile - tail.tile0;
         parts = tail.splits, z = over % parts, tile = tail.tile0 + over / parts;
         sb0 = nb * z / parts, sb1 = nb * (z + 1) / parts;
@@ -1028,7 +1030,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
             phase(sb, C3{});
         }
         barrier();
-        if (parts > 1) {  // (unscaled, every element of the tile, in the order of the matrix core's registers: see gemm_add_tall_kernel)
+        if (TAIL && parts > 1) {  // (unscaled, every element of the tile, in the order of the matrix core's registers: see gemm_add_tall_kernel)
             float* dst = tail.part + ((size_t)(z * tail.tiles + tile - tail.tile0) * 4 + me) * (MT * 4 * 1024) + lane * 4;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -2099,7 +2101,8 @@ static int skn_gemm_init(skn_ctx* ctx) {
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 2, true>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 2>() + 32 * 2 * 2 * 4));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 1, false>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 1>() + 32 * 2 * 1 * 4));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 1, true>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 1>() + 32 * 2 * 1 * 4));
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_tall_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kTlLds));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_tall_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, kTlLds));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_tall_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, kTlLds));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_hilo_frag_kernel<1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 1 * 3 * 4096));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_hilo_frag_kernel<2, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 2 * 3 * 4096));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_hilo_frag_kernel<4, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 4 * 3 * 4096));
@@ -2208,7 +2211,7 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
         for (int i = 0; i < 3; i++) fs.tile0[i] = tall_tile0[i];
         fs.n_tiles = tall_cols;
         tail.part = (float*)(ws + af_bytes + sf_bytes + is_bytes);
-        skn_launch(ctx, gemm_q4k_tall_kernel, dim3(tail.tile0 + tail.tiles * tail.splits), dim3(512), kTlLds, (const u32x4*)afrag, (const u32x4*)sfrag, fs,
+        skn_launch(ctx, tail.tiles ? gemm_q4k_tall_kernel<true> : gemm_q4k_tall_kernel<false>, dim3(tail.tile0 + tail.tiles * tail.splits), dim3(512), kTlLds, (const u32x4*)afrag, (const u32x4*)sfrag, fs,
                    (const float*)isc, m, k, m_tiles, (uint32_t)((size_t)m_pad * k * 2), tail);
         SKN_LAUNCH_CHECK(ctx);
         if (tail.tiles) {
