@@ -2064,10 +2064,10 @@ int skn_gemm_add_parts(skn_ctx* ctx, const float* part, int splits, int cols, co
     return SKN_OK;
 }
 
-// How many workgroups share a tile's k: as many as there are compute units for, at least one superblock for each of a
-// workgroup's four k-parts.  us per call, unsplit -> chosen: Q6_K 41 x 4096 x 11008 (64 tiles) 81 -> 34.5, 120 x 4096 x 11008
-// 106 -> 45, 200 x 4096 x 11008 (128 tiles) 108 -> 71; Q4_K 41 x 4096 x 11008 35.7 -> 24.6, 41 x 4096 x 4096 17.8 -> 15.1,
-// 200 x 4096 x 4096 25.9 -> 24.8.  Filling every compute unit twice is no gain (Q4_K 41 x 4096 x 11008 27.2, 120 x 4096 x 4096
+// How many workgroups share a tile's k: as many as there are compute units for, up to sixteen, at least one superblock for each
+// of a workgroup's four k-parts.  us per call, unsplit -> chosen: Q6_K 41 x 4096 x 11008 (64 tiles) 81 -> 34.5, 120 x 4096 x 11008
+// 106 -> 45, 200 x 4096 x 11008 (128 tiles) 108 -> 71; Q4_K 41 x 4096 x 11008 35.7 -> 24.6, 41 x 4096 x 4096 17.8 -> 15.1.
+// Filling every compute unit twice is no gain (Q4_K 41 x 4096 x 11008 27.2, 120 x 4096 x 4096
 // 21.5 against 18.7), nor is a second part for tiles that fill two thirds of the device (Q4_K 41 x 11008 x 4096 22.2 against
 // 19.6, Q6_K 333 x 4096 x 4096 59 against 54): the addition costs 3 us and the parts their way through memory.
 int skn_gemm_k_splits(const skn_ctx* ctx, int m, int tiles, int nb) {
@@ -2120,13 +2120,26 @@ static int skn_gemm_init(skn_ctx* ctx) {
 static skn_family register_family(skn_gemm_init);
 
 // The tiles past the last whole round of compute units: shared where at least two workgroups each find room in that round.
-static TallTail tall_tail(const skn_ctx* ctx, int tiles, int m_tiles, int nb) {
+static TallTail tall_tail(const skn_ctx* ctx, int tiles, int nb) {
     const int cus = ctx->compute_units, rest = tiles % cus;
     TallTail t = {tiles, 0, 1, nullptr};
     int splits = rest ? std::min(cus / rest, nb / 4) : 1;
     if (ctx->opt_gemm_split > 0) splits = std::min(ctx->opt_gemm_split, nb);
     if (rest == 0 || splits < 2) return t;
     return TallTail{tiles - rest, rest, splits, nullptr};
+}
+
+// The same for the Q4_K kernel of 64- and 128-row tiles, whose step along k is short: only where the steps saved (a group of
+// four superblocks each: 1.9 us on 64 rows, 3 us on 128) pay for the second launch and for the parts' way through memory (0.6 us
+// per MB; `cols` of all the launch's matrices).  Fitted to 290 shapes of 33 to 1024 rows, 256 to 11008 columns and k from 1536 to
+// 11008.  us per call, unsplit | split: 200 x 4096 x 2048 17.3 | 20.1, 512 x 2048 x 2048 19.0 | 24.4, 64 x 8192 x 2048 13.3 | 15.4, all
+// three unsplit now; 512 x 512 x 4096 27.0 | 20.4, 200 x 4096 x 6144 35.6 | 31.5, both split.
+static int q4k_splits(const skn_ctx* ctx, int m, int tile_rows, int tiles, int nb, int cols) {
+    const int splits = skn_gemm_k_splits(ctx, m, tiles, nb);
+    if (splits < 2 || ctx->opt_gemm_split > 0) return splits;
+    const int each = (nb + splits - 1) / splits, saved = (nb + 3) / 4 - (each + 3) / 4;
+    const double gain_us = tile_rows == 64 ? 1.9 * (saved - 1) : 3.0 * saved - 1.2;
+    return gain_us > 0.6e-6 * 4.0 * splits * m * cols ? splits : 1;
 }
 
 int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, const skn_gemm_src& src, int m,
@@ -2173,7 +2186,7 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     const bool tall = tall_fits && (ctx->opt_gemm_tile == 3 ||
                                     (ctx->opt_gemm_tile == 0 && m > 128 && 3 * tall_tiles >= 2 * tall_rounds * ctx->compute_units));
     TallTail tail = {tall_tiles, 0, 1, nullptr};
-    if (tall) tail = tall_tail(ctx, tall_tiles, (m + 255) / 256, k / 256);
+    if (tall) tail = tall_tail(ctx, tall_tiles, k / 256);
     const bool small_tiles = !tall && (ctx->opt_gemm_tile == 1 ||
                              (ctx->opt_gemm_tile == 0 && (m <= 128 || ((m + 127) / 128) * n_tiles_all > ctx->compute_units)));
     const int mt_rows = tall ? 256 : small_tiles ? 64 : 128;
@@ -2182,7 +2195,6 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     SKN_REQUIRE(ctx, af_bytes < ((size_t)1 << 31), SKN_ERR_SHAPE,
                 "Q4_K GEMM: %d rows of %d activations exceed the 2^30 elements one call takes", m, k);
     const size_t is_bytes = skn_align_up((size_t)m_pad * 4);
-    const int splits = tall ? 1 : skn_gemm_k_splits(ctx, m, m_tiles * fs.n_tiles, k / 256);
     skn_gemm_parts ps = {};
     ps.count = nseg, ps.pair = fs.pair;
     for (int i = 0; i < nseg; i++) {
@@ -2191,6 +2203,7 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
         fs.part_cols += segs[i].n;
     }
     for (int i = 0; i < 3; i++) fs.part_col0[i] = ps.col0[i];
+    const int splits = tall ? 1 : q4k_splits(ctx, m, mt_rows, m_tiles * fs.n_tiles, k / 256, fs.part_cols);
     fs.part_blocks = (k / 256 + splits - 1) / splits;
     const size_t part_bytes = tall ? (size_t)tail.tiles * tail.splits * 131072 : splits > 1 ? (size_t)splits * m * fs.part_cols * 4 : 0;
     uint8_t* ws;

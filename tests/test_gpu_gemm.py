@@ -243,6 +243,25 @@ def test_gemm_with_k_split_over_workgroups(hip, qtype, m, n, k):
             assert err <= TOL, f"{splits} parts, form {form}, tile {tile}: rel err {err}"
 
 
+@pytest.mark.parametrize("m,n,k,parts", [(200, 4096, 2048, False), (64, 8192, 2048, False), (128, 4096, 3072, False), (512, 2048, 2048, False),
+                                         (1024, 1024, 4096, False), (41, 4096, 11008, True), (41, 4096, 4096, True), (512, 512, 4096, True)])
+def test_gemm_q4k_k_is_split_only_where_that_pays(hip, m, n, k, parts):
+    """Activation pass and product; a third launch where k is divided over workgroups: not for rows so short that the addition
+    costs more than the steps it saves.  Sampled columns."""
+    assert hip.device_info()["compute_units"] == 256, "the shapes are chosen for 256 compute units"
+    raw = synth.weight(Q4_K, n, k, seed=m + n)
+    a = synth.activation_bf16((m, k), seed=k)
+    w, x, c = hip.to_device(raw), hip.to_device(a), hip.alloc(4 * m * n)
+    before = hip.stat("launches")
+    hip.gemm_q(Q4_K, w, n, k, x, m, c)
+    assert hip.stat("launches") - before == (3 if parts else 2)
+    cols = np.arange(0, n, 61)
+    want = oracle_c.gemm_q(Q4_K, raw.reshape(n, -1)[cols].reshape(-1), len(cols), k, a, m)
+    got = c.download(np.float32, m * n).reshape(m, n)
+    floor = 1e-3 * np.abs(got).max()
+    assert np.max(np.abs(got[:, cols] - want) / np.maximum(np.abs(want), floor)) <= TOL
+
+
 @pytest.mark.parametrize("n", [4096, 14336])
 def test_gemm_benchmark_shapes_q6k(hip, n):
     """M=512, K=4096 with Q6_K weights (the mixed-precision prefill case), sampled columns."""
