@@ -2130,15 +2130,15 @@ static TallTail tall_tail(const skn_ctx* ctx, int tiles, int nb) {
 }
 
 // The same for the Q4_K kernel of 64- and 128-row tiles, whose step along k is short: only where the steps saved (a group of
-// four superblocks each: 1.9 us on 64 rows, 3 us on 128) pay for the second launch and for the parts' way through memory (0.6 us
-// per MB; `cols` of all the launch's matrices).  Fitted to 290 shapes of 33 to 1024 rows, 256 to 11008 columns and k from 1536 to
-// 11008.  us per call, unsplit | split: 200 x 4096 x 2048 17.3 | 20.1, 512 x 2048 x 2048 19.0 | 24.4, 64 x 8192 x 2048 13.3 | 15.4, all
-// three unsplit now; 512 x 512 x 4096 27.0 | 20.4, 200 x 4096 x 6144 35.6 | 31.5, both split.
+// four superblocks each: 1.9 us on 64 rows, 3.4 us on 128) pay for the second launch, which costs as much as one of them, and for
+// the parts' way through memory (0.6 us per MB; `cols` of all the launch's matrices).  Fitted to 290 shapes of 33 to 1024 rows, 256 to
+// 11008 columns and k from 1536 to 11008.  us per call, unsplit | split: 200 x 4096 x 2048 17.3 | 20.1, 512 x 2048 x 2048 19.0 | 24.4,
+// 64 x 8192 x 2048 13.3 | 15.4, all three unsplit; 512 x 512 x 4096 27.0 | 20.4, 200 x 4096 x 6144 35.6 | 31.5, both split.
 static int q4k_splits(const skn_ctx* ctx, int m, int tile_rows, int tiles, int nb, int cols) {
     const int splits = skn_gemm_k_splits(ctx, m, tiles, nb);
     if (splits < 2 || ctx->opt_gemm_split > 0) return splits;
     const int each = (nb + splits - 1) / splits, saved = (nb + 3) / 4 - (each + 3) / 4;
-    const double gain_us = tile_rows == 64 ? 1.9 * (saved - 1) : 3.0 * saved - 1.2;
+    const double gain_us = (tile_rows == 64 ? 1.9 : 3.4) * (saved - 1);
     return gain_us > 0.6e-6 * 4.0 * splits * m * cols ? splits : 1;
 }
 

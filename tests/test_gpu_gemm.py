@@ -244,7 +244,7 @@ def test_gemm_with_k_split_over_workgroups(hip, qtype, m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k,parts", [(200, 4096, 2048, False), (64, 8192, 2048, False), (128, 4096, 3072, False), (512, 2048, 2048, False),
-                                         (1024, 1024, 4096, False), (41, 4096, 11008, True), (41, 4096, 4096, True), (512, 512, 4096, True)])
+                                         (1024, 1024, 4096, False), (200, 1024, 2048, False), (41, 4096, 11008, True), (41, 4096, 4096, True), (512, 512, 4096, True)])
 def test_gemm_q4k_k_is_split_only_where_that_pays(hip, m, n, k, parts):
     """Activation pass and product; a third launch where k is divided over workgroups: not for rows so short that the addition
     costs more than the steps it saves.  Sampled columns."""
