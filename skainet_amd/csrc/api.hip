@@ -304,6 +304,7 @@ int skn_get_stat(skn_ctx* ctx, const char* key, int64_t* value) {
     SKN_REQUIRE(nullptr, ctx != nullptr, SKN_ERR_ARG, "skn_get_stat: ctx is null");
     SKN_REQUIRE(ctx, key && value, SKN_ERR_ARG, "skn_get_stat: null pointer");
     if (!strcmp(key, "launches")) *value = ctx->stat_launches;
+    else if (!strcmp(key, "workgroups")) *value = ctx->stat_workgroups;
     else if (!strcmp(key, "graph.captures")) *value = ctx->stat_captures;
     else if (!strcmp(key, "llama.expanded_bytes")) *value = ctx->stat_expanded_bytes;
     else if (!strcmp(key, "profiler.attached")) *value = ctx->profiler_attached ? 1 : 0;

@@ -32,7 +32,7 @@ struct skn_ctx {
     int opt_q4k_waves = 0, opt_q4k_rows = 0, opt_attn_splits = 0, opt_llama_graph = 1, opt_llama_fused = 1, opt_gemm_tile = 0, opt_gemm_split = 0, opt_matvec_stage = 1, opt_llama_expand = 0, opt_test_rope_table = 0, opt_llama_attn_wide = 1, opt_gemm_q6k_fused = 1, opt_dense_tile = 0;
     int opt_generation = 0;          // bumped by every skn_set_option / skn_set_stream: captured work is stamped with it
     bool profiler_attached = false;  // a rocprofiler tool library is loaded into this process: graphs are not replayed
-    long long stat_launches = 0, stat_captures = 0;  // kernel launches issued (or recorded) / decode-step graphs captured
+    long long stat_launches = 0, stat_workgroups = 0, stat_captures = 0;  // kernel launches issued (or recorded) and their workgroups / decode-step graphs captured
     long long stat_expanded_bytes = 0;               // device bytes held by the decoders' expanded weight copies
     // scratch for split-context attention partials, grown on demand
     void* attn_scratch = nullptr;
@@ -126,6 +126,7 @@ int skn_fail(skn_ctx* ctx, int code, const char* fmt, ...);
 template <typename F, typename... Args>
 inline void skn_launch(skn_ctx* ctx, F kernel, dim3 grid, dim3 block, size_t lds, Args... args) {
     ctx->stat_launches++;
+    ctx->stat_workgroups += (long long)grid.x * grid.y * grid.z;
     if (ctx->prof_on && 2 * ctx->prof_used + 1 < ctx->prof_events.size()) {
         hipEvent_t e0 = ctx->prof_events[2 * ctx->prof_used], e1 = ctx->prof_events[2 * ctx->prof_used + 1];
         ctx->prof_used++;

@@ -1767,8 +1767,11 @@ int dispatch_q4k_fused(skn_ctx* ctx, const skn_q4k_segments& seg, int n_out, int
                     : launch_q4k_fused<STEPS, SKN_EPI_SWIGLU, false, F>(ctx, seg, n_out, nb, x, norm_w, eps, y, rope);
     // One row per wavefront where pairs would give fewer than two workgroups per compute unit (the output and down projections of
     // widths up to 8192): a decode step of the 7B shape at 150 tokens 1481 -> 1449 us, of 8 layers of width 2048 at 2000 tokens 299 ->
-    // 279.  Before, the plain matvec alone divided its rows so.
-    if (epi == SKN_EPI_ADD && !norm && n_out < 32 * ctx->compute_units)
+    // 279.  Not where the staging merges attention splits and twice the workgroups would read more than 16 MiB of partials in all
+    // (one | two rows per wavefront, four layers of the 7B shape at 640 tokens, four splits: 201 | 197 us a step; width 2048, eight
+    // splits of 32 heads, 4000 tokens: 125.5 | 127.2; width 4096 and two splits: no difference).
+    const bool merges_much = rope.merge_splits > 1 && (int64_t)(n_out / 8) * rope.merge_splits * nb * 1024 > (int64_t)16 << 20;
+    if (epi == SKN_EPI_ADD && !norm && n_out < 32 * ctx->compute_units && !merges_much)
         return launch_q4k_fused<STEPS, SKN_EPI_ADD, false, F, 1>(ctx, seg, n_out, nb, x, norm_w, eps, y, rope);
     if (epi == SKN_EPI_ADD)
         return norm ? launch_q4k_fused<STEPS, SKN_EPI_ADD, true, F>(ctx, seg, n_out, nb, x, norm_w, eps, y, rope)

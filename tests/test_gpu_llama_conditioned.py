@@ -197,6 +197,29 @@ def test_contexts_of_one_round_take_one_workgroup_per_head(hip, head_dim, contex
     model.free()
 
 
+@pytest.mark.parametrize("hidden,rows", [(4096, 2), (2048, 1)])
+def test_output_projection_that_merges_many_splits_takes_row_pairs(hip, hidden, rows):
+    """Every workgroup of the output projection reads the unmerged partials of all splits: pairs of rows per wavefront (half the
+    workgroups) where that is much (four splits of 4096 columns), single rows elsewhere.  Counted in the workgroups of a step
+    behind 600 tokens against one behind 40, which merges nothing: three more per head for the attention, and half of the projection's
+    hidden / 8 less."""
+    cfg = llama.Config(n_layer=1, hidden=hidden, ffn=512, n_head=hidden // 128, head_dim=128, vocab=256, max_tokens=768, page_tokens=256)
+    model = llama.LlamaModel(hip, cfg, weights=llama.random_weights(cfg, seed=5))
+    took = []
+    hip.set_option("llama.graph", 0)
+    try:
+        for context in (40, 600):
+            model.reset()
+            first = model.prefill(tokens(context, cfg.vocab, seed=2))
+            before = hip.stat("workgroups")
+            model.decode(first, 1)
+            took.append(hip.stat("workgroups") - before)
+    finally:
+        hip.set_option("llama.graph", 1)
+    assert took[1] - took[0] == 3 * cfg.n_head - (hidden // 8 - hidden // (8 * rows)), took
+    model.free()
+
+
 def test_several_steps_per_call_equal_one_step_per_call(hip):
     """skn_llama_decode with n steps feeds its own greedy tokens back: the same tokens and final logits as n calls."""
     cfg = CASES["q4_k_kv2"]
