@@ -222,10 +222,47 @@ int dev_alloc(skn_ctx* ctx, skn_llama* m, T** p, size_t count) {
 
 unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
 
-// The launches of one decode step (eagerly or under stream capture) at contexts of up to 128 * units tokens.
-int decode_step(skn_ctx* ctx, skn_llama* m, int units) {
+// The attention of a decode step at contexts of up to ctx_len tokens, rounded up to a power of two of 128 (the kernels derive their
+// ranges from the actual length, so one captured step serves every position up to there).
+struct AttnShape {
+    int splits;  // of the kernel that merges by itself; 0 where no layer runs it
+    int wide;    // workgroups of sixteen wavefronts per head, merged by the output projection; 0: the other kernel
+    int key() const { return splits | wide << 16; }
+};
+
+bool output_fused(const skn_ctx* ctx, const skn_llama_config& c, const skn_llama_layer& L) {
+    return ctx->opt_llama_fused && c.hidden <= 16384 && c.hidden % 256 == 0 && skn_matvec_fusable(L.type_o);
+}
+
+// A workgroup of sixteen wavefronts takes 32768 / head_dim tokens per round of requests.  Up to a round it has nothing to merge
+// (contexts of 120 - 184 tokens, 32 heads of 128: 5.1 us against 6.9 us for two splits behind a counter).
+// Beyond a round: 2, 4 or 8 (what the projection's staging is built to merge), no more workgroups than compute units (64 heads of
+// 128 at 1100 / 4000 tokens, two | four | eight: 245 | 244 | 268, 286 | 261 | 285), and as many as there are with eight only where
+// each has four rounds or more (32 heads of 128 at 1500 tokens, four | eight: 208 | 211; 32 of 256 at 640 / 4000: 250 | 259, 302 | 286).
+// "attn.splits" takes the place of the compute units' share.
+AttnShape attn_shape(skn_ctx* ctx, const skn_llama* m, int ctx_len) {
     const skn_llama_config& c = m->cfg;
-    const int n_splits = std::min(units, skn_attn_splits(ctx, c.n_head, c.max_tokens));
+    int units = 1;
+    while (units * 128 < ctx_len) units *= 2;
+    AttnShape s = {std::min(units, skn_attn_splits(ctx, c.n_head, c.max_tokens)), 0};
+    const int per_round = 32768 / c.head_dim, tokens = units * 128, share = ctx->opt_attn_splits > 0 ? ctx->opt_attn_splits : ctx->compute_units / c.n_head;
+    if (!ctx->opt_llama_attn_wide) return s;
+    if (tokens <= per_round) {
+        if (ctx->opt_attn_splits == 0) s.wide = 1;
+        return s;
+    }
+    if (share < 2) return s;
+    if (std::all_of(m->layers.begin(), m->layers.end(), [&](const skn_llama_layer& L) { return output_fused(ctx, c, L); })) s.splits = 0;
+    s.wide = 2;
+    while (s.wide < 8 && s.wide * per_round < tokens && 2 * s.wide <= share) s.wide *= 2;
+    if (s.wide == 8 && ctx->opt_attn_splits == 0 && 8 * c.n_head >= ctx->compute_units && tokens < 32 * per_round) s.wide = 4;
+    if (ctx->opt_llama_attn_wide > 1) s.wide = std::min(s.wide, ctx->opt_llama_attn_wide);  // (2, 4 or 8 caps the count)
+    return s;
+}
+
+// the launches of one decode step (eagerly or under stream capture)
+int decode_step(skn_ctx* ctx, skn_llama* m, const AttnShape& shape) {
+    const skn_llama_config& c = m->cfg;
     const int H = c.hidden, F = c.ffn, NH = c.n_head, D = c.head_dim, KVH = c.n_kv_head, KVD = KVH * D;
     const float scale = 1.0f / sqrtf((float)D);
     skn_launch(ctx, embed_rows_kernel, dim3(1), dim3(1024), 0, (const uint8_t*)m->w.tok_embd, m->w.type_embd, H,
@@ -241,7 +278,7 @@ int decode_step(skn_ctx* ctx, skn_llama* m, int units) {
         const bool fuse = ctx->opt_llama_fused && H <= 16384 && H % 256 == 0;
         // (q, k, v of different fusable formats: one fused launch per format, each with the rows of its matrices only)
         const bool f_qkv = fuse && skn_matvec_fusable(L.type_q) && skn_matvec_fusable(L.type_k) && skn_matvec_fusable(L.type_v);
-        const bool f_o = fuse && skn_matvec_fusable(L.type_o);
+        const bool f_o = output_fused(ctx, c, L);
         const bool f_gu = fuse && skn_matvec_fusable(L.type_gate) && L.type_up == L.type_gate;
         const bool f_down = ctx->opt_llama_fused && F <= 16384 && F % 256 == 0 && skn_matvec_fusable(L.type_down);
         if (f_qkv) {
@@ -298,13 +335,10 @@ int decode_step(skn_ctx* ctx, skn_llama* m, int units) {
                        kv->page_tokens, log2((double)c.rope_base));
             SKN_LAUNCH_CHECK(ctx);
         }
-        const int per_round = 32768 / D;  // tokens that a workgroup of sixteen wavefronts takes per round of requests
-        if (f_o && ctx->opt_llama_attn_wide && units * 128 > per_round) {
+        const int wide = shape.wide;
+        if (f_o && wide > 1) {
             // The attention leaves the partials of its splits unmerged and the output projection's staging merges them:
             // no device-wide counter, no store-then-reload chain inside the attention launch.
-            int wide = 2;  // 2, 4 or 8 (what the merge in the projection's staging is built for)
-            while (wide < 8 && wide * per_round < units * 128) wide *= 2;
-            if (ctx->opt_llama_attn_wide > 1) wide = std::min(wide, ctx->opt_llama_attn_wide);  // (tuning: 2, 4 or 8 caps the count)
             float* opart = m->attn_partial;
             float* ml = m->attn_partial + (size_t)wide * NH * D;
             SKN_TRY(skn_attn_launch_unmerged(ctx, kv, m->q, m->step.state + 2, 1, 0, wide, opart, ml, scale, m->att, NH));
@@ -316,16 +350,14 @@ int decode_step(skn_ctx* ctx, skn_llama* m, int units) {
             mg.merge_head_f4 = D / 4;
             SKN_TRY(skn_matvec_q4k_fused(ctx, wo, H, H, opart, nullptr, 0.f, m->x, SKN_EPI_ADD, &mg, L.type_o));
         } else if (f_o) {
-            // up to one round: a workgroup per head, nothing to merge (contexts of 120 - 184 tokens, 32 heads of 128: 5.1 us against
-            // 6.9 us for two splits behind a counter)
-            if (ctx->opt_llama_attn_wide)
+            if (wide)
                 SKN_TRY(skn_attn_launch_unmerged(ctx, kv, m->q, m->step.state + 2, 1, 0, 1, nullptr, nullptr, scale, m->att, NH));
             else
-                SKN_TRY(skn_attn_launch_ex(ctx, kv, m->q, m->step.state + 2, 1, 0, n_splits, m->attn_partial, m->attn_counters, scale, m->att, NH));
+                SKN_TRY(skn_attn_launch_ex(ctx, kv, m->q, m->step.state + 2, 1, 0, shape.splits, m->attn_partial, m->attn_counters, scale, m->att, NH));
             skn_q4k_segments wo = {{(const uint8_t*)L.wo, nullptr, nullptr}, {H, 0, 0}};
             SKN_TRY(skn_matvec_q4k_fused(ctx, wo, H, H, m->att, nullptr, 0.f, m->x, SKN_EPI_ADD, nullptr, L.type_o));
         } else {
-            SKN_TRY(skn_attn_launch_ex(ctx, kv, m->q, m->step.state + 2, 1, 0, n_splits, m->attn_partial, m->attn_counters, scale, m->att, NH));
+            SKN_TRY(skn_attn_launch_ex(ctx, kv, m->q, m->step.state + 2, 1, 0, shape.splits, m->attn_partial, m->attn_counters, scale, m->att, NH));
             SKN_TRY(skn_matvec_q(ctx, L.type_o, L.wo, H, H, m->att, m->proj));
             skn_launch(ctx, add_rows_kernel, dim3(nblk(H)), dim3(256), 0, m->x, (const float*)m->proj, (int64_t)H);
             SKN_LAUNCH_CHECK(ctx);
@@ -729,13 +761,11 @@ int skn_llama_decode(skn_ctx* ctx, skn_llama* m, int32_t first_token, int n_step
                 "skn_llama_decode: not available while per-launch timing is on (except with llama.graph = 0)");
     // every page the run will touch is mapped now; the step itself never talks to the host
     for (skn_kv* kv : m->kv) SKN_TRY(skn_kv_reserve(ctx, kv, 0, m->pos + n_steps));
-    // The longest context of this run, rounded up to a power of two of 128-token units, decides the attention's splits (the
-    // kernels derive their ranges from the actual length, so one captured step serves every position up to there): the step is
-    // captured again only when a sequence grows past 128, 256, 512, ... tokens, and a short context is not cut into
-    // more pieces than it has work for (sixteen splits of 600 tokens cost 2 % of the step against eight).
-    int units = 1;
-    while (units * 128 < m->pos + n_steps) units *= 2;
-    SKN_TRY(skn_stepper_run(ctx, &m->step, first_token, m->pos, n_steps, units, [&]() { return decode_step(ctx, m, units); },
+    // The step is captured again only when a sequence grows past 128, 256, 512, ... tokens and the attention takes another shape for
+    // it: a short context is not cut into more pieces than it has work for (sixteen splits of 600 tokens cost 2 % of the step
+    // against eight).
+    const AttnShape shape = attn_shape(ctx, m, m->pos + n_steps);
+    SKN_TRY(skn_stepper_run(ctx, &m->step, first_token, m->pos, n_steps, shape.key(), [&]() { return decode_step(ctx, m, shape); },
                             tokens_out_host));
     m->pos += n_steps;
     for (skn_kv* kv : m->kv) kv->len[0] = m->pos;

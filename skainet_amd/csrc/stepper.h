@@ -15,7 +15,7 @@ struct skn_stepper {
     int cap = 0;                    // tokens the array holds
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
-    int graph_key = 0;          // the shape the step was captured for (the caller's: its attention split count)
+    int graph_key = 0;          // the shape the step was captured for (the caller's: what its attention's launches depend on)
     int graph_generation = -1;  // ctx->opt_generation at capture: every option a step reads, and the stream
 };
 

@@ -220,6 +220,44 @@ def test_output_projection_that_merges_many_splits_takes_row_pairs(hip, hidden, 
     model.free()
 
 
+def test_attention_splits_option_bounds_the_decoders_splits(hip):
+    """600 tokens of heads of 128 take four splits by themselves; "attn.splits" = 2 makes them two, as the cap of llama.attn_wide does:
+    the same launches, so the same bits."""
+    cfg = llama.Config(n_layer=2, hidden=512, ffn=768, n_head=4, head_dim=128, vocab=512, max_tokens=640, page_tokens=16)
+    model = llama.LlamaModel(hip, cfg, weights=llama.conditioned_weights(cfg, SEED))
+    prompt, got = tokens(600, cfg.vocab, seed=2), {}
+    for key, value, back in (("attn.splits", 2, 0), ("llama.attn_wide", 2, 1), ("llama.attn_wide", 1, 1)):
+        model.reset()
+        model.prefill(prompt)
+        hip.set_option(key, value)
+        try:
+            model.decode(7, 4)
+        finally:
+            hip.set_option(key, back)
+        got[key, value] = model.logits().view(np.uint32)
+    assert np.array_equal(got["attn.splits", 2], got["llama.attn_wide", 2])
+    assert not np.array_equal(got["attn.splits", 2], got["llama.attn_wide", 1])
+    model.free()
+
+
+def test_step_is_captured_again_only_for_another_shape_of_the_attention(hip):
+    """Two heads of 256: eight splits from 1024 tokens on, the most there are, so the graph that was captured below 1024 serves the
+    steps past it, and past 2048."""
+    if hip.stat("profiler.attached"):
+        pytest.skip("a profiler is attached: steps are not captured")
+    cfg = llama.Config(n_layer=1, hidden=512, ffn=768, n_head=2, head_dim=256, vocab=512, max_tokens=2304, page_tokens=256)
+    model = llama.LlamaModel(hip, cfg, weights=llama.conditioned_weights(cfg, SEED))
+    model.prefill(tokens(1000, cfg.vocab, seed=2))
+    before = hip.stat("graph.captures")
+    model.decode(3, 8)
+    assert hip.stat("graph.captures") - before == 1
+    model.decode(3, 40)
+    model.prefill(tokens(1010, cfg.vocab, seed=3))
+    model.decode(3, 8)
+    assert hip.stat("graph.captures") - before == 1
+    model.free()
+
+
 def test_several_steps_per_call_equal_one_step_per_call(hip):
     """skn_llama_decode with n steps feeds its own greedy tokens back: the same tokens and final logits as n calls."""
     cfg = CASES["q4_k_kv2"]
