@@ -235,7 +235,9 @@ bool output_fused(const skn_ctx* ctx, const skn_llama_config& c, const skn_llama
 }
 
 // A workgroup of sixteen wavefronts takes 32768 / head_dim tokens per round of requests.  Up to a round it has nothing to merge
-// (contexts of 120 - 184 tokens, 32 heads of 128: 5.1 us against 6.9 us for two splits behind a counter).
+// (contexts of 120 - 184 tokens, 32 heads of 128: 5.1 us against 6.9 us for two splits behind a counter), but a short context is
+// done sooner by the smaller workgroups of the other kernel (us a step of four layers, that | this: 32 heads of 128 at 24 / 100
+// tokens 181 | 187, 188 | 189.5; 48 of 64 at 100 tokens 113 | 119; 8 of 256 at 24 / 80 tokens 102.4 | 104.5, 108 | 104.5).
 // Beyond a round: 2, 4 or 8 (what the projection's staging is built to merge), no more workgroups than compute units (64 heads of
 // 128 at 1100 / 4000 tokens, two | four | eight: 245 | 244 | 268, 286 | 261 | 285), and as many as there are with eight only where
 // each has four rounds or more (32 heads of 128 at 1500 tokens, four | eight: 208 | 211; 32 of 256 at 640 / 4000: 250 | 259, 302 | 286).
@@ -248,7 +250,7 @@ AttnShape attn_shape(skn_ctx* ctx, const skn_llama* m, int ctx_len) {
     const int per_round = 32768 / c.head_dim, tokens = units * 128, share = ctx->opt_attn_splits > 0 ? ctx->opt_attn_splits : ctx->compute_units / c.n_head;
     if (!ctx->opt_llama_attn_wide) return s;
     if (tokens <= per_round) {
-        if (ctx->opt_attn_splits == 0) s.wide = 1;
+        if (ctx->opt_attn_splits == 0 && ctx_len > std::min(128, per_round / 2)) s.wide = 1;
         return s;
     }
     if (share < 2) return s;

@@ -258,6 +258,26 @@ def test_step_is_captured_again_only_for_another_shape_of_the_attention(hip):
     model.free()
 
 
+@pytest.mark.parametrize("head_dim,context,wide", [(64, 20, 0), (64, 100, 0), (128, 20, 0), (128, 100, 0), (256, 20, 0), (256, 100, 1), (64, 200, 1), (128, 200, 1)])
+def test_short_contexts_take_the_smaller_workgroups(hip, head_dim, context, wide):
+    """Up to 128 tokens (64 at heads of 256) a step runs the attention kernel that it runs with llama.attn_wide off, and gives its bits;
+    past that another one, which adds in another order."""
+    cfg = llama.Config(n_layer=2, hidden=512, ffn=768, n_head=512 // head_dim, head_dim=head_dim, vocab=512, max_tokens=256, page_tokens=16)
+    model = llama.LlamaModel(hip, cfg, weights=llama.conditioned_weights(cfg, SEED))
+    prompt, got = tokens(context, cfg.vocab, seed=2), []
+    for option in (1, 0):
+        model.reset()
+        model.prefill(prompt)
+        hip.set_option("llama.attn_wide", option)
+        try:
+            model.decode(7, 8)
+        finally:
+            hip.set_option("llama.attn_wide", 1)
+        got.append(model.logits().view(np.uint32))
+    assert np.array_equal(*got) == (not wide)
+    model.free()
+
+
 def test_several_steps_per_call_equal_one_step_per_call(hip):
     """skn_llama_decode with n steps feeds its own greedy tokens back: the same tokens and final logits as n calls."""
     cfg = CASES["q4_k_kv2"]
