@@ -439,17 +439,19 @@ int launch_rows(skn_ctx* ctx, const skn_rstate* st, const float* r, const float*
 
 template <int L, int NW>
 int launch_step(skn_ctx* ctx, const skn_rstate* st, const skn_delta_step& p, float* state, const skn_beside* beside) {
-    if (beside) {
-        SKN_REQUIRE(ctx, beside->type == p.w2_type, SKN_ERR_TYPE, "delta rule: a product of another type beside a step");
-        skn_beside s = *beside;
-        skn_beside_plan(ctx, s, 64 * NW);
-        const dim3 grid((unsigned)(st->heads + s.blocks));
-        const int plane = skn_beside_plane(s);
-        const size_t lds = skn_beside_lds(s);
-        if (s.type == SKN_TYPE_F32) skn_launch(ctx, delta_step_beside_kernel<L, NW, float>, grid, dim3(64 * NW), lds, p, st->dim, state, st->heads, s, plane);
-        else skn_launch(ctx, delta_step_beside_kernel<L, NW, uint16_t>, grid, dim3(64 * NW), lds, p, st->dim, state, st->heads, s, plane);
-        SKN_LAUNCH_CHECK(ctx);
-        return SKN_OK;
+    if constexpr (8 * L > kDeltaPairDim) {
+        if (beside) {
+            SKN_REQUIRE(ctx, beside->type == p.w2_type, SKN_ERR_TYPE, "delta rule: a product of another type beside a step");
+            skn_beside s = *beside;
+            skn_beside_plan(ctx, s, 64 * NW);
+            const dim3 grid((unsigned)(st->heads + s.blocks));
+            const int plane = skn_beside_plane(s);
+            const size_t lds = skn_beside_lds(s);
+            if (s.type == SKN_TYPE_F32) skn_launch(ctx, delta_step_beside_kernel<L, NW, float>, grid, dim3(64 * NW), lds, p, st->dim, state, st->heads, s, plane);
+            else skn_launch(ctx, delta_step_beside_kernel<L, NW, uint16_t>, grid, dim3(64 * NW), lds, p, st->dim, state, st->heads, s, plane);
+            SKN_LAUNCH_CHECK(ctx);
+            return SKN_OK;
+        }
     }
     if (p.w2_type == SKN_TYPE_F32) skn_launch(ctx, delta_step_kernel<L, NW, float>, dim3(st->heads), dim3(64 * NW), 0, p, st->dim, state);
     else skn_launch(ctx, delta_step_kernel<L, NW, uint16_t>, dim3(st->heads), dim3(64 * NW), 0, p, st->dim, state);
@@ -488,6 +490,7 @@ int skn_delta_gate_rows(skn_ctx* ctx, const float* o, const float* g, int ldg, c
 }
 
 int skn_delta_step_launch(skn_ctx* ctx, skn_rstate* st, int seq, const skn_delta_step& p, const skn_beside* beside) {
+    SKN_REQUIRE(ctx, !beside || st->dim_pad > kDeltaPairDim, SKN_ERR_SHAPE, "delta rule: nothing runs beside a step of heads of %d channels", st->dim);
     float* s = st->seq_state(seq);
     switch (st->dim_pad) {
         case 32: return launch_step<4, 2>(ctx, st, p, s, beside);

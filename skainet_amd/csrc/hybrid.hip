@@ -199,14 +199,21 @@ skn_dense_out side_segment(const skn_hybrid* m, int l, const int32_t* tokens, vo
 
 // ---- decode -----------------------------------------------------------------------------------------------------------
 
-// The feed-forward's part of the output product, to run beside the mixer (no w: it stays in the output product).  Wherever the mixer
-// can take it: the two together read what they read apart, in a launch that is at least as full; the limit is the LDS that a launch
-// has without asking for more (feed-forwards of 14336 columns beside the delta rule, 12288, 10240 and 6144
-// beside attention heads of 64, 128 and 256).
+// The feed-forward's part of the output product, to run beside the mixer (no w: it stays in the output product).  Where it gains, us a
+// step of four layers, without | with: width 2048, 16 heads of 64, feed-forwards of 4096 / 5500 columns 114 | 110, 123 | 115; 1500
+// columns 101 | 100.  Not
+//   - beside a step of the delta rule with heads of up to 32 channels, whose workgroups have two wavefronts: each would stage the whole
+//     input for two rows (two layers, width 2048, 8192 columns 73.4 | 77.5; 14000 columns 93.5 | 107.6),
+//   - for rows of less than 2560 bytes, too few to pay for the larger launch (1000 columns, 32 heads of 64: width 2048 105.3 | 105.6,
+//     2560 115.3 | 116.8; 600 columns 112.5 | 115.5),
+//   - past the LDS that a launch has without asking for more (feed-forwards of 14336 columns beside the delta rule, 12288, 10240 and
+//     6144 beside attention heads of 64, 128 and 256).
 skn_beside ff_beside(const skn_hybrid* m, const Layer& L, float* x) {
     skn_beside s;
     const bool general_delta = L.p.mixer == SKN_MIX_GENERAL_DELTA;
     if (L.p.mixer != SKN_MIX_SHARED_ATTN && !general_delta) return s;
+    if (general_delta && L.state->dim_pad <= kDeltaPairDim) return s;
+    if (L.p.ff * (L.out.type == SKN_TYPE_F32 ? 4 : 2) < 2560) return s;
     s.type = L.out.type;
     s.rows = m->cfg.width;
     s.k_pad = L.out.k_pad - L.off_ff;

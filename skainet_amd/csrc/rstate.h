@@ -41,6 +41,7 @@ struct skn_delta_step {
 };
 int skn_delta_step_launch(skn_ctx* ctx, skn_rstate* st, int seq, const skn_delta_step& p, const struct skn_beside* beside = nullptr);
 constexpr size_t kDeltaStepLds = 8192;  // at most, of a workgroup without a product beside it
+constexpr int kDeltaPairDim = 32;       // heads padded to this many channels: workgroups of two wavefronts, which take nothing beside them
 
 // ---- gated delta rule with a decay per key channel (csrc/gated_delta.hip; equations: skn_channel_delta of the header) ----
 // Rows of a prompt at positions pos0 ..: q, k, v before their convolutions, beta and z, all [n][ld]; cq, ck, cv [n][ld] scratch for

@@ -59,6 +59,32 @@ def test_feed_forward_beside_the_mixer_of_a_step(hip, width, ff, dtype):
     m.free()
 
 
+def step_workgroups(hip, cfg, seed=3):
+    """What one decode step launches, eagerly."""
+    m = cases.device_model(hip, cfg, cases.weights(cfg, 4, seed=seed), "bfloat16")
+    m.prefill(cases.tokens(cfg, 3))
+    hip.set_option("llama.graph", 0)
+    try:
+        before = hip.stat("workgroups")
+        m.decode(1, 1)
+        return hip.stat("workgroups") - before
+    finally:
+        hip.set_option("llama.graph", 1)
+        m.free()
+
+
+def test_short_feed_forwards_and_small_heads_have_nothing_beside_the_mixer(hip):
+    """Seen in the workgroups of a step: a wavefront per row of 512 beside the mixer, eight to a workgroup.  32 more columns of the
+    feed-forward are four more workgroups of the input product and, past 2560 bytes a row, the 64 beside; heads of 32 channels take
+    two launches' worth of heads and nothing beside them."""
+    def taken(heads, dim, ff):
+        return step_workgroups(hip, cases.model([cases.delta(heads, dim, ff=ff)], width=512, vocab=40, groups=1))
+
+    assert taken(4, 64, 1280) - taken(4, 64, 1248) == 4 + 64
+    assert taken(4, 64, 1312) - taken(4, 64, 1280) == 4
+    assert taken(4, 64, 2048) - taken(8, 32, 2048) == 64 - 4
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_logits_do_not_depend_on_the_cut(hip, dtype):
     cfg, rank = cases.MODELS["mixed"]
