@@ -15,11 +15,15 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// Eight wavefronts per workgroup: a matrix of 2048 rows then reaches 256 compute units (sixteen: half of them), and up to three
-// workgroups share a compute unit.  A decode step of eight layers of width 2048 (945 MB of weights, 27 launches): 313 us; one
-// workgroup of sixteen wavefronts per compute unit 330, two of them 341; eight wavefronts, one / two / four workgroups per compute
-// unit 327 / 319 / 338; four wavefronts, two / four / six / eight workgroups 342 / 335 / 331 / 351.
-constexpr int kThreads = 512, kWaves = kThreads / 64, kPerCu = 3;
+// Workgroups of T threads.  Eight wavefronts where that makes at most a workgroup per compute unit (a matrix of 2048 rows reaches 256
+// of them, with sixteen wavefronts half: 5.5 against 5.9 us at 2048 rows, 4.8 against 5.2 at 1024), and behind a norm where the rows
+// fill the device twice (4288 rows 13.0 against 14.5 us, 6016 rows 14.0 against 15.3) or are a single turn of requests long (3232 rows
+// of 2048 7.95 against 8.34 us), up to three per compute unit.  Sixteen, one workgroup per compute unit, for what lies between, where
+// the compute units with two workgroups of eight would be the last (2560 rows of 14000 16.6 against 18.8 us, of 6000 8.2 against 9.1;
+// behind a norm 2624 rows of 2560 8.0 against 8.5, 3232 rows of 4096 9.9 against 11.0), and for more rows behind a plain staging
+// (6144 rows 6.7 against 7.1).  A decode step of eight layers of width 2048 (945 MB of weights, 27 launches): 313 us; sixteen wavefronts
+// everywhere 330, four 331 and more.
+constexpr int kPerCu = 3;
 constexpr int kR = 1;  // rows per wavefront and turn (measured with two as well: slower)
 constexpr int kU = 4;  // 16-byte pieces per row and lane in flight, twice
 constexpr int kMaxGroups = 256, kMaxMerge = 4096, kMaxSplits = 16;  // norm groups; heads x splits and splits of a merge
@@ -31,7 +35,9 @@ struct XPlanes {
     __device__ __forceinline__ float& at(int e) const { return reinterpret_cast<float*>(&quad(e >> 2))[e & 3]; }
 };
 
+template <int T>
 __device__ __forceinline__ void stage_group_norm(const skn_matvec_src& s, const XPlanes& xs, float* red) {
+    constexpr int kWaves = T / 64;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, quads = (s.k0 + 3) >> 2, gs = s.k0 / s.groups;
     // (pitches are multiples of 64 elements and their padding is zero: the last quad may be read whole)
     const bool few = s.groups <= 8 && (gs & 3) == 0;
@@ -40,7 +46,7 @@ __device__ __forceinline__ void stage_group_norm(const skn_matvec_src& s, const 
 #pragma unroll
         for (int g = 0; g < 8; g++) ss[g] = 0.f;
         const float inv_quads = 4.0f / (float)gs;
-        for (int q = tid; q < quads; q += kThreads) {
+        for (int q = tid; q < quads; q += T) {
             const float4 v = reinterpret_cast<const float4*>(s.x0)[q];
             xs.quad(q) = v;
             const float d = (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
@@ -61,14 +67,14 @@ __device__ __forceinline__ void stage_group_norm(const skn_matvec_src& s, const 
             red[8 * kWaves + tid] = 1.0f / sqrtf(t / (float)gs + s.eps);
         }
         __syncthreads();
-        for (int q = tid; q < quads; q += kThreads) {
+        for (int q = tid; q < quads; q += T) {
             const float r = red[8 * kWaves + (int)(((float)q + 0.5f) * inv_quads)];
             const float4 v = xs.quad(q), g = reinterpret_cast<const float4*>(s.norm_w)[q];
             xs.quad(q) = make_float4(v.x * r * g.x, v.y * r * g.y, v.z * r * g.z, v.w * r * g.w);
         }
         return;
     }
-    for (int e = tid; e < s.k0; e += kThreads) xs.at(e) = s.x0[e];
+    for (int e = tid; e < s.k0; e += T) xs.at(e) = s.x0[e];
     __syncthreads();
     for (int g = wave; g < s.groups; g += kWaves) {
         float ss = 0.f;
@@ -80,50 +86,53 @@ __device__ __forceinline__ void stage_group_norm(const skn_matvec_src& s, const 
         if (lane == 0) red[g] = 1.0f / sqrtf(ss / (float)gs + s.eps);
     }
     __syncthreads();
-    for (int e = tid; e < s.k0; e += kThreads) xs.at(e) *= red[e / gs] * s.norm_w[e];
+    for (int e = tid; e < s.k0; e += T) xs.at(e) *= red[e / gs] * s.norm_w[e];
 }
 
 // the sum over the workgroup (a barrier inside; red: one float per wavefront, used once)
+template <int T>
 __device__ __forceinline__ float block_sum(float v, float* red) {
     v = wave_sum(v);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     v = 0.f;
 #pragma unroll
-    for (int i = 0; i < kWaves; i++) v += red[i];
+    for (int i = 0; i < T / 64; i++) v += red[i];
     return v;
 }
 
 // (pitches are multiples of 64 elements and their padding is zero, as in stage_group_norm; a thread's quads stay its own)
+template <int T>
 __device__ __forceinline__ void stage_add_norm(const skn_matvec_src& s, const XPlanes& xs, float* red) {
     const int tid = threadIdx.x, quads = (s.k0 + 3) >> 2;
     auto square = [](const float4& v) { return (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w); };
     float ss = 0.f;
-    for (int q = tid; q < quads; q += kThreads) {
+    for (int q = tid; q < quads; q += T) {
         const float4 v = reinterpret_cast<const float4*>(s.add)[q];
         xs.quad(q) = v;
         ss += square(v);
     }
-    const float ry = 1.0f / sqrtf(block_sum(ss, red) / (float)s.k0 + s.eps);
+    const float ry = 1.0f / sqrtf(block_sum<T>(ss, red) / (float)s.k0 + s.eps);
     ss = 0.f;
-    for (int q = tid; q < quads; q += kThreads) {
+    for (int q = tid; q < quads; q += T) {
         const float4 y = xs.quad(q), x = reinterpret_cast<const float4*>(s.x0)[q], g = reinterpret_cast<const float4*>(s.add_w)[q];
         const float4 v = make_float4(fmaf(y.x * ry, g.x, x.x), fmaf(y.y * ry, g.y, x.y), fmaf(y.z * ry, g.z, x.z), fmaf(y.w * ry, g.w, x.w));
         xs.quad(q) = v;
         if (blockIdx.x == 0) reinterpret_cast<float4*>(s.x_out)[q] = v;
         ss += square(v);
     }
-    const float rx = 1.0f / sqrtf(block_sum(ss, red + kWaves) / (float)s.k0 + s.eps);
-    for (int q = tid; q < quads; q += kThreads) {
+    const float rx = 1.0f / sqrtf(block_sum<T>(ss, red + T / 64) / (float)s.k0 + s.eps);
+    for (int q = tid; q < quads; q += T) {
         const float4 v = xs.quad(q), g = reinterpret_cast<const float4*>(s.norm_w)[q];
         xs.quad(q) = make_float4(v.x * rx * g.x, v.y * rx * g.y, v.z * rx * g.z, v.w * rx * g.w);
     }
 }
 
 // red: heads x splits weights
+template <int T>
 __device__ __forceinline__ void stage_merge(const skn_matvec_src& s, const XPlanes& xs, float* red) {
     const int tid = threadIdx.x;
-    for (int h = tid; h < s.heads; h += kThreads) {
+    for (int h = tid; h < s.heads; h += T) {
         float2 ml[kMaxSplits];  // (all requested before the first is used)
 #pragma unroll
         for (int i = 0; i < kMaxSplits; i++) ml[i] = reinterpret_cast<const float2*>(s.ml)[min(i, s.splits - 1) * s.heads + h];
@@ -145,7 +154,7 @@ __device__ __forceinline__ void stage_merge(const skn_matvec_src& s, const XPlan
     if ((s.dim & 3) == 0) {
         const int dq = s.dim >> 2;
         const int64_t step = (int64_t)s.heads * s.dim_pad;
-        for (int q = tid; q < s.heads * dq; q += kThreads) {
+        for (int q = tid; q < s.heads * dq; q += T) {
             const int h = q / dq, c = q - h * dq;
             const float* p = s.x0 + (int64_t)h * s.dim_pad + 4 * c;
             float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -167,7 +176,7 @@ __device__ __forceinline__ void stage_merge(const skn_matvec_src& s, const XPlan
         }
         return;
     }
-    for (int e = tid; e < s.k0; e += kThreads) {
+    for (int e = tid; e < s.k0; e += T) {
         const int h = e / s.dim, d = e - h * s.dim;
         float a = 0.f;
         for (int i = 0; i < s.splits; i++) a = fmaf(red[h * s.splits + i], s.x0[((int64_t)i * s.heads + h) * s.dim_pad + d], a);
@@ -176,18 +185,18 @@ __device__ __forceinline__ void stage_merge(const skn_matvec_src& s, const XPlan
 }
 
 // W: uint16_t (bf16) or float.  LDS: two planes of `plane` float4, then the scratch of the staging.
-template <typename W, int MODE>
-__global__ __launch_bounds__(kThreads) void dense_matvec_kernel(const W* __restrict__ w, int rows, int k_pad, int ld, int plane,
-                                                                const float* __restrict__ bias, const skn_matvec_src src,
-                                                                const skn_dense_out out) {
+template <typename W, int MODE, int T>
+__global__ __launch_bounds__(T) void dense_matvec_kernel(const W* __restrict__ w, int rows, int k_pad, int ld, int plane,
+                                                         const float* __restrict__ bias, const skn_matvec_src src,
+                                                         const skn_dense_out out) {
     extern __shared__ __align__(16) float4 lds4[];
     constexpr int V = 16 / (int)sizeof(W);
     const XPlanes xs = {lds4, lds4 + plane};
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pieces = k_pad / V;                           // 16-byte pieces of a row
     const int turns = (pieces + 64 * kU - 1) / (64 * kU);   // requests per row, kU pieces per lane each
-    const int groups = (rows + kR - 1) / kR, stride = (int)gridDim.x * kWaves;
-    int grp = (int)blockIdx.x * kWaves + wave, turn = 0;
+    const int groups = (rows + kR - 1) / kR, stride = (int)gridDim.x * (T / 64);
+    int grp = (int)blockIdx.x * (T / 64) + wave, turn = 0;
 
     u32x4 cur[kR][kU], nxt[kR][kU];
     auto fetch = [&](u32x4(&buf)[kR][kU], int g, int t) __attribute__((always_inline)) {
@@ -201,22 +210,22 @@ __global__ __launch_bounds__(kThreads) void dense_matvec_kernel(const W* __restr
     fetch(cur, min(grp, groups - 1), 0);
 
     // ---- staging ----
-    if constexpr (MODE == SKN_XSRC_GROUP_NORM) stage_group_norm(src, xs, reinterpret_cast<float*>(lds4 + 2 * plane));
-    else if constexpr (MODE == SKN_XSRC_ADD_NORM) stage_add_norm(src, xs, reinterpret_cast<float*>(lds4 + 2 * plane));
-    else if constexpr (MODE == SKN_XSRC_MERGE) stage_merge(src, xs, reinterpret_cast<float*>(lds4 + 2 * plane));
+    if constexpr (MODE == SKN_XSRC_GROUP_NORM) stage_group_norm<T>(src, xs, reinterpret_cast<float*>(lds4 + 2 * plane));
+    else if constexpr (MODE == SKN_XSRC_ADD_NORM) stage_add_norm<T>(src, xs, reinterpret_cast<float*>(lds4 + 2 * plane));
+    else if constexpr (MODE == SKN_XSRC_MERGE) stage_merge<T>(src, xs, reinterpret_cast<float*>(lds4 + 2 * plane));
     else {
-        for (int q = tid; q < src.k0 >> 2; q += kThreads) xs.quad(q) = reinterpret_cast<const float4*>(src.x0)[q];
-        for (int e = (src.k0 & ~3) + tid; e < src.k0; e += kThreads) xs.at(e) = src.x0[e];
+        for (int q = tid; q < src.k0 >> 2; q += T) xs.quad(q) = reinterpret_cast<const float4*>(src.x0)[q];
+        for (int e = (src.k0 & ~3) + tid; e < src.k0; e += T) xs.at(e) = src.x0[e];
     }
     if (src.x1) {
-        for (int q = tid; q < src.k1 >> 2; q += kThreads) xs.quad((src.off1 >> 2) + q) = reinterpret_cast<const float4*>(src.x1)[q];
-        for (int e = (src.k1 & ~3) + tid; e < src.k1; e += kThreads) xs.at(src.off1 + e) = src.x1[e];
+        for (int q = tid; q < src.k1 >> 2; q += T) xs.quad((src.off1 >> 2) + q) = reinterpret_cast<const float4*>(src.x1)[q];
+        for (int e = (src.k1 & ~3) + tid; e < src.k1; e += T) xs.at(src.off1 + e) = src.x1[e];
     }
     {
         const int gap_end = src.x1 ? src.off1 : 8 * plane, tail = src.x1 ? src.off1 + src.k1 : 8 * plane;
         if constexpr (MODE == SKN_XSRC_GROUP_NORM || MODE == SKN_XSRC_ADD_NORM) __syncthreads();  // (its last quad may have been written past k0)
-        for (int e = src.k0 + tid; e < gap_end; e += kThreads) xs.at(e) = 0.f;
-        for (int e = tail + tid; e < 8 * plane; e += kThreads) xs.at(e) = 0.f;
+        for (int e = src.k0 + tid; e < gap_end; e += T) xs.at(e) = 0.f;
+        for (int e = tail + tid; e < 8 * plane; e += T) xs.at(e) = 0.f;
     }
     __syncthreads();
 
@@ -319,20 +328,30 @@ __global__ __launch_bounds__(kThreads) void dense_matvec_kernel(const W* __restr
 
 constexpr int kMaxLds = 160 * 1024;
 
-template <typename W, int MODE>
-int launch(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, const skn_dense_out& out) {
-    constexpr int V = 16 / (int)sizeof(W);
+constexpr bool stages_norm(int mode) { return mode == SKN_XSRC_GROUP_NORM || mode == SKN_XSRC_ADD_NORM; }
+
+template <typename W, int MODE, int T>
+int launch_threads(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, const skn_dense_out& out, int per_cu) {
+    constexpr int V = 16 / (int)sizeof(W), kWaves = T / 64;
     const int chunk = 64 * kU * V;  // elements of a turn: the planes hold whole turns
     const int plane = (w.k_pad + chunk - 1) / chunk * chunk / 8;
-    const size_t scratch = MODE == SKN_XSRC_GROUP_NORM || MODE == SKN_XSRC_ADD_NORM ? (kMaxGroups + 16 * kWaves) * 4 : MODE == SKN_XSRC_MERGE ? (size_t)src.heads * src.splits * 4 : 0;
+    const size_t scratch = stages_norm(MODE) ? (kMaxGroups + 16 * kWaves) * 4 : MODE == SKN_XSRC_MERGE ? (size_t)src.heads * src.splits * 4 : 0;
     const size_t lds = (size_t)plane * 32 + scratch;
     SKN_REQUIRE(ctx, lds <= kMaxLds, SKN_ERR_SHAPE, "dense matvec: %d columns need %zu bytes of LDS (at most %d)", w.k_pad, lds, kMaxLds);
     // no more workgroups than fit on the device at once: a staging serves all the rows its wavefronts walk through
-    const int groups = (w.rows + kR - 1) / kR, per_cu = std::min(kPerCu, (int)(kMaxLds / lds));
-    const int blocks = std::min((groups + kWaves - 1) / kWaves, per_cu * ctx->compute_units);
-    skn_launch(ctx, dense_matvec_kernel<W, MODE>, dim3((unsigned)blocks), dim3(kThreads), lds, (const W*)w.w, w.rows, w.k_pad, w.ld ? w.ld : w.k_pad, plane, w.bias, src, out);
+    const int groups = (w.rows + kR - 1) / kR;
+    const int blocks = std::min((groups + kWaves - 1) / kWaves, std::min(per_cu, (int)(kMaxLds / lds)) * ctx->compute_units);
+    skn_launch(ctx, dense_matvec_kernel<W, MODE, T>, dim3((unsigned)blocks), dim3(T), lds, (const W*)w.w, w.rows, w.k_pad, w.ld ? w.ld : w.k_pad, plane, w.bias, src, out);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
+}
+
+template <typename W, int MODE>
+int launch(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, const skn_dense_out& out) {
+    const int round = 8 * kR * ctx->compute_units;  // rows that a workgroup of eight wavefronts per compute unit has in hand
+    const bool one_turn = w.k_pad <= 64 * kU * 16 / (int)sizeof(W);
+    if (w.rows <= round || (stages_norm(MODE) && (one_turn || w.rows > 2 * round))) return launch_threads<W, MODE, 512>(ctx, w, src, out, kPerCu);
+    return launch_threads<W, MODE, 1024>(ctx, w, src, out, 1);
 }
 
 template <typename W>
@@ -345,7 +364,8 @@ int launch_mode(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src,
 
 template <typename W, int MODE>
 int allow_lds(skn_ctx* ctx) {
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)dense_matvec_kernel<W, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)dense_matvec_kernel<W, MODE, 512>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)dense_matvec_kernel<W, MODE, 1024>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
     return SKN_OK;
 }
 

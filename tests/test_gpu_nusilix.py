@@ -80,9 +80,30 @@ def test_short_feed_forwards_and_small_heads_have_nothing_beside_the_mixer(hip):
     def taken(heads, dim, ff):
         return step_workgroups(hip, cases.model([cases.delta(heads, dim, ff=ff)], width=512, vocab=40, groups=1))
 
-    assert taken(4, 64, 1280) - taken(4, 64, 1248) == 4 + 64
-    assert taken(4, 64, 1312) - taken(4, 64, 1280) == 4
-    assert taken(4, 64, 2048) - taken(8, 32, 2048) == 64 - 4
+    assert taken(1, 64, 1280) - taken(1, 64, 1248) == 4 + 64
+    assert taken(1, 64, 1312) - taken(1, 64, 1280) == 4
+    assert taken(1, 64, 1312) - taken(2, 32, 1312) == 64 - 1
+
+
+@pytest.mark.parametrize("extra", [-32, 0, 32])
+def test_rows_of_a_product_decide_the_size_of_its_workgroups(hip, extra):
+    """The output product of a step, at, below and above 2048 rows (a workgroup of eight wavefronts per compute unit; sixteen
+    wavefronts above) and the head behind its norm around 4096 (eight again above, and for rows of one turn of requests always),
+    against the oracle; their workgroups counted."""
+    def case(width, vocab):
+        return cases.model([cases.attention(1, 1, 16, ff=70)], width=width, vocab=vocab, groups=1)
+
+    cfg = case(2048 + extra, 4096 + extra)
+    w = cases.weights(cfg, 4, seed=extra + 50)
+    toks = cases.tokens(cfg, 3, seed=2)
+    m = cases.device_model(hip, cfg, w, "bfloat16")
+    cases.check(run(m, toks, [1] * 3), orc.forward(cfg, w, toks), "bfloat16", extra)
+    m.free()
+    if extra:  # (per 32 rows: four workgroups of eight wavefronts or two of sixteen; rows of 2048 and 4096 take 256)
+        base = step_workgroups(hip, case(2048, 32))
+        assert step_workgroups(hip, case(2048 + extra, 32)) - base == (-4 if extra < 0 else 130 - 256 + 1)  # (+ 1: the embedding, a workgroup per 2048 columns)
+        assert step_workgroups(hip, case(2112, 4096 + extra)) - step_workgroups(hip, case(2112, 4096)) == (-2 if extra < 0 else 516 - 256)
+        assert step_workgroups(hip, case(64, 4096 + extra)) - step_workgroups(hip, case(64, 4096)) == extra // 8
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
