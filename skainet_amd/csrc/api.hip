@@ -95,6 +95,7 @@ void skn_shutdown(skn_ctx* ctx) {
     if (ctx->attn_scratch) (void)hipFree(ctx->attn_scratch);
     if (ctx->attn_counters) (void)hipFree(ctx->attn_counters);
     if (ctx->gemm_ws) (void)hipFree(ctx->gemm_ws);
+    if (ctx->gemm_parts) (void)hipFree(ctx->gemm_parts);
     if (ctx->split_scratch) (void)hipFree(ctx->split_scratch);
     if (ctx->prefill_ws) (void)hipFree(ctx->prefill_ws);
     for (hipEvent_t e : ctx->prof_events) (void)hipEventDestroy(e);
@@ -294,6 +295,7 @@ int skn_set_option(skn_ctx* ctx, const char* key, int value) {
     else if (!strcmp(key, "gemm.q6k_fused")) ctx->opt_gemm_q6k_fused = value;
     else if (!strcmp(key, "matvec.stage")) ctx->opt_matvec_stage = value;
     else if (!strcmp(key, "test.rope_table")) ctx->opt_test_rope_table = value;
+    else if (!strcmp(key, "test.gemm_no_parts")) ctx->opt_test_gemm_no_parts = value;
     else if (!strcmp(key, "llama.attn_wide")) ctx->opt_llama_attn_wide = value;
     else return skn_fail(ctx, SKN_ERR_ARG, "skn_set_option: unknown option '%s'", key);
     ctx->opt_generation++;  // whatever was captured with the old settings is stale

@@ -2077,6 +2077,27 @@ int skn_gemm_k_splits(const skn_ctx* ctx, int m, int tiles, int nb) {
     return (nb + each - 1) / each;  // (no workgroup without a superblock)
 }
 
+static bool grow_parts(skn_ctx* ctx, size_t bytes) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;  // (asking for memory would end the capture)
+    }
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (ctx->gemm_parts && (hipStreamSynchronize(ctx->stream) != hipSuccess || hipFree(ctx->gemm_parts) != hipSuccess)) {
+        (void)hipGetLastError();
+        (void)hipFree(p);
+        return false;
+    }
+    ctx->gemm_parts = p;
+    ctx->gemm_parts_bytes = bytes;
+    return true;
+}
+
 int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out) {
     if (bytes > ctx->gemm_ws_bytes) {
         SKN_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -2089,9 +2110,17 @@ int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out) {
             return skn_fail(ctx, SKN_ERR_OOM, "skn_gemm_q: %zu bytes of workspace: %s", bytes, hipGetErrorString(e));
         }
         ctx->gemm_ws_bytes = bytes;
+        // (a workgroup per compute unit and up to 256 x 128 fp32 products of each: 32 MiB)
+        if (!ctx->gemm_parts) (void)grow_parts(ctx, (size_t)ctx->compute_units * 256 * 128 * 4);
     }
     *out = (uint8_t*)ctx->gemm_ws;
     return SKN_OK;
+}
+
+float* skn_gemm_parts_room(skn_ctx* ctx, size_t bytes) {
+    if (ctx->opt_test_gemm_no_parts) return nullptr;
+    if (bytes > ctx->gemm_parts_bytes && !grow_parts(ctx, bytes)) return nullptr;
+    return (float*)ctx->gemm_parts;
 }
 
 // Dynamic LDS above 48 KiB must be allowed per kernel and device; done once per context here so that no launch
@@ -2203,13 +2232,15 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
         fs.part_cols += segs[i].n;
     }
     for (int i = 0; i < 3; i++) fs.part_col0[i] = ps.col0[i];
-    const int splits = tall ? 1 : q4k_splits(ctx, m, mt_rows, m_tiles * fs.n_tiles, k / 256, fs.part_cols);
-    fs.part_blocks = (k / 256 + splits - 1) / splits;
-    const size_t part_bytes = tall ? (size_t)tail.tiles * tail.splits * 131072 : splits > 1 ? (size_t)splits * m * fs.part_cols * 4 : 0;
+    int splits = tall ? 1 : q4k_splits(ctx, m, mt_rows, m_tiles * fs.n_tiles, k / 256, fs.part_cols);
     uint8_t* ws;
-    int rc = skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes + part_bytes, &ws);
+    int rc = skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes, &ws);
     if (rc != SKN_OK) return rc;
-    if (splits > 1) fs.part = (float*)(ws + af_bytes + sf_bytes + is_bytes);
+    const size_t part_bytes = tall ? (size_t)tail.tiles * tail.splits * 131072 : splits > 1 ? (size_t)splits * m * fs.part_cols * 4 : 0;
+    float* part = part_bytes ? skn_gemm_parts_room(ctx, part_bytes) : nullptr;
+    if (!part) splits = 1, tail = TallTail{tall_tiles, 0, 1, nullptr};
+    fs.part_blocks = (k / 256 + splits - 1) / splits;
+    if (splits > 1) fs.part = part;
     _Float16* afrag = (_Float16*)ws;
     _Float16* sfrag = (_Float16*)(ws + af_bytes);
     float* isc = (float*)(ws + af_bytes + sf_bytes);
@@ -2223,7 +2254,7 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     if (tall) {
         for (int i = 0; i < 3; i++) fs.tile0[i] = tall_tile0[i];
         fs.n_tiles = tall_cols;
-        tail.part = (float*)(ws + af_bytes + sf_bytes + is_bytes);
+        tail.part = part;
         skn_launch(ctx, tail.tiles ? gemm_q4k_tall_kernel<true> : gemm_q4k_tall_kernel<false>, dim3(tail.tile0 + tail.tiles * tail.splits), dim3(512), kTlLds, (const u32x4*)afrag, (const u32x4*)sfrag, fs,
                    (const float*)isc, m, k, m_tiles, (uint32_t)((size_t)m_pad * k * 2), tail);
         SKN_LAUNCH_CHECK(ctx);
@@ -2337,11 +2368,12 @@ int skn_gemm_q6k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
         if (splits[i] > 1) part_bytes = std::max(part_bytes, (size_t)splits[i] * m * segs[i].n * 4);
     }
     uint8_t* ws;
-    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes + part_bytes, &ws);
+    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes, &ws);
     if (rc != SKN_OK) return rc;
     _Float16* afrag = (_Float16*)ws;
     float* isc = (float*)(ws + af_bytes);
-    float* part = (float*)(ws + af_bytes + is_bytes);
+    float* part = part_bytes ? skn_gemm_parts_room(ctx, part_bytes) : nullptr;
+    if (!part) splits[0] = splits[1] = splits[2] = 1;
     _Float16* no_sums = nullptr;
     switch (src.kind) {
         case SKN_SRC_BF16: launch_prep<SKN_SRC_BF16, false>(ctx, src, afrag, isc, no_sums, m, m_pad, k); break;

@@ -1,4 +1,6 @@
 """GPU parity: batched quantized GEMM (bf16 activations, fp32 out) through the C ABI vs the fp64-accumulated oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -260,6 +262,72 @@ def test_gemm_q4k_k_is_split_only_where_that_pays(hip, m, n, k, parts):
     got = c.download(np.float32, m * n).reshape(m, n)
     floor = 1e-3 * np.abs(got).max()
     assert np.max(np.abs(got[:, cols] - want) / np.maximum(np.abs(want), floor)) <= TOL
+
+
+@pytest.mark.parametrize("qtype,m,n,k,tile", [(Q4_K, 41, 512, 11008, 0), (Q4_K, 200, 512, 4096, 2), (Q4_K, 300, 384, 4096, 3), (Q6_K, 130, 256, 2816, 0), (synth.Q8_0, 33, 192, 4096, 0), (Q4_K, 7, 192, 4096, 0)])
+def test_gemm_without_room_for_parts_leaves_k_undivided(hip, qtype, m, n, k, tile):
+    """As where the device has no memory left for partial products: the call does what it does with "gemm.split" = 1, bit for bit."""
+    raw = synth.weight(qtype, n, k, seed=n)
+    a = synth.activation_bf16((m, k), seed=m)
+    got = {}
+    hip.set_option("gemm.tile", tile)
+    try:
+        for key, value in (("gemm.split", 1), ("test.gemm_no_parts", 1), ("gemm.split", 0)):
+            hip.set_option(key, value)
+            try:
+                got[key, value] = hip.gemm_q_host(qtype, raw, n, k, a, m).view(np.uint32)
+            finally:
+                hip.set_option(key, 0)
+    finally:
+        hip.set_option("gemm.tile", 0)
+    assert np.array_equal(got["gemm.split", 1], got["test.gemm_no_parts", 1])
+    assert not np.array_equal(got["gemm.split", 1], got["gemm.split", 0]), "the shape's k is not divided: nothing was tested"
+
+
+@pytest.mark.parametrize("qtype,m,n,k", [(Q6_K, 200, 1024, 11008), (Q4_K, 200, 1024, 11008), (synth.Q8_0, 200, 1024, 11008)])
+def test_gemm_that_divides_k_allocates_nothing_behind_one_of_as_many_rows(qtype, m, n, k):
+    """A caller that captures its calls into a graph runs one of the same activations first; products that divide k ask for no memory
+    of their own then.  Every replay against the eager result, with other work between."""
+    raw, a = synth.weight(qtype, n, k, seed=n), synth.activation_bf16((m, k), seed=m)
+    rt = runtime.load_library()  # (the HIP runtime's functions too: the library that the product is launched with)
+
+    def call(name, *args):
+        assert getattr(rt, name)(*args) == 0, name
+
+    stream, graph, replay = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    with runtime.Context(0) as ctx:
+        call("hipStreamCreate", C.byref(stream))
+        ctx.set_stream(stream)
+        w, x, c = ctx.to_device(raw), ctx.to_device(a), ctx.alloc(4 * m * n)
+
+        def result():
+            ctx.sync()
+            return c.download(np.float32, m * n).view(np.uint32)
+
+        ctx.set_option("gemm.split", 1)
+        ctx.gemm_q(qtype, w, n, k, x, m, c)  # (the same workspace, k undivided)
+        ctx.set_option("gemm.split", 0)
+        ctx.sync()
+        call("hipStreamBeginCapture", stream, 1)  # (of this thread's calls)
+        try:
+            ctx.gemm_q(qtype, w, n, k, x, m, c)
+        finally:
+            ended = rt.hipStreamEndCapture(stream, C.byref(graph))
+        assert ended == 0
+        call("hipGraphInstantiate", C.byref(replay), graph, None, None, C.c_size_t(0))
+        ctx.gemm_q(qtype, w, n, k, x, m, c)
+        want = result()
+        for _ in range(3):
+            ctx.memset(c, 0xFF, 4 * m * n)
+            ctx.sync()
+            call("hipGraphLaunch", replay, stream)
+            assert np.array_equal(result(), want)
+            ctx.gemm_q(qtype, w, n, k, x, m, c)
+            assert np.array_equal(result(), want)
+        call("hipGraphExecDestroy", replay)
+        call("hipGraphDestroy", graph)
+        ctx.set_stream(None)
+        call("hipStreamDestroy", stream)
 
 
 @pytest.mark.parametrize("n", [4096, 14336])
