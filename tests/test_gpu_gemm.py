@@ -375,6 +375,78 @@ def test_gemm_2000_rows_take_the_wide_tile_kernels_by_themselves(hip, t):
     assert err <= TOL, err
 
 
+def test_gemm_tiles_past_the_last_whole_round_share_their_k_by_themselves(hip):
+    """450 x 22000 x 2048 by the library's own choice: 344 tiles of 256 x 128, of which 256 fill the device and the last 88 (columns from
+    16384 on) have two workgroups each; a third launch adds them.  Columns of both kinds, the border between them and the last
+    ones, a last row tile of 194 rows."""
+    assert hip.device_info()["compute_units"] == 256, "the shape is chosen for 256 compute units"
+    m, n, k = 450, 22000, 2048
+    raw = synth.weight(Q4_K, n, k, seed=61)
+    a = synth.activation_bf16((m, k), seed=62)
+    w, x, c = hip.to_device(raw), hip.to_device(a), hip.alloc(4 * m * n)
+    hip.memset(c, 0xFF, 4 * m * n)
+    before = hip.stat("launches")
+    hip.gemm_q(Q4_K, w, n, k, x, m, c)
+    assert hip.stat("launches") - before == 3
+    got = c.download(np.float32, m * n).reshape(m, n)
+    assert np.all(np.isfinite(got))
+    cols = np.unique(np.concatenate([np.arange(0, n, 211), np.arange(16352, 16416), np.arange(n - 130, n)]))
+    want = oracle_c.gemm_q(Q4_K, raw.reshape(n, -1)[cols].reshape(-1), len(cols), k, a, m)
+    floor = 1e-3 * np.abs(got).max()
+    assert np.max(np.abs(got[:, cols] - want) / np.maximum(np.abs(want), floor)) <= TOL
+
+
+def _extreme_rows(m, k, seed):
+    """The rows of test_gemm_extreme_rows, then ordinary ones."""
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[0] = 0.0
+    x[1] = 0.0
+    x[1, 1029] = -3.0
+    x[2] *= 1.0e-30
+    x[3] *= np.exp2(rng.integers(-20, 20, size=k)).astype(np.float32)
+    x[4] = -np.abs(x[4])
+    x[5] = np.where(np.arange(k) % 2 == 0, 1.0, -1.0)
+    x[6] *= 6.0e4
+    x[7, : k // 2] = 0.0
+    return synth.f32_to_bf16_bits(x)
+
+
+@pytest.mark.parametrize("m,tile", [(8, 0), (8, 1), (8, 2), (8, 3), (40, 0), (40, 1), (40, 2), (40, 3)])
+def test_gemm_q4k_extreme_rows_on_every_tile(hip, m, tile):
+    """Up to 32 rows the library's own choice is the kernel for blocks of 32: the kernels of 64-, 128- and 256-row tiles, which a
+    decoder's short prompts take too, by option, and beyond 32 rows."""
+    n, k = 96, 2048
+    raw = synth.weight(Q4_K, n, k, seed=21)
+    a = _extreme_rows(m, k, seed=22)
+    hip.set_option("gemm.tile", tile)
+    try:
+        got = hip.gemm_q_host(Q4_K, raw, n, k, a, m)
+    finally:
+        hip.set_option("gemm.tile", 0)
+    want = oracle_c.gemm_q(Q4_K, raw, n, k, a, m)
+    assert np.all(got[0] == 0.0)
+    # (bounds as in test_gemm_extreme_rows: a column of the weights comes back to 1e-6 of its largest)
+    col = -3.0 * oracle_c.dequant(Q4_K, raw).reshape(n, k)[:, 1029]
+    assert np.abs(got[1] - col).max() <= 1e-6 * np.abs(col).max(), np.abs(got[1] - col).max() / np.abs(col).max()
+    for r in range(2, m):
+        assert oracle_np.rel_err(got[r], want[r]) <= TOL, r
+
+
+@pytest.mark.parametrize("k,fused", [(6464, 1), (6400, 0)])
+def test_gemm_general_path_of_several_128_row_tiles(hip, k, fused):
+    """260 rows on the general path: rows that are no whole groups of 256 elements, or by option."""
+    m, n = 260, 96
+    raw = synth.weight(Q8_0, n, k, seed=n + k)
+    a = synth.activation_bf16((m, k), seed=m + k)
+    hip.set_option("gemm.q6k_fused", fused)
+    try:
+        got = hip.gemm_q_host(Q8_0, raw, n, k, a, m)
+    finally:
+        hip.set_option("gemm.q6k_fused", 1)
+    assert oracle_np.rel_err(got, oracle_c.gemm_q(Q8_0, raw, n, k, a, m)) <= TOL
+
+
 def test_gemm_full_width_slice(hip):
     """The benchmark shape M=512, K=4096 at N=4096: checked on a strided sample of the oracle's columns."""
     m, n, k = 512, 4096, 4096

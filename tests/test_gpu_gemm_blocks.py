@@ -15,7 +15,7 @@ TOL = 1e-3
 @pytest.mark.parametrize("name", list(FORMATS))
 @pytest.mark.parametrize("m,n,k", [(1, 1, 256), (32, 64, 256), (33, 65, 512), (64, 63, 1280), (65, 100, 768), (128, 130, 2816), (129, 64, 1024), (3, 600, 16384)])
 def test_every_tile_height_and_remainder(hip, name, m, n, k):
-    """One row and column to ragged tiles of 32, 64 and 128 rows; fewer superblocks than a workgroup has k-parts, unequal
+    """One row and column to ragged tiles of 32 and 64 rows; fewer superblocks than a workgroup has k-parts, unequal
     parts, and the longest row the path takes; with k divided over workgroups as the library chooses, not at all, in unequal
     parts and superblock by superblock."""
     t = FORMATS[name]
@@ -67,3 +67,53 @@ def test_weights_off_the_16_byte_grid_take_the_general_path(hip):
     hip.gemm_q(synth.Q8_0, buf.ptr + 2, n, k, hip.to_device(a), m, c)
     got = c.download(np.float32, m * n).reshape(m, n)
     assert oracle_np.rel_err(got, oracle_c.gemm_q(synth.Q8_0, raw, n, k, a, m)) <= TOL
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 256), (32, 64, 256), (32, 65, 512), (17, 63, 1280), (31, 130, 2816), (3, 600, 16384)])
+def test_q4_k_of_up_to_32_rows(hip, m, n, k):
+    """Few rows of Q4_K take the same kernel: divisions of k as above, no row or column of a tile left over or missing."""
+    raw = synth.weight(synth.Q4_K, n, k, seed=n + k)
+    a = synth.activation_bf16((m, k), seed=m + 1)
+    want = oracle_c.gemm_q(synth.Q4_K, raw, n, k, a, m)
+    for splits in (0, 1, 3, 64):
+        hip.set_option("gemm.split", splits)
+        try:
+            got = hip.gemm_q_host(synth.Q4_K, raw, n, k, a, m)
+        finally:
+            hip.set_option("gemm.split", 0)
+        err = oracle_np.rel_err(got, want)
+        assert err <= TOL, f"{splits} parts: rel err {err}"
+
+
+@pytest.mark.parametrize("name,t", [("q4_k", synth.Q4_K), ("q5_k", synth.Q5_K)])
+def test_superblock_scales_far_apart(hip, name, t):
+    """d and dmin zero, negative, subnormal, from 2^-20 to 2^20 of each other and of the next superblock's, up to 32 rows (rows of
+    1e6, of 1e-6 and of zeros among them): each block's sum joins the total in fp32 with its own scale."""
+    m, n, k = 20, 64, 4096
+    nb = k // 256
+    rng = np.random.default_rng(92)
+    raw = synth.weight(t, n, k, seed=91).reshape(n, nb, -1).copy()
+    cases = [(0.0, 0.01), (0.0, 0.0), (-0.02, 0.01), (0.02, -0.01), (0.01, 0.0), (6e-8, 1e-7), (1e-5, 10.0), (1e-6, 1.0), (10.0, 1e-5), (500.0, 0.5),
+             (3e-5, 0.03), (0.03, 3e-5), (-1e-4, -20.0), (2e-7, 0.2)]
+    for col in range(n):
+        for sb in range(nb):
+            d = np.array(cases[rng.integers(len(cases))] if col < 48 else cases[(col + sb) % len(cases)], dtype=np.float16)
+            raw[col, sb, 0:4] = d.view(np.uint8)
+    raw[49, :, 0:2] = 0  # a column with no live superblock but its minima
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[0] *= 1e6
+    x[1] *= 1e-6
+    x[2] = 0.0
+    a = synth.f32_to_bf16_bits(x)
+    got = hip.gemm_q_host(t, raw.reshape(-1), n, k, a, m)
+    want = oracle_c.gemm_q(t, raw.reshape(-1), n, k, a, m)
+    assert np.all(np.isfinite(got)) and not np.any(got[2])
+    for r in (0, 1):
+        for col in range(n):
+            # a product of fp32 sums of exact terms: 2^-24 per addition of a chain of 2 * 128 of them and of the minima's sixteen, relative to
+            # the sum of the terms' magnitudes
+            w = oracle_c.dequant(t, raw[col].reshape(-1)).astype(np.float64)
+            size = np.sum(np.abs(w) * np.abs(oracle_np.bf16_to_f32(a).reshape(m, k)[r]))
+            assert abs(got[r, col] - want[r, col]) <= 300 * 2.0**-24 * size + 1e-30, (r, col)
+    for col in range(n):
+        assert oracle_np.rel_err(got[3:, col], want[3:, col]) <= TOL, col

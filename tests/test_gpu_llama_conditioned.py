@@ -179,6 +179,54 @@ def test_q6k_beside_another_format_in_one_launch(hip, other, six, hidden, n_kv):
     model.free()
 
 
+@pytest.mark.parametrize("hidden,other,six", [(2304, 12, ("wv",)), (2304, 13, ("wk", "wv")), (2304, 8, ("wq",)), (4096, 12, ("wv",)), (4352, 12, ("wq",)),
+                                              (4352, 13, ("wv",)), (4352, 8, ("wk", "wv")), (8448, 12, ("wv",)), (12544, 12, ("wk", "wv"))])
+def test_q6k_beside_another_format_in_rows_of_one_to_four_steps(hip, hidden, other, six):
+    """The same for rows beyond half a step, which every lane of a wavefront reads (2304 columns to 4096), and of two, three and four
+    steps, the last of them nearly empty."""
+    cfg = llama.Config(n_layer=1, hidden=hidden, ffn=256, n_head=hidden // 128, n_kv_head=2, head_dim=128, vocab=256, max_tokens=16, page_tokens=16,
+                       matrix_types={w: 14 if w in six else other for w in ("wq", "wk", "wv")})
+    w = llama.conditioned_weights(cfg, SEED)
+    ora, model = OracleLlama(cfg, w), llama.LlamaModel(hip, cfg, weights=w)
+    hip.set_option("llama.graph", 0)
+    try:
+        for i, t in enumerate(tokens(4, cfg.vocab)):
+            ora.step(t)
+            before = hip.stat("launches")
+            model.decode(t, 1)
+            assert hip.stat("launches") - before == 2 + 5 + 3, "q, k and v took more than one launch"
+            err = logit_err(model.logits(), ora.logits)
+            assert err <= DECODE_TOL, (hidden, other, six, i, err)
+    finally:
+        hip.set_option("llama.graph", 1)
+    model.free()
+
+
+def test_prompt_whose_grids_end_in_shared_tiles(hip):
+    """800 tokens of width 4096: q, k and v are 384 tiles of 256 x 128 and the gate / up pair 352, so the tiles past the first 256 share
+    their k -- those of the values among them, behind the border between two matrices -- and a launch more adds each.  Against the
+    same prompt on 128-row tiles, whose kernel is another and divides nothing."""
+    assert hip.device_info()["compute_units"] == 256, "the shape is chosen for 256 compute units"
+    cfg = llama.Config(n_layer=1, hidden=4096, ffn=5632, n_head=32, head_dim=128, vocab=256, max_tokens=832, page_tokens=64)
+    model = llama.LlamaModel(hip, cfg, weights=llama.conditioned_weights(cfg, SEED))
+    prompt, got, launches = tokens(800, cfg.vocab, seed=2), [], []
+    for options in ({}, {"gemm.split": 1}, {"gemm.split": 1, "gemm.tile": 2}):
+        for key, value in options.items():
+            hip.set_option(key, value)
+        try:
+            model.reset()
+            before = hip.stat("launches")
+            model.prefill(prompt)
+            launches.append(hip.stat("launches") - before)
+            got.append(model.logits())
+        finally:
+            for key in options:
+                hip.set_option(key, 0)
+    assert launches[0] == launches[1] + 2 == launches[2] + 2
+    assert logit_err(got[0], got[2]) <= PROMPT_TOL and logit_err(got[1], got[2]) <= PROMPT_TOL
+    model.free()
+
+
 @pytest.mark.parametrize("head_dim,context", [(64, 500), (128, 250), (256, 120)])
 def test_contexts_of_one_round_take_one_workgroup_per_head(hip, head_dim, context):
     """Decode steps up to, at and past the tokens that a workgroup takes in one round (512, 256, 128): one workgroup per head with
