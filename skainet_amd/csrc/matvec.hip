@@ -2018,6 +2018,17 @@ bool skn_matvec_fusable(int ggml_type) {
            ggml_type == SKN_TYPE_TQ1_0 || ggml_type == SKN_TYPE_TQ2_0;
 }
 
+// what the rotary epilogue asks of its arguments (a launch may carry a subset of q, k, v: an absent matrix has no rows)
+static int check_rope(skn_ctx* ctx, const skn_rope_epilogue* rope, const skn_q4k_segments& seg) {
+    SKN_REQUIRE(ctx, rope && rope->pos_dev && rope->page_table && rope->k_pool && rope->v_pool, SKN_ERR_ARG,
+                "fused matvec: the rotary epilogue needs its cache arguments");
+    SKN_REQUIRE(ctx, rope->head_dim > 0 && rope->head_dim % 2 == 0 && seg.rows[0] % rope->head_dim == 0 &&
+                         (seg.rows[1] == 0 || seg.rows[1] == rope->n_head * rope->head_dim) &&
+                         (seg.rows[2] == 0 || seg.rows[2] == rope->n_head * rope->head_dim),
+                SKN_ERR_SHAPE, "fused matvec: q/k/v rows do not match %d heads of %d", rope->n_head, rope->head_dim);
+    return SKN_OK;
+}
+
 // Fused matvec for the decoder, all matrices of one of the formats above; k <= 16384 (four unrolled steps).
 // Returns SKN_ERR_SHAPE otherwise.
 int skn_matvec_q4k_fused(skn_ctx* ctx, const skn_q4k_segments& seg, int n_out, int k, const float* x, const float* norm_w,
@@ -2045,15 +2056,8 @@ int skn_matvec_q4k_fused(skn_ctx* ctx, const skn_q4k_segments& seg, int n_out, i
         rope.merge_head_f4 = rope_in->merge_head_f4;
     }
     if (epi == SKN_EPI_ROPE) {
-        SKN_REQUIRE(ctx, rope_in && rope_in->pos_dev && rope_in->page_table && rope_in->k_pool && rope_in->v_pool,
-                    SKN_ERR_ARG, "fused Q4_K matvec: the rotary epilogue needs its cache arguments");
+        SKN_TRY(check_rope(ctx, rope_in, seg));
         rope = *rope_in;
-        // (a launch may carry a subset of q, k, v: an absent matrix has no rows)
-        SKN_REQUIRE(ctx, rope.head_dim > 0 && rope.head_dim % 2 == 0 && seg.rows[0] % rope.head_dim == 0 &&
-                             (seg.rows[1] == 0 || seg.rows[1] == rope.n_head * rope.head_dim) &&
-                             (seg.rows[2] == 0 || seg.rows[2] == rope.n_head * rope.head_dim),
-                    SKN_ERR_SHAPE, "fused Q4_K matvec: q/k/v rows do not match %d heads of %d", rope.n_head,
-                    rope.head_dim);
     }
     const int nb = k / 256;
 #define SKN_FUSED(F)                                                                                      \
@@ -2089,6 +2093,8 @@ int skn_matvec_fused_two(skn_ctx* ctx, const skn_q4k_segments& q6, int n_q6, con
                          const float* x, const float* norm_w, float eps, float* y, const skn_rope_epilogue& rope) {
     if (other_type != SKN_TYPE_Q4_K && other_type != SKN_TYPE_Q5_K && other_type != SKN_TYPE_Q8_0) return SKN_ERR_TYPE;
     SKN_REQUIRE(ctx, k > 0 && k % 256 == 0 && k <= 16384 && n_q6 > 0 && n_other > 0, SKN_ERR_SHAPE, "fused matvec of two formats: unsupported shape");
+    SKN_TRY(check_rope(ctx, &rope, q6));
+    SKN_TRY(check_rope(ctx, &rope, other));
     const uintptr_t mask = other_type == SKN_TYPE_Q8_0 ? 3 : 15;
     for (int i = 0; i < 3; i++)
         SKN_REQUIRE(ctx, (q6.rows[i] == 0 || (q6.w[i] && ((uintptr_t)q6.w[i] & 1) == 0)) && (other.rows[i] == 0 || (other.w[i] && ((uintptr_t)other.w[i] & mask) == 0)),
