@@ -417,7 +417,7 @@ int skn_shared_attn_step(skn_ctx* ctx, skn_kv* kv, int seq, const skn_shared_att
     a.out_type = SKN_TYPE_F32;
     if (!beside) return launch_attn<true>(ctx, kv, a, 1);
     skn_beside s = *beside;
-    skn_beside_plan(ctx, s, kThreads);
+    skn_beside_plan(ctx, s, kThreads, skn_shared_attn_step_lds(kv));
     return launch_attn<true>(ctx, kv, a, 1, s);
 }
 

@@ -443,7 +443,7 @@ int launch_step(skn_ctx* ctx, const skn_rstate* st, const skn_delta_step& p, flo
         if (beside) {
             SKN_REQUIRE(ctx, beside->type == p.w2_type, SKN_ERR_TYPE, "delta rule: a product of another type beside a step");
             skn_beside s = *beside;
-            skn_beside_plan(ctx, s, 64 * NW);
+            skn_beside_plan(ctx, s, 64 * NW, (6 * 8 * L + NW) * sizeof(float));
             const dim3 grid((unsigned)(st->heads + s.blocks));
             const int plane = skn_beside_plane(s);
             const size_t lds = skn_beside_lds(s);

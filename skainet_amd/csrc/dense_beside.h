@@ -26,8 +26,12 @@ static inline int skn_beside_plane(const skn_beside& s) {  // float4s of either 
     return (s.k_pad + chunk - 1) / chunk * chunk / 8;
 }
 static inline size_t skn_beside_lds(const skn_beside& s) { return (size_t)skn_beside_plane(s) * 32; }
-static inline void skn_beside_plan(const skn_ctx* ctx, skn_beside& s, int threads) {
-    const int waves = threads / 64, most = 1536 / threads > 0 ? 1536 / threads * ctx->compute_units : ctx->compute_units;
+// own_lds: of the launch's own kernel.  No more workgroups than fit on the device at once: a staging serves all the rows that its
+// wavefronts walk through.  (Delta heads of 64, feed-forwards of 14000 columns, of which two stagings fit a compute unit: three planned
+// workgroups against two, two layers of width 5120, 32 steps 6.26 | 6.16 ms; width 4608 6.26 | 6.14; width 6144 6.90 | 6.89.)
+static inline void skn_beside_plan(const skn_ctx* ctx, skn_beside& s, int threads, size_t own_lds) {
+    const int waves = threads / 64, fit = (int)(160 * 1024 / (skn_beside_lds(s) + own_lds)), by_threads = 1536 / threads;
+    const int per_cu = by_threads < fit ? by_threads : fit, most = (per_cu > 0 ? per_cu : 1) * ctx->compute_units;
     const int want = (s.rows + waves - 1) / waves;
     s.blocks = want < most ? want : most;
 }

@@ -59,9 +59,9 @@ def test_feed_forward_beside_the_mixer_of_a_step(hip, width, ff, dtype):
     m.free()
 
 
-def step_workgroups(hip, cfg, seed=3):
+def step_workgroups(hip, cfg, seed=3, weights=None):
     """What one decode step launches, eagerly."""
-    m = cases.device_model(hip, cfg, cases.weights(cfg, 4, seed=seed), "bfloat16")
+    m = cases.device_model(hip, cfg, cases.weights(cfg, 4, seed=seed) if weights is None else weights, "bfloat16")
     m.prefill(cases.tokens(cfg, 3))
     hip.set_option("llama.graph", 0)
     try:
@@ -83,6 +83,21 @@ def test_short_feed_forwards_and_small_heads_have_nothing_beside_the_mixer(hip):
     assert taken(1, 64, 1280) - taken(1, 64, 1248) == 4 + 64
     assert taken(1, 64, 1312) - taken(1, 64, 1280) == 4
     assert taken(1, 64, 1312) - taken(2, 32, 1312) == 64 - 1
+
+
+def test_product_beside_the_mixer_has_no_more_workgroups_than_fit(hip):
+    """Rows of 4224: a workgroup of eight wavefronts per eight of them beside the mixer, up to three per compute unit, which is all of
+    them while three stagings of the feed-forward fit its LDS (12288 columns) and two per compute unit from there on.  (Zeros for
+    weights: the workgroups are counted.)"""
+    assert hip.device_info()["compute_units"] == 256, "the width is chosen for 256 compute units"
+
+    def taken(ff):
+        cfg = cases.model([cases.delta(1, 64, ff=ff)], width=4224, vocab=40, groups=1)
+        shapes = nusilix.tensor_shapes(nusilix.config_from_json(cfg), 4)
+        return step_workgroups(hip, cfg, weights={name: np.zeros(shape, dtype=np.float32) for name, shape in shapes.items()})
+
+    # (the input product fills the device, three workgroups per compute unit, either way)
+    assert taken(12320) - taken(12288) == 512 - 528
 
 
 @pytest.mark.parametrize("extra", [-32, 0, 32])
