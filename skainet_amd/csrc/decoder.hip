@@ -613,7 +613,8 @@ int project_rows(skn_ctx* ctx, skn_llama* m, const int* types, const void* const
 
 // The same with the option llama.expand_weights: Q4_K matrices on their own kernel, the others through their kept copies
 // (`which`: the first matrix's place among a layer's seven), except that up to 256 rows the formats in blocks of 32 are faster from
-// their blocks (us per call, Q8_0, blocks | copy: 120 x 4096 x 4096 21.7 | 32, 333 x 4096 x 4096 38.7 | 34).
+// their blocks (us of a call's kernels, Q8_0, blocks | copy: 120 x 4096 x 4096 22.6 | 33.0, 333 x 4096 x 4096 39.0 | 36.5).  The copies
+// are made all the same: the option has the first prompt make them, whatever its length.
 static int project_expanded(skn_ctx* ctx, skn_llama* m, int l, int which, const int* types, const void* const* blocks, const int* rows, float* const* outs,
                             int count, int k, const float* x, const float* norm_w, int T, int accumulate) {
     const skn_gemm_src src = {norm_w ? SKN_SRC_RMSNORM : SKN_SRC_F32, x, norm_w, norm_w ? m->cfg.rms_eps : 0.f};

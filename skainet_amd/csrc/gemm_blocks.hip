@@ -1,5 +1,6 @@
-// Prompt GEMM for formats whose weights are d (q - zero) + m over blocks of 32 elements: Q8_0, Q4_0, Q4_1, Q5_0, Q5_1 and the
-// sub-blocks of Q5_K.  C[m, n] = sum_k A[m, k] w[n, k], activations as in gemm.hip (bf16 rows scaled to fp16 by a power of two).
+// Prompt GEMM for formats whose weights are d (q - zero) + m over blocks of 32 elements: Q8_0, Q4_0, Q4_1, Q5_0, Q5_1, the
+// sub-blocks of Q5_K, and those of Q4_K for up to 32 rows (above, Q4_K has kernels of its own in gemm.hip).
+// C[m, n] = sum_k A[m, k] w[n, k], activations as in gemm.hip (bf16 rows scaled to fp16 by a power of two).
 //
 // Bound by the matrix cores and the vector ALUs together for many rows, by the weight stream for few.  What the general path
 // does with these formats -- rewrite the weights as fp16 pairs (4 bytes per weight written and read again), then two matrix
@@ -9,13 +10,12 @@
 // rounded before those sums.  Minima: sum over a superblock of m_j times the sum of the activations of block j, one more matrix
 // instruction on the sums that the preparation pass leaves (fp16 pairs).
 //
-// Workgroup of four wavefronts, one per SIMD, tile (32 MT) x 64, k by superblock (256 elements) over the wavefronts and, where
-// the tiles do not fill the device, over workgroups too (gemm_tiles.h); the four partial tiles are added through LDS.  A wavefront
-// brings its superblock of 64 rows in with coalesced 16-byte loads one superblock ahead (registers, then LDS of its own: no
-// barrier in the loop) and reads the activations in fragment order, eight
-// (tiles of 128 rows: four) k-steps ahead.
+// Workgroup of four wavefronts, one per SIMD, tile (32 MT) x 64 (MT = 1 up to 32 rows, 2 above), k by superblock (256 elements)
+// over the wavefronts and, where the tiles do not fill the device, over workgroups too (gemm_tiles.h); the four partial tiles are
+// added through LDS.  A wavefront brings its superblock of 64 rows in with coalesced 16-byte loads one superblock ahead
+// (registers, then LDS of its own: no barrier in the loop) and reads the activations in fragment order, four k-steps ahead.
 //
-// us per call, before -> now (weights as fp16 pairs -> this): Q8_0 333 x 4096 x 4096 52.9 -> 38.7, 512 x 14336 x 4096 236 -> 121, 41 x 4096 x
+// us per call, before -> now (weights as fp16 pairs -> this): Q8_0 333 x 4096 x 4096 51.6 -> 36.4, 512 x 14336 x 4096 236 -> 121, 41 x 4096 x
 // 11008 102 -> 28.5; Q5_K 512 x 4096 x 4096 60 -> 40.4; Q4_0 5 x 4096 x 4096 36.6 -> 11.5.
 #include "gemm_blocks.h"
 #include "gemm_tiles.h"
