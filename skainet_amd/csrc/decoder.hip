@@ -585,7 +585,7 @@ int project_rows(skn_ctx* ctx, skn_llama* m, const int* types, const void* const
         const skn_gemm_seg seg = {blocks[i], rows[i], outs[i], accumulate};
         if (types[i] == SKN_TYPE_Q4_K && k <= 16384) q4[n4++] = seg;
         else if (types[i] == SKN_TYPE_Q6_K && skn_gemm_q6k_direct_ok(ctx, rows[i], k, T)) q6[n6++] = seg;
-        else if (skn_gemm_blocks_ok(ctx, types[i], blocks[i], rows[i], k, T)) bl_types[nbl] = types[i], bl[nbl++] = seg;
+        else if (skn_gemm_blocks_ok(ctx, types[i], blocks[i], rows[i], k, T) && skn_gemm_blocks_pay(types[i], rows[i], k, T, true)) bl_types[nbl] = types[i], bl[nbl++] = seg;
         else plain[np++] = i;
     }
     if (n4) SKN_TRY(skn_gemm_q4k_multi(ctx, q4, n4, k, src, T));

@@ -2306,7 +2306,7 @@ extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n,
         return skn_gemm_q6k_multi(ctx, &seg, 1, k, src, m);
     }
     // formats in blocks of 32: likewise
-    if (skn_gemm_blocks_ok(ctx, ggml_type, w_dev, n, k, m)) {
+    if (skn_gemm_blocks_ok(ctx, ggml_type, w_dev, n, k, m) && skn_gemm_blocks_pay(ggml_type, n, k, m, false)) {
         const skn_gemm_seg seg = {w_dev, n, c_dev, 0};
         return skn_gemm_blocks_multi(ctx, &ggml_type, &seg, 1, k, src, m);
     }

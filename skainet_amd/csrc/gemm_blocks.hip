@@ -561,6 +561,19 @@ bool skn_gemm_blocks_ok(const skn_ctx* ctx, int type, const void* w, int n, int 
            m_pad * k * 2 < ((size_t)1 << 31) && (size_t)n * (k / 256) * bytes < ((size_t)1 << 31);
 }
 
+// Unpacking a block once per 64 rows against once per call: what costs the most vector instructions, a fifth bit or minima, loses first.
+// Time of the general path over this one's, 600 to 14336 columns, k from 2048 to 11008:
+//   Q5_1  1280 rows 0.93 - 1.14, 1536 0.80 - 1.09, 2048 0.75 - 0.96, 4096 0.87 - 0.97; two layers' prompts of width 4096 1500 tokens 1.01,
+//         1800 0.99, 2048 0.92 (5019 | 4616 us), 3000 0.98, of width 2048 above 1.04 up to 3000
+//   Q4_1  1792 rows 0.95 - 1.14; 1920 to 3072 rows of 2560 to 8192 columns with k from 4096 on 0.87 - 1.06, 0.94 in the mean (2048 x 4096 x
+//         6144 267 | 232 us), other sizes 0.94 - 1.12; 4096 rows 0.98 - 1.13; prompts above 1.03 throughout
+//   Q8_0, Q4_0, Q5_0, Q5_K  0.91 - 1.6, above one in the mean at every number of rows; prompts above 1.1
+bool skn_gemm_blocks_pay(int type, int n, int k, int m, bool in_prompt) {
+    if (type == SKN_TYPE_Q5_1) return in_prompt ? m <= 1800 || k < 4096 : m <= 1400;
+    if (type == SKN_TYPE_Q4_1) return in_prompt || m <= 1850 || m > 3300 || k < 4096 || n < 2560 || n > 8192;
+    return true;
+}
+
 int skn_gemm_blocks_multi(skn_ctx* ctx, const int* types, const skn_gemm_seg* segs, int nseg, int k, const skn_gemm_src& src, int m) {
     SKN_REQUIRE(ctx, nseg >= 1 && nseg <= 3 && m > 0, SKN_ERR_ARG, "block GEMM: bad segment count or shape");
     SKN_REQUIRE(ctx, src.a && ((uintptr_t)src.a & (src.kind == SKN_SRC_BF16 ? 7 : 15)) == 0, SKN_ERR_ARG, "block GEMM: activations are null or misaligned");

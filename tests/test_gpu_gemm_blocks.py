@@ -117,3 +117,50 @@ def test_superblock_scales_far_apart(hip, name, t):
             assert abs(got[r, col] - want[r, col]) <= 300 * 2.0**-24 * size + 1e-30, (r, col)
     for col in range(n):
         assert oracle_np.rel_err(got[3:, col], want[3:, col]) <= TOL, col
+
+
+@pytest.mark.parametrize("name,m,n,k,direct", [("q5_1", 1400, 70, 512, True), ("q5_1", 1401, 70, 512, False), ("q4_1", 1850, 2560, 4096, True),
+                                               ("q4_1", 1851, 2560, 4096, False), ("q4_1", 1851, 2559, 4096, True), ("q4_1", 1851, 2560, 3840, True),
+                                               ("q4_1", 3300, 2560, 4096, False), ("q4_1", 3301, 2560, 4096, True), ("q5_0", 2000, 2560, 4096, True)])
+def test_many_rows_of_the_formats_that_unpack_slowest_take_the_weight_pass(hip, name, m, n, k, direct):
+    """Preparation and product where the kernel unpacks the blocks itself, a pass over the weights more where many rows share it; either
+    against the oracle, first and last rows, sampled columns."""
+    t = FORMATS[name]
+    raw, a = synth.weight(t, n, k, seed=n), synth.activation_bf16((m, k), seed=m)
+    w, x, c = hip.to_device(raw), hip.to_device(a), hip.alloc(4 * m * n)
+    hip.memset(c, 0xFF, 4 * m * n)
+    before = hip.stat("launches")
+    hip.gemm_q(t, w, n, k, x, m, c)
+    assert hip.stat("launches") - before == (2 if direct else 3)
+    got = c.download(np.float32, m * n).reshape(m, n)
+    assert np.all(np.isfinite(got))
+    cols = np.unique(np.concatenate([np.arange(0, n, 97), [n - 1]]))
+    rows = np.concatenate([np.arange(8), np.arange(m - 70, m)])
+    want = oracle_c.gemm_q(t, raw.reshape(n, -1)[cols].reshape(-1), len(cols), k, a.reshape(m, k)[rows], len(rows))
+    assert oracle_np.rel_err(got[np.ix_(rows, cols)], want) <= TOL
+
+
+def test_long_prompt_of_a_format_that_unpacks_slowest(hip):
+    """A prompt keeps the direct products of Q5_1 up to 1800 rows and for short rows; the others' results agree with them to the rounding
+    of the activations that a prompt's passes do one by one."""
+    from skainet_amd import llama
+
+    cfg = llama.Config(n_layer=1, hidden=512, ffn=4096, n_head=4, head_dim=128, vocab=256, max_tokens=1824, page_tokens=32, type_embd=synth.Q6_K,
+                       matrix_types={w: synth.Q5_1 for w in ("wq", "wk", "wv", "wo", "w_gate", "w_up", "w_down")})
+    model = llama.LlamaModel(hip, cfg, weights=llama.random_weights(cfg, seed=11))
+    ids = np.random.default_rng(3).integers(0, cfg.vocab, 1801).tolist()
+    took, logits = [], []
+    for tokens, fused in ((1800, 1), (1801, 1), (1801, 0)):
+        hip.set_option("gemm.q6k_fused", fused)
+        try:
+            model.reset()
+            before = hip.stat("launches")
+            model.prefill(ids[:tokens])
+            took.append(hip.stat("launches") - before)
+            logits.append(model.logits())
+        finally:
+            hip.set_option("gemm.q6k_fused", 1)
+    # the down projection alone has rows of 4096: a conversion, three launches and an addition instead of a preparation and a product
+    assert took[1] - took[0] == 3
+    assert np.abs(logits[1] - logits[2]).max() <= 5e-3 * np.abs(logits[2]).max()
+    model.free()
