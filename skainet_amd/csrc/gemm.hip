@@ -2343,6 +2343,19 @@ bool skn_gemm_q6k_direct_ok(const skn_ctx* ctx, int n, int k, int m) {
            (size_t)n * (k / 256) * 210 < ((size_t)1 << 31);
 }
 
+// How many workgroups share the k of a tile of `rows` rows.  The column tiles go round the eight XCDs and their row tiles with them
+// (launch_q6k_gemm), so the fullest XCD decides: parts that need a second round of its compute units are walked one behind the other.
+// us per call, undivided | in two parts: 380 x 2688 x 4096 (eighteen tiles on an XCD of 32 units) 55.0 | 60.6, 600 x 1600 x 11008 (twenty) 139 | 151,
+// 1300 x 700 x 11008 (22) 148 | 161, against 380 x 2560 x 8192 (fifteen) 92.6 | 60.3 and 1300 x 512 x 11008 (eleven) 150 | 97; three parts
+// in two rounds gain: 1800 x 300 x 11008 154 | 127.
+static int q6k_splits(const skn_ctx* ctx, int m, int n, int rows, int nb) {
+    const int m_tiles = (m + rows - 1) / rows, n_tiles = (n + kBN - 1) / kBN, splits = skn_gemm_k_splits(ctx, m, m_tiles * n_tiles, nb);
+    if (splits < 2 || ctx->opt_gemm_split > 0) return splits;
+    const int on_xcd = 8 % m_tiles == 0 ? (n_tiles * m_tiles + 7) / 8 : (n_tiles + 7) / 8 * m_tiles, units = std::max(1, ctx->compute_units / 8);
+    const int each = (nb + splits - 1) / splits;
+    return (on_xcd * splits + units - 1) / units * each < (on_xcd + units - 1) / units * nb ? splits : 1;
+}
+
 int skn_gemm_q6k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, const skn_gemm_src& src, int m) {
     SKN_REQUIRE(ctx, nseg >= 1 && nseg <= 3 && m > 0, SKN_ERR_ARG, "Q6_K GEMM: bad segment count or shape");
     SKN_REQUIRE(ctx, src.a && ((uintptr_t)src.a & (src.kind == SKN_SRC_BF16 ? 7 : 15)) == 0, SKN_ERR_ARG,
@@ -2364,7 +2377,7 @@ int skn_gemm_q6k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     size_t part_bytes = 0;  // (the matrices' products run one after the other: they share the room for their parts)
     for (int i = 0; i < nseg; i++) {
         if (q6k_wide_tiles(ctx, segs[i].n, k, m)) continue;
-        splits[i] = skn_gemm_k_splits(ctx, m, ((m + 32 * mt - 1) / (32 * mt)) * ((segs[i].n + kBN - 1) / kBN), k / 256);
+        splits[i] = q6k_splits(ctx, m, segs[i].n, 32 * mt, k / 256);
         if (splits[i] > 1) part_bytes = std::max(part_bytes, (size_t)splits[i] * m * segs[i].n * 4);
     }
     uint8_t* ws;

@@ -264,6 +264,25 @@ def test_gemm_q4k_k_is_split_only_where_that_pays(hip, m, n, k, parts):
     assert np.max(np.abs(got[:, cols] - want) / np.maximum(np.abs(want), floor)) <= TOL
 
 
+@pytest.mark.parametrize("m,n,k,parts", [(380, 2688, 2048, False), (380, 2560, 2048, True), (1300, 700, 2048, False), (1300, 512, 2048, True),
+                                         (1800, 300, 4096, True), (128, 8192, 2048, True), (41, 4096, 4096, True)])
+def test_gemm_q6k_k_is_split_where_an_xcd_has_room_for_the_parts(hip, m, n, k, parts):
+    """The tiles of a column tile are on one XCD: two parts of more than sixteen of them would be walked one behind the other.  Activation
+    pass and product; a third launch adds parts.  First and last rows, sampled columns."""
+    assert hip.device_info()["compute_units"] == 256, "the shapes are chosen for 256 compute units"
+    raw, a = synth.weight(Q6_K, n, k, seed=m + n), synth.activation_bf16((m, k), seed=k)
+    w, x, c = hip.to_device(raw), hip.to_device(a), hip.alloc(4 * m * n)
+    hip.memset(c, 0xFF, 4 * m * n)
+    before = hip.stat("launches")
+    hip.gemm_q(Q6_K, w, n, k, x, m, c)
+    assert hip.stat("launches") - before == (3 if parts else 2)
+    got = c.download(np.float32, m * n).reshape(m, n)
+    assert np.all(np.isfinite(got))
+    cols, rows = np.arange(0, n, 61), np.concatenate([np.arange(8), np.arange(m - 30, m)])
+    want = oracle_c.gemm_q(Q6_K, raw.reshape(n, -1)[cols].reshape(-1), len(cols), k, a.reshape(m, k)[rows], len(rows))
+    assert oracle_np.rel_err(got[np.ix_(rows, cols)], want) <= TOL
+
+
 @pytest.mark.parametrize("qtype,m,n,k,tile", [(Q4_K, 41, 512, 11008, 0), (Q4_K, 200, 512, 4096, 2), (Q4_K, 300, 384, 4096, 3), (Q6_K, 130, 256, 2816, 0), (synth.Q8_0, 33, 192, 4096, 0), (Q4_K, 7, 192, 4096, 0)])
 def test_gemm_without_room_for_parts_leaves_k_undivided(hip, qtype, m, n, k, tile):
     """As where the device has no memory left for partial products: the call does what it does with "gemm.split" = 1, bit for bit."""
