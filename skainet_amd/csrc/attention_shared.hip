@@ -326,7 +326,7 @@ template <int D, bool STEP>
 int launch_dim(skn_ctx* ctx, const skn_kv* kv, const AttnArgs& a, int rows, const skn_beside& beside) {
     if (kv->elem_type == SKN_TYPE_F32) return launch_as<float, D, 1, STEP>(ctx, a, rows, beside);
     if constexpr (STEP) {
-        const int qg = heads_per_group(ctx, a.n_head / a.kv_heads, a.kv_heads, a.n_splits);
+        const int qg = heads_per_group(ctx, a.n_head / a.kv_heads, a.kv_heads, a.n_splits);  // (skn_shared_attn_step_workgroups)
         if (qg == 2) return launch_as<uint16_t, D, 2, true>(ctx, a, rows, beside);
     }
     return launch_as<uint16_t, D, 1, STEP>(ctx, a, rows, beside);
@@ -419,6 +419,11 @@ int skn_shared_attn_step(skn_ctx* ctx, skn_kv* kv, int seq, const skn_shared_att
     skn_beside s = *beside;
     skn_beside_plan(ctx, s, kThreads, skn_shared_attn_step_lds(kv));
     return launch_attn<true>(ctx, kv, a, 1, s);
+}
+
+int skn_shared_attn_step_workgroups(const skn_ctx* ctx, const skn_kv* kv, int n_head, int n_splits) {
+    const int per_kv = n_head / kv->n_head, qg = kv->elem_type == SKN_TYPE_F32 ? 1 : heads_per_group(ctx, per_kv, kv->n_head, n_splits);
+    return n_splits * kv->n_head * ((per_kv + qg - 1) / qg);
 }
 
 size_t skn_shared_attn_step_lds(const skn_kv* kv) { return (size_t)2 * kv->head_dim * (kWaves + 1) * sizeof(float) + 1024; }

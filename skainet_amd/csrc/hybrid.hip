@@ -206,14 +206,22 @@ skn_dense_out side_segment(const skn_hybrid* m, int l, const int32_t* tokens, vo
 //     input for two rows (two layers, width 2048, 8192 columns 73.4 | 77.5; 14000 columns 93.5 | 107.6),
 //   - for rows of less than 2560 bytes, too few to pay for the larger launch (1000 columns, 32 heads of 64: width 2048 105.3 | 105.6,
 //     2560 115.3 | 116.8; 600 columns 112.5 | 115.5),
+//   - beside an attention whose workgroups leave less than an eighth of the device in their last round, as the splits of long contexts
+//     do: the product would wait for them.  Two layers of 16 heads of 128 at 4200 tokens (256 workgroups), width 1024 / 2048 / 4096: 71.7 |
+//     75.5, 86.4 | 89.3, 132.6 | 136.4.  The step without over the step with, 224 workgroups 0.98 - 1.06, fewer 0.99 - 1.12, 320 and 384
+//     1.02 - 1.11,
 //   - past the LDS that a launch has without asking for more (feed-forwards of 14336 columns beside the delta rule, 12288, 10240 and
 //     6144 beside attention heads of 64, 128 and 256).
-skn_beside ff_beside(const skn_hybrid* m, const Layer& L, float* x) {
+skn_beside ff_beside(skn_ctx* ctx, const skn_hybrid* m, const Layer& L, int max_ctx, float* x) {
     skn_beside s;
     const bool general_delta = L.p.mixer == SKN_MIX_GENERAL_DELTA;
     if (L.p.mixer != SKN_MIX_SHARED_ATTN && !general_delta) return s;
     if (general_delta && L.state->dim_pad <= kDeltaPairDim) return s;
     if (L.p.ff * (L.out.type == SKN_TYPE_F32 ? 4 : 2) < 2560) return s;
+    if (!general_delta) {
+        const int units = ctx->compute_units, n = skn_shared_attn_step_workgroups(ctx, L.kv, L.shared.n_head, skn_shared_attn_splits(ctx, L.kv, L.shared.n_head, max_ctx));
+        if (8 * ((n - 1) % units + 1) > 7 * units) return s;
+    }
     s.type = L.out.type;
     s.rows = m->cfg.width;
     s.k_pad = L.out.k_pad - L.off_ff;
@@ -341,7 +349,7 @@ int decode_step(skn_ctx* ctx, skn_hybrid* m, int max_ctx) {
         skn_dense_mat out = L.out;
         skn_beside ff;
         if (L.p.ff && !L.p.norm2) {
-            ff = ff_beside(m, L, x);
+            ff = ff_beside(ctx, m, L, max_ctx, x);
             if (ff.w) {
                 out.k_pad = L.off_ff;
                 out.ld = L.out.k_pad;

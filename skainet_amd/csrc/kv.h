@@ -69,6 +69,7 @@ int skn_shared_attn_rows(skn_ctx* ctx, skn_kv* kv, int seq, const skn_shared_att
 int skn_shared_attn_step(skn_ctx* ctx, skn_kv* kv, int seq, const skn_shared_attn& p, const float* q, const float* k, const int32_t* state_dev,
                          int n_splits, float* opart, float* ml, float* out, const struct skn_beside* beside = nullptr);
 size_t skn_shared_attn_step_lds(const skn_kv* kv);  // at most, of a workgroup without a product beside it
+int skn_shared_attn_step_workgroups(const skn_ctx* ctx, const skn_kv* kv, int n_head, int n_splits);
 int skn_shared_attn_splits(skn_ctx* ctx, const skn_kv* kv, int n_head, int max_ctx);
 // the matrix-core form for prompts (csrc/attention_prefill.hip): fp16 caches, head_dim 64 or 128
 int skn_shared_attn_prefill_launch(skn_ctx* ctx, skn_kv* kv, int seq, const float* q_prep, int n_queries, int first_ctx, int n_head, float scale,

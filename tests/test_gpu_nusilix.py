@@ -59,10 +59,10 @@ def test_feed_forward_beside_the_mixer_of_a_step(hip, width, ff, dtype):
     m.free()
 
 
-def step_workgroups(hip, cfg, seed=3, weights=None):
-    """What one decode step launches, eagerly."""
-    m = cases.device_model(hip, cfg, cases.weights(cfg, 4, seed=seed) if weights is None else weights, "bfloat16")
-    m.prefill(cases.tokens(cfg, 3))
+def step_workgroups(hip, cfg, seed=3, weights=None, context=3):
+    """What one decode step behind `context` tokens launches, eagerly."""
+    m = cases.device_model(hip, cfg, cases.weights(cfg, 4, seed=seed) if weights is None else weights, "bfloat16", max_tokens=1024)
+    m.prefill(cases.tokens(cfg, context))
     hip.set_option("llama.graph", 0)
     try:
         before = hip.stat("workgroups")
@@ -83,6 +83,17 @@ def test_short_feed_forwards_and_small_heads_have_nothing_beside_the_mixer(hip):
     assert taken(1, 64, 1280) - taken(1, 64, 1248) == 4 + 64
     assert taken(1, 64, 1312) - taken(1, 64, 1280) == 4
     assert taken(1, 64, 1312) - taken(2, 32, 1312) == 64 - 1
+
+
+@pytest.mark.parametrize("heads,beside", [(28, True), (32, False)])
+def test_attention_that_fills_the_device_has_nothing_beside_it(hip, heads, beside):
+    """Heads of 256: eight splits instead of four past 512 tokens, 256 workgroups of 32 heads, one per compute unit; 28 heads leave an
+    eighth of the device.  Counted: the attention's own, and the 32 beside it of rows of 512, sixteen wavefronts each."""
+    assert hip.device_info()["compute_units"] == 256, "the heads are chosen for 256 compute units"
+    cfg = cases.model([cases.attention(heads, 1, 256, ff=1300)], width=512, vocab=40, groups=1)
+    w = cases.weights(cfg, 4, seed=4)
+    long, short = (step_workgroups(hip, cfg, weights=w, context=n) for n in (520, 260))
+    assert long - short == 4 * heads - (0 if beside else 32)
 
 
 def test_product_beside_the_mixer_has_no_more_workgroups_than_fit(hip):
