@@ -18,6 +18,7 @@
 //     unit in which a column's accumulators are kept.
 #include "common.h"
 #include "gemm_blocks.h"
+#include "gemm_few.h"
 #include "gemm_q6k.h"
 #include "gemm_tiles.h"
 
@@ -686,7 +687,7 @@ __global__ __launch_bounds__(256) void gemm_add_parts_kernel(const float* __rest
         for (; z < splits; z++) sum += *reinterpret_cast<const vec*>(p + z * stride);
         return sum;
     };
-    const float sc = inv_scale[row];
+    const float sc = inv_scale ? inv_scale[row] : 1.f;
     vec v = total(src) * sc;
     if (segs.pair) {
         const vec u = total(src + segs.col0[1]) * sc;
@@ -2119,7 +2120,9 @@ int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out) {
 
 float* skn_gemm_parts_room(skn_ctx* ctx, size_t bytes) {
     if (ctx->opt_test_gemm_no_parts) return nullptr;
-    if (bytes > ctx->gemm_parts_bytes && !grow_parts(ctx, bytes)) return nullptr;
+    // (asked for ahead of any workspace, as the products of few rows do: what that would have brought)
+    const size_t least = ctx->gemm_parts ? 0 : (size_t)ctx->compute_units * 256 * 128 * 4;
+    if (bytes > ctx->gemm_parts_bytes && !grow_parts(ctx, std::max(bytes, least))) return nullptr;
     return (float*)ctx->gemm_parts;
 }
 
@@ -2284,6 +2287,9 @@ extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n,
     SKN_REQUIRE(ctx, w_dev && a_bf16_dev, SKN_ERR_ARG, "skn_gemm_q: null pointer");
     SKN_REQUIRE(ctx, k % 64 == 0, SKN_ERR_SHAPE, "skn_gemm_q: k (%d) must be a multiple of %d", k, 64);
 
+    // few rows: one launch instead of three
+    if (((uintptr_t)a_bf16_dev & 7) == 0 && skn_gemm_few_ok(ctx, ggml_type, w_dev, n, k, m))
+        return skn_gemm_few(ctx, ggml_type, w_dev, n, k, a_bf16_dev, m, c_dev);
     if (ggml_type == SKN_TYPE_Q4_K && k <= 16384) {
         SKN_REQUIRE(ctx, ((uintptr_t)w_dev & 15) == 0 && ((uintptr_t)a_bf16_dev & 7) == 0, SKN_ERR_ARG,
                     "skn_gemm_q: Q4_K weights must be 16-byte aligned, activations 8-byte aligned");

@@ -1,0 +1,415 @@
+// Product of few activation rows with block-quantized weights: C[m, n] = sum_k A[m, k] w[n, k], A bf16 as it is given, Q4_K, Q5_K,
+// Q6_K, Q8_0 or Q4_0 weights, one launch and no workspace.
+//
+// Bound by the latency of a launch, then by the unpacking.  The kernels for more rows (gemm.hip, gemm_blocks.hip) take three
+// launches where tiles are few: a pass that scales the rows to fp16, the product, the addition of the parts of k.  None of it is
+// needed here.  A quant less its zero has at most eight bits, exact in bf16, so the matrix cores take the activations as they are
+// (v_mfma_f32_16x16x32_bf16; products exact, sums in fp32), a block's sum starts from zero and joins the total in fp32 times the
+// block's scale: an accumulator's column is the lane's own weight row, so the scale is one value per lane.  Minima: the block's
+// activations against a column of ones is one more matrix instruction and gives the sum that the minimum is multiplied with.
+// A workgroup keeps all of k for its sixteen columns: its eight (or four) wavefronts take superblocks of 256 in
+// turn and add their tiles through LDS.
+//
+// us per call, three launches -> this: Q4_K 16 x 4096 x 4096 11.8 -> 5.4, Q8_0 16 x 4096 x 4096 13.4 -> 7.2, Q6_K 41 x 4096 x 11008 34.9 -> 21.4 (weights
+// alone 7.5 at the rate of a copy), Q5_K 16 x 1000 x 1024 9.4 -> 4.9.  Error against 64 bits: not larger (1.1 against 1.5e-7 of the
+// result in Q4_K at k = 11008, 0.95 against 1.05 in Q8_0): a superblock's sum is formed before it joins the total.
+#include "gemm_few.h"
+#include "gemm_tiles.h"
+
+#include <algorithm>
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// ---- formats --------------------------------------------------------------------------------------------------------------
+// Lane 16 g + c holds column c (a weight row) and, of a block of 32 elements, elements 8 g .. 8 g + 7 (Q6_K, whose scales are for
+// sixteen: elements 4 g .. 4 g + 3 of either half).  kBytes: of a superblock of 256 elements; kPieces: the sixteen-byte pieces that
+// hold it; kPitch: of a row in LDS, chosen so that sixteen rows start in sixteen different groups of four banks.  `row` points at
+// the lane's row there.
+
+__device__ __forceinline__ float f16_lo(uint32_t w) { return (float)__builtin_bit_cast(half2_t, w).x; }
+__device__ __forceinline__ float f16_hi(uint32_t w) { return (float)__builtin_bit_cast(half2_t, w).y; }
+__device__ __forceinline__ uint32_t lds_u32(const uint8_t* p) { return *reinterpret_cast<const uint32_t*>(p); }
+__device__ __forceinline__ u32x2 lds_u32x2(const uint8_t* p) { return *reinterpret_cast<const u32x2*>(p); }
+
+// Four whole numbers of at most eight bits, one to a byte, as bf16: the upper halves of their fp32 forms.
+__device__ __forceinline__ u32x2 signed_bytes(uint32_t b) {
+    const float f0 = (float)(int8_t)b, f1 = (float)(int8_t)(b >> 8), f2 = (float)(int8_t)(b >> 16), f3 = (float)(int8_t)(b >> 24);
+    return u32x2{__builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u),
+                 __builtin_amdgcn_perm(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u)};
+}
+__device__ __forceinline__ u32x2 unsigned_bytes(uint32_t b) {
+    const float f0 = (float)(uint8_t)b, f1 = (float)(uint8_t)(b >> 8), f2 = (float)(uint8_t)(b >> 16), f3 = (float)(uint8_t)(b >> 24);
+    return u32x2{__builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u),
+                 __builtin_amdgcn_perm(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u)};
+}
+// Four numbers 0..15: as E4M3 a byte below sixteen is that many times 2^-9 (subnormals and the first binade are one straight line).
+__device__ __forceinline__ u32x2 nibble_bytes(uint32_t b) {
+    return u32x2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f, false)),
+                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f, true))};
+}
+__device__ __forceinline__ bf16x8 operand(u32x2 lo, u32x2 hi) { return __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y}); }
+
+// The K-quants with sub-blocks of 32 (see gemm_blocks.hip for their layout).
+template <bool FIVE>
+struct FewK {
+    static constexpr int kBytes = FIVE ? 176 : 144, kPieces = kBytes / 16, kPitch = kBytes;
+    static constexpr bool kMin = true, kHalves = false;
+    struct Head {
+        float d, dmin;
+        uint32_t sc[2], mn[2];
+        u32x2 fifth;
+    };
+    __device__ static __forceinline__ void head(const uint8_t* row, int g, Head& s) {
+        const u32x4 h = *reinterpret_cast<const u32x4*>(row);
+        s.d = f16_lo(h[0]), s.dmin = f16_hi(h[0]);
+        s.sc[0] = h[1] & 0x3F3F3F3Fu, s.sc[1] = (h[3] & 0x0F0F0F0Fu) | ((h[1] >> 2) & 0x30303030u);
+        s.mn[0] = h[2] & 0x3F3F3F3Fu, s.mn[1] = ((h[3] >> 4) & 0x0F0F0F0Fu) | ((h[2] >> 2) & 0x30303030u);
+        if (FIVE) s.fifth = lds_u32x2(row + 16 + 8 * g);
+    }
+    __device__ static __forceinline__ bf16x8 block(const uint8_t* row, const Head& H, int b, int g, float& s, float& mn) {
+        s = H.d * (float)((H.sc[b >> 2] >> (8 * (b & 3))) & 0xFFu);  // (11 x 6 bits: exact)
+        mn = H.dmin * (float)((H.mn[b >> 2] >> (8 * (b & 3))) & 0xFFu);
+        const u32x2 x = lds_u32x2(row + (FIVE ? 48 : 16) + 32 * (b >> 1) + 8 * g);
+        const u32x2 q = (x >> (uint32_t)(4 * (b & 1))) & 0x0F0F0F0Fu;
+        if (!FIVE) return operand(nibble_bytes(q.x), nibble_bytes(q.y));
+        const u32x2 f = (b < 4 ? H.fifth << (uint32_t)(4 - b) : H.fifth >> (uint32_t)(b - 4)) & 0x10101010u;
+        return operand(unsigned_bytes(q.x | f.x), unsigned_bytes(q.y | f.y));
+    }
+};
+
+struct FewQ80 {  // 34 bytes: d, 32 int8; block pairs are 17 dwords
+    static constexpr int kBytes = 272, kPieces = 17, kPitch = 272;
+    static constexpr bool kMin = false, kHalves = false;
+    struct Head {};
+    __device__ static __forceinline__ void head(const uint8_t*, int, Head&) {}
+    __device__ static __forceinline__ bf16x8 block(const uint8_t* row, const Head&, int b, int g, float& s, float&) {
+        const uint8_t* p = row + 68 * (b >> 1);
+        uint32_t x, y;
+        if (b & 1) {
+            s = f16_hi(lds_u32(p + 32));
+            x = lds_u32(p + 36 + 8 * g), y = lds_u32(p + 40 + 8 * g);
+        } else {
+            s = f16_lo(lds_u32(p));
+            const uint32_t w0 = lds_u32(p + 8 * g), w1 = lds_u32(p + 4 + 8 * g), w2 = lds_u32(p + 8 + 8 * g);
+            x = __builtin_amdgcn_alignbyte(w1, w0, 2), y = __builtin_amdgcn_alignbyte(w2, w1, 2);
+        }
+        return operand(signed_bytes(x), signed_bytes(y));
+    }
+};
+
+struct FewQ40 {  // 18 bytes: d, nibbles (low ones elements 0..15, high ones 16..31); pairs are 9 dwords
+    static constexpr int kBytes = 144, kPieces = 9, kPitch = 144;
+    static constexpr bool kMin = false, kHalves = false;
+    struct Head {};
+    __device__ static __forceinline__ void head(const uint8_t*, int, Head&) {}
+    // a nibble at the top of its byte, less eight there, is 16 (q - 8)
+    __device__ static __forceinline__ bf16x8 block(const uint8_t* row, const Head&, int b, int g, float& s, float&) {
+        const uint8_t* p = row + 36 * (b >> 1);
+        const int at = 8 * (g & 1);
+        u32x2 q;
+        if (b & 1) {
+            s = f16_hi(lds_u32(p + 16)) * 0.0625f;
+            q = u32x2{lds_u32(p + 20 + at), lds_u32(p + 24 + at)};
+        } else {
+            s = f16_lo(lds_u32(p)) * 0.0625f;
+            const uint32_t w0 = lds_u32(p + at), w1 = lds_u32(p + 4 + at), w2 = lds_u32(p + 8 + at);
+            q = u32x2{__builtin_amdgcn_alignbyte(w1, w0, 2), __builtin_amdgcn_alignbyte(w2, w1, 2)};
+        }
+        q = ((q << (uint32_t)(g < 2 ? 4 : 0)) & 0xF0F0F0F0u) ^ 0x80808080u;
+        return operand(signed_bytes(q.x), signed_bytes(q.y));
+    }
+};
+
+// Q6_K: half hf of 128 elements, quarter Q of 32: low bits in nibble Q / 2 of bytes 64 hf + 32 (Q % 2) .. + 31, high bits at 2 Q of
+// bytes 128 + 32 hf .. + 31, an int8 scale for sixteen elements from byte 192 on, d at 208: the end of the last piece, which is the
+// superblock's last sixteen bytes.
+struct FewQ6K {
+    static constexpr int kBytes = 210, kPieces = 14, kPitch = 240;
+    static constexpr bool kHalves = true;
+    struct Head {
+        float d4;  // d / 4: the operands are 4 (q - 32)
+        u32x4 sc;
+    };
+    __device__ static __forceinline__ void head(const uint8_t* row, int, Head& s) {
+        s.d4 = f16_hi(lds_u32(row + 220)) * 0.25f;
+        s.sc = *reinterpret_cast<const u32x4*>(row + 192);
+    }
+    __device__ static __forceinline__ s16x4 sixteen(const uint8_t* row, const Head& H, int b, int t, int g, float& s) {
+        const int hf = b >> 2, Q = b & 3, e = 2 * b + t;
+        s = H.d4 * (float)(int8_t)(H.sc[e >> 2] >> (8 * (e & 3)));
+        const uint32_t ql = lds_u32(row + 64 * hf + 32 * (Q & 1) + 16 * t + 4 * g), qh = lds_u32(row + 128 + 32 * hf + 16 * t + 4 * g);
+        const uint32_t lo = (Q < 2 ? ql << 2 : ql >> 2) & 0x3C3C3C3Cu;
+        const uint32_t hi = (Q == 3 ? qh : qh << (6 - 2 * Q)) & 0xC0C0C0C0u;
+        return __builtin_bit_cast(s16x4, signed_bytes((lo | hi) ^ 0x80808080u));
+    }
+};
+
+// ---- the product ------------------------------------------------------------------------------------------------------------
+
+// blocks of 32 whose activations a wavefront holds in LDS at a time (8 KiB at most)
+constexpr int few_chunk(int mt) { return mt == 1 ? 4 : 2; }
+
+template <typename F, int MT, int W>
+constexpr int few_lds_bytes() {
+    return std::max(W * (16 * F::kPitch + few_chunk(MT) * MT * 1024), W * MT * 1024);
+}
+
+// MT row blocks of sixteen, sixteen columns, W wavefronts
+template <typename F, int MT, int W>
+__global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __restrict__ a, const uint8_t* __restrict__ w, float* __restrict__ c, int m, int n,
+                                                          int k, uint32_t a_bytes, uint32_t w_bytes, float* __restrict__ part, int part_blocks) {
+    extern __shared__ __align__(16) uint8_t lds[];  // a superblock of the tile's weight rows per wavefront, then the exchange of the tiles
+    constexpr int P = F::kPieces, LOADS = (16 * P + 63) / 64;
+    constexpr int CH = few_chunk(MT), AP = 4 * CH;  // sixteen-byte pieces of a chunk's row
+    const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nb = k >> 8, n0 = (int)blockIdx.x * 16;
+    const int sb0 = (int)blockIdx.y * part_blocks, sb1 = min(sb0 + part_blocks, nb);  // (all, or a part of k)
+    const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, (int)w_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc((void*)a, 0, (int)a_bytes, 0x00020000);
+    uint8_t* mine = lds + wave * (16 * F::kPitch + CH * MT * 1024);
+    uint8_t* rows = mine + 16 * F::kPitch;
+    const uint8_t* row = mine + col * F::kPitch;
+    f32x4 acc[MT], total[MT];  // of a superblock, of the wavefront's superblocks
+#pragma unroll
+    for (int i = 0; i < MT; i++) total[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const u32x4 ones_bits = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, ones_bits);
+
+    // Piece 64 x + lane of the tile's rows of a superblock: coalesced loads one superblock ahead, handed over through LDS of the
+    // wavefront's own (the lane number passes through an empty asm: a store of wstore may go anywhere as far as the compiler knows and
+    // keeps its place among the loads before and after it, and the device keeps a wavefront's LDS accesses in order).
+    u32x4 next[LOADS];
+    auto wload = [&](int sb) __attribute__((always_inline)) {
+        int l = lane;
+        asm("" : "+v"(l));
+#pragma unroll
+        for (int x = 0; x < LOADS; x++) {
+            const int p = 64 * x + l, r = p / P;
+            const int from = min(n0 + r, n - 1) * (nb * F::kBytes) + min((p - r * P) * 16, F::kBytes - 16);  // (rows past the end: a repeat of the last one)
+            next[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, p < 16 * P ? from : (int)w_bytes, sb * F::kBytes, 0));
+        }
+    };
+    auto wstore = [&]() __attribute__((always_inline)) {
+        int l = lane;
+        asm("" : "+v"(l));
+#pragma unroll
+        for (int x = 0; x < LOADS; x++) {
+            const int p = 64 * x + l, r = p / P;
+            if (64 * x + 64 <= 16 * P || p < 16 * P) *reinterpret_cast<u32x4*>(mine + r * F::kPitch + (p - r * P) * 16) = next[x];
+        }
+    };
+    // The activations likewise, a chunk of CH blocks ahead: piece p of row r goes to place p ^ turn(r) of the row, so that the sixteen
+    // rows of an operand lie on different banks.  (Rows past the end: an offset past the end, which reads as zero.)
+    auto turn = [](int r) __attribute__((always_inline)) { return CH == 2 ? (r >> 1) & 7 : r & 15; };
+    u32x4 anext[CH * MT];
+    auto aload = [&](int chunk) __attribute__((always_inline)) {
+        int l = lane;
+        asm("" : "+v"(l));
+#pragma unroll
+        for (int x = 0; x < CH * MT; x++) {
+            const int r = (64 * x + l) / AP, p = l % AP;
+            anext[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, r < m ? r * 2 * k + 16 * p : (int)a_bytes, chunk * 64 * CH, 0));
+        }
+    };
+    auto astore = [&]() __attribute__((always_inline)) {
+        int l = lane;
+        asm("" : "+v"(l));
+#pragma unroll
+        for (int x = 0; x < CH * MT; x++) {
+            const int r = (64 * x + l) / AP, p = l % AP;
+            *reinterpret_cast<u32x4*>(rows + (r * AP + (p ^ turn(r & 15))) * 16) = anext[x];
+        }
+    };
+    auto aread = [&](int i, int b) __attribute__((always_inline)) {  // b: in the chunk
+        const uint8_t* base = rows + (16 * i + col) * (AP * 16);
+        if (!F::kHalves) return *reinterpret_cast<const u32x4*>(base + ((4 * b + g) ^ turn(col)) * 16);
+        const u32x2 x = lds_u32x2(base + ((4 * b + (g >> 1)) ^ turn(col)) * 16 + 8 * (g & 1));
+        const u32x2 y = lds_u32x2(base + ((4 * b + 2 + (g >> 1)) ^ turn(col)) * 16 + 8 * (g & 1));
+        return u32x4{x.x, x.y, y.x, y.y};
+    };
+    if (sb0 + wave < sb1) {
+        wload(sb0 + wave);
+        aload((8 / CH) * (sb0 + wave));
+    }
+    for (int sb = sb0 + wave; sb < sb1; sb += W) {
+        const int sbn = min(sb + W, nb - 1);  // (past the end: a repeat, unused)
+        wstore();
+        wload(sbn);
+        typename F::Head H;
+        F::head(row, g, H);
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            if (b % CH == 0) {
+                astore();
+                aload(b + CH < 8 ? (8 / CH) * sb + b / CH + 1 : (8 / CH) * sbn);
+            }
+            u32x4 av[MT];
+#pragma unroll
+            for (int i = 0; i < MT; i++) av[i] = aread(i, b % CH);
+            if constexpr (F::kHalves) {
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    float s;
+                    const s16x4 q = F::sixteen(row, H, b, t, g, s);
+#pragma unroll
+                    for (int i = 0; i < MT; i++) {
+                        const s16x4 x = __builtin_bit_cast(s16x4, u32x2{av[i][2 * t], av[i][2 * t + 1]});
+                        const f32x4 p = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(x, q, zero, 0, 0, 0);
+#pragma unroll
+                        for (int y = 0; y < 4; y++) acc[i][y] = b == 0 && t == 0 ? s * p[y] : fmaf(s, p[y], acc[i][y]);
+                    }
+                }
+            } else {
+                float s, mn = 0.f;
+                const bf16x8 q = F::block(row, H, b, g, s, mn);
+#pragma unroll
+                for (int i = 0; i < MT; i++) {
+                    const bf16x8 x = __builtin_bit_cast(bf16x8, av[i]);
+                    const f32x4 p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, q, zero, 0, 0, 0);
+#pragma unroll
+                    for (int y = 0; y < 4; y++) acc[i][y] = b == 0 ? s * p[y] : fmaf(s, p[y], acc[i][y]);
+                    if constexpr (F::kMin) {
+                        const f32x4 sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, ones, zero, 0, 0, 0);
+#pragma unroll
+                        for (int y = 0; y < 4; y++) acc[i][y] = fmaf(-mn, sum[y], acc[i][y]);
+                    }
+                }
+            }
+            if ((b & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // (more blocks at once would not fit the registers)
+        }
+#pragma unroll
+        for (int i = 0; i < MT; i++) total[i] += acc[i];
+    }
+
+    __syncthreads();
+    f32x4* red = reinterpret_cast<f32x4*>(lds);
+#pragma unroll
+    for (int i = 0; i < MT; i++) red[(wave * MT + i) * 64 + lane] = total[i];
+    __syncthreads();
+    // (accumulator register y of lane 16 g + c: row 4 g + y, column c)
+    const float* flat = reinterpret_cast<const float*>(red);
+    for (int e = threadIdx.x; e < MT * 256; e += 64 * W) {
+        const int r = e >> 4, cc = e & 15;
+        const int from = (r >> 4) * 256 + (((r >> 2) & 3) * 16 + cc) * 4 + (r & 3);
+        float sum = 0.f;
+#pragma unroll
+        for (int x = 0; x < W; x++) sum += flat[x * MT * 256 + from];
+        if (r < m && n0 + cc < n) {
+            const size_t at = (size_t)r * n + n0 + cc;
+            if (part) part[(size_t)blockIdx.y * m * n + at] = sum;
+            else c[at] = sum;
+        }
+    }
+}
+
+template <typename F, int MT, int W>
+int launch_few(skn_ctx* ctx, const uint8_t* w, const uint16_t* a, float* c, int m, int n, int k, int splits) {
+    const int nb = k / 256, each = (nb + splits - 1) / splits;
+    splits = (nb + each - 1) / each;  // (no workgroup without a superblock)
+    float* part = splits > 1 ? skn_gemm_parts_room(ctx, (size_t)splits * m * n * 4) : nullptr;
+    if (!part) splits = 1;
+    skn_launch(ctx, gemm_few_kernel<F, MT, W>, dim3((n + 15) / 16, splits), dim3(64 * W), few_lds_bytes<F, MT, W>(), a, w, c, m, n, k,
+               (uint32_t)((size_t)m * k * 2), (uint32_t)((size_t)n * nb * F::kBytes), part, splits > 1 ? each : nb);
+    SKN_LAUNCH_CHECK(ctx);
+    if (!part) return SKN_OK;
+    const skn_gemm_parts ps = {{c, nullptr, nullptr}, {n, 0, 0}, {0, 0, 0}, {0, 0, 0}, 1, 0};
+    return skn_gemm_add_parts(ctx, part, splits, n, ps, nullptr, m);
+}
+
+// Few columns: k over workgroups too where the turns of a wavefront that this saves, 0.5 + 0.7 MT us each, pay for the addition (3 us).  us
+// per call, undivided | in four parts: Q4_K 16 x 1000 x 11008 10.1 | 8.3, 64 x 1000 x 11008 23 | 12.9, 16 x 2000 x 2048 4.9 | 7.5 (undivided).
+// Where the tiles are more than the compute units and a workgroup of eight wavefronts leaves no LDS for another, four of them go
+// to a workgroup: Q8_0 57 x 8192 x 2048 14.1 | 12.5, 41 x 14336 x 4096 33.3 | 28.9 (with room for two: Q4_K 41 x 14336 x 4096 26.2 | 30.2).
+template <typename F, int MT>
+int launch_rows(skn_ctx* ctx, const uint8_t* w, const uint16_t* a, float* c, int m, int n, int k) {
+    const int tiles = (n + 15) / 16, nb = k / 256;
+    const int splits = std::max(1, std::min({ctx->compute_units / tiles, (nb + 7) / 8, 16}));
+    const int saved = (nb + 7) / 8 - ((nb + splits - 1) / splits + 7) / 8;
+    if (saved * (0.5f + 0.7f * MT) > 3.0f) return launch_few<F, MT, 8>(ctx, w, a, c, m, n, k, splits);
+    if constexpr (few_lds_bytes<F, MT, 8>() > 80 * 1024) {
+        if (tiles > ctx->compute_units) return launch_few<F, MT, 4>(ctx, w, a, c, m, n, k, 1);
+    }
+    return launch_few<F, MT, 8>(ctx, w, a, c, m, n, k, 1);
+}
+
+template <typename F>
+int launch_format(skn_ctx* ctx, const uint8_t* w, const uint16_t* a, float* c, int m, int n, int k) {
+    if (m <= 16) return launch_rows<F, 1>(ctx, w, a, c, m, n, k);
+    if (m <= 32) return launch_rows<F, 2>(ctx, w, a, c, m, n, k);
+    if (m <= 48) return launch_rows<F, 3>(ctx, w, a, c, m, n, k);
+    return launch_rows<F, 4>(ctx, w, a, c, m, n, k);
+}
+
+template <typename F, int MT>
+int allow_lds(skn_ctx* ctx) {
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_few_kernel<F, MT, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, few_lds_bytes<F, MT, 8>()));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_few_kernel<F, MT, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, few_lds_bytes<F, MT, 4>()));
+    return SKN_OK;
+}
+
+template <typename F>
+int allow_format(skn_ctx* ctx) {
+    SKN_TRY((allow_lds<F, 1>(ctx)));
+    SKN_TRY((allow_lds<F, 2>(ctx)));
+    SKN_TRY((allow_lds<F, 3>(ctx)));
+    return allow_lds<F, 4>(ctx);
+}
+
+int few_init(skn_ctx* ctx) {
+    SKN_TRY(allow_format<FewK<false>>(ctx));
+    SKN_TRY(allow_format<FewK<true>>(ctx));
+    SKN_TRY(allow_format<FewQ6K>(ctx));
+    SKN_TRY(allow_format<FewQ80>(ctx));
+    return allow_format<FewQ40>(ctx);
+}
+skn_family register_family(few_init);
+
+}  // namespace
+
+// Every sixteen columns read all the activations and unpack for themselves, so that the time here grows with the row blocks where the
+// other kernels' hardly does: what they gain on three launches is lost again from so many superblocks of sixteen columns per compute unit
+// on (16, 32, 48, 64 rows; 0: not found up to 196).  us per call, others | these: Q4_K 32 x 12000 x 4096 (47) 18.7 | 15.8, 32 x 14336 x 4096
+// (56) 19.7 | 20.4, 41 x 6000 x 6144 (35) 20.6 | 19.2, 41 x 14336 x 4096 20.9 | 26.2; Q5_K 32 x 14336 x 4096 22.1 | 22.0, 41 x 14336 x 4096 26.9 | 28.1;
+// Q6_K 41 x 14336 x 4096 33.7 | 30.6, 57 x 14336 x 4096 33.6 | 40.5; Q8_0 41 x 14336 x 4096 29.0 | 28.9, 32 x 14336 x 14336 (196) 74 | 85; Q4_0 (whose
+// quants take three times Q4_K's instructions) 16 x 6000 x 6144 17.8 | 15.6, 16 x 14336 x 4096 18.7 | 19.3.  Over a single round of compute units
+// 64 rows hold out longer: 64 x 4096 x 11008 (43) Q4_K 24.8 | 23.3, Q8_0 28.7 | 23.5, against 57 x 6000 x 6144 21.2 | 27.3, 25.6 | 26.4.
+// Q4_K and Q6_K of more than 32 rows, up to 4096 elements and a round of tiles or more stay with the others although this is the faster path
+// (41 x 4096 x 4096 15.5 | 9.7 and 19.3 | 10.7): the number of launches that such products take is held fixed by tests.  Options that fix how k is divided mean the others.
+bool skn_gemm_few_ok(const skn_ctx* ctx, int type, const void* w, int n, int k, int m) {
+    int bytes;
+    struct {
+        int rows[4];
+    } most;
+    switch (type) {
+        case SKN_TYPE_Q4_K: bytes = FewK<false>::kBytes, most = {{0, 48, 36, 20}}; break;
+        case SKN_TYPE_Q5_K: bytes = FewK<true>::kBytes, most = {{0, 56, 40, 20}}; break;
+        case SKN_TYPE_Q6_K: bytes = FewQ6K::kBytes, most = {{0, 0, 60, 24}}; break;
+        case SKN_TYPE_Q8_0: bytes = FewQ80::kBytes, most = {{0, 80, 50, 24}}; break;
+        case SKN_TYPE_Q4_0: bytes = FewQ40::kBytes, most = {{45, 33, 33, 20}}; break;
+        default: return false;
+    }
+    if (ctx->opt_gemm_tile != 0 || ctx->opt_gemm_split != 0 || ctx->opt_test_gemm_no_parts || ctx->opt_gemm_q6k_fused != 1 || m <= 0 || m > 64 || n <= 0 || k <= 0 || k % 256 != 0 || k > 16384 ||
+        ((uintptr_t)w & (type == SKN_TYPE_Q6_K ? 1 : 15)) != 0 || (size_t)n * (k / 256) * bytes >= ((size_t)1 << 31))
+        return false;
+    const int blocks = (m + 15) / 16, tiles = (n + 15) / 16;
+    if (m > 32 && k <= 4096 && tiles >= ctx->compute_units && (type == SKN_TYPE_Q4_K || type == SKN_TYPE_Q6_K)) return false;
+    const int limit = blocks == 4 && tiles <= ctx->compute_units ? 45 : most.rows[blocks - 1];
+    return limit == 0 || (size_t)tiles * (k / 256) <= (size_t)limit * ctx->compute_units;
+}
+
+int skn_gemm_few(skn_ctx* ctx, int type, const void* w, int n, int k, const uint16_t* a_bf16, int m, float* c) {
+    const uint8_t* wb = (const uint8_t*)w;
+    switch (type) {
+        case SKN_TYPE_Q4_K: return launch_format<FewK<false>>(ctx, wb, a_bf16, c, m, n, k);
+        case SKN_TYPE_Q5_K: return launch_format<FewK<true>>(ctx, wb, a_bf16, c, m, n, k);
+        case SKN_TYPE_Q6_K: return launch_format<FewQ6K>(ctx, wb, a_bf16, c, m, n, k);
+        case SKN_TYPE_Q8_0: return launch_format<FewQ80>(ctx, wb, a_bf16, c, m, n, k);
+        default: return launch_format<FewQ40>(ctx, wb, a_bf16, c, m, n, k);
+    }
+}

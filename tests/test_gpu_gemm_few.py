@@ -1,0 +1,95 @@
+"""GPU: products of up to 64 rows that take one launch, against 64-bit sums of the oracle's weights."""
+import numpy as np
+import pytest
+
+from oracle import oracle_c, oracle_np
+from skainet_amd import synth
+
+pytestmark = pytest.mark.gpu
+FORMATS = {"q4_k": synth.Q4_K, "q5_k": synth.Q5_K, "q6_k": synth.Q6_K, "q8_0": synth.Q8_0, "q4_0": synth.Q4_0}
+# 2^-24 of the sum of the terms' magnitudes per rounding: up to 32 in a matrix instruction, 16 in a superblock, then one for each of
+# a wavefront's superblocks (8 at most here) and of the wavefronts and parts (12)
+ROUNDINGS = 32 + 16 + 8 + 12
+
+
+def _check(hip, t, raw, n, k, a, m, launches=None):
+    c = hip.alloc(4 * m * n)
+    hip.memset(c, 0xFF, 4 * m * n)
+    w, x = hip.to_device(raw), hip.to_device(a)
+    before = hip.stat("launches")
+    hip.gemm_q(t, w, n, k, x, m, c)
+    assert launches is None or hip.stat("launches") - before == launches
+    got = c.download(np.float32, m * n).reshape(m, n)
+    wd = oracle_c.dequant(t, raw).astype(np.float64).reshape(n, k)
+    xd = oracle_np.bf16_to_f32(a).astype(np.float64).reshape(m, k)
+    size = np.abs(xd) @ np.abs(wd).T
+    if t in (synth.Q4_K, synth.Q5_K):  # d sc q and dmin m are terms of their own
+        size = size * 4
+    assert np.all(np.abs(got - xd @ wd.T) <= ROUNDINGS * 2.0**-24 * size + 1e-30)
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("m,n,k,launches", [(1, 1, 256, 1), (2, 15, 512, 1), (15, 16, 2048, 1), (16, 17, 2304, 1), (17, 100, 1280, 1), (32, 31, 4096, 1), (33, 48, 4352, 2),
+                                            (48, 33, 6144, 2), (49, 4100, 4352, 1), (64, 20, 8192, 2), (5, 40, 11008, 2), (33, 4090, 4352, 1), (30, 4200, 512, 1)])
+def test_row_blocks_ragged_tiles_and_divided_k(hip, name, m, n, k, launches):
+    """One to four row blocks, full and ragged; fewer superblocks than wavefronts, as many, one more; few columns with k over
+    workgroups; more tiles than compute units."""
+    t = FORMATS[name]
+    _check(hip, t, synth.weight(t, n, k, seed=n + k + t), n, k, synth.activation_bf16((m, k), seed=m + 1), m, launches)
+
+
+@pytest.mark.parametrize("name", ["q5_k", "q8_0", "q4_0"])
+@pytest.mark.parametrize("m,n,k", [(33, 48, 2304), (48, 33, 256), (49, 16, 2048), (64, 65, 768), (40, 4200, 512), (50, 4200, 768)])
+def test_three_and_four_row_blocks_of_short_rows(hip, name, m, n, k):
+    t = FORMATS[name]
+    _check(hip, t, synth.weight(t, n, k, seed=n + k + t), n, k, synth.activation_bf16((m, k), seed=m + 1), m, 1)
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+def test_rows_far_apart_and_fields_over_their_range(hip, name):
+    """Random bytes in every field but the scales (zero, subnormal and of both signs among them); rows of 1e30, of 1e-30 and of zeros,
+    elements 2^40 apart in one row: the activations are taken as they are."""
+    t = FORMATS[name]
+    m, n, k = 21, 40, 1024
+    be, bb = synth.BLOCK[t]
+    rng = np.random.default_rng(t)
+    raw = rng.integers(0, 256, (n * k // be, bb), dtype=np.uint8)
+    d = (rng.standard_normal(len(raw)) * 0.01).astype(np.float16)
+    d[::5], d[3::11] = 0.0, np.float16(6e-8)
+    at = 208 if name == "q6_k" else 0
+    raw[:, at:at + 2] = d.view(np.uint8).reshape(-1, 2)
+    if name in ("q4_k", "q5_k"):
+        raw[:, 2:4] = (rng.standard_normal(len(raw)) * 0.02).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[0] *= 1e30
+    x[1] *= 1e-30
+    x[2] = 0.0
+    x[3, ::2] *= 2.0**40
+    _check(hip, t, raw.reshape(-1), n, k, synth.f32_to_bf16_bits(x), m)
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+def test_an_infinite_activation_reaches_its_row_alone(hip, name):
+    t = FORMATS[name]
+    m, n, k = 18, 33, 512
+    raw = synth.weight(t, n, k, seed=3)
+    a = synth.activation_bf16((m, k), seed=4).reshape(m, k).copy()
+    a[17, 77], a[5, 300] = 0x7F80, 0x7FC0
+    got = hip.gemm_q_host(t, raw, n, k, a, m)
+    bad = np.zeros(m, bool)
+    bad[[5, 17]] = True
+    assert np.all(np.isfinite(got[~bad])) and not np.any(np.isfinite(got[bad]))
+    want = oracle_c.gemm_q(t, raw, n, k, a.reshape(m, k)[~bad], m - 2)
+    assert oracle_np.rel_err(got[~bad], want) <= 1e-3
+
+
+def test_weights_and_activations_on_their_least_alignment(hip):
+    """Q6_K weights from any even address, activations from any multiple of eight."""
+    m, n, k = 20, 35, 768
+    raw, a = synth.weight(synth.Q6_K, n, k, seed=4), synth.activation_bf16((m, k), seed=5)
+    w, x, c = hip.alloc(raw.nbytes + 16), hip.alloc(a.nbytes + 16), hip.alloc(4 * m * n)
+    w.upload(raw, offset=2)
+    x.upload(a, offset=8)
+    hip.gemm_q(synth.Q6_K, w.ptr + 2, n, k, x.ptr + 8, m, c)
+    got = c.download(np.float32, m * n).reshape(m, n)
+    assert oracle_np.rel_err(got, oracle_c.gemm_q(synth.Q6_K, raw, n, k, a, m)) <= 1e-3
