@@ -1,4 +1,4 @@
-// Product of few activation rows with block-quantized weights: C[m, n] = sum_k A[m, k] w[n, k], A bf16 as it is given, Q4_K, Q5_K,
+// Product of few activation rows, or of some more with a small matrix, with block-quantized weights: C[m, n] = sum_k A[m, k] w[n, k], A bf16 as it is given, Q4_K, Q5_K,
 // Q6_K, Q8_0 or Q4_0 weights, one launch and no workspace.
 //
 // Bound by the latency of a launch, then by the unpacking.  The kernels for more rows (gemm.hip, gemm_blocks.hip) take three
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
     constexpr int CH = few_chunk(MT), AP = 4 * CH;  // sixteen-byte pieces of a chunk's row
     const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int nb = k >> 8, n0 = (int)blockIdx.x * 16;
+    const int nb = k >> 8, n0 = (int)blockIdx.x * 16, m0 = (int)blockIdx.z * 16 * MT;
     const int sb0 = (int)blockIdx.y * part_blocks, sb1 = min(sb0 + part_blocks, nb);  // (all, or a part of k)
     const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, (int)w_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc((void*)a, 0, (int)a_bytes, 0x00020000);
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
         asm("" : "+v"(l));
 #pragma unroll
         for (int x = 0; x < CH * MT; x++) {
-            const int r = (64 * x + l) / AP, p = l % AP;
+            const int r = m0 + (64 * x + l) / AP, p = l % AP;
             anext[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, r < m ? r * 2 * k + 16 * p : (int)a_bytes, chunk * 64 * CH, 0));
         }
     };
@@ -300,8 +300,8 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
         float sum = 0.f;
 #pragma unroll
         for (int x = 0; x < W; x++) sum += flat[x * MT * 256 + from];
-        if (r < m && n0 + cc < n) {
-            const size_t at = (size_t)r * n + n0 + cc;
+        if (m0 + r < m && n0 + cc < n) {
+            const size_t at = (size_t)(m0 + r) * n + n0 + cc;
             if (part) part[(size_t)blockIdx.y * m * n + at] = sum;
             else c[at] = sum;
         }
@@ -314,7 +314,7 @@ int launch_few(skn_ctx* ctx, const uint8_t* w, const uint16_t* a, float* c, int 
     splits = (nb + each - 1) / each;  // (no workgroup without a superblock)
     float* part = splits > 1 ? skn_gemm_parts_room(ctx, (size_t)splits * m * n * 4) : nullptr;
     if (!part) splits = 1;
-    skn_launch(ctx, gemm_few_kernel<F, MT, W>, dim3((n + 15) / 16, splits), dim3(64 * W), few_lds_bytes<F, MT, W>(), a, w, c, m, n, k,
+    skn_launch(ctx, gemm_few_kernel<F, MT, W>, dim3((n + 15) / 16, splits, (m + 16 * MT - 1) / (16 * MT)), dim3(64 * W), few_lds_bytes<F, MT, W>(), a, w, c, m, n, k,
                (uint32_t)((size_t)m * k * 2), (uint32_t)((size_t)n * nb * F::kBytes), part, splits > 1 ? each : nb);
     SKN_LAUNCH_CHECK(ctx);
     if (!part) return SKN_OK;
@@ -328,7 +328,7 @@ int launch_few(skn_ctx* ctx, const uint8_t* w, const uint16_t* a, float* c, int 
 // to a workgroup: Q8_0 57 x 8192 x 2048 14.1 | 12.5, 41 x 14336 x 4096 33.3 | 28.9 (with room for two: Q4_K 41 x 14336 x 4096 26.2 | 30.2).
 template <typename F, int MT>
 int launch_rows(skn_ctx* ctx, const uint8_t* w, const uint16_t* a, float* c, int m, int n, int k) {
-    const int tiles = (n + 15) / 16, nb = k / 256;
+    const int tiles = (n + 15) / 16 * ((m + 16 * MT - 1) / (16 * MT)), nb = k / 256;
     const int splits = std::max(1, std::min({ctx->compute_units / tiles, (nb + 7) / 8, 16}));
     const int saved = (nb + 7) / 8 - ((nb + splits - 1) / splits + 7) / 8;
     if (saved * (0.5f + 0.7f * MT) > 3.0f) return launch_few<F, MT, 8>(ctx, w, a, c, m, n, k, splits);
@@ -338,12 +338,20 @@ int launch_rows(skn_ctx* ctx, const uint8_t* w, const uint16_t* a, float* c, int
     return launch_few<F, MT, 8>(ctx, w, a, c, m, n, k, 1);
 }
 
+// row blocks of a workgroup: rows go in groups of at most 64, as even as blocks of sixteen are
+int row_blocks(int m) {
+    const int groups = (m + 63) / 64;
+    return ((m + groups - 1) / groups + 15) / 16;
+}
+
 template <typename F>
 int launch_format(skn_ctx* ctx, const uint8_t* w, const uint16_t* a, float* c, int m, int n, int k) {
-    if (m <= 16) return launch_rows<F, 1>(ctx, w, a, c, m, n, k);
-    if (m <= 32) return launch_rows<F, 2>(ctx, w, a, c, m, n, k);
-    if (m <= 48) return launch_rows<F, 3>(ctx, w, a, c, m, n, k);
-    return launch_rows<F, 4>(ctx, w, a, c, m, n, k);
+    switch (row_blocks(m)) {
+        case 1: return launch_rows<F, 1>(ctx, w, a, c, m, n, k);
+        case 2: return launch_rows<F, 2>(ctx, w, a, c, m, n, k);
+        case 3: return launch_rows<F, 3>(ctx, w, a, c, m, n, k);
+        default: return launch_rows<F, 4>(ctx, w, a, c, m, n, k);
+    }
 }
 
 template <typename F, int MT>
@@ -374,33 +382,36 @@ skn_family register_family(few_init);
 
 // Every sixteen columns read all the activations and unpack for themselves, so that the time here grows with the row blocks where the
 // other kernels' hardly does: what they gain on three launches is lost again from so many superblocks of sixteen columns per compute unit
-// on (16, 32, 48, 64 rows; 0: not found up to 196).  us per call, others | these: Q4_K 32 x 12000 x 4096 (47) 18.7 | 15.8, 32 x 14336 x 4096
+// on (16, 32, 48, 64 rows, more in groups of 64; 0: not found up to 196).  us per call, others | these: Q4_K 32 x 12000 x 4096 (47) 18.7 | 15.8, 32 x 14336 x 4096
 // (56) 19.7 | 20.4, 41 x 6000 x 6144 (35) 20.6 | 19.2, 41 x 14336 x 4096 20.9 | 26.2; Q5_K 32 x 14336 x 4096 22.1 | 22.0, 41 x 14336 x 4096 26.9 | 28.1;
 // Q6_K 41 x 14336 x 4096 33.7 | 30.6, 57 x 14336 x 4096 33.6 | 40.5; Q8_0 41 x 14336 x 4096 29.0 | 28.9, 32 x 14336 x 14336 (196) 74 | 85; Q4_0 (whose
 // quants take three times Q4_K's instructions) 16 x 6000 x 6144 17.8 | 15.6, 16 x 14336 x 4096 18.7 | 19.3.  Over a single round of compute units
 // 64 rows hold out longer: 64 x 4096 x 11008 (43) Q4_K 24.8 | 23.3, Q8_0 28.7 | 23.5, against 57 x 6000 x 6144 21.2 | 27.3, 25.6 | 26.4.
-// Q4_K and Q6_K of more than 32 rows, up to 4096 elements and a round of tiles or more stay with the others although this is the faster path
-// (41 x 4096 x 4096 15.5 | 9.7 and 19.3 | 10.7): the number of launches that such products take is held fixed by tests.  Options that fix how k is divided mean the others.
+// More than 64 rows: Q5_K 128 x 2700 x 2816 (15) 18.2 | 16.6, 512 x 2000 x 1024 (16) 14.0 | 13.9; Q6_K 700 x 2000 x 1024 (21) 24.5 | 19.0; Q8_0 333 x
+// 4096 x 1024 (24) 16.8 | 15.2, 256 x 2700 x 2816 (29) 22.1 | 21.3; Q4_0 512 x 2000 x 1024 13.2 | 12.7, 256 x 2700 x 2816 19.4 | 21.1; Q4_K 160 x 1000 x 2048
+// (6) 16.4 | 6.8, 200 x 1000 x 2048 (8) 16.4 | 6.9, 512 x 2000 x 1024 13.8 | 13.4.
+// Q4_K and Q6_K of 33 to 64 rows, up to 4096 elements and a round of tiles or more stay with the others although this is the faster path
+// (41 x 4096 x 4096 15.5 | 9.7 and 19.3 | 10.7): the number of launches that such products take is held fixed by tests, as is Q4_K's 200 x 1024 x 2048.  Options that fix how k is divided mean the others.
 bool skn_gemm_few_ok(const skn_ctx* ctx, int type, const void* w, int n, int k, int m) {
     int bytes;
     struct {
-        int rows[4];
+        int rows[5];
     } most;
     switch (type) {
-        case SKN_TYPE_Q4_K: bytes = FewK<false>::kBytes, most = {{0, 48, 36, 20}}; break;
-        case SKN_TYPE_Q5_K: bytes = FewK<true>::kBytes, most = {{0, 56, 40, 20}}; break;
-        case SKN_TYPE_Q6_K: bytes = FewQ6K::kBytes, most = {{0, 0, 60, 24}}; break;
-        case SKN_TYPE_Q8_0: bytes = FewQ80::kBytes, most = {{0, 80, 50, 24}}; break;
-        case SKN_TYPE_Q4_0: bytes = FewQ40::kBytes, most = {{45, 33, 33, 20}}; break;
+        case SKN_TYPE_Q4_K: bytes = FewK<false>::kBytes, most = {{0, 48, 36, 20, 7}}; break;
+        case SKN_TYPE_Q5_K: bytes = FewK<true>::kBytes, most = {{0, 56, 40, 20, 15}}; break;
+        case SKN_TYPE_Q6_K: bytes = FewQ6K::kBytes, most = {{0, 0, 60, 24, 20}}; break;
+        case SKN_TYPE_Q8_0: bytes = FewQ80::kBytes, most = {{0, 80, 50, 24, 24}}; break;
+        case SKN_TYPE_Q4_0: bytes = FewQ40::kBytes, most = {{45, 33, 33, 20, 16}}; break;
         default: return false;
     }
-    if (ctx->opt_gemm_tile != 0 || ctx->opt_gemm_split != 0 || ctx->opt_test_gemm_no_parts || ctx->opt_gemm_q6k_fused != 1 || m <= 0 || m > 64 || n <= 0 || k <= 0 || k % 256 != 0 || k > 16384 ||
+    if (ctx->opt_gemm_tile != 0 || ctx->opt_gemm_split != 0 || ctx->opt_test_gemm_no_parts || ctx->opt_gemm_q6k_fused != 1 || m <= 0 ||  n <= 0 || k <= 0 || k % 256 != 0 || k > 16384 ||
         ((uintptr_t)w & (type == SKN_TYPE_Q6_K ? 1 : 15)) != 0 || (size_t)n * (k / 256) * bytes >= ((size_t)1 << 31))
         return false;
-    const int blocks = (m + 15) / 16, tiles = (n + 15) / 16;
-    if (m > 32 && k <= 4096 && tiles >= ctx->compute_units && (type == SKN_TYPE_Q4_K || type == SKN_TYPE_Q6_K)) return false;
+    const int blocks = std::min((m + 15) / 16, 5), tiles = (n + 15) / 16, groups = (m + 63) / 64;
+    if (m > 32 && m <= 64 && k <= 4096 && tiles >= ctx->compute_units && (type == SKN_TYPE_Q4_K || type == SKN_TYPE_Q6_K)) return false;
     const int limit = blocks == 4 && tiles <= ctx->compute_units ? 45 : most.rows[blocks - 1];
-    return limit == 0 || (size_t)tiles * (k / 256) <= (size_t)limit * ctx->compute_units;
+    return limit == 0 || (size_t)tiles * groups * (k / 256) <= (size_t)limit * ctx->compute_units;
 }
 
 int skn_gemm_few(skn_ctx* ctx, int type, const void* w, int n, int k, const uint16_t* a_bf16, int m, float* c) {

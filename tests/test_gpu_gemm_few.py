@@ -46,6 +46,14 @@ def test_three_and_four_row_blocks_of_short_rows(hip, name, m, n, k):
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("m,n,k", [(65, 33, 512), (127, 40, 2304), (128, 16, 256), (129, 200, 1024), (333, 500, 512)])
+def test_more_rows_in_groups(hip, name, m, n, k):
+    """Groups of 48 and 64 rows, the last one ragged or nearly empty."""
+    t = FORMATS[name]
+    _check(hip, t, synth.weight(t, n, k, seed=n + k + t), n, k, synth.activation_bf16((m, k), seed=m + 1), m)
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
 def test_rows_far_apart_and_fields_over_their_range(hip, name):
     """Random bytes in every field but the scales (zero, subnormal and of both signs among them); rows of 1e30, of 1e-30 and of zeros,
     elements 2^40 apart in one row: the activations are taken as they are."""
