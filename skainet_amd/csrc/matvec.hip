@@ -872,41 +872,39 @@ __device__ __forceinline__ float q6k_dot4(uint32_t v, const float4& x, float s) 
     return s;
 }
 
+// One row after the other: with the rows of a wavefront side by side the fused kernels held 151 registers (one workgroup of eight
+// wavefronts per compute unit); x read from LDS once per row instead costs less than the wavefronts that were missing.
 template <int R>
 __device__ __forceinline__ void q6k_step(const Q6kLoads (&L)[R], const float4* __restrict__ xs, const float* __restrict__ ss,
                                          int s, int lane, int hsel, float (&acc)[R]) {
-    float S[R][4];
+    const float4 sx = reinterpret_cast<const float4*>(ss)[s * 64 + lane];
 #pragma unroll
-    for (int r = 0; r < R; r++) S[r][0] = S[r][1] = S[r][2] = S[r][3] = 0.f;
+    for (int r = 0; r < R; r++) {
+        if (r > 0) asm volatile("" : "+v"(lane), "+v"(acc[r - 1]));
+        float S[4] = {};
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        float4 xq[4];
+        for (int i = 0; i < 4; i++) {
+            float4 xq[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) xq[q] = xs[(s * 16 + 4 * q + i) * kXPitch + lane];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
+            for (int q = 0; q < 4; q++) xq[q] = xs[(s * 16 + 4 * q + i) * kXPitch + lane];
             const uint32_t la = L[r].la[i], lb = L[r].lb[i], h = L[r].h[i];
             const uint32_t v0 = (la & 0x0F0F0F0Fu) | ((h << 4) & 0x30303030u);
             const uint32_t v1 = (lb & 0x0F0F0F0Fu) | ((h << 2) & 0x30303030u);
             const uint32_t v2 = ((la >> 4) & 0x0F0F0F0Fu) | (h & 0x30303030u);
             const uint32_t v3 = ((lb >> 4) & 0x0F0F0F0Fu) | ((h >> 2) & 0x30303030u);
-            S[r][0] = q6k_dot4(v0, xq[0], S[r][0]);
-            S[r][1] = q6k_dot4(v1, xq[1], S[r][1]);
-            S[r][2] = q6k_dot4(v2, xq[2], S[r][2]);
-            S[r][3] = q6k_dot4(v3, xq[3], S[r][3]);
+            S[0] = q6k_dot4(v0, xq[0], S[0]);
+            S[1] = q6k_dot4(v1, xq[1], S[1]);
+            S[2] = q6k_dot4(v2, xq[2], S[2]);
+            S[3] = q6k_dot4(v3, xq[3], S[3]);
         }
-    }
-    const float4 sx = reinterpret_cast<const float4*>(ss)[s * 64 + lane];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
         // scales hsel, hsel + 2, hsel + 4, hsel + 6 of the half's eight
         const uint32_t w0 = L[r].sc.x >> (8 * hsel), w1 = L[r].sc.y >> (8 * hsel);
         const float c0 = (float)(int)(int8_t)(w0 & 0xFF), c1 = (float)(int)(int8_t)((w0 >> 16) & 0xFF);
         const float c2 = (float)(int)(int8_t)(w1 & 0xFF), c3 = (float)(int)(int8_t)((w1 >> 16) & 0xFF);
-        float v = c0 * (S[r][0] - sx.x);
-        v = fmaf(c1, S[r][1] - sx.y, v);
-        v = fmaf(c2, S[r][2] - sx.z, v);
-        v = fmaf(c3, S[r][3] - sx.w, v);
+        float v = c0 * (S[0] - sx.x);
+        v = fmaf(c1, S[1] - sx.y, v);
+        v = fmaf(c2, S[2] - sx.z, v);
+        v = fmaf(c3, S[3] - sx.w, v);
         acc[r] += L[r].ok ? h2f_bits(L[r].d) * v : 0.f;
     }
 }
