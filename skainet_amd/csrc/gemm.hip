@@ -193,18 +193,22 @@ __global__ __launch_bounds__(64 * R) void prep_a_frag_kernel(const skn_gemm_src 
     }
 }
 
-// The same preparation with a row spread over two wavefronts (k <= 16384): every element is read from memory once and
+// The same preparation with a row spread over four wavefronts (k <= 16384): every element is read from memory once and
 // stays in registers through the three steps that the one-wavefront-per-row kernel above makes three passes for (sum of
-// squares, largest magnitude, conversion), two rows per workgroup, twice as many workgroups.  Thread t of a row takes
-// tasks t, t + 128, ... (task = chunk c, nibble dword dw: four elements at 64 c + 4 dw and four at 64 c + 32 + 4 dw);
+// squares, largest magnitude, conversion), two rows per workgroup.  Thread t of a row takes
+// tasks t, t + 256, ... (task = chunk c, nibble dword dw: four elements at 64 c + 4 dw and four at 64 c + 32 + 4 dw);
 // its sixteen-byte pieces go straight to their place in the fragment order.  Consecutive row pairs go to workgroups of
 // one XCD (blockIdx % 8), so that the 128-byte lines they share are completed in one L2.
+// Bound by the chain of latencies up to some thousand rows: the norm's weights are asked for with the row, and two wavefronts of a
+// SIMD hide each other's.  us, two wavefronts a row and the weights asked for when the norm was known -> this: 512 rows of 4096 behind a
+// norm 8.6 -> 7.6, 41 rows 6.2 -> 4.8, 2000 rows of 8192 25.2 -> 22.9, 512 rows of 11008 11.8 -> 11.7.
 template <int NT, int SRC, bool SUMS>
-__global__ __launch_bounds__(256) void prep_a_rows_kernel(const skn_gemm_src src, _Float16* __restrict__ afrag,
+__global__ __launch_bounds__(512) void prep_a_rows_kernel(const skn_gemm_src src, _Float16* __restrict__ afrag,
                                                          float* __restrict__ inv_scale, _Float16* __restrict__ sfrag,
                                                          int m, int k) {
-    __shared__ float red_ss[2][2], red_mx[2][2];
-    const int tid = threadIdx.x, t = tid & 127, rw = tid >> 7, wv = (tid >> 6) & 1;
+    constexpr int T = 256;  // threads of a row
+    __shared__ float red_ss[2][4], red_mx[2][4];
+    const int tid = threadIdx.x, t = tid & (T - 1), rw = tid / T, wv = (tid >> 6) & 3;
     const int n_pairs = gridDim.x, per_xcd = n_pairs >> 3;
     const int pair = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     const int row = 2 * pair + rw;
@@ -214,10 +218,11 @@ __global__ __launch_bounds__(256) void prep_a_rows_kernel(const skn_gemm_src src
     const float* xf = (const float*)src.a + row_off;
     const uint16_t* xb = (const uint16_t*)src.a + row_off;
     float v[NT][8];
+    float4 glo[SRC == SKN_SRC_RMSNORM ? NT : 1], ghi[SRC == SKN_SRC_RMSNORM ? NT : 1];
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < NT; j++) {
-        const int task = min(t + 128 * j, tasks - 1), c = task >> 3, dw = task & 7;
+        const int task = min(t + T * j, tasks - 1), c = task >> 3, dw = task & 7;
         const int e0 = 64 * c + 4 * dw;
         if (SRC == SKN_SRC_BF16) {
             const u32x2 lo = *reinterpret_cast<const u32x2*>(xb + e0), hi = *reinterpret_cast<const u32x2*>(xb + e0 + 32);
@@ -229,7 +234,11 @@ __global__ __launch_bounds__(256) void prep_a_rows_kernel(const skn_gemm_src src
             const float4 lo = *reinterpret_cast<const float4*>(xf + e0), hi = *reinterpret_cast<const float4*>(xf + e0 + 32);
             v[j][0] = lo.x, v[j][1] = lo.y, v[j][2] = lo.z, v[j][3] = lo.w;
             v[j][4] = hi.x, v[j][5] = hi.y, v[j][6] = hi.z, v[j][7] = hi.w;
-            if (SRC == SKN_SRC_RMSNORM && t + 128 * j < tasks)
+            if constexpr (SRC == SKN_SRC_RMSNORM) {
+                glo[j] = *reinterpret_cast<const float4*>((const float*)src.b + e0);
+                ghi[j] = *reinterpret_cast<const float4*>((const float*)src.b + e0 + 32);
+            }
+            if (SRC == SKN_SRC_RMSNORM && t + T * j < tasks)
                 ss += ((lo.x * lo.x + lo.y * lo.y) + (lo.z * lo.z + lo.w * lo.w)) + ((hi.x * hi.x + hi.y * hi.y) + (hi.z * hi.z + hi.w * hi.w));
         }
     }
@@ -238,20 +247,16 @@ __global__ __launch_bounds__(256) void prep_a_rows_kernel(const skn_gemm_src src
         ss = wave_sum(ss);
         if ((tid & 63) == 0) red_ss[rw][wv] = ss;
         __syncthreads();
-        r = 1.0f / sqrtf((red_ss[rw][0] + red_ss[rw][1]) / (float)k + src.eps);
+        r = 1.0f / sqrtf(((red_ss[rw][0] + red_ss[rw][1]) + (red_ss[rw][2] + red_ss[rw][3])) / (float)k + src.eps);
     }
     // the bf16 values the GEMM is defined on (fp32 sources: rounded to nearest even here), and their largest magnitude
     float mx = 0.f;
 #pragma unroll
     for (int j = 0; j < NT; j++) {
         if (SRC != SKN_SRC_BF16) {
-            const int task = min(t + 128 * j, tasks - 1), c = task >> 3, dw = task & 7;
-            float4 glo = make_float4(1.f, 1.f, 1.f, 1.f), ghi = glo;
-            if (SRC == SKN_SRC_RMSNORM) {
-                glo = *reinterpret_cast<const float4*>((const float*)src.b + 64 * c + 4 * dw);
-                ghi = *reinterpret_cast<const float4*>((const float*)src.b + 64 * c + 32 + 4 * dw);
-            }
-            const float g[8] = {glo.x, glo.y, glo.z, glo.w, ghi.x, ghi.y, ghi.z, ghi.w};
+            const float4 gl = SRC == SKN_SRC_RMSNORM ? glo[SRC == SKN_SRC_RMSNORM ? j : 0] : make_float4(1.f, 1.f, 1.f, 1.f);
+            const float4 gh = SRC == SKN_SRC_RMSNORM ? ghi[SRC == SKN_SRC_RMSNORM ? j : 0] : make_float4(1.f, 1.f, 1.f, 1.f);
+            const float g[8] = {gl.x, gl.y, gl.z, gl.w, gh.x, gh.y, gh.z, gh.w};
 #pragma unroll
             for (int x = 0; x < 8; x++) {
                 const float y = SRC == SKN_SRC_RMSNORM ? v[j][x] * r * g[x] : v[j][x];
@@ -267,7 +272,7 @@ __global__ __launch_bounds__(256) void prep_a_rows_kernel(const skn_gemm_src src
     mx = wave_max(mx);
     if ((tid & 63) == 0) red_mx[rw][wv] = mx;
     __syncthreads();
-    mx = real ? fmaxf(red_mx[rw][0], red_mx[rw][1]) : 0.f;
+    mx = real ? fmaxf(fmaxf(red_mx[rw][0], red_mx[rw][1]), fmaxf(red_mx[rw][2], red_mx[rw][3])) : 0.f;
     int e = 9;  // a zero row keeps scale 1
     if (mx > 0.f) e = (int)((__float_as_uint(mx) >> 23) & 0xFF) - 127;
     e = max(e, -100);
@@ -277,7 +282,7 @@ __global__ __launch_bounds__(256) void prep_a_rows_kernel(const skn_gemm_src src
     u32x4* out = reinterpret_cast<u32x4*>(afrag) + (size_t)mb * nch * 256 + rr;
 #pragma unroll
     for (int j = 0; j < NT; j++) {
-        const int task = t + 128 * j, c = task >> 3, dw = task & 7;
+        const int task = t + T * j, c = task >> 3, dw = task & 7;
         _Float16 l[4], u[4];
 #pragma unroll
         for (int x = 0; x < 4; x++) l[x] = (_Float16)(v[j][x] * scale), u[x] = (_Float16)(v[j][4 + x] * scale);
@@ -313,12 +318,12 @@ template <int SRC, bool SUMS>
 void launch_prep(skn_ctx* ctx, const skn_gemm_src& src, _Float16* afrag, float* isc, _Float16* sfrag, int m, int m_pad, int k) {
     // (m_pad is a multiple of 32: the pair count divides by the eight XCDs its workgroups are dealt to)
     if (k <= 16384 && m_pad % 16 == 0) {
-        const dim3 grid(m_pad / 2), block(256);
-        const int nt = (k / 8 + 127) / 128;
-        if (nt <= 4) skn_launch(ctx, prep_a_rows_kernel<4, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
-        else if (nt <= 8) skn_launch(ctx, prep_a_rows_kernel<8, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
-        else if (nt <= 12) skn_launch(ctx, prep_a_rows_kernel<12, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
-        else skn_launch(ctx, prep_a_rows_kernel<16, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
+        const dim3 grid(m_pad / 2), block(512);
+        const int nt = (k / 8 + 255) / 256;
+        if (nt <= 2) skn_launch(ctx, prep_a_rows_kernel<2, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
+        else if (nt <= 4) skn_launch(ctx, prep_a_rows_kernel<4, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
+        else if (nt <= 6) skn_launch(ctx, prep_a_rows_kernel<6, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
+        else skn_launch(ctx, prep_a_rows_kernel<8, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
     } else {
         skn_launch(ctx, prep_a_frag_kernel<4, SRC, SUMS>, dim3(m_pad / 4), dim3(256), 0, src, afrag, isc, sfrag, m, k);
     }

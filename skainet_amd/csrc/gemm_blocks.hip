@@ -40,10 +40,15 @@ __global__ __launch_bounds__(256) void prep_blocks_kernel(const skn_gemm_src src
     const int pieces = k >> 3;
     const size_t off = (size_t)(real ? row : 0) * k;
     float v[NT][8];
+    float4 g0[SRC == SKN_SRC_RMSNORM ? NT : 1], g1[SRC == SKN_SRC_RMSNORM ? NT : 1];  // (asked for with the row)
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < NT; j++) {
         const int p = min(tid + 256 * j, pieces - 1);
+        if constexpr (SRC == SKN_SRC_RMSNORM) {
+            const float4* g = reinterpret_cast<const float4*>((const float*)src.b + 8 * p);
+            g0[j] = g[0], g1[j] = g[1];
+        }
         if (SRC == SKN_SRC_BF16) {
             const u32x2* x = reinterpret_cast<const u32x2*>((const uint16_t*)src.a + off + 8 * p);
             const u32x2 a = x[0], b = x[1];
@@ -58,15 +63,14 @@ __global__ __launch_bounds__(256) void prep_blocks_kernel(const skn_gemm_src src
                 ss += ((a.x * a.x + a.y * a.y) + (a.z * a.z + a.w * a.w)) + ((b.x * b.x + b.y * b.y) + (b.z * b.z + b.w * b.w));
         }
     }
-    if (SRC == SKN_SRC_RMSNORM) {
+    if constexpr (SRC == SKN_SRC_RMSNORM) {
         ss = wave_sum(ss);
         if ((tid & 63) == 0) red[tid >> 6] = ss;
         __syncthreads();
         const float r = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)k + src.eps);
 #pragma unroll
         for (int j = 0; j < NT; j++) {
-            const float4* g = reinterpret_cast<const float4*>((const float*)src.b + 8 * min(tid + 256 * j, pieces - 1));
-            const float4 a = g[0], b = g[1];
+            const float4 a = g0[j], b = g1[j];
             const float gw[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
             for (int i = 0; i < 8; i++) v[j][i] = v[j][i] * r * gw[i];
