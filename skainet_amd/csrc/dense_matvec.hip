@@ -35,9 +35,52 @@ struct XPlanes {
     __device__ __forceinline__ float& at(int e) const { return reinterpret_cast<float*>(&quad(e >> 2))[e & 3]; }
 };
 
+// What the staging reads first, asked for ahead of the weights: requests are answered in order, so that behind the first weights
+// the input came no sooner than they did, and each vector that was asked for when it was needed cost another round trip before the
+// first multiplication.  Quads tid, tid + T, ... up to RQ; longer inputs read the rest as they go.  us, before -> now: 8192 x 2048 behind a
+// norm 10.2 -> 9.4, behind a sum and a norm 12.4 -> 10.9, 2624 x 2048 8.0 -> 7.2, 2048 x 2048 5.2 -> 4.6; a decode step of six layers of width
+// 2048 with side tables 15 us less, of eight with a delta rule 10 us less.  (The partials of a merge too, or the input of the columns beside
+// a mixer: 0.4 and 1.1 us more.)
+template <int MODE, int T>
+struct Ahead {
+    static constexpr bool kAdd = MODE == SKN_XSRC_ADD_NORM, kNorm = MODE == SKN_XSRC_GROUP_NORM || kAdd, kPlain = MODE == SKN_XSRC_PLAIN;
+    static constexpr int RQ = kPlain ? 4 : kNorm ? 2 : 1;
+    float4 x[RQ], w[kNorm ? RQ : 1], y[kAdd ? RQ : 1], yw[kAdd ? RQ : 1];
+    __device__ __forceinline__ void request(const skn_matvec_src& s) {
+        const int quads = kNorm ? (s.k0 + 3) >> 2 : s.k0 >> 2;
+#pragma unroll
+        for (int i = 0; i < RQ; i++) {
+            const int q = threadIdx.x + i * T;
+            if ((!kPlain && !kNorm) || q >= quads) continue;
+            if constexpr (kAdd) y[i] = reinterpret_cast<const float4*>(s.add)[q], yw[i] = reinterpret_cast<const float4*>(s.add_w)[q];
+            x[i] = reinterpret_cast<const float4*>(s.x0)[q];
+            if constexpr (kNorm) w[i] = reinterpret_cast<const float4*>(s.norm_w)[q];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+};
+
+// f(q, i): every quad of the thread's, i its place in Ahead (a constant) or -1
+template <int RQ, int T, int I = 0, typename F>
+__device__ __forceinline__ void each_quad(int quads, F&& f) {
+    if constexpr (I < RQ) {
+        const int q = threadIdx.x + I * T;
+        if (q < quads) f(q, std::integral_constant<int, I>{});
+        each_quad<RQ, T, I + 1>(quads, f);
+    } else {
+        for (int q = threadIdx.x + RQ * T; q < quads; q += T) f(q, std::integral_constant<int, -1>{});
+    }
+}
+
+template <int I, int N>
+__device__ __forceinline__ float4 ahead_or(std::integral_constant<int, I>, const float4 (&ahead)[N], const float* from, int q) {
+    if constexpr (I >= 0) return ahead[I];
+    else return reinterpret_cast<const float4*>(from)[q];
+}
+
 template <int T>
-__device__ __forceinline__ void stage_group_norm(const skn_matvec_src& s, const XPlanes& xs, float* red) {
-    constexpr int kWaves = T / 64;
+__device__ __forceinline__ void stage_group_norm(const skn_matvec_src& s, const Ahead<SKN_XSRC_GROUP_NORM, T>& ahead, const XPlanes& xs, float* red) {
+    constexpr int kWaves = T / 64, kRQ = Ahead<SKN_XSRC_GROUP_NORM, T>::RQ;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, quads = (s.k0 + 3) >> 2, gs = s.k0 / s.groups;
     // (pitches are multiples of 64 elements and their padding is zero: the last quad may be read whole)
     const bool few = s.groups <= 8 && (gs & 3) == 0;
@@ -46,14 +89,14 @@ __device__ __forceinline__ void stage_group_norm(const skn_matvec_src& s, const 
 #pragma unroll
         for (int g = 0; g < 8; g++) ss[g] = 0.f;
         const float inv_quads = 4.0f / (float)gs;
-        for (int q = tid; q < quads; q += T) {
-            const float4 v = reinterpret_cast<const float4*>(s.x0)[q];
+        each_quad<kRQ, T>(quads, [&](int q, auto i) __attribute__((always_inline)) {
+            const float4 v = ahead_or(i, ahead.x, s.x0, q);
             xs.quad(q) = v;
             const float d = (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
             const int g = (int)(((float)q + 0.5f) * inv_quads);
 #pragma unroll
-            for (int i = 0; i < 8; i++) ss[i] += i == g ? d : 0.f;
-        }
+            for (int n = 0; n < 8; n++) ss[n] += n == g ? d : 0.f;
+        });
 #pragma unroll
         for (int g = 0; g < 8; g++)
             if (g < s.groups) {
@@ -67,11 +110,11 @@ __device__ __forceinline__ void stage_group_norm(const skn_matvec_src& s, const 
             red[8 * kWaves + tid] = 1.0f / sqrtf(t / (float)gs + s.eps);
         }
         __syncthreads();
-        for (int q = tid; q < quads; q += T) {
+        each_quad<kRQ, T>(quads, [&](int q, auto i) __attribute__((always_inline)) {
             const float r = red[8 * kWaves + (int)(((float)q + 0.5f) * inv_quads)];
-            const float4 v = xs.quad(q), g = reinterpret_cast<const float4*>(s.norm_w)[q];
+            const float4 v = xs.quad(q), g = ahead_or(i, ahead.w, s.norm_w, q);
             xs.quad(q) = make_float4(v.x * r * g.x, v.y * r * g.y, v.z * r * g.z, v.w * r * g.w);
-        }
+        });
         return;
     }
     for (int e = tid; e < s.k0; e += T) xs.at(e) = s.x0[e];
@@ -103,39 +146,50 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 
 // (pitches are multiples of 64 elements and their padding is zero, as in stage_group_norm; a thread's quads stay its own)
 template <int T>
-__device__ __forceinline__ void stage_add_norm(const skn_matvec_src& s, const XPlanes& xs, float* red) {
-    const int tid = threadIdx.x, quads = (s.k0 + 3) >> 2;
+__device__ __forceinline__ void stage_add_norm(const skn_matvec_src& s, const Ahead<SKN_XSRC_ADD_NORM, T>& ahead, const XPlanes& xs, float* red) {
+    constexpr int kRQ = Ahead<SKN_XSRC_ADD_NORM, T>::RQ;
+    const int quads = (s.k0 + 3) >> 2;
     auto square = [](const float4& v) { return (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w); };
     float ss = 0.f;
-    for (int q = tid; q < quads; q += T) {
-        const float4 v = reinterpret_cast<const float4*>(s.add)[q];
+    each_quad<kRQ, T>(quads, [&](int q, auto i) __attribute__((always_inline)) {
+        const float4 v = ahead_or(i, ahead.y, s.add, q);
         xs.quad(q) = v;
         ss += square(v);
-    }
+    });
     const float ry = 1.0f / sqrtf(block_sum<T>(ss, red) / (float)s.k0 + s.eps);
     ss = 0.f;
-    for (int q = tid; q < quads; q += T) {
-        const float4 y = xs.quad(q), x = reinterpret_cast<const float4*>(s.x0)[q], g = reinterpret_cast<const float4*>(s.add_w)[q];
+    each_quad<kRQ, T>(quads, [&](int q, auto i) __attribute__((always_inline)) {
+        const float4 y = xs.quad(q), x = ahead_or(i, ahead.x, s.x0, q);
+        const float4 g = ahead_or(i, ahead.yw, s.add_w, q);
         const float4 v = make_float4(fmaf(y.x * ry, g.x, x.x), fmaf(y.y * ry, g.y, x.y), fmaf(y.z * ry, g.z, x.z), fmaf(y.w * ry, g.w, x.w));
         xs.quad(q) = v;
         if (blockIdx.x == 0) reinterpret_cast<float4*>(s.x_out)[q] = v;
         ss += square(v);
-    }
+    });
     const float rx = 1.0f / sqrtf(block_sum<T>(ss, red + T / 64) / (float)s.k0 + s.eps);
-    for (int q = tid; q < quads; q += T) {
-        const float4 v = xs.quad(q), g = reinterpret_cast<const float4*>(s.norm_w)[q];
+    each_quad<kRQ, T>(quads, [&](int q, auto i) __attribute__((always_inline)) {
+        const float4 v = xs.quad(q), g = ahead_or(i, ahead.w, s.norm_w, q);
         xs.quad(q) = make_float4(v.x * rx * g.x, v.y * rx * g.y, v.z * rx * g.z, v.w * rx * g.w);
-    }
+    });
 }
 
-// red: heads x splits weights
-template <int T>
-__device__ __forceinline__ void stage_merge(const skn_matvec_src& s, const XPlanes& xs, float* red) {
+// red: heads x splits weights.  weights(): asks for the first weights of the product; the maxima, sums and partials that are needed
+// first are asked for ahead of them (see Ahead).
+template <int T, typename F>
+__device__ __forceinline__ void stage_merge(const skn_matvec_src& s, const XPlanes& xs, float* red, F&& weights) {
     const int tid = threadIdx.x;
+    const bool quads = (s.dim & 3) == 0;
+    const int dq = s.dim >> 2;
+    const int64_t step = (int64_t)s.heads * s.dim_pad;
+    float2 ml0[kMaxSplits];
+#pragma unroll
+    for (int i = 0; i < kMaxSplits; i++) ml0[i] = reinterpret_cast<const float2*>(s.ml)[min(i, s.splits - 1) * s.heads + min(tid, s.heads - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+    weights();
     for (int h = tid; h < s.heads; h += T) {
         float2 ml[kMaxSplits];  // (all requested before the first is used)
 #pragma unroll
-        for (int i = 0; i < kMaxSplits; i++) ml[i] = reinterpret_cast<const float2*>(s.ml)[min(i, s.splits - 1) * s.heads + h];
+        for (int i = 0; i < kMaxSplits; i++) ml[i] = h == tid ? ml0[i] : reinterpret_cast<const float2*>(s.ml)[min(i, s.splits - 1) * s.heads + h];
         float m = s.sink ? 0.f : -INFINITY;
 #pragma unroll
         for (int i = 0; i < kMaxSplits; i++) m = fmaxf(m, ml[i].x);
@@ -151,9 +205,7 @@ __device__ __forceinline__ void stage_merge(const skn_matvec_src& s, const XPlan
             if (i < s.splits) red[h * s.splits + i] = ml[i].x * inv;
     }
     __syncthreads();
-    if ((s.dim & 3) == 0) {
-        const int dq = s.dim >> 2;
-        const int64_t step = (int64_t)s.heads * s.dim_pad;
+    if (quads) {
         for (int q = tid; q < s.heads * dq; q += T) {
             const int h = q / dq, c = q - h * dq;
             const float* p = s.x0 + (int64_t)h * s.dim_pad + 4 * c;
@@ -207,14 +259,17 @@ __global__ __launch_bounds__(T) void dense_matvec_kernel(const W* __restrict__ w
             for (int u = 0; u < kU; u++) buf[r][u] = row[min((t * kU + u) * 64 + lane, pieces - 1)];  // (past the end: times a zero of x)
         }
     };
-    fetch(cur, min(grp, groups - 1), 0);
+    constexpr int kRQ = Ahead<MODE, T>::RQ;
+    Ahead<MODE, T> ahead;
+    ahead.request(src);
+    if constexpr (MODE != SKN_XSRC_MERGE) fetch(cur, min(grp, groups - 1), 0);
 
     // ---- staging ----
-    if constexpr (MODE == SKN_XSRC_GROUP_NORM) stage_group_norm<T>(src, xs, reinterpret_cast<float*>(lds4 + 2 * plane));
-    else if constexpr (MODE == SKN_XSRC_ADD_NORM) stage_add_norm<T>(src, xs, reinterpret_cast<float*>(lds4 + 2 * plane));
-    else if constexpr (MODE == SKN_XSRC_MERGE) stage_merge<T>(src, xs, reinterpret_cast<float*>(lds4 + 2 * plane));
+    if constexpr (MODE == SKN_XSRC_GROUP_NORM) stage_group_norm<T>(src, ahead, xs, reinterpret_cast<float*>(lds4 + 2 * plane));
+    else if constexpr (MODE == SKN_XSRC_ADD_NORM) stage_add_norm<T>(src, ahead, xs, reinterpret_cast<float*>(lds4 + 2 * plane));
+    else if constexpr (MODE == SKN_XSRC_MERGE) stage_merge<T>(src, xs, reinterpret_cast<float*>(lds4 + 2 * plane), [&]() __attribute__((always_inline)) { fetch(cur, min(grp, groups - 1), 0); });
     else {
-        for (int q = tid; q < src.k0 >> 2; q += T) xs.quad(q) = reinterpret_cast<const float4*>(src.x0)[q];
+        each_quad<kRQ, T>(src.k0 >> 2, [&](int q, auto i) __attribute__((always_inline)) { xs.quad(q) = ahead_or(i, ahead.x, src.x0, q); });
         for (int e = (src.k0 & ~3) + tid; e < src.k0; e += T) xs.at(e) = src.x0[e];
     }
     if (src.x1) {
