@@ -136,7 +136,7 @@ __global__ __launch_bounds__(S::kThreads) void dense_gemm_kernel(const uint8_t* 
     // The tile goes through LDS (register x of lane 32 h + n: output row 8 (x / 4) + 4 h + x % 4 of its block, token n), so
     // that the epilogue is one short loop in which a thread has four consecutive outputs of one token and the threads
     // of a wavefront store whole rows of the tile.
-    constexpr int kPitch = S::kPitch, kQuads = kRowsW / 4;
+    constexpr int kPitch = S::kPitch, kQuads = kRowsW / 4, kTurn = S::kThreads / kQuads;  // (tokens at a time; threads past a whole number have none)
     float* tile_c = reinterpret_cast<float*>(lds);
     constexpr int kPart = 32 * WM * kPitch;  // floats of a group's pass
     const int q4 = 4 * (tid % kQuads), row = n0 + q4;  // (this thread's four rows are the same in every turn)
@@ -157,8 +157,8 @@ __global__ __launch_bounds__(S::kThreads) void dense_gemm_kernel(const uint8_t* 
                 *reinterpret_cast<float4*>(tile_c + group * kPart + (32 * wv_m + r32) * kPitch + wn + 32 * i + 8 * g + 4 * h) =
                     make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
         __syncthreads();
-        if (left <= 0) continue;
-        for (int tl = tid / kQuads; tl < 32 * WM; tl += S::kThreads / kQuads) {
+        if (left <= 0 || tid >= kTurn * kQuads) continue;
+        for (int tl = tid / kQuads; tl < 32 * WM; tl += kTurn) {
             const int t = m0 + (tl >> 5) * 32 * TM + 32 * j + (tl & 31);
             if (t >= m) continue;
             float4 c = *reinterpret_cast<const float4*>(tile_c + tl * kPitch + q4);
@@ -210,6 +210,8 @@ using Tile32x64Split = Shape<1, 2, 1, 1, 3, 4>;  // for few outputs: more and sh
 using Tile128x64 = Shape<2, 2, 2, 1, 3>;
 using Tile128x128 = Shape<2, 2, 2, 2, 2>;
 using Tile256x256 = Shape<4, 2, 2, 4, 2>;
+using Tile256x192 = Shape<4, 2, 2, 3, 2>;
+using Tile128x192 = Shape<2, 2, 2, 3, 2>;
 
 template <typename T, typename S>
 int launch_gemm(skn_ctx* ctx, const skn_dense_mat& w, const void* a, int lda, int m, const skn_dense_out& out) {
@@ -229,11 +231,15 @@ int pick_gemm(skn_ctx* ctx, const skn_dense_mat& w, const void* a, int lda, int 
         int rows_a, rows_w, resident;
         float alone, full;
     };
-    const Cost costs[4] = {{64, 64, 3, 25.f, 40.f}, {128, 64, 2, 31.f, 48.f}, {128, 128, 2, 59.f, 87.f}, {256, 256, 1, 145.f, 145.f}};
+    // (192 rows of weights fill the rounds of widths that 128 and 256 leave a third of idle.  us, the others | with them: 1000 x 10752 x 2048
+    // 101.7 | 84.4 in 256 x 192, 1000 x 18496 x 2048 159 | 153, 2048 x 5120 x 2048 85.4 | 65.6; not alone on a compute unit, 2048 x 3072 24.8 | 27.5)
+    const Cost costs[7] = {{64, 64, 3, 25.f, 40.f},     {128, 64, 2, 31.f, 48.f},    {128, 128, 2, 59.f, 87.f},  {256, 256, 1, 145.f, 145.f},
+                           {0, 0, 0, 0.f, 0.f},         {256, 192, 1, 116.f, 116.f}, {128, 192, 2, 80.f, 118.f}};
     int best = 0;
     float best_time = INFINITY;
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < 7; i++) {
         const Cost& c = costs[i];
+        if (c.resident == 0) continue;  // (the divided tile has a rule of its own below)
         const int tiles = ((m + c.rows_a - 1) / c.rows_a) * ((w.rows + c.rows_w - 1) / c.rows_w), round = c.resident * ctx->compute_units;
         const int rest = tiles % round;
         const float time = tiles / round * c.full + (rest == 0 ? 0.f : rest <= ctx->compute_units ? c.alone : c.full);
@@ -246,6 +252,8 @@ int pick_gemm(skn_ctx* ctx, const skn_dense_mat& w, const void* a, int lda, int 
         case 1: return launch_gemm<T, Tile128x64>(ctx, w, a, lda, m, out);
         case 2: return launch_gemm<T, Tile128x128>(ctx, w, a, lda, m, out);
         case 4: return launch_gemm<T, Tile32x64Split>(ctx, w, a, lda, m, out);
+        case 5: return launch_gemm<T, Tile256x192>(ctx, w, a, lda, m, out);
+        case 6: return launch_gemm<T, Tile128x192>(ctx, w, a, lda, m, out);
         default: return launch_gemm<T, Tile256x256>(ctx, w, a, lda, m, out);
     }
 }
@@ -262,6 +270,8 @@ int allow_all(skn_ctx* ctx) {
     SKN_TRY((allow_lds<T, Tile32x64Split>(ctx)));
     SKN_TRY((allow_lds<T, Tile128x64>(ctx)));
     SKN_TRY((allow_lds<T, Tile128x128>(ctx)));
+    SKN_TRY((allow_lds<T, Tile256x192>(ctx)));
+    SKN_TRY((allow_lds<T, Tile128x192>(ctx)));
     return allow_lds<T, Tile256x256>(ctx);
 }
 
