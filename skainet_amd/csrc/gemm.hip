@@ -2300,8 +2300,9 @@ extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n,
                     "skn_gemm_q: Q4_K weights must be 16-byte aligned, activations 8-byte aligned");
         const skn_gemm_seg seg = {w_dev, n, c_dev, 0};
         const skn_gemm_src src = {SKN_SRC_BF16, a_bf16_dev, nullptr, 0.f};
-        // up to 32 rows: the kernel for blocks of 32, whose tile has as many (us per call, this | that: 2 x 4096 x 4096 14.2 | 12.8, 16 x
-        // 4096 x 4096 14.3 | 12.3, 8 x 1000 x 2048 12.5 | 10.7; on two row blocks 41 x 4096 x 4096 15.2 | 14.9, 64 x 11008 x 4096 20.1 | 23.8)
+        // up to 32 rows (17 to 32 of matrices too large for the path above): the kernel for blocks of 32, whose tile has as many (us per
+        // call, this | that: 17 x 14336 x 4096 20.1 | 19.0, 17 x 8192 x 11008 30.3 | 27.9, 32 x 28672 x 4096 28.5 | 26.4, 32 x 11008 x 8192
+        // 29.5 | 29.3; on two row blocks 41 x 4096 x 4096 15.2 | 14.9, 64 x 11008 x 4096 20.1 | 23.8)
         if (ctx->opt_gemm_tile == 0 && m <= 32 && skn_gemm_blocks_ok(ctx, ggml_type, w_dev, n, k, m))
             return skn_gemm_blocks_multi(ctx, &ggml_type, &seg, 1, k, src, m);
         return skn_gemm_q4k_multi(ctx, &seg, 1, k, src, m);

@@ -1,5 +1,5 @@
 // Prompt products of weights in blocks of 32 (Q8_0, Q4_0, Q4_1, Q5_0, Q5_1, Q5_K; Q4_K too, which skn_gemm_q sends here up to 32
-// rows) behind the activation sources of the Q4_K one (internal to the library).
+// rows where gemm_few.h declines) behind the activation sources of the Q4_K one (internal to the library).
 #pragma once
 #include "common.h"
 

@@ -1,5 +1,6 @@
 // Prompt GEMM for formats whose weights are d (q - zero) + m over blocks of 32 elements: Q8_0, Q4_0, Q4_1, Q5_0, Q5_1, the
-// sub-blocks of Q5_K, and those of Q4_K for up to 32 rows (above, Q4_K has kernels of its own in gemm.hip).
+// sub-blocks of Q5_K, and those of Q4_K for up to 32 rows (above, Q4_K has kernels of its own in gemm.hip; few rows of
+// matrices that are not too large go to gemm_few.hip).
 // C[m, n] = sum_k A[m, k] w[n, k], activations as in gemm.hip (bf16 rows scaled to fp16 by a power of two).
 //
 // Bound by the matrix cores and the vector ALUs together for many rows, by the weight stream for few.  What the general path
