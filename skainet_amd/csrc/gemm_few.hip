@@ -10,7 +10,7 @@
 // A workgroup keeps all of k for its sixteen columns: its eight (or four) wavefronts take superblocks of 256 in
 // turn and add their tiles through LDS.
 //
-// us per call, three launches -> this: Q4_K 16 x 4096 x 4096 11.8 -> 5.0, Q8_0 16 x 4096 x 4096 13.4 -> 6.3, Q6_K 41 x 4096 x 11008 34.9 -> 21.4 (weights
+// us per call, three launches -> this: Q4_K 16 x 4096 x 4096 11.8 -> 5.0, Q8_0 16 x 4096 x 4096 13.4 -> 6.3, Q6_K 41 x 4096 x 11008 33.7 -> 21.5 (weights
 // alone 7.5 at the rate of a copy), Q5_K 16 x 1000 x 1024 9.4 -> 4.6.  Error against 64 bits: not larger (1.1 against 1.5e-7 of the
 // result in Q4_K at k = 11008, 0.95 against 1.05 in Q8_0): a superblock's sum is formed before it joins the total.
 #include "gemm_few.h"
@@ -35,21 +35,29 @@ __device__ __forceinline__ float f16_hi(uint32_t w) { return (float)__builtin_bi
 __device__ __forceinline__ uint32_t lds_u32(const uint8_t* p) { return *reinterpret_cast<const uint32_t*>(p); }
 __device__ __forceinline__ u32x2 lds_u32x2(const uint8_t* p) { return *reinterpret_cast<const u32x2*>(p); }
 
-// Four whole numbers of at most eight bits, one to a byte, as bf16: the upper halves of their fp32 forms.
+// Operands are quants times 2^-12: a block's sum of at most 32 products of up to 2^7 then stays in fp32's range for every finite
+// activation (as they are it leaves it from about 8e34 on although the result need not), and its scale brings the 2^12 back.
+constexpr float kUp = 0x1p12f;
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+// Four whole numbers of at most eight bits, one to a byte, as bf16: the upper halves of their fp32 forms, less twelve in the exponent
+// (zero stays zero: the subtraction stops there; Q8_0 8 x 4096 x 11008 11.4 us without it, 11.8 with, Q5_K 11.2, 12.0).
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+    const u16x2 x = __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(x, u16x2{12 << 7, 12 << 7}));
+}
 __device__ __forceinline__ u32x2 signed_bytes(uint32_t b) {
     const float f0 = (float)(int8_t)b, f1 = (float)(int8_t)(b >> 8), f2 = (float)(int8_t)(b >> 16), f3 = (float)(int8_t)(b >> 24);
-    return u32x2{__builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u),
-                 __builtin_amdgcn_perm(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u)};
+    return u32x2{bf16_pair(f0, f1), bf16_pair(f2, f3)};
 }
 __device__ __forceinline__ u32x2 unsigned_bytes(uint32_t b) {
     const float f0 = (float)(uint8_t)b, f1 = (float)(uint8_t)(b >> 8), f2 = (float)(uint8_t)(b >> 16), f3 = (float)(uint8_t)(b >> 24);
-    return u32x2{__builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u),
-                 __builtin_amdgcn_perm(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u)};
+    return u32x2{bf16_pair(f0, f1), bf16_pair(f2, f3)};
 }
 // Four numbers 0..15: as E4M3 a byte below sixteen is that many times 2^-9 (subnormals and the first binade are one straight line).
 __device__ __forceinline__ u32x2 nibble_bytes(uint32_t b) {
-    return u32x2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f, false)),
-                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f, true))};
+    return u32x2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f / kUp, false)),
+                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f / kUp, true))};
 }
 __device__ __forceinline__ bf16x8 operand(u32x2 lo, u32x2 hi) { return __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y}); }
 
@@ -65,7 +73,7 @@ struct FewK {
     };
     __device__ static __forceinline__ void head(const uint8_t* row, int g, Head& s) {
         const u32x4 h = *reinterpret_cast<const u32x4*>(row);
-        s.d = f16_lo(h[0]), s.dmin = f16_hi(h[0]);
+        s.d = f16_lo(h[0]) * kUp, s.dmin = f16_hi(h[0]) * kUp;
         s.sc[0] = h[1] & 0x3F3F3F3Fu, s.sc[1] = (h[3] & 0x0F0F0F0Fu) | ((h[1] >> 2) & 0x30303030u);
         s.mn[0] = h[2] & 0x3F3F3F3Fu, s.mn[1] = ((h[3] >> 4) & 0x0F0F0F0Fu) | ((h[2] >> 2) & 0x30303030u);
         if (FIVE) s.fifth = lds_u32x2(row + 16 + 8 * g);
@@ -90,10 +98,10 @@ struct FewQ80 {  // 34 bytes: d, 32 int8; block pairs are 17 dwords
         const uint8_t* p = row + 68 * (b >> 1);
         uint32_t x, y;
         if (b & 1) {
-            s = f16_hi(lds_u32(p + 32));
+            s = f16_hi(lds_u32(p + 32)) * kUp;
             x = lds_u32(p + 36 + 8 * g), y = lds_u32(p + 40 + 8 * g);
         } else {
-            s = f16_lo(lds_u32(p));
+            s = f16_lo(lds_u32(p)) * kUp;
             const uint32_t w0 = lds_u32(p + 8 * g), w1 = lds_u32(p + 4 + 8 * g), w2 = lds_u32(p + 8 + 8 * g);
             x = __builtin_amdgcn_alignbyte(w1, w0, 2), y = __builtin_amdgcn_alignbyte(w2, w1, 2);
         }
@@ -112,10 +120,10 @@ struct FewQ40 {  // 18 bytes: d, nibbles (low ones elements 0..15, high ones 16.
         const int at = 8 * (g & 1);
         u32x2 q;
         if (b & 1) {
-            s = f16_hi(lds_u32(p + 16)) * 0.0625f;
+            s = f16_hi(lds_u32(p + 16)) * (kUp / 16);
             q = u32x2{lds_u32(p + 20 + at), lds_u32(p + 24 + at)};
         } else {
-            s = f16_lo(lds_u32(p)) * 0.0625f;
+            s = f16_lo(lds_u32(p)) * (kUp / 16);
             const uint32_t w0 = lds_u32(p + at), w1 = lds_u32(p + 4 + at), w2 = lds_u32(p + 8 + at);
             q = u32x2{__builtin_amdgcn_alignbyte(w1, w0, 2), __builtin_amdgcn_alignbyte(w2, w1, 2)};
         }
@@ -131,11 +139,11 @@ struct FewQ6K {
     static constexpr int kBytes = 210, kPieces = 14, kPitch = 240;
     static constexpr bool kHalves = true;
     struct Head {
-        float d4;  // d / 4: the operands are 4 (q - 32)
+        float d4;  // d / 4 (times 2^12): the operands are 4 (q - 32)
         u32x4 sc;
     };
     __device__ static __forceinline__ void head(const uint8_t* row, int, Head& s) {
-        s.d4 = f16_hi(lds_u32(row + 220)) * 0.25f;
+        s.d4 = f16_hi(lds_u32(row + 220)) * (kUp / 4);
         s.sc = *reinterpret_cast<const u32x4*>(row + 192);
     }
     __device__ static __forceinline__ s16x4 sixteen(const uint8_t* row, const Head& H, int b, int t, int g, float& s) {
@@ -178,7 +186,7 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
 #pragma unroll
     for (int i = 0; i < MT; i++) total[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    const u32x4 ones_bits = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+    const u32x4 ones_bits = {0x39803980u, 0x39803980u, 0x39803980u, 0x39803980u};  // (2^-12)
     const bf16x8 ones = __builtin_bit_cast(bf16x8, ones_bits);
 
     // The tile's rows of a superblock: coalesced loads one superblock ahead, handed over through LDS of the wavefront's own (the lane

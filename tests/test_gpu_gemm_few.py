@@ -77,6 +77,28 @@ def test_rows_far_apart_and_fields_over_their_range(hip, name):
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("size", [2.0**127, 2.0**-125])
+def test_activations_at_either_end_of_their_range(hip, name, size):
+    """Largest finite activations with weights that bring the sums back into range (a block's sum of quants alone would leave it);
+    least normal ones with scales as large as the format has."""
+    t = FORMATS[name]
+    m, n, k = 18, 33, 512
+    be, bb = synth.BLOCK[t]
+    raw = np.frombuffer(synth.weight(t, n, k, seed=9).tobytes(), np.uint8).reshape(-1, bb).copy()
+    scale = np.float16(2.0**-20 if size > 1 else 1000.0)
+    at = 208 if name == "q6_k" else 0
+    for f in ((0, 2) if name in ("q4_k", "q5_k") else (at,)):
+        raw[:, f:f + 2] = np.full(len(raw), scale).view(np.uint8).reshape(-1, 2)
+    x = np.random.default_rng(t).uniform(0.5, 1.9, (m, k)).astype(np.float32) * np.float32(size)
+    a = synth.f32_to_bf16_bits(x)
+    got = hip.gemm_q_host(t, raw.reshape(-1), n, k, a, m).reshape(m, n)
+    wd = oracle_c.dequant(t, raw.reshape(-1)).astype(np.float64).reshape(n, k)
+    xd = oracle_np.bf16_to_f32(a).astype(np.float64).reshape(m, k)
+    bound = np.abs(xd) @ np.abs(wd).T * (4 if name in ("q4_k", "q5_k") else 1)
+    assert np.all(np.abs(got - xd @ wd.T) <= ROUNDINGS * 2.0**-24 * bound)
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
 def test_an_infinite_activation_reaches_its_row_alone(hip, name):
     t = FORMATS[name]
     m, n, k = 18, 33, 512
