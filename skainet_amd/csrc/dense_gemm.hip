@@ -232,7 +232,9 @@ int pick_gemm(skn_ctx* ctx, const skn_dense_mat& w, const void* a, int lda, int 
         float alone, full;
     };
     // (192 rows of weights fill the rounds of widths that 128 and 256 leave a third of idle.  us, the others | with them: 1000 x 10752 x 2048
-    // 101.7 | 84.4 in 256 x 192, 1000 x 18496 x 2048 159 | 153, 2048 x 5120 x 2048 85.4 | 65.6; not alone on a compute unit, 2048 x 3072 24.8 | 27.5)
+    // 101.7 | 84.4 in 256 x 192, 2048 x 5120 x 2048 85.4 | 65.6.  Only with four fifths of the last round:
+    // the next 128 x 128 tiles start as earlier ones end, so that theirs costs less than is reckoned here; prompts of 1444 whose products
+    // are 186 and some 370 tiles of 256 x 192, k = 576 to 2048: 1 to 7 % slower in 192 rows)
     const Cost costs[7] = {{64, 64, 3, 25.f, 40.f},     {128, 64, 2, 31.f, 48.f},    {128, 128, 2, 59.f, 87.f},  {256, 256, 1, 145.f, 145.f},
                            {0, 0, 0, 0.f, 0.f},         {256, 192, 1, 116.f, 116.f}, {128, 192, 2, 80.f, 118.f}};
     int best = 0;
@@ -242,6 +244,7 @@ int pick_gemm(skn_ctx* ctx, const skn_dense_mat& w, const void* a, int lda, int 
         if (c.resident == 0) continue;  // (the divided tile has a rule of its own below)
         const int tiles = ((m + c.rows_a - 1) / c.rows_a) * ((w.rows + c.rows_w - 1) / c.rows_w), round = c.resident * ctx->compute_units;
         const int rest = tiles % round;
+        if (c.rows_w == 192 && rest != 0 && 5 * rest < 4 * (rest <= ctx->compute_units ? ctx->compute_units : round)) continue;
         const float time = tiles / round * c.full + (rest == 0 ? 0.f : rest <= ctx->compute_units ? c.alone : c.full);
         if (time < best_time) best = i, best_time = time;
     }
