@@ -201,13 +201,15 @@ __global__ __launch_bounds__(64 * R) void prep_a_frag_kernel(const skn_gemm_src 
 // one XCD (blockIdx % 8), so that the 128-byte lines they share are completed in one L2.
 // Bound by the chain of latencies up to some thousand rows: the norm's weights are asked for with the row, and two wavefronts of a
 // SIMD hide each other's.  us, two wavefronts a row and the weights asked for when the norm was known -> this: 512 rows of 4096 behind a
-// norm 8.6 -> 7.6, 41 rows 6.2 -> 4.8, 2000 rows of 8192 25.2 -> 22.9, 512 rows of 11008 11.8 -> 11.7.
+// norm 7.9 -> 7.4, 41 rows 5.8 -> 5.0 (0.1 to 0.2 of them for the order of the squares below); without a norm 2000 rows of 8192 25.2 -> 22.9,
+// 512 rows of 11008 11.8 -> 11.7.
 template <int NT, int SRC, bool SUMS>
 __global__ __launch_bounds__(512) void prep_a_rows_kernel(const skn_gemm_src src, _Float16* __restrict__ afrag,
                                                          float* __restrict__ inv_scale, _Float16* __restrict__ sfrag,
                                                          int m, int k) {
     constexpr int T = 256;  // threads of a row
-    __shared__ float red_ss[2][4], red_mx[2][4];
+    __shared__ float red_ss[2][2], red_mx[2][4];
+    __shared__ float upper[SRC == SKN_SRC_RMSNORM ? 2 * NT * (T / 2) : 1];
     const int tid = threadIdx.x, t = tid & (T - 1), rw = tid / T, wv = (tid >> 6) & 3;
     const int n_pairs = gridDim.x, per_xcd = n_pairs >> 3;
     const int pair = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
@@ -219,7 +221,7 @@ __global__ __launch_bounds__(512) void prep_a_rows_kernel(const skn_gemm_src src
     const uint16_t* xb = (const uint16_t*)src.a + row_off;
     float v[NT][8];
     float4 glo[SRC == SKN_SRC_RMSNORM ? NT : 1], ghi[SRC == SKN_SRC_RMSNORM ? NT : 1];
-    float ss = 0.f;
+    float squares[SRC == SKN_SRC_RMSNORM ? NT : 1];
 #pragma unroll
     for (int j = 0; j < NT; j++) {
         const int task = min(t + T * j, tasks - 1), c = task >> 3, dw = task & 7;
@@ -237,17 +239,32 @@ __global__ __launch_bounds__(512) void prep_a_rows_kernel(const skn_gemm_src src
             if constexpr (SRC == SKN_SRC_RMSNORM) {
                 glo[j] = *reinterpret_cast<const float4*>((const float*)src.b + e0);
                 ghi[j] = *reinterpret_cast<const float4*>((const float*)src.b + e0 + 32);
+                squares[j] = ((lo.x * lo.x + lo.y * lo.y) + (lo.z * lo.z + lo.w * lo.w)) + ((hi.x * hi.x + hi.y * hi.y) + (hi.z * hi.z + hi.w * hi.w));
             }
-            if (SRC == SKN_SRC_RMSNORM && t + T * j < tasks)
-                ss += ((lo.x * lo.x + lo.y * lo.y) + (lo.z * lo.z + lo.w * lo.w)) + ((hi.x * hi.x + hi.y * hi.y) + (hi.z * hi.z + hi.w * hi.w));
         }
     }
     float r = 1.f;
-    if (SRC == SKN_SRC_RMSNORM) {
-        ss = wave_sum(ss);
-        if ((tid & 63) == 0) red_ss[rw][wv] = ss;
+    if constexpr (SRC == SKN_SRC_RMSNORM) {
+        // A row's sum of squares does not depend on how many wavefronts a row has: tasks u, u + 128, ... in turn (u < 128), then the
+        // lanes of a wavefront, then the two halves.  The upper two wavefronts hand their tasks' sums to the lower two.
+        float* const theirs = upper + rw * NT * (T / 2) + (t & (T / 2 - 1));
+        if (t >= T / 2) {
+#pragma unroll
+            for (int j = 0; j < NT; j++) theirs[j * (T / 2)] = squares[j];
+        }
         __syncthreads();
-        r = 1.0f / sqrtf(((red_ss[rw][0] + red_ss[rw][1]) + (red_ss[rw][2] + red_ss[rw][3])) / (float)k + src.eps);
+        if (t < T / 2) {
+            float ss = 0.f;
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                if (t + T * j < tasks) ss += squares[j];
+                if (t + T * j + T / 2 < tasks) ss += theirs[j * (T / 2)];
+            }
+            ss = wave_sum(ss);
+            if ((tid & 63) == 0) red_ss[rw][wv] = ss;
+        }
+        __syncthreads();
+        r = 1.0f / sqrtf((red_ss[rw][0] + red_ss[rw][1]) / (float)k + src.eps);
     }
     // the bf16 values the GEMM is defined on (fp32 sources: rounded to nearest even here), and their largest magnitude
     float mx = 0.f;
