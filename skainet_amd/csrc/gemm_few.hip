@@ -14,6 +14,7 @@
 // alone 7.5 at the rate of a copy), Q5_K 16 x 1000 x 1024 9.4 -> 4.6.  Error against 64 bits: not larger (1.1 against 1.5e-7 of the
 // result in Q4_K at k = 11008, 0.95 against 1.05 in Q8_0): a superblock's sum is formed before it joins the total.
 #include "gemm_few.h"
+#include "gemm_few_loads.h"
 #include "gemm_tiles.h"
 
 #include <algorithm>
@@ -172,7 +173,7 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
                                                           int k, uint32_t a_bytes, uint32_t w_bytes, float* __restrict__ part, int part_blocks) {
     extern __shared__ __align__(16) uint8_t lds[];  // a superblock of the tile's weight rows per wavefront, then the exchange of the tiles
     constexpr int P = F::kPieces;
-    constexpr int CH = few_chunk(MT), AP = 4 * CH;  // sixteen-byte pieces of a chunk's row
+    constexpr int CH = few_chunk(MT);
     const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nb = k >> 8, n0 = (int)blockIdx.x * 16, m0 = (int)blockIdx.z * 16 * MT;
@@ -191,43 +192,43 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
 
     // The tile's rows of a superblock: coalesced loads one superblock ahead, handed over through LDS of the wavefront's own (the lane
     // number passes through an empty asm: a store may go anywhere as far as the compiler knows and keeps its place among the loads before
-    // and after it, and the device keeps a wavefront's LDS accesses in order).  A row's first pieces go to WIDE neighbouring lanes, 64 / WIDE
-    // rows at a time, those past them to REST lanes: from one load to the next only scalar offsets change.  (Rows past the last one and
-    // lanes without a piece: an offset past the end, which reads as zero.  With addresses formed per lane and load by division: Q4_K 16 x 4096 x
-    // 4096 5.6 us against 5.0, Q8_0 16 x 14000 x 1536 10.1 against 8.4.)
-    constexpr int WIDE = P > 12 ? 16 : 8, REST = P <= WIDE ? 0 : P - WIDE == 1 ? 1 : 4, LOADS = WIDE / 4 + (REST ? 1 : 0);
+    // and after it, and the device keeps a wavefront's LDS accesses in order).  Where they come from: gemm_few_loads.h; from one load to the
+    // next the offset grows by a scalar.  (With the offsets formed per lane and load by division: Q4_K 16 x 4096 x 4096 5.6 us against 5.0,
+    // Q8_0 16 x 14000 x 1536 10.1 against 8.4.)
+    using WL = FewWeightLoads<P, F::kBytes>;
+    constexpr int WIDE = WL::WIDE, LOADS = WL::COUNT + (WL::REST ? 1 : 0);
     int l = lane;
     asm("" : "+v"(l));
-    const int rb = nb * F::kBytes;
-    const int wfrom = l % WIDE < P ? (n0 + l / WIDE) * rb + min(l % WIDE * 16, F::kBytes - 16) : (int)w_bytes;
+    const uint32_t rb = (uint32_t)(nb * F::kBytes);
+    const uint32_t wfrom = WL::wide(l, n0, rb, w_bytes), restfrom = WL::rest(l, n0, rb, w_bytes);
     u32x4* const wto = reinterpret_cast<u32x4*>(mine + (l / WIDE) * F::kPitch + l % WIDE * 16);
-    const bool rest = REST && l / std::max(REST, 1) < 16 && WIDE + l % std::max(REST, 1) < P;
-    const int restfrom = rest ? (n0 + l / std::max(REST, 1)) * rb + (WIDE + l % std::max(REST, 1)) * 16 : (int)w_bytes;
-    u32x4* const restto = reinterpret_cast<u32x4*>(mine + (l / std::max(REST, 1)) * F::kPitch + (WIDE + l % std::max(REST, 1)) * 16);
+    u32x4* const restto = reinterpret_cast<u32x4*>(mine + WL::rest_row(l) * F::kPitch + WL::rest_piece(l) * 16);
     u32x4 next[LOADS];
     auto wload = [&](int sb) __attribute__((always_inline)) {
 #pragma unroll
-        for (int x = 0; x < WIDE / 4; x++)
-            next[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, wfrom, sb * F::kBytes + x * (64 / WIDE) * rb, 0));
-        if (REST) next[LOADS - 1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, restfrom, sb * F::kBytes, 0));
+        for (int x = 0; x < WL::COUNT; x++)
+            next[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)(wfrom + x * WL::step(rb)), sb * F::kBytes, 0));
+        if (WL::REST) next[LOADS - 1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)restfrom, sb * F::kBytes, 0));
     };
     auto wstore = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int x = 0; x < WIDE / 4; x++)
-            if (WIDE <= P || l % WIDE < P) wto[x * (64 / WIDE) * (F::kPitch / 16)] = next[x];
-        if (rest) *restto = next[LOADS - 1];
+        for (int x = 0; x < WL::COUNT; x++)
+            if (WL::wide_lane(l)) wto[x * (64 / WIDE) * (F::kPitch / 16)] = next[x];
+        if (WL::rest_lane(l)) *restto = next[LOADS - 1];
     };
     // The activations likewise, a chunk of CH blocks ahead, AP lanes to a row: piece p of row r goes to place p ^ turn(r) of the row, so
     // that the sixteen rows of an operand lie on different banks.
     auto turn = [](int r) __attribute__((always_inline)) { return CH == 2 ? (r >> 1) & 7 : r & 15; };
-    constexpr int AR = 64 / AP;  // rows of a load
-    const int afrom = (m0 + l / AP) * 2 * k + l % AP * 16, aplace = l % AP ^ turn(l / AP);
+    using AL = FewActivationLoads<CH>;
+    constexpr int AP = AL::LANES, AR = AL::ROWS;
+    const uint32_t afrom = AL::first(l, m0, 2u * k);
+    const int aplace = l % AP ^ turn(l / AP);
     uint8_t* const ato = rows + (l / AP) * (AP * 16);
     u32x4 anext[CH * MT];
     auto aload = [&](int chunk) __attribute__((always_inline)) {
 #pragma unroll
         for (int x = 0; x < CH * MT; x++)
-            anext[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, afrom, chunk * 64 * CH + x * AR * 2 * k, 0));
+            anext[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, (int)(afrom + x * AL::step(2u * k)), chunk * 64 * CH, 0));
     };
     auto astore = [&]() __attribute__((always_inline)) {
 #pragma unroll
