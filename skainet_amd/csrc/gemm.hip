@@ -709,7 +709,7 @@ __global__ __launch_bounds__(256) void gemm_add_parts_kernel(const float* __rest
         for (; z < splits; z++) sum += *reinterpret_cast<const vec*>(p + z * stride);
         return sum;
     };
-    const float sc = inv_scale ? inv_scale[row] : 1.f;
+    const float sc = inv_scale[row];
     vec v = total(src) * sc;
     if (segs.pair) {
         const vec u = total(src + segs.col0[1]) * sc;

@@ -36,29 +36,38 @@ __device__ __forceinline__ float f16_hi(uint32_t w) { return (float)__builtin_bi
 __device__ __forceinline__ uint32_t lds_u32(const uint8_t* p) { return *reinterpret_cast<const uint32_t*>(p); }
 __device__ __forceinline__ u32x2 lds_u32x2(const uint8_t* p) { return *reinterpret_cast<const u32x2*>(p); }
 
-// Operands are quants times 2^-12: a block's sum of at most 32 products of up to 2^7 then stays in fp32's range for every finite
-// activation (as they are it leaves it from about 8e34 on although the result need not), and its scale brings the 2^12 back.
-constexpr float kUp = 0x1p12f;
+// Range.  A tile is first summed in units of 2^-40, which the blocks' scales bring: the quants are operands as they are, every product of
+// a finite activation with one is exact (down to bf16's least subnormal), and no sum of a row of least activations loses bits.  What does not
+// fit there -- rows from about 2^47 on -- ends as an infinity or NaN, is seen when the tile is stored, and the tile is summed once more with
+// operands times 2^-100, in units of 2^60, where sums of the largest activations and weights of all formats fit; rows that need it are large
+// enough to lose nothing by it.  So a result is finite wherever it is for rows scaled to their largest element.  The first pass pays
+// for the subtraction below (Q8_0 8 x 4096 x 11008 11.4 us without it, 11.8 with, Q5_K 11.2, 12.0) and 0.1 to 0.3 us for looking at the sums
+// (16 x 4096 x 4096 in Q4_K 5.0, 5.0, in Q6_K 6.4, 6.8, in Q8_0 6.0, 6.2).
+constexpr float kUp = 0x1p40f;
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+struct Operands {
+    uint32_t down;  // off the exponents of a pair of bf16 operands: 0, 100
+    float nibble;   // 2^9, 2^-91
+};
 
-// Four whole numbers of at most eight bits, one to a byte, as bf16: the upper halves of their fp32 forms, less twelve in the exponent
-// (zero stays zero: the subtraction stops there; Q8_0 8 x 4096 x 11008 11.4 us without it, 11.8 with, Q5_K 11.2, 12.0).
-__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+// Four whole numbers of at most eight bits, one to a byte, as bf16: the upper halves of their fp32 forms (zero stays zero: the
+// subtraction stops there).
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi, const Operands& o) {
     const u16x2 x = __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u));
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(x, u16x2{12 << 7, 12 << 7}));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(x, __builtin_bit_cast(u16x2, o.down)));
 }
-__device__ __forceinline__ u32x2 signed_bytes(uint32_t b) {
+__device__ __forceinline__ u32x2 signed_bytes(uint32_t b, const Operands& o) {
     const float f0 = (float)(int8_t)b, f1 = (float)(int8_t)(b >> 8), f2 = (float)(int8_t)(b >> 16), f3 = (float)(int8_t)(b >> 24);
-    return u32x2{bf16_pair(f0, f1), bf16_pair(f2, f3)};
+    return u32x2{bf16_pair(f0, f1, o), bf16_pair(f2, f3, o)};
 }
-__device__ __forceinline__ u32x2 unsigned_bytes(uint32_t b) {
+__device__ __forceinline__ u32x2 unsigned_bytes(uint32_t b, const Operands& o) {
     const float f0 = (float)(uint8_t)b, f1 = (float)(uint8_t)(b >> 8), f2 = (float)(uint8_t)(b >> 16), f3 = (float)(uint8_t)(b >> 24);
-    return u32x2{bf16_pair(f0, f1), bf16_pair(f2, f3)};
+    return u32x2{bf16_pair(f0, f1, o), bf16_pair(f2, f3, o)};
 }
 // Four numbers 0..15: as E4M3 a byte below sixteen is that many times 2^-9 (subnormals and the first binade are one straight line).
-__device__ __forceinline__ u32x2 nibble_bytes(uint32_t b) {
-    return u32x2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f / kUp, false)),
-                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f / kUp, true))};
+__device__ __forceinline__ u32x2 nibble_bytes(uint32_t b, const Operands& o) {
+    return u32x2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, o.nibble, false)),
+                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, o.nibble, true))};
 }
 __device__ __forceinline__ bf16x8 operand(u32x2 lo, u32x2 hi) { return __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y}); }
 
@@ -79,14 +88,14 @@ struct FewK {
         s.mn[0] = h[2] & 0x3F3F3F3Fu, s.mn[1] = ((h[3] >> 4) & 0x0F0F0F0Fu) | ((h[2] >> 2) & 0x30303030u);
         if (FIVE) s.fifth = lds_u32x2(row + 16 + 8 * g);
     }
-    __device__ static __forceinline__ bf16x8 block(const uint8_t* row, const Head& H, int b, int g, float& s, float& mn) {
+    __device__ static __forceinline__ bf16x8 block(const uint8_t* row, const Head& H, int b, int g, const Operands& o, float& s, float& mn) {
         s = H.d * (float)((H.sc[b >> 2] >> (8 * (b & 3))) & 0xFFu);  // (11 x 6 bits: exact)
         mn = H.dmin * (float)((H.mn[b >> 2] >> (8 * (b & 3))) & 0xFFu);
         const u32x2 x = lds_u32x2(row + (FIVE ? 48 : 16) + 32 * (b >> 1) + 8 * g);
         const u32x2 q = (x >> (uint32_t)(4 * (b & 1))) & 0x0F0F0F0Fu;
-        if (!FIVE) return operand(nibble_bytes(q.x), nibble_bytes(q.y));
+        if (!FIVE) return operand(nibble_bytes(q.x, o), nibble_bytes(q.y, o));
         const u32x2 f = (b < 4 ? H.fifth << (uint32_t)(4 - b) : H.fifth >> (uint32_t)(b - 4)) & 0x10101010u;
-        return operand(unsigned_bytes(q.x | f.x), unsigned_bytes(q.y | f.y));
+        return operand(unsigned_bytes(q.x | f.x, o), unsigned_bytes(q.y | f.y, o));
     }
 };
 
@@ -95,7 +104,7 @@ struct FewQ80 {  // 34 bytes: d, 32 int8; block pairs are 17 dwords
     static constexpr bool kMin = false, kHalves = false;
     struct Head {};
     __device__ static __forceinline__ void head(const uint8_t*, int, Head&) {}
-    __device__ static __forceinline__ bf16x8 block(const uint8_t* row, const Head&, int b, int g, float& s, float&) {
+    __device__ static __forceinline__ bf16x8 block(const uint8_t* row, const Head&, int b, int g, const Operands& o, float& s, float&) {
         const uint8_t* p = row + 68 * (b >> 1);
         uint32_t x, y;
         if (b & 1) {
@@ -106,7 +115,7 @@ struct FewQ80 {  // 34 bytes: d, 32 int8; block pairs are 17 dwords
             const uint32_t w0 = lds_u32(p + 8 * g), w1 = lds_u32(p + 4 + 8 * g), w2 = lds_u32(p + 8 + 8 * g);
             x = __builtin_amdgcn_alignbyte(w1, w0, 2), y = __builtin_amdgcn_alignbyte(w2, w1, 2);
         }
-        return operand(signed_bytes(x), signed_bytes(y));
+        return operand(signed_bytes(x, o), signed_bytes(y, o));
     }
 };
 
@@ -116,7 +125,7 @@ struct FewQ40 {  // 18 bytes: d, nibbles (low ones elements 0..15, high ones 16.
     struct Head {};
     __device__ static __forceinline__ void head(const uint8_t*, int, Head&) {}
     // a nibble at the top of its byte, less eight there, is 16 (q - 8)
-    __device__ static __forceinline__ bf16x8 block(const uint8_t* row, const Head&, int b, int g, float& s, float&) {
+    __device__ static __forceinline__ bf16x8 block(const uint8_t* row, const Head&, int b, int g, const Operands& o, float& s, float&) {
         const uint8_t* p = row + 36 * (b >> 1);
         const int at = 8 * (g & 1);
         u32x2 q;
@@ -129,7 +138,7 @@ struct FewQ40 {  // 18 bytes: d, nibbles (low ones elements 0..15, high ones 16.
             q = u32x2{__builtin_amdgcn_alignbyte(w1, w0, 2), __builtin_amdgcn_alignbyte(w2, w1, 2)};
         }
         q = ((q << (uint32_t)(g < 2 ? 4 : 0)) & 0xF0F0F0F0u) ^ 0x80808080u;
-        return operand(signed_bytes(q.x), signed_bytes(q.y));
+        return operand(signed_bytes(q.x, o), signed_bytes(q.y, o));
     }
 };
 
@@ -140,20 +149,20 @@ struct FewQ6K {
     static constexpr int kBytes = 210, kPieces = 14, kPitch = 240;
     static constexpr bool kHalves = true;
     struct Head {
-        float d4;  // d / 4 (times 2^12): the operands are 4 (q - 32)
+        float d4;  // d / 4 (times 2^40): the operands are 4 (q - 32)
         u32x4 sc;
     };
     __device__ static __forceinline__ void head(const uint8_t* row, int, Head& s) {
         s.d4 = f16_hi(lds_u32(row + 220)) * (kUp / 4);
         s.sc = *reinterpret_cast<const u32x4*>(row + 192);
     }
-    __device__ static __forceinline__ s16x4 sixteen(const uint8_t* row, const Head& H, int b, int t, int g, float& s) {
+    __device__ static __forceinline__ s16x4 sixteen(const uint8_t* row, const Head& H, int b, int t, int g, const Operands& o, float& s) {
         const int hf = b >> 2, Q = b & 3, e = 2 * b + t;
         s = H.d4 * (float)(int8_t)(H.sc[e >> 2] >> (8 * (e & 3)));
         const uint32_t ql = lds_u32(row + 64 * hf + 32 * (Q & 1) + 16 * t + 4 * g), qh = lds_u32(row + 128 + 32 * hf + 16 * t + 4 * g);
         const uint32_t lo = (Q < 2 ? ql << 2 : ql >> 2) & 0x3C3C3C3Cu;
         const uint32_t hi = (Q == 3 ? qh : qh << (6 - 2 * Q)) & 0xC0C0C0C0u;
-        return __builtin_bit_cast(s16x4, signed_bytes((lo | hi) ^ 0x80808080u));
+        return __builtin_bit_cast(s16x4, signed_bytes((lo | hi) ^ 0x80808080u, o));
     }
 };
 
@@ -170,11 +179,11 @@ constexpr int few_lds_bytes() {
 // MT row blocks of sixteen, sixteen columns, W wavefronts
 template <typename F, int MT, int W>
 __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __restrict__ a, const uint8_t* __restrict__ w, float* __restrict__ c, int m, int n,
-                                                          int k, uint32_t a_bytes, uint32_t w_bytes, float* __restrict__ part, int part_blocks) {
+                                                          int k, uint32_t a_bytes, uint32_t w_bytes, double* __restrict__ part, int part_blocks) {
     extern __shared__ __align__(16) uint8_t lds[];  // a superblock of the tile's weight rows per wavefront, then the exchange of the tiles
     constexpr int P = F::kPieces;
     constexpr int CH = few_chunk(MT);
-    const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+    const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nb = k >> 8, n0 = (int)blockIdx.x * 16, m0 = (int)blockIdx.z * 16 * MT;
     const int sb0 = (int)blockIdx.y * part_blocks, sb1 = min(sb0 + part_blocks, nb);  // (all, or a part of k)
@@ -182,27 +191,18 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
     const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc((void*)a, 0, (int)a_bytes, 0x00020000);
     uint8_t* mine = lds + wave * (16 * F::kPitch + CH * MT * 1024);
     uint8_t* rows = mine + 16 * F::kPitch;
-    const uint8_t* row = mine + col * F::kPitch;
     f32x4 acc[MT], total[MT];  // of a superblock, of the wavefront's superblocks
-#pragma unroll
-    for (int i = 0; i < MT; i++) total[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    const u32x4 ones_bits = {0x39803980u, 0x39803980u, 0x39803980u, 0x39803980u};  // (2^-12)
-    const bf16x8 ones = __builtin_bit_cast(bf16x8, ones_bits);
 
-    // The tile's rows of a superblock: coalesced loads one superblock ahead, handed over through LDS of the wavefront's own (the lane
-    // number passes through an empty asm: a store may go anywhere as far as the compiler knows and keeps its place among the loads before
-    // and after it, and the device keeps a wavefront's LDS accesses in order).  Where they come from: gemm_few_loads.h; from one load to the
-    // next the offset grows by a scalar.  (With the offsets formed per lane and load by division: Q4_K 16 x 4096 x 4096 5.6 us against 5.0,
+    // The tile's rows of a superblock: coalesced loads one superblock ahead, handed over through LDS of the wavefront's own (the stores'
+    // lane number passes through an empty asm of its own: a store may go anywhere as far as the compiler knows and keeps its place among
+    // the loads before and after it, and the device keeps a wavefront's LDS accesses in order).  Where they come from: gemm_few_loads.h; from
+    // one load to the next the offset grows by a scalar.  (With the offsets formed per lane and load by division: Q4_K 16 x 4096 x 4096 5.6 us against 5.0,
     // Q8_0 16 x 14000 x 1536 10.1 against 8.4.)
     using WL = FewWeightLoads<P, F::kBytes>;
     constexpr int WIDE = WL::WIDE, LOADS = WL::COUNT + (WL::REST ? 1 : 0);
-    int l = lane;
-    asm("" : "+v"(l));
     const uint32_t rb = (uint32_t)(nb * F::kBytes);
-    const uint32_t wfrom = WL::wide(l, n0, rb, w_bytes), restfrom = WL::rest(l, n0, rb, w_bytes);
-    u32x4* const wto = reinterpret_cast<u32x4*>(mine + (l / WIDE) * F::kPitch + l % WIDE * 16);
-    u32x4* const restto = reinterpret_cast<u32x4*>(mine + WL::rest_row(l) * F::kPitch + WL::rest_piece(l) * 16);
+    const uint32_t wfrom = WL::wide(lane, n0, rb, w_bytes), restfrom = WL::rest(lane, n0, rb, w_bytes);
     u32x4 next[LOADS];
     auto wload = [&](int sb) __attribute__((always_inline)) {
 #pragma unroll
@@ -210,125 +210,179 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
             next[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)(wfrom + x * WL::step(rb)), sb * F::kBytes, 0));
         if (WL::REST) next[LOADS - 1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int)restfrom, sb * F::kBytes, 0));
     };
-    auto wstore = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int x = 0; x < WL::COUNT; x++)
-            if (WL::wide_lane(l)) wto[x * (64 / WIDE) * (F::kPitch / 16)] = next[x];
-        if (WL::rest_lane(l)) *restto = next[LOADS - 1];
-    };
-    // The activations likewise, a chunk of CH blocks ahead, AP lanes to a row: piece p of row r goes to place p ^ turn(r) of the row, so
-    // that the sixteen rows of an operand lie on different banks.
-    auto turn = [](int r) __attribute__((always_inline)) { return CH == 2 ? (r >> 1) & 7 : r & 15; };
+    // The activations likewise, a chunk of CH blocks ahead, AP lanes to a row.
     using AL = FewActivationLoads<CH>;
     constexpr int AP = AL::LANES, AR = AL::ROWS;
-    const uint32_t afrom = AL::first(l, m0, 2u * k);
-    const int aplace = l % AP ^ turn(l / AP);
-    uint8_t* const ato = rows + (l / AP) * (AP * 16);
+    const uint32_t afrom = AL::first(lane, m0, 2u * k);
     u32x4 anext[CH * MT];
     auto aload = [&](int chunk) __attribute__((always_inline)) {
 #pragma unroll
         for (int x = 0; x < CH * MT; x++)
             anext[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, (int)(afrom + x * AL::step(2u * k)), chunk * 64 * CH, 0));
     };
-    auto astore = [&]() __attribute__((always_inline)) {
+    auto fits = [](float x) __attribute__((always_inline)) { return fabsf(x) < INFINITY; };
+    uint32_t less = 0;  // (the second pass: 100)
+#pragma unroll 1
+    for (;;) {
+        asm volatile("" : "+s"(less));  // (one body for both)
+        const Operands o = {(less << 7) * 0x10001u, __uint_as_float((127u + 9u - less) << 23)};
+        const uint32_t one = 0x3F803F80u - o.down;
+        const u32x4 ones_bits = {one, one, one, one};
+        const bf16x8 ones = __builtin_bit_cast(bf16x8, ones_bits);
 #pragma unroll
-        for (int x = 0; x < CH * MT; x++)  // (the turns of a load's first row and of the lane's row in it share no bits)
-            *reinterpret_cast<u32x4*>(ato + x * AR * AP * 16 + (aplace ^ turn(x * AR & 15)) * 16) = anext[x];
-    };
-    auto aread = [&](int i, int b) __attribute__((always_inline)) {  // b: in the chunk
-        const uint8_t* base = rows + (16 * i + col) * (AP * 16);
-        if (!F::kHalves) return *reinterpret_cast<const u32x4*>(base + ((4 * b + g) ^ turn(col)) * 16);
-        const u32x2 x = lds_u32x2(base + ((4 * b + (g >> 1)) ^ turn(col)) * 16 + 8 * (g & 1));
-        const u32x2 y = lds_u32x2(base + ((4 * b + 2 + (g >> 1)) ^ turn(col)) * 16 + 8 * (g & 1));
-        return u32x4{x.x, x.y, y.x, y.y};
-    };
-    if (sb0 + wave < sb1) {
-        wload(sb0 + wave);
-        aload((8 / CH) * (sb0 + wave));
-    }
-    for (int sb = sb0 + wave; sb < sb1; sb += W) {
-        const int sbn = min(sb + W, nb - 1);  // (past the end: a repeat, unused)
-        wstore();
-        wload(sbn);
-        typename F::Head H;
-        F::head(row, g, H);
+        for (int i = 0; i < MT; i++) total[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (sb0 + wave < sb1) {
+            wload(sb0 + wave);
+            aload((8 / CH) * (sb0 + wave));
+        }
+        // (addresses in LDS are formed behind the first loads, which they would delay by up to 0.2 us: u of what is read, v of what is stored)
+        uint32_t u = lane, v = lane;
+        asm volatile("" : "+v"(u), "+v"(v));
+        const int col = u & 15u, g = u >> 4;
+        const uint8_t* row = mine + col * F::kPitch;
+        u32x4* const wto = reinterpret_cast<u32x4*>(mine + (v / WIDE) * F::kPitch + v % WIDE * 16);
+        u32x4* const restto = reinterpret_cast<u32x4*>(mine + WL::rest_row(v) * F::kPitch + WL::rest_piece(v) * 16);
+        auto wstore = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int b = 0; b < 8; b++) {
-            if (b % CH == 0) {
-                astore();
-                aload(b + CH < 8 ? (8 / CH) * sb + b / CH + 1 : (8 / CH) * sbn);
-            }
-            u32x4 av[MT];
+            for (int x = 0; x < WL::COUNT; x++)
+                if (WL::wide_lane(v)) wto[x * (64 / WIDE) * (F::kPitch / 16)] = next[x];
+            if (WL::rest_lane(v)) *restto = next[LOADS - 1];
+        };
+        // Activations: piece p of row r goes to place p ^ turn(r) of the row, so that the sixteen rows of an operand lie on different banks.
+        auto turn = [](int r) __attribute__((always_inline)) { return CH == 2 ? (r >> 1) & 7 : r & 15; };
+        const int aplace = v % AP ^ turn(v / AP);
+        uint8_t* const ato = rows + (v / AP) * (AP * 16);
+        auto astore = [&]() __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < MT; i++) av[i] = aread(i, b % CH);
-            if constexpr (F::kHalves) {
+            for (int x = 0; x < CH * MT; x++)  // (the turns of a load's first row and of the lane's row in it share no bits)
+                *reinterpret_cast<u32x4*>(ato + x * AR * AP * 16 + (aplace ^ turn(x * AR & 15)) * 16) = anext[x];
+        };
+        auto aread = [&](int i, int b) __attribute__((always_inline)) {  // b: in the chunk
+            const uint8_t* base = rows + (16 * i + col) * (AP * 16);
+            if (!F::kHalves) return *reinterpret_cast<const u32x4*>(base + ((4 * b + g) ^ turn(col)) * 16);
+            const u32x2 x = lds_u32x2(base + ((4 * b + (g >> 1)) ^ turn(col)) * 16 + 8 * (g & 1));
+            const u32x2 y = lds_u32x2(base + ((4 * b + 2 + (g >> 1)) ^ turn(col)) * 16 + 8 * (g & 1));
+            return u32x4{x.x, x.y, y.x, y.y};
+        };
+        for (int sb = sb0 + wave; sb < sb1; sb += W) {
+            const int sbn = min(sb + W, nb - 1);  // (past the end: a repeat, unused)
+            wstore();
+            wload(sbn);
+            typename F::Head H;
+            F::head(row, g, H);
 #pragma unroll
-                for (int t = 0; t < 2; t++) {
-                    float s;
-                    const s16x4 q = F::sixteen(row, H, b, t, g, s);
+            for (int b = 0; b < 8; b++) {
+                if (b % CH == 0) {
+                    astore();
+                    aload(b + CH < 8 ? (8 / CH) * sb + b / CH + 1 : (8 / CH) * sbn);
+                }
+                u32x4 av[MT];
+#pragma unroll
+                for (int i = 0; i < MT; i++) av[i] = aread(i, b % CH);
+                if constexpr (F::kHalves) {
+#pragma unroll
+                    for (int t = 0; t < 2; t++) {
+                        float s;
+                        const s16x4 q = F::sixteen(row, H, b, t, g, o, s);
+#pragma unroll
+                        for (int i = 0; i < MT; i++) {
+                            const s16x4 x = __builtin_bit_cast(s16x4, u32x2{av[i][2 * t], av[i][2 * t + 1]});
+                            const f32x4 p = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(x, q, zero, 0, 0, 0);
+#pragma unroll
+                            for (int y = 0; y < 4; y++) acc[i][y] = b == 0 && t == 0 ? s * p[y] : fmaf(s, p[y], acc[i][y]);
+                        }
+                    }
+                } else {
+                    float s, mn = 0.f;
+                    const bf16x8 q = F::block(row, H, b, g, o, s, mn);
 #pragma unroll
                     for (int i = 0; i < MT; i++) {
-                        const s16x4 x = __builtin_bit_cast(s16x4, u32x2{av[i][2 * t], av[i][2 * t + 1]});
-                        const f32x4 p = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(x, q, zero, 0, 0, 0);
+                        const bf16x8 x = __builtin_bit_cast(bf16x8, av[i]);
+                        const f32x4 p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, q, zero, 0, 0, 0);
 #pragma unroll
-                        for (int y = 0; y < 4; y++) acc[i][y] = b == 0 && t == 0 ? s * p[y] : fmaf(s, p[y], acc[i][y]);
+                        for (int y = 0; y < 4; y++) acc[i][y] = b == 0 ? s * p[y] : fmaf(s, p[y], acc[i][y]);
+                        if constexpr (F::kMin) {
+                            const f32x4 sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, ones, zero, 0, 0, 0);
+#pragma unroll
+                            for (int y = 0; y < 4; y++) acc[i][y] = fmaf(-mn, sum[y], acc[i][y]);
+                        }
                     }
                 }
-            } else {
-                float s, mn = 0.f;
-                const bf16x8 q = F::block(row, H, b, g, s, mn);
-#pragma unroll
-                for (int i = 0; i < MT; i++) {
-                    const bf16x8 x = __builtin_bit_cast(bf16x8, av[i]);
-                    const f32x4 p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, q, zero, 0, 0, 0);
-#pragma unroll
-                    for (int y = 0; y < 4; y++) acc[i][y] = b == 0 ? s * p[y] : fmaf(s, p[y], acc[i][y]);
-                    if constexpr (F::kMin) {
-                        const f32x4 sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, ones, zero, 0, 0, 0);
-#pragma unroll
-                        for (int y = 0; y < 4; y++) acc[i][y] = fmaf(-mn, sum[y], acc[i][y]);
-                    }
-                }
+                if ((b & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // (more blocks at once would not fit the registers)
             }
-            if ((b & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // (more blocks at once would not fit the registers)
-        }
 #pragma unroll
-        for (int i = 0; i < MT; i++) total[i] += acc[i];
-    }
+            for (int i = 0; i < MT; i++) total[i] += acc[i];
+        }
 
-    __syncthreads();
-    f32x4* red = reinterpret_cast<f32x4*>(lds);
+        float size = 0.f;
 #pragma unroll
-    for (int i = 0; i < MT; i++) red[(wave * MT + i) * 64 + lane] = total[i];
-    __syncthreads();
-    // (accumulator register y of lane 16 g + c: row 4 g + y, column c)
-    const float* flat = reinterpret_cast<const float*>(red);
-    for (int e = threadIdx.x; e < MT * 256; e += 64 * W) {
-        const int r = e >> 4, cc = e & 15;
-        const int from = (r >> 4) * 256 + (((r >> 2) & 3) * 16 + cc) * 4 + (r & 3);
-        float sum = 0.f;
+        for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int x = 0; x < W; x++) sum += flat[x * MT * 256 + from];
-        if (m0 + r < m && n0 + cc < n) {
+            for (int y = 0; y < 4; y++) size += fabsf(total[i][y]);
+        const bool left = __builtin_amdgcn_ballot_w64(!(size < 0x1p120f)) != 0;  // (below it the wavefronts' sums stay in range too)
+        __syncthreads();
+        f32x4* red = reinterpret_cast<f32x4*>(lds);
+        uint32_t* lefts = reinterpret_cast<uint32_t*>(red + W * MT * 64);
+#pragma unroll
+        for (int i = 0; i < MT; i++) red[(wave * MT + i) * 64 + lane] = total[i];
+        if (lane == 0) lefts[wave] = left;
+        __syncthreads();
+        uint32_t again = 0;
+#pragma unroll
+        for (int x = 0; x < W; x++) again |= lefts[x];
+        // (accumulator register y of lane 16 g + c: row 4 g + y, column c)
+        const float* flat = reinterpret_cast<const float*>(red);
+        uint32_t tid = threadIdx.x, z = blockIdx.y;
+        asm volatile("" : "+v"(tid), "+s"(z));  // (addresses of the outputs are formed here, not ahead of the loads)
+        for (int e = tid; e < MT * 256; e += 64 * W) {
+            const int r = e >> 4, cc = e & 15;
+            const int from = (r >> 4) * 256 + (((r >> 2) & 3) * 16 + cc) * 4 + (r & 3);
+            float sum = 0.f;
+#pragma unroll
+            for (int x = 0; x < W; x++) sum += flat[x * MT * 256 + from];
+            if (m0 + r >= m || n0 + cc >= n) continue;
             const size_t at = (size_t)(m0 + r) * n + n0 + cc;
-            if (part) part[(size_t)blockIdx.y * m * n + at] = sum;
-            else c[at] = sum;
+            // (the second pass replaces what the first could not hold)
+            if (part) {
+                double* to = part + (size_t)z * m * n + at;
+                if (!less || (fits(sum) && !fits((float)*to))) *to = (double)sum * (less ? 0x1p60 : 0x1p-40);
+            } else if (!less || (fits(sum) && !fits(c[at]))) {
+                c[at] = sum * (less ? 0x1p60f : 0x1p-40f);
+            }
         }
+        if (less || !__builtin_amdgcn_readfirstlane(again)) return;
+        less = 100;
+        __syncthreads();
     }
+}
+
+// The parts of divided k, in fp64: whatever units a tile was summed in.
+__global__ __launch_bounds__(256) void gemm_few_add_kernel(const double* __restrict__ part, int splits, size_t count, float* __restrict__ c) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= count) return;
+    double v[16];  // (at most sixteen parts, all asked for before the first is used)
+#pragma unroll
+    for (int z = 0; z < 16; z++) v[z] = z < splits ? part[z * count + i] : 0.0;
+    double sum = v[0];
+#pragma unroll
+    for (int z = 1; z < 16; z++) sum += v[z];
+    c[i] = (float)sum;
 }
 
 template <typename F, int MT, int W>
 int launch_few(skn_ctx* ctx, const uint8_t* w, const uint16_t* a, float* c, int m, int n, int k, int splits) {
     const int nb = k / 256, each = (nb + splits - 1) / splits;
     splits = (nb + each - 1) / each;  // (no workgroup without a superblock)
-    float* part = splits > 1 ? skn_gemm_parts_room(ctx, (size_t)splits * m * n * 4) : nullptr;
+    double* part = splits > 1 ? (double*)skn_gemm_parts_room(ctx, (size_t)splits * m * n * sizeof(double)) : nullptr;
     if (!part) splits = 1;
     skn_launch(ctx, gemm_few_kernel<F, MT, W>, dim3((n + 15) / 16, splits, (m + 16 * MT - 1) / (16 * MT)), dim3(64 * W), few_lds_bytes<F, MT, W>(), a, w, c, m, n, k,
                (uint32_t)((size_t)m * k * 2), (uint32_t)((size_t)n * nb * F::kBytes), part, splits > 1 ? each : nb);
     SKN_LAUNCH_CHECK(ctx);
     if (!part) return SKN_OK;
-    const skn_gemm_parts ps = {{c, nullptr, nullptr}, {n, 0, 0}, {0, 0, 0}, {0, 0, 0}, 1, 0};
-    return skn_gemm_add_parts(ctx, part, splits, n, ps, nullptr, m);
+    const size_t count = (size_t)m * n;
+    skn_launch(ctx, gemm_few_add_kernel, dim3((uint32_t)((count + 255) / 256)), dim3(256), 0, (const double*)part, splits, count, c);
+    SKN_LAUNCH_CHECK(ctx);
+    return SKN_OK;
 }
 
 // Few columns: k over workgroups too where the turns of a wavefront that this saves, 0.5 + 0.7 MT us each, pay for the addition (3 us).  us

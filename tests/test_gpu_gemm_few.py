@@ -25,7 +25,9 @@ def _check(hip, t, raw, n, k, a, m, launches=None):
     size = np.abs(xd) @ np.abs(wd).T
     if t in (synth.Q4_K, synth.Q5_K):  # d sc q and dmin m are terms of their own
         size = size * 4
-    assert np.all(np.abs(got - xd @ wd.T) <= ROUNDINGS * 2.0**-24 * size + 1e-30)
+    # (and half of the least subnormal, where the result is one)
+    assert np.all(np.abs(got - xd @ wd.T) <= ROUNDINGS * 2.0**-24 * size + 2.0**-150)
+    return got
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
@@ -96,6 +98,34 @@ def test_activations_at_either_end_of_their_range(hip, name, size):
     xd = oracle_np.bf16_to_f32(a).astype(np.float64).reshape(m, k)
     bound = np.abs(xd) @ np.abs(wd).T * (4 if name in ("q4_k", "q5_k") else 1)
     assert np.all(np.abs(got - xd @ wd.T) <= ROUNDINGS * 2.0**-24 * bound)
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("k,launches", [(512, 1), (10752, 2)])
+def test_sums_that_leave_the_range_on_their_way(hip, name, k, launches):
+    """Results of every size beside each other, k in one piece and divided: a row of 2^124 whose halves cancel (over wavefronts, over parts;
+    minima against scales in a block), rows of 2^60 and 2^100, of elements 2^40 apart, of zeros, of the least normal and of subnormal
+    activations, ordinary ones."""
+    assert hip.device_info()["compute_units"] == 256, "k is divided for 256 compute units"
+    t = FORMATS[name]
+    m, n = 20, 33
+    half = synth.weight(t, n, k // 2, seed=k + t).reshape(n, -1)
+    raw = np.concatenate([half, half], axis=1).reshape(-1)
+    rng = np.random.default_rng(t)
+    x = rng.standard_normal((m, k))
+    x[0] = 2.0**124 * (1 + rng.random(k))
+    x[0, k // 2:] = -x[0, : k // 2]
+    x[1] *= 2.0**60
+    x[2] *= 2.0**100
+    x[3] = 0.0
+    x[4] *= 2.0**100
+    x[4, ::2] *= 2.0**-40
+    x[5] = rng.uniform(1, 2, k) * 2.0**-126 * rng.choice([-1, 1], k)
+    x[6] = rng.integers(-127, 128, k) * 2.0**-133
+    a = synth.f32_to_bf16_bits(x.astype(np.float32)).reshape(m, k)
+    assert np.array_equal(a[0, k // 2:], a[0, : k // 2] ^ 0x8000)
+    got = _check(hip, t, raw, n, k, a, m, launches)
+    assert np.all(np.isfinite(got)) and np.all(got[3] == 0) and np.any(got[6])
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
