@@ -170,6 +170,7 @@ struct skn_gemm_src {
     const void* a;
     const void* b;
     float eps;  // SKN_SRC_RMSNORM
+    bool ahead = false;  // nothing is launched: the product's memory only, for a later call
 };
 struct skn_gemm_seg {
     const void* w;

@@ -2100,12 +2100,15 @@ int skn_gemm_k_splits(const skn_ctx* ctx, int m, int tiles, int nb) {
     return (nb + each - 1) / each;  // (no workgroup without a superblock)
 }
 
-static bool grow_parts(skn_ctx* ctx, size_t bytes) {
+static bool may_allocate(skn_ctx* ctx) {  // (asking for memory would end a capture)
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return false;  // (asking for memory would end the capture)
-    }
+    if (hipStreamIsCapturing(ctx->stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
+static bool grow_parts(skn_ctx* ctx, size_t bytes) {
+    if (!may_allocate(ctx)) return false;
     void* p = nullptr;
     if (hipMalloc(&p, bytes) != hipSuccess) {
         (void)hipGetLastError();
@@ -2121,8 +2124,8 @@ static bool grow_parts(skn_ctx* ctx, size_t bytes) {
     return true;
 }
 
-int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out) {
-    if (bytes > ctx->gemm_ws_bytes) {
+int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out, bool ahead) {
+    if (bytes > ctx->gemm_ws_bytes && !(ahead && !may_allocate(ctx))) {
         SKN_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (ctx->gemm_ws) SKN_HIP(ctx, hipFree(ctx->gemm_ws));
         ctx->gemm_ws = nullptr;
@@ -2142,7 +2145,7 @@ int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out) {
 
 float* skn_gemm_parts_room(skn_ctx* ctx, size_t bytes) {
     if (ctx->opt_test_gemm_no_parts) return nullptr;
-    // (asked for ahead of any workspace, as the products of few rows do: what that would have brought)
+    // (without a workspace yet, as under test or where that found no memory: what it would have brought)
     const size_t least = ctx->gemm_parts ? 0 : (size_t)ctx->compute_units * 256 * 128 * 4;
     if (bytes > ctx->gemm_parts_bytes && !grow_parts(ctx, std::max(bytes, least))) return nullptr;
     return (float*)ctx->gemm_parts;
@@ -2259,10 +2262,11 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     for (int i = 0; i < 3; i++) fs.part_col0[i] = ps.col0[i];
     int splits = tall ? 1 : q4k_splits(ctx, m, mt_rows, m_tiles * fs.n_tiles, k / 256, fs.part_cols);
     uint8_t* ws;
-    int rc = skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes, &ws);
+    int rc = skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes, &ws, src.ahead);
     if (rc != SKN_OK) return rc;
     const size_t part_bytes = tall ? (size_t)tail.tiles * tail.splits * 131072 : splits > 1 ? (size_t)splits * m * fs.part_cols * 4 : 0;
     float* part = part_bytes ? skn_gemm_parts_room(ctx, part_bytes) : nullptr;
+    if (src.ahead) return SKN_OK;
     if (!part) splits = 1, tail = TallTail{tall_tiles, 0, 1, nullptr};
     fs.part_blocks = (k / 256 + splits - 1) / splits;
     if (splits > 1) fs.part = part;
@@ -2294,29 +2298,13 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     return splits > 1 ? skn_gemm_add_parts(ctx, fs.part, splits, fs.part_cols, ps, isc, m) : SKN_OK;
 }
 
-extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n, int k, const uint16_t* a_bf16_dev,
-                          int m, float* c_dev) {
-    SKN_REQUIRE(nullptr, ctx != nullptr, SKN_ERR_ARG, "skn_gemm_q: ctx is null");
-    SKN_REQUIRE(ctx, skn_is_quant(ggml_type), SKN_ERR_TYPE, "skn_gemm_q: ggml type %d is not supported", ggml_type);
-    SKN_REQUIRE(ctx, n >= 0 && k >= 0 && m >= 0, SKN_ERR_ARG, "skn_gemm_q: negative shape");
-    int be, bb;
-    skn_type_block(ggml_type, &be, &bb);
-    SKN_REQUIRE(ctx, k % be == 0, SKN_ERR_SHAPE, "Quantized tensor row size (%d) is not a multiple of block size (%d)", k,
-                be);
-    if (n == 0 || m == 0) return SKN_OK;
-    SKN_REQUIRE(ctx, c_dev != nullptr, SKN_ERR_ARG, "skn_gemm_q: c is null");
-    if (k == 0) return skn_memset(ctx, c_dev, 0, (size_t)m * n * sizeof(float));
-    SKN_REQUIRE(ctx, w_dev && a_bf16_dev, SKN_ERR_ARG, "skn_gemm_q: null pointer");
-    SKN_REQUIRE(ctx, k % 64 == 0, SKN_ERR_SHAPE, "skn_gemm_q: k (%d) must be a multiple of %d", k, 64);
-
-    // few rows: one launch instead of three
-    if (((uintptr_t)a_bf16_dev & 7) == 0 && skn_gemm_few_ok(ctx, ggml_type, w_dev, n, k, m))
-        return skn_gemm_few(ctx, ggml_type, w_dev, n, k, a_bf16_dev, m, c_dev);
+// The product in a pass over the activations, one over the tiles and, where k is divided, one over the parts (and a pass over the
+// weights, in the general path).
+static int gemm_in_passes(skn_ctx* ctx, int ggml_type, const void* w_dev, int n, int k, const skn_gemm_src& src, int m, float* c_dev) {
     if (ggml_type == SKN_TYPE_Q4_K && k <= 16384) {
-        SKN_REQUIRE(ctx, ((uintptr_t)w_dev & 15) == 0 && ((uintptr_t)a_bf16_dev & 7) == 0, SKN_ERR_ARG,
+        SKN_REQUIRE(ctx, ((uintptr_t)w_dev & 15) == 0 && ((uintptr_t)src.a & 7) == 0, SKN_ERR_ARG,
                     "skn_gemm_q: Q4_K weights must be 16-byte aligned, activations 8-byte aligned");
         const skn_gemm_seg seg = {w_dev, n, c_dev, 0};
-        const skn_gemm_src src = {SKN_SRC_BF16, a_bf16_dev, nullptr, 0.f};
         // up to 32 rows (17 to 32 of matrices too large for the path above): the kernel for blocks of 32, whose tile has as many (us per
         // call, this | that: 17 x 14336 x 4096 20.1 | 19.0, 17 x 8192 x 11008 30.3 | 27.9, 32 x 28672 x 4096 28.5 | 26.4, 32 x 11008 x 8192
         // 29.5 | 29.3; on two row blocks 41 x 4096 x 4096 15.2 | 14.9, 64 x 11008 x 4096 20.1 | 23.8)
@@ -2327,8 +2315,7 @@ extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n,
 
     // general path.  Workspace: activations in fragment order (rows padded to whole tiles) + row scales, then
     // the weights as an fp16 pair in fragment order (rows padded to whole 64-column tiles)
-    SKN_REQUIRE(ctx, ((uintptr_t)a_bf16_dev & 7) == 0, SKN_ERR_ARG, "skn_gemm_q: activations must be 8-byte aligned");
-    const skn_gemm_src src = {SKN_SRC_BF16, a_bf16_dev, nullptr, 0.f};
+    SKN_REQUIRE(ctx, ((uintptr_t)src.a & 7) == 0, SKN_ERR_ARG, "skn_gemm_q: activations must be 8-byte aligned");
     // Q6_K with whole superblocks: the kernels that unpack the blocks themselves (no weight pass, no expanded copy)
     if (ggml_type == SKN_TYPE_Q6_K && skn_gemm_q6k_direct_ok(ctx, n, k, m)) {
         const skn_gemm_seg seg = {w_dev, n, c_dev, 0};
@@ -2339,6 +2326,7 @@ extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n,
         const skn_gemm_seg seg = {w_dev, n, c_dev, 0};
         return skn_gemm_blocks_multi(ctx, &ggml_type, &seg, 1, k, src, m);
     }
+    if (src.ahead) return SKN_OK;  // (no product of few rows has a format or a size that would come here)
     const int mt = skn_gemm_mt(m);
     const int m_pad = (m + 32 * mt - 1) / (32 * mt) * (32 * mt), n_pad = (n + kBN - 1) / kBN * kBN;
     const size_t af_bytes = skn_align_up((size_t)m_pad * k * 2), is_bytes = skn_align_up((size_t)m_pad * 4);
@@ -2354,6 +2342,30 @@ extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n,
     rc = skn_weights_hilo_frag(ctx, ggml_type, (const uint8_t*)w_dev, n, k, bfrag);
     if (rc != SKN_OK) return rc;
     return launch_hilo_gemm_mt(ctx, mt, (const u32x4*)afrag, (const u32x4*)bfrag, isc, c_dev, m, n, k, 0);
+}
+
+extern "C" int skn_gemm_q(skn_ctx* ctx, int ggml_type, const void* w_dev, int n, int k, const uint16_t* a_bf16_dev,
+                          int m, float* c_dev) {
+    SKN_REQUIRE(nullptr, ctx != nullptr, SKN_ERR_ARG, "skn_gemm_q: ctx is null");
+    SKN_REQUIRE(ctx, skn_is_quant(ggml_type), SKN_ERR_TYPE, "skn_gemm_q: ggml type %d is not supported", ggml_type);
+    SKN_REQUIRE(ctx, n >= 0 && k >= 0 && m >= 0, SKN_ERR_ARG, "skn_gemm_q: negative shape");
+    int be, bb;
+    skn_type_block(ggml_type, &be, &bb);
+    SKN_REQUIRE(ctx, k % be == 0, SKN_ERR_SHAPE, "Quantized tensor row size (%d) is not a multiple of block size (%d)", k,
+                be);
+    if (n == 0 || m == 0) return SKN_OK;
+    SKN_REQUIRE(ctx, c_dev != nullptr, SKN_ERR_ARG, "skn_gemm_q: c is null");
+    if (k == 0) return skn_memset(ctx, c_dev, 0, (size_t)m * n * sizeof(float));
+    SKN_REQUIRE(ctx, w_dev && a_bf16_dev, SKN_ERR_ARG, "skn_gemm_q: null pointer");
+    SKN_REQUIRE(ctx, k % 64 == 0, SKN_ERR_SHAPE, "skn_gemm_q: k (%d) must be a multiple of %d", k, 64);
+
+    // Few rows: one launch instead of three.  The memory that the three would take is asked for all the same: a caller that captures
+    // its calls runs one of the same activations first, and one of more columns may not be of few rows.
+    if (((uintptr_t)a_bf16_dev & 7) == 0 && skn_gemm_few_ok(ctx, ggml_type, w_dev, n, k, m)) {
+        (void)gemm_in_passes(ctx, ggml_type, w_dev, n, k, skn_gemm_src{SKN_SRC_BF16, a_bf16_dev, nullptr, 0.f, true}, m, c_dev);
+        return skn_gemm_few(ctx, ggml_type, w_dev, n, k, a_bf16_dev, m, c_dev);
+    }
+    return gemm_in_passes(ctx, ggml_type, w_dev, n, k, skn_gemm_src{SKN_SRC_BF16, a_bf16_dev, nullptr, 0.f}, m, c_dev);
 }
 
 namespace {
@@ -2410,11 +2422,12 @@ int skn_gemm_q6k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
         if (splits[i] > 1) part_bytes = std::max(part_bytes, (size_t)splits[i] * m * segs[i].n * 4);
     }
     uint8_t* ws;
-    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes, &ws);
+    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes, &ws, src.ahead);
     if (rc != SKN_OK) return rc;
     _Float16* afrag = (_Float16*)ws;
     float* isc = (float*)(ws + af_bytes);
     float* part = part_bytes ? skn_gemm_parts_room(ctx, part_bytes) : nullptr;
+    if (src.ahead) return SKN_OK;
     if (!part) splits[0] = splits[1] = splits[2] = 1;
     _Float16* no_sums = nullptr;
     switch (src.kind) {

@@ -598,11 +598,12 @@ int skn_gemm_blocks_multi(skn_ctx* ctx, const int* types, const skn_gemm_seg* se
     const size_t af_bytes = skn_align_up((size_t)m_pad * k * 2), sf_bytes = sums ? skn_align_up((size_t)m_pad * (k / 256) * 32) : 0;
     const size_t is_bytes = skn_align_up((size_t)m_pad * 4);
     uint8_t* ws;
-    SKN_TRY(skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes, &ws));
+    SKN_TRY(skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes, &ws, src.ahead));
     u32x4* afrag = (u32x4*)ws;
     _Float16* sfrag = (_Float16*)(ws + af_bytes);
     float* isc = (float*)(ws + af_bytes + sf_bytes);
     float* part = part_bytes ? skn_gemm_parts_room(ctx, part_bytes) : nullptr;
+    if (src.ahead) return SKN_OK;
     if (!part) splits[0] = splits[1] = splits[2] = 1;
     switch (src.kind) {
         case SKN_SRC_BF16: launch_prep<SKN_SRC_BF16>(ctx, src, sums, afrag, isc, sfrag, m, m_pad, k); break;

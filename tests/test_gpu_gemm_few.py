@@ -1,9 +1,11 @@
 """GPU: products of up to 64 rows that take one launch, against 64-bit sums of the oracle's weights."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from oracle import oracle_c, oracle_np
-from skainet_amd import synth
+from skainet_amd import runtime, synth
 
 pytestmark = pytest.mark.gpu
 FORMATS = {"q4_k": synth.Q4_K, "q5_k": synth.Q5_K, "q6_k": synth.Q6_K, "q8_0": synth.Q8_0, "q4_0": synth.Q4_0}
@@ -153,3 +155,49 @@ def test_weights_and_activations_on_their_least_alignment(hip):
     hip.gemm_q(synth.Q6_K, w.ptr + 2, n, k, x.ptr + 8, m, c)
     got = c.download(np.float32, m * n).reshape(m, n)
     assert oracle_np.rel_err(got, oracle_c.gemm_q(synth.Q6_K, raw, n, k, a, m)) <= 1e-3
+
+
+@pytest.mark.parametrize("name,m,n,wide,k", [("q8_0", 333, 1024, 4096, 4096), ("q5_k", 41, 512, 20000, 4096), ("q6_k", 33, 512, 20000, 4096), ("q4_k", 48, 512, 20000, 4096),
+                                             ("q4_k", 17, 256, 20000, 4096)])
+def test_a_call_of_few_rows_readies_a_captured_one_of_more_columns(name, m, n, wide, k):
+    """A caller that captures its calls runs one of the same activations first: what that one does not need itself is there for the
+    captured one, which takes three launches.  Every replay against the eager result, with other work between."""
+    t = FORMATS[name]
+    rt = runtime.load_library()  # (the HIP runtime's functions too)
+
+    def call(fn, *args):
+        assert getattr(rt, fn)(*args) == 0, fn
+
+    stream, graph, replay = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    with runtime.Context(0) as ctx:
+        call("hipStreamCreate", C.byref(stream))
+        ctx.set_stream(stream)
+        w, x = ctx.to_device(synth.weight(t, wide, k, seed=n)), ctx.to_device(synth.activation_bf16((m, k), seed=m))
+        c = ctx.alloc(4 * m * wide)
+        before = ctx.stat("launches")
+        ctx.gemm_q(t, w, n, k, x, m, c)
+        few = ctx.stat("launches") - before
+        ctx.sync()
+        before = ctx.stat("launches")
+        call("hipStreamBeginCapture", stream, 1)  # (of this thread's calls)
+        try:
+            ctx.gemm_q(t, w, wide, k, x, m, c)
+        finally:
+            ended = rt.hipStreamEndCapture(stream, C.byref(graph))
+        assert ended == 0
+        assert few == 1 and ctx.stat("launches") - before >= 2, "both take the same path: nothing was tested"
+        call("hipGraphInstantiate", C.byref(replay), graph, None, None, C.c_size_t(0))
+        ctx.gemm_q(t, w, wide, k, x, m, c)
+        ctx.sync()
+        want = c.download(np.float32, m * wide).view(np.uint32)
+        for _ in range(3):
+            ctx.memset(c, 0xFF, 4 * m * wide)
+            ctx.sync()
+            call("hipGraphLaunch", replay, stream)
+            ctx.sync()
+            assert np.array_equal(c.download(np.float32, m * wide).view(np.uint32), want)
+            ctx.gemm_q(t, w, n, k, x, m, c)
+        call("hipGraphExecDestroy", replay)
+        call("hipGraphDestroy", graph)
+        ctx.set_stream(None)
+        call("hipStreamDestroy", stream)
