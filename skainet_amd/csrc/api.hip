@@ -291,6 +291,7 @@ int skn_set_option(skn_ctx* ctx, const char* key, int value) {
     else if (!strcmp(key, "llama.expand_weights")) ctx->opt_llama_expand = value;
     else if (!strcmp(key, "gemm.tile")) ctx->opt_gemm_tile = value;
     else if (!strcmp(key, "gemm.split")) ctx->opt_gemm_split = value;
+    else if (!strcmp(key, "gemm.few")) ctx->opt_gemm_few = value;
     else if (!strcmp(key, "dense.tile")) ctx->opt_dense_tile = value;
     else if (!strcmp(key, "gemm.q6k_fused")) ctx->opt_gemm_q6k_fused = value;
     else if (!strcmp(key, "matvec.stage")) ctx->opt_matvec_stage = value;

@@ -468,7 +468,7 @@ bool skn_gemm_few_ok(const skn_ctx* ctx, int type, const void* w, int n, int k, 
         case SKN_TYPE_Q4_0: bytes = FewQ40::kBytes, most = {{45, 33, 33, 20, 16}}; break;
         default: return false;
     }
-    if (ctx->opt_gemm_tile != 0 || ctx->opt_gemm_split != 0 || ctx->opt_test_gemm_no_parts || ctx->opt_gemm_q6k_fused != 1 || m <= 0 ||  n <= 0 || k <= 0 || k % 256 != 0 || k > 16384 ||
+    if (ctx->opt_gemm_few != 1 || ctx->opt_gemm_tile != 0 || ctx->opt_gemm_split != 0 || ctx->opt_test_gemm_no_parts == 1 || ctx->opt_gemm_q6k_fused != 1 || m <= 0 || n <= 0 || k <= 0 || k % 256 != 0 || k > 16384 ||
         ((uintptr_t)w & (type == SKN_TYPE_Q6_K ? 1 : 15)) != 0 || (size_t)n * (k / 256) * bytes >= ((size_t)1 << 31))
         return false;
     const int blocks = std::min((m + 15) / 16, 5), tiles = (n + 15) / 16, groups = (m + 63) / 64;

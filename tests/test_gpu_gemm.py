@@ -433,8 +433,8 @@ def _extreme_rows(m, k, seed):
 
 @pytest.mark.parametrize("m,tile", [(8, 0), (8, 1), (8, 2), (8, 3), (40, 0), (40, 1), (40, 2), (40, 3)])
 def test_gemm_q4k_extreme_rows_on_every_tile(hip, m, tile):
-    """Up to 32 rows the library's own choice is the kernel for blocks of 32: the kernels of 64-, 128- and 256-row tiles, which a
-    decoder's short prompts take too, by option, and beyond 32 rows."""
+    """The library's own choice is one launch for so few rows of so few columns (the passes by option: test_gpu_gemm_passes.py); the kernels of
+    64-, 128- and 256-row tiles, which a decoder's short prompts take, by option."""
     n, k = 96, 2048
     raw = synth.weight(Q4_K, n, k, seed=21)
     a = _extreme_rows(m, k, seed=22)

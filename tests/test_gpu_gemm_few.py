@@ -1,4 +1,5 @@
-"""GPU: products of up to 64 rows that take one launch, against 64-bit sums of the oracle's weights."""
+"""GPU: products of few rows, and of more with a small matrix, that take one launch (two where k is divided) behind the activations as they
+are, against 64-bit sums of the oracle's weights."""
 import ctypes as C
 
 import numpy as np
@@ -14,13 +15,24 @@ FORMATS = {"q4_k": synth.Q4_K, "q5_k": synth.Q5_K, "q6_k": synth.Q6_K, "q8_0": s
 ROUNDINGS = 32 + 16 + 8 + 12
 
 
-def _check(hip, t, raw, n, k, a, m, launches=None):
-    c = hip.alloc(4 * m * n)
-    hip.memset(c, 0xFF, 4 * m * n)
-    w, x = hip.to_device(raw), hip.to_device(a)
+def _launches(hip, t, w, n, k, x, m, c):
     before = hip.stat("launches")
     hip.gemm_q(t, w, n, k, x, m, c)
-    assert launches is None or hip.stat("launches") - before == launches
+    return hip.stat("launches") - before
+
+
+def _check(hip, t, raw, n, k, a, m, launches=None):
+    c = hip.alloc(4 * m * n)
+    w, x = hip.to_device(raw), hip.to_device(a)
+    hip.set_option("gemm.few", 0)
+    try:
+        passes = _launches(hip, t, w, n, k, x, m, c)
+    finally:
+        hip.set_option("gemm.few", 1)
+    hip.memset(c, 0xFF, 4 * m * n)
+    took = _launches(hip, t, w, n, k, x, m, c)
+    assert took < passes, "the shape takes the passes: nothing was tested"
+    assert launches is None or took == launches
     got = c.download(np.float32, m * n).reshape(m, n)
     wd = oracle_c.dequant(t, raw).astype(np.float64).reshape(n, k)
     xd = oracle_np.bf16_to_f32(a).astype(np.float64).reshape(m, k)
@@ -33,20 +45,20 @@ def _check(hip, t, raw, n, k, a, m, launches=None):
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
-@pytest.mark.parametrize("m,n,k,launches", [(1, 1, 256, 1), (2, 15, 512, 1), (15, 16, 2048, 1), (16, 17, 2304, 1), (17, 100, 1280, 1), (32, 31, 4096, 1), (33, 48, 4352, 2),
-                                            (48, 33, 6144, 2), (49, 4100, 4352, 1), (64, 20, 8192, 2), (5, 40, 11008, 2), (33, 4090, 4352, 1), (30, 4200, 512, 1)])
-def test_row_blocks_ragged_tiles_and_divided_k(hip, name, m, n, k, launches):
+@pytest.mark.parametrize("m,n,k", [(1, 1, 256), (2, 15, 512), (15, 16, 2048), (16, 17, 2304), (17, 100, 1280), (32, 31, 4096), (33, 48, 4352), (48, 33, 6144),
+                                   (49, 4100, 4352), (64, 20, 8192), (5, 40, 11008), (33, 4090, 4352), (30, 4200, 512)])
+def test_row_blocks_ragged_tiles_and_divided_k(hip, name, m, n, k):
     """One to four row blocks, full and ragged; fewer superblocks than wavefronts, as many, one more; few columns with k over
     workgroups; more tiles than compute units."""
     t = FORMATS[name]
-    _check(hip, t, synth.weight(t, n, k, seed=n + k + t), n, k, synth.activation_bf16((m, k), seed=m + 1), m, launches)
+    _check(hip, t, synth.weight(t, n, k, seed=n + k + t), n, k, synth.activation_bf16((m, k), seed=m + 1), m)
 
 
 @pytest.mark.parametrize("name", ["q5_k", "q8_0", "q4_0"])
 @pytest.mark.parametrize("m,n,k", [(33, 48, 2304), (48, 33, 256), (49, 16, 2048), (64, 65, 768), (40, 4200, 512), (50, 4200, 768)])
 def test_three_and_four_row_blocks_of_short_rows(hip, name, m, n, k):
     t = FORMATS[name]
-    _check(hip, t, synth.weight(t, n, k, seed=n + k + t), n, k, synth.activation_bf16((m, k), seed=m + 1), m, 1)
+    _check(hip, t, synth.weight(t, n, k, seed=n + k + t), n, k, synth.activation_bf16((m, k), seed=m + 1), m)
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
@@ -78,6 +90,27 @@ def test_rows_far_apart_and_fields_over_their_range(hip, name):
     x[2] = 0.0
     x[3, ::2] *= 2.0**40
     _check(hip, t, raw.reshape(-1), n, k, synth.f32_to_bf16_bits(x), m)
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("m", [7, 40])
+def test_without_room_for_parts_k_is_undivided(hip, name, m):
+    """The same bits as from a matrix of so many more columns that no unit is left to divide k; others than with k divided."""
+    assert hip.device_info()["compute_units"] == 256, "k is divided for 256 compute units"
+    t, n, wide, k = FORMATS[name], 192, 2304, 11008
+    raw, a = synth.weight(t, wide, k, seed=m), synth.activation_bf16((m, k), seed=m + 1)
+    w, x, c = hip.to_device(raw), hip.to_device(a), hip.alloc(4 * m * wide)
+    assert _launches(hip, t, w, wide, k, x, m, c) == 1
+    want = c.download(np.float32, m * wide).reshape(m, wide)[:, :n]
+    assert _launches(hip, t, w, n, k, x, m, c) == 2
+    divided = c.download(np.float32, m * n).reshape(m, n)
+    hip.set_option("test.gemm_no_parts", 2)
+    try:
+        assert _launches(hip, t, w, n, k, x, m, c) == 1
+    finally:
+        hip.set_option("test.gemm_no_parts", 0)
+    got = c.download(np.float32, m * n).reshape(m, n)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)) and not np.array_equal(got, divided)
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
@@ -174,9 +207,7 @@ def test_a_call_of_few_rows_readies_a_captured_one_of_more_columns(name, m, n, w
         ctx.set_stream(stream)
         w, x = ctx.to_device(synth.weight(t, wide, k, seed=n)), ctx.to_device(synth.activation_bf16((m, k), seed=m))
         c = ctx.alloc(4 * m * wide)
-        before = ctx.stat("launches")
-        ctx.gemm_q(t, w, n, k, x, m, c)
-        few = ctx.stat("launches") - before
+        few = _launches(ctx, t, w, n, k, x, m, c)
         ctx.sync()
         before = ctx.stat("launches")
         call("hipStreamBeginCapture", stream, 1)  # (of this thread's calls)
