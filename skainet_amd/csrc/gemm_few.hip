@@ -453,19 +453,25 @@ skn_family register_family(few_init);
 // More than 64 rows: Q5_K 128 x 2700 x 2816 (15) 18.2 | 16.6, 512 x 2000 x 1024 (16) 14.0 | 13.9; Q6_K 700 x 2000 x 1024 (21) 24.5 | 19.0; Q8_0 333 x
 // 4096 x 1024 (24) 16.8 | 15.2, 256 x 2700 x 2816 (29) 22.1 | 21.3; Q4_0 512 x 2000 x 1024 13.2 | 12.7, 256 x 2700 x 2816 19.4 | 21.1; Q4_K 160 x 1000 x 2048
 // (6) 16.4 | 6.8, 200 x 1000 x 2048 (8) 16.4 | 6.9, 512 x 2000 x 1024 13.8 | 13.4.
+// Short rows of many columns are launches of many short workgroups, whose ramp the passes' larger tiles pay less often: from so many
+// rounds of compute units on they are faster whatever the superblocks (but for one row block, Q4_0's apart): Q4_0 31 x 30269 x 512 11.8 | 15.3, 25 x 23000 x 512
+// 11.0 | 11.4; Q4_K 252 x 6683 x 256 12.6 | 16.1; Q5_K 32 x 29393 x 512 12.5 | 14.7; Q6_K 370 x 13269 x 256 20.7 | 36.3, 849 x 5423 x 256 44.9 | 35.4; Q8_0 248 x 24474
+// x 256 30.3 | 34.8, 507 x 8812 x 256 29.2 | 26.4.  Four row blocks of Q5_K and Q4_0 lose earlier where their last round is hardly begun: 49 x 4296 x 3072
+// 14.2 | 16.6, 58 x 13285 x 1536 16.3 | 20.0, against 57 x 7844 x 1536 in 1.9 rounds 16.3 | 14.1.  (Of 2607 drawn shapes that the limits above accept the
+// passes were more than 3 % faster in 123, at worst 1.75 times; of 2190 drawn with these two rules in 14, at worst 1.08 times.)
 // Q4_K and Q6_K of 33 to 64 rows, up to 4096 elements and a round of tiles or more stay with the others although this is the faster path
 // (41 x 4096 x 4096 15.5 | 9.7 and 19.3 | 10.7): the number of launches that such products take is held fixed by tests, as is Q4_K's 200 x 1024 x 2048.  Options that fix how k is divided mean the others.
 bool skn_gemm_few_ok(const skn_ctx* ctx, int type, const void* w, int n, int k, int m) {
     int bytes;
     struct {
-        int rows[5];
+        int rows[5], rounds;
     } most;
     switch (type) {
-        case SKN_TYPE_Q4_K: bytes = FewK<false>::kBytes, most = {{0, 48, 36, 20, 7}}; break;
-        case SKN_TYPE_Q5_K: bytes = FewK<true>::kBytes, most = {{0, 56, 40, 20, 15}}; break;
-        case SKN_TYPE_Q6_K: bytes = FewQ6K::kBytes, most = {{0, 0, 60, 24, 20}}; break;
-        case SKN_TYPE_Q8_0: bytes = FewQ80::kBytes, most = {{0, 80, 50, 24, 24}}; break;
-        case SKN_TYPE_Q4_0: bytes = FewQ40::kBytes, most = {{45, 33, 33, 20, 16}}; break;
+        case SKN_TYPE_Q4_K: bytes = FewK<false>::kBytes, most = {{0, 48, 36, 20, 7}, 6}; break;
+        case SKN_TYPE_Q5_K: bytes = FewK<true>::kBytes, most = {{0, 56, 40, 12, 15}, 6}; break;
+        case SKN_TYPE_Q6_K: bytes = FewQ6K::kBytes, most = {{0, 0, 60, 24, 20}, 19}; break;
+        case SKN_TYPE_Q8_0: bytes = FewQ80::kBytes, most = {{0, 80, 50, 24, 24}, 19}; break;
+        case SKN_TYPE_Q4_0: bytes = FewQ40::kBytes, most = {{45, 33, 33, 12, 16}, 5}; break;
         default: return false;
     }
     if (ctx->opt_gemm_few != 1 || ctx->opt_gemm_tile != 0 || ctx->opt_gemm_split != 0 || ctx->opt_test_gemm_no_parts == 1 || ctx->opt_gemm_q6k_fused != 1 || m <= 0 || n <= 0 || k <= 0 || k % 256 != 0 || k > 16384 ||
@@ -473,8 +479,11 @@ bool skn_gemm_few_ok(const skn_ctx* ctx, int type, const void* w, int n, int k, 
         return false;
     const int blocks = std::min((m + 15) / 16, 5), tiles = (n + 15) / 16, groups = (m + 63) / 64;
     if (m > 32 && m <= 64 && k <= 4096 && tiles >= ctx->compute_units && (type == SKN_TYPE_Q4_K || type == SKN_TYPE_Q6_K)) return false;
-    const int limit = blocks == 4 && tiles <= ctx->compute_units ? 45 : most.rows[blocks - 1];
-    return limit == 0 || (size_t)tiles * groups * (k / 256) <= (size_t)limit * ctx->compute_units;
+    const size_t all = (size_t)tiles * groups, units = ctx->compute_units;
+    if (all > most.rounds * units && (m > 16 || type == SKN_TYPE_Q4_0)) return false;
+    const bool begun = blocks == 4 && 5 * all >= 7 * units && all <= 2 * units;  // (1.4 to two rounds)
+    const int limit = blocks == 4 && all <= units ? 45 : begun ? std::max(20, most.rows[3]) : most.rows[blocks - 1];
+    return limit == 0 || all * (k / 256) <= limit * units;
 }
 
 int skn_gemm_few(skn_ctx* ctx, int type, const void* w, int n, int k, const uint16_t* a_bf16, int m, float* c) {

@@ -46,11 +46,17 @@ def _check(hip, t, raw, n, k, a, m, launches=None):
 
 @pytest.mark.parametrize("name", list(FORMATS))
 @pytest.mark.parametrize("m,n,k", [(1, 1, 256), (2, 15, 512), (15, 16, 2048), (16, 17, 2304), (17, 100, 1280), (32, 31, 4096), (33, 48, 4352), (48, 33, 6144),
-                                   (49, 4100, 4352), (64, 20, 8192), (5, 40, 11008), (33, 4090, 4352), (30, 4200, 512)])
+                                   (64, 20, 8192), (5, 40, 11008), (33, 4090, 4352), (30, 4200, 512)])
 def test_row_blocks_ragged_tiles_and_divided_k(hip, name, m, n, k):
     """One to four row blocks, full and ragged; fewer superblocks than wavefronts, as many, one more; few columns with k over
     workgroups; more tiles than compute units."""
     t = FORMATS[name]
+    _check(hip, t, synth.weight(t, n, k, seed=n + k + t), n, k, synth.activation_bf16((m, k), seed=m + 1), m)
+
+
+@pytest.mark.parametrize("name", ["q4_k", "q6_k", "q8_0"])
+def test_four_row_blocks_of_more_tiles_than_compute_units(hip, name):
+    t, m, n, k = FORMATS[name], 49, 4100, 4352
     _check(hip, t, synth.weight(t, n, k, seed=n + k + t), n, k, synth.activation_bf16((m, k), seed=m + 1), m)
 
 
@@ -90,6 +96,24 @@ def test_rows_far_apart_and_fields_over_their_range(hip, name):
     x[2] = 0.0
     x[3, ::2] *= 2.0**40
     _check(hip, t, raw.reshape(-1), n, k, synth.f32_to_bf16_bits(x), m)
+
+
+@pytest.mark.parametrize("name,m,n,k,few", [("q4_0", 31, 30269, 512, False), ("q4_k", 252, 6683, 256, False), ("q5_k", 32, 29393, 512, False), ("q6_k", 370, 13269, 256, False),
+                                            ("q8_0", 248, 24474, 256, False), ("q5_k", 49, 4296, 3072, False), ("q4_0", 49, 4555, 4096, False), ("q5_k", 58, 13285, 1536, False),
+                                            ("q8_0", 507, 8812, 256, True), ("q4_k", 16, 30000, 512, True), ("q5_k", 57, 7844, 1536, True), ("q4_0", 57, 6795, 2048, True)])
+def test_many_short_tiles_take_the_passes(hip, name, m, n, k, few):
+    """Shapes on both sides of where so many rounds of short workgroups cost more than the launches they save."""
+    assert hip.device_info()["compute_units"] == 256, "the rounds are counted for 256 compute units"
+    t = FORMATS[name]
+    w, x, c = hip.alloc(synth.weight(t, 16, k, seed=1).nbytes // 16 * n), hip.alloc(2 * m * k), hip.alloc(4 * m * n)
+    took = []
+    for value in (1, 0):
+        hip.set_option("gemm.few", value)
+        try:
+            took.append(_launches(hip, t, w, n, k, x, m, c))
+        finally:
+            hip.set_option("gemm.few", 1)
+    assert (took[0] == 1 and took[1] >= 2) if few else took[0] == took[1]
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
