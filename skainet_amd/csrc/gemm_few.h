@@ -1,4 +1,4 @@
-// Products of few bf16 activation rows with Q4_K, Q5_K, Q6_K, Q8_0 or Q4_0 weights in one launch (internal to the library).
+// Products of few bf16 activation rows with Q4_K, Q5_K, Q6_K, Q8_0 or Q4_0 weights in one launch, two where k is divided (internal to the library).
 #pragma once
 #include "common.h"
 

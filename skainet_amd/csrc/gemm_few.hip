@@ -1,17 +1,17 @@
 // Product of few activation rows, or of some more with a small matrix, with block-quantized weights: C[m, n] = sum_k A[m, k] w[n, k], A bf16 as it is given, Q4_K, Q5_K,
-// Q6_K, Q8_0 or Q4_0 weights, one launch and no workspace.
+// Q6_K, Q8_0 or Q4_0 weights: one launch, or two and room for the parts where few columns have their k divided.
 //
 // Bound by the latency of a launch, then by the unpacking.  The kernels for more rows (gemm.hip, gemm_blocks.hip) take three
 // launches where tiles are few: a pass that scales the rows to fp16, the product, the addition of the parts of k.  None of it is
-// needed here.  A quant less its zero has at most eight bits, exact in bf16, so the matrix cores take the activations as they are
+// needed here but, for few columns, the last.  A quant less its zero has at most eight bits, exact in bf16, so the matrix cores take the activations as they are
 // (v_mfma_f32_16x16x32_bf16; products exact, sums in fp32), a block's sum starts from zero and joins the total in fp32 times the
 // block's scale: an accumulator's column is the lane's own weight row, so the scale is one value per lane.  Minima: the block's
 // activations against a column of ones is one more matrix instruction and gives the sum that the minimum is multiplied with.
-// A workgroup keeps all of k for its sixteen columns: its eight (or four) wavefronts take superblocks of 256 in
+// A workgroup keeps all of k, or its part, for its sixteen columns: its eight (or four) wavefronts take superblocks of 256 in
 // turn and add their tiles through LDS.
 //
-// us per call, three launches -> this: Q4_K 16 x 4096 x 4096 11.8 -> 5.0, Q8_0 16 x 4096 x 4096 13.4 -> 6.3, Q6_K 41 x 4096 x 11008 33.7 -> 21.5 (weights
-// alone 7.5 at the rate of a copy), Q5_K 16 x 1000 x 1024 9.4 -> 4.6.  Error against 64 bits: not larger (1.1 against 1.5e-7 of the
+// us per call, three launches -> this: Q4_K 16 x 4096 x 4096 11.7 -> 5.3, Q8_0 16 x 4096 x 4096 13.1 -> 6.4, Q6_K 41 x 4096 x 11008 33.5 -> 21.1 (weights
+// alone 7.5 at the rate of a copy), Q5_K 64 x 2048 x 2048 12.9 -> 7.0.  Error against 64 bits: not larger (1.1 against 1.5e-7 of the
 // result in Q4_K at k = 11008, 0.95 against 1.05 in Q8_0): a superblock's sum is formed before it joins the total.
 #include "gemm_few.h"
 #include "gemm_few_loads.h"
