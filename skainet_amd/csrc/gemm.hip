@@ -193,7 +193,7 @@ __global__ __launch_bounds__(64 * R) void prep_a_frag_kernel(const skn_gemm_src 
     }
 }
 
-// The same preparation with a row spread over four wavefronts (k <= 16384): every element is read from memory once and
+// The same preparation with a row spread over four wavefronts (k <= 16384; two up to k = 1024): every element is read from memory once and
 // stays in registers through the three steps that the one-wavefront-per-row kernel above makes three passes for (sum of
 // squares, largest magnitude, conversion), two rows per workgroup.  Thread t of a row takes
 // tasks t, t + 256, ... (task = chunk c, nibble dword dw: four elements at 64 c + 4 dw and four at 64 c + 32 + 4 dw);
@@ -203,14 +203,16 @@ __global__ __launch_bounds__(64 * R) void prep_a_frag_kernel(const skn_gemm_src 
 // SIMD hide each other's.  us, two wavefronts a row and the weights asked for when the norm was known -> this: 512 rows of 4096 behind a
 // norm 7.9 -> 7.4, 41 rows 5.8 -> 5.0 (0.1 to 0.2 of them for the order of the squares below); without a norm 2000 rows of 8192 25.2 -> 22.9,
 // 512 rows of 11008 11.8 -> 11.7.
-template <int NT, int SRC, bool SUMS>
-__global__ __launch_bounds__(512) void prep_a_rows_kernel(const skn_gemm_src src, _Float16* __restrict__ afrag,
+// Rows of up to 1024 elements have a task for 128 threads only: two wavefronts a row there.  us of a Q4_K call, four | two wavefronts: 4000 x
+// 2048 x 256 22.7 | 20.0, 4000 x 2048 x 1024 36.1 | 32.9, 130 x 12000 x 512 16.6 | 16.2.
+template <int NT, int SRC, bool SUMS, int T>
+__global__ __launch_bounds__(2 * T) void prep_a_rows_kernel(const skn_gemm_src src, _Float16* __restrict__ afrag,
                                                          float* __restrict__ inv_scale, _Float16* __restrict__ sfrag,
                                                          int m, int k) {
-    constexpr int T = 256;  // threads of a row
-    __shared__ float red_ss[2][2], red_mx[2][4];
-    __shared__ float upper[SRC == SKN_SRC_RMSNORM ? 2 * NT * (T / 2) : 1];
-    const int tid = threadIdx.x, t = tid & (T - 1), rw = tid / T, wv = (tid >> 6) & 3;
+    static_assert(T == 128 || T == 256);  // threads of a row
+    __shared__ float red_ss[2][2], red_mx[2][T / 64];
+    __shared__ float upper[SRC == SKN_SRC_RMSNORM && T == 256 ? 2 * NT * 128 : 1];
+    const int tid = threadIdx.x, t = tid & (T - 1), rw = tid / T, wv = (tid >> 6) & (T / 64 - 1);
     const int n_pairs = gridDim.x, per_xcd = n_pairs >> 3;
     const int pair = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     const int row = 2 * pair + rw;
@@ -247,18 +249,20 @@ __global__ __launch_bounds__(512) void prep_a_rows_kernel(const skn_gemm_src src
     if constexpr (SRC == SKN_SRC_RMSNORM) {
         // A row's sum of squares does not depend on how many wavefronts a row has: tasks u, u + 128, ... in turn (u < 128), then the
         // lanes of a wavefront, then the two halves.  The upper two wavefronts hand their tasks' sums to the lower two.
-        float* const theirs = upper + rw * NT * (T / 2) + (t & (T / 2 - 1));
-        if (t >= T / 2) {
+        float* const theirs = upper + (T == 256 ? rw * NT * 128 + (t & 127) : 0);
+        if constexpr (T == 256) {
+            if (t >= 128) {
 #pragma unroll
-            for (int j = 0; j < NT; j++) theirs[j * (T / 2)] = squares[j];
+                for (int j = 0; j < NT; j++) theirs[j * 128] = squares[j];
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        if (t < T / 2) {
+        if (t < 128) {
             float ss = 0.f;
 #pragma unroll
             for (int j = 0; j < NT; j++) {
                 if (t + T * j < tasks) ss += squares[j];
-                if (t + T * j + T / 2 < tasks) ss += theirs[j * (T / 2)];
+                if (T == 256 && t + T * j + 128 < tasks) ss += theirs[j * 128];
             }
             ss = wave_sum(ss);
             if ((tid & 63) == 0) red_ss[rw][wv] = ss;
@@ -289,7 +293,9 @@ __global__ __launch_bounds__(512) void prep_a_rows_kernel(const skn_gemm_src src
     mx = wave_max(mx);
     if ((tid & 63) == 0) red_mx[rw][wv] = mx;
     __syncthreads();
-    mx = real ? fmaxf(fmaxf(red_mx[rw][0], red_mx[rw][1]), fmaxf(red_mx[rw][2], red_mx[rw][3])) : 0.f;
+    mx = fmaxf(red_mx[rw][0], red_mx[rw][1]);
+    if constexpr (T == 256) mx = fmaxf(mx, fmaxf(red_mx[rw][2], red_mx[rw][3]));
+    if (!real) mx = 0.f;
     int e = 9;  // a zero row keeps scale 1
     if (mx > 0.f) e = (int)((__float_as_uint(mx) >> 23) & 0xFF) - 127;
     e = max(e, -100);
@@ -337,10 +343,11 @@ void launch_prep(skn_ctx* ctx, const skn_gemm_src& src, _Float16* afrag, float* 
     if (k <= 16384 && m_pad % 16 == 0) {
         const dim3 grid(m_pad / 2), block(512);
         const int nt = (k / 8 + 255) / 256;
-        if (nt <= 2) skn_launch(ctx, prep_a_rows_kernel<2, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
-        else if (nt <= 4) skn_launch(ctx, prep_a_rows_kernel<4, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
-        else if (nt <= 6) skn_launch(ctx, prep_a_rows_kernel<6, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
-        else skn_launch(ctx, prep_a_rows_kernel<8, SRC, SUMS>, grid, block, 0, src, afrag, isc, sfrag, m, k);
+        if (k <= 1024) skn_launch(ctx, prep_a_rows_kernel<1, SRC, SUMS, 128>, grid, dim3(256), 0, src, afrag, isc, sfrag, m, k);
+        else if (nt <= 2) skn_launch(ctx, prep_a_rows_kernel<2, SRC, SUMS, 256>, grid, block, 0, src, afrag, isc, sfrag, m, k);
+        else if (nt <= 4) skn_launch(ctx, prep_a_rows_kernel<4, SRC, SUMS, 256>, grid, block, 0, src, afrag, isc, sfrag, m, k);
+        else if (nt <= 6) skn_launch(ctx, prep_a_rows_kernel<6, SRC, SUMS, 256>, grid, block, 0, src, afrag, isc, sfrag, m, k);
+        else skn_launch(ctx, prep_a_rows_kernel<8, SRC, SUMS, 256>, grid, block, 0, src, afrag, isc, sfrag, m, k);
     } else {
         skn_launch(ctx, prep_a_frag_kernel<4, SRC, SUMS>, dim3(m_pad / 4), dim3(256), 0, src, afrag, isc, sfrag, m, k);
     }
