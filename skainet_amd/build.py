@@ -13,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -20,6 +21,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libskainet_hip.so")
 DENSE_LIB = os.path.join(HERE, "libskainet_dense.so")
+PYCALL = os.path.join(HERE, "_pycall" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 # the sources of the layer-list decoder over bf16 / fp32 weights and of nothing else (seconds to compile; the
 # block-quantized matvecs alone take minutes)
 DENSE_SOURCES = ("api", "kvcache", "stepper", "dense_gemm", "dense_matvec", "dense_rows", "attention_prefill", "attention_shared",
@@ -70,7 +72,19 @@ def build_library(jobs=8, verbose=False, save_temps=False, dense_only=False):
     # linked beside its place and moved there: no process ever loads a half-written library
     _run([hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wl,--no-undefined", "-o", lib + ".new", *objs])
     os.replace(lib + ".new", lib)
+    build_pycall()
     return lib
+
+
+def build_pycall():
+    """The Python callables of the hot entry points (csrc/pycall.c).  Without Python's headers or a C compiler the binding calls
+    through ctypes alone."""
+    include = sysconfig.get_paths()["include"]
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if cc is None or not os.path.exists(os.path.join(include, "Python.h")):
+        return
+    _run([cc, "-O2", "-Wall", "-shared", "-fPIC", "-I", include, os.path.join(CSRC, "pycall.c"), "-o", PYCALL + ".new"])
+    os.replace(PYCALL + ".new", PYCALL)
 
 
 def ensure_library():

@@ -220,8 +220,36 @@ def load_library():
             fn = getattr(lib, name)
             fn.restype = restype
             fn.argtypes = argtypes
+        _bind_direct(lib, path)
         _LIB = lib
     return _LIB
+
+
+# The calls that a program makes once per product or attention step: (context, arguments as their C functions take them) -> return
+# code.  csrc/pycall.c has the same for plain ints without the 1.2 us that ctypes takes; other arguments come here from there.
+def _matvec_q(handle, ggml_type, w, n, k, x, y):
+    return _LIB.skn_matvec_q(handle, ggml_type, _ptr(w), n, k, _ptr(x), _ptr(y))
+
+
+def _gemm_q(handle, ggml_type, w, n, k, a, m, c):
+    return _LIB.skn_gemm_q(handle, ggml_type, _ptr(w), n, k, _ptr(a), m, _ptr(c))
+
+
+def _attn_decode(handle, kv, q, n_ctx, scale, out):
+    return _LIB.skn_attn_decode(handle, kv, _ptr(q), n_ctx, scale, _ptr(out))
+
+
+def _bind_direct(lib, path):
+    global _matvec_q, _gemm_q, _attn_decode
+    try:
+        from . import _pycall
+    except ImportError:  # (not built: no headers of this Python)
+        return
+    if path == DENSE_LIB_PATH:
+        return
+    for name, general in (("matvec_q", _matvec_q), ("gemm_q", _gemm_q), ("attn_decode", _attn_decode)):
+        _pycall.bind(name, C.cast(getattr(lib, "skn_" + name), C.c_void_p).value, general)
+    _matvec_q, _gemm_q, _attn_decode = _pycall.matvec_q, _pycall.gemm_q, _pycall.attn_decode
 
 
 def _not_built(name):
@@ -360,7 +388,9 @@ class KVCache:
         arr = None if n_ctx is None else (C.c_int32 * len(n_ctx))(*[int(v) for v in n_ctx])
         if n_ctx is not None and len(n_ctx) != self.n_seq:
             raise ValueError("n_ctx needs one entry per sequence")
-        self.ctx._check(self.ctx.lib.skn_attn_decode(self.ctx.handle, self.handle, _ptr(q_dev), arr, scale, _ptr(out_dev)))
+        rc = _attn_decode(self.ctx.handle, self.handle, q_dev, arr, scale, out_dev)
+        if rc:
+            self.ctx._check(rc)
 
     def attn_decode_static(self, q_dev, out_dev, scale):
         """skn_attn_decode over all cached tokens with the library's static scratch (allocates nothing)."""
@@ -625,10 +655,14 @@ class Context:
         self._check(self.lib.skn_dequant(self.handle, ggml_type, _ptr(w_dev), n_elems, _ptr(out_dev)))
 
     def matvec_q(self, ggml_type, w_dev, n, k, x_dev, y_dev):
-        self._check(self.lib.skn_matvec_q(self.handle, ggml_type, _ptr(w_dev), n, k, _ptr(x_dev), _ptr(y_dev)))
+        rc = _matvec_q(self.handle, ggml_type, w_dev, n, k, x_dev, y_dev)
+        if rc:
+            self._check(rc)
 
     def gemm_q(self, ggml_type, w_dev, n, k, a_bf16_dev, m, c_dev):
-        self._check(self.lib.skn_gemm_q(self.handle, ggml_type, _ptr(w_dev), n, k, _ptr(a_bf16_dev), m, _ptr(c_dev)))
+        rc = _gemm_q(self.handle, ggml_type, w_dev, n, k, a_bf16_dev, m, c_dev)
+        if rc:
+            self._check(rc)
 
     def gemm_expanded_bytes(self, ggml_type, n, k):
         out = C.c_size_t(0)

@@ -1,0 +1,77 @@
+"""The direct Python callables of the hot entry points hand over what ctypes hands over, and leave everything else to it."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from skainet_amd import runtime
+
+pycall = pytest.importorskip("skainet_amd._pycall")
+
+_V, _I = C.c_void_p, C.c_int
+SIGNATURES = {"matvec_q": [_V, _I, _V, _I, _I, _V, _V], "gemm_q": [_V, _I, _V, _I, _I, _V, _I, _V],
+              "attn_decode": [_V, _V, _V, C.POINTER(C.c_int32), C.c_float, _V]}
+CASES = {
+    "matvec_q": [(1, 12, 2, 3, 4, 5, 6), (2**48 + 16, 14, 2**63 + 32, -1, 2**31 - 1, 2**64 - 16, 0), (-16, 12, 2**64 + 16, 2**32 + 7, -2**31, 1, 1),
+                 (1, np.int64(12), np.int64(64), 3, 4, None, 6), (1, True, 2, 3, 4, 5, 6)],
+    "gemm_q": [(1, 8, 2, 3, 4, 5, 6, 7), (2**48, 13, 2**63, -5, 2**33 + 1, 2**50, 2**40, 2**62), (1, 8, None, 3, 4, 5, 6, 7)],
+    "attn_decode": [(1, 2, 3, None, 0.0883883, 4), (2**48, 2**63, 2**50, None, 1e-50, 0), (1, 2, 3, (C.c_int32 * 2)(7, 9), 0.5, 4), (1, 2, 3, None, 1, 4)],
+}
+
+
+@pytest.mark.parametrize("name,args", [(n, a) for n in CASES for a in CASES[n]])
+def test_the_arguments_arrive_as_through_ctypes(name, args):
+    seen = []
+
+    def record(*a):
+        seen.append(tuple(None if v is None else v[0:2] if isinstance(v, C.POINTER(C.c_int32)) and v else float(v) if isinstance(v, float) else
+                          None if isinstance(v, C.POINTER(C.c_int32)) else v for v in a))
+        return -7
+
+    fn = C.CFUNCTYPE(C.c_int, *SIGNATURES[name])(record)
+    lib = runtime.load_library()
+
+    def general(*a):
+        return fn(*[runtime._ptr(v) if t is _V else v for v, t in zip(a, SIGNATURES[name])])
+
+    at = C.cast(fn, C.c_void_p).value
+    library_at = C.cast(getattr(lib, "skn_" + name), C.c_void_p).value
+    try:
+        pycall.bind(name, at, general)
+        assert getattr(pycall, name)(*args) == -7
+        assert general(*args) == -7
+    finally:
+        pycall.bind(name, library_at, _GENERAL[name])
+    assert seen[0] == seen[1]
+
+
+def _refuse(*_):
+    raise TypeError("the general call")
+
+
+@pytest.mark.parametrize("name,args", [("matvec_q", (1, 12, 2, 3, 4, 5)), ("matvec_q", (1, 12.0, 2, 3, 4, 5, 6)), ("gemm_q", (1, 12, "w", 3, 4, 5, 6, 7)),
+                                       ("attn_decode", (1, 2, 3, [4], 0.5, 5))])
+def test_other_arguments_go_to_the_general_call(name, args):
+    lib = runtime.load_library()
+    library_at = C.cast(getattr(lib, "skn_" + name), C.c_void_p).value
+    try:
+        pycall.bind(name, library_at, _refuse)
+        with pytest.raises(TypeError, match="the general call"):
+            getattr(pycall, name)(*args)
+    finally:
+        pycall.bind(name, library_at, _GENERAL[name])
+
+
+def _matvec(handle, ggml_type, w, n, k, x, y):
+    return runtime.load_library().skn_matvec_q(handle, ggml_type, runtime._ptr(w), n, k, runtime._ptr(x), runtime._ptr(y))
+
+
+def _gemm(handle, ggml_type, w, n, k, a, m, c):
+    return runtime.load_library().skn_gemm_q(handle, ggml_type, runtime._ptr(w), n, k, runtime._ptr(a), m, runtime._ptr(c))
+
+
+def _attn(handle, kv, q, n_ctx, scale, out):
+    return runtime.load_library().skn_attn_decode(handle, kv, runtime._ptr(q), n_ctx, scale, runtime._ptr(out))
+
+
+_GENERAL = {"matvec_q": _matvec, "gemm_q": _gemm, "attn_decode": _attn}
