@@ -44,7 +44,15 @@ __global__ __launch_bounds__(256) void attn_frag_kernel(const uint16_t* __restri
     constexpr int kPieces = D / 8;             // 16-byte pieces of a row
     constexpr int kPitch = D + 8;              // LDS row pitch in halves
     __shared__ __align__(16) uint16_t vt[32 * kPitch];
-    const int tile = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
+    // (a head's tiles by the XCD that will read them: the pages of a head come through one L2 and its operands leave through the same;
+    // 512 x 32 heads of 128 6.4 -> 4.6 us)
+    int tile = blockIdx.x, head = blockIdx.y;
+    if (gridDim.y % 8 == 0) {
+        const int id = tile + (int)gridDim.x * head;
+        tile = (id >> 3) % (int)gridDim.x;
+        head = (id & 7) + 8 * ((id >> 3) / (int)gridDim.x);
+    }
+    const int tid = threadIdx.x;
     u32x4* kout = kfrag + ((size_t)head * n_tiles + tile) * (D / 16) * 64;
     u32x4* vout = vfrag + ((size_t)head * n_tiles + tile) * (D / 16) * 64;
     for (int i = tid; i < 32 * kPieces; i += 256) {
@@ -83,7 +91,7 @@ __global__ __launch_bounds__(256) void attn_frag_kernel(const uint16_t* __restri
     }
 }
 
-// grid (query blocks of 32, heads), four wavefronts each; the block with the most keys first.
+// Workgroups of four wavefronts, one per 32 query rows and head, the blocks with the most keys first.
 // q, out: fp32 [n_queries][n_head][D]; query row t attends to keys [0, first_ctx + t).
 // Keys are DK, values DV elements wide (one size D except where a latent's expanded keys carry a rotated part).
 // kBias: the scores lose slope_h * distance, slope_h = 2^(-8 (h + 1) / n_head).  kRanged: a query sees a range of the keys, scores
@@ -102,17 +110,37 @@ struct PrefillExt {
 // What bounds it: the vector instructions of the softmax between the matrix products (45 % of the clocks of a SIMD against 22 % of
 // matrix instructions at 2000 queries, 32 heads of 64), so the loop has as few as it can: a weight is one exp2 instruction, no test per
 // element for a query that has seen nothing yet, masks only in tiles where some query needs them; the four wavefronts share the
-// merge.  Whole calls with the copy of the keys, before and after: 2000 x 32 heads x 64 87.8 -> 66.6 us, 2048 x 16 x 128
-// 87.2 -> 76.2, 512 x 32 x 128 27.9 -> 26.2, 1000 x 32 x 64 37.1 -> 30.3.  Three wavefronts per SIMD where the registers allow it (D = 64).
+// merge.  Whole calls with the copy of the keys, with the longer loop and with this one: 2000 x 32 heads x 64 87.8 | 66.6 us, 2048 x 16 x 128
+// 87.2 | 76.2; with the rows of q and the placement below 55 and 59 (512 x 32 x 128 26.6 -> 18.5, 1000 x 32 x 64 31 -> 21.6).  Three wavefronts per SIMD where the registers allow it (D = 64).
+// The block of queries and the head of a workgroup.  Workgroups go to the eight XCDs in turn, and each XCD has an L2 of its own (4
+// MiB): the heads that read one cached head stay on one XCD where there are eight of them or a multiple, so that its keys and values
+// come through one L2 only.  In the plain order every XCD read every head, more than its L2 holds, and that traffic was half the time:
+// 512 x 32 heads of 128 25.6 -> 20.1 us, 2048 x 16 of 128 76 -> 60, 1000 x 32 of 64 30 -> 23.7, 2000 x 32 of 64 64 -> 56.  Other counts of
+// heads: the plain order.
+__device__ __forceinline__ void prefill_place(int id, int q_blocks, int n_head, int kv_group, int& qb, int& head) {
+    const int group = (n_head / kv_group) % 8 == 0 ? kv_group : 1, units = n_head / group;
+    if (units % 8 == 0) {
+        const int slot = id >> 3, row = units / 8 * group;  // (of an XCD: all of its heads for one block of queries, then the next block)
+        const int i = slot % row;
+        qb = q_blocks - 1 - slot / row;
+        head = ((id & 7) + 8 * (i / group)) * group + i % group;
+    } else {
+        qb = q_blocks - 1 - id % q_blocks;
+        head = id / q_blocks;
+    }
+}
+
 template <int DK, int DV, int KIND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DK > 128 ? 1 : DK > 64 ? 2 : 3))) void attn_prefill_kernel(const float* __restrict__ q, const u32x4* __restrict__ kfrag,
                                                           const u32x4* __restrict__ vfrag, float* __restrict__ out,
                                                           int n_queries, int n_head, int kv_group, int first_ctx, int n_tiles,
                                                           float scale_log2e, PrefillExt ext) {
     constexpr int KS = DK / 16, VS = DV / 16, DB = DV / 32;
-    __shared__ float part[4][DB * 16 + 2][64];  // running maximum, sum and accumulators of the wavefronts
+    __shared__ __align__(16) float part[4][DB * 16 + 2][64];  // running maximum, sum and accumulators of the wavefronts
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, n = lane & 31;
-    const int qb = (int)gridDim.x - 1 - (int)blockIdx.x, head = blockIdx.y;
+    const int q_blocks = (n_queries + 31) >> 5;
+    int qb, head;
+    prefill_place(blockIdx.x, q_blocks, n_head, kv_group, qb, head);
     const int t = min(32 * qb + n, n_queries - 1);  // (rows past the end repeat the last one and are not stored)
     const int n_ctx = first_ctx + t;                // keys this lane's query sees
     // the last tile any query of the block needs
@@ -124,19 +152,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DK > 128 ? 
     const int first_key = KIND == kRanged ? ext.range.first(n_ctx - 1) : 0;
     const int last_first_key = KIND == kRanged ? ext.range.first(first_ctx + min(32 * qb + 31, n_queries - 1) - 1) : 0;  // of the block's last query
 
-    // q as the column operand: lane 32 h + n holds elements 16 s + 8 h .. + 7 of query n, as an fp16 pair
+    // (grouped queries: kv_group consecutive query heads read the keys and values of one cached head)
+    const u32x4* kp = kfrag + ((size_t)(head / kv_group) * n_tiles - tile0) * KS * 64 + lane;
+    const u32x4* vp = vfrag + ((size_t)(head / kv_group) * n_tiles - tile0) * VS * 64 + lane;
+    u32x4 kf[KS];
+#pragma unroll
+    for (int s = 0; s < KS; s++) kf[s] = kp[((size_t)min(first_tile + wave, last_tile) * KS + s) * 64];
+    // q as the column operand: lane 32 h + n holds elements 16 s + 8 h .. + 7 of query n, as an fp16 pair.  The rows come in whole, once
+    // for the workgroup, and change hands in LDS (16-byte unit u of row r at u ^ (r & 15): sixteen rows' units in different banks).  Read
+    // by each wavefront in operand order a request was 32 rows of 32 bytes: 512 x 32 heads of 128 26.4 -> 25.6 us, 1000 x 32 of 64
+    // 30.7 -> 29.9 (whole calls, here and below).
     half8_t qh[KS], ql[KS];
-    const float* qr = q + ((size_t)t * n_head + head) * DK + 8 * h;
-#pragma unroll
-    for (int s = 0; s < KS; s++) {
-        const float4 a = *reinterpret_cast<const float4*>(qr + 16 * s), b = *reinterpret_cast<const float4*>(qr + 16 * s + 4);
-        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            _Float16 x, y;
-            skn_split_hilo(v[i] * scale_log2e, x, y);
-            qh[s][i] = x, ql[s][i] = y;
+    {
+        constexpr int kUnits = DK / 4;
+        float4* qs = reinterpret_cast<float4*>(&part[0][0][0]);
+        for (int i = threadIdx.x; i < 32 * kUnits; i += 256) {
+            const int r = i / kUnits, u = i - r * kUnits;
+            qs[r * kUnits + (u ^ (r & 15))] = reinterpret_cast<const float4*>(q + ((size_t)min(32 * qb + r, n_queries - 1) * n_head + head) * DK)[u];
         }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+            const float4 a = qs[n * kUnits + ((4 * s + 2 * h) ^ (n & 15))], b = qs[n * kUnits + ((4 * s + 2 * h + 1) ^ (n & 15))];
+            const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                _Float16 x, y;
+                skn_split_hilo(v[i] * scale_log2e, x, y);
+                qh[s][i] = x, ql[s][i] = y;
+            }
+        }
+        __syncthreads();  // (the merge writes over the rows)
     }
     float16_t o[DB];
 #pragma unroll
@@ -146,12 +192,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DK > 128 ? 
     const float slope = KIND == kBias ? exp2f(-8.0f * (float)(head + 1) / (float)n_head) * 1.4426950408889634f : 0.f;
     float mrun = -INFINITY, lrun = 0.f;  // running maximum (both halves agree) and this half's share of the sum
 
-    // (grouped queries: kv_group consecutive query heads read the keys and values of one cached head)
-    const u32x4* kp = kfrag + ((size_t)(head / kv_group) * n_tiles - tile0) * KS * 64 + lane;
-    const u32x4* vp = vfrag + ((size_t)(head / kv_group) * n_tiles - tile0) * VS * 64 + lane;
-    u32x4 kf[KS];
-#pragma unroll
-    for (int s = 0; s < KS; s++) kf[s] = kp[((size_t)min(first_tile + wave, last_tile) * KS + s) * 64];
     for (int tile = first_tile + wave; tile <= last_tile; tile += 4) {
         u32x4 vf[VS];
 #pragma unroll
@@ -304,7 +344,7 @@ int launch_prefill(skn_ctx* ctx, skn_kv* kv, int seq, const float* q_dev, int n_
                (const int32_t*)(kv->page_table_dev + (size_t)seq * kv->pages_per_seq), kv->n_head,
                kv->page_tokens, n_tokens, ext.tile0, n_tiles, kfrag, vfrag);
     SKN_LAUNCH_CHECK(ctx);
-    skn_launch(ctx, attn_prefill_kernel<D, D, KIND>, dim3((n_queries + 31) / 32, n_q_head), dim3(256), 0, q_dev, (const u32x4*)kfrag,
+    skn_launch(ctx, attn_prefill_kernel<D, D, KIND>, dim3((unsigned)((n_queries + 31) / 32) * n_q_head), dim3(256), 0, q_dev, (const u32x4*)kfrag,
                (const u32x4*)vfrag, out_dev, n_queries, n_q_head, n_q_head / kv->n_head, first_ctx, n_tiles,
                scale * 1.4426950408889634f, ext);
     SKN_LAUNCH_CHECK(ctx);
@@ -387,7 +427,7 @@ int launch_latent(skn_ctx* ctx, const uint16_t* k, int ldk, const uint16_t* rot,
     SKN_LAUNCH_CHECK(ctx);
     float scale;
     const PrefillExt ext = ranged_ext(p, token0 / 32, &scale);
-    skn_launch(ctx, attn_prefill_kernel<DK, DV, kRanged>, dim3((n_queries + 31) / 32, n_head), dim3(256), 0, q_prep, (const u32x4*)kfrag, (const u32x4*)vfrag,
+    skn_launch(ctx, attn_prefill_kernel<DK, DV, kRanged>, dim3((unsigned)((n_queries + 31) / 32) * n_head), dim3(256), 0, q_prep, (const u32x4*)kfrag, (const u32x4*)vfrag,
                (float*)p.out, n_queries, n_head, 1, pos0 + 1, n_tiles, scale * 1.4426950408889634f, ext);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
