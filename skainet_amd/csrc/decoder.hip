@@ -546,7 +546,7 @@ int skn_llama_free(skn_ctx* ctx, skn_llama* m) {
 int skn_llama_reset(skn_ctx* ctx, skn_llama* m) {
     SKN_REQUIRE(nullptr, ctx != nullptr, SKN_ERR_ARG, "skn_llama_reset: ctx is null");
     SKN_REQUIRE(ctx, m != nullptr, SKN_ERR_ARG, "skn_llama_reset: model is null");
-    for (skn_kv* kv : m->kv) SKN_TRY(skn_kv_reset(ctx, kv, 0));
+    for (skn_kv* kv : m->kv) skn_kv_release(kv, 0);
     m->pos = 0;
     return SKN_OK;
 }

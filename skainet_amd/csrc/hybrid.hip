@@ -760,7 +760,7 @@ int skn_hybrid_reset(skn_ctx* ctx, skn_hybrid* m) {
     SKN_REQUIRE(nullptr, ctx != nullptr, SKN_ERR_ARG, "skn_hybrid_reset: ctx is null");
     SKN_REQUIRE(ctx, m != nullptr, SKN_ERR_ARG, "skn_hybrid_reset: model is null");
     for (Layer& L : m->layers) {
-        if (L.owns_kv) SKN_TRY(skn_kv_reset(ctx, L.kv, 0));
+        if (L.owns_kv) skn_kv_release(L.kv, 0);
         if (L.state) SKN_TRY(skn_rstate_reset(ctx, L.state, 0));
     }
     m->pos = 0;

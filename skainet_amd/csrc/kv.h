@@ -30,7 +30,8 @@ struct skn_kv {
     int32_t* len_dev = nullptr;         // [n_seq] tokens held, the kernels' source of append positions
     int32_t* nctx_dev = nullptr;        // [n_seq] staging for explicit attention lengths
     int* ticket_dev = nullptr;          // workgroups of an append launch count themselves in (zero between launches)
-    std::vector<int32_t> page_table;    // host mirror
+    std::vector<int32_t> page_table;    // pages mapped, -1: none
+    std::vector<int32_t> page_table_on_device;  // what has been uploaded (entries of pages given back stay)
     std::vector<int32_t> len;           // host mirror
     std::vector<int32_t> free_pages;    // stack of unmapped page ids
     std::vector<int32_t> nctx_host;     // keeps explicit attention lengths alive while their upload is queued
@@ -38,6 +39,10 @@ struct skn_kv {
 
 // Maps pages so that sequence `seq` can hold `new_len` tokens; uploads new table entries on the stream.
 int skn_kv_reserve(skn_ctx* ctx, skn_kv* kv, int seq, int new_len);
+
+// Gives a sequence's pages back without the device length being set to zero (skn_kv_reset does both): for a decoder, whose kernels take
+// every length from elsewhere.
+void skn_kv_release(skn_kv* kv, int seq);
 
 // Counts n more tokens into a sequence whose rows were written by a kernel outside the cache code (pages reserved
 // by the caller): host mirror and device length.
