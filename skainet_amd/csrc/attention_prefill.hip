@@ -96,7 +96,7 @@ __global__ __launch_bounds__(256) void attn_frag_kernel(const uint16_t* __restri
 // Keys are DK, values DV elements wide (one size D except where a latent's expanded keys carry a rotated part).
 // kBias: the scores lose slope_h * distance, slope_h = 2^(-8 (h + 1) / n_head).  kRanged: a query sees a range of the keys, scores
 // may be capped (then scale_log2e carries 2 log2 e scale / cap), the softmax may have a sink, the output may be gated.
-// With either, the output is `dim` of DV elements per head in rows of ldo, fp32 or bf16.
+// With either, the output is `dim` of DV elements per head in rows of ldo; fp32 or bf16 in all.
 enum { kCausal = 0, kBias = 1, kRanged = 2 };
 struct PrefillExt {
     int dim = 0, ldo = 0, out_type = SKN_TYPE_F32;
@@ -299,7 +299,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DK > 128 ? 
             y[i] = v * inv;
         }
         if (KIND == kCausal) {
-            *reinterpret_cast<float4*>(out + ((size_t)t * n_head + head) * DV + d0) = make_float4(y[0], y[1], y[2], y[3]);
+            const size_t at = ((size_t)t * n_head + head) * DV + d0;
+            if (ext.out_type == SKN_TYPE_F32) *reinterpret_cast<float4*>(out + at) = make_float4(y[0], y[1], y[2], y[3]);
+            else
+                *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + at) =
+                    make_uint2(skn_bf16_bits(y[0]) | (uint32_t)skn_bf16_bits(y[1]) << 16, skn_bf16_bits(y[2]) | (uint32_t)skn_bf16_bits(y[3]) << 16);
             continue;
         }
 #pragma unroll
@@ -466,13 +470,16 @@ int skn_latent_prefill_launch(skn_ctx* ctx, const uint16_t* k, int ldk, const ui
 // Shared with the decoder.  Query row t of n_queries attends to the first first_ctx + t tokens of sequence seq
 // (first_ctx >= 1; all of them must be cached).  head_dim 64 or 128.
 int skn_attn_prefill_launch(skn_ctx* ctx, skn_kv* kv, int seq, const float* q_dev, int n_queries, int first_ctx, float scale,
-                            float* out_dev, int n_q_head) {
+                            void* out, int n_q_head, int out_type) {
+    float* out_dev = (float*)out;
+    PrefillExt ext;
+    ext.out_type = out_type;
     SKN_REQUIRE(ctx, kv->kind == SKN_KV_PLAIN, SKN_ERR_STATE, "attention: not a cache of fp16 keys and values (skn_attn_shared, _ranged and _latent read the others)");
     if (n_q_head <= 0) n_q_head = kv->n_head;
     SKN_REQUIRE(ctx, n_q_head % kv->n_head == 0, SKN_ERR_SHAPE,
                 "attention: %d query heads are not a multiple of the %d cached heads", n_q_head, kv->n_head);
-    if (kv->head_dim == 64) return launch_prefill<64, kCausal>(ctx, kv, seq, q_dev, n_queries, first_ctx, scale, out_dev, n_q_head);
-    if (kv->head_dim == 128) return launch_prefill<128, kCausal>(ctx, kv, seq, q_dev, n_queries, first_ctx, scale, out_dev, n_q_head);
+    if (kv->head_dim == 64) return launch_prefill<64, kCausal>(ctx, kv, seq, q_dev, n_queries, first_ctx, scale, out_dev, n_q_head, ext);
+    if (kv->head_dim == 128) return launch_prefill<128, kCausal>(ctx, kv, seq, q_dev, n_queries, first_ctx, scale, out_dev, n_q_head, ext);
     return skn_fail(ctx, SKN_ERR_SHAPE, "skn_attn_prefill: head_dim %d is not supported (64 or 128)", kv->head_dim);
 }
 

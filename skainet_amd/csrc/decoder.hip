@@ -25,7 +25,8 @@ struct skn_llama {
     // prompt buffers (grown to the longest prompt seen)
     int prompt_cap = 0;
     float *px = nullptr, *pxn = nullptr, *pq = nullptr, *pk = nullptr, *pv = nullptr, *patt = nullptr, *pproj = nullptr;
-    float *pgate = nullptr, *pup = nullptr, *pmid = nullptr, *ppartial = nullptr;
+    float *pgate = nullptr, *pup = nullptr, *ppartial = nullptr;
+    uint16_t* pmid = nullptr;  // the rows of a SwiGLU, as the products behind it take them
     uint16_t *pb16 = nullptr, *pk16 = nullptr, *pv16 = nullptr;
     int32_t *ptok = nullptr, *pnctx = nullptr;
     // fp16-pair copies of the matrices that are not Q4_K, for the prompt GEMMs (made on first use when the option
@@ -182,12 +183,18 @@ __global__ void add_rows_kernel(float* __restrict__ y, const float* __restrict__
     if (i < n) y[i] += x[i];
 }
 
-__global__ void swiglu_rows_kernel(const float* __restrict__ g, const float* __restrict__ u, float* __restrict__ out,
-                                   int64_t n) {
+__device__ __forceinline__ uint16_t bf16_bits(float x) {
+    const uint32_t u = __float_as_uint(x);
+    return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
+}
+
+template <typename OUT>  // float, or uint16_t: bf16
+__global__ void swiglu_rows_kernel(const float* __restrict__ g, const float* __restrict__ u, OUT* __restrict__ out, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
-        const float a = g[i];
-        out[i] = a / (1.0f + expf(-a)) * u[i];
+        const float a = g[i], y = a / (1.0f + expf(-a)) * u[i];
+        if constexpr (sizeof(OUT) == 2) out[i] = bf16_bits(y);
+        else out[i] = y;
     }
 }
 
@@ -372,7 +379,7 @@ int decode_step(skn_ctx* ctx, skn_llama* m, const AttnShape& shape) {
             SKN_LAUNCH_CHECK(ctx);
             SKN_TRY(skn_matvec_q(ctx, L.type_gate, L.w_gate, F, H, m->xn, m->gate));
             SKN_TRY(skn_matvec_q(ctx, L.type_up, L.w_up, F, H, m->xn, m->up));
-            skn_launch(ctx, swiglu_rows_kernel, dim3(nblk(F)), dim3(256), 0, (const float*)m->gate, (const float*)m->up,
+            skn_launch(ctx, swiglu_rows_kernel<float>, dim3(nblk(F)), dim3(256), 0, (const float*)m->gate, (const float*)m->up,
                        m->mid, (int64_t)F);
             SKN_LAUNCH_CHECK(ctx);
         }
@@ -571,14 +578,11 @@ static int expanded_copy(skn_ctx* ctx, skn_llama* m, int l, int which, int type,
     return SKN_OK;
 }
 
-// Prompt rows times up to three matrices of any formats, one activation source (fp32 rows, with RMSNorm when norm_w
-// is given).  Matrices whose GEMM unpacks the blocks itself (Q4_K, Q6_K, the formats in blocks of 32) go behind its fused
+// Prompt rows times up to three matrices of any formats, one activation source.  Matrices whose GEMM unpacks the blocks itself (Q4_K, Q6_K, the formats in blocks of 32) go behind its fused
 // activation pass -- the row-wise work inside the pass, one pass per kind of GEMM, a residual (`accumulate`) in the store --,
 // the others through a norm, a bf16 conversion, skn_gemm_q per matrix and an add.
 int project_rows(skn_ctx* ctx, skn_llama* m, const int* types, const void* const* blocks, const int* rows, float* const* outs,
-                 int count, int k, const float* x, const float* norm_w, int T, int accumulate) {
-    const skn_llama_config& c = m->cfg;
-    const skn_gemm_src src = {norm_w ? SKN_SRC_RMSNORM : SKN_SRC_F32, x, norm_w, norm_w ? c.rms_eps : 0.f};
+                 int count, int k, const skn_gemm_src& src, int T, int accumulate) {
     skn_gemm_seg q4[3], q6[3], bl[3];
     int n4 = 0, n6 = 0, nbl = 0, np = 0, bl_types[3], plain[3];
     for (int i = 0; i < count; i++) {
@@ -592,20 +596,26 @@ int project_rows(skn_ctx* ctx, skn_llama* m, const int* types, const void* const
     if (n6) SKN_TRY(skn_gemm_q6k_multi(ctx, q6, n6, k, src, T));
     if (nbl) SKN_TRY(skn_gemm_blocks_multi(ctx, bl_types, bl, nbl, k, src, T));
     if (!np) return SKN_OK;
-    if (norm_w) {
-        skn_launch(ctx, rmsnorm_rows_kernel, dim3(T), dim3(256), 0, x, norm_w, m->pxn, k, c.rms_eps);
-        SKN_LAUNCH_CHECK(ctx);
+    const uint16_t* rows16 = (const uint16_t*)src.a;
+    if (src.kind != SKN_SRC_BF16) {
+        const float* x = (const float*)src.a;
+        if (src.kind == SKN_SRC_RMSNORM) {
+            skn_launch(ctx, rmsnorm_rows_kernel, dim3(T), dim3(256), 0, x, (const float*)src.b, m->pxn, k, src.eps);
+            SKN_LAUNCH_CHECK(ctx);
+            x = m->pxn;
+        }
+        SKN_TRY(to_bf16(ctx, x, m->pb16, (int64_t)T * k));
+        rows16 = m->pb16;
     }
-    SKN_TRY(to_bf16(ctx, norm_w ? m->pxn : x, m->pb16, (int64_t)T * k));
     for (int j = 0; j < np; j++) {
         const int i = plain[j];
         if (accumulate) {
-            SKN_TRY(skn_gemm_q(ctx, types[i], blocks[i], rows[i], k, m->pb16, T, m->pproj));
+            SKN_TRY(skn_gemm_q(ctx, types[i], blocks[i], rows[i], k, rows16, T, m->pproj));
             skn_launch(ctx, add_rows_kernel, dim3(nblk((int64_t)T * rows[i])), dim3(256), 0, outs[i], (const float*)m->pproj,
                        (int64_t)T * rows[i]);
             SKN_LAUNCH_CHECK(ctx);
         } else {
-            SKN_TRY(skn_gemm_q(ctx, types[i], blocks[i], rows[i], k, m->pb16, T, outs[i]));
+            SKN_TRY(skn_gemm_q(ctx, types[i], blocks[i], rows[i], k, rows16, T, outs[i]));
         }
     }
     return SKN_OK;
@@ -616,8 +626,7 @@ int project_rows(skn_ctx* ctx, skn_llama* m, const int* types, const void* const
 // their blocks (us of a call's kernels, Q8_0, blocks | copy: 120 x 4096 x 4096 22.6 | 33.0, 333 x 4096 x 4096 39.0 | 36.5).  The copies
 // are made all the same: the option has the first prompt make them, whatever its length.
 static int project_expanded(skn_ctx* ctx, skn_llama* m, int l, int which, const int* types, const void* const* blocks, const int* rows, float* const* outs,
-                            int count, int k, const float* x, const float* norm_w, int T, int accumulate) {
-    const skn_gemm_src src = {norm_w ? SKN_SRC_RMSNORM : SKN_SRC_F32, x, norm_w, norm_w ? m->cfg.rms_eps : 0.f};
+                            int count, int k, const skn_gemm_src& src, int T, int accumulate) {
     skn_gemm_seg q4[3], ex[3], bl[3];
     int n4 = 0, nx = 0, nbl = 0, bl_types[3];
     for (int i = 0; i < count; i++) {
@@ -678,59 +687,58 @@ int skn_llama_prefill(skn_ctx* ctx, skn_llama* m, const int32_t* tokens_host, in
         // other formats with the option llama.expand_weights: their fp16-pair copies are kept, and the general GEMM
         // takes the fp32 rows as the Q4_K one does (norm and rounding inside its activation pass, residual in its store)
         const bool expand = ctx->opt_llama_expand != 0 && H % 64 == 0 && F % 64 == 0;
+        const skn_gemm_src normed = {SKN_SRC_RMSNORM, m->px, L.attn_norm, c.rms_eps}, normed2 = {SKN_SRC_RMSNORM, m->px, L.ffn_norm, c.rms_eps};
         if (q4k_qkv) {  // RMSNorm inside the activation pass, one launch for the three projections
             const skn_gemm_seg qkv[3] = {{L.wq, H, m->pq, 0}, {L.wk, KVD, m->pk, 0}, {L.wv, KVD, m->pv, 0}};
-            const skn_gemm_src src = {SKN_SRC_RMSNORM, m->px, L.attn_norm, c.rms_eps};
-            SKN_TRY(skn_gemm_q4k_multi(ctx, qkv, 3, H, src, T));
+            SKN_TRY(skn_gemm_q4k_multi(ctx, qkv, 3, H, normed, T));
         } else {
             const int types[3] = {L.type_q, L.type_k, L.type_v}, rows[3] = {H, KVD, KVD};
             const void* blocks[3] = {L.wq, L.wk, L.wv};
             float* outs[3] = {m->pq, m->pk, m->pv};
-            if (expand) SKN_TRY(project_expanded(ctx, m, l, 0, types, blocks, rows, outs, 3, H, m->px, L.attn_norm, T, 0));
-            else SKN_TRY(project_rows(ctx, m, types, blocks, rows, outs, 3, H, m->px, L.attn_norm, T, 0));
+            if (expand) SKN_TRY(project_expanded(ctx, m, l, 0, types, blocks, rows, outs, 3, H, normed, T, 0));
+            else SKN_TRY(project_rows(ctx, m, types, blocks, rows, outs, 3, H, normed, T, 0));
         }
         skn_launch(ctx, rope_store_kernel, rope_grid(ctx, T, NH, D), dim3(256), (size_t)D / 2 * sizeof(float2), m->pq, (const float*)m->pk, (const float*)m->pv,
                    kv->k_pool, kv->v_pool, (const int32_t*)kv->page_table_dev, (const int32_t*)(m->step.state + 1), NH, KVH, D,
                    kv->page_tokens, log2((double)c.rope_base));
         SKN_LAUNCH_CHECK(ctx);
         // query row t attends to the first pos0 + t + 1 tokens of the (single) sequence
+        const skn_gemm_src att = {D <= 128 ? SKN_SRC_BF16 : SKN_SRC_F32, m->patt, nullptr, 0.f};
         if (D <= 128)
-            SKN_TRY(skn_attn_prefill_launch(ctx, kv, 0, m->pq, T, pos0 + 1, scale, m->patt, NH));
+            SKN_TRY(skn_attn_prefill_launch(ctx, kv, 0, m->pq, T, pos0 + 1, scale, m->patt, NH, SKN_TYPE_BF16));
         else
             SKN_TRY(skn_attn_launch_ex(ctx, kv, m->pq, m->pnctx, T, 0, n_splits, m->ppartial, m->pcounters, scale, m->patt, NH));
         if (q4k_o) {  // the residual is added by the GEMM's store
             const skn_gemm_seg wo = {L.wo, H, m->px, 1};
-            const skn_gemm_src src = {SKN_SRC_F32, m->patt, nullptr, 0.f};
-            SKN_TRY(skn_gemm_q4k_multi(ctx, &wo, 1, H, src, T));
+            SKN_TRY(skn_gemm_q4k_multi(ctx, &wo, 1, H, att, T));
         } else {
             const void* blocks[1] = {L.wo};
             float* outs[1] = {m->px};
-            if (expand) SKN_TRY(project_expanded(ctx, m, l, 3, &L.type_o, blocks, &H, outs, 1, H, m->patt, nullptr, T, 1));
-            else SKN_TRY(project_rows(ctx, m, &L.type_o, blocks, &H, outs, 1, H, m->patt, nullptr, T, 1));
+            if (expand) SKN_TRY(project_expanded(ctx, m, l, 3, &L.type_o, blocks, &H, outs, 1, H, att, T, 1));
+            else SKN_TRY(project_rows(ctx, m, &L.type_o, blocks, &H, outs, 1, H, att, T, 1));
         }
         if (q4k_gu) {  // RMSNorm inside the activation pass, SwiGLU inside the store: gate and up never reach memory
-            const skn_gemm_seg gu[2] = {{L.w_gate, F, m->pmid, 0}, {L.w_up, F, m->pmid, 0}};
-            const skn_gemm_src src = {SKN_SRC_RMSNORM, m->px, L.ffn_norm, c.rms_eps};
-            SKN_TRY(skn_gemm_q4k_multi(ctx, gu, 2, H, src, T, true));
+            const skn_gemm_seg gu[2] = {{L.w_gate, F, nullptr, 0}, {L.w_up, F, nullptr, 0}};
+            SKN_TRY(skn_gemm_q4k_multi(ctx, gu, 2, H, normed2, T, m->pmid));
         } else {
             const int types[2] = {L.type_gate, L.type_up}, rows[2] = {F, F};
             const void* blocks[2] = {L.w_gate, L.w_up};
             float* outs[2] = {m->pgate, m->pup};
-            if (expand) SKN_TRY(project_expanded(ctx, m, l, 4, types, blocks, rows, outs, 2, H, m->px, L.ffn_norm, T, 0));
-            else SKN_TRY(project_rows(ctx, m, types, blocks, rows, outs, 2, H, m->px, L.ffn_norm, T, 0));
-            skn_launch(ctx, swiglu_rows_kernel, dim3(nblk((int64_t)T * F)), dim3(256), 0, (const float*)m->pgate,
+            if (expand) SKN_TRY(project_expanded(ctx, m, l, 4, types, blocks, rows, outs, 2, H, normed2, T, 0));
+            else SKN_TRY(project_rows(ctx, m, types, blocks, rows, outs, 2, H, normed2, T, 0));
+            skn_launch(ctx, swiglu_rows_kernel<uint16_t>, dim3(nblk((int64_t)T * F)), dim3(256), 0, (const float*)m->pgate,
                        (const float*)m->pup, m->pmid, (int64_t)T * F);
             SKN_LAUNCH_CHECK(ctx);
         }
+        const skn_gemm_src mid = {SKN_SRC_BF16, m->pmid, nullptr, 0.f};
         if (q4k_down) {
             const skn_gemm_seg down = {L.w_down, H, m->px, 1};  // residual added by the store
-            const skn_gemm_src mid = {SKN_SRC_F32, m->pmid, nullptr, 0.f};
             SKN_TRY(skn_gemm_q4k_multi(ctx, &down, 1, F, mid, T));
         } else {
             const void* blocks[1] = {L.w_down};
             float* outs[1] = {m->px};
-            if (expand) SKN_TRY(project_expanded(ctx, m, l, 6, &L.type_down, blocks, &H, outs, 1, F, m->pmid, nullptr, T, 1));
-            else SKN_TRY(project_rows(ctx, m, &L.type_down, blocks, &H, outs, 1, F, m->pmid, nullptr, T, 1));
+            if (expand) SKN_TRY(project_expanded(ctx, m, l, 6, &L.type_down, blocks, &H, outs, 1, F, mid, T, 1));
+            else SKN_TRY(project_rows(ctx, m, &L.type_down, blocks, &H, outs, 1, F, mid, T, 1));
         }
         // the cache of this layer now holds pos0 + T tokens
         kv->len[0] = pos0 + T;

@@ -362,8 +362,8 @@ struct Q4kFragSegs {
     int tile0[3];       // first column tile of each matrix (unused entries: n_tiles)
     int n_tiles;
     // pair != 0: w[0], w[1] are the gate and up matrices of a SwiGLU; a tile holds the same 32 columns of both
-    // (its two 32-column halves) and stores silu(gate) * up into c[0]
-    int pair;
+    // (its two 32-column halves) and stores silu(gate) * up there, in bf16
+    uint16_t* pair;
     // gemm_q4k_frag_kernel with k split over workgroups (gridDim.y of them per tile): the unscaled partial products go to
     // part[blockIdx.y][m][part_cols], matrix i at column part_col0[i] (a pair: gate, then up); null: no split
     float* part;
@@ -403,7 +403,7 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
     // tile -> (row tile, weight matrix, column tile): the column tiles of up to three matrices sharing the
     // activations are laid side by side
     const int mt = blockIdx.x / segs.n_tiles, tn = blockIdx.x - mt * segs.n_tiles;
-    const bool pair = segs.pair != 0;
+    const bool pair = segs.pair != nullptr;
     const int seg = pair ? 0 : (tn >= segs.tile0[2] ? 2 : (tn >= segs.tile0[1] ? 1 : 0));
     const uint8_t* __restrict__ w = segs.w[seg];
     float* __restrict__ c = segs.c[seg];
@@ -660,8 +660,7 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                                 continue;
                             }
                             const float sc = isc_lds[row - MH * mt * MT * 32];
-                            const float a = g * sc;
-                            c[(size_t)row * n + col] = a / (1.0f + expf(-a)) * (u * sc);  // silu(gate) * up
+                            segs.pair[(size_t)row * n + col] = swiglu_bf16(g * sc, u * sc);
                         }
                     }
                 }
@@ -720,9 +719,11 @@ __global__ __launch_bounds__(256) void gemm_add_parts_kernel(const float* __rest
     vec v = total(src) * sc;
     if (segs.pair) {
         const vec u = total(src + segs.col0[1]) * sc;
+        typedef uint16_t bits_vec __attribute__((ext_vector_type(W)));
+        bits_vec bits;
 #pragma unroll
-        for (int i = 0; i < W; i++) v[i] = v[i] / (1.0f + expf(-v[i])) * u[i];
-        *reinterpret_cast<vec*>(segs.c[0] + (size_t)row * segs.n[0] + col) = v;
+        for (int i = 0; i < W; i++) bits[i] = swiglu_bf16(v[i], u[i]);
+        *reinterpret_cast<bits_vec*>(segs.pair + (size_t)row * segs.n[0] + col) = bits;
         return;
     }
     const int i = segs.count > 2 && col >= segs.col0[2] ? 2 : (segs.count > 1 && col >= segs.col0[1] ? 1 : 0);
@@ -767,7 +768,7 @@ constexpr int kTlLds = 3 * kTlStage + 2 * kTlAux + 128 * 4 + 256 * 4;
 
 // One to three matrices per launch as in gemm_q4k_frag_kernel (tile0 counts 128-column tiles here); pair: a tile holds
 // the same 64 columns of the gate and the up matrix -- producers 0 and 1 unpack the gate's, 2 and 3 the up's, so a
-// consumer's column blocks 0, 1 and 2, 3 meet lane by lane in the store -- and stores silu(gate) * up into c[0].
+// consumer's column blocks 0, 1 and 2, 3 meet lane by lane in the store -- and stores silu(gate) * up in bf16.
 // TAIL: the last tiles are shared by tail.splits workgroups each, neighbours in the grid, with a part of k each (a template
 // parameter: grids without such tiles were 0.5 us slower at 512 x 14336 x 4096 for the division).
 template <bool TAIL>
@@ -788,7 +789,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
         sb0 = nb * z / parts, sb1 = nb * (z + 1) / parts;
     }
     const int mt = tile % m_tiles, tn = tile / m_tiles;  // (the row tiles of a column tile run side by side)
-    const bool pair = segs.pair != 0;
+    const bool pair = segs.pair != nullptr;
     const int seg = pair ? 0 : (tn >= segs.tile0[2] ? 2 : (tn >= segs.tile0[1] ? 1 : 0));
     const int n = segs.n[seg];
     const int n0 = pair ? tn * 64 : (tn - segs.tile0[seg]) * 128;  // first column of the tile in its matrix (pair: in both)
@@ -1090,8 +1091,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                         // register x of lane l: row 8 (x / 4) + 4 (l / 32) + x % 4 of the 32 x 32 tile
                         const int row = (mb0 + i) * 32 + 8 * (x >> 2) + 4 * h + (x & 3);
                         if (row < m && col < n) {
-                            const float g = acc[i][jj][x] * ug * sc[x], u = acc[i][jj + 2][x] * uu * sc[x];
-                            c[(size_t)row * n + col] = g / (1.0f + expf(-g)) * u;  // silu(gate) * up
+                            segs.pair[(size_t)row * n + col] = swiglu_bf16(acc[i][jj][x] * ug * sc[x], acc[i][jj + 2][x] * uu * sc[x]);
                         }
                     }
                 }
@@ -1114,7 +1114,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
 __global__ __launch_bounds__(256) void gemm_add_tall_kernel(const TallTail tail, const Q4kFragSegs segs, const float* __restrict__ inv_scale, int m, int m_tiles) {
     const int tile = tail.tile0 + (int)blockIdx.x, mt = tile % m_tiles, tn = tile / m_tiles, lane = threadIdx.x & 63, j = threadIdx.x >> 6;
     const int i = blockIdx.y, row0 = mt * 256 + 32 * i;  // (consumer i / 2, its row block i % 2)
-    const bool pair = segs.pair != 0;
+    const bool pair = segs.pair != nullptr;
     if (row0 >= m || (pair && j > 1)) return;
     const int seg = pair ? 0 : (tn >= segs.tile0[2] ? 2 : (tn >= segs.tile0[1] ? 1 : 0));
     const int n = segs.n[seg], col = (pair ? tn * 64 : (tn - segs.tile0[seg]) * 128) + 32 * j + (lane & 31);
@@ -1141,7 +1141,7 @@ __global__ __launch_bounds__(256) void gemm_add_tall_kernel(const TallTail tail,
         if (row >= m) continue;
         const float sc = inv_scale[row], g = v[x] * sc;
         float* dst = c + (size_t)row * n + col;
-        if (pair) *dst = g / (1.0f + expf(-g)) * (u[x] * sc);  // silu(gate) * up
+        if (pair) segs.pair[(size_t)row * n + col] = swiglu_bf16(g, u[x] * sc);
         else *dst = segs.accumulate[seg] != 0 ? *dst + g : g;
     }
 }
@@ -2207,7 +2207,7 @@ static int q4k_splits(const skn_ctx* ctx, int m, int tile_rows, int tiles, int n
 }
 
 int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, const skn_gemm_src& src, int m,
-                       bool swiglu_pair) {
+                       uint16_t* swiglu_pair) {
     SKN_REQUIRE(ctx, nseg >= 1 && nseg <= 3 && m > 0 && k > 0 && k % 256 == 0 && k <= 16384, SKN_ERR_ARG,
                 "Q4_K GEMM: bad segment count or shape");
     SKN_REQUIRE(ctx, !swiglu_pair || (nseg == 2 && segs[0].n == segs[1].n && !segs[0].accumulate), SKN_ERR_ARG,
@@ -2216,14 +2216,14 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     int tiles = 0;
     for (int i = 0; i < 3; i++) {
         const skn_gemm_seg& s = segs[i < nseg ? i : nseg - 1];
-        SKN_REQUIRE(ctx, s.w && s.c && s.n > 0 && ((uintptr_t)s.w & 15) == 0, SKN_ERR_ARG,
+        SKN_REQUIRE(ctx, s.w && (s.c || swiglu_pair) && s.n > 0 && ((uintptr_t)s.w & 15) == 0, SKN_ERR_ARG,
                     "Q4_K GEMM: weights must be non-null and 16-byte aligned");
         fs.w[i] = (const uint8_t*)s.w, fs.c[i] = s.c, fs.n[i] = s.n, fs.accumulate[i] = s.accumulate, fs.tile0[i] = tiles;
         if (i < nseg) tiles += (s.n + kBN - 1) / kBN;
     }
     for (int i = nseg; i < 3; i++) fs.tile0[i] = tiles;
     fs.n_tiles = swiglu_pair ? (segs[0].n + 31) / 32 : tiles;
-    fs.pair = swiglu_pair ? 1 : 0;
+    fs.pair = swiglu_pair;
     SKN_REQUIRE(ctx, src.a && ((uintptr_t)src.a & (src.kind == SKN_SRC_BF16 ? 7 : 15)) == 0, SKN_ERR_ARG,
                 "Q4_K GEMM: activations are null or misaligned");
     SKN_REQUIRE(ctx, src.kind == SKN_SRC_BF16 || src.kind == SKN_SRC_F32 || (src.b && ((uintptr_t)src.b & 15) == 0),

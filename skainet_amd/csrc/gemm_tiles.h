@@ -61,11 +61,15 @@ __device__ __forceinline__ uint32_t bf16_rne(float f) {
     return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
 }
 
+// an element of a SwiGLU pair: silu(gate) up as the bf16 that the product it goes into is defined on
+__device__ __forceinline__ uint16_t swiglu_bf16(float g, float u) { return (uint16_t)bf16_rne(g / (1.0f + expf(-g)) * u); }
+
 // Matrices that share a division of k: the parts of their products lie side by side, col0 the first column of each.
 struct skn_gemm_parts {
     float* c[3];
     int n[3], col0[3], accumulate[3];
-    int count, pair;
+    int count;
+    uint16_t* pair;  // not null: the first two are the gate and up matrices of a SwiGLU, which goes here
 };
 
 int skn_gemm_add_parts(skn_ctx* ctx, const float* part, int splits, int cols, const skn_gemm_parts& segs, const float* inv_scale, int m);

@@ -57,7 +57,7 @@ int skn_attn_launch_ex(skn_ctx* ctx, skn_kv* kv, const float* q_dev, const int32
 int skn_attn_splits(skn_ctx* ctx, int pairs, int max_ctx);
 // Causal attention of n_queries rows of one sequence: row t attends to its first first_ctx + t tokens (head_dim 64 / 128).
 int skn_attn_prefill_launch(skn_ctx* ctx, skn_kv* kv, int seq, const float* q_dev, int n_queries, int first_ctx, float scale,
-                            float* out_dev, int n_q_head = 0);
+                            void* out_dev, int n_q_head = 0, int out_type = SKN_TYPE_F32);  // F32 or BF16
 
 // ---- attention over a shared cache (csrc/attention_shared.hip; parameters: skn_shared_attn of the header) ----
 // Rows of a prompt: q [n][n_head * dim] (pitch ldq) and k [n][kv heads * dim] (pitch ldk), projected with bias, of tokens at
