@@ -26,7 +26,7 @@ struct skn_llama {
     int prompt_cap = 0;
     float *px = nullptr, *pxn = nullptr, *pq = nullptr, *pk = nullptr, *pv = nullptr, *patt = nullptr, *pproj = nullptr;
     float *pgate = nullptr, *pup = nullptr, *ppartial = nullptr;
-    uint16_t* pmid = nullptr;  // the rows of a SwiGLU, as the products behind it take them
+    float* pmid = nullptr;  // the rows of a SwiGLU: bf16 where the product's store forms them (a Q4_K pair), else fp32
     uint16_t *pb16 = nullptr, *pk16 = nullptr, *pv16 = nullptr;
     int32_t *ptok = nullptr, *pnctx = nullptr;
     // fp16-pair copies of the matrices that are not Q4_K, for the prompt GEMMs (made on first use when the option
@@ -183,18 +183,12 @@ __global__ void add_rows_kernel(float* __restrict__ y, const float* __restrict__
     if (i < n) y[i] += x[i];
 }
 
-__device__ __forceinline__ uint16_t bf16_bits(float x) {
-    const uint32_t u = __float_as_uint(x);
-    return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-}
-
-template <typename OUT>  // float, or uint16_t: bf16
-__global__ void swiglu_rows_kernel(const float* __restrict__ g, const float* __restrict__ u, OUT* __restrict__ out, int64_t n) {
+__global__ void swiglu_rows_kernel(const float* __restrict__ g, const float* __restrict__ u, float* __restrict__ out,
+                                   int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
-        const float a = g[i], y = a / (1.0f + expf(-a)) * u[i];
-        if constexpr (sizeof(OUT) == 2) out[i] = bf16_bits(y);
-        else out[i] = y;
+        const float a = g[i];
+        out[i] = a / (1.0f + expf(-a)) * u[i];
     }
 }
 
@@ -379,7 +373,7 @@ int decode_step(skn_ctx* ctx, skn_llama* m, const AttnShape& shape) {
             SKN_LAUNCH_CHECK(ctx);
             SKN_TRY(skn_matvec_q(ctx, L.type_gate, L.w_gate, F, H, m->xn, m->gate));
             SKN_TRY(skn_matvec_q(ctx, L.type_up, L.w_up, F, H, m->xn, m->up));
-            skn_launch(ctx, swiglu_rows_kernel<float>, dim3(nblk(F)), dim3(256), 0, (const float*)m->gate, (const float*)m->up,
+            skn_launch(ctx, swiglu_rows_kernel, dim3(nblk(F)), dim3(256), 0, (const float*)m->gate, (const float*)m->up,
                        m->mid, (int64_t)F);
             SKN_LAUNCH_CHECK(ctx);
         }
@@ -719,18 +713,19 @@ int skn_llama_prefill(skn_ctx* ctx, skn_llama* m, const int32_t* tokens_host, in
         }
         if (q4k_gu) {  // RMSNorm inside the activation pass, SwiGLU inside the store: gate and up never reach memory
             const skn_gemm_seg gu[2] = {{L.w_gate, F, nullptr, 0}, {L.w_up, F, nullptr, 0}};
-            SKN_TRY(skn_gemm_q4k_multi(ctx, gu, 2, H, normed2, T, m->pmid));
+            SKN_TRY(skn_gemm_q4k_multi(ctx, gu, 2, H, normed2, T, (uint16_t*)m->pmid));
         } else {
             const int types[2] = {L.type_gate, L.type_up}, rows[2] = {F, F};
             const void* blocks[2] = {L.w_gate, L.w_up};
             float* outs[2] = {m->pgate, m->pup};
             if (expand) SKN_TRY(project_expanded(ctx, m, l, 4, types, blocks, rows, outs, 2, H, normed2, T, 0));
             else SKN_TRY(project_rows(ctx, m, types, blocks, rows, outs, 2, H, normed2, T, 0));
-            skn_launch(ctx, swiglu_rows_kernel<uint16_t>, dim3(nblk((int64_t)T * F)), dim3(256), 0, (const float*)m->pgate,
+            skn_launch(ctx, swiglu_rows_kernel, dim3(nblk((int64_t)T * F)), dim3(256), 0, (const float*)m->pgate,
                        (const float*)m->pup, m->pmid, (int64_t)T * F);
             SKN_LAUNCH_CHECK(ctx);
         }
-        const skn_gemm_src mid = {SKN_SRC_BF16, m->pmid, nullptr, 0.f};
+        // (a pair of another format: fp32, which the direct products' preparation rounds and the general path converts)
+        const skn_gemm_src mid = {q4k_gu ? SKN_SRC_BF16 : SKN_SRC_F32, m->pmid, nullptr, 0.f};
         if (q4k_down) {
             const skn_gemm_seg down = {L.w_down, H, m->px, 1};  // residual added by the store
             SKN_TRY(skn_gemm_q4k_multi(ctx, &down, 1, F, mid, T));
