@@ -682,7 +682,7 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                     store_tile_part(sum, segs.part + (size_t)blockIdx.y * m * segs.part_cols + segs.part_col0[seg], segs.part_cols, (mb0 + i) * 32,
                                     n0 + 32 * j, m, n, lane);
                 else
-                    store_tile_scaled(sum, c, n, (mb0 + i) * 32, n0 + 32 * j, m, n, sc, lane, segs.accumulate[seg] != 0);
+                    store_tile(sum, c, n, (mb0 + i) * 32, n0 + 32 * j, m, n, sc, lane, segs.accumulate[seg] != 0);
             }
         }
     }
@@ -1102,7 +1102,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                 const float unit = *reinterpret_cast<const float*>(fin + (j * 32 + r) * 4);
 #pragma unroll
                 for (int x = 0; x < 16; x++) acc[i][j][x] *= unit;
-                store_tile_scaled(acc[i][j], c, n, (mb0 + i) * 32, n0 + 32 * j, m, n, sc, lane, segs.accumulate[seg] != 0);
+                store_tile(acc[i][j], c, n, (mb0 + i) * 32, n0 + 32 * j, m, n, sc, lane, segs.accumulate[seg] != 0);
             }
         }
     }
@@ -1131,19 +1131,23 @@ __global__ __launch_bounds__(256) void gemm_add_tall_kernel(const TallTail tail,
                 v[4 * x] += p.x, v[4 * x + 1] += p.y, v[4 * x + 2] += p.z, v[4 * x + 3] += p.w;
             }
     };
-    float v[16], u[16];
+    float v[16], u[16], sc[16];
+    row_scales(inv_scale, row0, lane, sc);
     total(j, v);
     if (pair) total(j + 2, u);
-    if (col >= n) return;
+    if (pair) {
+        if (col >= n) return;
 #pragma unroll
-    for (int x = 0; x < 16; x++) {
-        const int row = row0 + 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3);
-        if (row >= m) continue;
-        const float sc = inv_scale[row], g = v[x] * sc;
-        float* dst = c + (size_t)row * n + col;
-        if (pair) segs.pair[(size_t)row * n + col] = swiglu_bf16(g, u[x] * sc);
-        else *dst = segs.accumulate[seg] != 0 ? *dst + g : g;
+        for (int x = 0; x < 16; x++) {
+            const int row = row0 + 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3);
+            if (row < m) segs.pair[(size_t)row * n + col] = swiglu_bf16(v[x] * sc[x], u[x] * sc[x]);
+        }
+        return;
     }
+    float16_t sum;
+#pragma unroll
+    for (int x = 0; x < 16; x++) sum[x] = v[x];
+    store_tile(sum, c, n, row0, col - (lane & 31), m, n, sc, lane, segs.accumulate[seg] != 0);
 }
 
 // ---- general path: activations x (hi + lo * 2^-11) weights, both operands loaded in fragment order ---------
@@ -1225,6 +1229,9 @@ void gemm_hilo_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restr
 
     // hi + lo * 2^-11, then the four partial tiles: tile t = 2 i + j belongs to wavefront t % 4, the other three
     // hand theirs over
+    float sc[(MT + 1) / 2][16];
+#pragma unroll
+    for (int y = 0; y < (MT + 1) / 2; y++) row_scales(inv_scale, (mt * MT + min((kq >> 1) + 2 * y, MT - 1)) * 32, lane, sc[y]);
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
@@ -1250,7 +1257,7 @@ void gemm_hilo_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restr
                 for (int o = 0; o < 3; o++)
 #pragma unroll
                     for (int x = 0; x < 16; x++) sum[x] += red[(t * 3 + o) * 1024 + 64 * x + lane];
-                store_tile(sum, c, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, inv_scale, lane, accumulate != 0);
+                store_tile(sum, c, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, sc[i >> 1], lane, accumulate != 0);
             }
         }
 }
@@ -1472,6 +1479,10 @@ void gemm_q6k_frag_kernel(const u32x4* __restrict__ afrag, const uint8_t* __rest
     }
 
     // the four partial tiles: tile t = 2 i + j belongs to wavefront t % 4, the other three hand theirs over
+    float sc[(MT + 1) / 2][16];
+    if constexpr (!SPLIT)
+#pragma unroll
+        for (int y = 0; y < (MT + 1) / 2; y++) row_scales(inv_scale, (mt * MT + min((kq >> 1) + 2 * y, MT - 1)) * 32, lane, sc[y]);
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
@@ -1496,7 +1507,7 @@ void gemm_q6k_frag_kernel(const u32x4* __restrict__ afrag, const uint8_t* __rest
 #pragma unroll
                     for (int x = 0; x < 16; x++) sum[x] += red[(t * 3 + o) * 1024 + 64 * x + lane];
                 if constexpr (SPLIT) store_tile_part(sum, part + (size_t)blockIdx.y * m * n, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, lane);
-                else store_tile(sum, c, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, inv_scale, lane, accumulate != 0);
+                else store_tile(sum, c, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, sc[i >> 1], lane, accumulate != 0);
             }
         }
 }
@@ -1746,6 +1757,10 @@ void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restri
             phase(i, C3{});
         }
         barrier();
+        float sc[(MT + 1) / 2][16];
+        if constexpr (!SPLIT)
+#pragma unroll
+            for (int y = 0; y < (MT + 1) / 2; y++) row_scales(inv_scale, (mt * MT + min((kq >> 1) + 2 * y, MT - 1)) * 32, lane, sc[y]);
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const float unit = *reinterpret_cast<const float*>(aux + 512 + (j * 32 + r) * 4);
@@ -1774,7 +1789,7 @@ void gemm_q6k_pc_kernel(const u32x4* __restrict__ afrag, const uint8_t* __restri
 #pragma unroll
                         for (int x = 0; x < 16; x++) sum[x] += red[(t * 3 + o) * 1024 + 64 * x + lane];
                     if constexpr (SPLIT) store_tile_part(sum, part + (size_t)blockIdx.y * m * n, n, (mt * MT + ii) * 32, tn * kBN + 32 * j, m, n, lane);
-                    else store_tile(sum, c, n, (mt * MT + ii) * 32, tn * kBN + 32 * j, m, n, inv_scale, lane, accumulate != 0);
+                    else store_tile(sum, c, n, (mt * MT + ii) * 32, tn * kBN + 32 * j, m, n, sc[ii >> 1], lane, accumulate != 0);
                 }
             }
     }
@@ -2038,7 +2053,7 @@ void gemm_q6k_tall_kernel(const u32x4* __restrict__ afrag, const uint8_t* __rest
                 const float unit = fin[j * 32 + r];
 #pragma unroll
                 for (int x = 0; x < 16; x++) acc[i][j][x] *= unit;
-                store_tile_scaled(acc[i][j], c, n, (mb0 + i) * 32, n0 + 32 * j, m, n, sc, lane, accumulate != 0);
+                store_tile(acc[i][j], c, n, (mb0 + i) * 32, n0 + 32 * j, m, n, sc, lane, accumulate != 0);
             }
         }
     }

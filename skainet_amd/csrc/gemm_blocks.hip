@@ -16,8 +16,8 @@
 // added through LDS.  A wavefront brings its superblock of 64 rows in with coalesced 16-byte loads one superblock ahead
 // (registers, then LDS of its own: no barrier in the loop) and reads the activations in fragment order, four k-steps ahead.
 //
-// us per call, before -> now (weights as fp16 pairs -> this): Q8_0 333 x 4096 x 4096 51.6 -> 36.4, 512 x 14336 x 4096 236 -> 121, 41 x 4096 x
-// 11008 102 -> 28.5; Q5_K 512 x 4096 x 4096 60 -> 40.4; Q4_0 5 x 4096 x 4096 36.6 -> 11.5.
+// us per call, before -> now (weights as fp16 pairs -> this): Q8_0 333 x 4096 x 4096 51.6 -> 35.9, 512 x 14336 x 4096 236 -> 115, 41 x 4096 x
+// 11008 102 -> 28.5; Q5_K 512 x 4096 x 4096 60 -> 39.2; Q4_0 5 x 4096 x 4096 36.6 -> 11.5.
 #include "gemm_blocks.h"
 #include "gemm_tiles.h"
 
@@ -460,6 +460,8 @@ void gemm_blocks_kernel(const u32x4* __restrict__ afrag, const u32x4* __restrict
     }
 
     // the four partial tiles: tile t = 2 i + j belongs to wavefront t % 4, the other three hand theirs over
+    float sc[16];
+    if (!part) row_scales(inv_scale, (mt * MT + min(kq >> 1, MT - 1)) * 32, lane, sc);
     __syncthreads();
     float* red = reinterpret_cast<float*>(lds);
 #pragma unroll
@@ -486,7 +488,7 @@ void gemm_blocks_kernel(const u32x4* __restrict__ afrag, const u32x4* __restrict
 #pragma unroll
                     for (int x = 0; x < 16; x++) sum[x] += red[(t * 3 + o) * 1024 + 64 * x + lane];
                 if (part) store_tile_part(sum, part + (size_t)blockIdx.y * m * n, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, lane);
-                else store_tile(sum, c, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, inv_scale, lane, accumulate != 0);
+                else store_tile(sum, c, n, (mt * MT + i) * 32, tn * kBN + 32 * j, m, n, sc, lane, accumulate != 0);
             }
         }
 }

@@ -17,32 +17,40 @@ static inline size_t skn_align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 // row blocks per tile where the tile follows the rows: 32 MT rows
 static inline int skn_gemm_mt(int m) { return m <= 32 ? 1 : (m <= 64 ? 2 : 4); }
 
-// C tile store: acc register r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32 of the 32x32 tile
-__device__ __forceinline__ void store_tile(const float16_t& acc, float* __restrict__ c, int ldc, int row0, int col0,
-                                           int m, int n, const float* __restrict__ inv_scale, int lane,
-                                           bool accumulate = false) {
-    const int col = col0 + (lane & 31);
+// The row scales a tile's store needs: sc[r] is that of the row register r holds (store_tile).  inv_scale has a value for every row of
+// the padded tiles.  Read ahead of the exchange of the partial tiles, sixteen bytes at a time: read one by one beside their stores, each
+// was waited for under its own row check (Q8_0 333 x 4096 x 4096 37.3 -> 35.9 us, Q6_K 1000 x 14336 x 4096 299 -> 286).
+__device__ __forceinline__ void row_scales(const float* __restrict__ inv_scale, int row0, int lane, float (&sc)[16]) {
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row < m && col < n) {
-            float* dst = c + (size_t)row * ldc + col;
-            *dst = accumulate ? *dst + acc[r] * inv_scale[row] : acc[r] * inv_scale[row];
-        }
+    for (int a = 0; a < 4; a++) {
+        const float4 v = *reinterpret_cast<const float4*>(inv_scale + row0 + 8 * a + 4 * (lane >> 5));
+        sc[4 * a] = v.x, sc[4 * a + 1] = v.y, sc[4 * a + 2] = v.z, sc[4 * a + 3] = v.w;
     }
 }
 
-// the same with the sixteen row scales in hand (sc[r]: the scale of the row that register r holds)
-__device__ __forceinline__ void store_tile_scaled(const float16_t& acc, float* __restrict__ c, int ldc, int row0, int col0,
-                                                  int m, int n, const float (&sc)[16], int lane, bool accumulate) {
+// C tile store: acc register r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32 of the 32x32 tile.  What a tile is added to is
+// read as a whole first (for rows and columns outside, the edge's: unused), sixteen loads in flight instead of a load, a wait and a
+// store in turn: a 512-token prompt of 32 layers of width 4096, whose residual stream two products a layer are added to, 10.81 -> 10.40 ms.
+__device__ __forceinline__ void store_tile(const float16_t& acc, float* __restrict__ c, int ldc, int row0, int col0, int m, int n,
+                                           const float (&sc)[16], int lane, bool accumulate) {
     const int col = col0 + (lane & 31);
+    float v[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = acc[r] * sc[r];
+    if (accumulate) {
+        float old[16];
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            old[r] = c[(size_t)min(row, m - 1) * ldc + min(col, n - 1)];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++) v[r] += old[r];
+    }
 #pragma unroll
     for (int r = 0; r < 16; r++) {
         const int row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row < m && col < n) {
-            float* dst = c + (size_t)row * ldc + col;
-            *dst = accumulate ? *dst + acc[r] * sc[r] : acc[r] * sc[r];
-        }
+        if (row < m && col < n) c[(size_t)row * ldc + col] = v[r];
     }
 }
 
