@@ -18,6 +18,7 @@
 #include "gemm_tiles.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -41,8 +42,10 @@ __device__ __forceinline__ u32x2 lds_u32x2(const uint8_t* p) { return *reinterpr
 // fit there -- rows from about 2^47 on -- ends as an infinity or NaN, is seen when the tile is stored, and the tile is summed once more with
 // operands times 2^-100, in units of 2^60, where sums of the largest activations and weights of all formats fit; rows that need it are large
 // enough to lose nothing by it.  So a result is finite wherever it is for rows scaled to their largest element.  The first pass pays
-// for the subtraction below (Q8_0 8 x 4096 x 11008 11.4 us without it, 11.8 with, Q5_K 11.2, 12.0) and 0.1 to 0.3 us for looking at the sums
-// (16 x 4096 x 4096 in Q4_K 5.0, 5.0, in Q6_K 6.4, 6.8, in Q8_0 6.0, 6.2).
+// 0.1 to 0.3 us for looking at the sums (16 x 4096 x 4096 in Q4_K 5.0, 5.0, in Q6_K 6.4, 6.8, in Q8_0 6.0, 6.2) and, where one body of code serves both
+// passes, for the subtraction below.  The formats that gain by a body for each have kTwoBodies: Q5_K 1.05 times as fast in the mean over
+// 42 shapes (5 x 4096 x 11008 10.9 -> 10.0 us), Q4_0 1.02 (16 x 4096 x 4096 6.7 -> 6.4); Q8_0 and Q4_K, of which some are faster and some slower
+// for it (Q8_0 16 x 512 x 4096 5.5 -> 5.2, 16 x 4096 x 11008 11.8 -> 12.1; Q4_K 16 x 2048 x 2048 3.9 -> 3.7, 16 x 12000 x 1024 5.3 -> 5.5), and Q6_K (1.01) keep one.
 constexpr float kUp = 0x1p40f;
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 struct Operands {
@@ -75,7 +78,7 @@ __device__ __forceinline__ bf16x8 operand(u32x2 lo, u32x2 hi) { return __builtin
 template <bool FIVE>
 struct FewK {
     static constexpr int kBytes = FIVE ? 176 : 144, kPieces = kBytes / 16, kPitch = kBytes;
-    static constexpr bool kMin = true, kHalves = false;
+    static constexpr bool kMin = true, kHalves = false, kTwoBodies = FIVE;
     struct Head {
         float d, dmin;
         uint32_t sc[2], mn[2];
@@ -101,7 +104,7 @@ struct FewK {
 
 struct FewQ80 {  // 34 bytes: d, 32 int8; block pairs are 17 dwords
     static constexpr int kBytes = 272, kPieces = 17, kPitch = 272;
-    static constexpr bool kMin = false, kHalves = false;
+    static constexpr bool kMin = false, kHalves = false, kTwoBodies = false;
     struct Head {};
     __device__ static __forceinline__ void head(const uint8_t*, int, Head&) {}
     __device__ static __forceinline__ bf16x8 block(const uint8_t* row, const Head&, int b, int g, const Operands& o, float& s, float&) {
@@ -121,7 +124,7 @@ struct FewQ80 {  // 34 bytes: d, 32 int8; block pairs are 17 dwords
 
 struct FewQ40 {  // 18 bytes: d, nibbles (low ones elements 0..15, high ones 16..31); pairs are 9 dwords
     static constexpr int kBytes = 144, kPieces = 9, kPitch = 144;
-    static constexpr bool kMin = false, kHalves = false;
+    static constexpr bool kMin = false, kHalves = false, kTwoBodies = true;
     struct Head {};
     __device__ static __forceinline__ void head(const uint8_t*, int, Head&) {}
     // a nibble at the top of its byte, less eight there, is 16 (q - 8)
@@ -147,7 +150,7 @@ struct FewQ40 {  // 18 bytes: d, nibbles (low ones elements 0..15, high ones 16.
 // superblock's last sixteen bytes.
 struct FewQ6K {
     static constexpr int kBytes = 210, kPieces = 14, kPitch = 240;
-    static constexpr bool kHalves = true;
+    static constexpr bool kHalves = true, kTwoBodies = false;
     struct Head {
         float d4;  // d / 4 (times 2^40): the operands are 4 (q - 32)
         u32x4 sc;
@@ -221,10 +224,8 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
             anext[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, (int)(afrom + x * AL::step(2u * k)), chunk * 64 * CH, 0));
     };
     auto fits = [](float x) __attribute__((always_inline)) { return fabsf(x) < INFINITY; };
-    uint32_t less = 0;  // (the second pass: 100)
-#pragma unroll 1
-    for (;;) {
-        asm volatile("" : "+s"(less));  // (one body for both)
+    const auto pass = [&](auto which) __attribute__((always_inline)) {
+        const uint32_t less = which;  // (the second pass: 100)
         const Operands o = {(less << 7) * 0x10001u, __uint_as_float((127u + 9u - less) << 23)};
         const uint32_t one = 0x3F803F80u - o.down;
         const u32x4 ones_bits = {one, one, one, one};
@@ -350,9 +351,21 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
                 c[at] = sum * (less ? 0x1p60f : 0x1p-40f);
             }
         }
-        if (less || !__builtin_amdgcn_readfirstlane(again)) return;
-        less = 100;
+        return !less && __builtin_amdgcn_readfirstlane(again) != 0;
+    };
+    if constexpr (F::kTwoBodies) {
+        if (!pass(std::integral_constant<uint32_t, 0>{})) return;
         __syncthreads();
+        (void)pass(std::integral_constant<uint32_t, 100>{});
+    } else {
+        uint32_t less = 0;
+#pragma unroll 1
+        for (;;) {
+            asm volatile("" : "+s"(less));  // (one body for both)
+            if (!pass(less)) return;
+            less = 100;
+            __syncthreads();
+        }
     }
 }
 
