@@ -43,9 +43,10 @@ __device__ __forceinline__ u32x2 lds_u32x2(const uint8_t* p) { return *reinterpr
 // operands times 2^-100, in units of 2^60, where sums of the largest activations and weights of all formats fit; rows that need it are large
 // enough to lose nothing by it.  So a result is finite wherever it is for rows scaled to their largest element.  The first pass pays
 // 0.1 to 0.3 us for looking at the sums (16 x 4096 x 4096 in Q4_K 5.0, 5.0, in Q6_K 6.4, 6.8, in Q8_0 6.0, 6.2) and, where one body of code serves both
-// passes, for the subtraction below.  The formats that gain by a body for each have kTwoBodies: Q5_K 1.05 times as fast in the mean over
-// 42 shapes (5 x 4096 x 11008 10.9 -> 10.0 us), Q4_0 1.02 (16 x 4096 x 4096 6.7 -> 6.4); Q8_0 and Q4_K, of which some are faster and some slower
-// for it (Q8_0 16 x 512 x 4096 5.5 -> 5.2, 16 x 4096 x 11008 11.8 -> 12.1; Q4_K 16 x 2048 x 2048 3.9 -> 3.7, 16 x 12000 x 1024 5.3 -> 5.5), and Q6_K (1.01) keep one.
+// passes, for the subtraction below.  kTwoBodies: from so many row blocks on a format has a body for each.  Q5_K is 1.05 times as fast for it in the mean over
+// 42 shapes (5 x 4096 x 11008 10.9 -> 10.0 us), Q4_0 1.02 (16 x 4096 x 4096 6.7 -> 6.4), Q6_K of more than sixteen rows 1.01 to 1.03 (32 x 6000 x 6144 17.5 -> 17.1); Q6_K of
+// up to sixteen, Q8_0 and Q4_K, which gain at some sizes and lose at others (Q6_K 16 x 2048 x 2048 5.0 -> 5.1; Q8_0 16 x 512 x 4096 5.5 -> 5.2, 16 x 4096 x 11008 11.8 -> 12.1; Q4_K
+// 16 x 2048 x 2048 3.9 -> 3.7, 16 x 12000 x 1024 5.3 -> 5.5), keep one.
 constexpr float kUp = 0x1p40f;
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 struct Operands {
@@ -78,7 +79,8 @@ __device__ __forceinline__ bf16x8 operand(u32x2 lo, u32x2 hi) { return __builtin
 template <bool FIVE>
 struct FewK {
     static constexpr int kBytes = FIVE ? 176 : 144, kPieces = kBytes / 16, kPitch = kBytes;
-    static constexpr bool kMin = true, kHalves = false, kTwoBodies = FIVE;
+    static constexpr bool kMin = true, kHalves = false;
+    static constexpr int kTwoBodies = FIVE ? 1 : 5;
     struct Head {
         float d, dmin;
         uint32_t sc[2], mn[2];
@@ -104,7 +106,8 @@ struct FewK {
 
 struct FewQ80 {  // 34 bytes: d, 32 int8; block pairs are 17 dwords
     static constexpr int kBytes = 272, kPieces = 17, kPitch = 272;
-    static constexpr bool kMin = false, kHalves = false, kTwoBodies = false;
+    static constexpr bool kMin = false, kHalves = false;
+    static constexpr int kTwoBodies = 5;
     struct Head {};
     __device__ static __forceinline__ void head(const uint8_t*, int, Head&) {}
     __device__ static __forceinline__ bf16x8 block(const uint8_t* row, const Head&, int b, int g, const Operands& o, float& s, float&) {
@@ -124,7 +127,8 @@ struct FewQ80 {  // 34 bytes: d, 32 int8; block pairs are 17 dwords
 
 struct FewQ40 {  // 18 bytes: d, nibbles (low ones elements 0..15, high ones 16..31); pairs are 9 dwords
     static constexpr int kBytes = 144, kPieces = 9, kPitch = 144;
-    static constexpr bool kMin = false, kHalves = false, kTwoBodies = true;
+    static constexpr bool kMin = false, kHalves = false;
+    static constexpr int kTwoBodies = 1;
     struct Head {};
     __device__ static __forceinline__ void head(const uint8_t*, int, Head&) {}
     // a nibble at the top of its byte, less eight there, is 16 (q - 8)
@@ -150,7 +154,8 @@ struct FewQ40 {  // 18 bytes: d, nibbles (low ones elements 0..15, high ones 16.
 // superblock's last sixteen bytes.
 struct FewQ6K {
     static constexpr int kBytes = 210, kPieces = 14, kPitch = 240;
-    static constexpr bool kHalves = true, kTwoBodies = false;
+    static constexpr bool kHalves = true;
+    static constexpr int kTwoBodies = 2;
     struct Head {
         float d4;  // d / 4 (times 2^40): the operands are 4 (q - 32)
         u32x4 sc;
@@ -351,10 +356,10 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
                 c[at] = sum * (less ? 0x1p60f : 0x1p-40f);
             }
         }
-        return !less && __builtin_amdgcn_readfirstlane(again) != 0;
+        return less || !__builtin_amdgcn_readfirstlane(again);  // (done)
     };
-    if constexpr (F::kTwoBodies) {
-        if (!pass(std::integral_constant<uint32_t, 0>{})) return;
+    if constexpr (MT >= F::kTwoBodies) {
+        if (pass(std::integral_constant<uint32_t, 0>{})) return;
         __syncthreads();
         (void)pass(std::integral_constant<uint32_t, 100>{});
     } else {
@@ -362,7 +367,7 @@ __global__ __launch_bounds__(64 * W) void gemm_few_kernel(const uint16_t* __rest
 #pragma unroll 1
         for (;;) {
             asm volatile("" : "+s"(less));  // (one body for both)
-            if (!pass(less)) return;
+            if (pass(less)) return;
             less = 100;
             __syncthreads();
         }
