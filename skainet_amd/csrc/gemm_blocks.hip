@@ -872,9 +872,9 @@ int superblock_bytes(int t) {
 }
 
 // The kernel of 96-row tiles: where it has a tile for each compute unit at most and the 64-row one more than that.  Those then run beside
-// each other on some units and alone on others, which wait.  us per call, 64 rows | 96: Q8_0 333 x 4096 x 4096 35.6 | 32.1, 90 x 14774 x 13568 102 | 85,
-// 164 x 6786 x 2304 24.5 | 23.2, 299 x 3074 x 768 11.0 | 11.0; Q4_0 333 x 4096 x 4096 34.1 | 30.4, 1428 x 645 x 9984 82.5 | 65.8; Q5_K 333 x 4096 x 4096 38.4 | 34.1 (36
-// drawn shapes of this range, three formats: 1.00 to 1.25 times as fast).  In more rounds the smaller tiles are the faster ones: Q8_0 512 x
+// each other on some units and alone on others, which wait.  us per call, 64 rows | 96: Q8_0 333 x 4096 x 4096 36.0 | 32.1, 90 x 14774 x 13568 100 | 85,
+// 164 x 6786 x 2304 24.8 | 23.2; Q4_0 333 x 4096 x 4096 34.1 | 30.4, 1428 x 645 x 9984 83 | 66; Q5_K 333 x 4096 x 4096 38.7 | 34.3 (30 shapes of this range, three
+// formats: 1.05 to 1.26 times as fast, 1.12 in the mean).  In more rounds the smaller tiles are the faster ones: Q8_0 512 x
 // 4096 x 4096 39.6 | 56, 1000 x 4096 x 11008 163 | 189; and tiles that leave half of the device idle have their k divided instead.
 bool one_round_of_pc(const skn_ctx* ctx, int type, int n, int m) {
     const int columns = ((n + kBN - 1) / kBN + 7) / 8 * 8;  // (of the grid)
