@@ -2122,7 +2122,7 @@ int skn_gemm_k_splits(const skn_ctx* ctx, int m, int tiles, int nb) {
     return (nb + each - 1) / each;  // (no workgroup without a superblock)
 }
 
-bool skn_gemm_may_allocate(skn_ctx* ctx) {  // (asking for memory would end a capture)
+static bool may_allocate(skn_ctx* ctx) {  // (asking for memory would end a capture)
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone) return true;
     (void)hipGetLastError();
@@ -2130,7 +2130,7 @@ bool skn_gemm_may_allocate(skn_ctx* ctx) {  // (asking for memory would end a ca
 }
 
 static bool grow_parts(skn_ctx* ctx, size_t bytes) {
-    if (!skn_gemm_may_allocate(ctx)) return false;
+    if (!may_allocate(ctx)) return false;
     void* p = nullptr;
     if (hipMalloc(&p, bytes) != hipSuccess) {
         (void)hipGetLastError();
@@ -2147,7 +2147,7 @@ static bool grow_parts(skn_ctx* ctx, size_t bytes) {
 }
 
 int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out, bool ahead) {
-    if (bytes > ctx->gemm_ws_bytes && !(ahead && !skn_gemm_may_allocate(ctx))) {
+    if (bytes > ctx->gemm_ws_bytes && !(ahead && !may_allocate(ctx))) {
         SKN_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (ctx->gemm_ws) SKN_HIP(ctx, hipFree(ctx->gemm_ws));
         ctx->gemm_ws = nullptr;

@@ -19,6 +19,7 @@
 // us per call, before -> now (weights as fp16 pairs -> this): Q8_0 333 x 4096 x 4096 51.6 -> 32.1, 512 x 14336 x 4096 236 -> 115, 41 x 4096 x
 // 11008 102 -> 28.5; Q5_K 512 x 4096 x 4096 60 -> 39.2; Q4_0 5 x 4096 x 4096 36.6 -> 11.5.
 #include "gemm_blocks.h"
+#include "gemm_blocks_rows.h"
 #include "gemm_tiles.h"
 
 #include <algorithm>
@@ -561,6 +562,7 @@ void gemm_blocks_pc_kernel(const u32x4* __restrict__ afrag, const u32x4* __restr
                            uint32_t a_bytes, uint32_t w_bytes) {
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr int MT = kPcMT;
+    static_assert(MT == 3, "skn_blocks_of_96");
     constexpr int P = F::kBytes / 16;  // sixteen-byte pieces of a row's superblock
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), kq = wave & 3;
     const int h = lane >> 5, r = lane & 31;
@@ -666,9 +668,10 @@ void gemm_blocks_pc_kernel(const u32x4* __restrict__ afrag, const u32x4* __restr
         }
     } else {
         const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc((void*)afrag, 0, (int)a_bytes, 0x00020000);
+        int block[MT];
         uint32_t abase[MT];
 #pragma unroll
-        for (int i = 0; i < MT; i++) abase[i] = (uint32_t)(mt * MT + i) * (uint32_t)k * 64u;
+        for (int i = 0; i < MT; i++) block[i] = skn_blocks_of_96(mt * MT + i, m), abase[i] = (uint32_t)block[i] * (uint32_t)k * 64u;
         constexpr int RING = 4;  // k-steps
         u32x4 a[RING][MT];
         auto afetch = [&](int step, int slot) __attribute__((always_inline)) {  // step: 16 per superblock, absolute
@@ -697,7 +700,8 @@ void gemm_blocks_pc_kernel(const u32x4* __restrict__ afrag, const u32x4* __restr
         };
 #pragma unroll
         for (int x = 0; x < RING; x++) afetch(16 * min(kq, nb - 1) + x, x);
-        if ((int)threadIdx.x < 32 * MT) scales[threadIdx.x] = inv_scale[32 * MT * mt + (int)threadIdx.x];
+        if ((int)threadIdx.x < 32 * MT)
+            scales[threadIdx.x] = inv_scale[32 * skn_blocks_of_96(mt * MT + ((int)threadIdx.x >> 5), m) + r];
         barrier();
         // (a pair without a superblock in the last turn only keeps the barriers: a branch around the multiplications inside this loop would
         // have every wait for an activation wait for the newest one)
@@ -708,7 +712,7 @@ void gemm_blocks_pc_kernel(const u32x4* __restrict__ afrag, const u32x4* __restr
             u32x4 sf[MT];
             if constexpr (F::kMin) {
 #pragma unroll
-                for (int x = 0; x < MT; x++) sf[x] = sfrag[((size_t)(mt * MT + x) * nb + sb) * 64 + lane];
+                for (int x = 0; x < MT; x++) sf[x] = sfrag[((size_t)block[x] * nb + sb) * 64 + lane];
             }
 #pragma unroll
             for (int b = 0; b < 8; b++) {
@@ -808,7 +812,7 @@ int launch_blocks(skn_ctx* ctx, const u32x4* afrag, const u32x4* sfrag, const fl
 template <typename F>
 int launch_pc(skn_ctx* ctx, const u32x4* afrag, const u32x4* sfrag, const float* isc, const skn_gemm_seg& seg, int m, int k) {
     const int m_tiles = (m + 32 * kPcMT - 1) / (32 * kPcMT), n_tiles = (seg.n + kBN - 1) / kBN;
-    const uint32_t a_bytes = (uint32_t)((size_t)m_tiles * 32 * kPcMT * k * 2), w_bytes = (uint32_t)((size_t)seg.n * (k / 256) * F::kBytes);
+    const uint32_t a_bytes = (uint32_t)((size_t)skn_blocks_padded_rows(m) * k * 2), w_bytes = (uint32_t)((size_t)seg.n * (k / 256) * F::kBytes);
     skn_launch(ctx, gemm_blocks_pc_kernel<F>, dim3((n_tiles + 7) / 8 * 8 * m_tiles), dim3(512), pc_lds_bytes<F>(), afrag, sfrag, (const uint8_t*)seg.w, isc, seg.c, m,
                seg.n, k, m_tiles, n_tiles, seg.accumulate, a_bytes, w_bytes);
     SKN_LAUNCH_CHECK(ctx);
@@ -911,8 +915,7 @@ int skn_gemm_blocks_multi(skn_ctx* ctx, const int* types, const skn_gemm_seg* se
     SKN_REQUIRE(ctx, src.a && ((uintptr_t)src.a & (src.kind == SKN_SRC_BF16 ? 7 : 15)) == 0, SKN_ERR_ARG, "block GEMM: activations are null or misaligned");
     SKN_REQUIRE(ctx, src.kind == SKN_SRC_BF16 || src.kind == SKN_SRC_F32 || (src.b && ((uintptr_t)src.b & 15) == 0), SKN_ERR_ARG,
                 "block GEMM: second activation operand is null or misaligned");
-    const int mt = m <= 32 ? 1 : 2, m_tiles = (m + 32 * mt - 1) / (32 * mt);
-    int m_pad = m_tiles * 32 * mt;
+    const int mt = m <= 32 ? 1 : 2, m_pad = skn_blocks_padded_rows(m), m_tiles = m_pad / (32 * mt);
     bool pc[3] = {false, false, false};
     int splits[3] = {1, 1, 1};
     size_t part_bytes = 0;  // (the products run one after the other: they share the room for their parts)
@@ -925,17 +928,10 @@ int skn_gemm_blocks_multi(skn_ctx* ctx, const int* types, const skn_gemm_seg* se
         pc[i] = splits[i] == 1 && one_round_of_pc(ctx, types[i], segs[i].n, m);
         sums = sums || has_minima(types[i]);
     }
-    const auto workspace = [&](int rows) {
-        return skn_align_up((size_t)rows * k * 2) + (sums ? skn_align_up((size_t)rows * (k / 256) * 32) : 0) + skn_align_up((size_t)rows * 4);
-    };
-    if (pc[0] || pc[1] || pc[2]) {  // (rows padded to both tiles; where a capture holds too little for that, the smaller tiles need less)
-        const int rows = std::max(m_pad, (m + 32 * kPcMT - 1) / (32 * kPcMT) * (32 * kPcMT));
-        if (workspace(rows) <= ctx->gemm_ws_bytes || skn_gemm_may_allocate(ctx)) m_pad = rows;
-        else pc[0] = pc[1] = pc[2] = false;
-    }
     const size_t af_bytes = skn_align_up((size_t)m_pad * k * 2), sf_bytes = sums ? skn_align_up((size_t)m_pad * (k / 256) * 32) : 0;
+    const size_t is_bytes = skn_align_up((size_t)m_pad * 4);
     uint8_t* ws;
-    SKN_TRY(skn_gemm_workspace(ctx, workspace(m_pad), &ws, src.ahead));
+    SKN_TRY(skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes, &ws, src.ahead));
     u32x4* afrag = (u32x4*)ws;
     _Float16* sfrag = (_Float16*)(ws + af_bytes);
     float* isc = (float*)(ws + af_bytes + sf_bytes);

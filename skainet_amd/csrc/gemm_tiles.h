@@ -82,7 +82,6 @@ struct skn_gemm_parts {
 
 int skn_gemm_add_parts(skn_ctx* ctx, const float* part, int splits, int cols, const skn_gemm_parts& segs, const float* inv_scale, int m);
 int skn_gemm_k_splits(const skn_ctx* ctx, int m, int tiles, int nb);
-bool skn_gemm_may_allocate(skn_ctx* ctx);  // false in a capture
 // grows the context's GEMM workspace; the pointer stays valid until the next growth.  `ahead`: for a later call (skn_gemm_src); what a
 // capture does not allow is left out.
 int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out, bool ahead = false);

@@ -215,7 +215,7 @@ def test_weights_and_activations_on_their_least_alignment(hip):
 
 
 @pytest.mark.parametrize("name,m,n,wide,k", [("q8_0", 333, 1024, 4096, 4096), ("q5_k", 41, 512, 20000, 4096), ("q6_k", 33, 512, 20000, 4096), ("q4_k", 48, 512, 20000, 4096),
-                                             ("q4_k", 17, 256, 20000, 4096)])
+                                             ("q4_k", 17, 256, 20000, 4096), ("q8_0", 200, 1024, 5000, 4096), ("q5_k", 200, 960, 5000, 4096)])
 def test_a_call_of_few_rows_readies_a_captured_one_of_more_columns(name, m, n, wide, k):
     """A caller that captures its calls runs one of the same activations first: what that one does not need itself is there for the
     captured one, which takes three launches.  Every replay against the eager result, with other work between."""
