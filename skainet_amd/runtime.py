@@ -227,19 +227,23 @@ def load_library():
 
 # The calls that a program makes once per product or attention step: (context, arguments as their C functions take them) -> return
 # code.  csrc/pycall.c has the same for plain ints without the 1.2 us that ctypes takes; other arguments come here from there.
-def _matvec_q(handle, ggml_type, w, n, k, x, y):
+def _matvec_q_general(handle, ggml_type, w, n, k, x, y):
     return _LIB.skn_matvec_q(handle, ggml_type, _ptr(w), n, k, _ptr(x), _ptr(y))
 
 
-def _gemm_q(handle, ggml_type, w, n, k, a, m, c):
+def _gemm_q_general(handle, ggml_type, w, n, k, a, m, c):
     return _LIB.skn_gemm_q(handle, ggml_type, _ptr(w), n, k, _ptr(a), m, _ptr(c))
 
 
-def _attn_decode(handle, kv, q, n_ctx, scale, out):
+def _attn_decode_general(handle, kv, q, n_ctx, scale, out):
     return _LIB.skn_attn_decode(handle, kv, _ptr(q), n_ctx, scale, _ptr(out))
 
 
+_matvec_q, _gemm_q, _attn_decode = _matvec_q_general, _gemm_q_general, _attn_decode_general
+
+
 def _bind_direct(lib, path):
+    """Binds the callables of csrc/pycall.c, any number of times: two threads may load the library at once."""
     global _matvec_q, _gemm_q, _attn_decode
     try:
         from . import _pycall
@@ -247,7 +251,7 @@ def _bind_direct(lib, path):
         return
     if path == DENSE_LIB_PATH:
         return
-    for name, general in (("matvec_q", _matvec_q), ("gemm_q", _gemm_q), ("attn_decode", _attn_decode)):
+    for name, general in (("matvec_q", _matvec_q_general), ("gemm_q", _gemm_q_general), ("attn_decode", _attn_decode_general)):
         _pycall.bind(name, C.cast(getattr(lib, "skn_" + name), C.c_void_p).value, general)
     _matvec_q, _gemm_q, _attn_decode = _pycall.matvec_q, _pycall.gemm_q, _pycall.attn_decode
 

@@ -1,9 +1,11 @@
 """The direct Python callables of the hot entry points hand over what ctypes hands over, and leave everything else to it."""
 import ctypes as C
+import types
 
 import numpy as np
 import pytest
 
+import skainet_amd
 from skainet_amd import runtime
 
 pycall = pytest.importorskip("skainet_amd._pycall")
@@ -75,3 +77,18 @@ def _attn(handle, kv, q, n_ctx, scale, out):
 
 
 _GENERAL = {"matvec_q": _matvec, "gemm_q": _gemm, "attn_decode": _attn}
+
+
+def test_a_second_load_binds_the_same_general_calls(monkeypatch):
+    """Two threads may both load the library first: the callable that is bound second must not get itself as its general call, which it
+    would then call without end."""
+    bound = []
+    lib = runtime.load_library()
+    fake = types.SimpleNamespace(bind=lambda name, at, general: bound.append((name, general)), matvec_q=len, gemm_q=len, attn_decode=len)
+    monkeypatch.setattr(skainet_amd, "_pycall", fake)
+    for name in SIGNATURES:
+        monkeypatch.setattr(runtime, "_" + name, getattr(runtime, "_" + name))  # (put back afterwards)
+    for _ in range(2):
+        runtime._bind_direct(lib, runtime.LIB_PATH)
+    assert len(bound) == 6 and bound[:3] == bound[3:]
+    assert all(isinstance(general, types.FunctionType) for _, general in bound)
