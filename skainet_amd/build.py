@@ -77,14 +77,22 @@ def build_library(jobs=8, verbose=False, save_temps=False, dense_only=False):
 
 
 def build_pycall():
-    """The Python callables of the hot entry points (csrc/pycall.c).  Without Python's headers or a C compiler the binding calls
-    through ctypes alone."""
+    """The Python callables of the hot entry points (csrc/pycall.c).  They are optional: where they cannot be built -- no headers of this
+    Python, no C compiler or one that fails -- the binding calls through ctypes alone, and none of other sources is left behind."""
     include = sysconfig.get_paths()["include"]
     cc = shutil.which("gcc") or shutil.which("cc")
-    if cc is None or not os.path.exists(os.path.join(include, "Python.h")):
-        return
-    _run([cc, "-O2", "-Wall", "-shared", "-fPIC", "-I", include, os.path.join(CSRC, "pycall.c"), "-o", PYCALL + ".new"])
-    os.replace(PYCALL + ".new", PYCALL)
+    why = "no C compiler" if cc is None else "" if os.path.exists(os.path.join(include, "Python.h")) else f"no Python.h in {include}"
+    if not why:
+        try:
+            _run([cc, "-O2", "-Wall", "-shared", "-fPIC", "-I", include, os.path.join(CSRC, "pycall.c"), "-o", PYCALL + ".new"])
+            os.replace(PYCALL + ".new", PYCALL)
+            return
+        except (RuntimeError, OSError) as e:
+            why = str(e)
+    for path in (PYCALL, PYCALL + ".new"):
+        if os.path.exists(path):
+            os.remove(path)
+    print(f"built without {os.path.basename(PYCALL)}, hot calls go through ctypes: {why}", file=sys.stderr)
 
 
 def ensure_library():

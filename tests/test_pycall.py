@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import skainet_amd
-from skainet_amd import runtime
+from skainet_amd import build, runtime
 
 pycall = pytest.importorskip("skainet_amd._pycall")
 
@@ -92,3 +92,20 @@ def test_a_second_load_binds_the_same_general_calls(monkeypatch):
         runtime._bind_direct(lib, runtime.LIB_PATH)
     assert len(bound) == 6 and bound[:3] == bound[3:]
     assert all(isinstance(general, types.FunctionType) for _, general in bound)
+
+
+@pytest.mark.parametrize("stop", ["compiler fails", "no compiler"])
+def test_the_library_is_built_without_them_where_they_cannot_be(monkeypatch, tmp_path, capsys, stop):
+    target = tmp_path / "_pycall.so"
+    target.write_bytes(b"of older sources")
+    monkeypatch.setattr(build, "PYCALL", str(target))
+    if stop == "no compiler":
+        monkeypatch.setattr(build.shutil, "which", lambda name: None)
+    else:
+        cc = tmp_path / "cc"
+        cc.write_text("#!/bin/sh\necho no space left\nexit 1\n")
+        cc.chmod(0o755)
+        monkeypatch.setattr(build.shutil, "which", lambda name: str(cc))
+    build.build_pycall()
+    assert not target.exists()
+    assert ("no space left" if stop == "compiler fails" else "no C compiler") in capsys.readouterr().err
