@@ -1,6 +1,7 @@
 // Paged KV cache object shared by the cache kernels, decode attention and the decoder.
 #pragma once
 #include "common.h"
+#include "kv_table.h"
 
 // what the pools hold
 enum {
@@ -31,7 +32,7 @@ struct skn_kv {
     int32_t* nctx_dev = nullptr;        // [n_seq] staging for explicit attention lengths
     int* ticket_dev = nullptr;          // workgroups of an append launch count themselves in (zero between launches)
     std::vector<int32_t> page_table;    // pages mapped, -1: none
-    std::vector<int32_t> page_table_on_device;  // what has been uploaded (entries of pages given back stay)
+    skn_device_table on_device;         // what page_table_dev holds (entries of pages given back stay)
     std::vector<int32_t> len;           // host mirror
     std::vector<int32_t> free_pages;    // stack of unmapped page ids
     std::vector<int32_t> nctx_host;     // keeps explicit attention lengths alive while their upload is queued
@@ -40,8 +41,8 @@ struct skn_kv {
 // Maps pages so that sequence `seq` can hold `new_len` tokens; uploads new table entries on the stream.
 int skn_kv_reserve(skn_ctx* ctx, skn_kv* kv, int seq, int new_len);
 
-// Gives a sequence's pages back without the device length being set to zero (skn_kv_reset does both): for a decoder, whose kernels take
-// every length from elsewhere.
+// Gives a sequence's pages back and leaves its device length as it is (skn_kv_reset sets that to zero too): for a decoder, whose kernels
+// take every length from elsewhere.  len_dev of its cache means nothing from then on: what reads it takes no decoder's cache.
 void skn_kv_release(skn_kv* kv, int seq);
 
 // Counts n more tokens into a sequence whose rows were written by a kernel outside the cache code (pages reserved

@@ -9,7 +9,6 @@
 
 namespace {
 
-constexpr int32_t kUnknownPage = -2;  // in page_table_on_device
 constexpr int kMaxAppend = 64;  // entries per launch of the scattered append
 
 struct AppendArgs {
@@ -83,9 +82,11 @@ __global__ void kv_set_len_kernel(int32_t* len, int seq, int n_seq, int value, i
 // (the last page first: the next sequence takes them in the order they were mapped in, and finds its table as it is on the device)
 void release_pages(skn_kv* kv, int seq) {
     for (int p = kv->pages_per_seq - 1; p >= 0; p--) {
-        int32_t& e = kv->page_table[(size_t)seq * kv->pages_per_seq + p];
+        const size_t at = (size_t)seq * kv->pages_per_seq + p;
+        int32_t& e = kv->page_table[at];
         if (e >= 0) {
             kv->free_pages.push_back(e);
+            kv->on_device.given_back(at);
             e = -1;
         }
     }
@@ -108,19 +109,15 @@ int skn_kv_reserve(skn_ctx* ctx, skn_kv* kv, int seq, int new_len) {
     // What the device's table lacks.  An upload is a launch of 5 us beside the kernels, and a sequence that is started again gets the
     // pages it had: a prompt of 512 tokens through 32 layers of the 7B shape 11.0 -> 10.7 ms (with no launch for the
     // lengths in a decoder's reset).
-    int32_t* on_device = &kv->page_table_on_device[(size_t)seq * kv->pages_per_seq];
-    int first_new = 0, last_new = need - 1;
-    while (first_new < need && on_device[first_new] == row[first_new]) first_new++;
-    while (last_new > first_new && on_device[last_new] == row[last_new]) last_new--;
-    if (first_new < need) {
-        const int n = last_new - first_new + 1;
+    const size_t at = (size_t)seq * kv->pages_per_seq;
+    int first, last;
+    if (kv->on_device.lacks(at, row, need, first, last)) {
         // the host vector outlives the copy: the call is synchronous for pageable memory
-        SKN_HIP(ctx, hipMemcpyAsync(kv->page_table_dev + (size_t)seq * kv->pages_per_seq + first_new, row + first_new, (size_t)n * sizeof(int32_t),
-                                    hipMemcpyHostToDevice, ctx->stream));
-        // (recorded into a graph, the copy is made when that is launched, if ever: the entries are uploaded again next time)
+        SKN_HIP(ctx, hipMemcpyAsync(kv->page_table_dev + at + first, row + first, (size_t)(last - first + 1) * sizeof(int32_t), hipMemcpyHostToDevice,
+                                    ctx->stream));
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         SKN_HIP(ctx, hipStreamIsCapturing(ctx->stream, &capture));
-        for (int p = first_new; p <= last_new; p++) on_device[p] = capture == hipStreamCaptureStatusNone ? row[p] : kUnknownPage;
+        kv->on_device.uploaded(at, row, first, last, capture != hipStreamCaptureStatusNone);
     }
     return SKN_OK;
 }
@@ -183,7 +180,7 @@ static int kv_create(skn_ctx* ctx, int n_seq, int n_head, int head_dim, int page
         return rc;
     }
     kv->page_table.assign((size_t)n_seq * kv->pages_per_seq, -1);
-    kv->page_table_on_device.assign((size_t)n_seq * kv->pages_per_seq, -1);
+    kv->on_device.assign((size_t)n_seq * kv->pages_per_seq);
     kv->len.assign(n_seq, 0);
     kv->free_pages.reserve(kv->n_pages);
     for (int p = kv->n_pages - 1; p >= 0; p--) kv->free_pages.push_back(p);

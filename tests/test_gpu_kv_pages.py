@@ -1,5 +1,5 @@
-"""GPU: a cache's page table on the device after sequences have given their pages back: started again in the same order (nothing to upload), in another
-one, longer and shorter than before."""
+"""GPU: a cache's page table on the device after sequences have given their pages back: started again in the same order, in another
+one, longer and shorter than before, alone or all at once.  (Which entries are uploaded: tests/test_kv_table.py.)"""
 import numpy as np
 import pytest
 
