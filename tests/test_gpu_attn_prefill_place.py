@@ -1,10 +1,12 @@
 """GPU: prompt attention at the counts of heads for which its workgroups are placed differently -- the cached heads, else the query heads, else neither
 a multiple of eight -- with ragged blocks of queries, and the rows of q in blocks that are not full."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from oracle import oracle_c, oracle_np
-from skainet_amd import runtime
+from skainet_amd import runtime, synth
 from test_gpu_lebelix_ops import ranged_case, ranged_oracle, rel
 
 pytestmark = pytest.mark.gpu
@@ -37,4 +39,23 @@ def test_grouped_heads(hip, heads, kv_heads):
     kv = runtime.RangedKVCache(hip, 1, kv_heads, dim, vdim, 16, 96, runtime.F16)
     got = kv.attend(0, p, q, k, v, gate)
     assert rel(got, want) < 5e-3  # (fp16 rows: the bar of the other ranged tests)
+    kv.free()
+
+
+@pytest.mark.parametrize("heads,n,dim", [(8, 33, 64), (7, 70, 128), (16, 1, 128)])
+def test_rows_in_bf16_are_the_fp32_rows_rounded(hip, heads, n, dim):
+    """What a decoder's prompt asks of it (skn_attn_prefill_launch with an output type) against the public call on the same cache."""
+    rng = np.random.default_rng(heads + n)
+    q = rng.standard_normal((n, heads, dim)).astype(np.float32)
+    kv = hip.kv_cache(1, heads, dim, 16, n + 16)
+    kv.append_run(0, hip.to_device(synth.kv_f16((n, heads, dim), seed=1)), hip.to_device(synth.kv_f16((n, heads, dim), seed=2)), n)
+    q_dev, wide, narrow = hip.to_device(q), hip.alloc(q.nbytes), hip.alloc(q.nbytes)
+    kv.attn_prefill(0, q_dev, n, wide, dim ** -0.5)
+    hip.memset(narrow, 0xFF, q.nbytes)
+    fn = hip.lib._Z23skn_attn_prefill_launchP7skn_ctxP6skn_kviPKfiifPvii
+    fn.restype, fn.argtypes = C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_float, C.c_void_p, C.c_int, C.c_int]
+    hip._check(fn(hip.handle, kv.handle, 0, q_dev.ptr, n, 1, dim ** -0.5, narrow.ptr, heads, runtime.BF16))
+    got, want = narrow.download(np.uint16, 2 * q.size), synth.f32_to_bf16_bits(wide.download(np.float32, q.size))
+    assert np.array_equal(got[: q.size], want)
+    assert np.all(got[q.size :] == 0xFFFF)  # (nothing behind them)
     kv.free()
