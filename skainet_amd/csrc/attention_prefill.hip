@@ -107,16 +107,12 @@ struct PrefillExt {
     const float* gate = nullptr;
     int ldg = 0;
 };
-// What bounds it: the vector instructions of the softmax between the matrix products (45 % of the clocks of a SIMD against 22 % of
-// matrix instructions at 2000 queries, 32 heads of 64), so the loop has as few as it can: a weight is one exp2 instruction, no test per
-// element for a query that has seen nothing yet, masks only in tiles where some query needs them; the four wavefronts share the
-// merge.  Whole calls with the copy of the keys, with the longer loop and with this one: 2000 x 32 heads x 64 87.8 | 66.6 us, 2048 x 16 x 128
-// 87.2 | 76.2; with the rows of q and the placement below 55 and 59 (512 x 32 x 128 26.6 -> 18.5, 1000 x 32 x 64 31 -> 21.6).  Three wavefronts per SIMD where the registers allow it (D = 64).
+
 // The block of queries and the head of a workgroup.  Workgroups go to the eight XCDs in turn, and each XCD has an L2 of its own (4
 // MiB): the heads that read one cached head stay on one XCD where there are eight of them or a multiple, so that its keys and values
 // come through one L2 only.  In the plain order every XCD read every head, more than its L2 holds, and that traffic was half the time:
-// 512 x 32 heads of 128 25.6 -> 20.1 us, 2048 x 16 of 128 76 -> 60, 1000 x 32 of 64 30 -> 23.7, 2000 x 32 of 64 64 -> 56.  Other counts of
-// heads: the plain order.
+// 512 x 32 heads of 128 25.6 -> 20.1 us, 2048 x 16 of 128 76 -> 60, 1000 x 32 of 64 30 -> 23.7, 2000 x 32 of 64 64 -> 56.  Where only the query
+// heads are a multiple of eight, those are placed each by itself; other counts of heads: the plain order.
 __device__ __forceinline__ void prefill_place(int id, int q_blocks, int n_head, int kv_group, int& qb, int& head) {
     const int group = (n_head / kv_group) % 8 == 0 ? kv_group : 1, units = n_head / group;
     if (units % 8 == 0) {
@@ -130,6 +126,11 @@ __device__ __forceinline__ void prefill_place(int id, int q_blocks, int n_head, 
     }
 }
 
+// attn_prefill_kernel.  What bounds it: the vector instructions of the softmax between the matrix products (45 % of the clocks of a SIMD against 22 % of
+// matrix instructions at 2000 queries, 32 heads of 64), so the loop has as few as it can: a weight is one exp2 instruction, no test per
+// element for a query that has seen nothing yet, masks only in tiles where some query needs them; the four wavefronts share the
+// merge.  Whole calls with the copy of the keys, with the longer loop and with this one: 2000 x 32 heads x 64 87.8 | 66.6 us, 2048 x 16 x 128
+// 87.2 | 76.2; with the rows of q in LDS and the placement above 55 and 59 (512 x 32 x 128 26.6 -> 18.5, 1000 x 32 x 64 31 -> 21.6).  Three wavefronts per SIMD where the registers allow it (D = 64).
 template <int DK, int DV, int KIND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DK > 128 ? 1 : DK > 64 ? 2 : 3))) void attn_prefill_kernel(const float* __restrict__ q, const u32x4* __restrict__ kfrag,
                                                           const u32x4* __restrict__ vfrag, float* __restrict__ out,

@@ -616,9 +616,12 @@ int project_rows(skn_ctx* ctx, skn_llama* m, const int* types, const void* const
 }
 
 // The same with the option llama.expand_weights: Q4_K matrices on their own kernel, the others through their kept copies
-// (`which`: the first matrix's place among a layer's seven), except that up to 256 rows the formats in blocks of 32 are faster from
-// their blocks (us of a call's kernels, Q8_0, blocks | copy: 120 x 4096 x 4096 22.6 | 33.0, 333 x 4096 x 4096 39.0 | 36.5).  The copies
-// are made all the same: the option has the first prompt make them, whatever its length.
+// (`which`: the first matrix's place among a layer's seven), except that up to 256 rows the formats in blocks of 32 are multiplied from
+// their blocks: faster there in each of six shapes and six formats (us of a product, Q8_0, blocks | copy: 120 x 4096 x 4096 22 | 32,
+// 256 x 4096 x 4096 29 | 34, 256 x 2048 x 8192 32 | 51; Q5_1, which gains the least, 256 x 4096 x 4096 33 | 34).  Above the line Q5_1 loses soon
+// (512 x 4096 x 4096 48 | 41) and all formats from 2000 rows on (Q8_0 2000 x 4096 x 4096 170 | 143); between, the others' blocks are as fast or
+// faster (Q8_0 333 x 4096 x 4096 35 | 36, 512 x 11008 x 4096 97 | 102, 512 x 4096 x 4096 43 | 41).  The copies are made all the same: the option
+// has the first prompt make them, whatever its length.
 static int project_expanded(skn_ctx* ctx, skn_llama* m, int l, int which, const int* types, const void* const* blocks, const int* rows, float* const* outs,
                             int count, int k, const skn_gemm_src& src, int T, int accumulate) {
     skn_gemm_seg q4[3], ex[3], bl[3];

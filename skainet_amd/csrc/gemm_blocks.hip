@@ -876,10 +876,11 @@ int superblock_bytes(int t) {
 }
 
 // The kernel of 96-row tiles: where it has a tile for each compute unit at most and the 64-row one more than that.  Those then run beside
-// each other on some units and alone on others, which wait.  us per call, 64 rows | 96: Q8_0 333 x 4096 x 4096 36.0 | 32.1, 90 x 14774 x 13568 100 | 85,
-// 164 x 6786 x 2304 24.8 | 23.2; Q4_0 333 x 4096 x 4096 34.1 | 30.4, 1428 x 645 x 9984 83 | 66; Q5_K 333 x 4096 x 4096 38.7 | 34.3 (30 shapes of this range, three
-// formats: 1.05 to 1.26 times as fast, 1.12 in the mean).  In more rounds the smaller tiles are the faster ones: Q8_0 512 x
-// 4096 x 4096 39.6 | 56, 1000 x 4096 x 11008 163 | 189; and tiles that leave half of the device idle have their k divided instead.
+// each other on some units and alone on others, which wait.  us per call, 64 rows | 96: Q8_0 333 x 4096 x 4096 38.4 | 35.1, 84 x 16021 x 13312 93.9 | 87.6,
+// 71 x 8954 x 2048 20.7 | 17.8; 333 x 4096 x 4096 in Q4_0 35.4 | 33.2, Q4_1 38.4 | 34.8, Q5_0 38.9 | 35.0, Q5_1 43.1 | 36.4, Q5_K 37.8 | 35.0.  Over 34 shapes of
+// this range each of the six formats gains: 1.02 to 1.16 times as fast, 1.07 to 1.11 in the mean of a format, Q5_1 1.10 to 1.31 and 1.21.  In more rounds the
+// smaller tiles are the faster ones: Q8_0 512 x 4096 x 4096 39.6 | 56, 1000 x 4096 x 11008 163 | 189; and tiles that leave half of the device idle have their
+// k divided instead.
 bool one_round_of_pc(const skn_ctx* ctx, int type, int n, int m) {
     const int columns = ((n + kBN - 1) / kBN + 7) / 8 * 8;  // (of the grid)
     return type != SKN_TYPE_Q4_K && m > 64 && ctx->opt_gemm_split == 0 && (int64_t)columns * ((m + 63) / 64) > ctx->compute_units &&

@@ -43,9 +43,9 @@ __device__ __forceinline__ u32x2 lds_u32x2(const uint8_t* p) { return *reinterpr
 // operands times 2^-100, in units of 2^60, where sums of the largest activations and weights of all formats fit; rows that need it are large
 // enough to lose nothing by it.  So a result is finite wherever it is for rows scaled to their largest element.  The first pass pays
 // 0.1 to 0.3 us for looking at the sums (16 x 4096 x 4096 in Q4_K 5.0, 5.0, in Q6_K 6.4, 6.8, in Q8_0 6.0, 6.2) and, where one body of code serves both
-// passes, for the subtraction below.  kTwoBodies: from so many row blocks on a format has a body for each.  Q5_K is 1.05 times as fast for it in the mean over
-// 42 shapes (5 x 4096 x 11008 10.9 -> 10.0 us), Q4_0 1.02 (16 x 4096 x 4096 6.7 -> 6.4), Q6_K of more than sixteen rows 1.01 to 1.03 (32 x 6000 x 6144 17.5 -> 17.1); Q6_K of
-// up to sixteen, Q8_0 and Q4_K, which gain at some sizes and lose at others (Q6_K 16 x 2048 x 2048 5.0 -> 5.1; Q8_0 16 x 512 x 4096 5.5 -> 5.2, 16 x 4096 x 11008 11.8 -> 12.1; Q4_K
+// passes, for the subtraction below.  kTwoBodies: from so many row blocks on a format has a body for each.  Over 45 drawn shapes each, where runs of one
+// build differ by 0.8 %, Q5_K is 1.04 times as fast for it in the mean (5 x 4096 x 11008 10.9 -> 10.0 us), Q4_0 1.03 (16 x 4096 x 4096 6.7 -> 6.4), Q6_K of more
+// than sixteen rows 1.02 (32 x 6000 x 6144 17.5 -> 17.1); Q6_K of up to sixteen, Q8_0 and Q4_K, which gain at some sizes and lose at others (Q6_K 16 x 2048 x 2048 5.0 -> 5.1; Q8_0 16 x 512 x 4096 5.5 -> 5.2, 16 x 4096 x 11008 11.8 -> 12.1; Q4_K
 // 16 x 2048 x 2048 3.9 -> 3.7, 16 x 12000 x 1024 5.3 -> 5.5), keep one.
 constexpr float kUp = 0x1p40f;
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
@@ -470,7 +470,9 @@ skn_family register_family(few_init);
 // 64 rows hold out longer: 64 x 4096 x 11008 (43) Q4_K 24.8 | 23.3, Q8_0 28.7 | 23.5, against 57 x 6000 x 6144 21.2 | 27.3, 25.6 | 26.4.
 // More than 64 rows: Q5_K 128 x 2700 x 2816 (15) 18.2 | 16.6, 512 x 2000 x 1024 (16) 14.0 | 13.9; Q6_K 700 x 2000 x 1024 (21) 24.5 | 19.0; Q8_0 333 x
 // 4096 x 1024 (24) 16.8 | 15.2, 256 x 2700 x 2816 (29) 22.1 | 21.3; Q4_0 512 x 2000 x 1024 13.2 | 12.7, 256 x 2700 x 2816 19.4 | 21.1; Q4_K 160 x 1000 x 2048
-// (6) 16.4 | 6.8, 200 x 1000 x 2048 (8) 16.4 | 6.9, 512 x 2000 x 1024 13.8 | 13.4.
+// (6) 16.4 | 6.8, 200 x 1000 x 2048 (8) 16.4 | 6.9, 512 x 2000 x 1024 13.8 | 13.4.  (The others there had tiles of 64 rows.  Where they take 96 now, these are
+// still 1.16, 1.11 and 1.14 times as fast in the mean over forty shapes each of Q8_0, Q4_0 and Q5_K that come here, and at worst 1.04, 1.08 and 1.08 times
+// as slow, in the upper half of the limits: Q4_0 254 x 4907 x 512 (10) 12.7 | 13.7, 268 x 3547 x 768 (13) 12.7 | 13.6.)
 // Short rows of many columns are launches of many short workgroups, whose ramp the passes' larger tiles pay less often: from so many
 // rounds of compute units on they are faster whatever the superblocks (but for one row block, Q4_0's apart): Q4_0 31 x 30269 x 512 11.8 | 15.3, 25 x 23000 x 512
 // 11.0 | 11.4; Q4_K 252 x 6683 x 256 12.6 | 16.1; Q5_K 32 x 29393 x 512 12.5 | 14.7; Q6_K 370 x 13269 x 256 20.7 | 36.3, 849 x 5423 x 256 44.9 | 35.4; Q8_0 248 x 24474
