@@ -49,6 +49,7 @@ struct skn_ctx {
     // GEMM workspace (fp16 activations, dequantized weight pairs), grown on demand
     void* gemm_ws = nullptr;
     size_t gemm_ws_bytes = 0;
+    bool gemm_ws_kept = false;  // a capture uses it although it is less than such a call asks for: only a call that needs more grows it
     void* gemm_parts = nullptr;  // partial products of GEMMs whose k several workgroups share (gemm_tiles.h)
     size_t gemm_parts_bytes = 0;
 };

@@ -21,6 +21,7 @@
 #include "gemm_few.h"
 #include "gemm_q6k.h"
 #include "gemm_tiles.h"
+#include "gemm_rows.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -2146,18 +2147,29 @@ static bool grow_parts(skn_ctx* ctx, size_t bytes) {
     return true;
 }
 
-int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out, bool ahead) {
-    if (bytes > ctx->gemm_ws_bytes && !(ahead && !may_allocate(ctx))) {
+int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, size_t most, uint8_t** out, bool ahead) {
+    most = std::max(bytes, most);
+    bool grow = bytes > ctx->gemm_ws_bytes && !(ahead && !may_allocate(ctx));
+    if (bytes <= ctx->gemm_ws_bytes && most > ctx->gemm_ws_bytes && !ctx->gemm_ws_kept) {
+        grow = may_allocate(ctx);
+        ctx->gemm_ws_kept = !grow;
+    }
+    if (grow) {
         SKN_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (ctx->gemm_ws) SKN_HIP(ctx, hipFree(ctx->gemm_ws));
         ctx->gemm_ws = nullptr;
         ctx->gemm_ws_bytes = 0;
-        hipError_t e = hipMalloc(&ctx->gemm_ws, bytes);
+        ctx->gemm_ws_kept = false;
+        hipError_t e = hipMalloc(&ctx->gemm_ws, most);
+        if (e != hipSuccess && most > bytes) {
+            (void)hipGetLastError();
+            e = hipMalloc(&ctx->gemm_ws, most = bytes);
+        }
         if (e != hipSuccess) {
             (void)hipGetLastError();
             return skn_fail(ctx, SKN_ERR_OOM, "skn_gemm_q: %zu bytes of workspace: %s", bytes, hipGetErrorString(e));
         }
-        ctx->gemm_ws_bytes = bytes;
+        ctx->gemm_ws_bytes = most;
         // (a workgroup per compute unit and up to 256 x 128 fp32 products of each: 32 MiB)
         if (!ctx->gemm_parts) (void)grow_parts(ctx, (size_t)ctx->compute_units * 256 * 128 * 4);
     }
@@ -2284,7 +2296,8 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     for (int i = 0; i < 3; i++) fs.part_col0[i] = ps.col0[i];
     int splits = tall ? 1 : q4k_splits(ctx, m, mt_rows, m_tiles * fs.n_tiles, k / 256, fs.part_cols);
     uint8_t* ws;
-    int rc = skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes, &ws, src.ahead);
+    const size_t most_rows = skn_tall_rows(m), most = skn_align_up(most_rows * k * 2) + skn_align_up(most_rows * (k / 256) * 16 * 2) + skn_align_up(most_rows * 4);
+    int rc = skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes, most, &ws, src.ahead);
     if (rc != SKN_OK) return rc;
     const size_t part_bytes = tall ? (size_t)tail.tiles * tail.splits * 131072 : splits > 1 ? (size_t)splits * m * fs.part_cols * 4 : 0;
     float* part = part_bytes ? skn_gemm_parts_room(ctx, part_bytes) : nullptr;
@@ -2353,7 +2366,8 @@ static int gemm_in_passes(skn_ctx* ctx, int ggml_type, const void* w_dev, int n,
     const int m_pad = (m + 32 * mt - 1) / (32 * mt) * (32 * mt), n_pad = (n + kBN - 1) / kBN * kBN;
     const size_t af_bytes = skn_align_up((size_t)m_pad * k * 2), is_bytes = skn_align_up((size_t)m_pad * 4);
     uint8_t* ws;
-    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes + (size_t)n_pad * k * 4, &ws);
+    const size_t bytes = af_bytes + is_bytes + (size_t)n_pad * k * 4;
+    int rc = skn_gemm_workspace(ctx, bytes, bytes, &ws);
     if (rc != SKN_OK) return rc;
     _Float16* afrag = (_Float16*)ws;
     float* isc = (float*)(ws + af_bytes);
@@ -2444,7 +2458,8 @@ int skn_gemm_q6k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
         if (splits[i] > 1) part_bytes = std::max(part_bytes, (size_t)splits[i] * m * segs[i].n * 4);
     }
     uint8_t* ws;
-    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes, &ws, src.ahead);
+    const size_t most_rows = skn_tall_rows(m);
+    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes, skn_align_up(most_rows * k * 2) + skn_align_up(most_rows * 4), &ws, src.ahead);
     if (rc != SKN_OK) return rc;
     _Float16* afrag = (_Float16*)ws;
     float* isc = (float*)(ws + af_bytes);
@@ -2496,7 +2511,7 @@ int skn_gemm_expanded_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, in
     SKN_REQUIRE(ctx, af_bytes < ((size_t)1 << 31), SKN_ERR_SHAPE,
                 "expanded GEMM: %d rows of %d activations exceed the 2^30 elements one call takes", m, k);
     uint8_t* ws;
-    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes, &ws);
+    int rc = skn_gemm_workspace(ctx, af_bytes + is_bytes, af_bytes + is_bytes, &ws);
     if (rc != SKN_OK) return rc;
     _Float16* afrag = (_Float16*)ws;
     float* isc = (float*)(ws + af_bytes);

@@ -19,7 +19,7 @@
 // us per call, before -> now (weights as fp16 pairs -> this): Q8_0 333 x 4096 x 4096 51.6 -> 32.1, 512 x 14336 x 4096 236 -> 115, 41 x 4096 x
 // 11008 102 -> 28.5; Q5_K 512 x 4096 x 4096 60 -> 39.2; Q4_0 5 x 4096 x 4096 36.6 -> 11.5.
 #include "gemm_blocks.h"
-#include "gemm_blocks_rows.h"
+#include "gemm_rows.h"
 #include "gemm_tiles.h"
 
 #include <algorithm>
@@ -932,7 +932,7 @@ int skn_gemm_blocks_multi(skn_ctx* ctx, const int* types, const skn_gemm_seg* se
     const size_t af_bytes = skn_align_up((size_t)m_pad * k * 2), sf_bytes = sums ? skn_align_up((size_t)m_pad * (k / 256) * 32) : 0;
     const size_t is_bytes = skn_align_up((size_t)m_pad * 4);
     uint8_t* ws;
-    SKN_TRY(skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes, &ws, src.ahead));
+    SKN_TRY(skn_gemm_workspace(ctx, af_bytes + sf_bytes + is_bytes, af_bytes + sf_bytes + is_bytes, &ws, src.ahead));
     u32x4* afrag = (u32x4*)ws;
     _Float16* sfrag = (_Float16*)(ws + af_bytes);
     float* isc = (float*)(ws + af_bytes + sf_bytes);

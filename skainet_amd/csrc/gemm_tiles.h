@@ -82,9 +82,10 @@ struct skn_gemm_parts {
 
 int skn_gemm_add_parts(skn_ctx* ctx, const float* part, int splits, int cols, const skn_gemm_parts& segs, const float* inv_scale, int m);
 int skn_gemm_k_splits(const skn_ctx* ctx, int m, int tiles, int nb);
-// grows the context's GEMM workspace; the pointer stays valid until the next growth.  `ahead`: for a later call (skn_gemm_src); what a
-// capture does not allow is left out.
-int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, uint8_t** out, bool ahead = false);
+// grows the context's GEMM workspace; the pointer stays valid until the next growth.  `most`: what a call of the same type, m and k may need
+// with another matrix, which is there after the first call outside a capture.  `ahead`: for a later call (skn_gemm_src); what a capture does
+// not allow is left out.
+int skn_gemm_workspace(skn_ctx* ctx, size_t bytes, size_t most, uint8_t** out, bool ahead = false);
 // Room for partial products, to be asked for behind the workspace; null where there is none: k stays undivided.  What the library's
 // own divisions take at most comes with the context's first workspace, so that a call allocates no more often than it would undivided
 // (a caller that captures a call has run one that needed as much of the workspace).

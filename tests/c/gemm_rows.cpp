@@ -1,9 +1,10 @@
 // Walks the row blocks of the products on 96-row tiles: every one lies inside the operands' layout, and a block with rows of the output is
-// the block itself.  Prints the number of blocks looked at.
+// the block itself.  The room of the other formats' operands takes every height of tile.  Prints the number of blocks looked at.
 #include <cstdio>
 #include <cstdlib>
+#include <initializer_list>
 
-#include "gemm_blocks_rows.h"
+#include "gemm_rows.h"
 
 int main() {
     long long looked = 0;
@@ -14,6 +15,8 @@ int main() {
             const int from = skn_blocks_of_96(block, m);
             ok = ok && from >= 0 && 32 * from + 32 <= rows && (32 * block >= m || from == block);
         }
+        for (int height : {32, 64, 128, 256})
+            if (m > 128 || height < 128) ok = ok && skn_tall_rows(m) >= (m + height - 1) / height * height;
         if (!ok) {
             std::printf("%d rows\n", m);
             return 1;

@@ -215,7 +215,7 @@ def test_weights_and_activations_on_their_least_alignment(hip):
 
 
 @pytest.mark.parametrize("name,m,n,wide,k", [("q8_0", 333, 1024, 4096, 4096), ("q5_k", 41, 512, 20000, 4096), ("q6_k", 33, 512, 20000, 4096), ("q4_k", 48, 512, 20000, 4096),
-                                             ("q4_k", 17, 256, 20000, 4096), ("q8_0", 200, 1024, 5000, 4096), ("q5_k", 200, 960, 5000, 4096)])
+                                             ("q4_k", 17, 256, 20000, 4096), ("q8_0", 200, 1024, 5000, 4096), ("q5_k", 200, 960, 5000, 4096), ("q4_k", 300, 1024, 14336, 1024), ("q6_k", 300, 1024, 14336, 1024)])
 def test_a_call_of_few_rows_readies_a_captured_one_of_more_columns(name, m, n, wide, k):
     """A caller that captures its calls runs one of the same activations first: what that one does not need itself is there for the
     captured one, which takes three launches.  Every replay against the eager result, with other work between."""
@@ -256,3 +256,41 @@ def test_a_call_of_few_rows_readies_a_captured_one_of_more_columns(name, m, n, w
         call("hipGraphDestroy", graph)
         ctx.set_stream(None)
         call("hipStreamDestroy", stream)
+
+
+def test_a_workspace_that_a_capture_uses_is_not_grown_for_other_matrices_of_its_rows():
+    """A call captured without one of its type before, in a workspace that is enough for its tiles but not for the highest of its rows: the same
+    call outside the capture leaves that workspace where it is."""
+    m, n, k, t = 300, 2048, 1024, synth.Q6_K
+    rt = runtime.load_library()
+    stream, graph, replay = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    with runtime.Context(0) as ctx:
+        assert rt.hipStreamCreate(C.byref(stream)) == 0
+        ctx.set_stream(stream)
+        ctx.set_option("gemm.few", 0)
+        w8, x8 = ctx.to_device(synth.weight(synth.Q8_0, n, k, seed=1)), ctx.to_device(synth.activation_bf16((384, k), seed=2))
+        w, x = ctx.to_device(synth.weight(t, n, k, seed=3)), ctx.to_device(synth.activation_bf16((m, k), seed=4))
+        c = ctx.alloc(4 * 384 * n)
+        ctx.gemm_q(synth.Q8_0, w8, n, k, x8, 384, c)  # (operands of 384 rows: what 128-row tiles of 300 take, 256-row ones 512)
+        ctx.sync()
+        assert rt.hipStreamBeginCapture(stream, 1) == 0
+        try:
+            ctx.gemm_q(t, w, n, k, x, m, c)
+        finally:
+            ended = rt.hipStreamEndCapture(stream, C.byref(graph))
+        assert ended == 0 and rt.hipGraphInstantiate(C.byref(replay), graph, None, None, C.c_size_t(0)) == 0
+        free, total = C.c_size_t(), C.c_size_t()
+        assert rt.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        ctx.gemm_q(t, w, n, k, x, m, c)
+        ctx.sync()
+        want, before = c.download(np.float32, m * n).view(np.uint32), free.value
+        assert rt.hipMemGetInfo(C.byref(free), C.byref(total)) == 0 and free.value == before
+        for _ in range(3):
+            ctx.memset(c, 0xFF, 4 * m * n)
+            ctx.sync()
+            assert rt.hipGraphLaunch(replay, stream) == 0
+            ctx.sync()
+            assert np.array_equal(c.download(np.float32, m * n).view(np.uint32), want)
+        assert rt.hipGraphExecDestroy(replay) == 0 and rt.hipGraphDestroy(graph) == 0
+        ctx.set_stream(None)
+        assert rt.hipStreamDestroy(stream) == 0
