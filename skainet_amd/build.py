@@ -32,6 +32,9 @@ ARCH = "gfx950"
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc", "-Wall", "-Wno-unused-function",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # the first sixteen dwords of a kernel's arguments are in scalar registers when a wavefront starts (single values up to the first struct), a
+    # load's latency less ahead of its first request: 0.3 us of a launch of 8 MB
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
 ]
 
 

@@ -1,9 +1,12 @@
-// Batch-1 product of a stacked dense matrix (bf16 or fp32 weights) with an fp32 vector: bound by the weight stream.
+// Batch-1 product of a stacked dense matrix (bf16 or fp32 weights) with an fp32 vector: bound by the weight stream, and a small one by
+// the chain of latencies from the launch's arguments to its last store.
 //
-// The input is staged once per workgroup in LDS -- plain, divided group by group by its root mean square (the norm ahead
+// dense_matvec_once_kernel (most calls): a workgroup has a few rows, its wavefronts share them piece by piece, and everything is asked for
+// at once.  dense_matvec_kernel (inputs whose preparation is large beside the rows of one workgroup, see once_rows): the input
+// is staged once per workgroup in LDS -- plain, divided group by group by its root mean square (the norm ahead
 // of a layer), or with the split partials of an attention merged on the way in -- as two planes of float4 (even and odd
 // fours of elements), so that the eight activations of a 16-byte piece of bf16 weights are two conflict-free 16-byte
-// reads.  A wavefront takes a row at a time and walks on through the stacked rows; its next requests are under way while it
+// reads; a wavefront takes a row at a time and walks on through the stacked rows; its next requests are under way while it
 // multiplies, the first ones from before the staging.  Epilogue: bias and the operation
 // of the segment, or the residual sum; a key projection also goes to its page of the cache.
 #include "dense.h"
@@ -15,14 +18,14 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// Workgroups of T threads.  Eight wavefronts where that makes at most a workgroup per compute unit (a matrix of 2048 rows reaches 256
+// Workgroups of T threads of the staged kernel (figures of calls that dense_matvec_once_kernel takes now too: the rule is from before it).  Eight
+// wavefronts where that makes at most a workgroup per compute unit (a matrix of 2048 rows reaches 256
 // of them, with sixteen wavefronts half: 5.5 against 5.9 us at 2048 rows, 4.8 against 5.2 at 1024), and behind a norm where the rows
 // fill the device twice (4288 rows 13.0 against 14.5 us, 6016 rows 14.0 against 15.3) or are a single turn of requests long (3232 rows
 // of 2048 7.95 against 8.34 us), up to three per compute unit.  Sixteen, one workgroup per compute unit, for what lies between, where
 // the compute units with two workgroups of eight would be the last (2560 rows of 14000 16.6 against 18.8 us, of 6000 8.2 against 9.1;
 // behind a norm 2624 rows of 2560 8.0 against 8.5, 3232 rows of 4096 9.9 against 11.0), and for more rows behind a plain staging
-// (6144 rows 6.7 against 7.1).  A decode step of eight layers of width 2048 (945 MB of weights, 27 launches): 313 us; sixteen wavefronts
-// everywhere 330, four 331 and more.
+// (6144 rows 6.7 against 7.1).
 constexpr int kPerCu = 3;
 constexpr int kR = 1;  // rows per wavefront and turn (measured with two as well: slower)
 constexpr int kU = 4;  // 16-byte pieces per row and lane in flight, twice
@@ -381,6 +384,379 @@ __global__ __launch_bounds__(T) void dense_matvec_kernel(const W* __restrict__ w
     }
 }
 
+// ---- every request at once ----------------------------------------------------------------------------------------------------
+// R rows to a workgroup; each of its wavefronts has PW pieces of 1 KiB of every one of them and the same pieces of the input in its
+// registers, so that the input passes neither LDS nor a barrier ahead of the products, and all that the workgroup reads is under way
+// before it waits for anything.  A factor of the whole input (one norm group) goes to the results; the wavefronts' sums meet in LDS, sixteen
+// threads end a row.  What a launch of a few megabytes costs beside its bytes is dependent steps: arguments that are needed
+// first are single values, which the device hands a wavefront in registers (build.py), and those of an epilogue that is not taken are
+// not read.  us per launch in a captured graph, weights from memory, dense_matvec_kernel -> this: 2048 x 2048 4.85 -> 3.5, 256 x 2048
+// and 2048 x 256 together 8.8 -> 4.8, 2048 x 8192 8.9 -> 7.3, behind a norm 8192 x 2048 8.7 -> 7.5 and 32000 x 2048 24.8 -> 22.8, behind a sum and
+// a norm 2624 x 2048 6.8 -> 4.9; a bare read of 8.4 MB 2.95, of 33.6 MB 6.6.  Over 240 shapes 1.2 (merges) to 1.4 (norms) times as fast in the mean of a mode.
+struct OnceArgs {
+    const float *add, *add_w;               // of a sum
+    float* x_out;
+    int groups, group_size;                 // of the norm
+    float eps, mult;
+    int cache_seg, mul_seg;
+    const float *ml, *gate;                 // of a merge
+    int heads, dim, dim_pad, splits, sink;
+    skn_dense_seg seg;                      // the first
+    int starts[kDenseMaxSegs];              // first rows of the segments
+};
+
+// a[0..N) summed over the 64 lanes, four of them in a register: lane 16 j (and the fifteen behind it) of register i has a[index(i, j)]
+template <int N>
+struct LaneSums {
+    static constexpr int kRegs = (N + 3) / 4, kPairs = (N + 1) / 2;
+    float v[kRegs];
+    __device__ __forceinline__ explicit LaneSums(const float (&a)[N]) {
+        float h[kPairs];
+#pragma unroll
+        for (int i = 0; i < kPairs; i++) {
+            const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[2 * i]), 2 * i + 1 < N ? __float_as_uint(a[2 * i + 1]) : 0u, false, false);
+            h[i] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+        }
+#pragma unroll
+        for (int i = 0; i < kRegs; i++) {
+            const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[2 * i]), 2 * i + 1 < kPairs ? __float_as_uint(h[2 * i + 1]) : 0u, false, false);
+            v[i] = row16_sum(__uint_as_float(s[0]) + __uint_as_float(s[1]));
+        }
+    }
+    static __device__ __forceinline__ int index(int i, int j) { return 4 * i + (j >> 1) + 2 * (j & 1); }
+};
+
+constexpr int kOnceGroups = 8;  // norm groups
+
+constexpr int kOnceParts = 16;  // wavefronts of a workgroup, half of them where the input is worked on (a merge has a hundred registers of partials)
+
+// W: uint16_t (bf16) or float.  X: 1, or 2 with a second input (SKN_XSRC_PLAIN); the most splits that are merged (SKN_XSRC_MERGE).
+// parts_nseg: wavefronts of the workgroup, segments << 16.
+template <typename W, int MODE, int PW, int R, int SP>
+__global__ __launch_bounds__(64 * (MODE == SKN_XSRC_MERGE ? kOnceParts / 2 : kOnceParts)) void dense_matvec_once_kernel(
+    const float* __restrict__ x_in, const void* __restrict__ w, const float* __restrict__ bias, float* resid, int k, int row_bytes, int last_piece,
+    uint32_t parts_nseg, int resid_rows, const float* __restrict__ norm_w, const OnceArgs args, const skn_dense_out out) {
+    constexpr int V = 16 / (int)sizeof(W), Q = V / 4;
+    constexpr bool kAdd = MODE == SKN_XSRC_ADD_NORM, kNorm = MODE == SKN_XSRC_GROUP_NORM || kAdd, kMerge = MODE == SKN_XSRC_MERGE;
+    constexpr int SC = SP < 8 ? SP : 8;                       // splits requested ahead
+    __shared__ float sums[R][kOnceParts];                     // of rows, by part
+    __shared__ float squares[kOnceGroups + 1][kOnceParts];
+    const int tid = threadIdx.x, lane = tid & 63, part = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int parts = (int)(parts_nseg & 0xFFFFu), nseg = (int)(parts_nseg >> 16);
+    const int row0 = (int)blockIdx.x * R;
+
+    // ---- requests: the input's first, they are answered in order ----
+    const int quad0 = (part * PW * 64 + lane) * Q;
+    float4 x[PW][Q], wq[kNorm ? PW : 1][Q], y[kAdd ? PW : 1][Q], yw[kAdd ? PW : 1][Q];
+    int left[PW];  // columns from the lane's first one of a piece on
+    float2 ml[PW][SP];
+    float4 parted[PW][SC][Q], gate[kMerge ? PW : 1][Q];
+    const float* of_head[PW];
+    int64_t next_split = 0;
+    if constexpr (kMerge) next_split = (int64_t)args.heads * args.dim_pad;
+#pragma unroll
+    for (int p = 0; p < PW; p++) {
+        const int quad = quad0 + p * 64 * Q;
+        left[p] = k - 4 * quad;
+        if constexpr (kMerge) {
+            const int e = min(4 * quad, k - V), h = e / args.dim;  // (a lane's columns of a piece are of one head)
+            of_head[p] = x_in + (int64_t)h * args.dim_pad + (e - h * args.dim);
+#pragma unroll
+            for (int i = 0; i < SP; i++) ml[p][i] = reinterpret_cast<const float2*>(args.ml)[min(i, args.splits - 1) * args.heads + h];
+#pragma unroll
+            for (int i = 0; i < SC; i++)
+#pragma unroll
+                for (int j = 0; j < Q; j++) parted[p][i][j] = reinterpret_cast<const float4*>(of_head[p] + min(i, args.splits - 1) * next_split)[j];
+            if (args.gate)
+#pragma unroll
+                for (int j = 0; j < Q; j++) gate[p][j] = reinterpret_cast<const float4*>(args.gate + e)[j];
+            continue;
+        }
+#pragma unroll
+        for (int i = 0; i < Q; i++) {
+            const uint32_t at = 16u * (uint32_t)min(quad + i, (k - 1) >> 2);
+            if constexpr (kAdd) y[p][i] = *reinterpret_cast<const float4*>((const char*)args.add + at), yw[p][i] = *reinterpret_cast<const float4*>((const char*)args.add_w + at);
+            x[p][i] = *reinterpret_cast<const float4*>((const char*)x_in + at);
+            if constexpr (kNorm) wq[p][i] = *reinterpret_cast<const float4*>((const char*)norm_w + at);
+        }
+    }
+    const int my = row0 + min(tid >> 4, R - 1);  // the row that this thread and fifteen others end
+    const float bias_v = bias ? bias[my] : 0.f;
+    const float resid_v = resid ? resid[min(my, resid_rows - 1)] : 0.f;
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 c[R][PW];
+    const char* rows = (const char*)w + (int64_t)row0 * row_bytes;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int p = 0; p < PW; p++)
+            c[r][p] = *reinterpret_cast<const u32x4*>(rows + (int64_t)r * row_bytes + (uint32_t)min((part * PW + p) * 1024 + lane * 16, last_piece));  // (past the end: times zeros)
+    __builtin_amdgcn_sched_barrier(0);
+
+    // the segment of the workgroup's rows (a power of two of them, at most 32: they are of one segment)
+    int si = 0;
+    if (nseg > 1) {
+#pragma unroll
+        for (int q = 1; q < kDenseMaxSegs; q++) si = q < nseg && row0 >= args.starts[q] ? q : si;
+    }
+    const skn_dense_seg sg = nseg > 1 ? out.seg[si] : args.seg;
+    int cache_page = 0, cache_slot = 0;
+    if (args.cache_seg == si) {
+        const int pos = *out.pos_dev;
+        cache_page = out.page_table[pos / out.page_tokens];
+        cache_slot = pos % out.page_tokens;
+    }
+    auto mul_of = [&](int row) __attribute__((always_inline)) {
+        return skn_table_at(out.mul_table, out.mul_type, (int64_t)*out.mul_tokens * out.mul_ld + out.mul_col + min(row - sg.row0, sg.rows - 1));
+    };
+    const float mul_v = args.mul_seg == si ? mul_of(my) : 1.f;
+
+    // ---- the input ----
+    auto square = [](const float4& v) { return (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w); };
+    auto sum_of = [&](const float* from) __attribute__((always_inline)) {  // of the parts
+        const float t = from[lane & (kOnceParts - 1)];
+        return row16_sum((lane & (kOnceParts - 1)) < parts ? t : 0.f);
+    };
+    if constexpr (kMerge) {
+#pragma unroll
+        for (int p = 0; p < PW; p++) {
+            float m = args.sink ? 0.f : -INFINITY;
+#pragma unroll
+            for (int i = 0; i < SP; i++) m = fmaxf(m, ml[p][i].x);
+            float l = args.sink ? __builtin_amdgcn_exp2f(-m) : 0.f;
+#pragma unroll
+            for (int i = 0; i < SP; i++) {
+                ml[p][i].x = i < args.splits ? __builtin_amdgcn_exp2f(ml[p][i].x - m) : 0.f;  // (an empty split: exp2(-inf) = 0)
+                l = fmaf(ml[p][i].x, ml[p][i].y, l);
+            }
+            const float inv = 1.0f / l;
+#pragma unroll
+            for (int j = 0; j < Q; j++) x[p][j] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int i = 0; i < SP; i++) {
+                const float f = ml[p][i].x * inv;
+#pragma unroll
+                for (int j = 0; j < Q; j++) {
+                    const float4 v = i < SC ? parted[p][i % SC][j] : reinterpret_cast<const float4*>(of_head[p] + min(i, args.splits - 1) * next_split)[j];
+                    float4& a = x[p][j];
+                    a.x = fmaf(f, v.x, a.x), a.y = fmaf(f, v.y, a.y), a.z = fmaf(f, v.z, a.z), a.w = fmaf(f, v.w, a.w);
+                }
+            }
+            if (args.gate)
+#pragma unroll
+                for (int j = 0; j < Q; j++) x[p][j].x *= gate[p][j].x, x[p][j].y *= gate[p][j].y, x[p][j].z *= gate[p][j].z, x[p][j].w *= gate[p][j].w;
+        }
+    }
+    if (4 * (parts * PW * 64 * Q) > k) {  // (what is past the last column counts as zero)
+#pragma unroll
+        for (int p = 0; p < PW; p++)
+#pragma unroll
+            for (int i = 0; i < Q; i++) {
+                const int n = left[p] - 4 * i;
+                auto cut = [&](float4& v) __attribute__((always_inline)) {
+                    v.x = n > 0 ? v.x : 0.f, v.y = n > 1 ? v.y : 0.f, v.z = n > 2 ? v.z : 0.f, v.w = n > 3 ? v.w : 0.f;
+                };
+                cut(x[p][i]);
+                if constexpr (kAdd) cut(y[p][i]), cut(yw[p][i]);
+                if constexpr (kNorm) cut(wq[p][i]);
+            }
+    }
+    if constexpr (kAdd) {
+        float ss = 0.f;
+#pragma unroll
+        for (int p = 0; p < PW; p++)
+#pragma unroll
+            for (int i = 0; i < Q; i++) ss += square(y[p][i]);
+        ss = wave_sum(ss);
+        if (lane == 0) squares[kOnceGroups][part] = ss;
+        __syncthreads();
+        const float ry = 1.0f / sqrtf(sum_of(squares[kOnceGroups]) / (float)k + args.eps);
+#pragma unroll
+        for (int p = 0; p < PW; p++)
+#pragma unroll
+            for (int i = 0; i < Q; i++) {
+                float4& v = x[p][i];
+                const float4 a = y[p][i], g = yw[p][i];
+                v.x = fmaf(a.x * ry, g.x, v.x), v.y = fmaf(a.y * ry, g.y, v.y), v.z = fmaf(a.z * ry, g.z, v.z), v.w = fmaf(a.w * ry, g.w, v.w);
+                if (blockIdx.x == 0 && left[p] > 4 * i) reinterpret_cast<float4*>(args.x_out)[quad0 + p * 64 * Q + i] = v;
+            }
+    }
+    const bool one_norm = kAdd || (kNorm && args.groups == 1);  // (its factor goes to the results)
+    if constexpr (kNorm) {
+        if (one_norm) {
+            float ss = 0.f;
+#pragma unroll
+            for (int p = 0; p < PW; p++)
+#pragma unroll
+                for (int i = 0; i < Q; i++) ss += square(x[p][i]);
+            ss = wave_sum(ss);
+            if (lane == 0) squares[0][part] = ss;
+        } else {
+            int g[PW];
+            float d[PW];
+#pragma unroll
+            for (int p = 0; p < PW; p++) {
+                g[p] = min(4 * (quad0 + p * 64 * Q), k - 1) / args.group_size;  // (a lane's columns of a piece are of one group)
+                d[p] = 0.f;
+#pragma unroll
+                for (int i = 0; i < Q; i++) d[p] += square(x[p][i]);
+            }
+            for (int n = 0; n < args.groups; n++) {
+                float t = 0.f;
+#pragma unroll
+                for (int p = 0; p < PW; p++) t += g[p] == n ? d[p] : 0.f;
+                t = wave_sum(t);
+                if (lane == 0) squares[n][part] = t;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int p = 0; p < PW; p++) {
+                float t = 0.f;
+                for (int i = 0; i < parts; i++) t += squares[g[p]][i];
+                const float r = 1.0f / sqrtf(t / (float)args.group_size + args.eps);
+#pragma unroll
+                for (int i = 0; i < Q; i++) x[p][i].x *= r, x[p][i].y *= r, x[p][i].z *= r, x[p][i].w *= r;
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < PW; p++)
+#pragma unroll
+            for (int i = 0; i < Q; i++) {
+                const float4 g = wq[p][i];
+                x[p][i].x *= g.x, x[p][i].y *= g.y, x[p][i].z *= g.z, x[p][i].w *= g.w;
+            }
+    }
+
+    // ---- the products ----
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        acc[r] = 0.f;
+#pragma unroll
+        for (int p = 0; p < PW; p++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t d = c[r][p][j];
+                if constexpr (sizeof(W) == 2) {
+                    const float4 v = x[p][j >> 1];
+                    acc[r] = fmaf(__uint_as_float(d << 16), (j & 1) ? v.z : v.x, acc[r]);
+                    acc[r] = fmaf(__uint_as_float(d & 0xFFFF0000u), (j & 1) ? v.w : v.y, acc[r]);
+                } else {
+                    const float4 v = x[p][0];
+                    acc[r] = fmaf(__uint_as_float(d), j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w, acc[r]);
+                }
+            }
+    }
+    const LaneSums<R> total(acc);
+#pragma unroll
+    for (int i = 0; i < LaneSums<R>::kRegs; i++) {
+        const int r = LaneSums<R>::index(i, lane >> 4);
+        if ((lane & 15) == 0 && r < R) sums[r][part] = total.v[i];
+    }
+    __syncthreads();
+
+    // ---- a row to sixteen threads ----
+    for (int m = tid >> 4; m < R; m += 4 * parts) {
+        const bool first = m == tid >> 4;  // (the only turn but for a single wavefront of eight rows)
+        const int row = row0 + m, r = row - sg.row0;
+        float z = sum_of(sums[m]);
+        if (one_norm) z *= 1.0f / sqrtf(sum_of(squares[0]) / (float)k + args.eps);
+        z += first ? bias_v : bias ? bias[row] : 0.f;
+        if ((tid & 15) != 0) continue;
+        if (resid) {
+            if (row < resid_rows) resid[row] = fmaf(args.mult, z, first ? resid_v : resid[row]);
+            continue;
+        }
+        if (r >= sg.rows) continue;
+        z = skn_dense_op(sg.op, z, sg.p0, sg.p1);
+        if (args.mul_seg == si) z *= first ? mul_v : mul_of(row);
+        if (sg.out_type == SKN_TYPE_F32) ((float*)sg.out)[r] = z;
+        else ((uint16_t*)sg.out)[r] = skn_bf16_bits(z);
+        if (args.cache_seg == si) {
+            const int h = r / out.dim;
+            const int64_t at = (((int64_t)cache_page * out.kv_heads + h) * out.page_tokens + cache_slot) * out.dim_pad + (r - h * out.dim);
+            if (out.elem_type == SKN_TYPE_F32) ((float*)out.k_pool)[at] = z;
+            else ((uint16_t*)out.k_pool)[at] = __half_as_ushort(__float2half_rn(z));
+        }
+    }
+}
+
+template <typename W, int MODE, int PW, int R, int SP>
+int launch_once(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, const skn_dense_out& out, int parts) {
+    OnceArgs a = {};
+    a.add = src.add, a.add_w = src.add_w, a.x_out = src.x_out;
+    a.groups = src.groups, a.group_size = src.k0 / src.groups, a.eps = src.eps, a.mult = out.mult;
+    a.cache_seg = out.cache_seg, a.mul_seg = out.mul_seg;
+    a.ml = src.ml, a.gate = src.gate, a.heads = src.heads, a.dim = src.dim, a.dim_pad = src.dim_pad, a.splits = src.splits, a.sink = src.sink;
+    if (out.nseg > 0) a.seg = out.seg[0];
+    for (int q = 0; q < out.nseg; q++) a.starts[q] = out.seg[q].row0;
+    skn_launch(ctx, dense_matvec_once_kernel<W, MODE, PW, R, SP>, dim3((unsigned)(w.rows / R)), dim3(64 * parts), 0, src.x0, w.w, w.bias,
+               out.nseg == 0 ? out.resid : (float*)nullptr, src.k0, (w.ld ? w.ld : w.k_pad) * (int)sizeof(W), w.k_pad * (int)sizeof(W) - 16,
+               (uint32_t)(parts | out.nseg << 16), out.resid_rows, src.norm_w, a, out);
+    SKN_LAUNCH_CHECK(ctx);
+    return SKN_OK;
+}
+
+// Rows of a workgroup of dense_matvec_once_kernel whose `parts` wavefronts share `rows` rows; 0: the input takes so much that many rows are better
+// behind one staging of it.  Four rows where the input is taken as it is (two where that leaves compute units without work): 2048 x 2048
+// 3.52 | 3.49 | 3.59 us with 2 | 4 | 8, 2048 x 8192 8.0 | 7.3 | 7.7, 256 x 2048 and 2048 x 256 4.96 | 4.80 | 5.20.  A norm's launch takes rounds of compute
+// units, a round of 2, 4, 8, 16 rows as 0.38, 0.6, 1, 1.9 (960 x 3072 behind a sum and a norm 5.2 | 4.2 | 4.6 | 5.5, 2624 x 3072 9.5 | 7.4 | 7.2 | 6.1, 5120 x
+// 3072 15.0 | 10.8 | 9.6 | 10.2): over eighty shapes of a mode this is 1 % off the best number in the mean.  The staged kernel: behind a sum and a norm 13312 x 2048
+// 11.8 | 12.7 us, x 3072 16.6 | 18.6, but 8192 x 2048 9.8 | 8.2, 5120 x 4096 12.2 | 11.3; behind a merge of eight splits 4096 x 3072 9.5 | 9.7, 2624 x 4096 9.6 |
+// 10.4, but 5120 x 2048 9.1 | 8.5, 2048 x 4096 7.7 | 7.0.
+int once_rows(int mode, int rows, int parts, int units) {
+    const int64_t pieces = (int64_t)rows * parts;
+    if (mode == SKN_XSRC_PLAIN) return parts == 1 ? 8 : rows <= 2 * units ? 2 : 4;
+    if (mode == SKN_XSRC_MERGE) return pieces > 80 * units ? 0 : rows <= 4 * units ? 4 : 8;
+    if (mode == SKN_XSRC_ADD_NORM && pieces > 176 * units) return 0;
+    const float round_cost[4] = {0.38f, 0.6f, 1.0f, 1.9f};
+    int best = 0;
+    float least = INFINITY;
+    for (int i = 0; i < 4; i++) {
+        const int r = 2 << i;
+        const float rounds = (float)rows / (float)(r * units), cost = round_cost[i] * (0.7f * ceilf(rounds) + 0.3f * rounds);
+        if (r <= 8 * parts && cost < least) best = r, least = cost;
+    }
+    return best;
+}
+
+// SKN_ERR_TYPE, without a message: not a call for dense_matvec_once_kernel
+template <typename W, int MODE>
+int try_once(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, const skn_dense_out& out) {
+    constexpr int V = 16 / (int)sizeof(W);
+    const int pieces = (w.k_pad + 64 * V - 1) / (64 * V);
+    const int pw = MODE != SKN_XSRC_PLAIN || pieces <= kOnceParts ? 1 : pieces <= 2 * kOnceParts ? 2 : 4, parts = (pieces + pw - 1) / pw;
+    if (src.x1 || parts > (MODE == SKN_XSRC_PLAIN ? kOnceParts : kOnceParts / 2) || (int64_t)(w.ld ? w.ld : w.k_pad) * (int)sizeof(W) >= (int64_t)1 << 30) return SKN_ERR_TYPE;
+    const int r = once_rows(MODE, w.rows, parts, ctx->compute_units);
+    if constexpr (MODE == SKN_XSRC_MERGE) {
+        if (src.dim % V != 0 || r == 0) return SKN_ERR_TYPE;
+        auto rows = [&](auto four) {
+            constexpr int R = decltype(four)::value ? 4 : 8;
+            return src.splits <= 2   ? launch_once<W, MODE, 1, R, 2>(ctx, w, src, out, parts)
+                   : src.splits <= 4 ? launch_once<W, MODE, 1, R, 4>(ctx, w, src, out, parts)
+                   : src.splits <= 8 ? launch_once<W, MODE, 1, R, 8>(ctx, w, src, out, parts)
+                                     : launch_once<W, MODE, 1, R, 16>(ctx, w, src, out, parts);
+        };
+        return r == 4 ? rows(std::true_type{}) : rows(std::false_type{});
+    } else if constexpr (MODE == SKN_XSRC_PLAIN) {
+        if (pw == 4) return launch_once<W, MODE, 4, 4, 1>(ctx, w, src, out, parts);
+        if (pw == 2) return launch_once<W, MODE, 2, 4, 1>(ctx, w, src, out, parts);
+        return r == 2   ? launch_once<W, MODE, 1, 2, 1>(ctx, w, src, out, parts)
+               : r == 4 ? launch_once<W, MODE, 1, 4, 1>(ctx, w, src, out, parts)
+                        : launch_once<W, MODE, 1, 8, 1>(ctx, w, src, out, parts);
+    } else {
+        // (a norm group takes whole requests of a lane)
+        if (src.groups > kOnceGroups || (src.groups > 1 && (MODE == SKN_XSRC_ADD_NORM || src.k0 / src.groups % V != 0))) return SKN_ERR_TYPE;
+        switch (r) {
+            case 2: return launch_once<W, MODE, 1, 2, 1>(ctx, w, src, out, parts);
+            case 4: return launch_once<W, MODE, 1, 4, 1>(ctx, w, src, out, parts);
+            case 8: return launch_once<W, MODE, 1, 8, 1>(ctx, w, src, out, parts);
+            case 16: return launch_once<W, MODE, 1, 16, 1>(ctx, w, src, out, parts);
+            default: return SKN_ERR_TYPE;
+        }
+    }
+}
+
 constexpr int kMaxLds = 160 * 1024;
 
 constexpr bool stages_norm(int mode) { return mode == SKN_XSRC_GROUP_NORM || mode == SKN_XSRC_ADD_NORM; }
@@ -411,6 +787,11 @@ int launch(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, cons
 
 template <typename W>
 int launch_mode(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, const skn_dense_out& out) {
+    const int rc = src.mode == SKN_XSRC_GROUP_NORM ? try_once<W, SKN_XSRC_GROUP_NORM>(ctx, w, src, out)
+                   : src.mode == SKN_XSRC_ADD_NORM ? try_once<W, SKN_XSRC_ADD_NORM>(ctx, w, src, out)
+                   : src.mode == SKN_XSRC_MERGE    ? try_once<W, SKN_XSRC_MERGE>(ctx, w, src, out)
+                                                   : try_once<W, SKN_XSRC_PLAIN>(ctx, w, src, out);
+    if (rc != SKN_ERR_TYPE) return rc;
     if (src.mode == SKN_XSRC_GROUP_NORM) return launch<W, SKN_XSRC_GROUP_NORM>(ctx, w, src, out);
     if (src.mode == SKN_XSRC_ADD_NORM) return launch<W, SKN_XSRC_ADD_NORM>(ctx, w, src, out);
     if (src.mode == SKN_XSRC_MERGE) return launch<W, SKN_XSRC_MERGE>(ctx, w, src, out);
