@@ -38,8 +38,9 @@ __device__ __forceinline__ float dot8(const u32x4& k, const float (&qf)[8]) {
 template <int D, bool POW2>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
     const uint16_t* __restrict__ k_pool, const uint16_t* __restrict__ v_pool, const int32_t* __restrict__ table,
-    const int32_t* __restrict__ nctx, const float* __restrict__ q, float* partial, int* counters, float* __restrict__ out,
-    int n_head, int kv_heads, int page_tokens, int page_shift, int pages_per_seq, int n_splits, float scale, int seq_fixed) {
+    const int32_t* __restrict__ nctx, const float* __restrict__ q, int n_head, int kv_heads, int page_shift, int pages_per_seq,
+    int n_splits, int seq_fixed, int page_tokens, float scale, float* partial, int* counters, float* __restrict__ out) {
+    // (up to seq_fixed the arguments are in scalar registers from the start, and nothing else is needed before the first keys)
     constexpr int LPT = D / 8;                        // lanes per token
     constexpr int G = 64 / LPT;                       // token groups (streams) per wavefront
     constexpr int NS = (kAttnThreads / 64) * G;       // streams per workgroup
@@ -233,9 +234,9 @@ constexpr int kWideThreads = 1024;
 template <int D, bool POW2>
 __global__ __launch_bounds__(kWideThreads) void attn_decode_wide_kernel(
     const uint16_t* __restrict__ k_pool, const uint16_t* __restrict__ v_pool, const int32_t* __restrict__ table,
-    const int32_t* __restrict__ nctx, const float* __restrict__ q, float* __restrict__ opart, float* __restrict__ ml,
-    float* __restrict__ out, int n_head, int kv_heads, int page_tokens, int page_shift, int pages_per_seq, int n_splits,
-    float scale, int seq_fixed) {
+    const int32_t* __restrict__ nctx, const float* __restrict__ q, int n_head, int kv_heads, int page_shift, int pages_per_seq,
+    int n_splits, int seq_fixed, int page_tokens, float scale, float* __restrict__ opart, float* __restrict__ ml,
+    float* __restrict__ out) {
     constexpr int LPT = D / 8, G = 64 / LPT, W = kWideThreads / 64, NS = W * G, U = kUnroll;
     __shared__ float so[W][D];
     __shared__ float sm[W], sl[W];
@@ -390,12 +391,12 @@ int skn_attn_launch_ex(skn_ctx* ctx, skn_kv* kv, const float* q_dev, const int32
     do {                                                                                                           \
         if (page_shift >= 0)                                                                                       \
             skn_launch(ctx, attn_decode_kernel<DD, true>, grid, block, 0, kv->k_pool, kv->v_pool,                  \
-                       kv->page_table_dev, nctx_dev, q_dev, partial, counters, out_dev, n_q_head, kv->n_head,      \
-                       kv->page_tokens, page_shift, kv->pages_per_seq, n_splits, scale, seq_fixed);                \
+                       kv->page_table_dev, nctx_dev, q_dev, n_q_head, kv->n_head, page_shift, kv->pages_per_seq,   \
+                       n_splits, seq_fixed, kv->page_tokens, scale, partial, counters, out_dev);                   \
         else                                                                                                       \
             skn_launch(ctx, attn_decode_kernel<DD, false>, grid, block, 0, kv->k_pool, kv->v_pool,                 \
-                       kv->page_table_dev, nctx_dev, q_dev, partial, counters, out_dev, n_q_head, kv->n_head,      \
-                       kv->page_tokens, page_shift, kv->pages_per_seq, n_splits, scale, seq_fixed);                \
+                       kv->page_table_dev, nctx_dev, q_dev, n_q_head, kv->n_head, page_shift, kv->pages_per_seq,   \
+                       n_splits, seq_fixed, kv->page_tokens, scale, partial, counters, out_dev);                   \
     } while (0)
     if (D == 64) SKN_ATTN_LAUNCH(64);
     else if (D == 128) SKN_ATTN_LAUNCH(128);
@@ -423,12 +424,12 @@ int skn_attn_launch_unmerged(skn_ctx* ctx, skn_kv* kv, const float* q_dev, const
     do {                                                                                                               \
         if (page_shift >= 0)                                                                                           \
             skn_launch(ctx, attn_decode_wide_kernel<DD, true>, grid, block, 0, kv->k_pool, kv->v_pool, kv->page_table_dev, \
-                       nctx_dev, q_dev, opart, ml, out_dev, n_q_head, kv->n_head, kv->page_tokens, page_shift,         \
-                       kv->pages_per_seq, n_splits, scale, seq_fixed);                                                 \
+                       nctx_dev, q_dev, n_q_head, kv->n_head, page_shift, kv->pages_per_seq, n_splits, seq_fixed,      \
+                       kv->page_tokens, scale, opart, ml, out_dev);                                                    \
         else                                                                                                           \
             skn_launch(ctx, attn_decode_wide_kernel<DD, false>, grid, block, 0, kv->k_pool, kv->v_pool, kv->page_table_dev, \
-                       nctx_dev, q_dev, opart, ml, out_dev, n_q_head, kv->n_head, kv->page_tokens, page_shift,         \
-                       kv->pages_per_seq, n_splits, scale, seq_fixed);                                                 \
+                       nctx_dev, q_dev, n_q_head, kv->n_head, page_shift, kv->pages_per_seq, n_splits, seq_fixed,      \
+                       kv->page_tokens, scale, opart, ml, out_dev);                                                    \
     } while (0)
     if (D == 64) SKN_ATTN_WIDE(64);
     else if (D == 128) SKN_ATTN_WIDE(128);

@@ -1469,8 +1469,11 @@ __device__ __forceinline__ float4 q4k_merge_splits(const float4* __restrict__ pa
 // residual stream, or applies SwiGLU to a (gate, up) row pair.  Two rows per wavefront, or one where rows are added into few
 // outputs (see dispatch_q4k_fused).  F: the format of all the matrices, as in matvec_q4k_kernel; block: the workgroup's place
 // among those that share the matrices.
+// w0, w1, rows0 and pos_dev are fields of the structs, passed apart: what a workgroup's first requests need stands ahead of the structs among a
+// kernel's arguments, where the first sixteen dwords arrive in scalar registers (the build's -amdgpu-kernarg-preload-count).
 template <int STEPS, int EPI, bool NORM, int F, int R, bool HALF = false>
-__device__ __forceinline__ void q4k_fused_block(const skn_q4k_segments& seg, const float* __restrict__ x, const float* __restrict__ norm_w, float eps,
+__device__ __forceinline__ void q4k_fused_block(const uint8_t* __restrict__ w0, const uint8_t* __restrict__ w1, int rows0, const int32_t* __restrict__ pos_dev,
+                                                const skn_q4k_segments& seg, const float* __restrict__ x, const float* __restrict__ norm_w, float eps,
                                                 float* __restrict__ y, int n_out, int nb, const skn_rope_epilogue& rope, int block) {
     static_assert(R == 2 || EPI == SKN_EPI_ADD, "row pairs");
     static_assert(!HALF || (STEPS == 1 && R == 2), "rows of half a step");
@@ -1500,7 +1503,7 @@ __device__ __forceinline__ void q4k_fused_block(const skn_q4k_segments& seg, con
     int rope_pos = 0, rope_page = 0;
     double rope_freq = 0.0;  // (the pair's frequency out of the model's table, requested with the position)
     if (EPI == SKN_EPI_ROPE) {
-        rope_pos = rope.pos_dev[0];
+        rope_pos = pos_dev[0];
         if (rope.inv_freq)
             rope_freq = rope.inv_freq[q4k_rope_elem(seg, rope, min(block * 8 + (int)(threadIdx.x >> 6), (n_out + 1) / 2 - 1)) >> 1];
     }
@@ -1537,18 +1540,18 @@ __device__ __forceinline__ void q4k_fused_block(const skn_q4k_segments& seg, con
     if (EPI == SKN_EPI_SWIGLU) {
         const int i = min(unit, n_out - 1);
         row_ok[0] = row_ok[1] = unit < n_out;
-        rowp[0] = seg.w[0] + (size_t)i * row_bytes;
-        rowp[1] = seg.w[1] + (size_t)i * row_bytes;
+        rowp[0] = w0 + (size_t)i * row_bytes;
+        rowp[1] = w1 + (size_t)i * row_bytes;
     } else {
 #pragma unroll
         for (int r = 0; r < R; r++) {
             int row = unit * R + r;
             row_ok[r] = row < n_out;
             row = min(row, n_out - 1);
-            const uint8_t* base = seg.w[0];
-            if (row >= seg.rows[0]) {
-                row -= seg.rows[0];
-                base = seg.w[1];
+            const uint8_t* base = w0;
+            if (row >= rows0) {
+                row -= rows0;
+                base = w1;
                 if (row >= seg.rows[1]) {
                     row -= seg.rows[1];
                     base = seg.w[2];
@@ -1700,20 +1703,24 @@ __device__ __forceinline__ void q4k_fused_block(const skn_q4k_segments& seg, con
 }
 
 template <int STEPS, int EPI, bool NORM, int F = kFmtQ4K, int R = 2, bool HALF = false>
-__global__ __launch_bounds__(512) void matvec_q4k_fused_kernel(skn_q4k_segments seg, const float* __restrict__ x,
-                                                               const float* __restrict__ norm_w, float eps,
-                                                               float* __restrict__ y, int n_out, int nb,
-                                                               skn_rope_epilogue rope) {
-    q4k_fused_block<STEPS, EPI, NORM, F, R, HALF>(seg, x, norm_w, eps, y, n_out, nb, rope, (int)blockIdx.x);
+__global__ __launch_bounds__(512) void matvec_q4k_fused_kernel(const uint8_t* __restrict__ w0, const uint8_t* __restrict__ w1, const float* __restrict__ x,
+                                                               const float* __restrict__ norm_w, float* __restrict__ y,
+                                                               const int32_t* __restrict__ pos_dev, int n_out, int nb, int rows0, float eps,
+                                                               skn_q4k_segments seg, skn_rope_epilogue rope) {
+    q4k_fused_block<STEPS, EPI, NORM, F, R, HALF>(w0, w1, rows0, pos_dev, seg, x, norm_w, eps, y, n_out, nb, rope, (int)blockIdx.x);
 }
 
 // q, k and v in two formats (mixed files give the values more bits): the workgroups of both in one launch, the larger blocks first.
 template <int STEPS, int FA, int FB, bool HALF = false>
-__global__ __launch_bounds__(512) void matvec_fused_two_formats_kernel(skn_q4k_segments sa, skn_q4k_segments sb, const float* __restrict__ x,
-                                                                      const float* __restrict__ norm_w, float eps, float* __restrict__ y,
-                                                                      int n_a, int n_b, int blocks_a, int nb, skn_rope_epilogue rope) {
-    if ((int)blockIdx.x < blocks_a) q4k_fused_block<STEPS, SKN_EPI_ROPE, true, FA, 2, HALF>(sa, x, norm_w, eps, y, n_a, nb, rope, (int)blockIdx.x);
-    else q4k_fused_block<STEPS, SKN_EPI_ROPE, true, FB, 2, HALF>(sb, x, norm_w, eps, y, n_b, nb, rope, (int)blockIdx.x - blocks_a);
+__global__ __launch_bounds__(512) void matvec_fused_two_formats_kernel(const uint8_t* __restrict__ wa, const uint8_t* __restrict__ wb,
+                                                                      const float* __restrict__ x, const float* __restrict__ norm_w,
+                                                                      const int32_t* __restrict__ pos_dev, int blocks_a, int nb, int n_a, int n_b,
+                                                                      int rows_a, int rows_b, skn_q4k_segments sa, skn_q4k_segments sb, float eps,
+                                                                      float* __restrict__ y, skn_rope_epilogue rope) {
+    if ((int)blockIdx.x < blocks_a) q4k_fused_block<STEPS, SKN_EPI_ROPE, true, FA, 2, HALF>(wa, sa.w[1], rows_a, pos_dev, sa, x, norm_w, eps, y, n_a, nb, rope, (int)blockIdx.x);
+    else
+        q4k_fused_block<STEPS, SKN_EPI_ROPE, true, FB, 2, HALF>(wb, sb.w[1], rows_b, pos_dev, sb, x, norm_w, eps, y, n_b, nb, rope,
+                                                               (int)blockIdx.x - blocks_a);
 }
 
 template <int F>
@@ -1733,8 +1740,8 @@ int launch_fused_beside_q6k(skn_ctx* ctx, const skn_q4k_segments& q6, int n_q6, 
     auto kernel = matvec_fused_two_formats_kernel<STEPS, kFmtQ6K, F>;
     if constexpr (STEPS == 1)
         if (nb <= kHalfStep) kernel = matvec_fused_two_formats_kernel<1, kFmtQ6K, F, true>;
-    skn_launch(ctx, kernel, dim3((unsigned)blocks), dim3(512), fused_lds_bytes<kFmtQ6K>(STEPS), q6, other, x, norm_w, eps, y, n_q6, n_other, blocks_q6, nb,
-               rope);
+    skn_launch(ctx, kernel, dim3((unsigned)blocks), dim3(512), fused_lds_bytes<kFmtQ6K>(STEPS), q6.w[0], other.w[0], x, norm_w, rope.pos_dev, blocks_q6, nb, n_q6,
+               n_other, q6.rows[0], other.rows[0], q6, other, eps, y, rope);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
@@ -1748,7 +1755,7 @@ int launch_q4k_fused(skn_ctx* ctx, const skn_q4k_segments& seg, int n_out, int n
     auto kernel = matvec_q4k_fused_kernel<STEPS, EPI, NORM, F, R>;
     if constexpr (STEPS == 1 && R == 2 && NORM && (EPI == SKN_EPI_ROPE || EPI == SKN_EPI_SWIGLU))
         if (nb <= kHalfStep) kernel = matvec_q4k_fused_kernel<1, EPI, true, F, 2, true>;
-    skn_launch(ctx, kernel, grid, block, lds, seg, x, norm_w, eps, y, n_out, nb, rope);
+    skn_launch(ctx, kernel, grid, block, lds, seg.w[0], seg.w[1], x, norm_w, y, rope.pos_dev, n_out, nb, seg.rows[0], eps, seg, rope);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
