@@ -401,77 +401,159 @@ struct StepArgs {
     float* state;
 };
 
-// row . t over rank_pad columns (zeros of the row from its rank on), shared by eight lanes; the total in all of them
+// Eight lanes share a row of the low-rank products: lane l has the pieces of eight columns 8 l, 64 + 8 l, ..
 template <typename W>
-__device__ __forceinline__ float low_rank_dot(const W* row, const float* t, int rank_pad, int l) {
-    float z = 0.f;
-#pragma unroll 2
-    for (int i = 8 * l; i < rank_pad; i += 64) {
-        float f[8];
-        const float4 a = *reinterpret_cast<const float4*>(t + i), b = *reinterpret_cast<const float4*>(t + i + 4);
-        if constexpr (sizeof(W) == 2) {
-            const uint4 w = *reinterpret_cast<const uint4*>(row + i);
-            const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+struct Piece8;
+template <>
+struct Piece8<uint16_t> {
+    uint4 w;
+    __device__ __forceinline__ void load(const uint16_t* p) { w = *reinterpret_cast<const uint4*>(p); }
+    __device__ __forceinline__ void get(float (&f)[8]) const {
+        const uint32_t u[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-            for (int j = 0; j < 4; j++) f[2 * j] = __uint_as_float(u[j] << 16), f[2 * j + 1] = __uint_as_float(u[j] & 0xFFFF0000u);
-        } else {
-            const float4 c = *reinterpret_cast<const float4*>(row + i), d = *reinterpret_cast<const float4*>(row + i + 4);
-            f[0] = c.x, f[1] = c.y, f[2] = c.z, f[3] = c.w, f[4] = d.x, f[5] = d.y, f[6] = d.z, f[7] = d.w;
-        }
-        z += ((f[0] * a.x + f[1] * a.y) + (f[2] * a.z + f[3] * a.w)) + ((f[4] * b.x + f[5] * b.y) + (f[6] * b.z + f[7] * b.w));
+        for (int j = 0; j < 4; j++) f[2 * j] = __uint_as_float(u[j] << 16), f[2 * j + 1] = __uint_as_float(u[j] & 0xFFFF0000u);
     }
-    return lane_group_sum<8>(z);
+};
+template <>
+struct Piece8<float> {
+    float4 c, d;
+    __device__ __forceinline__ void load(const float* p) { c = *reinterpret_cast<const float4*>(p), d = *reinterpret_cast<const float4*>(p + 4); }
+    __device__ __forceinline__ void get(float (&f)[8]) const { f[0] = c.x, f[1] = c.y, f[2] = c.z, f[3] = c.w, f[4] = d.x, f[5] = d.y, f[6] = d.z, f[7] = d.w; }
+};
+
+template <typename W>
+__device__ __forceinline__ float piece_dot(const Piece8<W>& row, const Vec8& t) {
+    float f[8];
+    row.get(f);
+    const float* a = t.v;
+    return ((f[0] * a[0] + f[1] * a[1]) + (f[2] * a[2] + f[3] * a[3])) + ((f[4] * a[4] + f[5] * a[5]) + (f[6] * a[6] + f[7] * a[7]));
 }
 
-// one workgroup of NW wavefronts per head
+// The first N pieces of a row of the low-rank products (two: ranks up to 128) and of the vector, requested ahead.
+template <typename W, int N>
+struct LowRank {
+    Piece8<W> w[N];
+    Vec8 t[N];
+    __device__ __forceinline__ void load(const W* row, const float* x, int rank_pad, int l) {
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            if (64 * i < rank_pad) w[i].load(row + 64 * i + 8 * l), t[i].load(x + 64 * i + 8 * l);
+    }
+    // row . x over rank_pad columns (zeros of the row from its rank on); the total in all eight lanes
+    __device__ __forceinline__ float dot(const W* row, const float* x, int rank_pad, int l) const {
+        float z = piece_dot(w[0], t[0]);
+#pragma unroll
+        for (int i = 1; i < N; i++)
+            if (64 * i < rank_pad) z += piece_dot(w[i], t[i]);
+        for (int i = 64 * N + 8 * l; i < rank_pad; i += 64) {
+            Piece8<W> p;
+            Vec8 v;
+            p.load(row + i), v.load(x + i);
+            z += piece_dot(p, v);
+        }
+        return lane_group_sum<8>(z);
+    }
+};
+
+// what a channel's convolution reads: the inputs j tokens back and their taps
+struct ConvPoint {
+    float x[kMaxTaps], w[kMaxTaps];
+    int which, d, c;
+};
+
+// One workgroup of NW wavefronts per head.  It is a chain of latencies on few workgroups (a megabyte of state is 64 KB for each of
+// sixteen): everything that it reads is requested before the first value is waited for -- the state, rows of both low-rank products, their
+// vectors, biases, taps and the convolutions' inputs -- and two barriers are met instead of three.  Sixteen heads of 128 x 128
+// behind four taps and ranks of 128: 11.9 us when one loop's requests followed the other's sums, 8.7 now.
+// (Up to vdim the arguments arrive in scalar registers.)
 template <int L, int NW, typename W>
-__global__ __launch_bounds__(64 * NW) void gated_step_kernel(const StepArgs a) {
-    constexpr int DP = 8 * L, CW = 64 / L, kThreads = 64 * NW, kCols = NW * CW, kPasses = 256 / kCols;  // columns per wavefront, per pass
+__global__ __launch_bounds__(64 * NW) void gated_step_kernel(float* __restrict__ states, const int32_t* __restrict__ step, const W* __restrict__ w_a,
+                                                             const float* __restrict__ a_low, const W* __restrict__ w_g, const float* __restrict__ g_low,
+                                                             int rank_a_pad, int rank_g_pad, int dim, int vdim, const StepArgs a) {
+    constexpr int DP = 8 * L, CW = 64 / L, kThreads = 64 * NW, kCols = NW * CW, kPasses = 256 / kCols, kGroups = kThreads / 8;  // columns per wavefront, per pass
+    static_assert(kThreads >= 256, "a thread for every value channel");
     __shared__ __align__(16) float vec[3][DP];  // q, k, factors
-    __shared__ float sv[256], sg[256], so[256], red[NW];
+    __shared__ float sv[256], sg[256], so[256];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = blockIdx.x, rl = lane & (L - 1), per_kv = a.heads / a.kv_heads, kvh = h / per_kv;
-    const int dim = a.dim, vdim = a.vdim, qk = a.kv_heads * dim;
+    const int qk = a.kv_heads * dim, n_taps = a.n_taps, l = tid & 7, r0 = tid >> 3;
     const skn_gated_step& p = a.p;
+    const int pos = step[1];
     // the state first: it does not wait for anything
     Vec8 s[kPasses];
-    float* sp = a.state + ((int64_t)h * vdim) * DP + 8 * rl;
+    float* sp = states + ((int64_t)h * vdim) * DP + 8 * rl;
 #pragma unroll
     for (int i = 0; i < kPasses; i++)
         if (i * kCols < vdim) s[i].load(sp + (int64_t)min(i * kCols + wave * CW + lane / L, vdim - 1) * DP);
-    const int pos = p.state[1];
-    const float beta = p.beta[h];
-    // factors of the key channels and gates of the value channels: eight lanes per row of the second matrices
-    for (int r = tid >> 3; r < DP + vdim; r += kThreads / 8) {
-        const int d = r - DP, l = tid & 7;
-        if (r < DP) {
-            const float z = low_rank_dot((const W*)p.w_a + (int64_t)(h * dim + min(r, dim - 1)) * p.rank_a_pad, p.a_low, p.rank_a_pad, l);
-            if (l == 0) vec[2][r] = r < dim ? __builtin_amdgcn_exp2f(log2_factor(z + p.bias_a[h * dim + r], a.rate[h])) : 0.f;
-        } else {
-            const float z = low_rank_dot((const W*)p.w_g + (int64_t)(h * vdim + d) * p.rank_g_pad, p.g_low, p.rank_g_pad, l);
-            if (l == 0) sg[d] = skn_sigmoid(z);
-        }
-    }
+    // the first rows of factors and of gates that this group of eight lanes has (DP and vdim may hold more than one turn)
+    const auto row_a = [&](int r) { return w_a + (int64_t)(h * dim + min(r, dim - 1)) * rank_a_pad; };
+    const auto row_g = [&](int d) { return w_g + (int64_t)(h * vdim + min(d, vdim - 1)) * rank_g_pad; };
+    // (what the registers of sixteen wavefronts hold beside the state: not all of it for 32-bit weights or 256 channels)
+    constexpr bool kAheadA = L <= 16, kAheadG = L < 16 || (L == 16 && sizeof(W) == 2);
+    LowRank<W, kAheadG ? 2 : 1> fa, fg;
+    if (kAheadA) fa.load(row_a(r0), a_low, rank_a_pad, l);
+    if (kAheadG) fg.load(row_g(r0), g_low, rank_g_pad, l);
+    const float bias0 = p.bias_a[h * dim + min(r0, dim - 1)], norm = p.norm[h * vdim + min(tid, vdim - 1)];
+    const float beta = p.beta[h], rate = a.rate[h];
     // convolutions: channels q, k of the head's q/k head, then v
-    for (int i = tid; i < 2 * DP + vdim; i += kThreads) {
-        const int which = i < DP ? 0 : i < 2 * DP ? 1 : 2, d = i - which * DP;
-        if (which < 2 && d >= dim) {
-            vec[which][d] = 0.f;
-            continue;
+    const int slot = pos % n_taps;
+    const auto conv_load = [&](ConvPoint& v, int i) __attribute__((always_inline)) {
+        v.which = i < DP ? 0 : i < 2 * DP ? 1 : 2, v.d = i - v.which * DP;
+        const int d = min(v.d, (v.which < 2 ? dim : vdim) - 1);  // (past the end: a valid channel, unused)
+        v.c = v.which < 2 ? v.which * qk + kvh * dim + d : 2 * qk + h * vdim + d;
+        v.x[0] = (v.which == 0 ? p.q + kvh * dim : v.which == 1 ? p.k + kvh * dim : p.v + h * vdim)[d];
+        const float* w = a.taps + (int64_t)v.c * n_taps;
+        v.w[0] = w[n_taps - 1];
+#pragma unroll
+        for (int j = 1; j < kMaxTaps; j++) {
+            if (j >= n_taps || j > pos) break;
+            const int at = slot - j < 0 ? slot - j + n_taps : slot - j;
+            v.x[j] = a.ring[(int64_t)at * a.channels + v.c];
+            v.w[j] = w[n_taps - 1 - j];
         }
-        const int c = which < 2 ? which * qk + kvh * dim + d : 2 * qk + h * vdim + d;
-        const float x = (which == 0 ? p.q + kvh * dim : which == 1 ? p.k + kvh * dim : p.v + h * vdim)[d];
-        const float* w = a.taps + (int64_t)c * a.n_taps;
-        float y = x * w[a.n_taps - 1];
-        for (int j = 1; j < a.n_taps; j++) {
-            const int at = pos - j;
-            if (at >= 0) y = fmaf(a.ring[(int64_t)(at % a.n_taps) * a.channels + c], w[a.n_taps - 1 - j], y);
+    };
+    const auto conv_finish = [&](const ConvPoint& v) __attribute__((always_inline)) {
+        if (v.which < 2 && v.d >= dim) {
+            vec[v.which][v.d] = 0.f;
+            return;
+        }
+        float y = v.x[0] * v.w[0];
+#pragma unroll
+        for (int j = 1; j < kMaxTaps; j++) {
+            if (j >= n_taps || j > pos) break;
+            y = fmaf(v.x[j], v.w[j], y);
         }
         // (this token's slot is none of those that are read; the heads that share a q/k head leave it to the first)
-        if (which == 2 || h % per_kv == 0) a.ring[(int64_t)(pos % a.n_taps) * a.channels + c] = x;
-        if (which < 2) vec[which][d] = silu(y);
-        else sv[d] = silu(y);
+        if (v.which == 2 || h % per_kv == 0) a.ring[(int64_t)slot * a.channels + v.c] = v.x[0];
+        if (v.which < 2) vec[v.which][v.d] = silu(y);
+        else sv[v.d] = silu(y);
+    };
+    const int points = 2 * DP + vdim;
+    {
+        ConvPoint first;
+        if (kAheadA && tid < points) conv_load(first, tid);
+        const auto factor = [&](int r, float z, float b) {
+            if (l == 0) vec[2][r] = r < dim ? __builtin_amdgcn_exp2f(log2_factor(z + b, rate)) : 0.f;
+        };
+        if (!kAheadA) fa.load(row_a(r0), a_low, rank_a_pad, l);
+        if (r0 < DP) factor(r0, fa.dot(row_a(r0), a_low, rank_a_pad, l), bias0);
+        for (int r = r0 + kGroups; r < DP; r += kGroups) {
+            fa.load(row_a(r), a_low, rank_a_pad, l);
+            factor(r, fa.dot(row_a(r), a_low, rank_a_pad, l), p.bias_a[h * dim + min(r, dim - 1)]);
+        }
+        for (int d = r0; d < vdim; d += kGroups) {
+            if (!kAheadG || d != r0) fg.load(row_g(d), g_low, rank_g_pad, l);
+            const float z = fg.dot(row_g(d), g_low, rank_g_pad, l);
+            if (l == 0) sg[d] = skn_sigmoid(z);
+        }
+        if (!kAheadA && tid < points) conv_load(first, tid);
+        if (tid < points) conv_finish(first);
     }
-    __syncthreads();
+    for (int i = tid + kThreads; i < points; i += kThreads) {
+        ConvPoint more;
+        conv_load(more, i);
+        conv_finish(more);
+    }
+    lds_barrier();
     float sq = 0.f, sk = 0.f;  // (every wavefront for itself)
     for (int d = lane; d < DP; d += 64) sq = fmaf(vec[0][d], vec[0][d], sq), sk = fmaf(vec[1][d], vec[1][d], sk);
     const float fq = 1.0f / (sqrtf(wave_sum(sq) + kUnitEps) * sqrtf((float)dim)), fk = 1.0f / sqrtf(wave_sum(sk) + kUnitEps);
@@ -496,17 +578,16 @@ __global__ __launch_bounds__(64 * NW) void gated_step_kernel(const StepArgs a) {
             if (rl == 0) so[col] = o;
         }
     }
-    __syncthreads();
-    float ss = 0.f;
-    for (int d = tid; d < vdim; d += kThreads) ss = fmaf(so[d], so[d], ss);
-    ss = wave_sum(ss);
-    if (lane == 0) red[wave] = ss;
-    __syncthreads();
-    ss = 0.f;
+    lds_barrier();
+    if (wave * 64 >= vdim) return;
+    float ss = 0.f;  // (every wavefront for itself, sixty-four channels at a time)
 #pragma unroll
-    for (int i = 0; i < NW; i++) ss += red[i];
+    for (int i = 0; i < 4; i++) {
+        const float o = 64 * i + lane < vdim ? so[64 * i + lane] : 0.f;
+        if (64 * i < vdim) ss += wave_sum(o * o);
+    }
     const float inv = 1.0f / sqrtf(ss / (float)vdim + p.eps);
-    for (int d = tid; d < vdim; d += kThreads) p.y[h * vdim + d] = so[d] * inv * p.norm[h * vdim + d] * sg[d];
+    if (tid < vdim) p.y[h * vdim + tid] = so[tid] * inv * norm * sg[tid];
 }
 
 template <int DP>
@@ -523,8 +604,14 @@ int launch_rows(skn_ctx* ctx, const skn_rstate* st, const ChunkArgs& a, float* s
 
 template <int L, int NW>
 int launch_step(skn_ctx* ctx, const StepArgs& a) {
-    if (a.p.w_type == SKN_TYPE_F32) skn_launch(ctx, gated_step_kernel<L, NW, float>, dim3(a.heads), dim3(64 * NW), 0, a);
-    else skn_launch(ctx, gated_step_kernel<L, NW, uint16_t>, dim3(a.heads), dim3(64 * NW), 0, a);
+    const skn_gated_step& p = a.p;
+    const dim3 grid(a.heads), block(64 * NW);
+    if (p.w_type == SKN_TYPE_F32)
+        skn_launch(ctx, gated_step_kernel<L, NW, float>, grid, block, 0, a.state, p.state, (const float*)p.w_a, p.a_low, (const float*)p.w_g, p.g_low, p.rank_a_pad,
+                   p.rank_g_pad, a.dim, a.vdim, a);
+    else
+        skn_launch(ctx, gated_step_kernel<L, NW, uint16_t>, grid, block, 0, a.state, p.state, (const uint16_t*)p.w_a, p.a_low, (const uint16_t*)p.w_g, p.g_low,
+                   p.rank_a_pad, p.rank_g_pad, a.dim, a.vdim, a);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
