@@ -93,13 +93,13 @@ __device__ __forceinline__ void shared_attn_block(const AttnArgs& p, const int s
     // what does not wait for the position is requested first: the token's projections, whose norms are computed while the
     // first cached rows are on their way
     float4 q4, k4;
-    float q_elem = 0.f;
+    float q_elem = 0.f, q_weight = 0.f, k_weight = 0.f;
     if constexpr (STEP) {
         static_assert(QG * D <= kThreads, "one element of the group's queries per thread");
         q4 = first_quad(p.q, p.n_head * p.dim);
         k4 = first_quad(p.k, p.kv_heads * p.dim);
         const int i = tid / D, d = tid - i * D, h = min(h0 + i, h_end - 1);
-        if (tid < QG * D && d < p.dim) q_elem = p.q[h * p.dim + d] * p.q_norm[h * p.dim + d] * p.k_norm[kvh * p.dim + d];
+        if (tid < QG * D && d < p.dim) q_elem = p.q[h * p.dim + d], q_weight = p.q_norm[h * p.dim + d], k_weight = p.k_norm[kvh * p.dim + d];
     }
     const int n = STEP ? p.state[2] : p.first_ctx + row;
     const int per = ((n + p.n_splits - 1) / p.n_splits + NS - 1) / NS * NS;
@@ -116,7 +116,7 @@ __device__ __forceinline__ void shared_attn_block(const AttnArgs& p, const int s
             const int t = max(min(base + u * NS + stream, t_end - 1), 0);  // past the end: a valid row, masked below
             const int pi = (int)(((float)t + 0.5f) * p.inv_page), slot = t - pi * p.page_tokens;  // (exact below 2^22 tokens)
             int page = __shfl(my_page, pi & 63, 64);
-            if (pi >= 64) page = p.table[pi];
+            if (pi >= 64) page = far_page(p.table, pi);
             rows[u].load(pool + (((int64_t)page * p.kv_heads + kvh) * p.page_tokens + slot) * D + c * 8);
             cs[u] = p.key_scale[(int64_t)page * p.page_tokens + slot];
         }
@@ -125,7 +125,7 @@ __device__ __forceinline__ void shared_attn_block(const AttnArgs& p, const int s
 
     float qf[QG][8], fq = p.scale_log2e, newest_scale = 0.f;
     if constexpr (STEP) {
-        if (tid < QG * D) qs[tid] = q_elem;  // (the barrier of the sums covers it)
+        if (tid < QG * D) qs[tid] = q_elem * q_weight * k_weight;  // (the barrier of the sums covers it)
         float sq = sum_squares(q4, p.q, p.n_head * p.dim), sk = sum_squares(k4, p.k, p.kv_heads * p.dim);
         block_sum2(sq, sk, red);
         newest_scale = 1.0f / sqrtf(sk / (float)(p.kv_heads * p.dim) + p.eps);
@@ -201,12 +201,14 @@ __device__ __forceinline__ void shared_attn_block(const AttnArgs& p, const int s
                 for (int j = 0; j < 8; j++) o[i][j] = fmaf(pr[i][u], vf[j], o[i][j]);
         }
     };
-    for (int base = t_begin; base < t_end; base += NS * U) {
+    int base = t_begin;
+    for (; base + NS * U < t_end; base += NS * U) {
         fetch(nxt, cs_nxt, base + NS * U);
         absorb(cur, cs_cur, base);
 #pragma unroll
         for (int u = 0; u < U; u++) cur[u] = nxt[u], cs_cur[u] = cs_nxt[u];
     }
+    if (base < t_end) absorb(cur, cs_cur, base);
 
     // the G streams of the wavefront (lanes with the same c hold the same elements), then the wavefronts through LDS
 #pragma unroll
