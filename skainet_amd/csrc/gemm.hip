@@ -772,7 +772,11 @@ constexpr int kTlLds = 3 * kTlStage + 2 * kTlAux + 128 * 4 + 256 * 4;
 // consumer's column blocks 0, 1 and 2, 3 meet lane by lane in the store -- and stores silu(gate) * up in bf16.
 // TAIL: the last tiles are shared by tail.splits workgroups each, neighbours in the grid, with a part of k each (a template
 // parameter: grids without such tiles were 0.5 us slower at 512 x 14336 x 4096 for the division).
-template <bool TAIL>
+// CB: column blocks of 32 in a tile.  Three (256 x 96) where they make one round of compute units that four leave a quarter and more of
+// idle (a loop of 96 columns takes 0.83 of the time of one of 128, bound by the same phases: q, k and v of 512 x 4096 in 12288 columns 73.2 -> 60.8
+// us, 704 -> 848 TFLOP/s; 2000 x 2048 in 3072 41.3 -> 35.9); tile0 and n_tiles count blocks of 32 there, so that a tile may hold the end of one matrix and the start of the next, and the
+// fourth producer only keeps the barriers.
+template <bool TAIL, int CB>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restrict__ sfrag, const Q4kFragSegs segs,
                           const float* __restrict__ inv_scale, int m, int k, int m_tiles, uint32_t a_bytes, const TallTail tail) {
@@ -790,10 +794,14 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
         sb0 = nb * z / parts, sb1 = nb * (z + 1) / parts;
     }
     const int mt = tile % m_tiles, tn = tile / m_tiles;  // (the row tiles of a column tile run side by side)
-    const bool pair = segs.pair != nullptr;
-    const int seg = pair ? 0 : (tn >= segs.tile0[2] ? 2 : (tn >= segs.tile0[1] ? 1 : 0));
+    static_assert(CB == 4 || (CB == 3 && !TAIL), "tiles of 128 columns, or of 96 with k undivided");
+    const bool pair = CB == 4 && segs.pair != nullptr;
+    auto matrix_of = [&](int unit) __attribute__((always_inline)) { return unit >= segs.tile0[2] ? 2 : (unit >= segs.tile0[1] ? 1 : 0); };
+    // (CB 3: of this producer's block of columns; a consumer looks its three up when it stores)
+    const int unit = CB == 4 ? tn : tn * CB + min(me, CB - 1);
+    const int seg = pair ? 0 : matrix_of(unit);
     const int n = segs.n[seg];
-    const int n0 = pair ? tn * 64 : (tn - segs.tile0[seg]) * 128;  // first column of the tile in its matrix (pair: in both)
+    const int n0 = pair ? tn * 64 : CB == 4 ? (tn - segs.tile0[seg]) * 128 : (unit - segs.tile0[seg]) * 32;  // first column of the tile in its matrix (pair: in both)
     float* __restrict__ c = segs.c[seg];
     uint8_t* stage = lds;
     uint8_t* aux = lds + 3 * kTlStage;
@@ -813,11 +821,13 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
         b_cur = b_nxt, b_nxt = b_nx2, b_nx2 = t;
     };
 
-    if (producer) {
+    if (CB < 4 && producer && me >= CB) {
+        for (int i = 2 + 4 * (sb1 - sb0); i > 0; i--) barrier();
+    } else if (producer) {
         const uint8_t* w = segs.w[pair ? me >> 1 : seg];
         const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, n * nb * 144, 0x00020000);  // (checked by the caller to fit)
         const int col = 32 * me + r;  // column of the tile
-        const int wrow = min(n0 + (pair ? 32 * (me & 1) + r : col), n - 1) * nb * 144;
+        const int wrow = min(n0 + (pair ? 32 * (me & 1) + r : CB == 4 ? col : r), n - 1) * nb * 144;
         // One set of registers for the header and the four nibble pieces; each is requested again, for the next
         // superblock, right after it is unpacked: four phases before its next use.
         u32x4 hd, q[4];
@@ -939,7 +949,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
         if (h == 0) *reinterpret_cast<float*>(fin + col * 4) = cs;
         barrier();
     } else {
-        constexpr int MT = 2;
+        constexpr int MT = 2, NT = MT * CB;  // (tile t: row block t / CB, column block t % CB)
         const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc((void*)afrag, 0, (int)a_bytes, 0x00020000);
         const int mb0 = mt * 8 + me * MT;  // first row block of this consumer
         uint32_t abase[MT];
@@ -952,20 +962,22 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
             for (int i = 0; i < MT; i++)
                 a[slot][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, lane * 16, (int)(abase[i] + (uint32_t)step * 1024u), 0));
         };
-        float16_t acc[MT][4];
+        float16_t acc[MT][CB];
 #pragma unroll
         for (int i = 0; i < MT; i++)
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < CB; j++)
 #pragma unroll
                 for (int x = 0; x < 16; x++) acc[i][j][x] = 0.f;
         u32x4 sf[MT];
-        half8_t fb[2][4];  // the weight fragments of a k-step, read while the step before it is multiplied; step 0 of a phase in fb[0]
-        float ratio[4] = {1.f, 1.f, 1.f, 1.f};  // of the superblock being entered, by column block
-        // tile t = 4 i + j changes its unit: half `part` of its sixteen registers
+        half8_t fb[2][CB];  // the weight fragments of a k-step, read while the step before it is multiplied; step 0 of a phase in fb[0]
+        float ratio[CB];  // of the superblock being entered, by column block
+#pragma unroll
+        for (int j = 0; j < CB; j++) ratio[j] = 1.f;
+        // tile t changes its unit: half `part` of its sixteen registers
         auto rescale = [&](int t, int part) __attribute__((always_inline)) {
 #pragma unroll
-            for (int x = 0; x < 8; x++) acc[t >> 2][t & 3][8 * part + x] *= ratio[t & 3];
+            for (int x = 0; x < 8; x++) acc[t / CB][t % CB][8 * part + x] *= ratio[t % CB];
         };
         auto fence = [&]() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
         auto phase = [&](int sb, auto cc_const) __attribute__((always_inline)) {
@@ -978,36 +990,36 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
             }
             const uint8_t* src = stage + b_cur + lane * 16;
             const uint8_t* srcn = stage + b_nxt + lane * 16;
-            half8_t vh[4], vl[4];
-            float rnext[4];
+            half8_t vh[CB], vl[CB];
+            float rnext[CB];
             if (cc == 3) {  // (the ratios of the next superblock, left by the producers a phase ago: used at the end of this phase)
 #pragma unroll
-                for (int j = 0; j < 4; j++) rnext[j] = *reinterpret_cast<const float*>(axn + 128 * 32 + (j * 32 + r) * 4);
+                for (int j = 0; j < CB; j++) rnext[j] = *reinterpret_cast<const float*>(axn + 128 * 32 + (j * 32 + r) * 4);
             }
 #pragma unroll
             for (int s4 = 0; s4 < 4; s4++) {
                 const int step = 4 * cc + s4, slot = step & 7;
                 if (s4 < 3) {
 #pragma unroll
-                    for (int j = 0; j < 4; j++) fb[(s4 + 1) & 1][j] = *reinterpret_cast<const half8_t*>(src + (s4 + 1) * 4096 + j * 1024);
+                    for (int j = 0; j < CB; j++) fb[(s4 + 1) & 1][j] = *reinterpret_cast<const half8_t*>(src + (s4 + 1) * 4096 + j * 1024);
                 } else if (cc < 3) {  // the next phase's first step: complete since the barrier before this phase
 #pragma unroll
-                    for (int j = 0; j < 4; j++) fb[0][j] = *reinterpret_cast<const half8_t*>(srcn + j * 1024);
+                    for (int j = 0; j < CB; j++) fb[0][j] = *reinterpret_cast<const half8_t*>(srcn + j * 1024);
                 } else {
 #pragma unroll
-                    for (int j = 0; j < 4; j++) vh[j] = *reinterpret_cast<const half8_t*>(ax + (j * 32 + r) * 32);
+                    for (int j = 0; j < CB; j++) vh[j] = *reinterpret_cast<const half8_t*>(ax + (j * 32 + r) * 32);
                 }
                 fence();
                 if (cc == 0 && s4 == 0) {
-                    // the superblock's first step: tiles 3 .. 7 change their unit between its matrix instructions
+                    // the superblock's first step: the tiles from 3 on change their unit between its matrix instructions
                     // (tiles 0 .. 2 did before the barrier)
 #pragma unroll
-                    for (int t = 0; t < 8; t++) {
-                        acc[t >> 2][t & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a[slot][t >> 2]), fb[0][t & 3],
-                                                                                    acc[t >> 2][t & 3], 0, 0, 0);
+                    for (int t = 0; t < NT; t++) {
+                        acc[t / CB][t % CB] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a[slot][t / CB]), fb[0][t % CB],
+                                                                                    acc[t / CB][t % CB], 0, 0, 0);
                         fence();
                         if (t < 4) rescale(3 + (t >> 1), t & 1);
-                        if (t >= 4 && t < 7) rescale(t + 1, 0), rescale(t + 1, 1);
+                        if (t >= 4 && t < NT - 1) rescale(t + 1, 0), rescale(t + 1, 1);
                         fence();
                     }
                 } else {
@@ -1015,7 +1027,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                     for (int i = 0; i < MT; i++) {
                         const half8_t fa = __builtin_bit_cast(half8_t, a[slot][i]);
 #pragma unroll
-                        for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa, fb[s4 & 1][j], acc[i][j], 0, 0, 0);
+                        for (int j = 0; j < CB; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa, fb[s4 & 1][j], acc[i][j], 0, 0, 0);
                     }
                 }
                 afetch(16 * sb + step + 7, (step + 7) & 7);
@@ -1025,25 +1037,26 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                 // The "- dmin * m" term of the superblock (the two products of a tile eight instructions apart), and
                 // under it the reads for what follows: the low parts, then the next phase's first step.
 #pragma unroll
-                for (int j = 0; j < 4; j++) vl[j] = *reinterpret_cast<const half8_t*>(ax + (j * 32 + r) * 32 + 16);
+                for (int j = 0; j < CB; j++) vl[j] = *reinterpret_cast<const half8_t*>(ax + (j * 32 + r) * 32 + 16);
                 fence();
 #pragma unroll
                 for (int i = 0; i < MT; i++)
 #pragma unroll
-                    for (int j = 0; j < 4; j++)
+                    for (int j = 0; j < CB; j++)
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, sf[i]), vh[j], acc[i][j], 0, 0, 0);
                 fence();
 #pragma unroll
-                for (int j = 0; j < 4; j++) fb[0][j] = *reinterpret_cast<const half8_t*>(srcn + j * 1024);
+                for (int j = 0; j < CB; j++) fb[0][j] = *reinterpret_cast<const half8_t*>(srcn + j * 1024);
 #pragma unroll
-                for (int j = 0; j < 4; j++) ratio[j] = sb + 1 < sb1 ? rnext[j] : 1.0f;  // (none after the last superblock)
+                for (int j = 0; j < CB; j++) ratio[j] = sb + 1 < sb1 ? rnext[j] : 1.0f;  // (none after the last superblock)
                 fence();
                 // tiles 0 .. 2 change their unit between the last of these instructions
 #pragma unroll
-                for (int t = 0; t < 8; t++) {
-                    acc[t >> 2][t & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, sf[t >> 2]), vl[t & 3], acc[t >> 2][t & 3], 0, 0, 0);
+                for (int t = 0; t < NT; t++) {
+                    acc[t / CB][t % CB] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, sf[t / CB]), vl[t % CB], acc[t / CB][t % CB], 0, 0, 0);
                     fence();
-                    if (t >= 2) rescale((t - 2) >> 1, t & 1);
+                    if (CB == 4 && t >= 2) rescale((t - 2) >> 1, t & 1);
+                    if (CB == 3 && t >= 3) rescale(t - 3, 0), rescale(t - 3, 1);
                     fence();
                 }
             }
@@ -1054,7 +1067,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
         for (int s = 0; s < 7; s++) afetch(16 * sb0 + s, s);
         barrier();
 #pragma unroll
-        for (int j = 0; j < 4; j++) fb[0][j] = *reinterpret_cast<const half8_t*>(stage + b_cur + lane * 16 + j * 1024);
+        for (int j = 0; j < CB; j++) fb[0][j] = *reinterpret_cast<const half8_t*>(stage + b_cur + lane * 16 + j * 1024);
         for (int sb = sb0; sb < sb1; sb++) {
             phase(sb, C0{});
             phase(sb, C1{});
@@ -1062,7 +1075,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
             phase(sb, C3{});
         }
         barrier();
-        if (TAIL && parts > 1) {  // (unscaled, every element of the tile, in the order of the matrix core's registers: see gemm_add_tall_kernel)
+        if constexpr (TAIL) if (parts > 1) {  // (unscaled, every element of the tile, in the order of the matrix core's registers: see gemm_add_tall_kernel)
             float* dst = tail.part + ((size_t)(z * tail.tiles + tile - tail.tile0) * 4 + me) * (MT * 4 * 1024) + lane * 4;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -1081,7 +1094,7 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
             float sc[16];
 #pragma unroll
             for (int x = 0; x < 16; x++) sc[x] = isc_lds[(me * MT + i) * 32 + 8 * (x >> 2) + 4 * h + (x & 3)];
-            if (pair) {
+            if constexpr (CB == 4) if (pair) {
 #pragma unroll
                 for (int jj = 0; jj < 2; jj++) {
                     const float ug = *reinterpret_cast<const float*>(fin + (jj * 32 + r) * 4);
@@ -1099,11 +1112,17 @@ void gemm_q4k_tall_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
                 continue;
             }
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
+            for (int j = 0; j < CB; j++) {
                 const float unit = *reinterpret_cast<const float*>(fin + (j * 32 + r) * 4);
 #pragma unroll
                 for (int x = 0; x < 16; x++) acc[i][j][x] *= unit;
-                store_tile(acc[i][j], c, n, (mb0 + i) * 32, n0 + 32 * j, m, n, sc, lane, segs.accumulate[seg] != 0);
+                if constexpr (CB == 4) {
+                    store_tile(acc[i][j], c, n, (mb0 + i) * 32, n0 + 32 * j, m, n, sc, lane, segs.accumulate[seg] != 0);
+                } else {
+                    const int at = tn * CB + j, s = matrix_of(at);
+                    if (at < segs.n_tiles)
+                        store_tile(acc[i][j], segs.c[s], segs.n[s], (mb0 + i) * 32, (at - segs.tile0[s]) * 32, m, segs.n[s], sc, lane, segs.accumulate[s] != 0);
+                }
             }
         }
     }
@@ -2192,8 +2211,9 @@ static int skn_gemm_init(skn_ctx* ctx) {
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 2, true>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 2>() + 32 * 2 * 2 * 4));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 1, false>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 1>() + 32 * 2 * 1 * 4));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_frag_kernel<2, 1, true>, hipFuncAttributeMaxDynamicSharedMemorySize, frag_lds_bytes<2, 1>() + 32 * 2 * 1 * 4));
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_tall_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, kTlLds));
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_tall_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, kTlLds));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_tall_kernel<false, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, kTlLds));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_tall_kernel<true, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, kTlLds));
+    SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_q4k_tall_kernel<false, 3>, hipFuncAttributeMaxDynamicSharedMemorySize, kTlLds));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_hilo_frag_kernel<1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 1 * 3 * 4096));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_hilo_frag_kernel<2, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 2 * 3 * 4096));
     SKN_HIP(ctx, hipFuncSetAttribute((const void*)gemm_hilo_frag_kernel<4, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 4 * 3 * 4096));
@@ -2263,21 +2283,25 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     const int n_tiles_all = fs.n_tiles;
     // 256 x 128 tiles (the kernel that unpacks the weights once per tile) where they keep at least two thirds of the
     // compute units busy over their rounds: the 14336-column matrices, a q,k,v group and a gate / up pair at 512 rows
-    int tall_cols = 0, tall_tile0[3] = {0, 0, 0};
+    int tall_cols = 0, tall_tile0[3] = {0, 0, 0}, blocks = 0, block0[3] = {0, 0, 0};
     bool tall_fits = true;
     for (int i = 0; i < nseg; i++) {
-        tall_tile0[i] = tall_cols;
-        tall_cols += (segs[i].n + 127) / 128;
+        tall_tile0[i] = tall_cols, block0[i] = blocks;
+        tall_cols += (segs[i].n + 127) / 128, blocks += (segs[i].n + 31) / 32;
         tall_fits = tall_fits && (size_t)segs[i].n * (k / 256) * 144 < ((size_t)1 << 31);
     }
-    for (int i = nseg; i < 3; i++) tall_tile0[i] = tall_cols;
+    for (int i = nseg; i < 3; i++) tall_tile0[i] = tall_cols, block0[i] = blocks;
     if (swiglu_pair) tall_cols = (segs[0].n + 63) / 64;
     const int tall_tiles = ((m + 255) / 256) * tall_cols;
     const int tall_rounds = (tall_tiles + ctx->compute_units - 1) / ctx->compute_units;
-    const bool tall = tall_fits && (ctx->opt_gemm_tile == 3 ||
+    const bool tall = tall_fits && (ctx->opt_gemm_tile == 3 || (ctx->opt_gemm_tile == 4 && !swiglu_pair) ||
                                     (ctx->opt_gemm_tile == 0 && m > 128 && 3 * tall_tiles >= 2 * tall_rounds * ctx->compute_units));
     TallTail tail = {tall_tiles, 0, 1, nullptr};
     if (tall) tail = tall_tail(ctx, tall_tiles, k / 256);
+    // 96 columns where they save a round's worth by more than they cost: only what has no last tiles to share (their sums' chains would grow)
+    const int narrow_tiles = ((m + 255) / 256) * ((blocks + 2) / 3), narrow_rounds = (narrow_tiles + ctx->compute_units - 1) / ctx->compute_units;
+    const bool narrow = tall && !swiglu_pair && (ctx->opt_gemm_tile == 4 || (ctx->opt_gemm_tile == 0 && tail.tiles == 0 && 17 * narrow_rounds < 20 * tall_rounds));
+    if (narrow) tail = TallTail{narrow_tiles, 0, 1, nullptr};
     const bool small_tiles = !tall && (ctx->opt_gemm_tile == 1 ||
                              (ctx->opt_gemm_tile == 0 && (m <= 128 || ((m + 127) / 128) * n_tiles_all > ctx->compute_units)));
     const int mt_rows = tall ? 256 : small_tiles ? 64 : 128;
@@ -2302,7 +2326,7 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     const size_t part_bytes = tall ? (size_t)tail.tiles * tail.splits * 131072 : splits > 1 ? (size_t)splits * m * fs.part_cols * 4 : 0;
     float* part = part_bytes ? skn_gemm_parts_room(ctx, part_bytes) : nullptr;
     if (src.ahead) return SKN_OK;
-    if (!part) splits = 1, tail = TallTail{tall_tiles, 0, 1, nullptr};
+    if (!part) splits = 1, tail = TallTail{narrow ? narrow_tiles : tall_tiles, 0, 1, nullptr};
     fs.part_blocks = (k / 256 + splits - 1) / splits;
     if (splits > 1) fs.part = part;
     _Float16* afrag = (_Float16*)ws;
@@ -2316,10 +2340,10 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
     }
     SKN_LAUNCH_CHECK(ctx);
     if (tall) {
-        for (int i = 0; i < 3; i++) fs.tile0[i] = tall_tile0[i];
-        fs.n_tiles = tall_cols;
+        for (int i = 0; i < 3; i++) fs.tile0[i] = narrow ? block0[i] : tall_tile0[i];
+        fs.n_tiles = narrow ? blocks : tall_cols;
         tail.part = part;
-        skn_launch(ctx, tail.tiles ? gemm_q4k_tall_kernel<true> : gemm_q4k_tall_kernel<false>, dim3(tail.tile0 + tail.tiles * tail.splits), dim3(512), kTlLds, (const u32x4*)afrag, (const u32x4*)sfrag, fs,
+        skn_launch(ctx, narrow ? gemm_q4k_tall_kernel<false, 3> : tail.tiles ? gemm_q4k_tall_kernel<true, 4> : gemm_q4k_tall_kernel<false, 4>, dim3(tail.tile0 + tail.tiles * tail.splits), dim3(512), kTlLds, (const u32x4*)afrag, (const u32x4*)sfrag, fs,
                    (const float*)isc, m, k, m_tiles, (uint32_t)((size_t)m_pad * k * 2), tail);
         SKN_LAUNCH_CHECK(ctx);
         if (tail.tiles) {
