@@ -338,9 +338,148 @@ __global__ __launch_bounds__(2 * T) void prep_a_rows_kernel(const skn_gemm_src s
     }
 }
 
+// The same with four rows per workgroup, sixteen lanes of a wavefront on each, T threads a row (128; 256 where a row's elements would take too many
+// registers).  The kernel above writes sixteen bytes a lane, 512 bytes apart: two million requests for 2000 rows of 8192, which the L2 takes
+// one by one.  Here the lanes exchange their pieces before the store, so that four of them write the 64 bytes that four neighbouring rows have of
+// a fragment.  A row's squares are added in the same order as above.
+// bf16 rows, us, two rows a workgroup -> four: 2000 x 4096 12.6 -> 10.0, 2000 x 8192 20.0 -> 14.1, 4000 x 8192 31.8 -> 24.0, 2000 x 11008 25.3 -> 21.2.
+template <int NT, int SRC, bool SUMS, int T>
+__global__ __launch_bounds__(4 * T) void prep_a_quads_kernel(const skn_gemm_src src, _Float16* __restrict__ afrag, float* __restrict__ inv_scale,
+                                                             _Float16* __restrict__ sfrag, int m, int k) {
+    constexpr bool kNorm = SRC == SKN_SRC_RMSNORM;
+    constexpr int W = T / 16;  // wavefronts
+    static_assert(T == 128 || (T == 256 && !kNorm), "the order of the squares is that of 128 threads");
+    __shared__ float red_ss[kNorm ? 4 : 1][W], red_mx[4][W];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, rw = lane >> 4, t = wave * 16 + (lane & 15);
+    const int per_xcd = gridDim.x >> 3, quad = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3), row = 4 * quad + rw;
+    const bool real = row < m;
+    const size_t row_off = (size_t)(real ? row : 0) * k;
+    const int tasks = k >> 3, nch = k >> 6, nb = k >> 8;
+    const float* xf = (const float*)src.a + row_off;
+    const uint16_t* xb = (const uint16_t*)src.a + row_off;
+    float v[NT][8];
+    float4 glo[kNorm ? NT : 1], ghi[kNorm ? NT : 1];
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const int task = min(t + T * j, tasks - 1), c = task >> 3, dw = task & 7;
+        const int e0 = 64 * c + 4 * dw;
+        if (SRC == SKN_SRC_BF16) {
+            const u32x2 lo = *reinterpret_cast<const u32x2*>(xb + e0), hi = *reinterpret_cast<const u32x2*>(xb + e0 + 32);
+            v[j][0] = __uint_as_float(lo.x << 16), v[j][1] = __uint_as_float(lo.x & 0xFFFF0000u);
+            v[j][2] = __uint_as_float(lo.y << 16), v[j][3] = __uint_as_float(lo.y & 0xFFFF0000u);
+            v[j][4] = __uint_as_float(hi.x << 16), v[j][5] = __uint_as_float(hi.x & 0xFFFF0000u);
+            v[j][6] = __uint_as_float(hi.y << 16), v[j][7] = __uint_as_float(hi.y & 0xFFFF0000u);
+        } else {
+            const float4 lo = *reinterpret_cast<const float4*>(xf + e0), hi = *reinterpret_cast<const float4*>(xf + e0 + 32);
+            v[j][0] = lo.x, v[j][1] = lo.y, v[j][2] = lo.z, v[j][3] = lo.w;
+            v[j][4] = hi.x, v[j][5] = hi.y, v[j][6] = hi.z, v[j][7] = hi.w;
+            if constexpr (kNorm) {
+                glo[j] = *reinterpret_cast<const float4*>((const float*)src.b + e0);
+                ghi[j] = *reinterpret_cast<const float4*>((const float*)src.b + e0 + 32);
+            }
+        }
+    }
+    float r = 1.f;
+    if constexpr (kNorm) {
+        // tasks t, t + 128, ... in turn, then the lanes of sixteen, then the sixteens as a wavefront's sum and the two halves add them
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+            if (t + T * j < tasks) ss += ((v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3])) +
+                                         ((v[j][4] * v[j][4] + v[j][5] * v[j][5]) + (v[j][6] * v[j][6] + v[j][7] * v[j][7]));
+        ss = lane_group_sum<16>(ss);
+        if ((lane & 15) == 0) red_ss[rw][wave] = ss;
+        __syncthreads();
+        const float* z = red_ss[rw];
+        r = 1.0f / sqrtf((((z[0] + z[1]) + (z[2] + z[3])) + ((z[4] + z[5]) + (z[6] + z[7]))) / (float)k + src.eps);
+    }
+    // the bf16 values the GEMM is defined on (fp32 sources: rounded to nearest even here), and their largest magnitude
+    float mx = 0.f;
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        if (SRC != SKN_SRC_BF16) {
+            const float4 gl = kNorm ? glo[kNorm ? j : 0] : make_float4(1.f, 1.f, 1.f, 1.f);
+            const float4 gh = kNorm ? ghi[kNorm ? j : 0] : make_float4(1.f, 1.f, 1.f, 1.f);
+            const float g[8] = {gl.x, gl.y, gl.z, gl.w, gh.x, gh.y, gh.z, gh.w};
+#pragma unroll
+            for (int x = 0; x < 8; x++) {
+                const float y = kNorm ? v[j][x] * r * g[x] : v[j][x];
+                v[j][x] = __uint_as_float(bf16_rne(y) << 16);
+            }
+        }
+#pragma unroll
+        for (int x = 0; x < 8; x++) {
+            const float f = fabsf(v[j][x]);
+            if (f == f && f < INFINITY) mx = fmaxf(mx, f);
+        }
+    }
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    if ((lane & 15) == 0) red_mx[rw][wave] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < W; i++) mx = fmaxf(mx, red_mx[rw][i]);
+    if (!real) mx = 0.f;
+    int e = 9;  // a zero row keeps scale 1
+    if (mx > 0.f) e = (int)((__float_as_uint(mx) >> 23) & 0xFF) - 127;
+    e = max(e, -100);
+    const float scale = real ? __uint_as_float((uint32_t)(127 + 9 - e) << 23) : 0.f;
+    if (t == 0 && real) inv_scale[row] = __uint_as_float((uint32_t)(127 - 9 + e) << 23);
+    const int mb = row >> 5, rr = row & 31;  // (a quad lies in one row block)
+    // lane 4 i + r of the store has piece i of the wavefront's sixteen and row r of its four
+    const int from = 4 * (16 * (lane & 3) + (lane >> 2)), to_row = 4 * (quad & 7) + (lane & 3);
+    u32x4* out = reinterpret_cast<u32x4*>(afrag) + (size_t)mb * nch * 256 + to_row;
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const int task = t + T * j, c = task >> 3, dw = task & 7;
+        _Float16 l[4], u[4];
+#pragma unroll
+        for (int x = 0; x < 4; x++) l[x] = (_Float16)(v[j][x] * scale), u[x] = (_Float16)(v[j][4 + x] * scale);
+        half8_t o;
+        o[0] = l[0], o[1] = l[2], o[2] = u[0], o[3] = u[2], o[4] = l[1], o[5] = l[3], o[6] = u[1], o[7] = u[3];
+        const u32x4 mine = __builtin_bit_cast(u32x4, o);
+        u32x4 theirs;
+#pragma unroll
+        for (int x = 0; x < 4; x++) theirs[x] = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)mine[x]);
+        const int their_task = wave * 16 + (lane >> 2) + T * j, tc = their_task >> 3, tdw = their_task & 7;
+        if (their_task < tasks) out[((size_t)tc * 4 + (tdw & 3)) * 64 + (tdw >> 2) * 32] = theirs;
+        if (SUMS) {  // totals over the eight lanes of the chunk
+            float sl = ((float)l[0] + (float)l[1]) + ((float)l[2] + (float)l[3]);
+            float su = ((float)u[0] + (float)u[1]) + ((float)u[2] + (float)u[3]);
+            sl += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(sl), 0xB1, 0xF, 0xF, true));
+            su += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(su), 0xB1, 0xF, 0xF, true));
+            sl += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(sl), 0x4E, 0xF, 0xF, true));
+            su += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(su), 0x4E, 0xF, 0xF, true));
+            sl += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(sl), 0x141, 0xF, 0xF, true));
+            su += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(su), 0x141, 0xF, 0xF, true));
+            if (dw == 0 && task < tasks) {
+                _Float16 h0, h1, l0, l1;
+                skn_split_hilo(sl * 0x1p-12f, h0, l0);
+                skn_split_hilo(su * 0x1p-12f, h1, l1);
+                _Float16* sf = sfrag + ((size_t)mb * nb + (c >> 2)) * 512 + 2 * (c & 3);
+                half2_t vh = {h0, h1}, vl = {l0, l1};
+                *reinterpret_cast<half2_t*>(sf + rr * 8) = vh;
+                *reinterpret_cast<half2_t*>(sf + (32 + rr) * 8) = vl;
+            }
+        }
+    }
+}
+
 template <int SRC, bool SUMS>
 void launch_prep(skn_ctx* ctx, const skn_gemm_src& src, _Float16* afrag, float* isc, _Float16* sfrag, int m, int m_pad, int k) {
     // (m_pad is a multiple of 32: the pair count divides by the eight XCDs its workgroups are dealt to)
+    // Four rows a workgroup where those fill the device, without a norm to wait for half of it (two rows | four, us: 333 x 4096 7.1 | 7.3, 512 x 4096
+    // 7.2 | 7.0, behind a norm 7.4 | 7.9, 2000 x 2048 behind a norm 10.9 | 8.4, 333 x 11008 10.4 | 11.8, 512 x 11008 10.8 | 10.2, 1000 x 11008
+    // 14.3 | 11.4), and what their registers hold: up to 4096 elements behind a norm, 12288 otherwise.
+    constexpr int kPlain = SRC == SKN_SRC_RMSNORM ? SKN_SRC_F32 : SRC;  // (the wider forms have no norm: not reached with one)
+    if (m_pad % 32 == 0 && m_pad / 4 >= ctx->compute_units / (SRC == SKN_SRC_RMSNORM ? 1 : 2) && k <= (SRC == SKN_SRC_RMSNORM ? 4096 : 12288)) {
+        const dim3 grid(m_pad / 4);
+        if (k <= 2048) skn_launch(ctx, prep_a_quads_kernel<2, SRC, SUMS, 128>, grid, dim3(512), 0, src, afrag, isc, sfrag, m, k);
+        else if (k <= 4096) skn_launch(ctx, prep_a_quads_kernel<4, SRC, SUMS, 128>, grid, dim3(512), 0, src, afrag, isc, sfrag, m, k);
+        else if (k <= 8192) skn_launch(ctx, prep_a_quads_kernel<4, kPlain, SUMS, 256>, grid, dim3(1024), 0, src, afrag, isc, sfrag, m, k);
+        else skn_launch(ctx, prep_a_quads_kernel<6, kPlain, SUMS, 256>, grid, dim3(1024), 0, src, afrag, isc, sfrag, m, k);
+        return;
+    }
     if (k <= 16384 && m_pad % 16 == 0) {
         const dim3 grid(m_pad / 2), block(512);
         const int nt = (k / 8 + 255) / 256;
