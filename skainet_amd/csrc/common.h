@@ -278,6 +278,13 @@ __device__ __forceinline__ float lane_group_sum(float v) {
     return v;
 }
 
+// sixteen bytes per lane from `lane_off` + `off` of a resource to LDS, the wavefront's one after the other from `to` on
+__device__ __forceinline__ void skn_load_to_lds(__amdgpu_buffer_rsrc_t from, uint8_t* to, int lane_off, int off) {
+#ifdef __HIP_DEVICE_COMPILE__  // (the host's pass has no such builtin)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)to, 16, lane_off, off, 0, 0);
+#endif
+}
+
 // Little-endian loads from addresses that are only 2-byte (or 1-byte) aligned.
 __device__ __forceinline__ uint32_t load_u32_a2(const uint8_t* p) {
     const uint16_t* q = reinterpret_cast<const uint16_t*>(p);

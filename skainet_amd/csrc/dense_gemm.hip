@@ -51,13 +51,6 @@ __device__ __forceinline__ float16_t mma(const u32x4& a, const u32x4& b, float16
     }
 }
 
-// sixteen bytes per lane from `lane_off` + `off` of a resource to LDS, the wavefront's one after the other from `to` on
-__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t from, uint8_t* to, int lane_off, int off) {
-#ifdef __HIP_DEVICE_COMPILE__  // (the host's pass has no such builtin)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)to, 16, lane_off, off, 0, 0);
-#endif
-}
-
 // T: uint16_t (bf16) or float.  lda_b, ldw_b: row pitches in bytes; slices = k_pad bytes / 128.
 template <typename T, typename S>
 __global__ __launch_bounds__(S::kThreads) void dense_gemm_kernel(const uint8_t* __restrict__ a, int64_t lda_b, int m, const uint8_t* __restrict__ w,
@@ -101,10 +94,10 @@ __global__ __launch_bounds__(S::kThreads) void dense_gemm_kernel(const uint8_t* 
         uint8_t* to = lds + buf;
 #pragma unroll
         for (int i = 0; i < kReqA; i++)
-            load_to_lds(res_a, to + (wave * kReqA + i) * 1024, from_a[i], slice * kSlice);
+            skn_load_to_lds(res_a, to + (wave * kReqA + i) * 1024, from_a[i], slice * kSlice);
 #pragma unroll
         for (int i = 0; i < kReqW; i++)
-            load_to_lds(res_w, to + kRowsA * kSlice + (wave * kReqW + i) * 1024, from_w[i], slice * kSlice);
+            skn_load_to_lds(res_w, to + kRowsA * kSlice + (wave * kReqW + i) * 1024, from_w[i], slice * kSlice);
     };
 
     float16_t acc[TN][TM];

@@ -513,9 +513,11 @@ struct Q4kFragSegs {
 
 // the kernel's LDS (weight buffers, then the tile exchange) exceeds the static limit (the scales of the tile's rows follow it): dynamic, opted in per
 // device by skn_gemm_init
+// A buffer of weights: the 32 rows of each half of the tile's columns in nineteen pieces of 1 KiB (32 x 37 slots of sixteen bytes, the rest unused)
+constexpr int kWHalf = 19, kWBuf = 2 * kWHalf * 1024;
 template <int MT, int MH>
 constexpr int frag_lds_bytes() {
-    return 2 * kBN * kWPitch > MT * MH * 24576 ? 2 * kBN * kWPitch : MT * MH * 24576;
+    return 2 * kWBuf > MT * MH * 24576 ? 2 * kWBuf : MT * MH * 24576;
 }
 
 // Accumulators: acc holds the running sum of a column in units of cs = d * 2^14 of the latest superblock whose d
@@ -527,7 +529,6 @@ template <int MT, int MH, bool SPLIT>
 __global__ __launch_bounds__(256 * MH) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restrict__ sfrag, const Q4kFragSegs segs,
                           const float* __restrict__ inv_scale, int m, int k, uint32_t a_bytes) {
-    constexpr int kWBuf = kBN * kWPitch;
     extern __shared__ __align__(16) uint8_t lds[];  // max(2 kWBuf, MT x 48 KiB) bytes
     const int tid = threadIdx.x, lane = tid & 63;
     // (the wavefront's index as a scalar: everything derived from it -- its row blocks, its superblocks, the
@@ -550,22 +551,24 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
     const int n = segs.n[seg];
     const int mb0 = (MH * mt + mh) * MT, n0 = pair ? tn * 32 : (tn - segs.tile0[seg]) * kBN;
 
-    // Weight staging, global memory straight into LDS: a wavefront-wide load fills 64 sixteen-byte slots
-    // i * 64 + lane; slot P holds piece P % 37 of tile row P / 37 (36 pieces = the 576 bytes of four
-    // superblocks, the 37th a pad that repeats the last).  The 37 loads of a group are dealt round the wavefronts.  Completion is waited for
-    // with the vector-memory counter before the barrier that publishes the buffer.
+    // Weight staging, memory straight into LDS: a wavefront-wide load fills 64 sixteen-byte slots of a half of the buffer; slot P holds piece
+    // P % 37 of row P / 37 of that half (36 pieces = the 576 bytes of four superblocks, the 37th a pad that repeats the last).  The 38 loads of a
+    // group are dealt round the wavefronts (whose last may be the 38th again: no branch, so that the compiler can count).  Completion is waited
+    // for with the vector-memory counter before the barrier that publishes the buffer.
+    // Buffer loads: one with a 64-bit address passes for a load that LDS may answer, and from it on the compiler waited for all loads that
+    // were out, the next group's weights ahead of this group's first product (us: 120 x 4096 x 4096 17.9 ->
+    // 16.2, in two parts of k 11008 25.3 -> 22.3, gate and up of 11008 41.3 -> 39.2, 2000 x 2048 and 8192 66.6 -> 62.0 in the mean).
+    const uint8_t* w_hi = pair ? segs.w[1] + (size_t)n0 * nb * 144 : w + (size_t)min(n0 + 32, n - 1) * nb * 144;  // (pair: rows 32 .. are the up matrix)
+    const int rows_lo = min(n - n0, 32), rows_hi = pair ? rows_lo : max(min(n - n0 - 32, 32), 1);
+    const __amdgpu_buffer_rsrc_t res_lo = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * nb * 144), 0, rows_lo * nb * 144, 0x00020000);
+    const __amdgpu_buffer_rsrc_t res_hi = __builtin_amdgcn_make_buffer_rsrc((void*)w_hi, 0, rows_hi * nb * 144, 0x00020000);
     auto wfetch = [&](int g, int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int x = 0; x < (kWPieces + 4 * MH - 1) / (4 * MH); x++) {
-            const int i = wave + 4 * MH * x;
-            if (i < kWPieces) {
-                const int p = i * 64 + lane, row = p / kWPieces, col = min(p - kWPieces * row, 35);
-                const int off = min(sb0 * 144 + g * 576 + col * 16, nb * 144 - 16);  // (a short last group repeats the row's last piece)
-                const uint8_t* wsrc = pair && row >= 32 ? segs.w[1] : w;  // (pair: tile rows 32.. are the up matrix)
-                const uint8_t* src = wsrc + (size_t)min(n0 + (pair ? row & 31 : row), n - 1) * nb * 144 + off;
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                                 (__attribute__((address_space(3))) void*)(lds + buf * kWBuf + i * 1024), 16, 0, 0);
-            }
+        for (int x = 0; x < (2 * kWHalf + 4 * MH - 1) / (4 * MH); x++) {
+            const int i = min(wave + 4 * MH * x, 2 * kWHalf - 1), hi = i >= kWHalf;
+            const int p = (i - hi * kWHalf) * 64 + lane, row = p / kWPieces, col = min(p - kWPieces * row, 35);
+            const int off = min(sb0 * 144 + g * 576 + col * 16, nb * 144 - 16);  // (a short last group repeats the row's last piece)
+            skn_load_to_lds(hi ? res_hi : res_lo, lds + buf * kWBuf + i * 1024, min(row, (hi ? rows_hi : rows_lo) - 1) * nb * 144 + off, 0);
         }
     };
 
@@ -606,13 +609,13 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
-    for (int g = 0; g < groups; g++) {
+    auto group = [&](int g, auto more) __attribute__((always_inline)) {
         const int sb = sb0 + 4 * g + kq;
-        if (g + 1 < groups) wfetch(g + 1, (g + 1) & 1);
+        if constexpr (decltype(more)::value) wfetch(g + 1, (g + 1) & 1);
         if (sb < sb1) {
             // this lane's weight rows (one per 32-column tile): the 144 bytes of superblock sb
             const uint8_t* wl = lds + (g & 1) * kWBuf + r * kWPitch + kq * 144;
-            constexpr int kTile = 32 * kWPitch;  // the lane's row of the second 32-column tile
+            constexpr int kTile = kWHalf * 1024;  // the lane's row of the second 32-column tile
             u32x4 hd[2], sf[MT];
 #pragma unroll
             for (int j = 0; j < 2; j++) hd[j] = *reinterpret_cast<const u32x4*>(wl + j * kTile);
@@ -746,8 +749,12 @@ void gemm_q4k_frag_kernel(const u32x4* __restrict__ afrag, const u32x4* __restri
         // complete in order: once all but the newest 8 MT have landed, so have they.
         if (sb < sb1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * MT) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    }
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), in a form that the compiler counts with
+        asm volatile("s_barrier" ::: "memory");
+    };
+    // (the last group apart: what is out behind its fragments is known where nothing is requested on condition)
+    for (int g = 0; g + 1 < groups; g++) group(g, std::true_type{});
+    if (groups > 0) group(groups - 1, std::false_type{});
     // back to true units
 #pragma unroll
     for (int i = 0; i < MT; i++)
