@@ -12,6 +12,7 @@
 // The fp32 form reads the same 16-byte pieces (four elements, half a wavefront each) and issues four matrix instructions
 // per piece: k is summed in another order than it lies in memory, the same for both operands.
 #include "dense.h"
+#include "dense_plan.h"
 
 #include <type_traits>
 
@@ -263,46 +264,16 @@ int launch_gemm(skn_ctx* ctx, const skn_dense_mat& w, const void* a, int lda, in
 
 template <typename T>
 int pick_gemm(skn_ctx* ctx, const skn_dense_mat& w, const void* a, int lda, int m, const skn_dense_out& out) {
-    // Each shape's time, us, fitted to 476 shapes (40 to 2048 tokens, 256 to 18496 rows, k from 512 to 8192, weights not in any cache): of a launch, of
-    // the loop over k = 4096 with one, two or three tiles on a compute unit, and of the store of a tile to each.  On those shapes the choice
-    // takes 1.015 times the best one's time in the mean, 1 / 1.047 of what it took before, when it knew no k and no stores (2048 x 2048 x 8192
-    // 94 -> 88 us, 1000 x 18496 x 2048 in a model 151 -> 142), and at worst 1.035 times as long.  Rows of less than 512 elements, and fp32, whose loop is all of
-    // the time, are reckoned with as if k were 4096.
-    struct Cost {
-        int rows_a, rows_w, resident;
-        float launch, loop[3], store;
-    };
-    const Cost costs[8] = {{64, 64, 3, 8.2f, {28.6f, 38.8f, 35.4f}, 0.8f}, {128, 64, 2, 10.3f, {33.f, 51.8f}, 3.6f}, {128, 128, 2, 8.6f, {65.9f, 62.f}, 5.5f},
-                           {256, 256, 1, 12.2f, {88.3f}, 22.7f},           {0, 0, 0, 0.f, {0.f}, 0.f},               {256, 192, 1, 13.f, {60.1f}, 21.5f},
-                           {128, 192, 2, 20.6f, {47.f, 55.8f}, 8.9f},      {128, 128, 1, 7.7f, {49.8f}, 5.f}};
-    const int units = ctx->compute_units;
-    const bool known = sizeof(T) == 2 && w.k_pad >= 512;
-    const float length = known ? (float)w.k_pad / 4096.f : 1.f;
-    int best = 0;
-    float best_time = INFINITY;
-    for (int i = 0; i < 8; i++) {
-        const Cost& c = costs[i];
-        if (c.resident == 0) continue;  // (the divided tile has a rule of its own below)
-        const int tiles = ((m + c.rows_a - 1) / c.rows_a) * ((w.rows + c.rows_w - 1) / c.rows_w), round = c.resident * units;
-        const int rest = tiles % round;
-        // (128 x 192 is for the rounds of widths that 128 and 256 leave a third of idle)
-        if (!known && c.rows_w == 192 && rest != 0 && 5 * rest < 4 * (rest <= units ? units : round)) continue;
-        const float loops = tiles / round * c.loop[c.resident - 1] + (rest == 0 ? 0.f : c.loop[(rest - 1) / units]);
-        const float time = c.launch + length * loops + (float)tiles / units * c.store;
-        if (time < best_time) best = i, best_time = time;
-    }
-    // Few outputs: k divided in four (rows of half as many slices where half of the compute units have a tile: 40 x 512 x 512 7.3 -> 5.0 us)
-    const int few = ((m + 31) / 32) * ((w.rows + 63) / 64), row_slices = w.k_pad * (int)sizeof(T) / kSlice;
-    if ((few <= units && row_slices >= 16) || (2 * few <= units && row_slices >= 8)) best = 4;
+    int best = skn_dense_tile((int)sizeof(T), m, w.rows, w.k_pad, ctx->compute_units);
     if (ctx->opt_dense_tile > 0) best = ctx->opt_dense_tile - 1;
     switch (best) {
-        case 0: return launch_gemm<T, Tile64x64>(ctx, w, a, lda, m, out);
-        case 1: return launch_gemm<T, Tile128x64>(ctx, w, a, lda, m, out);
-        case 2: return launch_gemm<T, Tile128x128>(ctx, w, a, lda, m, out);
-        case 4: return launch_gemm<T, Tile32x64Split>(ctx, w, a, lda, m, out);
-        case 5: return launch_gemm<T, Tile256x192>(ctx, w, a, lda, m, out);
-        case 6: return launch_gemm<T, Tile128x192>(ctx, w, a, lda, m, out);
-        case 7: return launch_gemm<T, Tile128x128Split>(ctx, w, a, lda, m, out);
+        case SKN_TILE_64x64: return launch_gemm<T, Tile64x64>(ctx, w, a, lda, m, out);
+        case SKN_TILE_128x64: return launch_gemm<T, Tile128x64>(ctx, w, a, lda, m, out);
+        case SKN_TILE_128x128: return launch_gemm<T, Tile128x128>(ctx, w, a, lda, m, out);
+        case SKN_TILE_32x64_K4: return launch_gemm<T, Tile32x64Split>(ctx, w, a, lda, m, out);
+        case SKN_TILE_256x192: return launch_gemm<T, Tile256x192>(ctx, w, a, lda, m, out);
+        case SKN_TILE_128x192: return launch_gemm<T, Tile128x192>(ctx, w, a, lda, m, out);
+        case SKN_TILE_128x128_K2: return launch_gemm<T, Tile128x128Split>(ctx, w, a, lda, m, out);
         default: return launch_gemm<T, Tile256x256>(ctx, w, a, lda, m, out);
     }
 }

@@ -1,0 +1,76 @@
+"""CPU: which tile a dense product takes (csrc/dense_plan.h, which the library asks, compiled for the host)."""
+import os
+import random
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+UNITS = 256
+BF16, F32 = 2, 4
+# tokens, weight rows of a tile; the fifth has k divided in four
+TILES = [(64, 64), (128, 64), (128, 128), (256, 256), (32, 64), (256, 192), (128, 192), (128, 128)]
+K4 = 4
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("no g++")
+    exe = str(tmp_path_factory.mktemp("plan") / "plan")
+    subprocess.run([gxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-I", os.path.join(ROOT, "skainet_amd", "csrc"), "-o", exe,
+                    os.path.join(ROOT, "tests", "c", "dense_plan.cpp")], check=True)
+
+    def ask(what, questions):
+        text = "".join(" ".join(map(str, (what, *q))) + "\n" for q in questions)
+        lines = subprocess.run([exe], input=text, capture_output=True, text=True, timeout=100, check=True).stdout.split("\n")[:-1]
+        assert len(lines) == len(questions)
+        return [tuple(map(int, line.split())) for line in lines]
+
+    return ask
+
+
+def _tiles(plan, shapes):
+    return [t for t, in plan("tile", [(*s, UNITS) for s in shapes])]
+
+
+def _busiest(tile, m, rows):
+    """outputs of the compute unit that has the most"""
+    a, w = TILES[tile]
+    return -(-(-(-m // a) * -(-rows // w)) // UNITS) * a * w
+
+
+# fp32, whose loop is all of a product's time, and bf16 rows of less than 512 elements, which the costs in us were not fitted to
+@pytest.mark.parametrize("size,longest", [(F32, 10240), (BF16, 448)])
+def test_where_the_loop_is_all_no_compute_unit_has_much_more_than_it_must(plan, size, longest):
+    rng = random.Random(size)
+    shapes = [(size, rng.randint(1, 4096), 32 * rng.randint(1, 800), 64 * rng.randint(1, longest // 64)) for _ in range(3000)]
+    for (_, m, rows, k), tile in zip(shapes, _tiles(plan, shapes)):
+        if tile != K4:
+            assert _busiest(tile, m, rows) <= 1.5 * min(_busiest(t, m, rows) for t in range(len(TILES)) if t != K4), (m, rows, k, tile)
+
+
+# (measured, us: 1000 x 8512 x 2048 in fp32 339 on 64 x 64 and 515 on 256 x 256, see csrc/dense_plan.h)
+@pytest.mark.parametrize("shape,tile", [((F32, 1000, 8512, 2048), 0), ((F32, 954, 8512, 2048), 0), ((F32, 512, 18496, 2048), 1), ((F32, 1700, 10752, 2048), 2),
+                                        ((F32, 2048, 10752, 2048), 2), ((BF16, 1000, 8512, 256), 0), ((BF16, 954, 8512, 448), 0), ((BF16, 1700, 10752, 256), 2)])
+def test_fp32_and_short_rows(plan, shape, tile):
+    assert _tiles(plan, [shape]) == [tile]
+
+
+# one measured shape for each tile that is the fastest of all there (profiles/dense_gemm_tiles.md)
+@pytest.mark.parametrize("m,rows,k,tile", [(333, 5120, 512, 0), (200, 5120, 4096, 1), (2048, 4096, 8192, 2), (1500, 8192, 4096, 3), (512, 18496, 4096, 5),
+                                           (512, 10752, 4096, 6), (512, 8192, 8192, 7)])
+def test_bf16_by_the_fitted_costs(plan, m, rows, k, tile):
+    assert _tiles(plan, [(BF16, m, rows, k)]) == [tile]
+
+
+# 32 x 64 tiles with k divided in four: up to half of the compute units with rows of eight slices of 128 bytes, all of them with sixteen
+@pytest.mark.parametrize("size", [BF16, F32])
+@pytest.mark.parametrize("slices,rows", [(8, 8192), (15, 8192), (16, 16384), (64, 16384)])
+def test_few_outputs(plan, size, slices, rows):
+    k = slices * 128 // size
+    at, past, wide = _tiles(plan, [(size, 32, rows, k), (size, 32, rows + 32, k), (size, 33, rows, k)])
+    assert at == K4 and past != K4 and wide != K4
+    assert _tiles(plan, [(size, 32, 64, 7 * 128 // size)]) != [K4]
