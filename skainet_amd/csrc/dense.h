@@ -5,8 +5,8 @@
 // (padding rows are zeros).  What happens to the rows of a projection -- bias, activation, where they go -- is a segment.
 #pragma once
 #include "common.h"
+#include "dense_plan.h"
 
-constexpr int kDenseRowPad = 32, kDenseColPad = 64;
 static inline int skn_pad_rows(int n) { return (n + kDenseRowPad - 1) / kDenseRowPad * kDenseRowPad; }
 static inline int skn_pad_cols(int k) { return (k + kDenseColPad - 1) / kDenseColPad * kDenseColPad; }
 
@@ -64,11 +64,11 @@ struct skn_dense_out {
 // C[m, rows] from A [m][lda] of the matrix's type (lda elements, a multiple of 64, zeros from k to k_pad).
 int skn_dense_gemm(skn_ctx* ctx, const skn_dense_mat& w, const void* a, int lda, int m, const skn_dense_out& out);
 
-// The input of a matvec, staged once per workgroup.
-enum { SKN_XSRC_PLAIN = 0, SKN_XSRC_GROUP_NORM = 1, SKN_XSRC_MERGE = 2, SKN_XSRC_ADD_NORM = 3 };
+// The input of a matvec.  Vectors of k0 columns (x0, norm_w, add, add_w, x_out) are 16-byte aligned and have room for whole fours of them: up to
+// three elements past k0 may be read, and count as zero.
 struct skn_matvec_src {
     int mode = SKN_XSRC_PLAIN;
-    const float* x0 = nullptr;      // columns [0, k0); 16-byte aligned
+    const float* x0 = nullptr;      // columns [0, k0)
     int k0 = 0;
     const float* x1 = nullptr;      // columns [off1, off1 + k1), optional
     int off1 = 0, k1 = 0;

@@ -12,7 +12,6 @@
 // The fp32 form reads the same 16-byte pieces (four elements, half a wavefront each) and issues four matrix instructions
 // per piece: k is summed in another order than it lies in memory, the same for both operands.
 #include "dense.h"
-#include "dense_plan.h"
 
 #include <type_traits>
 

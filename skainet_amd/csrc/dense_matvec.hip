@@ -2,7 +2,7 @@
 // the chain of latencies from the launch's arguments to its last store.
 //
 // dense_matvec_once_kernel (most calls): a workgroup has a few rows, its wavefronts share them piece by piece, and everything is asked for
-// at once.  dense_matvec_kernel (inputs whose preparation is large beside the rows of one workgroup, see once_rows): the input
+// at once.  dense_matvec_kernel (inputs whose preparation is large beside the rows of one workgroup, see csrc/dense_plan.h): the input
 // is staged once per workgroup in LDS -- plain, divided group by group by its root mean square (the norm ahead
 // of a layer), or with the split partials of an attention merged on the way in -- as two planes of float4 (even and odd
 // fours of elements), so that the eight activations of a 16-byte piece of bf16 weights are two conflict-free 16-byte
@@ -426,10 +426,6 @@ struct LaneSums {
     static __device__ __forceinline__ int index(int i, int j) { return 4 * i + (j >> 1) + 2 * (j & 1); }
 };
 
-constexpr int kOnceGroups = 8;  // norm groups
-
-constexpr int kOnceParts = 16;  // wavefronts of a workgroup, half of them where the input is worked on (a merge has a hundred registers of partials)
-
 // W: uint16_t (bf16) or float.  X: 1, or 2 with a second input (SKN_XSRC_PLAIN); the most splits that are merged (SKN_XSRC_MERGE).
 // parts_nseg: wavefronts of the workgroup, segments << 16.
 template <typename W, int MODE, int PW, int R, int SP>
@@ -686,7 +682,7 @@ int launch_once(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src,
     OnceArgs a = {};
     a.add = src.add, a.add_w = src.add_w, a.x_out = src.x_out;
     a.groups = src.groups, a.group_size = src.k0 / src.groups, a.eps = src.eps, a.mult = out.mult;
-    a.cache_seg = out.cache_seg, a.mul_seg = out.mul_seg;
+    a.cache_seg = out.nseg > 0 ? out.cache_seg : -1, a.mul_seg = out.nseg > 0 ? out.mul_seg : -1;  // (the residual form has no segments)
     a.ml = src.ml, a.gate = src.gate, a.heads = src.heads, a.dim = src.dim, a.dim_pad = src.dim_pad, a.splits = src.splits, a.sink = src.sink;
     if (out.nseg > 0) a.seg = out.seg[0];
     for (int q = 0; q < out.nseg; q++) a.starts[q] = out.seg[q].row0;
@@ -697,39 +693,15 @@ int launch_once(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src,
     return SKN_OK;
 }
 
-// Rows of a workgroup of dense_matvec_once_kernel whose `parts` wavefronts share `rows` rows; 0: the input takes so much that many rows are better
-// behind one staging of it.  Four rows where the input is taken as it is (two where that leaves compute units without work): 2048 x 2048
-// 3.52 | 3.49 | 3.59 us with 2 | 4 | 8, 2048 x 8192 8.0 | 7.3 | 7.7, 256 x 2048 and 2048 x 256 4.96 | 4.80 | 5.20.  A norm's launch takes rounds of compute
-// units, a round of 2, 4, 8, 16 rows as 0.38, 0.6, 1, 1.9 (960 x 3072 behind a sum and a norm 5.2 | 4.2 | 4.6 | 5.5, 2624 x 3072 9.5 | 7.4 | 7.2 | 6.1, 5120 x
-// 3072 15.0 | 10.8 | 9.6 | 10.2): over eighty shapes of a mode this is 1 % off the best number in the mean.  The staged kernel: behind a sum and a norm 13312 x 2048
-// 11.8 | 12.7 us, x 3072 16.6 | 18.6, but 8192 x 2048 9.8 | 8.2, 5120 x 4096 12.2 | 11.3; behind a merge of eight splits 4096 x 3072 9.5 | 9.7, 2624 x 4096 9.6 |
-// 10.4, but 5120 x 2048 9.1 | 8.5, 2048 x 4096 7.7 | 7.0.
-int once_rows(int mode, int rows, int parts, int units) {
-    const int64_t pieces = (int64_t)rows * parts;
-    if (mode == SKN_XSRC_PLAIN) return parts == 1 ? 8 : rows <= 2 * units ? 2 : 4;
-    if (mode == SKN_XSRC_MERGE) return pieces > 80 * units ? 0 : rows <= 4 * units ? 4 : 8;
-    if (mode == SKN_XSRC_ADD_NORM && pieces > 176 * units) return 0;
-    const float round_cost[4] = {0.38f, 0.6f, 1.0f, 1.9f};
-    int best = 0;
-    float least = INFINITY;
-    for (int i = 0; i < 4; i++) {
-        const int r = 2 << i;
-        const float rounds = (float)rows / (float)(r * units), cost = round_cost[i] * (0.7f * ceilf(rounds) + 0.3f * rounds);
-        if (r <= 8 * parts && cost < least) best = r, least = cost;
-    }
-    return best;
-}
-
 // SKN_ERR_TYPE, without a message: not a call for dense_matvec_once_kernel
 template <typename W, int MODE>
 int try_once(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, const skn_dense_out& out) {
-    constexpr int V = 16 / (int)sizeof(W);
-    const int pieces = (w.k_pad + 64 * V - 1) / (64 * V);
-    const int pw = MODE != SKN_XSRC_PLAIN || pieces <= kOnceParts ? 1 : pieces <= 2 * kOnceParts ? 2 : 4, parts = (pieces + pw - 1) / pw;
-    if (src.x1 || parts > (MODE == SKN_XSRC_PLAIN ? kOnceParts : kOnceParts / 2) || (int64_t)(w.ld ? w.ld : w.k_pad) * (int)sizeof(W) >= (int64_t)1 << 30) return SKN_ERR_TYPE;
-    const int r = once_rows(MODE, w.rows, parts, ctx->compute_units);
+    skn_dense_call call = {MODE, (int)sizeof(W), w.rows, w.k_pad, w.ld ? w.ld : w.k_pad, src.k0, src.groups, src.dim, src.x1 != nullptr, out.nseg, {}};
+    for (int i = 0; i < out.nseg; i++) call.row0[i] = out.seg[i].row0;
+    const skn_dense_once plan = skn_dense_once_plan(call, ctx->compute_units);
+    const int r = plan.rows, parts = plan.parts;
+    if (r == 0) return SKN_ERR_TYPE;
     if constexpr (MODE == SKN_XSRC_MERGE) {
-        if (src.dim % V != 0 || r == 0) return SKN_ERR_TYPE;
         auto rows = [&](auto four) {
             constexpr int R = decltype(four)::value ? 4 : 8;
             return src.splits <= 2   ? launch_once<W, MODE, 1, R, 2>(ctx, w, src, out, parts)
@@ -739,20 +711,17 @@ int try_once(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, co
         };
         return r == 4 ? rows(std::true_type{}) : rows(std::false_type{});
     } else if constexpr (MODE == SKN_XSRC_PLAIN) {
-        if (pw == 4) return launch_once<W, MODE, 4, 4, 1>(ctx, w, src, out, parts);
-        if (pw == 2) return launch_once<W, MODE, 2, 4, 1>(ctx, w, src, out, parts);
+        if (plan.pieces == 4) return launch_once<W, MODE, 4, 4, 1>(ctx, w, src, out, parts);
+        if (plan.pieces == 2) return launch_once<W, MODE, 2, 4, 1>(ctx, w, src, out, parts);
         return r == 2   ? launch_once<W, MODE, 1, 2, 1>(ctx, w, src, out, parts)
                : r == 4 ? launch_once<W, MODE, 1, 4, 1>(ctx, w, src, out, parts)
                         : launch_once<W, MODE, 1, 8, 1>(ctx, w, src, out, parts);
     } else {
-        // (a norm group takes whole requests of a lane)
-        if (src.groups > kOnceGroups || (src.groups > 1 && (MODE == SKN_XSRC_ADD_NORM || src.k0 / src.groups % V != 0))) return SKN_ERR_TYPE;
         switch (r) {
             case 2: return launch_once<W, MODE, 1, 2, 1>(ctx, w, src, out, parts);
             case 4: return launch_once<W, MODE, 1, 4, 1>(ctx, w, src, out, parts);
             case 8: return launch_once<W, MODE, 1, 8, 1>(ctx, w, src, out, parts);
-            case 16: return launch_once<W, MODE, 1, 16, 1>(ctx, w, src, out, parts);
-            default: return SKN_ERR_TYPE;
+            default: return launch_once<W, MODE, 1, 16, 1>(ctx, w, src, out, parts);
         }
     }
 }

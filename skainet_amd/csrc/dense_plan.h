@@ -1,6 +1,9 @@
 // Which kernel and tile a dense product takes (plain C++, so that a host program can ask for any shape and any number of compute units).
 #pragma once
 #include <cmath>
+#include <cstdint>
+
+constexpr int kDenseRowPad = 32, kDenseColPad = 64;  // what the projections of a stacked matrix and its rows are padded to
 
 // ---- tiles of the batched GEMM (dense_gemm.hip), tokens x weight rows; "dense.tile" is one more than these -----------------
 enum {
@@ -59,4 +62,65 @@ static inline int skn_dense_tile(int elem_bytes, int m, int rows, int k_pad, int
     const int few = ((m + 31) / 32) * ((rows + 63) / 64), slices = k_pad * elem_bytes / 128;
     if ((few <= units && slices >= 16) || (2 * few <= units && slices >= 8)) best = SKN_TILE_32x64_K4;
     return best;
+}
+
+// ---- the batch-1 product (dense_matvec.hip) ----------------------------------------------------------------------------------
+enum { SKN_XSRC_PLAIN = 0, SKN_XSRC_GROUP_NORM = 1, SKN_XSRC_MERGE = 2, SKN_XSRC_ADD_NORM = 3 };  // what its input is made of (dense.h)
+
+struct skn_dense_call {
+    int mode, elem_bytes, rows, k_pad;
+    int64_t ld;               // elements from row to row
+    int k0, groups, dim;      // columns of the input, norm groups, elements of a merged head
+    bool second_input;
+    int nseg;                 // segments and where they begin; 0: residual form
+    int row0[8];
+};
+
+constexpr int kOnceGroups = 8;  // norm groups
+constexpr int kOnceParts = 16;  // wavefronts of a workgroup on a plain input, half of them where the input is worked on
+
+// dense_matvec_once_kernel: wavefronts of a workgroup, 1 KiB pieces of a row that each has, rows; rows 0: the staged kernel.
+struct skn_dense_once {
+    int parts, pieces, rows;
+};
+
+// Rows of a workgroup whose `parts` wavefronts share `rows` rows; 0: the input takes so much that many rows are better
+// behind one staging of it.  Four rows where the input is taken as it is (two where that leaves compute units without work): 2048 x 2048
+// 3.52 | 3.49 | 3.59 us with 2 | 4 | 8, 2048 x 8192 8.0 | 7.3 | 7.7, 256 x 2048 and 2048 x 256 4.96 | 4.80 | 5.20.  A norm's launch takes rounds of compute
+// units, a round of 2, 4, 8, 16 rows as 0.38, 0.6, 1, 1.9 (960 x 3072 behind a sum and a norm 5.2 | 4.2 | 4.6 | 5.5, 2624 x 3072 9.5 | 7.4 | 7.2 | 6.1, 5120 x
+// 3072 15.0 | 10.8 | 9.6 | 10.2): over eighty shapes of a mode this is 1 % off the best number in the mean.  The staged kernel: behind a sum and a norm 13312 x 2048
+// 11.8 | 12.7 us, x 3072 16.6 | 18.6, but 8192 x 2048 9.8 | 8.2, 5120 x 4096 12.2 | 11.3; behind a merge of eight splits 4096 x 3072 9.5 | 9.7, 2624 x 4096 9.6 |
+// 10.4, but 5120 x 2048 9.1 | 8.5, 2048 x 4096 7.7 | 7.0.
+static inline int skn_dense_once_rows(int mode, int rows, int parts, int units) {
+    const int64_t pieces = (int64_t)rows * parts;
+    if (mode == SKN_XSRC_PLAIN) return parts == 1 ? 8 : rows <= 2 * units ? 2 : 4;
+    if (mode == SKN_XSRC_MERGE) return pieces > 80 * units ? 0 : rows <= 4 * units ? 4 : 8;
+    if (mode == SKN_XSRC_ADD_NORM && pieces > 176 * units) return 0;
+    const float round_cost[4] = {0.38f, 0.6f, 1.0f, 1.9f};
+    int best = 0;
+    float least = INFINITY;
+    for (int i = 0; i < 4; i++) {
+        const int r = 2 << i;
+        const float rounds = (float)rows / (float)(r * units), cost = round_cost[i] * (0.7f * std::ceil(rounds) + 0.3f * rounds);
+        if (r <= 8 * parts && cost < least) best = r, least = cost;
+    }
+    return best;
+}
+
+static inline skn_dense_once skn_dense_once_plan(const skn_dense_call& c, int units) {
+    const int v = 16 / c.elem_bytes, pieces = (c.k_pad + 64 * v - 1) / (64 * v);  // elements of a request, 1 KiB pieces of a row
+    const int each = c.mode != SKN_XSRC_PLAIN || pieces <= kOnceParts ? 1 : pieces <= 2 * kOnceParts ? 2 : 4, parts = (pieces + each - 1) / each;
+    const skn_dense_once staged = {0, 0, 0};
+    if (c.second_input || parts > (c.mode == SKN_XSRC_PLAIN ? kOnceParts : kOnceParts / 2) || c.ld * c.elem_bytes >= (int64_t)1 << 30) return staged;
+    // The kernel has whole workgroups of rows, each of one segment: stacked as the projections of a matrix are, the first from its first
+    // row on.  (The staged kernel goes row by row, and leaves out what lies ahead of the first segment.)
+    if (c.rows % kDenseRowPad != 0) return staged;
+    for (int i = 0; i < c.nseg; i++)
+        if (c.row0[i] % kDenseRowPad != 0 || (i == 0 ? c.row0[0] != 0 : c.row0[i] <= c.row0[i - 1])) return staged;
+    // a head, a norm group takes whole requests of a lane
+    if (c.mode == SKN_XSRC_MERGE && c.dim % v != 0) return staged;
+    if (c.mode == SKN_XSRC_GROUP_NORM && (c.groups > kOnceGroups || (c.groups > 1 && c.k0 / c.groups % v != 0))) return staged;
+    if (c.mode == SKN_XSRC_ADD_NORM && c.groups != 1) return staged;
+    const int r = each > 1 ? 4 : skn_dense_once_rows(c.mode, c.rows, parts, units);
+    return r == 0 ? staged : skn_dense_once{parts, each, r};
 }

@@ -1,4 +1,4 @@
-"""CPU: which tile a dense product takes (csrc/dense_plan.h, which the library asks, compiled for the host)."""
+"""CPU: which kernel and tile a dense product takes (csrc/dense_plan.h, which the library asks, compiled for the host)."""
 import os
 import random
 import shutil
@@ -74,3 +74,28 @@ def test_few_outputs(plan, size, slices, rows):
     at, past, wide = _tiles(plan, [(size, 32, rows, k), (size, 32, rows + 32, k), (size, 33, rows, k)])
     assert at == K4 and past != K4 and wide != K4
     assert _tiles(plan, [(size, 32, 64, 7 * 128 // size)]) != [K4]
+
+
+PLAIN, NORM, MERGE, ADD_NORM = range(4)
+STAGED = (0, 0, 0)
+
+
+def _once(plan, mode=PLAIN, size=BF16, rows=2048, k=2048, ld=None, groups=1, dim=128, second=False, segments=(0,)):
+    return plan("once", [(mode, size, rows, k, ld or k, k, groups, dim, int(second), UNITS, len(segments), *segments)])[0]
+
+
+# a workgroup of the kernel that asks for everything at once has whole rows of one segment, and the segments cover the rows from the first on
+@pytest.mark.parametrize("mode", [PLAIN, NORM, MERGE, ADD_NORM])
+@pytest.mark.parametrize("rows,segments", [(2048 + 16, (0,)), (2048 + 1, ()), (2048, (32,)), (2048, (0, 1000)), (2048, (16, 1024)), (2048, (0, 1024, 512)), (2048, (0, 0))])
+def test_rows_that_are_not_stacked_as_projections_are_staged(plan, mode, rows, segments):
+    assert _once(plan, mode, rows=2048, segments=(0, 32, 1024)) != STAGED and _once(plan, mode, rows=2048, segments=()) != STAGED
+    assert _once(plan, mode, rows=rows, segments=segments) == STAGED
+
+
+@pytest.mark.parametrize("size", [BF16, F32])
+def test_rows_of_a_workgroup_divide_the_padding(plan, size):
+    calls = [(mode, size, rows, k, k, k, 1, 128, 0, UNITS, 1, 0) for mode in (PLAIN, NORM, MERGE, ADD_NORM) for rows in (32, 512, 2624, 8192, 32000)
+             for k in range(64, 40000, 192)]
+    for call, (parts, pieces, r) in zip(calls, plan("once", calls)):
+        if (parts, pieces, r) != STAGED:
+            assert 32 % r == 0 and parts <= (16 if call[0] == PLAIN else 8) and parts * pieces * 1024 >= call[3] * size
