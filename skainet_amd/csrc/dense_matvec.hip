@@ -241,9 +241,8 @@ __device__ __forceinline__ void stage_merge(const skn_matvec_src& s, const XPlan
 
 // W: uint16_t (bf16) or float.  LDS: two planes of `plane` float4, then the scratch of the staging.
 template <typename W, int MODE, int T>
-__global__ __launch_bounds__(T) void dense_matvec_kernel(const W* __restrict__ w, int rows, int k_pad, int ld, int plane,
-                                                         const float* __restrict__ bias, const skn_matvec_src src,
-                                                         const skn_dense_out out) {
+__device__ __forceinline__ void dense_matvec_rows(const W* __restrict__ w, int rows, int k_pad, int ld, int plane, const float* __restrict__ bias,
+                                                  const skn_matvec_src& src, const skn_dense_out& out) {
     extern __shared__ __align__(16) float4 lds4[];
     constexpr int V = 16 / (int)sizeof(W);
     const XPlanes xs = {lds4, lds4 + plane};
@@ -384,6 +383,21 @@ __global__ __launch_bounds__(T) void dense_matvec_kernel(const W* __restrict__ w
     }
 }
 
+template <typename W, int MODE, int T>
+__global__ __launch_bounds__(T) void dense_matvec_kernel(const W* __restrict__ w, int rows, int k_pad, int ld, int plane,
+                                                         const float* __restrict__ bias, const skn_matvec_src src,
+                                                         const skn_dense_out out) {
+    dense_matvec_rows<W, MODE, T>(w, rows, k_pad, ld, plane, bias, src, out);
+}
+
+// Behind a norm in groups the struct comes first, so that no argument arrives in registers (build.py): us of the other order | this one, 4096 x 5120
+// 11.5 | 10.9, 2624 x 5120 9.7 | 9.3, 4096 x 8192 16.6 | 16.1 (a merge is 4 % slower without: 4096 x 3072 9.6 | 10.1).
+template <typename W, int T>
+__global__ __launch_bounds__(T) void dense_matvec_norm_kernel(const skn_matvec_src src, const W* __restrict__ w, int rows, int k_pad, int ld, int plane,
+                                                              const float* __restrict__ bias, const skn_dense_out out) {
+    dense_matvec_rows<W, SKN_XSRC_GROUP_NORM, T>(w, rows, k_pad, ld, plane, bias, src, out);
+}
+
 // ---- every request at once ----------------------------------------------------------------------------------------------------
 // R rows to a workgroup; each of its wavefronts has PW pieces of 1 KiB of every one of them and the same pieces of the input in its
 // registers, so that the input passes neither LDS nor a barrier ahead of the products, and all that the workgroup reads is under way
@@ -392,7 +406,8 @@ __global__ __launch_bounds__(T) void dense_matvec_kernel(const W* __restrict__ w
 // first are single values, which the device hands a wavefront in registers (build.py), and those of an epilogue that is not taken are
 // not read.  us per launch in a captured graph, weights from memory, dense_matvec_kernel -> this: 2048 x 2048 4.85 -> 3.5, 256 x 2048
 // and 2048 x 256 together 8.8 -> 4.8, 2048 x 8192 8.9 -> 7.3, behind a norm 8192 x 2048 8.7 -> 7.5 and 32000 x 2048 24.8 -> 22.8, behind a sum and
-// a norm 2624 x 2048 6.8 -> 4.9; a bare read of 8.4 MB 2.95, of 33.6 MB 6.6.  Over 240 shapes 1.2 (merges) to 1.4 (norms) times as fast in the mean of a mode.
+// a norm 2624 x 2048 6.8 -> 4.9; a bare read of 8.4 MB 2.95, of 33.6 MB 6.6.  In the
+// mean of a mode 1.1 (merges of sixteen) to 1.27 (plain) times as fast, by shape in profiles/dense_matvec_once.md.
 struct OnceArgs {
     const float *add, *add_w;               // of a sum
     float* x_out;
@@ -426,10 +441,11 @@ struct LaneSums {
     static __device__ __forceinline__ int index(int i, int j) { return 4 * i + (j >> 1) + 2 * (j & 1); }
 };
 
-// W: uint16_t (bf16) or float.  X: 1, or 2 with a second input (SKN_XSRC_PLAIN); the most splits that are merged (SKN_XSRC_MERGE).
+// W: uint16_t (bf16) or float.  SP: the most splits that are merged (SKN_XSRC_MERGE).  parts: a merge keeps a hundred registers of partials, a
+// sum and norm four vectors, so that these have half as many wavefronts as a plain input.
 // parts_nseg: wavefronts of the workgroup, segments << 16.
 template <typename W, int MODE, int PW, int R, int SP>
-__global__ __launch_bounds__(64 * (MODE == SKN_XSRC_MERGE ? kOnceParts / 2 : kOnceParts)) void dense_matvec_once_kernel(
+__global__ __launch_bounds__(64 * (MODE == SKN_XSRC_PLAIN ? kOnceParts : kOnceParts / 2)) void dense_matvec_once_kernel(
     const float* __restrict__ x_in, const void* __restrict__ w, const float* __restrict__ bias, float* resid, int k, int row_bytes, int last_piece,
     uint32_t parts_nseg, int resid_rows, const float* __restrict__ norm_w, const OnceArgs args, const skn_dense_out out) {
     constexpr int V = 16 / (int)sizeof(W), Q = V / 4;
@@ -653,7 +669,7 @@ __global__ __launch_bounds__(64 * (MODE == SKN_XSRC_MERGE ? kOnceParts / 2 : kOn
 
     // ---- a row to sixteen threads ----
     for (int m = tid >> 4; m < R; m += 4 * parts) {
-        const bool first = m == tid >> 4;  // (the only turn but for a single wavefront of eight rows)
+        const bool first = m == tid >> 4;  // (the only turn unless there are more than four rows to a wavefront)
         const int row = row0 + m, r = row - sg.row0;
         float z = sum_of(sums[m]);
         if (one_norm) z *= 1.0f / sqrtf(sum_of(squares[0]) / (float)k + args.eps);
@@ -696,7 +712,7 @@ int launch_once(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src,
 // SKN_ERR_TYPE, without a message: not a call for dense_matvec_once_kernel
 template <typename W, int MODE>
 int try_once(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src, const skn_dense_out& out) {
-    skn_dense_call call = {MODE, (int)sizeof(W), w.rows, w.k_pad, w.ld ? w.ld : w.k_pad, src.k0, src.groups, src.dim, src.x1 != nullptr, out.nseg, {}};
+    skn_dense_call call = {MODE, (int)sizeof(W), w.rows, w.k_pad, w.ld ? w.ld : w.k_pad, src.k0, src.groups, src.dim, src.splits, src.x1 != nullptr, out.nseg, {}};
     for (int i = 0; i < out.nseg; i++) call.row0[i] = out.seg[i].row0;
     const skn_dense_once plan = skn_dense_once_plan(call, ctx->compute_units);
     const int r = plan.rows, parts = plan.parts;
@@ -741,7 +757,9 @@ int launch_threads(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& s
     // no more workgroups than fit on the device at once: a staging serves all the rows its wavefronts walk through
     const int groups = (w.rows + kR - 1) / kR;
     const int blocks = std::min((groups + kWaves - 1) / kWaves, std::min(per_cu, (int)(kMaxLds / lds)) * ctx->compute_units);
-    skn_launch(ctx, dense_matvec_kernel<W, MODE, T>, dim3((unsigned)blocks), dim3(T), lds, (const W*)w.w, w.rows, w.k_pad, w.ld ? w.ld : w.k_pad, plane, w.bias, src, out);
+    const int ld = w.ld ? w.ld : w.k_pad;
+    if constexpr (MODE == SKN_XSRC_GROUP_NORM) skn_launch(ctx, dense_matvec_norm_kernel<W, T>, dim3((unsigned)blocks), dim3(T), lds, src, (const W*)w.w, w.rows, w.k_pad, ld, plane, w.bias, out);
+    else skn_launch(ctx, dense_matvec_kernel<W, MODE, T>, dim3((unsigned)blocks), dim3(T), lds, (const W*)w.w, w.rows, w.k_pad, ld, plane, w.bias, src, out);
     SKN_LAUNCH_CHECK(ctx);
     return SKN_OK;
 }
@@ -769,8 +787,13 @@ int launch_mode(skn_ctx* ctx, const skn_dense_mat& w, const skn_matvec_src& src,
 
 template <typename W, int MODE>
 int allow_lds(skn_ctx* ctx) {
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)dense_matvec_kernel<W, MODE, 512>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
-    SKN_HIP(ctx, hipFuncSetAttribute((const void*)dense_matvec_kernel<W, MODE, 1024>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+    if constexpr (MODE == SKN_XSRC_GROUP_NORM) {
+        SKN_HIP(ctx, hipFuncSetAttribute((const void*)dense_matvec_norm_kernel<W, 512>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+        SKN_HIP(ctx, hipFuncSetAttribute((const void*)dense_matvec_norm_kernel<W, 1024>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+    } else {
+        SKN_HIP(ctx, hipFuncSetAttribute((const void*)dense_matvec_kernel<W, MODE, 512>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+        SKN_HIP(ctx, hipFuncSetAttribute((const void*)dense_matvec_kernel<W, MODE, 1024>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+    }
     return SKN_OK;
 }
 

@@ -70,7 +70,7 @@ enum { SKN_XSRC_PLAIN = 0, SKN_XSRC_GROUP_NORM = 1, SKN_XSRC_MERGE = 2, SKN_XSRC
 struct skn_dense_call {
     int mode, elem_bytes, rows, k_pad;
     int64_t ld;               // elements from row to row
-    int k0, groups, dim;      // columns of the input, norm groups, elements of a merged head
+    int k0, groups, dim, splits;  // columns of the input, norm groups, elements of a merged head, its splits
     bool second_input;
     int nseg;                 // segments and where they begin; 0: residual form
     int row0[8];
@@ -88,21 +88,25 @@ struct skn_dense_once {
 // behind one staging of it.  Four rows where the input is taken as it is (two where that leaves compute units without work): 2048 x 2048
 // 3.52 | 3.49 | 3.59 us with 2 | 4 | 8, 2048 x 8192 8.0 | 7.3 | 7.7, 256 x 2048 and 2048 x 256 4.96 | 4.80 | 5.20.  A norm's launch takes rounds of compute
 // units, a round of 2, 4, 8, 16 rows as 0.38, 0.6, 1, 1.9 (960 x 3072 behind a sum and a norm 5.2 | 4.2 | 4.6 | 5.5, 2624 x 3072 9.5 | 7.4 | 7.2 | 6.1, 5120 x
-// 3072 15.0 | 10.8 | 9.6 | 10.2): over eighty shapes of a mode this is 1 % off the best number in the mean.  The staged kernel: behind a sum and a norm 13312 x 2048
-// 11.8 | 12.7 us, x 3072 16.6 | 18.6, but 8192 x 2048 9.8 | 8.2, 5120 x 4096 12.2 | 11.3; behind a merge of eight splits 4096 x 3072 9.5 | 9.7, 2624 x 4096 9.6 |
-// 10.4, but 5120 x 2048 9.1 | 8.5, 2048 x 4096 7.7 | 7.0.
-static inline int skn_dense_once_rows(int mode, int rows, int parts, int units) {
+// 3072 15.0 | 10.8 | 9.6 | 10.2); more than two rounds of sixteen fp32 rows are better as eights (12000 x 1536 15.4 | 13.7, 16384 x 1536 19.4 | 18.4).
+// The staged kernel, us of it | of the other: behind a sum and a norm 13312 x 2048 11.8 | 12.7, x 3072 16.6 | 18.6, and from two rounds of sixteen bf16 rows on, each
+// of three pieces or more, 13312 x 1536 9.9 | 11.3, 9600 x 2048 10.5 | 11.2, but 8192 x 2048 10.2 | 8.9, 16384 x 1024 9.7 | 9.3; behind a merge of eight splits
+// 4096 x 3072 9.5 | 9.7, 2624 x 4096 9.6 | 10.4, but 5120 x 2048 9.1 | 8.5, 2048 x 4096 7.7 | 7.0; of sixteen, whose partials are twice as many, 2624 x 3072 9.6 | 11.1,
+// 5120 x 2048 9.8 | 10.7, but 8192 x 1024 8.8 | 8.2.  All shapes of profiles/dense_matvec_once.md, and those between, are within 3.5 % of the
+// staged kernel or faster (but 16384 x 3072 behind a norm, 18.9 | 19.6).
+static inline int skn_dense_once_rows(int mode, int elem_bytes, int rows, int parts, int splits, int units) {
     const int64_t pieces = (int64_t)rows * parts;
     if (mode == SKN_XSRC_PLAIN) return parts == 1 ? 8 : rows <= 2 * units ? 2 : 4;
-    if (mode == SKN_XSRC_MERGE) return pieces > 80 * units ? 0 : rows <= 4 * units ? 4 : 8;
-    if (mode == SKN_XSRC_ADD_NORM && pieces > 176 * units) return 0;
+    if (mode == SKN_XSRC_MERGE) return pieces > (splits > 8 && parts > 2 ? 60 : 80) * units ? 0 : rows <= 4 * units ? 4 : 8;
+    if (mode == SKN_XSRC_ADD_NORM && (pieces > 176 * units || (elem_bytes == 2 && parts > 2 && rows > 32 * units))) return 0;
     const float round_cost[4] = {0.38f, 0.6f, 1.0f, 1.9f};
     int best = 0;
     float least = INFINITY;
+    const int most = mode == SKN_XSRC_GROUP_NORM && elem_bytes == 4 && rows > 32 * units ? 8 : 16;
     for (int i = 0; i < 4; i++) {
         const int r = 2 << i;
         const float rounds = (float)rows / (float)(r * units), cost = round_cost[i] * (0.7f * std::ceil(rounds) + 0.3f * rounds);
-        if (r <= 8 * parts && cost < least) best = r, least = cost;
+        if (r <= 8 * parts && r <= most && cost < least) best = r, least = cost;
     }
     return best;
 }
@@ -121,6 +125,6 @@ static inline skn_dense_once skn_dense_once_plan(const skn_dense_call& c, int un
     if (c.mode == SKN_XSRC_MERGE && c.dim % v != 0) return staged;
     if (c.mode == SKN_XSRC_GROUP_NORM && (c.groups > kOnceGroups || (c.groups > 1 && c.k0 / c.groups % v != 0))) return staged;
     if (c.mode == SKN_XSRC_ADD_NORM && c.groups != 1) return staged;
-    const int r = each > 1 ? 4 : skn_dense_once_rows(c.mode, c.rows, parts, units);
+    const int r = each > 1 ? 4 : skn_dense_once_rows(c.mode, c.elem_bytes, c.rows, parts, c.splits, units);
     return r == 0 ? staged : skn_dense_once{parts, each, r};
 }

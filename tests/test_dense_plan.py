@@ -80,8 +80,8 @@ PLAIN, NORM, MERGE, ADD_NORM = range(4)
 STAGED = (0, 0, 0)
 
 
-def _once(plan, mode=PLAIN, size=BF16, rows=2048, k=2048, ld=None, groups=1, dim=128, second=False, segments=(0,)):
-    return plan("once", [(mode, size, rows, k, ld or k, k, groups, dim, int(second), UNITS, len(segments), *segments)])[0]
+def _once(plan, mode=PLAIN, size=BF16, rows=2048, k=2048, ld=None, groups=1, dim=128, splits=8, second=False, segments=(0,)):
+    return plan("once", [(mode, size, rows, k, ld or k, k, groups, dim, splits, int(second), UNITS, len(segments), *segments)])[0]
 
 
 # a workgroup of the kernel that asks for everything at once has whole rows of one segment, and the segments cover the rows from the first on
@@ -94,8 +94,29 @@ def test_rows_that_are_not_stacked_as_projections_are_staged(plan, mode, rows, s
 
 @pytest.mark.parametrize("size", [BF16, F32])
 def test_rows_of_a_workgroup_divide_the_padding(plan, size):
-    calls = [(mode, size, rows, k, k, k, 1, 128, 0, UNITS, 1, 0) for mode in (PLAIN, NORM, MERGE, ADD_NORM) for rows in (32, 512, 2624, 8192, 32000)
+    calls = [(mode, size, rows, k, k, k, 1, 128, 8, 0, UNITS, 1, 0) for mode in (PLAIN, NORM, MERGE, ADD_NORM) for rows in (32, 512, 2624, 8192, 32000)
              for k in range(64, 40000, 192)]
     for call, (parts, pieces, r) in zip(calls, plan("once", calls)):
         if (parts, pieces, r) != STAGED:
             assert 32 % r == 0 and parts <= (16 if call[0] == PLAIN else 8) and parts * pieces * 1024 >= call[3] * size
+
+
+# Rows of a workgroup at the rules' edges, each side the faster one of what was measured (profiles/dense_matvec_once.md).
+@pytest.mark.parametrize("mode,size,rows,k,splits,r", [
+    (PLAIN, BF16, 512, 4096, 1, 2), (PLAIN, BF16, 544, 4096, 1, 4), (PLAIN, BF16, 4096, 512, 1, 8), (PLAIN, BF16, 4096, 8192 + 64, 1, 4), (PLAIN, BF16, 32, 32768 + 64, 1, 0),
+    (NORM, BF16, 64, 2048, 1, 2), (NORM, BF16, 2048, 2048, 1, 8), (NORM, BF16, 4096, 2048, 1, 16), (NORM, BF16, 4096, 4096, 1, 16), (NORM, BF16, 4096, 4096 + 64, 1, 0),
+    (NORM, BF16, 12000, 3072, 1, 16), (NORM, F32, 8192, 1536, 1, 16), (NORM, F32, 12000, 1536, 1, 8), (NORM, F32, 4096, 2048 + 64, 1, 0),
+    (ADD_NORM, BF16, 8192, 2048, 1, 16), (ADD_NORM, BF16, 9600, 2048, 1, 0), (ADD_NORM, BF16, 13312, 1536, 1, 0), (ADD_NORM, BF16, 16384, 1024, 1, 16),
+    (ADD_NORM, BF16, 5632, 4096, 1, 8), (ADD_NORM, BF16, 5664, 4096, 1, 0), (ADD_NORM, F32, 9600, 1024, 1, 8), (ADD_NORM, F32, 12000, 1024, 1, 0),
+    (MERGE, BF16, 1024, 2048, 8, 4), (MERGE, BF16, 5120, 2048, 8, 8), (MERGE, BF16, 5152, 2048, 8, 0), (MERGE, BF16, 5120, 2048, 9, 0), (MERGE, BF16, 5120, 1536, 16, 8),
+    (MERGE, BF16, 2624, 3072, 16, 0), (MERGE, BF16, 8192, 1024, 16, 8), (MERGE, BF16, 2048, 4096 + 128, 8, 0)])
+def test_rows_of_a_workgroup(plan, mode, size, rows, k, splits, r):
+    assert _once(plan, mode, size, rows, k, splits=splits)[2] == r
+
+
+def test_what_only_the_staged_kernel_takes(plan):
+    assert _once(plan, PLAIN, second=True) == STAGED
+    assert _once(plan, NORM, groups=8)[2] and _once(plan, NORM, k=2304, groups=9) == STAGED
+    assert _once(plan, NORM, k=2064, groups=4) == STAGED and _once(plan, NORM, F32, k=2064 - 16, groups=4)[2]  # (516 elements: no whole requests of eight)
+    assert _once(plan, MERGE, dim=20, k=640) == STAGED and _once(plan, MERGE, F32, dim=20, k=640)[2]
+    assert _once(plan, PLAIN, ld=1 << 29) == STAGED
