@@ -918,8 +918,8 @@ constexpr int kTlLds = 3 * kTlStage + 2 * kTlAux + 128 * 4 + 256 * 4;
 // consumer's column blocks 0, 1 and 2, 3 meet lane by lane in the store -- and stores silu(gate) * up in bf16.
 // TAIL: the last tiles are shared by tail.splits workgroups each, neighbours in the grid, with a part of k each (a template
 // parameter: grids without such tiles were 0.5 us slower at 512 x 14336 x 4096 for the division).
-// CB: column blocks of 32 in a tile.  Three (256 x 96) where they make one round of compute units that four leave a quarter and more of
-// idle (a loop of 96 columns takes 0.83 of the time of one of 128, bound by the same phases: q, k and v of 512 x 4096 in 12288 columns 73.2 -> 60.8
+// CB: column blocks of 32 in a tile.  Three (256 x 96) where their rounds of compute units cost less than those of four (a loop of 96 columns takes
+// 0.83 of the time of one of 128, bound by the same phases: q, k and v of 512 x 4096 in 12288 columns 73.2 -> 60.8
 // us, 704 -> 848 TFLOP/s; 2000 x 2048 in 3072 41.3 -> 35.9); tile0 and n_tiles count blocks of 32 there, so that a tile may hold the end of one matrix and the start of the next, and the
 // fourth producer only keeps the barriers.
 template <bool TAIL, int CB>
@@ -2444,7 +2444,10 @@ int skn_gemm_q4k_multi(skn_ctx* ctx, const skn_gemm_seg* segs, int nseg, int k, 
                                     (ctx->opt_gemm_tile == 0 && m > 128 && 3 * tall_tiles >= 2 * tall_rounds * ctx->compute_units));
     TallTail tail = {tall_tiles, 0, 1, nullptr};
     if (tall) tail = tall_tail(ctx, tall_tiles, k / 256);
-    // 96 columns where they save a round's worth by more than they cost: only what has no last tiles to share (their sums' chains would grow)
+    // 96 columns where their rounds, at 0.85 of the time of one of 128 columns, are the shorter: one round where 128 columns leave a quarter and more of
+    // it idle, and with rows of less than eight superblocks two against two, three against three or seven against six (us of 128 | of 96: 1024 x 11264 x 1024
+    // 47.8 | 42.6, 1024 x 12288 x 512 35.1 | 31.2, 768 x 24000 x 1536 92.0 | 81.0, 2048 x 20608 x 1792 201 | 192; three against two, not taken: 700 x 16384 x
+    // 1024 47.9 | 56.1).  Only what has no last tiles to share (their sums' chains would grow).
     const int narrow_tiles = ((m + 255) / 256) * ((blocks + 2) / 3), narrow_rounds = (narrow_tiles + ctx->compute_units - 1) / ctx->compute_units;
     const bool narrow = tall && !swiglu_pair && (ctx->opt_gemm_tile == 4 || (ctx->opt_gemm_tile == 0 && tail.tiles == 0 && 17 * narrow_rounds < 20 * tall_rounds));
     if (narrow) tail = TallTail{narrow_tiles, 0, 1, nullptr};

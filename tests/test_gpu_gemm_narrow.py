@@ -51,11 +51,12 @@ def test_tiles_that_hold_the_columns_of_two_and_three_matrices(hip, case):
     assert conditioned.logit_err(_with_tile(hip, 4, logits), first) <= conditioned.PROMPT_TOL
 
 
-# (rows, columns) whose 256 x 128 tiles are 192 and 193 of 256 compute units: one round of 96-column tiles and not
-@pytest.mark.parametrize("n,narrow", [(12288, True), (12288 + 32, False)])
-def test_where_the_library_picks_them(hip, n, narrow):
+# Tiles of 256 x 128 and of 256 x 96 for 256 compute units: 192 and 256, one round each; 194 and 258, one and two; 352 and 472, two each (short rows, whose last
+# tiles are not shared); 388 and 516, two and three; 564 and 750, three each; 1288 and 1720, six and seven.
+@pytest.mark.parametrize("m,n,k,narrow", [(512, 12288, 256, True), (512, 12288 + 32, 256, False), (1024, 11264, 1024, True), (1024, 12288 + 32, 512, False), (768, 24000, 512, True),
+                                          (2048, 20608, 256, True)])
+def test_where_the_library_picks_them(hip, m, n, k, narrow):
     assert hip.device_info()["compute_units"] == 256, "the widths are chosen for 256 compute units"
-    m, k = 512, 256
     raw, a = synth.weight(Q4_K, n, k, seed=5), synth.activation_bf16((m, k), seed=6)
 
     def product(tile):
@@ -64,6 +65,6 @@ def test_where_the_library_picks_them(hip, n, narrow):
         return got, hip.stat("workgroups") - before
 
     (got, took), (wide, wide_took), (_, narrow_took) = product(0), product(3), product(4)
-    assert narrow_took - wide_took == 2 * (-(-n // 96) - -(-n // 128))
+    assert narrow_took - wide_took == -(-m // 256) * (-(-n // 96) - -(-n // 128))
     assert took == (narrow_took if narrow else wide_took)
     assert np.array_equal(wide.view(np.uint32), got.view(np.uint32))
