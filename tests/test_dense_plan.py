@@ -6,6 +6,8 @@ import subprocess
 
 import pytest
 
+import test_gpu_dense_once as steps
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 UNITS = 256
 BF16, F32 = 2, 4
@@ -59,9 +61,10 @@ def test_fp32_and_short_rows(plan, shape, tile):
     assert _tiles(plan, [shape]) == [tile]
 
 
-# one measured shape for each tile that is the fastest of all there (profiles/dense_gemm_tiles.md)
+# one measured shape for each tile that is the fastest of all there (profiles/dense_gemm_tiles.md), and those of test_gpu_dense_split.py
 @pytest.mark.parametrize("m,rows,k,tile", [(333, 5120, 512, 0), (200, 5120, 4096, 1), (2048, 4096, 8192, 2), (1500, 8192, 4096, 3), (512, 18496, 4096, 5),
-                                           (512, 10752, 4096, 6), (512, 8192, 8192, 7)])
+                                           (512, 10752, 4096, 6), (512, 8192, 8192, 7), (2048, 2048, 4160, 7), (1000, 2048, 4160, 1), (100, 2048, 4160, K4),
+                                           (2048, 4224, 2048, 5), (1000, 4224, 2048, 2), (100, 4224, 2048, 0)])
 def test_bf16_by_the_fitted_costs(plan, m, rows, k, tile):
     assert _tiles(plan, [(BF16, m, rows, k)]) == [tile]
 
@@ -120,3 +123,26 @@ def test_what_only_the_staged_kernel_takes(plan):
     assert _once(plan, NORM, k=2064, groups=4) == STAGED and _once(plan, NORM, F32, k=2064 - 16, groups=4)[2]  # (516 elements: no whole requests of eight)
     assert _once(plan, MERGE, dim=20, k=640) == STAGED and _once(plan, MERGE, F32, dim=20, k=640)[2]
     assert _once(plan, PLAIN, ld=1 << 29) == STAGED
+
+
+def _pad(n, to):
+    return -(-n // to) * to
+
+
+@pytest.mark.parametrize("size", [BF16, F32])
+def test_what_the_decode_steps_of_the_gpu_tests_reach(plan, size):
+    """The lists of test_gpu_dense_once.py have every form of the kernel that asks for everything at once, and the staged one for each input."""
+    def forms(mode, products, **how):
+        out = set()
+        for n, k, groups, dim, splits in products:
+            parts, pieces, r = _once(plan, mode, size, _pad(n, 32), _pad(k, 64), groups=groups, dim=dim, splits=splits)
+            out.add((pieces, r) if mode == PLAIN else (min(s for s in (2, 4, 8, 16) if splits <= s), r) if mode == MERGE and r else r)
+        return out
+
+    rows = {0, 2, 4, 8, 16}
+    assert forms(PLAIN, [(w, ff, 1, 1, 1) for w, ff, _ in steps.WIDTHS] + [(min(w, 100), w, 1, 1, 1) for w, _, _ in steps.WIDTHS]) >= {(1, 2), (1, 4), (1, 8), (2, 4), (4, 4)}
+    assert forms(ADD_NORM, [(v, w, 1, 1, 1) for w, _, v in steps.WIDTHS]) >= rows
+    assert forms(NORM, [(ff, w, 1, 1, 1) for w, ff, _ in steps.WIDTHS]) >= rows
+    assert forms(NORM, [(v, w, g, 1, 1) for w, g, v in steps.GROUPS]) >= rows
+    merged = [(w, h * d, 1, d, s) for h, _, d, w, _, s in steps.MERGES if s > 1]
+    assert forms(MERGE, merged) >= {0, (2, 4), (4, 4), (4, 8), (8, 4), (16, 4), (16, 8)}

@@ -5,7 +5,7 @@ import pytest
 
 import test_gpu_prompt_norm as prompt_norm
 from oracle import oracle_c, oracle_np
-from skainet_amd import llama, synth
+from skainet_amd import synth
 
 pytestmark = pytest.mark.gpu
 Q4_K, Q6_K = synth.Q4_K, synth.Q6_K
@@ -21,19 +21,20 @@ def test_rows_do_not_depend_on_how_many_a_workgroup_has(hip, m, k):
     hip.set_option("gemm.split", 1)
     hip.set_option("gemm.few", 0)
     try:
+        before = hip.stat("workgroups")
         got = hip.gemm_q_host(Q4_K, raw, n, k, a, m)
+        took = hip.stat("workgroups") - before
         want = np.concatenate([hip.gemm_q_host(Q4_K, raw, n, k, np.ascontiguousarray(a[i:i + 256]), len(a[i:i + 256])) for i in range(0, m, 256)])
     finally:
         hip.set_option("gemm.tile", 0)
         hip.set_option("gemm.split", 0)
         hip.set_option("gemm.few", 1)
+    rows = -(-m // 128) * 128
+    assert took == rows // (4 if k <= 12288 else 2) + rows // 128  # (the pass and the tiles)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
     assert oracle_np.rel_err(hip.gemm_q_host(Q6_K, synth.weight(Q6_K, n, k, seed=k), n, k, a, m), oracle_c.gemm_q(Q6_K, synth.weight(Q6_K, n, k, seed=k), n, k, a, m)) <= 1e-3
 
 
 @pytest.mark.parametrize("hidden", [1280, 4096])
-def test_rows_behind_a_norm_round_as_few_rows_do(hip, monkeypatch, hidden):
-    config, prefill = llama.Config, llama.LlamaModel.prefill
-    monkeypatch.setattr(llama, "Config", lambda **kw: config(**{**kw, "max_tokens": 1008}))
-    monkeypatch.setattr(llama.LlamaModel, "prefill", lambda self, tokens: prefill(self, tokens[:1] * 1000))
-    prompt_norm.test_rows_behind_a_norm_round_as_two_wavefronts_sum_them(hip, hidden)
+def test_rows_behind_a_norm_round_as_few_rows_do(hip, hidden):
+    prompt_norm.check_rounding(hip, hidden, tokens=1000, max_tokens=1008)

@@ -47,9 +47,8 @@ def _one_hot_q4k(rows, k, places):
     return w.reshape(-1)
 
 
-@pytest.mark.parametrize("hidden", [1280, 4096, 5120])
-def test_rows_behind_a_norm_round_as_two_wavefronts_sum_them(hip, hidden):
-    """Norm weights for which one bit of the sum decides bf16 roundings, through a layer of one-hot matrices: values, attention over two
+def check_rounding(hip, hidden, tokens, max_tokens):
+    """Norm weights for which one bit of the sum decides bf16 roundings, through a layer of one-hot matrices: values, attention over
     equal tokens, residual, head.  Elements of odd places in the rounding, others beside them as a measure."""
     rng, probes = np.random.default_rng(hidden), 32
     for _ in range(1000):  # (squares of eleven bits and their pairs are exact: only the order of the sums rounds)
@@ -69,7 +68,7 @@ def test_rows_behind_a_norm_round_as_two_wavefronts_sum_them(hip, hidden):
             g[e] = tries[np.argmin(here)]
     assert decided >= 8
     value = _bf16(x[at] * two * g[at])
-    cfg = llama.Config(n_layer=1, hidden=hidden, ffn=256, n_head=hidden // 128, n_kv_head=1, head_dim=128, vocab=probes, max_tokens=16, page_tokens=16,
+    cfg = llama.Config(n_layer=1, hidden=hidden, ffn=256, n_head=hidden // 128, n_kv_head=1, head_dim=128, vocab=probes, max_tokens=max_tokens, page_tokens=16,
                        rms_eps=EPS, type_embd=0, type_head=0)
     ones, q4 = np.ones(hidden, F32), synth.Q4_K
     head = np.zeros((probes, hidden), F32)
@@ -81,7 +80,7 @@ def test_rows_behind_a_norm_round_as_two_wavefronts_sum_them(hip, hidden):
          "l0.wo": (q4, _one_hot_q4k(hidden, hidden, [(e, j) for j, e in enumerate(at)])), "l0.w_gate": (q4, short), "l0.w_up": (q4, short), "l0.w_down": (q4, short),
          "l0.attn_norm": (None, g), "l0.ffn_norm": (None, ones)}
     model = llama.LlamaModel(hip, cfg, weights=w)
-    model.prefill([0, 0])
+    model.prefill([0] * tokens)
     got = model.logits()
     model.free()
     y = x.astype(np.float64)
@@ -89,3 +88,8 @@ def test_rows_behind_a_norm_round_as_two_wavefronts_sum_them(hip, hidden):
     want = y[at] / np.sqrt(np.mean(y * y) + EPS)
     # a rounding the other way moves its element by a part in 512 at least (and the norm, if all go that way, by half as much)
     assert np.all(np.abs(got - want) <= 2.0**-12 * np.abs(want)), np.abs(got / want - 1).max()
+
+
+@pytest.mark.parametrize("hidden", [1280, 4096, 5120])
+def test_rows_behind_a_norm_round_as_two_wavefronts_sum_them(hip, hidden):
+    check_rounding(hip, hidden, tokens=2, max_tokens=16)
