@@ -33,7 +33,8 @@ FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc", "-Wall", "-Wno-unused-function",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # the first sixteen dwords of a kernel's arguments are in scalar registers when a wavefront starts (single values up to the first struct), a
-    # load's latency less ahead of its first request: 0.3 us of a launch of 8 MB
+    # load's latency less ahead of its first request: a Q4_K matvec of 4096 x 4096 in a captured graph 4.45 -> 4.13 us from memory, 3.22 -> 3.15 where
+    # its matrix is in a cache
     "-mllvm", "-amdgpu-kernarg-preload-count=16",
 ]
 

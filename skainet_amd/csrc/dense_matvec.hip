@@ -18,14 +18,12 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// Workgroups of T threads of the staged kernel (figures of calls that dense_matvec_once_kernel takes now too: the rule is from before it).  Eight
-// wavefronts where that makes at most a workgroup per compute unit (a matrix of 2048 rows reaches 256
-// of them, with sixteen wavefronts half: 5.5 against 5.9 us at 2048 rows, 4.8 against 5.2 at 1024), and behind a norm where the rows
-// fill the device twice (4288 rows 13.0 against 14.5 us, 6016 rows 14.0 against 15.3) or are a single turn of requests long (3232 rows
-// of 2048 7.95 against 8.34 us), up to three per compute unit.  Sixteen, one workgroup per compute unit, for what lies between, where
-// the compute units with two workgroups of eight would be the last (2560 rows of 14000 16.6 against 18.8 us, of 6000 8.2 against 9.1;
-// behind a norm 2624 rows of 2560 8.0 against 8.5, 3232 rows of 4096 9.9 against 11.0), and for more rows behind a plain staging
-// (6144 rows 6.7 against 7.1).
+// Workgroups of T threads of the staged kernel, us of eight wavefronts | of sixteen.  Eight where that makes at most a workgroup per compute unit (two inputs 1344 x 8192
+// 7.7 | 9.4, 2048 x 8192 9.3 | 10.3), and behind a norm where the rows fill the device twice (13312 x 5120 25.5 | 27.0, behind a sum too 18496 x 2048 15.1 | 16.2) or
+// are a single turn of requests long, up to three per compute unit.  Sixteen, one workgroup per compute unit, for what lies between, where the compute units with two
+// workgroups of eight would be the last (two inputs 2624 x 8192 11.9 | 11.3; behind a norm 2624 x 5120 10.4 | 9.4, 4096 x 5120 11.7 | 10.9), and for more rows
+// behind a plain staging (6432 x 2048 7.8 | 7.5).  Over 831 calls that it gets, by type and input, 1.00 to 1.02 times the better one's time in the mean, at worst 1.22 (two
+// inputs 5120 x 8192 17.2 | 21.0: where sixteen leave a turn nearly empty).
 constexpr int kPerCu = 3;
 constexpr int kR = 1;  // rows per wavefront and turn (measured with two as well: slower)
 constexpr int kU = 4;  // 16-byte pieces per row and lane in flight, twice
@@ -42,8 +40,8 @@ struct XPlanes {
 // the input came no sooner than they did, and each vector that was asked for when it was needed cost another round trip before the
 // first multiplication.  Quads tid, tid + T, ... up to RQ; longer inputs read the rest as they go.  us, before -> now: 8192 x 2048 behind a
 // norm 10.2 -> 9.4, behind a sum and a norm 12.4 -> 10.9, 2624 x 2048 8.0 -> 7.2, 2048 x 2048 5.2 -> 4.6; a decode step of six layers of width
-// 2048 with side tables 15 us less, of eight with a delta rule 10 us less.  (The partials of a merge too, or the input of the columns beside
-// a mixer: 0.4 and 1.1 us more.)
+// 2048 with side tables 15 us less, of eight with a delta rule 10 us less (taken before dense_matvec_once_kernel, which has these calls now and does the
+// same for all that it reads).  (The partials of a merge too, or the input of the columns beside a mixer: 0.4 and 1.1 us more.)
 template <int MODE, int T>
 struct Ahead {
     static constexpr bool kAdd = MODE == SKN_XSRC_ADD_NORM, kNorm = MODE == SKN_XSRC_GROUP_NORM || kAdd, kPlain = MODE == SKN_XSRC_PLAIN;
@@ -404,10 +402,10 @@ __global__ __launch_bounds__(T) void dense_matvec_norm_kernel(const skn_matvec_s
 // before it waits for anything.  A factor of the whole input (one norm group) goes to the results; the wavefronts' sums meet in LDS, sixteen
 // threads end a row.  What a launch of a few megabytes costs beside its bytes is dependent steps: arguments that are needed
 // first are single values, which the device hands a wavefront in registers (build.py), and those of an epilogue that is not taken are
-// not read.  us per launch in a captured graph, weights from memory, dense_matvec_kernel -> this: 2048 x 2048 4.85 -> 3.5, 256 x 2048
-// and 2048 x 256 together 8.8 -> 4.8, 2048 x 8192 8.9 -> 7.3, behind a norm 8192 x 2048 8.7 -> 7.5 and 32000 x 2048 24.8 -> 22.8, behind a sum and
-// a norm 2624 x 2048 6.8 -> 4.9; a bare read of 8.4 MB 2.95, of 33.6 MB 6.6.  In the
-// mean of a mode 1.1 (merges of sixteen) to 1.27 (plain) times as fast, by shape in profiles/dense_matvec_once.md.
+// not read.  us per launch in a captured graph, weights from memory, dense_matvec_kernel -> this: 2048 x 2048 4.95 -> 3.73, 256 x 2048
+// 3.42 -> 2.71, 2048 x 8192 9.0 -> 7.6, behind a norm 8192 x 2048 8.8 -> 7.9 and 32000 x 2048 24.3 -> 22.4, behind a sum and
+// a norm 2624 x 2048 6.6 -> 4.8; a bare read of 8.4 MB 2.95, of 33.6 MB 6.6.  In the
+// mean of a mode 1.11 (merges of sixteen) to 1.27 (plain) times as fast in bf16, 1.06 to 1.26 in fp32 (profiles/dense_matvec_once.md).
 struct OnceArgs {
     const float *add, *add_w;               // of a sum
     float* x_out;
