@@ -33,6 +33,13 @@ static inline int skn_dense_tile(int elem_bytes, int m, int rows, int k_pad, int
         {64, 64, 3, 8.2f, {28.6f, 38.8f, 35.4f}, 0.8f}, {128, 64, 2, 10.3f, {33.f, 51.8f}, 3.6f}, {128, 128, 2, 8.6f, {65.9f, 62.f}, 5.5f},
         {256, 256, 1, 12.2f, {88.3f}, 22.7f},           {0, 0, 0, 0.f, {0.f}, 0.f},               {256, 192, 1, 13.f, {60.1f}, 21.5f},
         {128, 192, 2, 20.6f, {47.f, 55.8f}, 8.9f},      {128, 128, 1, 7.7f, {49.8f}, 5.f}};
+    // Rows of 8192 and more, fitted to 160 shapes (40 to 8192 tokens, 256 to 18496 rows, k to 18432): a long loop takes up to 1.5 times as long a piece of k in the
+    // larger tiles as the costs above have it.  us, by those | by these: 2048 x 4096 x 18432 408 | 333, x 10240 239 | 199, 4096 x 2048 x 10240 232 | 198, 8192 x 4096 x
+    // 8192 555 | 479; 1.003 times the best one's time in the mean of 100 shapes that the fit above never saw.
+    static const skn_dense_tile_cost longer[8] = {
+        {64, 64, 3, 2.4f, {22.2f, 31.3f, 41.7f}, 0.f}, {128, 64, 2, 0.f, {27.5f, 44.3f}, 3.9f}, {128, 128, 2, 0.f, {53.9f, 68.6f}, 1.4f},
+        {256, 256, 1, 0.f, {84.4f}, 69.4f},            {0, 0, 0, 0.f, {0.f}, 0.f},              {256, 192, 1, 0.f, {73.6f}, 44.9f},
+        {128, 192, 2, 0.f, {62.3f, 81.8f}, 7.4f},      {128, 128, 1, 0.f, {43.1f}, 7.1f}};
     // fp32, and shorter rows: of the loop alone, in relative units.  An fp32 loop takes sixteen times as long, so that launches and stores are
     // nothing beside it, and in rows of less than 512 elements it is not what the fit above saw.  us at fp32, by the fitted costs | by these: 1000 x 8512 x 2048
     // 515 | 339, 954 x 8512 x 2048 485 | 282, 512 x 18496 x 2048 489 | 391, 1700 x 10752 x 2048 976 | 692, 2048 x 10752 x 2048 977 | 727, 1000 x 18496 x 512
@@ -41,7 +48,7 @@ static inline int skn_dense_tile(int elem_bytes, int m, int rows, int k_pad, int
         {64, 64, 3, 0.f, {25.f, 40.f, 40.f}, 0.f}, {128, 64, 2, 0.f, {31.f, 48.f}, 0.f}, {128, 128, 2, 0.f, {59.f, 87.f}, 0.f},  {256, 256, 1, 0.f, {145.f}, 0.f},
         {0, 0, 0, 0.f, {0.f}, 0.f},                {256, 192, 1, 0.f, {116.f}, 0.f},     {128, 192, 2, 0.f, {80.f, 118.f}, 0.f}, {128, 128, 0, 0.f, {0.f}, 0.f}};
     const bool known = elem_bytes == 2 && k_pad >= 512;
-    const skn_dense_tile_cost* costs = known ? fitted : loops;
+    const skn_dense_tile_cost* costs = !known ? loops : k_pad < 8192 ? fitted : longer;
     const float length = known ? (float)k_pad / 4096.f : 1.f;
     int best = 0;
     float best_time = INFINITY;

@@ -64,7 +64,9 @@ def test_fp32_and_short_rows(plan, shape, tile):
 # one measured shape for each tile that is the fastest of all there (profiles/dense_gemm_tiles.md), and those of test_gpu_dense_split.py
 @pytest.mark.parametrize("m,rows,k,tile", [(333, 5120, 512, 0), (200, 5120, 4096, 1), (2048, 4096, 8192, 2), (1500, 8192, 4096, 3), (512, 18496, 4096, 5),
                                            (512, 10752, 4096, 6), (512, 8192, 8192, 7), (2048, 2048, 4160, 7), (1000, 2048, 4160, 1), (100, 2048, 4160, K4),
-                                           (2048, 4224, 2048, 5), (1000, 4224, 2048, 2), (100, 4224, 2048, 0)])
+                                           (2048, 4224, 2048, 5), (1000, 4224, 2048, 2), (100, 4224, 2048, 0),
+                                           (2048, 4096, 10240, 2), (2048, 4096, 18432, 2), (4096, 2048, 10240, 2), (8192, 4096, 8192, 3), (4096, 6432, 8192, 3),
+                                           (1000, 10752, 10240, 6), (512, 18496, 14336, 5), (2048, 2048, 10240, 7)])
 def test_bf16_by_the_fitted_costs(plan, m, rows, k, tile):
     assert _tiles(plan, [(BF16, m, rows, k)]) == [tile]
 
