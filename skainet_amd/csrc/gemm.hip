@@ -470,9 +470,10 @@ void launch_prep(skn_ctx* ctx, const skn_gemm_src& src, _Float16* afrag, float* 
     // (m_pad is a multiple of 32: the pair count divides by the eight XCDs its workgroups are dealt to)
     // Four rows a workgroup where those fill the device, without a norm to wait for half of it (two rows | four, us: 333 x 4096 7.1 | 7.3, 512 x 4096
     // 7.2 | 7.0, behind a norm 7.4 | 7.9, 2000 x 2048 behind a norm 10.9 | 8.4, 333 x 11008 10.4 | 11.8, 512 x 11008 10.8 | 10.2, 1000 x 11008
-    // 14.3 | 11.4), and what their registers hold: up to 4096 elements behind a norm, 12288 otherwise.
+    // 14.3 | 11.4), and what their registers hold: up to 4096 elements behind a norm, 12288 otherwise.  Not rows of less than 1024, which leave lanes without any
+    // (whole products of Q4_K: 8192 x 256 x 256 17.8 | 20.9, 8192 x 1024 x 512 28.0 | 31.1, 4096 x 2048 x 512 24.2 | 25.6; at k = 1024 within 3 % or faster).
     constexpr int kPlain = SRC == SKN_SRC_RMSNORM ? SKN_SRC_F32 : SRC;  // (the wider forms have no norm: not reached with one)
-    if (m_pad % 32 == 0 && m_pad / 4 >= ctx->compute_units / (SRC == SKN_SRC_RMSNORM ? 1 : 2) && k <= (SRC == SKN_SRC_RMSNORM ? 4096 : 12288)) {
+    if (k >= 1024 && m_pad % 32 == 0 && m_pad / 4 >= ctx->compute_units / (SRC == SKN_SRC_RMSNORM ? 1 : 2) && k <= (SRC == SKN_SRC_RMSNORM ? 4096 : 12288)) {
         const dim3 grid(m_pad / 4);
         if (k <= 2048) skn_launch(ctx, prep_a_quads_kernel<2, SRC, SUMS, 128>, grid, dim3(512), 0, src, afrag, isc, sfrag, m, k);
         else if (k <= 4096) skn_launch(ctx, prep_a_quads_kernel<4, SRC, SUMS, 128>, grid, dim3(512), 0, src, afrag, isc, sfrag, m, k);
