@@ -307,6 +307,7 @@ int skn_dense_gemm(skn_ctx* ctx, const skn_dense_mat& w, const void* a, int lda,
     SKN_REQUIRE(ctx, w.w && a && m > 0 && w.rows > 0 && w.rows % kDenseRowPad == 0 && w.k_pad > 0 && w.k_pad % kDenseColPad == 0, SKN_ERR_ARG,
                 "dense GEMM: bad shape (%d tokens, %d x %d)", m, w.rows, w.k_pad);
     SKN_REQUIRE(ctx, lda >= w.k_pad && lda % kDenseColPad == 0, SKN_ERR_SHAPE, "dense GEMM: activation pitch %d for %d columns", lda, w.k_pad);
+    SKN_REQUIRE(ctx, skn_dense_pitch_ok(w.type == SKN_TYPE_F32 ? 4 : 2, lda), SKN_ERR_SHAPE, "dense GEMM: rows of %d elements are too long", lda);
     SKN_REQUIRE(ctx, (((uintptr_t)w.w | (uintptr_t)a) & 15) == 0, SKN_ERR_ARG, "dense GEMM: operands must be 16-byte aligned");
     SKN_REQUIRE(ctx, out.nseg >= 0 && out.nseg <= kDenseMaxSegs && (out.nseg > 0 || out.resid), SKN_ERR_ARG, "dense GEMM: no output");
     for (int i = 0; i < out.nseg; i++)

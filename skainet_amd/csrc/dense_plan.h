@@ -17,6 +17,9 @@ enum {
     SKN_TILE_128x128_K2 = 7  // k divided in two
 };
 
+// Whether 32-bit offsets reach every element of a tile's rows (256 at most) whose pitch is `pitch` elements.
+static inline bool skn_dense_pitch_ok(int elem_bytes, int64_t pitch) { return pitch * elem_bytes * 256 <= INT32_MAX; }
+
 // A shape's time: of a launch, of the loop over k = 4096 with one, two or three tiles on a compute unit, and of the store of a tile to each.
 struct skn_dense_tile_cost {
     int rows_a, rows_w, resident;  // resident 0: not chosen by its cost

@@ -1,5 +1,6 @@
 // Answers what a dense product would take, a line for each line read:
 //   tile bytes m rows k units                                                          -> the tile
+//   pitch bytes elements                                                               -> whether the GEMM's offsets reach all of a tile
 //   once mode bytes rows k_pad ld k0 groups dim splits second_input units segments row0 .. -> wavefronts, pieces each, rows of a workgroup (0: staged)
 #include <cstdio>
 #include <cstring>
@@ -17,6 +18,8 @@ int main() {
     while (std::scanf("%15s", what) == 1) {
         if (std::strcmp(what, "tile") == 0 && read(v, 5)) {
             std::printf("%d\n", skn_dense_tile(v[0], v[1], v[2], v[3], v[4]));
+        } else if (std::strcmp(what, "pitch") == 0 && read(v, 2)) {
+            std::printf("%d\n", (int)skn_dense_pitch_ok(v[0], v[1]));
         } else if (std::strcmp(what, "once") == 0 && read(v, 12) && v[11] >= 0 && v[11] <= 8) {
             skn_dense_call c = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9] != 0, v[11], {}};
             if (!read(c.row0, c.nseg)) return 1;

@@ -81,6 +81,13 @@ def test_few_outputs(plan, size, slices, rows):
     assert _tiles(plan, [(size, 32, 64, 7 * 128 // size)]) != [K4]
 
 
+def test_pitches_whose_tiles_need_more_than_32_bit_offsets_are_refused(plan):
+    """(the kernel's offsets from a tile's first row: 255 rows and the row's own bytes)"""
+    for size in (BF16, F32):
+        most = (2**31 - 1) // (256 * size)
+        assert plan("pitch", [(size, 64), (size, 40064), (size, most), (size, most + 1)]) == [(1,), (1,), (1,), (0,)]
+
+
 PLAIN, NORM, MERGE, ADD_NORM = range(4)
 STAGED = (0, 0, 0)
 
