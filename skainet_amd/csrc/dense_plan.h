@@ -95,10 +95,12 @@ struct skn_dense_once {
 };
 
 // Rows of a workgroup whose `parts` wavefronts share `rows` rows; 0: the input takes so much that many rows are better
-// behind one staging of it.  Four rows where the input is taken as it is (two where that leaves compute units without work): 2048 x 2048
-// 3.52 | 3.49 | 3.59 us with 2 | 4 | 8, 2048 x 8192 8.0 | 7.3 | 7.7, 256 x 2048 and 2048 x 256 4.96 | 4.80 | 5.20.  A norm's launch takes rounds of compute
-// units, a round of 2, 4, 8, 16 rows as 0.38, 0.6, 1, 1.9 (960 x 3072 behind a sum and a norm 5.2 | 4.2 | 4.6 | 5.5, 2624 x 3072 9.5 | 7.4 | 7.2 | 6.1, 5120 x
-// 3072 15.0 | 10.8 | 9.6 | 10.2); more than two rounds of sixteen fp32 rows are better as eights (12000 x 1536 15.4 | 13.7, 16384 x 1536 19.4 | 18.4).
+// behind one staging of it.  (Figures of one comparison are of one sweep; two sweeps differ by boxes and by what a cache holds.)
+// Four rows where the input is taken as it is (two where that leaves compute units without work): 2048 x 2048 3.52 | 3.49 | 3.59 us
+// with 2 | 4 | 8, 2048 x 8192 8.0 | 7.3 | 7.7, 256 x 2048 and 2048 x 256 4.96 | 4.80 | 5.20.  A norm's launch takes rounds of compute
+// units, a round of 2, 4, 8, 16 rows as 0.38, 0.6, 1, 1.9 (960 x 3072 behind a sum and a norm 5.2 | 4.2 | 4.6 | 5.5, 2624 x 3072
+// 9.5 | 7.4 | 7.2 | 6.1, 5120 x 3072 15.0 | 10.8 | 9.6 | 10.2); more than two rounds of sixteen fp32 rows are better as eights
+// (12000 x 1536 15.4 | 13.7, 16384 x 1536 19.4 | 18.4).
 // The staged kernel, us of it | of the other: behind a sum and a norm 13312 x 2048 11.8 | 12.7, x 3072 16.6 | 18.6, and from two rounds of sixteen bf16 rows on, each
 // of three pieces or more, 13312 x 1536 9.9 | 11.3, 9600 x 2048 10.5 | 11.2, but 8192 x 2048 10.2 | 8.9, 16384 x 1024 9.7 | 9.3; behind a merge of eight splits
 // 4096 x 3072 9.5 | 9.7, 2624 x 4096 9.6 | 10.4, but 5120 x 2048 9.1 | 8.5, 2048 x 4096 7.7 | 7.0; of sixteen, whose partials are twice as many, 2624 x 3072 9.6 | 11.1,
